@@ -21,6 +21,7 @@
 // token use the same values -- so the scan's different rounding of m does not show in the output.
 //
 // MODE 0: an item is a whole segment, from the slot's state (or zero) to the slot's state.
+// (Portions of more than 16 tokens take tile_state.hip where it has their D; what follows is for the others.)
 // Long segments are cut into chunks ([n][4]: segment, first row, rows, -) that run in parallel:
 // MODE 1: a chunk from a zero state: its end state goes to cs [chunks][H][D][V].  What carries a start state
 //         through the chunk goes beside it: for the matrix memory the product of the forget factors (cdec)
@@ -565,12 +566,19 @@ K8S_API int k8s_gated_delta(const void* qkv, int dt, const float* a, const float
                  : launch_matrix_state<0, float>(p, n_seg, n_chunks, seg_chunk0, s);
 }
 
-// out = S^T q raw (q unscaled), mul [T][H] = what it is to be multiplied by; scale_out != 0: out *= mul here
+namespace k8s {
+int matrix_memory_tiles(const float* x, int xs, const float* ab, float* state, float* nstate, const int* seg_row0,
+                        const int* seg_pos0, const int* seg_slot, float* nq, float* out, int n_seg, int H, int D, int V, hipStream_t s,
+                        const int* tiles, int n_tiles, const int* seg_tile0, float* ws);   // tile_state.hip
+}
+
+// out = S^T q raw (q unscaled), mul [T][H] = what it is to be multiplied by; scale_out != 0: out *= mul here.
+// tile_ws: chunks are tiles of 16 rows and tile_state.hip works through them in this workspace (cs, cx, cdec unused)
 K8S_API int k8s_matrix_memory(const float* x, int xs, const float* gate_bias, float cap, float* state, float* nstate,
                               float* mstate, const int* seg_row0, const int* seg_pos0, const int* seg_slot, float* ab,
                               float* nq, float* mul, float* out, int n_seg, int T, int H, int D, int V, float den_eps,
                               int scale_out, hipStream_t s, const int* chunks, int n_chunks, const int* seg_chunk0,
-                              float* cs, float* cx, float* cdec) {
+                              float* cs, float* cx, float* cdec, float* tile_ws) {
   if (n_seg <= 0 || T <= 0) return 0;
   if (D < 1 || D > 256 || cap <= 0.f) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(memory_gates_kernel, dim3((n_seg * H + 3) / 4), dim3(256), 0, s, x, xs, gate_bias, cap, mstate,
@@ -594,7 +602,9 @@ K8S_API int k8s_matrix_memory(const float* x, int xs, const float* gate_bias, fl
   p.cs = cs;
   p.cx = cx;
   p.cdec = cdec;
-  const int rc = launch_matrix_state<1, float>(p, n_seg, n_chunks, seg_chunk0, s);
+  const int rc = tile_ws ? matrix_memory_tiles(x, xs, ab, state, nstate, seg_row0, seg_pos0, seg_slot, nq, out, n_seg, H, D, V, s,
+                                               chunks, n_chunks, seg_chunk0, tile_ws)
+                         : launch_matrix_state<1, float>(p, n_seg, n_chunks, seg_chunk0, s);
   if (rc) return rc;
   hipLaunchKernelGGL(memory_den_kernel, dim3((T * H + 255) / 256), dim3(256), 0, s, nq, ab, mul, T * H,
                      1.f / sqrtf((float)D), den_eps);

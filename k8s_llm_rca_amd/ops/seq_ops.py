@@ -1105,6 +1105,23 @@ def _mat_chunks(seg: SegMeta, H: int, V: int):
     if seg.n_seg * H * -(-V // 64) >= MAT_FILL_GROUPS:
         return None
     return seg.chunk_ranges(MAT_CHUNK, 2 * MAT_CHUNK)
+
+
+MAT_TILE = 16       # tokens per tile of the matrix-core form
+
+
+def _mat_tiles(seg: SegMeta, kind: int, H: int, D: int, V: int):
+    """(tiles, first tile of every segment, floats of workspace) for the matrix-core form of the delta rule (``kind`` 0) or
+    the matrix memory (1), or None: no portion is long enough, or no form for ``D``.  Where the line lies (16 heads, D 64,
+    V 128; token by token or in chunks -> tiles, us):  delta rule, one sequence of 16 / 17 / 129 tokens 21 -> 21 / 23 -> 19 /
+    165 -> 29, 64 of 17 tokens 72 -> 52;  memory, one of 17 / 33 / 129 tokens 23 -> 27 / 30 -> 28 / 73 -> 29, 64 of 17 tokens
+    68 -> 48 -- its own steps are cheaper, so that few sequences need two tiles before the tiles' launch pays."""
+    per = lib().k8s_tile_state_ws(kind, D)
+    few = seg.n_seg * H * -(-V // 64) < MAT_FILL_GROUPS
+    cr = seg.chunk_ranges(MAT_TILE, 2 * MAT_TILE if kind == 1 and few else MAT_TILE) if per else None
+    return None if cr is None else (*cr, cr[0].shape[0] * H * per + 256)
+
+
 UNIT_EPS = 1e-6     # q and k of the delta rule: x / sqrt(sum(x^2) + UNIT_EPS)
 
 
@@ -1124,8 +1141,19 @@ def gated_delta(qkv: torch.Tensor, H: int, G: int, D: int, V: int, a: torch.Tens
         assert beta.dtype == torch.float32 and beta.stride(1) == 1 and beta.shape[1] >= H
         assert rate.dtype == dt_bias.dtype == torch.float32 and rate.numel() == H and dt_bias.numel() == H * D
         assert state.is_contiguous() and state.shape[1:] == (H, D, V)
-        # long portions: chunks in parallel (end states and step-matrix products from zero / identity, a carry
-        # over the chunks, the chunks again from their start states); short ones token by token
+        got = _mat_tiles(seg, 0, H, D, V)
+        if got is not None:
+            tiles, t0, n = got
+            ws = scratch(n, torch.float32, qkv.device)
+            check(lib().k8s_gated_delta_tiles(ptr(qkv), _dt(qkv.dtype), ptr(a), ptr(rate), ptr(dt_bias), ptr(beta),
+                                              beta.stride(0), ptr(state), ptr(seg.seg_row0), ptr(seg.seg_pos0),
+                                              ptr(seg.seg_slot), ptr(out),
+                                              seg.n_seg, H, G, D, V, float(UNIT_EPS), stream_ptr(qkv), ptr(tiles),
+                                              tiles.shape[0], ptr(t0), ptr(ws)),
+                  "gated_delta_tiles")
+            return out
+        # other sizes, long portions: chunks in parallel (end states and step-matrix products from zero / identity, a
+        # carry over the chunks, the chunks again from their start states); short ones token by token
         cr = _mat_chunks(seg, H, V)
         chunks, c0, cs, cx, nch = None, None, None, None, 0
         if cr is not None:
@@ -1183,11 +1211,15 @@ def matrix_memory(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tens
         ab = scratch(T * H * 3, torch.float32, x.device)
         nq = scratch(T * H, torch.float32, x.device)
         mul = scratch((T, H), torch.float32, x.device)
-        # long portions: chunks in parallel (end states from zero, a carry over the chunks, the chunks again
+        # other sizes, long portions: chunks in parallel (end states from zero, a carry over the chunks, the chunks again
         # from their start states); short ones token by token
-        cr = _mat_chunks(seg, H, V)
-        chunks, c0, cs, cx, cdec, nch = None, None, None, None, None, 0
-        if cr is not None:
+        got = _mat_tiles(seg, 1, H, D, V)
+        cr = _mat_chunks(seg, H, V) if got is None else None
+        chunks, c0, cs, cx, cdec, nch, tws = None, None, None, None, None, 0, None
+        if got is not None:
+            chunks, c0, n = got
+            nch, tws = chunks.shape[0], scratch(n, torch.float32, x.device)
+        elif cr is not None:
             chunks, c0 = cr
             nch = chunks.shape[0]
             cs = scratch(nch * H * D * V, torch.float32, x.device)
@@ -1197,7 +1229,7 @@ def matrix_memory(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tens
                                       ptr(mstate), ptr(seg.seg_row0), ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(ab),
                                       ptr(nq), ptr(mul), ptr(out), seg.n_seg, T, H, D, V, float(DEN_EPS),
                                       0 if defer_scale else 1, stream_ptr(x), ptr(chunks), nch, ptr(c0), ptr(cs),
-                                      ptr(cx), ptr(cdec)), "matrix_memory")
+                                      ptr(cx), ptr(cdec), ptr(tws)), "matrix_memory")
         return (out, mul) if defer_scale else out
     HD, HV = H * D, H * V
     q = x[:, :HD].view(T, H, D) * D ** -0.5

@@ -1,0 +1,120 @@
+"""Portions of more than 16 tokens through the delta rule and the matrix memory in tiles on the matrix cores, against the
+recurrences token by token in 64 bits: tile remainders, every state height with a form, decays from none to total."""
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from k8s_llm_rca_amd.ops import seq_ops as S
+
+DT = torch.float64
+gpu = pytest.mark.gpu
+
+
+def seg_meta(lens, pos0, slots, dev):
+    row0 = [0]
+    for n in lens:
+        row0.append(row0[-1] + n)
+
+    def i32(v):
+        return torch.tensor(v, dtype=torch.int32, device=dev)
+    return S.SegMeta(len(lens), i32([s for s, n in enumerate(lens) for _ in range(n)]), i32(row0), i32(pos0), i32(slots),
+                     i32([[0]] * len(lens)), row0, list(pos0), list(slots))
+
+
+def close(got, want, lens):
+    """fp32 sums over at most the whole portion: a few roundings (2^-24) per term, in every token's own order."""
+    tol = 16 * 2.0 ** -24 * math.sqrt(max(lens)) * float(want.abs().max())
+    assert float((got.double().cpu() - want).abs().max()) < tol
+
+
+# lengths around the tile, a continuing sequence, a single token beside it, slots out of order
+SEGS = [((17, 1, 33), (0, 5, 9), (2, 0, 1)), ((47, 32), (3, 0), (0, 1)), ((16, 65, 2), (7, 1, 0), (1, 2, 0))]
+
+
+@gpu
+@pytest.mark.parametrize("lens,pos0,slots", SEGS)
+@pytest.mark.parametrize("H,G,D,V", [(2, 1, 16, 24), (2, 2, 32, 7), (4, 2, 64, 128), (1, 1, 96, 65), (2, 1, 128, 64)])
+@pytest.mark.parametrize("strength", [0.1, 2.0, 60.0])
+def test_delta_rule_in_tiles(H, G, D, V, lens, pos0, slots, strength):
+    g = torch.Generator().manual_seed(D + len(lens))
+    T = sum(lens)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g, dtype=DT)
+    x = rnd(T, 2 * G * D + H * V).float()
+    a, beta, bias = rnd(T, H * D).float(), rnd(T, H).float(), rnd(H * D).float()
+    rate = (strength * torch.exp(0.5 * rnd(H))).float()
+    a[::5] += 8.0                              # total decay beside channels that keep nearly all
+    state = rnd(3, H, D, V).float()
+    xd = x.double()
+    q, k, v = xd[:, :G * D].view(T, G, D), xd[:, G * D:2 * G * D].view(T, G, D), xd[:, 2 * G * D:].view(T, H, V)
+    q = (q / torch.sqrt((q * q).sum(-1, keepdim=True) + 1e-6) * D ** -0.5).repeat_interleave(H // G, 1)
+    k = (k / torch.sqrt((k * k).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(H // G, 1)
+    dec = torch.exp(-rate.double()[:, None] * F.softplus(a.double() + bias.double()).view(T, H, D))
+    bt = torch.sigmoid(beta.double())
+    want, end, r = torch.zeros(T, H, V, dtype=DT), state.double(), 0
+    for n, p0, sl in zip(lens, pos0, slots):
+        Sm = end[sl].clone() if p0 else torch.zeros(H, D, V, dtype=DT)
+        for i in range(r, r + n):
+            Sm = dec[i][:, :, None] * Sm
+            u = bt[i][:, None] * (v[i] - torch.einsum("hdv,hd->hv", Sm, k[i]))
+            Sm = Sm + k[i][:, :, None] * u[:, None]
+            want[i] = torch.einsum("hdv,hd->hv", Sm, q[i])
+        end[sl], r = Sm, r + n
+    dev = torch.device("cuda")
+    st = state.to(dev)
+    assert S._mat_tiles(seg_meta(lens, pos0, slots, dev), 0, H, D, V) is not None
+    got = S.gated_delta(x.to(dev), H, G, D, V, a.to(dev), rate.to(dev), bias.to(dev), beta.to(dev), st,
+                        seg_meta(lens, pos0, slots, dev))
+    close(got.view(T, H, V), want, lens)
+    close(st, end, lens)
+
+
+@gpu
+@pytest.mark.parametrize("lens,pos0,slots", SEGS)
+@pytest.mark.parametrize("H,D,V", [(2, 16, 24), (3, 32, 7), (2, 64, 128), (1, 96, 63), (2, 128, 64)])
+@pytest.mark.parametrize("cap", [0.5, 15.0])
+def test_matrix_memory_in_tiles(H, D, V, lens, pos0, slots, cap):
+    g = torch.Generator().manual_seed(D + len(lens))
+    T = sum(lens)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g, dtype=DT)
+    x = rnd(T, 2 * H * (D + V) + 2 * H).float()
+    x[:, -2 * H:] *= 6.0
+    gb = rnd(2 * H).float()
+    st = [rnd(3, H, D, V).float(), rnd(3, H, D).float(), rnd(3, H).float()]
+    xd = x.double()
+    q, k = xd[:, :H * D].view(T, H, D) * D ** -0.5, xd[:, H * D:2 * H * D].view(T, H, D)
+    v = xd[:, 2 * H * D:2 * H * D + H * V].view(T, H, V)
+    gates = cap * torch.tanh((xd[:, -2 * H:] + gb.double()) / cap)
+    gi, gf = gates[:, :H], F.logsigmoid(gates[:, H:])
+    want, end, r = torch.zeros(T, H, V, dtype=DT), [t.double() for t in st], 0
+    for n, p0, sl in zip(lens, pos0, slots):
+        Sm, nn, m = ([e[sl].clone() for e in end] if p0 else
+                     [torch.zeros(H, D, V, dtype=DT), torch.zeros(H, D, dtype=DT), torch.zeros(H, dtype=DT)])
+        for i in range(r, r + n):
+            mn = torch.maximum(gf[i] + m, gi[i])
+            fa, ia = torch.exp(gf[i] + m - mn), torch.exp(gi[i] - mn)
+            Sm = fa[:, None, None] * Sm + (ia[:, None] * k[i])[:, :, None] * v[i][:, None]
+            nn, m = fa[:, None] * nn + ia[:, None] * k[i], mn
+            den = torch.maximum((nn * q[i]).sum(-1).abs(), torch.exp(-m)) + S.DEN_EPS
+            want[i] = torch.einsum("hdv,hd->hv", Sm, q[i]) / den[:, None]
+        for e, t in zip(end, (Sm, nn, m)):
+            e[sl] = t
+        r += n
+    dev = torch.device("cuda")
+    std = [t.to(dev) for t in st]
+    assert S._mat_tiles(seg_meta(lens, pos0, slots, dev), 1, H, D, V) is not None
+    o = S.matrix_memory(x.to(dev), H, D, V, gb.to(dev), cap, *std, seg_meta(lens, pos0, slots, dev)).view(T, H, V)
+    # a denominator near its floor e^(-m) + 1e-6 or of cancelling terms magnifies both sides alike: errors are taken
+    # against the token's own largest output, gates of up to exp(cap) against 64-bit ones
+    err = ((o.double().cpu() - want).abs().amax(-1) / want.abs().amax(-1)).flatten()
+    assert float(err.median()) < 4e-6 and float(err.max()) < 2e-3
+    # the running maximum comes from a scan over sums of up to n log gates of size cap (2^-24 each of a partial sum of up
+    # to n cap, a few roundings deep); the states are e^(-m) times the unstabilised ones, so its error is their relative one
+    rel = 16 * 2.0 ** -24 * math.sqrt(max(lens)) + 2 * max(lens) * cap * 2.0 ** -24
+    for got, e in zip(std, end):
+        assert float((got.double().cpu() - e).abs().max()) < rel * float(e.abs().max())
