@@ -22,7 +22,7 @@
 //   holds H M heads laid out [h][m] and the key pages G M heads [g][m]: map m of head h scores against key
 //   head (h / (H / G)) M + m and applies its weights to value head h / (H / G); the output is [T][H][M][V],
 //   each map's result by itself (fp32 where the caller joins the maps).
-//   The visible keys of a row are two runs, [a0, a1) (kept first tokens) and [lo, pos]; both kernels walk
+//   The visible keys of a row are two runs, [a0, a1) (kept first tokens) and [lo, pos]; the kernels (the vector-pipe one: rows_attn.hip) walk
 //   them as one virtual range whose tile borders depend on the row's position only, so a row's result
 //   does not depend on how the prompt was cut or on what else is in the step.
 //
@@ -30,15 +30,10 @@
 // Scores, weights and accumulation are fp32; TA (bf16 as uint16_t, or float) is the type of q, the pages
 // and the output.
 #include "common.h"
+#include "key_runs.h"
 
 namespace k8s {
 
-template <typename T>
-__device__ __forceinline__ float lda(const T* p, size_t i);
-template <>
-__device__ __forceinline__ float lda<float>(const float* p, size_t i) { return p[i]; }
-template <>
-__device__ __forceinline__ float lda<uint16_t>(const uint16_t* p, size_t i) { return bf2f(p[i]); }
 template <typename T>
 __device__ __forceinline__ void sta(T* p, size_t i, float v);
 template <>
@@ -322,121 +317,6 @@ __global__ void __launch_bounds__(256) attn_prep_half_kernel(const float* __rest
   write_values<TA, TR>(x, qs, r0, nr, NV, v_col, bias, slots, vc, vt, BS, tid);
 }
 
-// The visible keys of position `pos`: [a0, a1) and [lo, pos], walked as x in [0, nA + nB).
-struct KeyRuns {
-  int a0, nA, lo, total;
-  __device__ __forceinline__ int key(int x) const { return x < nA ? a0 + x : lo + (x - nA); }
-};
-
-__device__ __forceinline__ KeyRuns key_runs(int pos, int chunk, int window, int keep_first) {
-  KeyRuns k;
-  k.a0 = chunk > 0 ? (pos / chunk) * chunk : 0;
-  k.lo = k.a0;
-  k.nA = 0;
-  if (window > 0) {
-    k.lo = max(k.a0, pos - window + 1);
-    k.nA = max(0, min(keep_first, k.lo) - k.a0);
-  }
-  k.total = k.nA + pos - k.lo + 1;
-  return k;
-}
-
-constexpr int kMaskTile = 64;   // keys per tile: one per lane
-constexpr int kMaskOut = 32;    // outputs per thread: H * V <= 256 * kMaskOut
-
-template <typename TA>
-__device__ __forceinline__ float mask_score(const float* q, const TA* __restrict__ kc, const int* __restrict__ bt, int BS,
-                                            int NK, int D, int g, int j, float scale, float softcap) {
-  const TA* kr = kc + ((size_t)bt[j / BS] * BS + (j % BS)) * NK + (size_t)g * D;
-  float a = 0.f;
-  for (int d = 0; d < D; ++d) a = fmaf(q[d], lda(kr, d), a);
-  a *= scale;
-  return softcap > 0.f ? softcap * tanhf(a / softcap) : a;
-}
-
-// One workgroup per row, two passes over the row's visible keys in tiles of 64:
-//   1. per head the maximum (the sink included) and the denominator, online (a wave per head);
-//   2. scores again -> weights in LDS -> times the values (a thread per output column).
-template <typename TA, typename TO>
-__global__ void __launch_bounds__(256) masked_attn_rows_kernel(const TA* __restrict__ q, const TA* __restrict__ kc,
-                                                               const TA* __restrict__ vc,
-                                                               const int* __restrict__ block_tables, int maxb,
-                                                               const int* __restrict__ row_seg,
-                                                               const int* __restrict__ seg_row0,
-                                                               const int* __restrict__ seg_pos0,
-                                                               const float* __restrict__ sink,
-                                                               const float* __restrict__ gate, int gs,
-                                                               TO* __restrict__ out, int H, int G, int D, int V, int BS,
-                                                               int chunk, int window, int keep_first, float scale,
-                                                               float softcap, int M) {
-  // H counts the query heads of D entries (heads x maps); hpg of them share a key / value head group
-  extern __shared__ float sm[];
-  float* qf = sm;                      // [H][D]
-  float* p = qf + H * D;               // [H][64]
-  float* mh = p + H * kMaskTile;       // [H]
-  float* lh = mh + H;                  // [H]
-  const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int sg = row_seg[r], pos = seg_pos0[sg] + r - seg_row0[sg];
-  const KeyRuns kr = key_runs(pos, chunk, window, keep_first);
-  const int* bt = block_tables + (size_t)sg * maxb;
-  const int NK = G * M * D, NV = G * V, hpg = H / (G * M);
-  for (int i = tid; i < H * D; i += 256) qf[i] = lda(q, (size_t)r * H * D + i);
-  __syncthreads();
-  for (int h = wv; h < H; h += 4) {
-    const int g = (h / M / hpg) * M + h % M;
-    float m = sink ? sink[h] : -INFINITY, l = sink ? 1.f : 0.f;
-    for (int x0 = 0; x0 < kr.total; x0 += kMaskTile) {
-      const int x = x0 + lane;
-      const bool ok = x < kr.total;
-      const float s = ok ? mask_score(qf + h * D, kc, bt, BS, NK, D, g, kr.key(x), scale, softcap) : -INFINITY;
-      const float mn = fmaxf(m, wave_max(s));     // finite: every tile holds a visible key
-      l = l * expf(m - mn) + wave_sum(ok ? expf(s - mn) : 0.f);
-      m = mn;
-    }
-    if (lane == 0) {
-      mh[h] = m;
-      lh[h] = l;
-    }
-  }
-  __syncthreads();
-  float acc[kMaskOut];
-#pragma unroll
-  for (int i = 0; i < kMaskOut; ++i) acc[i] = 0.f;
-  for (int x0 = 0; x0 < kr.total; x0 += kMaskTile) {
-    for (int h = wv; h < H; h += 4) {
-      const int x = x0 + lane;
-      const bool ok = x < kr.total;
-      const float s =
-          ok ? mask_score(qf + h * D, kc, bt, BS, NK, D, (h / M / hpg) * M + h % M, kr.key(x), scale, softcap) : 0.f;
-      p[h * kMaskTile + lane] = ok ? expf(s - mh[h]) / lh[h] : 0.f;
-    }
-    __syncthreads();
-    const int nk = min(kMaskTile, kr.total - x0);
-#pragma unroll
-    for (int i = 0; i < kMaskOut; ++i) {
-      const int o = tid + i * 256;
-      if (o < H * V) {
-        const int h = o / V, v = o - h * V, g = h / M / hpg;
-        float a = acc[i];
-        for (int jj = 0; jj < nk; ++jj) {
-          const int j = kr.key(x0 + jj);
-          a = fmaf(p[h * kMaskTile + jj], lda(vc, ((size_t)bt[j / BS] * BS + (j % BS)) * NV + (size_t)g * V + v), a);
-        }
-        acc[i] = a;
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < kMaskOut; ++i) {
-    const int o = tid + i * 256;
-    if (o < H * V) {
-      float a = acc[i];
-      if (gate) a *= 1.f / (1.f + expf(-gate[(size_t)r * gs + o / V]));
-      sta(out, (size_t)r * H * V + o, a);   // (gates count heads x maps like H)
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------------------------
 // Matrix-core form (bf16, v_mfma_f32_16x16x32_bf16), one pass with an online softmax.  A work item is a
@@ -846,33 +726,6 @@ K8S_API int k8s_attn_prep_half(const float* x, int qs, int H, int G, int D, int 
     else K8S_PH(float, 1);
   }
 #undef K8S_PH
-  return (int)hipGetLastError();
-}
-
-K8S_API int k8s_masked_attn_rows(const void* q, const void* kc, const void* vc, const int* block_tables, int maxb,
-                                 const int* row_seg, const int* seg_row0, const int* seg_pos0, const float* sink,
-                                 const float* gate, int gs, void* out, int T, int H, int G, int D, int V, int BS,
-                                 int chunk, int window, int keep_first, float scale, float softcap, int dt,
-                                 hipStream_t s, int maps, int out_f32) {
-  if (T <= 0) return 0;
-  if (maps < 1) return (int)hipErrorInvalidValue;
-  const int HQ = H * maps;
-  const size_t lds = (size_t)(HQ * D + HQ * kMaskTile + 2 * HQ) * sizeof(float);
-  if (H < 1 || G < 1 || H % G || HQ * V > 256 * kMaskOut || chunk < 0 || window < 0 || keep_first < 0 ||
-      lds > 64 * 1024)
-    return (int)hipErrorInvalidValue;
-#define K8S_ROWS(TA, TO)                                                                                             \
-  hipLaunchKernelGGL((masked_attn_rows_kernel<TA, TO>), dim3(T), dim3(256), lds, s, (const TA*)q, (const TA*)kc,    \
-                     (const TA*)vc, block_tables, maxb, row_seg, seg_row0, seg_pos0, sink, gate, gs, (TO*)out, HQ, G, \
-                     D, V, BS, chunk, window, keep_first, scale, softcap, maps)
-  if (dt == 0 && out_f32) {
-    K8S_ROWS(uint16_t, float);
-  } else if (dt == 0) {
-    K8S_ROWS(uint16_t, uint16_t);
-  } else {
-    K8S_ROWS(float, float);
-  }
-#undef K8S_ROWS
   return (int)hipGetLastError();
 }
 

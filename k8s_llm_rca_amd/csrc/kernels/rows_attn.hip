@@ -1,0 +1,369 @@
+// Softmax attention of single rows over paged keys and values on the vector pipes, fp32 arithmetic: fp32 models, and head
+// sizes the matrix-core kernels do not take.  The masks are masked_attn.hip's, the latent form latent_attn.hip's: there all
+// heads share a cache row of W = R + RP numbers, which is the key, and whose first R numbers are the value.
+//
+// A row's visible keys are cut into parts of 128 by their place in its own key range.  Within a part the scores of up to
+// eight heads of one key head meet in LDS -- a lane has one key and up to four heads, so that a key's numbers are read once
+// for them -- then their softmax, then a thread walks the part's keys for one value column and the heads again.  Parts are
+// joined in order with fixed multiply-adds, by the workgroup itself where there are rows enough to fill the chip, by a
+// second kernel where few rows are spread over a workgroup per part: both do the same arithmetic, so a row's result does
+// not depend on how the prompt was cut or on what else is in the step.
+//
+// What bounds it: the scores (one lane reads a whole key, 16 bytes at a time) and latency at few rows, for which reason the
+// heads and the parts are spread over workgroups.  fp32, 16 heads over 2 of 128, two rows at 340 keys: 980 us (a
+// workgroup per row, all heads one after the other, the scores formed twice) -> 28 us; 666 rows of two prompts: 1451 ->
+// 122 us; latent (16 heads, 256 + 64 numbers): 706 -> 39 and 719 -> 196 us.
+#include "common.h"
+#include "key_runs.h"
+
+namespace k8s {
+
+constexpr int kRaKeys = 128;    // keys of a part
+constexpr int kRaHeads = 8;     // heads of a workgroup
+
+template <typename T>
+__device__ __forceinline__ float rld(const T* p, size_t i);
+template <>
+__device__ __forceinline__ float rld<float>(const float* p, size_t i) { return p[i]; }
+template <>
+__device__ __forceinline__ float rld<uint16_t>(const uint16_t* p, size_t i) { return bf2f(p[i]); }
+template <typename T>
+__device__ __forceinline__ void rst(T* p, size_t i, float v);
+template <>
+__device__ __forceinline__ void rst<float>(float* p, size_t i, float v) { p[i] = v; }
+template <>
+__device__ __forceinline__ void rst<uint16_t>(uint16_t* p, size_t i, float v) { p[i] = f2bf(v); }
+__device__ __forceinline__ f32x4 rld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ f32x4 rld4(const uint16_t* p) {
+  const u16x4 v = *reinterpret_cast<const u16x4*>(p);
+  return f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
+}
+
+struct RowsArgs {
+  const void* q;               // entry d < D1 of head h of row t at t * qst + h * qsh + d
+  long qst, qsh;
+  const float* q2;             // entries D1 .. D1 + D2 at (t * H + h) * D2 (latent form)
+  int D1, D2;
+  const void* kc;              // a key's entries of key head i at slot * ks + i * D
+  const void* vc;              // a value's of value head g at slot * vs + g * V
+  int ks, vs;
+  const int* bt;
+  int maxb;
+  const int* row_seg;
+  const int* seg_row0;
+  const int* seg_pos0;
+  const float* sink;
+  const float* gate;
+  int gs;
+  void* out;                   // entry c of head h of row t at t * ost + h * osh + c
+  long ost, osh;
+  int H, G, M, V, BS;          // H counts heads x maps
+  int row_base, chunk, window, keep_first;
+  float scale, softcap;
+  float* po;                   // [T][H][n_parts][V], null: the workgroup joins the parts
+  float* pml;                  // [T][H][n_parts][2]
+  int n_parts;
+};
+
+// (m, l) and the outputs of a further part; the running maximum may be -inf, the part's is finite
+__device__ __forceinline__ void ra_join(float& m, float& l, float mp, float lp, float& a, float& b) {
+  const float mn = fmaxf(m, mp);
+  a = expf(m - mn);
+  b = expf(mp - mn);
+  l = fmaf(l, a, __fmul_rn(lp, b));
+  m = mn;
+}
+__device__ __forceinline__ float ra_join_out(float o, float a, float op, float b) { return fmaf(o, a, __fmul_rn(op, b)); }
+
+template <typename TQ, typename TC, typename TO, bool VEC>
+__global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int D = p.D1 + p.D2, V = p.V, hpg = p.H / (p.G * p.M);
+  const int HB = min(hpg, kRaHeads), nhb = (hpg + HB - 1) / HB, nvb = (V + 255) / 256;
+  float* sq = sm;                                   // [HB][D4]
+  const int D4 = (D + 3) & ~3;
+  float* sp = sq + HB * D4;                         // [HB][128]
+  float* sl = sp + HB * kRaKeys;                    // [HB][2]: m, l of the part
+  int* ss = reinterpret_cast<int*>(sl + 2 * HB);    // [128]: cache slots
+  const int r = p.row_base + blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  int gi = blockIdx.y;
+  const int vb = gi % nvb;
+  gi /= nvb;
+  const int hb = gi % nhb, gm = gi / nhb, g = gm / p.M;
+  const int nh = min(HB, hpg - hb * HB);
+  auto head = [&](int i) { return (g * hpg + hb * HB + i) * p.M + gm % p.M; };
+  const int sg = p.row_seg[r], pos = p.seg_pos0[sg] + r - p.seg_row0[sg];
+  const KeyRuns kr = key_runs(pos, p.chunk, p.window, p.keep_first);
+  const int x_lo = p.po ? blockIdx.z * kRaKeys : 0, x_hi = p.po ? min(kr.total, x_lo + kRaKeys) : kr.total;
+  if (x_lo >= x_hi) return;
+  const int* bt = p.bt + (size_t)sg * p.maxb;
+  for (int i = tid; i < nh * D; i += 256) {
+    const int h = i / D, d = i - h * D;
+    sq[h * D4 + d] = d < p.D1 ? rld((const TQ*)p.q, (size_t)r * p.qst + (size_t)head(h) * p.qsh + d)
+                              : p.q2[((size_t)r * p.H + head(h)) * p.D2 + d - p.D1];
+  }
+  // this thread's value column and heads
+  const int v0 = vb * 256, vc = min(V - v0, 256), tpc = 256 / vc, hs = tid / vc, col = tid - hs * vc;
+  const bool own = hs < tpc;
+  const TC* kbase = (const TC*)p.kc + (size_t)gm * D;
+  const TC* vbase = (const TC*)p.vc + (size_t)g * V + v0 + col;
+  float m[kRaHeads], l[kRaHeads], o[kRaHeads];      // of head hs + k tpc
+#pragma unroll
+  for (int k = 0; k < kRaHeads; ++k) {
+    const int h = hs + k * tpc;
+    const bool on = own && h < nh && p.sink && !p.po;
+    m[k] = on ? p.sink[head(h)] : -INFINITY;
+    l[k] = on ? 1.f : 0.f;
+    o[k] = 0.f;
+  }
+  for (int x0 = x_lo; x0 < x_hi; x0 += kRaKeys) {
+    const int nk = min(kRaKeys, x_hi - x0);
+    __syncthreads();                                // the part before is read no more
+    if (tid < kRaKeys) {
+      const int j = kr.key(x0 + min(tid, nk - 1));
+      ss[tid] = bt[j / p.BS] * p.BS + j % p.BS;
+    }
+    __syncthreads();
+    {  // scores: a wave has 64 keys and every other head
+      const int x = (wv & 1) * 64 + lane, h0 = wv >> 1;
+      if ((wv & 1) * 64 < nk && h0 < nh) {
+        const TC* kp = kbase + (size_t)ss[x] * p.ks;
+        const float* q0 = sq + h0 * D4;
+        const float* qh[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) qh[k] = h0 + 2 * k < nh ? q0 + 2 * k * D4 : q0;
+        float a[4] = {0.f, 0.f, 0.f, 0.f};
+        if (VEC) {
+#pragma unroll 4
+          for (int d = 0; d < D; d += 4) {
+            const f32x4 kv = rld4(kp + d);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const f32x4 qv = *reinterpret_cast<const f32x4*>(qh[k] + d);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) a[k] = fmaf(qv[e], kv[e], a[k]);
+            }
+          }
+        } else {
+          for (int d = 0; d < D; ++d) {
+            const float kv = rld(kp, d);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) a[k] = fmaf(qh[k][d], kv, a[k]);
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (h0 + 2 * k < nh) {
+            float s = a[k] * p.scale;
+            if (p.softcap > 0.f) s = p.softcap * tanhf(s / p.softcap);
+            sp[(h0 + 2 * k) * kRaKeys + x] = x < nk ? s : -INFINITY;
+          }
+      } else if (h0 < nh) {
+        for (int h = h0; h < nh; h += 2) sp[h * kRaKeys + x] = -INFINITY;
+      }
+    }
+    __syncthreads();
+    for (int h = wv; h < nh; h += 4) {              // the part's softmax, a wave per head
+      const float s0 = sp[h * kRaKeys + lane], s1 = sp[h * kRaKeys + 64 + lane];
+      const float mp = wave_max(fmaxf(s0, s1));     // finite: a part holds a visible key
+      const float e0 = expf(s0 - mp), e1 = expf(s1 - mp);
+      sp[h * kRaKeys + lane] = e0;
+      sp[h * kRaKeys + 64 + lane] = e1;
+      const float lp = wave_sum(e0 + e1);
+      if (lane == 0) {
+        sl[2 * h] = mp;
+        sl[2 * h + 1] = lp;
+      }
+    }
+    __syncthreads();
+    if (own) {
+      float op[kRaHeads];
+#pragma unroll
+      for (int k = 0; k < kRaHeads; ++k) op[k] = 0.f;
+      const int nk4 = (nk + 3) & ~3;                // (weights past nk are zero, their slots repeat the last)
+      for (int j = 0; j < nk4; j += 4) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = rld(vbase, (size_t)ss[j + e] * p.vs);
+#pragma unroll
+        for (int k = 0; k < kRaHeads; ++k) {
+          const int h = hs + k * tpc;
+          if (h < nh) {
+            const f32x4 w = *reinterpret_cast<const f32x4*>(sp + h * kRaKeys + j);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) op[k] = fmaf(w[e], v[e], op[k]);
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kRaHeads; ++k) {
+        const int h = hs + k * tpc;
+        if (h < nh) {
+          if (p.po) {
+            const size_t at = ((size_t)blockIdx.x * p.H + head(h)) * p.n_parts + blockIdx.z;
+            p.po[at * V + v0 + col] = op[k];
+            if (col == 0 && vb == 0) {
+              p.pml[at * 2] = sl[2 * h];
+              p.pml[at * 2 + 1] = sl[2 * h + 1];
+            }
+          } else {
+            float a, b;
+            ra_join(m[k], l[k], sl[2 * h], sl[2 * h + 1], a, b);
+            o[k] = ra_join_out(o[k], a, op[k], b);
+          }
+        }
+      }
+    }
+  }
+  if (p.po || !own) return;
+#pragma unroll
+  for (int k = 0; k < kRaHeads; ++k) {
+    const int h = hs + k * tpc;
+    if (h < nh) {
+      const int hh = head(h);
+      float v = o[k] / l[k];
+      if (p.gate) v *= 1.f / (1.f + expf(-p.gate[(size_t)r * p.gs + hh]));
+      rst((TO*)p.out, (size_t)r * p.ost + (size_t)hh * p.osh + v0 + col, v);
+    }
+  }
+}
+
+// joins the parts of a (row, head) in order
+template <typename TO>
+__global__ void __launch_bounds__(256) rows_attn_merge_kernel(RowsArgs p) {
+  const int r = p.row_base + blockIdx.x, hh = blockIdx.y;
+  const int sg = p.row_seg[r], pos = p.seg_pos0[sg] + r - p.seg_row0[sg];
+  const int n = (key_runs(pos, p.chunk, p.window, p.keep_first).total + kRaKeys - 1) / kRaKeys;
+  const size_t at = ((size_t)blockIdx.x * p.H + hh) * p.n_parts;
+  for (int c = threadIdx.x; c < p.V; c += blockDim.x) {
+    float m = p.sink ? p.sink[hh] : -INFINITY, l = p.sink ? 1.f : 0.f, o = 0.f;
+    for (int k = 0; k < n; ++k) {
+      float a, b;
+      ra_join(m, l, p.pml[(at + k) * 2], p.pml[(at + k) * 2 + 1], a, b);
+      o = ra_join_out(o, a, p.po[(at + k) * p.V + c], b);
+    }
+    float v = o / l;
+    if (p.gate) v *= 1.f / (1.f + expf(-p.gate[(size_t)r * p.gs + hh]));
+    rst((TO*)p.out, (size_t)r * p.ost + (size_t)hh * p.osh + c, v);
+  }
+}
+
+template <typename TQ, typename TC, typename TO>
+static int launch_rows(const RowsArgs& p, int T, hipStream_t s) {
+  const int D = p.D1 + p.D2, hpg = p.H / (p.G * p.M), HB = hpg < kRaHeads ? hpg : kRaHeads;
+  const size_t lds = sizeof(float) * ((size_t)HB * ((D + 3) / 4 * 4) + HB * kRaKeys + 2 * HB + kRaKeys);
+  const dim3 grid(T, p.G * p.M * ((hpg + HB - 1) / HB) * ((p.V + 255) / 256), p.po ? p.n_parts : 1);
+  // four numbers of a key at a time where every key starts on such a border
+  const bool vec = D % 4 == 0 && p.ks % 4 == 0 && ((uintptr_t)p.kc & (4 * sizeof(TC) - 1)) == 0;
+  auto k = vec ? rows_attn_kernel<TQ, TC, TO, true> : rows_attn_kernel<TQ, TC, TO, false>;
+  if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
+    return (int)hipGetLastError();
+  hipLaunchKernelGGL(k, grid, dim3(256), lds, s, p);
+  if (p.po)
+    hipLaunchKernelGGL((rows_attn_merge_kernel<TO>), dim3(T, p.H), dim3(p.V >= 256 ? 256 : (p.V + 63) / 64 * 64), 0, s, p);
+  return (int)hipGetLastError();
+}
+
+}  // namespace k8s
+
+using namespace k8s;
+
+// n_parts > 0: a workgroup per part of 128 visible keys (n_parts: at least the parts of the row that sees most), joined from
+// po [T][H maps][n_parts][V] and pml [.. ][2]; 0: a workgroup walks all parts
+K8S_API int k8s_masked_attn_rows(const void* q, const void* kc, const void* vc, const int* block_tables, int maxb,
+                                 const int* row_seg, const int* seg_row0, const int* seg_pos0, const float* sink,
+                                 const float* gate, int gs, void* out, int T, int H, int G, int D, int V, int BS,
+                                 int chunk, int window, int keep_first, float scale, float softcap, int dt,
+                                 hipStream_t s, int maps, int out_f32, int n_parts, float* po, float* pml) {
+  if (T <= 0) return 0;
+  if (maps < 1) return (int)hipErrorInvalidValue;
+  const int HQ = H * maps;
+  // (a row's queries and outputs: at most 64 KB and 8192 numbers)
+  if (H < 1 || G < 1 || H % G || D < 1 || V < 1 || HQ * V > 8192 || chunk < 0 || window < 0 || keep_first < 0 ||
+      (size_t)(HQ * D + HQ * 64 + 2 * HQ) * sizeof(float) > 64 * 1024 || (n_parts > 0 && (!po || !pml)))
+    return (int)hipErrorInvalidValue;
+  RowsArgs p{};
+  p.q = q;
+  p.qst = (long)HQ * D;
+  p.qsh = D;
+  p.D1 = D;
+  p.kc = kc;
+  p.vc = vc;
+  p.ks = G * maps * D;
+  p.vs = G * V;
+  p.bt = block_tables;
+  p.maxb = maxb;
+  p.row_seg = row_seg;
+  p.seg_row0 = seg_row0;
+  p.seg_pos0 = seg_pos0;
+  p.sink = sink;
+  p.gate = gate;
+  p.gs = gs;
+  p.out = out;
+  p.ost = (long)HQ * V;
+  p.osh = V;
+  p.H = HQ;
+  p.G = G;
+  p.M = maps;
+  p.V = V;
+  p.BS = BS;
+  p.chunk = chunk;
+  p.window = window;
+  p.keep_first = keep_first;
+  p.scale = scale;
+  p.softcap = softcap;
+  p.n_parts = n_parts;
+  p.po = n_parts > 0 ? po : nullptr;
+  p.pml = pml;
+  if (dt == 0 && out_f32) return launch_rows<uint16_t, uint16_t, float>(p, T, s);
+  if (dt == 0) return launch_rows<uint16_t, uint16_t, uint16_t>(p, T, s);
+  return launch_rows<float, float, float>(p, T, s);
+}
+
+// Rows row_base .. row_base + n_rows of the step.  dt: 0 = bf16 cache and output, 1 = fp32.
+K8S_API int k8s_latent_attn_rows(const float* qa, const void* cache, const int* bt, int maxb, const int* row_seg,
+                                 const int* seg_row0, const int* seg_pos0, const float* gate, int ldg, void* out,
+                                 int row_base, int n_rows, int H, int R, int BS, float scale, int dt,
+                                 hipStream_t s, long qst, long qsh, const float* qr, int RP, long ost, long osh,
+                                 int window, const float* sink, int n_parts, float* po, float* pml) {
+  if (n_rows <= 0) return 0;
+  if (H <= 0 || R <= 0 || R > 2048 || RP < 0 || (RP && !qr) || window < 0 || (n_parts > 0 && (!po || !pml)))
+    return (int)hipErrorInvalidValue;
+  // (the widest cache rows: as many heads' queries as make 2048 numbers, 32 keys and their scores within 160 KB)
+  const size_t hg = 2048 / R < H ? (2048 / R < 64 ? 2048 / R : 64) : (H < 64 ? H : 64);
+  if ((hg * (R + RP) + 32 * (size_t)(R + RP + 1) + 35 * hg) * sizeof(float) > 160 * 1024) return (int)hipErrorInvalidValue;
+  RowsArgs p{};
+  p.q = qa;
+  p.qst = qst;
+  p.qsh = qsh;
+  p.q2 = qr;
+  p.D1 = R;
+  p.D2 = RP;
+  p.kc = cache;
+  p.vc = cache;
+  p.ks = R + RP;
+  p.vs = R + RP;
+  p.bt = bt;
+  p.maxb = maxb;
+  p.row_seg = row_seg;
+  p.seg_row0 = seg_row0;
+  p.seg_pos0 = seg_pos0;
+  p.sink = sink;
+  p.gate = gate;
+  p.gs = ldg;
+  p.out = out;
+  p.ost = ost;
+  p.osh = osh;
+  p.H = H;
+  p.G = 1;
+  p.M = 1;
+  p.V = R;
+  p.BS = BS;
+  p.row_base = row_base;
+  p.window = window;
+  p.scale = scale;
+  p.n_parts = n_parts;
+  p.po = n_parts > 0 ? po : nullptr;
+  p.pml = pml;
+  return dt == 0 ? launch_rows<float, uint16_t, uint16_t>(p, n_rows, s) : launch_rows<float, float, float>(p, n_rows, s);
+}

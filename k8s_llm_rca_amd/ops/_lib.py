@@ -94,7 +94,7 @@ _SIGS = {
     "k8s_rotated_tail": [P, P, P, I, I, I, I, I, I, P],
     "k8s_latent_attn_mfma_ok": [I, I],
     "k8s_latent_attn_mfma": [P, P, P, P, I, P, I, P, I, P, P, P, I, I, P, I, I, I, I, F, I, I, P, L, L, P, I, L, L, I, P],
-    "k8s_latent_attn_rows": [P, P, P, I, P, P, P, P, I, P, I, I, I, I, I, F, I, P, L, L, P, I, L, L, I, P],
+    "k8s_latent_attn_rows": [P, P, P, I, P, P, P, P, I, P, I, I, I, I, I, F, I, P, L, L, P, I, L, L, I, P, I, P, P],
     "k8s_polynorm": [P, P, P, I, I, F, I, P],
     "k8s_glu_clamp": [P, P, I, I, F, F, F, I, P],
     "k8s_router": [P, P, I, I, I, I, I, I, P, P, I, P, P, F, I, P, F, I, I],
@@ -125,7 +125,7 @@ _SIGS = {
     "k8s_rope_table": [P, P, F, P, I, I, P],
     "k8s_attn_prep_pairs": [P, I, I, I, I, I, I, P, P, P, P, I, P, I, I, P, I, P],
     "k8s_attn_prep_half": [P, I, I, I, I, I, I, P, P, P, P, P, I, P, I, I, P, I, P, P, F, I, P],
-    "k8s_masked_attn_rows": [P, P, P, P, I, P, P, P, P, P, I, P, I, I, I, I, I, I, I, I, I, F, F, I, P, I, I],
+    "k8s_masked_attn_rows": [P, P, P, P, I, P, P, P, P, P, I, P, I, I, I, I, I, I, I, I, I, F, F, I, P, I, I, I, P, P],
     "k8s_masked_attn_mfma_ok": [I, I, I, I],
     "k8s_masked_attn_mfma": [P, P, P, P, I, P, I, P, P, I, P, I, I, I, I, I, I, I, I, F, F, P, I, I, P, P, I, I],
     "k8s_gated_delta": [P, I, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, F, P, P, I, P, P, P],

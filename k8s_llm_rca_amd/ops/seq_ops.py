@@ -313,6 +313,32 @@ def rotated_tail(q: torch.Tensor, cs: torch.Tensor, H: int, N: int, pad: int) ->
     return out
 
 
+ROWS_PART = 128     # visible keys per part of the vector-pipe attention
+ROWS_HEADS = 8      # heads of one key head per workgroup of it
+ROWS_FILL = 512     # workgroups from which it walks a row's parts itself
+
+
+def _rows_parts(seg: SegMeta, T: int, heads: int, per_key: int, V: int, dev, chunk: int = 0, window: int = 0,
+                keep_first: int = 0) -> tuple:
+    """(parts, scratch for their outputs, for their maxima and sums) of a step of the vector-pipe attention whose rows do
+    not fill the chip: a workgroup per part of a row's keys, the same sums either way.  (0, None, None): a workgroup per
+    row and group of heads.  One workgroup -> parts, us, fp32, 16 heads over 2 of 128: 2 rows at 340 keys 55 -> 27, 16 at
+    1024 visible ones 148 -> 28, 128 at 300 68 -> 52, 256 at 400 113 -> 118 (the line; past it the parts save a tenth at
+    most and write heads x parts results per row).  ``per_key``: heads that share a key."""
+    groups = heads // per_key * -(-per_key // ROWS_HEADS) * -(-V // 256)
+    if T * groups >= ROWS_FILL:
+        return 0, None, None
+    most = max((p + b - a for p, a, b in zip(seg.pos0_host, seg.row0_host[:-1], seg.row0_host[1:])), default=0)
+    if chunk > 0:
+        most = min(most, chunk)
+    if window > 0:
+        most = min(most, window + keep_first)
+    parts = -(-most // ROWS_PART)
+    if parts <= 1:
+        return 0, None, None
+    return (parts, scratch(T * heads * parts * V, torch.float32, dev), scratch(T * heads * parts * 2, torch.float32, dev))
+
+
 def mfma_tiles(R: int, dtype, device, tail: int = 0) -> int:
     """Query tiles per wave the MFMA attention kernels run prompt portions with for latent rank ``R`` and cache rows of
     ``R + tail`` numbers (0: they do not take these sizes or this type -- the vector-pipe kernel runs instead)."""
@@ -390,12 +416,13 @@ def latent_attention(qa: torch.Tensor, cache: torch.Tensor, gate: Optional[torch
         assert qr is None or (qr.dtype == torch.float32 and qr.is_contiguous() and qr.shape == (T, H, W - R))
         assert sink is None or (sink.dtype == torch.float32 and sink.numel() == H)
         assert seg.block_tables.is_contiguous()
+        parts, po, pml = _rows_parts(seg, T, H, H, R, qa.device, window=int(window))
         check(lib().k8s_latent_attn_rows(ptr(qa), ptr(cache), ptr(seg.block_tables), seg.block_tables.shape[1],
                                          ptr(seg.row_seg), ptr(seg.seg_row0), ptr(seg.seg_pos0), ptr(gate),
                                          gate.stride(0) if gate is not None else 0, ptr(out), 0, T, H, R, BS,
                                          float(scale), _dt(out_dtype), stream_ptr(qa), qa.stride(0), qa.stride(1),
-                                         ptr(qr), W - R, out.stride(0), out.stride(1), int(window), ptr(sink)),
-              "latent_attn_rows")
+                                         ptr(qr), W - R, out.stride(0), out.stride(1), int(window), ptr(sink), parts,
+                                         ptr(po), ptr(pml)), "latent_attn_rows")
         return out
     flat = cache.view(-1, W)
     for s in range(seg.n_seg):
@@ -1006,11 +1033,12 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
                                              ptr(pml), ptr(po), int(maps), int(out_f32)), "masked_attn_mfma")
             return out
         assert vc is not None          # the vector-pipe kernel reads token-major values
+        parts, po, pml = _rows_parts(seg, T, HQ, H // G, V, q.device, int(chunk), int(window), int(keep_first))
         check(lib().k8s_masked_attn_rows(ptr(q), ptr(kc), ptr(vc), ptr(seg.block_tables), seg.block_tables.shape[1],
                                          ptr(seg.row_seg), ptr(seg.seg_row0), ptr(seg.seg_pos0), ptr(sink), ptr(gate),
                                          gs, ptr(out), T, H, G, D, V, BS, int(chunk), int(window), int(keep_first),
                                          float(scale), float(softcap), _dt(q.dtype), stream_ptr(q), int(maps),
-                                         int(out_f32)), "masked_attn_rows")
+                                         int(out_f32), parts, ptr(po), ptr(pml)), "masked_attn_rows")
         return out
     kf, vf = kc.view(-1, G, maps, D), vc.view(-1, G, V)
     rep = H // G
