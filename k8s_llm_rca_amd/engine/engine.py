@@ -161,6 +161,10 @@ class LLMEngine(SchedulerMixin, StepExecMixin, GraphRunnerMixin, SamplerMixin):
         self._mask_ver = -1
         self._graphs: Dict[tuple, tuple] = {}
         self._graph_pool = None
+        # graphs of models in the segment layout: (rows, block-table width) -> (graph, static input, logits)
+        self._seg_graphs: Dict[tuple, tuple] = {}
+        self._seg_seen: Dict[tuple, int] = {}
+        self._seg_stream = None
         self._static = None
         self._pf_ws = None  # prefill split-KV partials (allocated on first split step)
         # multi-token decode items (a short chunk's tokens read their shared keys

@@ -4,6 +4,9 @@ Pure-decode steps replay one captured graph per batch bucket; the decode work
 list, its item count and the keys per item are read on the device, so one
 graph serves every context mix.  Static input buffers are filled from one
 pinned staging copy per replay.
+
+Models in the segment layout that declare ``segment_graphs`` replay one graph
+per (rows, block-table width): see :meth:`GraphRunnerMixin._seg_graph_step`.
 """
 from __future__ import annotations
 
@@ -23,11 +26,30 @@ from ..knobs import KNOBS
 from ..ops import attention as A
 from ..ops import sampling as SMP
 from ..ops._lib import scratch
+from ..ops.seq_ops import SegMeta, SegStepInputs
 from ..utils import tracing
 from .structured import GrammarState
 from .types import PART_MIN, SPEC, InFlight, Request, Sequence, _LazySample, _spec_tok
 
 log = logging.getLogger("k8s_llm_rca_amd.engine.engine")
+
+
+# Steps of a shape that run eagerly before it is captured (they also leave nothing to be set up inside the capture).  A
+# capture costs 2 to 4 ms, a replay saves 0.4 to 0.5 ms of a step (fikerax-1b, 1 / 7 / 64 rows: 1.14 / 1.20 / 1.85 ms of
+# which the host's launches take most -> 0.71 / 0.88 / 1.38; lizesun-1b, 8 layers: 1.17 / 1.27 / 1.66 -> 0.77 / 0.87 / 1.10),
+# so a shape that came three times is taken to come ten times more.
+SEG_GRAPH_AFTER = 3
+SEG_GRAPHS = 32         # graphs an engine keeps (least recently replayed ones go)
+
+
+class _DecodeSegments(SegMeta):
+    """The segments of a step of single tokens whose work items lie in a captured graph's static input."""
+
+    def attn_items(self, tokens_per_item: int) -> tuple:
+        return self.items, self.items[:0], self.pos0_host[0] + 1
+
+    def tile_items(self, tokens_per_item: int) -> torch.Tensor:
+        return self.items
 
 
 class GraphRunnerMixin:
@@ -228,3 +250,93 @@ class GraphRunnerMixin:
         if n_sel:
             return out.index_select(0, dev_flat[o_sel:o_sel + n_sel].long())
         return out[:B]
+
+    # ------------------------------------------- HIP graphs of the segment layout
+    def _seg_graph_step(self, decode: List[Tuple[Sequence, int]], sample_idx: List[int]) -> Optional[torch.Tensor]:
+        """A step of one token each for ``decode``'s sequences as a graph replay; None: the step runs eagerly (several rows
+        of one sequence, too many rows, or a shape that has not come often enough).  A graph fixes the number of rows
+        and how many cache pages the attention's grids are laid out for (the width of the block tables: a power of two up to
+        8 pages, then in steps of 8, past 128 of 32); everything else a step's kernels need -- tokens, positions, cache and state slots,
+        pages, work items -- is read from one static buffer that each step fills with one copy.  The logits are copied
+        out: what a step returns stays the caller's."""
+        B, BS = len(decode), self.kv.block_size
+        if B > max(self.cfg.graph_batch_sizes) or len(set(id(s) for s, _ in decode)) != B:
+            return None
+        pages = max(s.n_cached + j for s, j in decode) // BS + 1
+        width = 1 << (pages - 1).bit_length() if pages <= 8 else -(-pages // 8) * 8 if pages <= 128 else -(-pages // 32) * 32
+        key = (B, width)
+        got = self._seg_graphs.pop(key, None)
+        if got is None:
+            if len(self._seg_seen) > 4096:
+                self._seg_seen.clear()
+            n = self._seg_seen[key] = self._seg_seen.get(key, 0) + 1
+            if n <= SEG_GRAPH_AFTER:
+                return None
+        flat = np.zeros(8 * B + B * width, dtype=np.int32)
+        ids, pos, slots, slot = flat[:4 * B].reshape(4, B)
+        items, bt = flat[4 * B:8 * B].reshape(B, 4), flat[8 * B:].reshape(B, width)
+        for i, (s, j) in enumerate(decode):
+            p = s.n_cached + j
+            n = p // BS + 1
+            ids[i], pos[i], slots[i] = s.tokens[p], p, s.blocks[n - 1] * BS + p % BS
+            if self.states is not None:
+                if s.slot is None:
+                    raise RuntimeError(f"sequence {s.id} runs without a state slot")
+                slot[i] = s.slot
+            items[i] = i, i, 1, p
+            bt[i, :n] = s.blocks[:n]
+        host = torch.from_numpy(flat).pin_memory()
+        if got is None:
+            got = self._seg_capture(B, width, host)
+        else:
+            got[1].copy_(host, non_blocking=True)
+        self._trace_mark()
+        self._seg_graphs[key] = got            # now the most recently replayed one
+        graph, _, out, _ = got
+        graph.replay()
+        if sample_idx == list(range(B)):
+            return out.clone()
+        return out.index_select(0, torch.tensor(sample_idx, dtype=torch.long).pin_memory().to(self.device,
+                                                                                              non_blocking=True))
+
+    def _seg_capture(self, B: int, width: int, host: torch.Tensor) -> tuple:
+        """(graph, its static input holding ``host``, its logits [B, vocab], its step) of a step of ``B`` single tokens.  The
+        step is kept with the graph: every tensor in it is read by each replay, the row offsets too, which no copy fills."""
+        t0 = time.perf_counter()
+        cur = torch.cuda.current_stream(self.device)
+        while len(self._seg_graphs) >= SEG_GRAPHS:
+            cur.synchronize()                  # its last replay may still run
+            self._seg_graphs.pop(next(iter(self._seg_graphs)))
+        flat = host.to(self.device, non_blocking=True)
+        ids, pos, slots, slot = flat[:4 * B].view(4, B).unbind(0)
+        rows = torch.arange(B + 1, dtype=torch.int32, device=self.device)
+        seg = _DecodeSegments(n_seg=B, row_seg=rows[:B], seg_row0=rows, seg_pos0=pos, seg_slot=slot,
+                              block_tables=flat[8 * B:].view(B, width), row0_host=list(range(B + 1)),
+                              pos0_host=[width * self.kv.block_size - 1] * B, slot_host=[0] * B, n_single=B)
+        seg.items = flat[4 * B:8 * B].view(B, 4)
+        inp = SegStepInputs(ids, pos, slots, seg, torch.arange(B, device=self.device))
+        states = self.states.t if self.states is not None else {}
+        if self._graph_pool is None:
+            self._graph_pool = torch.cuda.graph_pool_handle()
+        if self._seg_stream is None:
+            self._seg_stream = torch.cuda.Stream(self.device)
+        graph = torch.cuda.CUDAGraph()
+        # (not torch.cuda.graph: it gives the allocator's free blocks back to the device, which the next prompt then
+        # has to take anew; no cyclic collection while the stream captures, as in _capture)
+        gc_was_on = gc.isenabled()
+        gc.disable()
+        self._seg_stream.wait_stream(cur)
+        try:
+            with torch.cuda.stream(self._seg_stream):
+                graph.capture_begin(pool=self._graph_pool, capture_error_mode="thread_local")
+                try:
+                    out = self.model.forward(inp, *self.kv.tensors(), states)
+                finally:
+                    graph.capture_end()
+        finally:
+            if gc_was_on:
+                gc.enable()
+        cur.wait_stream(self._seg_stream)
+        self.stats["captures"] += 1
+        self.stats["capture_s"] += time.perf_counter() - t0
+        return graph, flat, out, inp

@@ -127,10 +127,17 @@ class StepExecMixin:
             self.stats["decode_steps"] += 1
             kind = "graph"
         else:
-            out = self._forward_eager(decode, chunks, sample_idx, spec)
+            out = None
+            if (not chunks and decode and spec is None and self.cfg.use_graphs and self.device.type == "cuda"
+                    and getattr(self.model, "segment_graphs", False)):
+                out = self._seg_graph_step(decode, sample_idx)
+            kind = "eager" if out is None else "graph"
+            if out is None:
+                out = self._forward_eager(decode, chunks, sample_idx, spec)
+            else:
+                self.stats["graph_steps"] += 1
             if not chunks:
                 self.stats["decode_steps"] += 1
-            kind = "eager"
         t1 = time.perf_counter()
         dt = t1 - t0
         self.stats["forward_s"] += dt

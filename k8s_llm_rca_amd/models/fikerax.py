@@ -204,6 +204,7 @@ PRESETS: Dict[str, FikeraxConfig] = {
 class FikeraxModel:
     step_layout = "segments"   # the engine packs steps as segments (ops.seq_ops.SegStepInputs)
     graph_capturable = False
+    segment_graphs = True      # steps of single tokens replay HIP graphs (engine/graph_runner.py)
 
     def __init__(self, cfg: FikeraxConfig, device, dtype=torch.bfloat16, pc: Optional[ParallelContext] = None,
                  seed: int = 0, init: bool = True):

@@ -1,0 +1,80 @@
+"""Steps of single tokens of the segment-layout models as graph replays: every replay against the eager step, with prompts,
+other batches and eager work between, over block-table widths, slots and pages that change hands, and bounded in number."""
+import pytest
+import torch
+
+from k8s_llm_rca_amd.engine import graph_runner as G
+from k8s_llm_rca_amd.engine.engine import EngineConfig, LLMEngine
+
+pytestmark = pytest.mark.gpu
+
+
+def engine(model, dtype, graphs):
+    return LLMEngine(EngineConfig(model=model, device="cuda", dtype=dtype, num_blocks=96, block_size=64, max_context=2048,
+                                  state_slots=6, use_graphs=graphs, prefix_sharing=False, max_decode_seqs=64,
+                                  temperature=0.0, seed=3))
+
+
+def schedule(eng):
+    """Logits of a schedule of prompts and single tokens: batches of 3, 2 and 1 that come back after one another, a sequence
+    that grows over block-table widths of 1, 2 and 4 pages, releases in between, wanted rows left out and reordered."""
+    g = torch.Generator().manual_seed(1)
+
+    def toks(n):
+        return torch.randint(0, eng.mc.vocab_size, (n,), generator=g).tolist()
+    out, a, b, c = [], eng.new_sequence(), eng.new_sequence(), eng.new_sequence()
+    out.append(eng.feed([(a, toks(50), [49]), (b, toks(3), [0, 2]), (c, toks(100), [])]))
+    for i in range(12):
+        out.append(eng.feed([(a, toks(1), [0]), (b, toks(1), [0]), (c, toks(1), [0])]))
+        if i % 3 == 2:
+            torch.randn(512, 512, device="cuda").mm(torch.randn(512, 512, device="cuda")).sum().item()
+    for _ in range(6):
+        out.append(eng.feed([(c, toks(1), [0]), (a, toks(1), [])]))
+    eng.release_sequence(b)
+    d = eng.new_sequence()
+    out.append(eng.feed([(d, toks(30), [29]), (a, toks(1), [0])]))
+    for _ in range(8):
+        out.append(eng.feed([(d, toks(1), [0]), (c, toks(1), [0]), (a, toks(1), [0])]))
+    for _ in range(70):
+        out.append(eng.feed([(a, toks(1), [0])]))
+    out.append(eng.feed([(a, toks(90), [89])]))
+    for _ in range(6):
+        out.append(eng.feed([(a, toks(1), [0])]))
+    return out
+
+
+@pytest.mark.parametrize("model", ["tiny-fikerax", "tiny-lizesun"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_replays_equal_eager_steps(model, dtype, monkeypatch):
+    want = schedule(engine(model, dtype, False))
+    eng = engine(model, dtype, True)
+    got = schedule(eng)
+    torch.cuda.synchronize()
+    assert eng.stats["graph_steps"] > 60 and eng.stats["captures"] >= 4
+    for w, x in zip(want, got):       # (all kept until here: what a step returned is not the next one's buffer)
+        assert w.shape == x.shape and torch.equal(w, x)
+    # the same schedule again on graphs and slots that exist, then with room for two graphs only
+    before = eng.stats["captures"]
+    for sid in list(eng.seqs):
+        eng.release_sequence(sid)
+    assert all(torch.equal(w, x) for w, x in zip(want, schedule(eng)))
+    assert eng.stats["captures"] == before
+    monkeypatch.setattr(G, "SEG_GRAPHS", 2)
+    for sid in list(eng.seqs):
+        eng.release_sequence(sid)
+    assert all(torch.equal(w, x) for w, x in zip(want, schedule(eng)))
+
+
+@pytest.mark.parametrize("model", ["tiny-fikerax", "tiny-lizesun"])
+def test_generation_with_and_without_graphs(model):
+    texts = []
+    for graphs in (False, True):
+        eng = engine(model, torch.float32, graphs)
+        done = {}
+        for i, n in enumerate((5, 70, 12)):
+            prompt = torch.randint(0, eng.mc.vocab_size, (n,), generator=torch.Generator().manual_seed(n)).tolist()
+            eng.submit(eng.new_sequence(), prompt, max_new=20 + i, on_done=lambda gen, st, i=i: done.__setitem__(i, list(gen)))
+        eng.run_until_idle()
+        texts.append(done)
+        assert (eng.stats["graph_steps"] > 0) == graphs
+    assert texts[0] == texts[1] and len(texts[0]) == 3
