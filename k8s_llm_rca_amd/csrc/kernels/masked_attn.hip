@@ -180,20 +180,31 @@ __device__ __forceinline__ void sta4<uint16_t>(uint16_t* p, size_t i, const f32x
 }
 
 // The value columns of TR rows from r0 (nr of them exist) to their pages: row-major, and a column of TR rows whose slots
-// are TR aligned neighbours of one page to the transposed page in one store.
-template <typename TA, int TR>
+// are TR aligned neighbours of one page to the transposed page in one store.  MIX: kept as projected (v_keep) and mixed
+// with another layer's (v_other) on the way, where these are given.
+template <typename TA, int TR, bool MIX>
 __device__ __forceinline__ void write_values(const float* __restrict__ x, int qs, int r0, int nr, int NV, int v_col,
                                              const float* __restrict__ bias, const int* __restrict__ slots,
-                                             TA* __restrict__ vc, TA* __restrict__ vt, int BS, int tid) {
+                                             TA* __restrict__ vc, TA* __restrict__ vt, int BS, int tid, int threads,
+                                             float lam, const float* __restrict__ v_other, float* __restrict__ v_keep) {
   if (NV == 0) return;
   const int s0 = slots[r0];
   bool run = TR > 1 && nr == TR && s0 >= 0 && s0 % TR == 0 && BS % TR == 0;    // then a page holds all TR
   for (int k = 1; k < nr; ++k) run = run && slots[r0 + k] == s0 + k;
-  for (int c = tid; c < NV; c += 256) {
+  for (int c = tid; c < NV; c += threads) {
     const float vb = bias ? bias[v_col + c] : 0.f;
     float v[TR];
 #pragma unroll
     for (int k = 0; k < TR; ++k) v[k] = k < nr ? x[(size_t)(r0 + k) * qs + v_col + c] + vb : 0.f;
+    if (MIX) {
+#pragma unroll
+      for (int k = 0; k < TR; ++k)
+        if (k < nr) {
+          const size_t o = (size_t)(r0 + k) * NV + c;
+          if (v_keep) v_keep[o] = v[k];
+          if (v_other) v[k] = (1.f - lam) * v[k] + lam * v_other[o];
+        }
+    }
     if (vt && run) {
       const int page = s0 / BS;
       TA* o = vt + ((size_t)page * NV + c) * BS + (s0 - page * BS);
@@ -247,24 +258,29 @@ __global__ void __launch_bounds__(256) attn_prep_pairs_kernel(const float* __res
       if (sl >= 0) sta4(kc, (size_t)sl * NK + (c - NQ), v);
     }
   }
-  write_values<TA, TR>(x, qs, r0, nr, NV, v_col, nullptr, slots, vc, vt, BS, tid);
+  write_values<TA, TR, false>(x, qs, r0, nr, NV, v_col, nullptr, slots, vc, vt, BS, tid, 256, 0.f, nullptr, nullptr);
 }
 
 // The preparation with rotation halves (i with i + rot / 2), biases and a norm per head behind the rotation, cos | sin from
 // the table:  D / 8 neighbouring lanes (a power of two) hold a head, each two groups of four entries -- rotated ones and
 // their partners, or eight neighbours behind the rotated part -- so the rotation needs no exchange, the norm a few
-// cross-lane sums, and every access is 16 bytes.
-template <typename TA, int TR>
-__global__ void __launch_bounds__(256) attn_prep_half_kernel(const float* __restrict__ x, int qs, int H, int G, int NV, int D,
+// cross-lane sums, and every access is 16 bytes.  16 heads of 128 over 2 with values mixed across layers, 16384 rows: 226 us
+// (attn_prep_kernel: a row's heads through LDS, a double-precision angle per pair where they are rotated) -> 134 us, one
+// row 15 -> 4.9 us.  TR = 1 (few rows): threads of their own for the values, so that a row is one pass of loads.
+template <typename TA, int TR, bool MIX>
+__global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(const float* __restrict__ x, int qs, int H, int G, int NV, int D,
                                                              int v_col, const float* __restrict__ bias,
                                                              const int* __restrict__ slots, TA* __restrict__ kc,
                                                              TA* __restrict__ vc, TA* __restrict__ vt, int BS,
                                                              TA* __restrict__ q_out, int rot, const float* __restrict__ cs,
                                                              int norm, const float* __restrict__ q_w,
-                                                             const float* __restrict__ k_w, float eps, int T) {
+                                                             const float* __restrict__ k_w, float eps, int T, float lam,
+                                                             const float* __restrict__ v_other,
+                                                             float* __restrict__ v_keep) {
   const int r0 = blockIdx.x * TR, tid = threadIdx.x, half = rot >> 1, lph = D >> 3, units = H + G;
   const int nr = min(TR, T - r0), n = units * lph;
-  for (int i = tid; i < nr * n; i += 256) {
+  const int heads = TR == 1 ? min((int)blockDim.x - 64, (n + 63) & ~63) : 256;      // threads of the heads
+  for (int i = tid; i < nr * n && tid < heads; i += heads) {
     const int rr = i / n, u = (i - rr * n) / lph, j = i & (lph - 1), r = r0 + rr;
     const bool turn = 8 * j < rot;
     const int a = turn ? 4 * j : 8 * j, b = turn ? a + half : a + 4;
@@ -314,7 +330,11 @@ __global__ void __launch_bounds__(256) attn_prep_half_kernel(const float* __rest
       }
     }
   }
-  write_values<TA, TR>(x, qs, r0, nr, NV, v_col, bias, slots, vc, vt, BS, tid);
+  if (TR > 1)
+    write_values<TA, TR, MIX>(x, qs, r0, nr, NV, v_col, bias, slots, vc, vt, BS, tid, 256, lam, v_other, v_keep);
+  else if (tid >= heads)
+    write_values<TA, TR, MIX>(x, qs, r0, nr, NV, v_col, bias, slots, vc, vt, BS, tid - heads, blockDim.x - heads, lam,
+                              v_other, v_keep);
 }
 
 
@@ -709,22 +729,32 @@ K8S_API int k8s_attn_prep_pairs(const float* x, int qs, int H, int G, int D, int
 K8S_API int k8s_attn_prep_half(const float* x, int qs, int H, int G, int D, int NV, int v_col, const float* bias,
                                const int* slots, void* kc, void* vc, void* vt, int BS, void* q_out, int dt, int rot,
                                const float* cs, int norm, const float* q_w, const float* k_w, float eps, int T,
-                               hipStream_t s) {
+                               hipStream_t s, float lam, const float* v_other, float* v_keep) {
   if (T <= 0) return 0;
   if (H < 1 || G < 0 || D < 8 || D > 512 || (D & (D - 1)) || qs % 4 || rot < 0 || rot > D || rot % 8 || (rot && !cs) ||
       NV < 0 || v_col < 0 || BS < 1 || (G > 0 && !kc) || (NV > 0 && !vc && !vt) || norm < 0 || norm > 1 ||
       ((uintptr_t)x & 15) || ((uintptr_t)cs & 15))
     return (int)hipErrorInvalidValue;
-#define K8S_PH(TA, TR)                                                                                                   \
-  hipLaunchKernelGGL((attn_prep_half_kernel<TA, TR>), dim3((T + TR - 1) / TR), dim3(256), 0, s, x, qs, H, G, NV, D, v_col, \
-                     bias, slots, (TA*)kc, (TA*)vc, (TA*)vt, BS, (TA*)q_out, rot, cs, norm, q_w, k_w, eps, T)
-  if (dt == 0) {
-    if (T > 1024) K8S_PH(uint16_t, 8);
-    else K8S_PH(uint16_t, 1);
-  } else {
-    if (T > 1024) K8S_PH(float, 8);
-    else K8S_PH(float, 1);
+  const int one = (H + G) * (D / 8), want = (one + 63) / 64 * 64 + (NV + 63) / 64 * 64;     // threads of a row's one pass
+  const int row_threads = want < 128 ? 128 : (want > 1024 ? 1024 : want);
+#define K8S_PH(TA, TR, MIX)                                                                                             \
+  hipLaunchKernelGGL((attn_prep_half_kernel<TA, TR, MIX>), dim3((T + TR - 1) / TR), dim3(TR == 1 ? row_threads : 256), 0, s, x, qs, H, G, NV, D, \
+                     v_col, bias, slots, (TA*)kc, (TA*)vc, (TA*)vt, BS, (TA*)q_out, rot, cs, norm, q_w, k_w, eps, T, lam, \
+                     v_other, v_keep)
+#define K8S_PH_T(TA)                                   \
+  if (v_other || v_keep) {                             \
+    if (T > 1024) K8S_PH(TA, 8, true);                 \
+    else K8S_PH(TA, 1, true);                          \
+  } else {                                             \
+    if (T > 1024) K8S_PH(TA, 8, false);                \
+    else K8S_PH(TA, 1, false);                         \
   }
+  if (dt == 0) {
+    K8S_PH_T(uint16_t)
+  } else {
+    K8S_PH_T(float)
+  }
+#undef K8S_PH_T
 #undef K8S_PH
   return (int)hipGetLastError();
 }

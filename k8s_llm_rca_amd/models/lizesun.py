@@ -224,6 +224,7 @@ class LizesunModel:
         self.delta_of: List[Optional[int]] = []
         self.mem_of: List[Optional[int]] = []
         self.vmix_first: Optional[int] = None                     # the first layer that mixes values
+        self.ropes: Dict[Tuple[int, float], S.Rope] = {}          # every distinct rotation of the stack
         n_delta = n_mem = 0
         vmix_width = None
         for i, L in enumerate(cfg.layers):
@@ -243,6 +244,9 @@ class LizesunModel:
             if L.kind == "parallel":
                 if L.left.rot_dims % 2 or L.left.rot_dims > L.left.dim:
                     raise ValueError(f"layer {i}: an even rot.dims <= dim")
+                key = (L.left.rot_dims, L.left.rot_base)
+                if key[0] and key not in self.ropes:
+                    self.ropes[key] = S.make_rope(*key, self.device)
                 self.mem_of.append(n_mem)
                 n_mem += 1
             else:
@@ -396,15 +400,19 @@ class LizesunModel:
                                gate=x[:, H * D + G * (D + V):], vt=vts[ci])
         return self._lin32(o, L["wo"])
 
-    def _parallel(self, li: int, h, inp: S.SegStepInputs, kcs, vcs, vts, states):
+    def _parallel(self, li: int, h, inp: S.SegStepInputs, kcs, vcs, vts, states, tables: dict):
         L, spec = self.layers[li], self.cfg.layers[li]
         a, b = spec.left, spec.right
         ci, j = self.cache_of[li], self.mem_of[li]
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
         nl = H * D + G * (D + V)
         x = self._lin32(h, L["w_in"])                                  # left q | k | v, right q | k | v | g | i | f
+        key = (a.rot_dims, a.rot_base)
+        rope = self.ropes.get(key)
+        if rope is not None and key not in tables:                     # cos | sin of the step's positions, made once
+            tables[key] = S.rope_table(inp.positions, rope)
         q = S.attn_prep(x[:, :nl], None, H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], self.dtype, norm=True,
-                        eps=self.cfg.norm_eps, rot_dims=a.rot_dims, rot_base=a.rot_base, vt=vts[ci])
+                        eps=self.cfg.norm_eps, rope=rope, rope_cs=tables.get(key), vt=vts[ci])
         ol = S.masked_attention(q, H, G, D, V, kcs[ci], vcs[ci], inp.seg, a.scale, window=a.window,
                                 keep_first=a.keep_first, sink=L["sink"], vt=vts[ci])
         xr = x[:, nl:]
@@ -440,6 +448,7 @@ class LizesunModel:
         first = self.layers[0]["norm1"] if nl else (1.0, None, None)
         h = N.embed_scale_dyt(inp.input_ids, self.embed, cfg.embed_scale, x, *first, out_dtype=dt)
         vmix: dict = {}
+        tables: dict = {}
         for li, (spec, L) in enumerate(zip(cfg.layers, self.layers)):
             nxt = self.layers[li + 1]["norm1"] if li + 1 < nl else (1.0, None, None)   # the final norm: wanted rows only
             after = L["norm2"] if spec.ff else nxt
@@ -447,7 +456,7 @@ class LizesunModel:
                 h = N.add_dyt(x, self._chunk_attention(li, h, inp, kcs, vcs, vts, vmix), 1.0, None, 1.0, *after,
                               out_dtype=dt)
             elif spec.kind == "parallel":
-                yl, yr = self._parallel(li, h, inp, kcs, vcs, vts, states)
+                yl, yr = self._parallel(li, h, inp, kcs, vcs, vts, states, tables)
                 h = N.add_dyt(x, yl, spec.left_scale, yr, spec.right_scale, *after, out_dtype=dt)
             else:
                 h = N.add_dyt(x, self._delta(li, h, inp, states), 1.0, None, 1.0, *after, out_dtype=dt)

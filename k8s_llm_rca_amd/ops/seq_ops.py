@@ -911,13 +911,14 @@ def attn_prep(qkv: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D
                                             ptr(vt), BS, ptr(q_out), _dt(out_dtype), int(rot_dims), ptr(rope_cs), T,
                                             stream_ptr(qkv)), "attn_prep_pairs")
             return q_out
-        if (mode < 2 and v_other is None and v_keep is None and not tq_every and 8 <= D <= 512 and D & (D - 1) == 0
+        if (mode < 2 and not tq_every and 8 <= D <= 512 and D & (D - 1) == 0
                 and qkv.stride(0) % 4 == 0 and qkv.data_ptr() % 16 == 0 and rot_dims % 8 == 0
                 and (rot_dims == 0 or (rope is not None and not rope.pairs and rope_cs is not None))):
             # a head's entries meet in its rotation and its norm alone: a few lanes per head, no LDS
             check(lib().k8s_attn_prep_half(ptr(qkv), qkv.stride(0), HQ, GK, D, NV, v_col, ptr(bias), ptr(slots), ptr(kc),
                                            ptr(vc), ptr(vt), BS, ptr(q_out), _dt(out_dtype), int(rot_dims), ptr(rope_cs),
-                                           mode, ptr(q_w), ptr(k_w), float(eps), T, stream_ptr(qkv)), "attn_prep_half")
+                                           mode, ptr(q_w), ptr(k_w), float(eps), T, stream_ptr(qkv), float(lam),
+                                           ptr(v_other), ptr(v_keep)), "attn_prep_half")
             return q_out
         check(lib().k8s_attn_prep(ptr(qkv), qkv.stride(0), ptr(bias), HQ, GK, D, NV, ptr(positions), ptr(slots),
                                   ptr(kc), ptr(vc), ptr(vt), BS, ptr(q_out), _dt(out_dtype), mode, ptr(q_w),

@@ -1,0 +1,48 @@
+"""The q / k / v preparation without LDS over the forms it takes, device against CPU: kept and mixed values beside rotation
+halves, biases and head norms, values that are the keys, rows with and without a slot, one row and many."""
+import pytest
+import torch
+
+from k8s_llm_rca_amd.ops import seq_ops as S
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T", [1, 5, 1031])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,D,V,rot,v_is_k", [(16, 2, 128, 128, 0, False), (3, 1, 32, 20, 16, False),
+                                                (4, 4, 16, 16, 16, True), (40, 8, 64, 64, 24, False)])
+@pytest.mark.parametrize("keep,other", [(True, False), (False, True), (True, True), (False, False)])
+def test_forms(T, dt, H, G, D, V, rot, v_is_k, keep, other):
+    BS, pages = 32, 40
+    g = torch.Generator().manual_seed(T + D)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g)
+    NK, NV = G * D, G * V
+    width = H * D + NK + (0 if v_is_k else NV)
+    x = rnd(T, width + 4)
+    slots = torch.randperm(pages * BS, generator=g)[:T].to(torch.int32)
+    if T > 1000:
+        slots[:512] = torch.arange(512, dtype=torch.int32) + 64       # runs of aligned neighbours among scattered ones
+        slots[512:] = torch.arange(T - 512, dtype=torch.int32) + 64 + 512
+    slots[T // 2] = -1
+    pos = torch.randint(0, 5000, (T,), generator=g).to(torch.int32)
+    bias, q_w, k_w, v_other = rnd(width), rnd(D), rnd(D), rnd(T, NV)
+    got = {}
+    for dev in ("cpu", "cuda"):
+        kc, vc, vt = (torch.zeros(pages, BS, NK, dtype=dt), torch.zeros(pages, BS, NV, dtype=dt),
+                      torch.zeros(pages, NV, BS, dtype=dt))
+        kc, vc, vt = kc.to(dev), vc.to(dev), vt.to(dev)
+        kept = torch.zeros(T, NV, device=dev) if keep else None
+        rope = S.make_rope(rot, 10000.0, dev) if rot else None
+        p = pos.to(dev)
+        q = S.attn_prep(x.to(dev)[:, :width], bias.to(dev), H, G, D, V, p, slots.to(dev), kc, vc, dt, norm=True,
+                        q_w=q_w.to(dev), k_w=k_w.to(dev), eps=1e-5, lam=0.3, v_other=v_other.to(dev) if other else None,
+                        v_keep=kept, vt=vt, v_is_k=v_is_k, rope=rope, rope_cs=S.rope_table(p, rope) if rot else None)
+        got[dev] = [t.float().cpu() for t in (q, kc, vc, vt) + ((kept,) if keep else ())]
+    for a, b in zip(got["cuda"], got["cpu"]):
+        # fp32: sums of D squares in another order, a few roundings; bf16: at most one step of its last place, 2^-7 of the
+        # power of two below the value
+        tol = 2e-5 if dt == torch.float32 else 2.0 ** -7
+        assert float(((a - b).abs() / b.abs().clamp_min(1.0)).max()) <= tol
