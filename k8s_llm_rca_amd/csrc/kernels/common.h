@@ -97,6 +97,35 @@ __device__ __forceinline__ void sum_splits8(const float* p, size_t stride, int s
   }
 }
 
+// Four neighbouring entries of a sum of n planes (split-K partials, `step` apart), in plane order p0 + p1 + ...  Two, four and
+// eight planes are loaded before the first addition.
+template <int N>
+__device__ __forceinline__ f32x4 sum_planes4_n(const float* p, size_t step) {
+  f32x4 v[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = *reinterpret_cast<const f32x4*>(p + k * step);
+#pragma unroll
+  for (int k = 1; k < N; ++k) v[0] += v[k];
+  return v[0];
+}
+__device__ __forceinline__ f32x4 sum_planes4(const float* p, size_t step, int n) {
+  switch (n) {
+    case 1: return *reinterpret_cast<const f32x4*>(p);
+    case 2: return sum_planes4_n<2>(p, step);
+    case 4: return sum_planes4_n<4>(p, step);
+    case 8: return sum_planes4_n<8>(p, step);
+  }
+  f32x4 v = *reinterpret_cast<const f32x4*>(p);
+  for (int k = 1; k < n; ++k) v += *reinterpret_cast<const f32x4*>(p + k * step);
+  return v;
+}
+__device__ __forceinline__ float sum_planes(const float* p, size_t step, int n) {
+  float v = p[0];
+#pragma unroll 8
+  for (int k = 1; k < n; ++k) v += p[k * step];
+  return v;
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

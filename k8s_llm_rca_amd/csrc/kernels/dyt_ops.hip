@@ -33,22 +33,23 @@ __device__ __forceinline__ void st4<uint16_t>(uint16_t* p, size_t i, const float
   *reinterpret_cast<u16x4*>(p + i) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
 }
 
-// x += sy * y + sy2 * y2 (y, y2 optional);  out = tanh(alpha x) w + b (w optional).  n4 = T * W / 4.
+// x += sy * y + sy2 * y2 (y, y2 optional, each the sum of yp / yp2 planes);  out = tanh(alpha x) w + b (w optional).
+// n4 = T * W / 4.
 template <typename TA>
 __global__ void __launch_bounds__(256) add_dyt4_kernel(float* __restrict__ x, const float* __restrict__ y, float sy,
                                                        const float* __restrict__ y2, float sy2, float alpha,
                                                        const float* __restrict__ w, const float* __restrict__ b,
-                                                       TA* __restrict__ out, size_t n4, int W) {
+                                                       TA* __restrict__ out, size_t n4, int W, int yp, int yp2) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
     const size_t e = i * 4;
     const int c = (int)(e % (size_t)W);
     f32x4 xv = *reinterpret_cast<const f32x4*>(x + e);
     if (y) {
-      const f32x4 yv = *reinterpret_cast<const f32x4*>(y + e);
+      const f32x4 yv = sum_planes4(y + e, n4 * 4, yp);
 #pragma unroll
       for (int k = 0; k < 4; ++k) xv[k] = fmaf(sy, yv[k], xv[k]);
       if (y2) {
-        const f32x4 zv = *reinterpret_cast<const f32x4*>(y2 + e);
+        const f32x4 zv = sum_planes4(y2 + e, n4 * 4, yp2);
 #pragma unroll
         for (int k = 0; k < 4; ++k) xv[k] = fmaf(sy2, zv[k], xv[k]);
       }
@@ -68,13 +69,13 @@ template <typename TA>
 __global__ void __launch_bounds__(256) add_dyt1_kernel(float* __restrict__ x, const float* __restrict__ y, float sy,
                                                        const float* __restrict__ y2, float sy2, float alpha,
                                                        const float* __restrict__ w, const float* __restrict__ b,
-                                                       TA* __restrict__ out, size_t n, int W) {
+                                                       TA* __restrict__ out, size_t n, int W, int yp, int yp2) {
   for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) {
     const int c = (int)(e % (size_t)W);
     float xv = x[e];
     if (y) {
-      xv = fmaf(sy, y[e], xv);
-      if (y2) xv = fmaf(sy2, y2[e], xv);
+      xv = fmaf(sy, sum_planes(y + e, n, yp), xv);
+      if (y2) xv = fmaf(sy2, sum_planes(y2 + e, n, yp2), xv);
       x[e] = xv;
     }
     if (w) std_(out, e, fmaf(tanhf(alpha * xv), w[c], b[c]));
@@ -134,24 +135,24 @@ static int grid_for(size_t items) {
 using namespace k8s;
 
 K8S_API int k8s_add_dyt(float* x, const float* y, float sy, const float* y2, float sy2, float alpha, const float* w,
-                        const float* b, void* out, int odt, int T, int W, hipStream_t s) {
+                        const float* b, void* out, int odt, int T, int W, hipStream_t s, int yp, int yp2) {
   if (T <= 0 || W <= 0) return 0;
-  if ((w == nullptr) != (out == nullptr) || (w && !b) || (y2 && !y)) return (int)hipErrorInvalidValue;
+  if ((w == nullptr) != (out == nullptr) || (w && !b) || (y2 && !y) || yp < 1 || yp2 < 1) return (int)hipErrorInvalidValue;
   const size_t n = (size_t)T * W;
   if (W % 4 == 0) {
     if (odt == 0)
       hipLaunchKernelGGL((add_dyt4_kernel<uint16_t>), dim3(grid_for(n / 4)), dim3(256), 0, s, x, y, sy, y2, sy2, alpha, w,
-                         b, (uint16_t*)out, n / 4, W);
+                         b, (uint16_t*)out, n / 4, W, yp, yp2);
     else
       hipLaunchKernelGGL((add_dyt4_kernel<float>), dim3(grid_for(n / 4)), dim3(256), 0, s, x, y, sy, y2, sy2, alpha, w, b,
-                         (float*)out, n / 4, W);
+                         (float*)out, n / 4, W, yp, yp2);
   } else {
     if (odt == 0)
       hipLaunchKernelGGL((add_dyt1_kernel<uint16_t>), dim3(grid_for(n)), dim3(256), 0, s, x, y, sy, y2, sy2, alpha, w, b,
-                         (uint16_t*)out, n, W);
+                         (uint16_t*)out, n, W, yp, yp2);
     else
       hipLaunchKernelGGL((add_dyt1_kernel<float>), dim3(grid_for(n)), dim3(256), 0, s, x, y, sy, y2, sy2, alpha, w, b,
-                         (float*)out, n, W);
+                         (float*)out, n, W, yp, yp2);
   }
   return (int)hipGetLastError();
 }

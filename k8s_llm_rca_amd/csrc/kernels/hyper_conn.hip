@@ -66,7 +66,7 @@ __device__ __forceinline__ void norm_row(const float* u, float ss, float* red, c
 constexpr int kMaxStreams = 16;   // the form for any count: one column per thread, the streams in a local array
 
 // S streams at compile time (S > 0) or S_ <= kMaxStreams of them (S == 0).
-// y: fp32 rows [T][W], or (inv given) rows of yp in expert order weighted by ew [T][K].
+// y: fp32 rows [yp][T][W] whose planes are summed, or (inv given) rows of yp in expert order weighted by ew [T][K].
 // out / mix: this sublayer's; in / nw: the next one's (h null: nothing reads the streams next).
 // eid (optional) [T]: token ids whose rows of emb, times es, are added to every stream.
 template <int S, int VEC, typename TY, typename TA>
@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(1024) hyper_step_kernel(float* __restrict__ x,
                                                          const float* __restrict__ mix, const float* __restrict__ in,
                                                          const float* __restrict__ nw, float eps, TA* __restrict__ h,
                                                          int W, int S_, const int* __restrict__ eid,
-                                                         const TA* __restrict__ emb, float es) {
+                                                         const TA* __restrict__ emb, float es, int yp) {
   extern __shared__ float u[];
   __shared__ float red[16];
   constexpr int SM = S > 0 ? S : kMaxStreams;
@@ -100,8 +100,18 @@ __global__ void __launch_bounds__(1024) hyper_step_kernel(float* __restrict__ x,
 #pragma unroll
         for (int k = 0; k < VEC; ++k) yv[k] = fmaf(wj, ev[k], yv[k]);
       }
+    } else if constexpr (VEC == 4 && sizeof(TY) == 4) {
+      const f32x4 v = sum_planes4((const float*)y + o + c, (size_t)gridDim.x * W, yp);
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) yv[k] = v[k];
     } else {
       ldv<VEC>(y, o + c, yv);
+      for (int p = 1; p < yp; ++p) {
+        float pv[VEC];
+        ldv<VEC>(y, (size_t)p * gridDim.x * W + o + c, pv);
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) yv[k] += pv[k];
+      }
     }
     float uv[VEC], av[VEC];
 #pragma unroll
@@ -210,11 +220,11 @@ static bool hyper_row_ok(int W) { return W > 0 && (size_t)W * sizeof(float) <= 6
 template <int VEC, typename TY, typename TA>
 static void hyper_step_launch(float* x, const void* y, const int* inv, const float* ew, int K, const float* out,
                               const float* mix, const float* in, const float* nw, float eps, void* h, int T, int S,
-                              int W, const int* eid, const void* emb, float es, hipStream_t s) {
+                              int W, const int* eid, const void* emb, float es, int yp, hipStream_t s) {
   const dim3 g(T), b(hyper_threads(T, W, VEC));
 #define K8S_HS(SS)                                                                                              \
   hipLaunchKernelGGL((hyper_step_kernel<SS, VEC, TY, TA>), g, b, W * sizeof(float), s, x, (const TY*)y, inv, ew, K, \
-                     out, mix, in, nw, eps, (TA*)h, W, S, eid, (const TA*)emb, es)
+                     out, mix, in, nw, eps, (TA*)h, W, S, eid, (const TA*)emb, es, yp)
   switch (S) {
     case 1: K8S_HS(1); break;
     case 2: K8S_HS(2); break;
@@ -229,23 +239,23 @@ static void hyper_step_launch(float* x, const void* y, const int* inv, const flo
 
 using namespace k8s;
 
-// ydt / hdt / edt: 0 bf16, 1 fp32.  inv null: y is fp32 [T][W].  emb has the type of h.
+// ydt / hdt / edt: 0 bf16, 1 fp32.  inv null: y is fp32 [yp][T][W].  emb has the type of h.
 K8S_API int k8s_hyper_step(float* x, const void* y, int ydt, const int* inv, const float* ew, int K, const float* out,
                            const float* mix, const float* in, const float* nw, float eps, void* h, int hdt, int T, int S,
-                           int W, hipStream_t s, const int* eid, const void* emb, float es) {
+                           int W, hipStream_t s, const int* eid, const void* emb, float es, int yp) {
   if (T <= 0) return 0;
   if (!hyper_row_ok(W) || S < 1 || S > kMaxStreams || !y || !out || !mix || (h && (!in || !nw)) ||
-      (inv && (!ew || K < 1)) || (!inv && ydt != 1) || (eid && !emb))
+      yp < 1 || (inv && (!ew || K < 1 || yp != 1)) || (!inv && ydt != 1) || (eid && !emb))
     return (int)hipErrorInvalidValue;
 #define K8S_HY(VEC)                                                                                               \
   if (ydt == 0 && hdt == 0)                                                                                       \
-    hyper_step_launch<VEC, uint16_t, uint16_t>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, s);             \
+    hyper_step_launch<VEC, uint16_t, uint16_t>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, s);         \
   else if (ydt == 0)                                                                                              \
-    hyper_step_launch<VEC, uint16_t, float>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, s);                \
+    hyper_step_launch<VEC, uint16_t, float>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, s);            \
   else if (hdt == 0)                                                                                              \
-    hyper_step_launch<VEC, float, uint16_t>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, s);                \
+    hyper_step_launch<VEC, float, uint16_t>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, s);            \
   else                                                                                                            \
-    hyper_step_launch<VEC, float, float>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, s)
+    hyper_step_launch<VEC, float, float>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, s)
   if (W % 4 == 0 && S <= 4) {
     K8S_HY(4);
   } else {

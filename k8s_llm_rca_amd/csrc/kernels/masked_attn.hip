@@ -186,7 +186,8 @@ template <typename TA, int TR, bool MIX>
 __device__ __forceinline__ void write_values(const float* __restrict__ x, int qs, int r0, int nr, int NV, int v_col,
                                              const float* __restrict__ bias, const int* __restrict__ slots,
                                              TA* __restrict__ vc, TA* __restrict__ vt, int BS, int tid, int threads,
-                                             float lam, const float* __restrict__ v_other, float* __restrict__ v_keep) {
+                                             float lam, const float* __restrict__ v_other, float* __restrict__ v_keep,
+                                             int planes = 1, size_t pstep = 0) {
   if (NV == 0) return;
   const int s0 = slots[r0];
   bool run = TR > 1 && nr == TR && s0 >= 0 && s0 % TR == 0 && BS % TR == 0;    // then a page holds all TR
@@ -195,7 +196,7 @@ __device__ __forceinline__ void write_values(const float* __restrict__ x, int qs
     const float vb = bias ? bias[v_col + c] : 0.f;
     float v[TR];
 #pragma unroll
-    for (int k = 0; k < TR; ++k) v[k] = k < nr ? x[(size_t)(r0 + k) * qs + v_col + c] + vb : 0.f;
+    for (int k = 0; k < TR; ++k) v[k] = k < nr ? sum_planes(x + (size_t)(r0 + k) * qs + v_col + c, pstep, TR == 1 ? planes : 1) + vb : 0.f;
     if (MIX) {
 #pragma unroll
       for (int k = 0; k < TR; ++k)
@@ -276,7 +277,7 @@ __global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(co
                                                              int norm, const float* __restrict__ q_w,
                                                              const float* __restrict__ k_w, float eps, int T, float lam,
                                                              const float* __restrict__ v_other,
-                                                             float* __restrict__ v_keep) {
+                                                             float* __restrict__ v_keep, int planes, size_t pstep) {
   const int r0 = blockIdx.x * TR, tid = threadIdx.x, half = rot >> 1, lph = D >> 3, units = H + G;
   const int nr = min(TR, T - r0), n = units * lph;
   const int heads = TR == 1 ? min((int)blockDim.x - 64, (n + 63) & ~63) : 256;      // threads of the heads
@@ -285,7 +286,7 @@ __global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(co
     const bool turn = 8 * j < rot;
     const int a = turn ? 4 * j : 8 * j, b = turn ? a + half : a + 4;
     const float* p = x + (size_t)r * qs + u * D;
-    f32x4 va = *reinterpret_cast<const f32x4*>(p + a), vb = *reinterpret_cast<const f32x4*>(p + b);
+    f32x4 va = sum_planes4(p + a, pstep, TR == 1 ? planes : 1), vb = sum_planes4(p + b, pstep, TR == 1 ? planes : 1);
     if (bias) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
@@ -334,7 +335,7 @@ __global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(co
     write_values<TA, TR, MIX>(x, qs, r0, nr, NV, v_col, bias, slots, vc, vt, BS, tid, 256, lam, v_other, v_keep);
   else if (tid >= heads)
     write_values<TA, TR, MIX>(x, qs, r0, nr, NV, v_col, bias, slots, vc, vt, BS, tid - heads, blockDim.x - heads, lam,
-                              v_other, v_keep);
+                              v_other, v_keep, planes, pstep);
 }
 
 
@@ -725,22 +726,23 @@ K8S_API int k8s_attn_prep_pairs(const float* x, int qs, int H, int G, int D, int
 }
 
 // D 8, 16, .. 512 (powers of two), qs a multiple of 4, rot a multiple of 8 with its table, x / q_out / kc / cs 16-byte
-// aligned (8 for bf16 outputs); norm 0 / 1 as in k8s_attn_prep
+// aligned (8 for bf16 outputs); norm 0 / 1 as in k8s_attn_prep.  planes > 1 (T <= 1024): x is the sum of as many, pstep
+// (a multiple of 4) numbers apart
 K8S_API int k8s_attn_prep_half(const float* x, int qs, int H, int G, int D, int NV, int v_col, const float* bias,
                                const int* slots, void* kc, void* vc, void* vt, int BS, void* q_out, int dt, int rot,
                                const float* cs, int norm, const float* q_w, const float* k_w, float eps, int T,
-                               hipStream_t s, float lam, const float* v_other, float* v_keep) {
+                               hipStream_t s, float lam, const float* v_other, float* v_keep, int planes, long pstep) {
   if (T <= 0) return 0;
   if (H < 1 || G < 0 || D < 8 || D > 512 || (D & (D - 1)) || qs % 4 || rot < 0 || rot > D || rot % 8 || (rot && !cs) ||
       NV < 0 || v_col < 0 || BS < 1 || (G > 0 && !kc) || (NV > 0 && !vc && !vt) || norm < 0 || norm > 1 ||
-      ((uintptr_t)x & 15) || ((uintptr_t)cs & 15))
+      planes < 1 || (planes > 1 && (T > 1024 || pstep % 4)) || ((uintptr_t)x & 15) || ((uintptr_t)cs & 15))
     return (int)hipErrorInvalidValue;
   const int one = (H + G) * (D / 8), want = (one + 63) / 64 * 64 + (NV + 63) / 64 * 64;     // threads of a row's one pass
   const int row_threads = want < 128 ? 128 : (want > 1024 ? 1024 : want);
 #define K8S_PH(TA, TR, MIX)                                                                                             \
   hipLaunchKernelGGL((attn_prep_half_kernel<TA, TR, MIX>), dim3((T + TR - 1) / TR), dim3(TR == 1 ? row_threads : 256), 0, s, x, qs, H, G, NV, D, \
                      v_col, bias, slots, (TA*)kc, (TA*)vc, (TA*)vt, BS, (TA*)q_out, rot, cs, norm, q_w, k_w, eps, T, lam, \
-                     v_other, v_keep)
+                     v_other, v_keep, planes, pstep)
 #define K8S_PH_T(TA)                                   \
   if (v_other || v_keep) {                             \
     if (T > 1024) K8S_PH(TA, 8, true);                 \

@@ -242,36 +242,46 @@ __global__ void __launch_bounds__(256) postnorm_kernel(float* __restrict__ x, co
 // entries 2i, 2i + 1 are turned by the angle whose cosine and sine stand in
 // cs [T][RD] (cos | sin) and go behind the latent in the cache row, padded with
 // zeros to RP numbers (the row is KR + RP wide; the twin holds the latent only).
-template <typename TW, typename TA>
-__global__ void __launch_bounds__(256) latent_norm_kernel(const float* __restrict__ dn, int ld,
+// PLANES: dn is the sum of several planes, pstep apart, formed once in LDS (16-byte loads: ld, pstep and the row's length are
+// multiples of 4).
+template <typename TW, typename TA, bool PLANES>
+__global__ void __launch_bounds__(PLANES ? 512 : 256) latent_norm_kernel(const float* __restrict__ dn, int ld,
                                                           const TW* __restrict__ wq, const TW* __restrict__ wkv,
                                                           const int* __restrict__ slots, TA* __restrict__ cq,
                                                           TA* __restrict__ cache, TA* __restrict__ cache_t, int BS,
                                                           int QR, int KR, float eps, int RD, int RP,
-                                                          const float* __restrict__ cs) {
+                                                          const float* __restrict__ cs, int planes, size_t pstep) {
+  extern __shared__ float lrow[];                            // [QR + KR + RD], several planes only: their sum
+  constexpr int NT = PLANES ? 512 : 256;
   __shared__ float scratch[16];
   const int t = blockIdx.x;
-  const float* row = dn + (size_t)t * ld;
+  const float* mrow = dn + (size_t)t * ld;
+  if (PLANES) {
+    for (int c = 4 * threadIdx.x; c < QR + KR + RD; c += 4 * blockDim.x)
+      *reinterpret_cast<f32x4*>(lrow + c) = sum_planes4(mrow + c, pstep, planes);
+    __syncthreads();
+  }
+  const auto row = [&] { if constexpr (PLANES) return (const float*)lrow; else return mrow; }();
   float ss = 0.f;
-  for (int c = threadIdx.x; c < QR; c += 256) ss = fmaf(row[c], row[c], ss);
+  for (int c = threadIdx.x; c < QR; c += NT) ss = fmaf(row[c], row[c], ss);
   ss = block_sum(ss, scratch);
   float inv = 1.f / sqrtf(ss / (float)QR + eps);
-  for (int c = threadIdx.x; c < QR; c += 256) stf(cq, (size_t)t * QR + c, row[c] * inv * ldf(wq, c));
+  for (int c = threadIdx.x; c < QR; c += NT) stf(cq, (size_t)t * QR + c, row[c] * inv * ldf(wq, c));
   if (KR <= 0) return;
   const int slot = slots[t];
   ss = 0.f;
-  for (int c = threadIdx.x; c < KR; c += 256) ss = fmaf(row[QR + c], row[QR + c], ss);
+  for (int c = threadIdx.x; c < KR; c += NT) ss = fmaf(row[QR + c], row[QR + c], ss);
   ss = block_sum(ss, scratch);
   inv = 1.f / sqrtf(ss / (float)KR + eps);
   if (slot < 0) return;
   const size_t page = slot / BS, off = slot - page * BS;
-  for (int c = threadIdx.x; c < KR; c += 256) {
+  for (int c = threadIdx.x; c < KR; c += NT) {
     const float v = row[QR + c] * inv * ldf(wkv, c);
     stf(cache, (size_t)slot * (KR + RP) + c, v);
     if (cache_t) stf(cache_t, (page * KR + c) * BS + off, v);   // the transposed pages [pages][KR][BS]
   }
   const int half = RD >> 1;
-  for (int i = threadIdx.x; i < RP; i += 256) {
+  for (int i = threadIdx.x; i < RP; i += NT) {
     float v = 0.f;
     if (i < RD) {
       const float* p = row + QR + KR + (i & ~1);
@@ -385,12 +395,20 @@ K8S_API int k8s_postnorm(float* x, const void* y, int y_dt, const void* w, int w
 
 K8S_API int k8s_latent_norm(const float* dn, int ld, const void* wq, const void* wkv, const int* slots, void* cq,
                             void* cache, void* cache_t, int BS, int T, int QR, int KR, float eps, int dt,
-                            hipStream_t s, int RD, int RP, const float* cs) {
+                            hipStream_t s, int RD, int RP, const float* cs, int planes, long pstep) {
   if (T <= 0) return 0;
-  if (RD < 0 || (RD & 1) || RP < RD || (RP & 1) || (RD && (!cs || KR <= 0))) return (int)hipErrorInvalidValue;
-  K8S_DT2(dt, hipLaunchKernelGGL((latent_norm_kernel<TW, TA>), dim3(T), dim3(256), 0, s, dn, ld, (const TW*)wq,
-                                  (const TW*)wkv, slots, (TA*)cq, (TA*)cache, (TA*)cache_t, BS, QR, KR, eps,
-                                  RD, RP, cs));
+  const size_t lds = (size_t)(QR + KR + RD) * sizeof(float);
+  if (planes < 1 || (planes > 1 && (lds > 48 * 1024 || lds % 16 || ld % 4 || pstep % 4 || ((uintptr_t)dn & 15))) || RD < 0 || (RD & 1) || RP < RD || (RP & 1) || (RD && (!cs || KR <= 0))) return (int)hipErrorInvalidValue;
+#define K8S_LN(PL, LDS)                                                                                              \
+  K8S_DT2(dt, hipLaunchKernelGGL((latent_norm_kernel<TW, TA, PL>), dim3(T), dim3(PL ? 512 : 256), LDS, s, dn, ld, (const TW*)wq, \
+                                 (const TW*)wkv, slots, (TA*)cq, (TA*)cache, (TA*)cache_t, BS, QR, KR, eps, RD, RP, cs, \
+                                 planes, (size_t)pstep))
+  if (planes > 1) {
+    K8S_LN(true, lds);
+  } else {
+    K8S_LN(false, 0);
+  }
+#undef K8S_LN
   return (int)hipGetLastError();
 }
 

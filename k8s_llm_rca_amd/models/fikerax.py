@@ -32,7 +32,7 @@ import torch
 from ..ops import moe as M
 from ..ops import norm as N
 from ..ops import seq_ops as S
-from ..ops.linear import linear, proj_f32out, swiglu_gemm
+from ..ops.linear import linear, proj_f32out, proj_planes, swiglu_gemm
 from ..parallel.groups import ParallelContext, single
 
 TAIL_ALIGN = 32     # the rotated key part of a latent cache row is filled up to a multiple of this
@@ -381,21 +381,21 @@ class FikeraxModel:
         x = linear(h, L["w_in"])                                             # q | k | v | gate as activations
         o = S.decay_attention(x, c.heads, c.dim, c.vdim, L["decay"], state, inp.seg, silu=True)
         y = S.head_norm_gate(o, x[:, x.shape[1] - HV:], L["mem_norm"], 1, HV, self.cfg.norm_eps, self.dtype)
-        return proj_f32out(y, L["wo"])
+        return proj_planes(y, L["wo"])
 
     def _attention(self, i: int, h: torch.Tensor, inp: S.SegStepInputs, tables, kc, vc, vt) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
-        x = proj_f32out(h, L["w_in"])
+        x = proj_planes(h, L["w_in"])
         q = S.attn_prep(x, L["b_in"], c.heads, c.kv_heads, c.dim, c.vdim, inp.positions, inp.slots, kc, vc, self.dtype,
                         norm="head", eps=self.cfg.norm_eps, rope=self.ropes[i], rope_cs=self._table(i, inp, tables), vt=vt)
         o = S.masked_attention(q, c.heads, c.kv_heads, c.dim, c.vdim, kc, vc, inp.seg, c.scale, window=c.window, vt=vt)
-        return proj_f32out(o, L["wo"])
+        return proj_planes(o, L["wo"])
 
     def _latent_attention(self, i: int, h: torch.Tensor, inp: S.SegStepInputs, tables, cache, cache_t) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
         T, H, D, R, V, KR = h.shape[0], c.heads, c.dim, c.rot_dim, c.vdim, c.kv_rank
         cs = self._table(i, inp, tables)
-        dn = proj_f32out(h, L["w_in"])                                        # [T, q_rank + KR + R] fp32
+        dn = proj_planes(h, L["w_in"])                                        # [., T, q_rank + KR + R] fp32
         cq = S.latent_norm(dn, L["dq_norm"], L["dkv_norm"], inp.slots, cache, c.q_rank, KR, self.cfg.norm_eps, self.dtype,
                            cache_t=cache_t, tail=R, tail_cs=cs)
         q = linear(cq, L["w_uq"])                                             # [T, H (D + R)]
@@ -409,14 +409,14 @@ class FikeraxModel:
                                    qr=qr.float() if qr is not None else None, **kw)
         ov = torch.empty(T, H, V, dtype=self.dtype, device=h.device)
         torch.bmm(o.transpose(0, 1), L["uv_t"], out=ov.transpose(0, 1))       # written token-major: W_o reads it as it is
-        return proj_f32out(ov.view(T, H * V), L["wo"])
+        return proj_planes(ov.view(T, H * V), L["wo"])
 
     def _dense(self, i: int, h: torch.Tensor) -> torch.Tensor:
         L = self.layers[i]
         a = swiglu_gemm(h, L["w13"])                                          # one launch where a fused kernel takes the shape
         if a is None:
             a = M.glu_clamp(linear(h, L["w13"]), 1.0, math.inf, 0.0)          # silu(gate) * up
-        return proj_f32out(a, L["w2"])
+        return proj_planes(a, L["w2"])
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[Optional[torch.Tensor]],
                 vts: List[Optional[torch.Tensor]], states: Optional[Dict[str, torch.Tensor]] = None,
@@ -448,7 +448,7 @@ class FikeraxModel:
                 h = N.hyper_step(x, y, one, mix1, inn=one, nw=L["norm2"], eps=eps, out_dtype=dt)
                 y = self._dense(i, h)
             if layers_out is not None:
-                layers_out.append(x[:, 0] + y)
+                layers_out.append(x[:, 0] + y.sum(0))
             h = N.hyper_step(x, y, one, mix1, **into)
         return proj_f32out(N.hyper_read(x, inp.logits_idx, self.final_norm, eps, dt), self.head)
 

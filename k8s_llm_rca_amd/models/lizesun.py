@@ -35,7 +35,7 @@ import torch
 
 from ..ops import norm as N
 from ..ops import seq_ops as S
-from ..ops.linear import linear, linear_f32out
+from ..ops.linear import linear, proj_f32out, proj_planes
 from ..parallel.groups import ParallelContext, single
 
 
@@ -374,10 +374,6 @@ class LizesunModel:
         return n + sum(size(t) for t in (self.embed, self.lm_head, self.final_norm))
 
     # -------------------------------------------------------------- forward
-    def _lin32(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-        """x @ w.T with an fp32 result (fp32 accumulation either way)."""
-        return linear_f32out(x, w) if self.dtype == torch.bfloat16 else linear(x, w)
-
     def _act(self, x32: torch.Tensor) -> torch.Tensor:
         """A column slice of an fp32 GEMM result as the next GEMM's operand."""
         return x32.to(self.dtype).contiguous()
@@ -386,7 +382,7 @@ class LizesunModel:
         L, a = self.layers[li], self.cfg.layers[li].attn
         ci = self.cache_of[li]
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
-        x = self._lin32(h, L["w_in"])                                  # [T, H D + G D + G V + H] fp32
+        x = proj_f32out(h, L["w_in"])                                  # [T, H D + G D + G V + H] fp32
         keep = other = None
         if a.v_mix:
             if li == self.vmix_first:
@@ -398,7 +394,7 @@ class LizesunModel:
                         vt=vts[ci])
         o = S.masked_attention(q, H, G, D, V, kcs[ci], vcs[ci], inp.seg, a.scale, softcap=a.softcap, chunk=a.chunk,
                                gate=x[:, H * D + G * (D + V):], vt=vts[ci])
-        return self._lin32(o, L["wo"])
+        return proj_planes(o, L["wo"])
 
     def _parallel(self, li: int, h, inp: S.SegStepInputs, kcs, vcs, vts, states, tables: dict):
         L, spec = self.layers[li], self.cfg.layers[li]
@@ -406,7 +402,7 @@ class LizesunModel:
         ci, j = self.cache_of[li], self.mem_of[li]
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
         nl = H * D + G * (D + V)
-        x = self._lin32(h, L["w_in"])                                  # left q | k | v, right q | k | v | g | i | f
+        x = proj_f32out(h, L["w_in"])                                  # left q | k | v, right q | k | v | g | i | f
         key = (a.rot_dims, a.rot_base)
         rope = self.ropes.get(key)
         if rope is not None and key not in tables:                     # cos | sin of the step's positions, made once
@@ -421,20 +417,20 @@ class LizesunModel:
                                  states[f"memn{j}"], states[f"memm{j}"], inp.seg, defer_scale=True)
         orr = S.head_norm_gate(o, xr[:, 2 * hd + hv:2 * hd + 2 * hv], L["mem_norm"], b.heads, b.vdim,
                                self.cfg.norm_eps, self.dtype, mul=mul)
-        return self._lin32(ol, L["wo_l"]), self._lin32(orr, L["wo_r"])
+        return proj_planes(ol, L["wo_l"]), proj_planes(orr, L["wo_r"])
 
     def _delta(self, li: int, h, inp: S.SegStepInputs, states) -> torch.Tensor:
         L, c = self.layers[li], self.cfg.layers[li].delta
         j, ra, rg = self.delta_of[li], L["ra"], L["rg"]
         qkv = linear(h, L["w_qkv"])                                    # [T, 2 G D + H V]
         qkv = S.short_conv(qkv, L["conv_w"], None, states[f"dconv{j}"], inp.seg, act=True)
-        agb = self._lin32(h, L["w_agb"])                               # [T, ra + rg + H] fp32
-        dec = self._lin32(self._act(agb[:, :ra]), L["w_a2"])           # [T, H D] fp32, before bias and softplus
-        gate = self._lin32(self._act(agb[:, ra:ra + rg]), L["w_g2"])   # [T, H V] fp32, before the sigmoid
+        agb = proj_f32out(h, L["w_agb"])                               # [T, ra + rg + H] fp32
+        dec = proj_f32out(self._act(agb[:, :ra]), L["w_a2"])           # [T, H D] fp32, before bias and softplus
+        gate = proj_f32out(self._act(agb[:, ra:ra + rg]), L["w_g2"])   # [T, H V] fp32, before the sigmoid
         o = S.gated_delta(qkv, c.heads, c.kv_heads, c.dim, c.vdim, dec, L["rate"], L["dt_bias"], agb[:, ra + rg:],
                           states[f"delta{j}"], inp.seg)
         o = S.head_norm_gate(o, gate, L["delta_norm"], c.heads, c.vdim, self.cfg.norm_eps, self.dtype)
-        return self._lin32(o, L["wo"])
+        return proj_planes(o, L["wo"])
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[torch.Tensor],
                 vts: List[Optional[torch.Tensor]], states: Dict[str, torch.Tensor],
@@ -461,13 +457,13 @@ class LizesunModel:
             else:
                 h = N.add_dyt(x, self._delta(li, h, inp, states), 1.0, None, 1.0, *after, out_dtype=dt)
             if spec.ff:
-                y = self._lin32(N.relu_sq(linear(h, L["w_up"])), L["w_down"])
+                y = proj_planes(N.relu_sq(linear(h, L["w_up"])), L["w_down"])
                 h = N.add_dyt(x, y, 1.0, None, 1.0, *nxt, out_dtype=dt)
             if layers_out is not None:
                 layers_out.append(x.clone())
         xr = x.index_select(0, inp.logits_idx).contiguous()
         h = N.add_dyt(xr, None, 1.0, None, 1.0, *self.final_norm, out_dtype=dt)
-        return self._lin32(h, self.lm_head)
+        return proj_f32out(h, self.lm_head)
 
 
 def random_tensors(cfg: LizesunConfig, seed: int = 0, device="cpu") -> Dict[str, torch.Tensor]:

@@ -90,7 +90,7 @@ _SIGS = {
     "k8s_mingru_scan": [P, P, P, P, P, P, P, P, I, I, I, P],
     "k8s_mingru_chunked": [P, P, P, P, P, I, P, P, P, P, P, P, I, I, P],
     "k8s_postnorm": [P, P, I, P, I, P, I, I, F, F, P],
-    "k8s_latent_norm": [P, I, P, P, P, P, P, P, I, I, I, I, F, I, P, I, I, P],
+    "k8s_latent_norm": [P, I, P, P, P, P, P, P, I, I, I, I, F, I, P, I, I, P, I, L],
     "k8s_rotated_tail": [P, P, P, I, I, I, I, I, I, P],
     "k8s_latent_attn_mfma_ok": [I, I],
     "k8s_latent_attn_mfma": [P, P, P, P, I, P, I, P, I, P, P, P, I, I, P, I, I, I, I, F, I, I, P, L, L, P, I, L, L, I, P],
@@ -118,13 +118,13 @@ _SIGS = {
     "k8s_window_attn_mfma_ok": [I, I, I, I],
     "k8s_window_attn_mfma": [P, I, P, P, P, I, P, I, P, P, P, P, I, I, I, I, I, I, F, P, I, I, P, P],
     "k8s_window_attn_rows": [P, I, P, P, P, I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
-    "k8s_add_dyt": [P, P, F, P, F, F, P, P, P, I, I, I, P],
+    "k8s_add_dyt": [P, P, F, P, F, F, P, P, P, I, I, I, P, I, I],
     "k8s_embed_scale_dyt": [P, P, I, F, P, F, P, P, P, I, I, I, P],
     "k8s_relu_sq": [P, P, ctypes.c_long, I, P],
     "k8s_attn_prep": [P, I, P, I, I, I, I, P, P, P, P, P, I, P, I, I, P, P, F, I, F, F, P, P, I, P, I, F, I, P, F, I, P],
     "k8s_rope_table": [P, P, F, P, I, I, P],
     "k8s_attn_prep_pairs": [P, I, I, I, I, I, I, P, P, P, P, I, P, I, I, P, I, P],
-    "k8s_attn_prep_half": [P, I, I, I, I, I, I, P, P, P, P, P, I, P, I, I, P, I, P, P, F, I, P, F, P, P],
+    "k8s_attn_prep_half": [P, I, I, I, I, I, I, P, P, P, P, P, I, P, I, I, P, I, P, P, F, I, P, F, P, P, I, L],
     "k8s_masked_attn_rows": [P, P, P, P, I, P, P, P, P, P, I, P, I, I, I, I, I, I, I, I, I, F, F, I, P, I, I, I, P, P],
     "k8s_masked_attn_mfma_ok": [I, I, I, I],
     "k8s_masked_attn_mfma": [P, P, P, P, I, P, I, P, P, I, P, I, I, I, I, I, I, I, I, F, F, P, I, I, P, P, I, I],
@@ -134,7 +134,7 @@ _SIGS = {
     "k8s_gated_delta_tiles": [P, I, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, F, P, P, I, P, P],
     "k8s_head_norm_gate": [P, P, I, P, I, P, I, I, I, F, I, P, P, I, F, F, I],
     "k8s_ssd_scan": [P, I, P, I, I, P, I, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, I, P, P, I, P, P, P],
-    "k8s_hyper_step": [P, P, I, P, P, I, P, P, P, P, F, P, I, I, I, I, P, P, P, F],
+    "k8s_hyper_step": [P, P, I, P, P, I, P, P, P, P, F, P, I, I, I, I, P, P, P, F, I],
     "k8s_hyper_embed": [P, P, I, F, P, I, P, P, F, P, I, I, I, P],
     "k8s_hyper_read": [P, P, I, I, P, P, F, P, I, I, P],
     "k8s_walks": [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P, P, P, P],

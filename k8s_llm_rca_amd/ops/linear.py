@@ -131,6 +131,10 @@ def linear_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 SKINNY_F32_MAX_M = 32
+# rows x columns of the skinny kernel's fp32 form: every 16-column workgroup reads all rows again, so a wide weight leaves it
+# at fewer rows (us, hipBLASLt / skinny: 8192 x 2048 at 16 rows 13.0 / 10.9, at 32 12.9 / 15.4; 8736 x 2048 at 7 / 16 / 32
+# 14.2 / 12.2, 14.2 / 14.4, 14.3 / 21.2; 2560 x 2048 at 32 9.8 / 8.0)
+SKINNY_F32_MAX_MN = 144 * 1024
 
 
 def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -140,13 +144,48 @@ def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return linear(x, w)
     M, K = x.shape
     N = w.shape[0]
-    if (_enabled and 0 < M <= SKINNY_F32_MAX_M and N * K <= SKINNY_MAX_NK and K % 256 == 0 and N % 16 == 0
-            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.dtype == torch.bfloat16 and w.is_contiguous()):
+    if (_enabled and 0 < M <= SKINNY_F32_MAX_M and M * N <= SKINNY_F32_MAX_MN and N * K <= SKINNY_MAX_NK
+            and K % 256 == 0 and N % 16 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.dtype == torch.bfloat16 and w.is_contiguous()):
         out = torch.empty((M, N), dtype=torch.float32, device=x.device)
         check(lib().k8s_gemm_skinny_f32(ptr(x), x.stride(0), ptr(w), ptr(out), N, M, N, K, stream_ptr(x)),
               "gemm_skinny_f32")
         return out
     return linear_f32out(x, w)
+
+
+PLANE_CFG = 14          # gemm_stream's LDS-DMA form with 4 stages
+PLANE_WGS = 256         # workgroups (64-column strips x K ranges) a product is cut into
+
+
+def plane_splits(M: int, N: int, K: int) -> int:
+    """K ranges :func:`proj_planes` cuts a product of a few rows into (1: one plane).  A product this narrow has a
+    workgroup per 64 columns, and 2048 columns leave seven of eight compute units idle: K is cut until every one has a
+    range.  us with cold weights, hipBLASLt / the skinny kernel / planes (the consumer's reads not counted):
+    2048 x 2048, 1 / 16 / 64 rows 8.1 / 4.9 / 4.1, 8.3 / 6.2 / 4.6, 8.9 / 11.7 / 5.4;  K 8192 12.4 / 12.6 / 8.5,
+    12.5 / 17.5 / 9.2, 21.8 / 38 / 10.1, at 128 rows 20.8 / -- / 12.8.  Past 64 rows a short K loses it again to the planes'
+    reads (128 rows, K 2048: 8.8 / -- / 7.3 + 8 planes of a megabyte)."""
+    if N % 64 or not (0 < M <= 64 or (M <= 128 and K >= 4096)):
+        return 1
+    s = 8
+    while s > 1 and (N // 64 * s > PLANE_WGS or K < 128 * s or not stream_shape_ok(M, N, K, PLANE_CFG, s)):
+        s //= 2
+    return s
+
+
+def proj_planes(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``x @ w.T`` in fp32 as planes [S, M, N] whose sum over S is the product (bf16 operands, fp32 accumulation): for
+    consumers that read it once and add the planes on the way in.  S = 1 wherever the planes do not pay."""
+    M, K = x.shape
+    N = w.shape[0]
+    if (x.is_cuda and x.dtype == torch.bfloat16 == w.dtype and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.is_contiguous() and x.data_ptr() % 16 == 0 == w.data_ptr() % 16):
+        S = plane_splits(M, N, K)
+        if S > 1:
+            out = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
+            check(lib().k8s_gemm_stream_part(ptr(x), x.stride(0), ptr(w), None, N, M, N, K, PLANE_CFG, S, ptr(out),
+                                             stream_ptr(x)), "gemm_stream_part")
+            return out
+    return proj_f32out(x, w)[None]
 
 
 def reserve_lib_workspace(dev: torch.device, claim_stream: int = None) -> None:

@@ -295,20 +295,23 @@ def embed_scale_dyt(ids: torch.Tensor, embed: torch.Tensor, scale: float, x_out:
 def add_dyt(x: torch.Tensor, y: Optional[torch.Tensor], sy: float = 1.0, y2: Optional[torch.Tensor] = None,
             sy2: float = 1.0, alpha: float = 1.0, w: Optional[torch.Tensor] = None, b: Optional[torch.Tensor] = None,
             out_dtype=None) -> Optional[torch.Tensor]:
-    """In place on the fp32 residual: ``x += sy * y (+ sy2 * y2)`` (``y`` None: nothing is added); with
+    """In place on the fp32 residual: ``x += sy * y (+ sy2 * y2)`` (``y`` None: nothing is added; [S, T, W]: the sum of its
+    planes, :func:`..ops.linear.proj_planes`); with
     ``w, b`` also returns ``tanh(alpha x) * w + b`` of the new rows as activations (the next sublayer's
     input norm, same pass)."""
     T, W = x.shape
     h = torch.empty(T, W, dtype=out_dtype, device=x.device) if w is not None else None
     if use_hip(x):
         for t in (x, y, y2):
-            assert t is None or (t.dtype == torch.float32 and t.is_contiguous() and t.shape == (T, W))
-        assert y is not None or y2 is None
+            assert t is None or (t.dtype == torch.float32 and t.is_contiguous() and t.shape[-2:] == (T, W) and t.dim() <= 3)
+        assert (y is not None or y2 is None) and x.dim() == 2
+        yp, yp2 = (t.shape[0] if t is not None and t.dim() == 3 else 1 for t in (y, y2))
         if y is None and h is None:
             return None
         check(lib().k8s_add_dyt(ptr(x), ptr(y), float(sy), ptr(y2), float(sy2), float(alpha), ptr(w), ptr(b), ptr(h),
-                                _odt(out_dtype) if h is not None else 1, T, W, stream_ptr(x)), "add_dyt")
+                                _odt(out_dtype) if h is not None else 1, T, W, stream_ptr(x), yp, yp2), "add_dyt")
         return h
+    y, y2 = (t.sum(0) if t is not None and t.dim() == 3 else t for t in (y, y2))
     if y is not None:
         x.add_(sy * y if y2 is None else sy * y + sy2 * y2)
     if h is not None:
@@ -354,7 +357,7 @@ def hyper_step(x: torch.Tensor, y: torch.Tensor, out: torch.Tensor, mix: torch.T
                inn: Optional[torch.Tensor] = None, nw: Optional[torch.Tensor] = None, eps: float = 0.0,
                out_dtype=None, again: Optional[tuple] = None) -> Optional[torch.Tensor]:
     """In place on the streams ``x`` [T, S, W]: ``x_r <- sum_s mix[s, r] x_s + out[r] y`` (all at once from the old ones).
-    ``y``: fp32 rows [T, W], or with ``experts = (inv, w)`` the experts' output rows in expert order, joined on the way in
+    ``y``: fp32 rows [T, W] or planes [S, T, W] of them that are summed (:func:`..ops.linear.proj_planes`), or with ``experts = (inv, w)`` the experts' output rows in expert order, joined on the way in
     as ``sum_k w[t, k] y[inv[t K + k]]`` (``inv`` from :func:`..ops.moe.align`, ``w`` [T, K] fp32).  With ``inn, nw`` also
     returns the next sublayer's input ``rms(sum_s inn[s] x_s) * nw`` of the new streams as activations.  ``again =
     (ids, embed, scale)``: the embedding output ``embed[ids] * scale`` is added to every stream as well, in front of that
@@ -363,16 +366,17 @@ def hyper_step(x: torch.Tensor, y: torch.Tensor, out: torch.Tensor, mix: torch.T
     read = nw is not None
     ids, embed, escale = again if again is not None else (None, None, 0.0)
     if use_hip(x):
-        assert x.dtype == torch.float32 and x.is_contiguous() and y.is_contiguous() and y.shape[1] == W
+        assert x.dtype == torch.float32 and x.is_contiguous() and y.is_contiguous() and y.shape[-1] == W
+        yp = y.shape[0] if y.dim() == 3 else 1
         assert out.dtype == mix.dtype == torch.float32 and out.numel() == S and mix.is_contiguous() and mix.numel() == S * S
         inv, ew, K = None, None, 0
         if experts is not None:
             inv, ew = experts
             K = ew.shape[1]
             assert ew.dtype == torch.float32 and ew.is_contiguous() and ew.shape[0] == T
-            assert inv.dtype == torch.int32 and inv.numel() == T * K and y.shape[0] == T * K
+            assert inv.dtype == torch.int32 and inv.numel() == T * K and y.shape == (T * K, W)
         else:
-            assert y.dtype == torch.float32 and y.shape[0] == T
+            assert y.dtype == torch.float32 and y.shape[-2] == T and y.dim() <= 3
         h = None
         if again is not None:
             assert read and embed.dtype == out_dtype and embed.is_contiguous() and embed.shape[1] == W
@@ -382,11 +386,13 @@ def hyper_step(x: torch.Tensor, y: torch.Tensor, out: torch.Tensor, mix: torch.T
             h = torch.empty(T, W, dtype=out_dtype, device=x.device)
         check(lib().k8s_hyper_step(ptr(x), ptr(y), _odt(y.dtype), ptr(inv), ptr(ew), K, ptr(out), ptr(mix), ptr(inn),
                                    ptr(nw), float(eps), ptr(h), _odt(out_dtype) if read else 1, T, S, W, stream_ptr(x),
-                                   ptr(ids), ptr(embed), float(escale)), "hyper_step")
+                                   ptr(ids), ptr(embed), float(escale), yp), "hyper_step")
         return h
     if experts is not None:
         inv, ew = experts
         y = (y.float()[inv.long()].view(T, ew.shape[1], W) * ew[:, :, None]).sum(1)
+    elif y.dim() == 3:
+        y = y.sum(0)
     x.copy_(torch.einsum("sr,tsw->trw", mix, x) + out[None, :, None] * y[:, None])
     if again is not None:
         x += (embed[ids.long()].float() * escale)[:, None]

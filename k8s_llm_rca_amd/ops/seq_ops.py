@@ -256,7 +256,17 @@ def latent_norm(dn: torch.Tensor, wq: torch.Tensor, wkv: Optional[torch.Tensor],
     to its transposed twin ``cache_t`` [pages, kv_rank, BS] when given (the MFMA kernels' PV operand).
     ``tail`` > 0: as many further columns of ``dn`` are a key part shared by all heads; its neighbouring entries
     2i, 2i + 1 are turned by ``tail_cs`` [T, tail] (a :func:`rope_table`) and stand behind the latent in the cache
-    rows [pages, BS, kv_rank + pad], filled up with zeros."""
+    rows [pages, BS, kv_rank + pad], filled up with zeros.  ``dn`` [S, T, ..]: the sum of its planes
+    (:func:`.linear.proj_planes`)."""
+    planes, pstep = 1, 0
+    if dn.dim() == 3:
+        if dn.shape[0] == 1:
+            dn = dn[0]
+        elif use_hip(dn) and not (dn.stride(0) % 4 or dn.stride(1) % 4 or dn.data_ptr() % 16
+                                  or (q_rank + (kv_rank if wkv is not None else 0) + tail) % 4):
+            planes, pstep, dn = dn.shape[0], dn.stride(0), dn[0]      # added where the rows are read
+        else:
+            dn = dn.sum(0)
     T = dn.shape[0]
     cq = torch.empty(T, q_rank, dtype=out_dtype, device=dn.device)
     kr = kv_rank if wkv is not None else 0
@@ -270,7 +280,7 @@ def latent_norm(dn: torch.Tensor, wq: torch.Tensor, wkv: Optional[torch.Tensor],
         assert not tail or (kr and tail_cs.dtype == torch.float32 and tail_cs.is_contiguous() and tail_cs.shape == (T, tail))
         check(lib().k8s_latent_norm(ptr(dn), dn.stride(0), ptr(wq), ptr(wkv), ptr(slots), ptr(cq), ptr(cache),
                                     ptr(ct), cache.shape[1] if kr else 1, T, q_rank, kr, float(eps),
-                                    _dt(out_dtype), stream_ptr(dn), tail, pad, ptr(tail_cs)), "latent_norm")
+                                    _dt(out_dtype), stream_ptr(dn), tail, pad, ptr(tail_cs), planes, pstep), "latent_norm")
         return cq
     q = dn[:, :q_rank]
     cq.copy_((q * torch.rsqrt(q.pow(2).mean(-1, keepdim=True) + eps) * wq.float()).to(out_dtype))
@@ -877,7 +887,17 @@ def attn_prep(qkv: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D
     ``v_other`` the values become ``(1 - lam) v + lam v_other``.  ``v_is_k``: there are no value columns, the values
     are the keys as projected (before norm and rotation; V = M D).  k and v go to the pages ``kc`` [pages, BS, G M D] /
     ``vc`` [pages, BS, G V] at ``slots`` (and v to the transposed twin ``vt`` when given, then ``vc`` may be None); q is returned [T, H M D] as
-    activations.  ``G = 0``: only queries (a layer that reads another layer's pages)."""
+    activations.  ``G = 0``: only queries (a layer that reads another layer's pages).  ``qkv`` [S, T, ..]: the sum of its
+    planes (:func:`.linear.proj_planes`)."""
+    planes, pstep = 1, 0
+    if qkv.dim() == 3:
+        if qkv.shape[0] > 1 and use_hip(qkv) and norm in (False, None, True, "head") and not q_temp and 8 <= D <= 512 \
+                and D & (D - 1) == 0 and (rope is None or (rope_cs is not None and not rope.pairs and rope.dims % 8 == 0)) \
+                and not (rope is None and rot_dims) and qkv.stride(1) % 4 == 0 and qkv.data_ptr() % 16 == 0 \
+                and qkv.stride(0) % 4 == 0 and qkv.shape[1] <= 1024 and (norm or bias is not None):
+            planes, pstep, qkv = qkv.shape[0], qkv.stride(0), qkv[0]      # added where the rows are read
+        else:
+            qkv = qkv[0] if qkv.shape[0] == 1 else qkv.sum(0)
     T = qkv.shape[0]
     HQ, GK = H * maps, G * maps
     NQ, NK, NV = HQ * D, GK * D, G * V
@@ -918,7 +938,7 @@ def attn_prep(qkv: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D
             check(lib().k8s_attn_prep_half(ptr(qkv), qkv.stride(0), HQ, GK, D, NV, v_col, ptr(bias), ptr(slots), ptr(kc),
                                            ptr(vc), ptr(vt), BS, ptr(q_out), _dt(out_dtype), int(rot_dims), ptr(rope_cs),
                                            mode, ptr(q_w), ptr(k_w), float(eps), T, stream_ptr(qkv), float(lam),
-                                           ptr(v_other), ptr(v_keep)), "attn_prep_half")
+                                           ptr(v_other), ptr(v_keep), planes, pstep), "attn_prep_half")
             return q_out
         check(lib().k8s_attn_prep(ptr(qkv), qkv.stride(0), ptr(bias), HQ, GK, D, NV, ptr(positions), ptr(slots),
                                   ptr(kc), ptr(vc), ptr(vt), BS, ptr(q_out), _dt(out_dtype), mode, ptr(q_w),
