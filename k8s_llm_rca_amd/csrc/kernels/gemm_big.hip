@@ -187,7 +187,7 @@ struct RopeArgs {
 // act columns, W has 2I rows, I = N); MODE 2: the qkv projection with RoPE on q
 // and k and the paged K / V write in the epilogue (N = (nq + 2 nkv) 128; the
 // rope_kv_kernel's arithmetic and rounding: bit-identical to GEMM + k8s_rope_kv);
-// MODE 3 (grouped only): MODE 0 with max(., 0)^2 of every output.
+// MODE 3: MODE 0 with max(., 0)^2 of every output.
 // VAR bit 0: ping-pong stagger of waves
 // 4-7; bit 1: s_setprio(1) around the MFMA clusters; bit 2: the 32x32x16 MFMA
 // (1 = the default).
@@ -673,7 +673,7 @@ static int big_launch(const void* x, int ldx, const void* w, void* y, int ldy, i
   using namespace k8s::big;
   if (M <= 0) return 0;
   if (splits < 1 || K % (2 * BK * splits) || K < 2 * BK || ldx % 8 || ldx < K || ldy < N || N <= 0 ||
-      ((mode == 0 || mode == 2) && N % BN) || (mode == 1 && N % 128) || mode < 0 || mode > 2 ||
+      (mode != 1 && N % BN) || (mode == 1 && N % 128) || mode < 0 || mode > 3 ||
       ((uintptr_t)x % 16) || ((uintptr_t)w % 16) || (mode != 1 && (ldy % 8 || (uintptr_t)y % 16)) ||
       (mode == 1 && (ldy % 4 || (uintptr_t)y % 8)) || (splits > 1 && (mode != 0 || part == nullptr)))
     return (int)hipErrorInvalidValue;
@@ -690,9 +690,12 @@ static int big_launch(const void* x, int ldx, const void* w, void* y, int ldy, i
   } else if (mode == 1) {
     rc = (var & 4) ? launch<1, 5>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s)
                    : launch<1, 1>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s);
-  } else {
+  } else if (mode == 2) {
     rc = (var & 4) ? launch<2, 5>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s)
                    : launch<2, 1>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s);
+  } else {
+    rc = (var & 4) ? launch<3, 5>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s)
+                   : launch<3, 1>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s);
   }
   if (rc || splits == 1 || !reduce) return rc;
   const long blocks = ((long)M * N / 8 + 255) / 256;
@@ -757,7 +760,8 @@ K8S_API long k8s_gemm_big_tail_foreign() {
 }
 
 // mode 0: y[M][N] = x . w^T (w [N][K], N % 256 == 0);
-// mode 1: y[M][N] = silu(x . w[0:N]^T) * (x . w[N:2N]^T) (w [2N][K], N % 128 == 0).
+// mode 1: y[M][N] = silu(x . w[0:N]^T) * (x . w[N:2N]^T) (w [2N][K], N % 128 == 0);
+// mode 3: y[M][N] = max(x . w^T, 0)^2.
 // var: schedule variant (bit 0: ping-pong stagger, bit 1: s_setprio around the
 // MFMA clusters, bit 2: 32x32x16 MFMA; 1 / 3 / 5 / 7 are built).
 // K % 128 == 0, ldx % 8 == 0, ldy % 8 (mode 0) / 4 (mode 1) == 0, 16-byte

@@ -455,7 +455,7 @@ template <int MTW, int NB, int NF, bool HAND, bool PUSH = false>
 __global__ void __launch_bounds__(256) gemm_glds_kernel(const uint16_t* __restrict__ x, int ldx,
                                                         const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
                                                         int ldy, float* __restrict__ part, int M, int N, int K,
-                                                        int kslice, int silu_i, K8sPush push) {
+                                                        int kslice, int silu_i, int act, K8sPush push) {
   __shared__ __attribute__((aligned(16))) uint16_t sm[glds_lds_elems<MTW, NB, NF>()];
   // strip: 16 NF W rows (plain: output columns n0 ..; SwiGLU: 8 NF act columns n0 ..)
   const int n0 = blockIdx.x * (silu_i ? 8 : 16) * NF, split = blockIdx.y, kbeg = split * kslice;
@@ -471,7 +471,7 @@ __global__ void __launch_bounds__(256) gemm_glds_kernel(const uint16_t* __restri
   else if (silu_i)
     glds_store<MTW, NF>(acc, M, y + n0, ldy, nullptr, 0, true);
   else if (gridDim.y == 1)
-    glds_store<MTW, NF>(acc, M, y + n0, ldy, nullptr, 0);
+    glds_store<MTW, NF>(acc, M, y + n0, ldy, nullptr, 0, false, act);
   else
     glds_store<MTW, NF>(acc, M, nullptr, 0, part + (size_t)split * M * N + n0, N);
 }
@@ -572,17 +572,17 @@ static bool glds_hand() { return knob(kKnobGldsHand) != 0; }
 template <int MTW, int NB, int NF = 4>
 static hipError_t launch_glds(dim3 grid, hipStream_t s, const uint16_t* x, int ldx, const uint16_t* w, uint16_t* y,
                               int ldy, float* part, int M, int N, int K, int kslice, int silu_i,
-                              const K8sPush* push = nullptr) {
+                              const K8sPush* push = nullptr, int act = 0) {
   const K8sPush none{};
   if (push)
     hipLaunchKernelGGL((gemm_glds_kernel<MTW, NB, NF, true, true>), grid, dim3(256), 0, s, x, ldx, w, y, ldy, part, M,
-                       N, K, kslice, 0, *push);
+                       N, K, kslice, 0, 0, *push);
   else if (glds_hand())
     hipLaunchKernelGGL((gemm_glds_kernel<MTW, NB, NF, true>), grid, dim3(256), 0, s, x, ldx, w, y, ldy, part, M, N,
-                       K, kslice, silu_i, none);
+                       K, kslice, silu_i, act, none);
   else
     hipLaunchKernelGGL((gemm_glds_kernel<MTW, NB, NF, false>), grid, dim3(256), 0, s, x, ldx, w, y, ldy, part, M, N,
-                       K, kslice, silu_i, none);
+                       K, kslice, silu_i, act, none);
   return hipGetLastError();
 }
 
@@ -600,19 +600,25 @@ using namespace k8s;
 
 // cfg: register-ring depth U (4 or 8), or 10 + NB for the LDS-DMA kernel (NB = 3..6
 // stages; 5 and 6 for M <= 64), or 20 + NB for the LDS-DMA kernel on 128-column
-// strips (NB = 3, or 4 for M <= 192; N % 128 == 0).  splits > 1 needs `part` =
+// strips (NB = 3, or 4 for M <= 192; N % 128 == 0), or 30 + NB on 32-column strips (NB = 4 or 6, M <= 128; N % 32
+// == 0).  The narrow strips are for weights of 2k..8k rows: at 64 columns they leave half the 256 CUs or more without
+// a workgroup, and cutting K instead costs a pass over the partials.  8192 x 2048, 16 / 64 / 128 rows, us: 64 columns
+// 11.8 / 12.8 / 16.2, 64 columns and two K ranges 10.6 / 11.9 / 15.2, 32 columns 10.0 / 11.1 / 13.7 (weights alone at
+// 4.95 TB/s: 6.8).  Past one strip per CU they lose (8736 rows, 64 rows of X: 17.2 against 15.3 of hipBLASLt).
+// splits > 1 needs `part` =
 // splits * M * N fp32; reduce = 0 leaves the partials for a fused consumer.
 // silu: w is the gate_up weight [2N][K] (gate rows first) and y[M][N] = silu(x Wg^T) * (x Wu^T)
 // (splits == 1 only: the nonlinearity needs the whole K sum).
 static int stream_launch(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int cfg,
                          int splits, void* part, bool reduce, hipStream_t s, bool silu = false,
-                         const K8sPush* push = nullptr) {
+                         const K8sPush* push = nullptr, int act = 0) {
   // push (splits == 1): the LDS-DMA kernel's own epilogue pushes; splits > 1: the reduce pass does
   const K8sPush* gpush = (push && splits == 1) ? push : nullptr;
   if (push && (silu || !reduce || (splits == 1 && cfg < 13))) return (int)hipErrorInvalidValue;
-  const int bn = (cfg > 20 ? 128 : kSBN) / (silu ? 2 : 1);  // output columns per strip
+  if (act && (act != 1 || silu || push || splits != 1 || cfg < 13)) return (int)hipErrorInvalidValue;
+  const int bn = (cfg > 30 ? 32 : cfg > 20 ? 128 : kSBN) / (silu ? 2 : 1);  // output columns per strip
   if (M <= 0 || M > 256 || N % bn || splits < 1 || K % (splits * kSC) || (splits > 1 && part == nullptr) ||
-      (cfg != 4 && cfg != 8 && (cfg < 13 || cfg > 16) && cfg != 23 && cfg != 24) || ldx % 8 ||
+      (cfg != 4 && cfg != 8 && (cfg < 13 || cfg > 16) && cfg != 23 && cfg != 24 && cfg != 34 && cfg != 36) || ldx % 8 ||
       (splits > 1 && (M * N) % 8) || ((splits == 1 || reduce) && ldy < N) || (silu && splits != 1))
     return (int)hipErrorInvalidValue;
   const int silu_i = silu ? N : 0;
@@ -621,7 +627,8 @@ static int stream_launch(const void* x, int ldx, const void* w, void* y, int ldy
   if (cfg < 10 && (kslice / kSC) % cfg) return (int)hipErrorInvalidValue;
   const int mtw = ((M + 15) / 16 + 3) / 4;  // 16-row fragments per wave (4 waves)
   // LDS-DMA stages of (64 + 64 * mtw) x 64 bf16 must fit the 160 KB of LDS
-  if ((cfg == 14 && mtw > 3) || (cfg > 14 && cfg < 20 && mtw > 1) || (cfg == 24 && mtw > 3))
+  if ((cfg == 14 && mtw > 3) || (cfg > 14 && cfg < 20 && mtw > 1) || (cfg == 24 && mtw > 3) ||
+      (cfg > 30 && (mtw > 2 || push)))
     return (int)hipErrorInvalidValue;
   if (cfg == 8 && mtw > 2) return (int)hipErrorInvalidValue;  // an 8-deep X ring would not fit the VGPRs
   const dim3 grid(N / bn, splits);
@@ -631,8 +638,9 @@ static int stream_launch(const void* x, int ldx, const void* w, void* y, int ldy
   float* pp = (float*)part;
   hipError_t e;
 #define K8S_SL(MT, UU) e = launch_stream<MT, UU>(grid, s, xx, ldx, ww, yy, ldy, pp, M, N, K, kslice, silu_i)
-#define K8S_GL(MT, NB) e = launch_glds<MT, NB>(grid, s, xx, ldx, ww, yy, ldy, pp, M, N, K, kslice, silu_i, gpush)
-#define K8S_GW(MT, NB) e = launch_glds<MT, NB, 8>(grid, s, xx, ldx, ww, yy, ldy, pp, M, N, K, kslice, silu_i, gpush)
+#define K8S_GL(MT, NB) e = launch_glds<MT, NB>(grid, s, xx, ldx, ww, yy, ldy, pp, M, N, K, kslice, silu_i, gpush, act)
+#define K8S_GW(MT, NB) e = launch_glds<MT, NB, 8>(grid, s, xx, ldx, ww, yy, ldy, pp, M, N, K, kslice, silu_i, gpush, act)
+#define K8S_GN(MT, NB) e = launch_glds<MT, NB, 2>(grid, s, xx, ldx, ww, yy, ldy, pp, M, N, K, kslice, silu_i, nullptr, act)
   if (cfg == 23) {
     switch (mtw) {
       case 1: K8S_GW(1, 3); break;
@@ -645,6 +653,16 @@ static int stream_launch(const void* x, int ldx, const void* w, void* y, int ldy
       case 1: K8S_GW(1, 4); break;
       case 2: K8S_GW(2, 4); break;
       default: K8S_GW(3, 4); break;
+    }
+  } else if (cfg == 36) {
+    switch (mtw) {
+      case 1: K8S_GN(1, 6); break;
+      default: K8S_GN(2, 6); break;
+    }
+  } else if (cfg == 34) {
+    switch (mtw) {
+      case 1: K8S_GN(1, 4); break;
+      default: K8S_GN(2, 4); break;
     }
   } else if (cfg == 13) {
     switch (mtw) {
@@ -680,6 +698,7 @@ static int stream_launch(const void* x, int ldx, const void* w, void* y, int ldy
 #undef K8S_SL
 #undef K8S_GL
 #undef K8S_GW
+#undef K8S_GN
   if (e != hipSuccess) return (int)e;
   if (splits > 1 && push) {
     hipLaunchKernelGGL(gemm_stream_reduce_push_kernel, dim3(N / 64), dim3(256), 0, s, (const float*)part, splits, M, N,
@@ -695,6 +714,12 @@ static int stream_launch(const void* x, int ldx, const void* w, void* y, int ldy
 K8S_API int k8s_gemm_stream(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int cfg,
                             int splits, void* part, hipStream_t s) {
   return stream_launch(x, ldx, w, y, ldy, M, N, K, cfg, splits, part, true, s);
+}
+
+// act 1: y = max(x . w^T, 0)^2 (the LDS-DMA forms, one K range).
+K8S_API int k8s_gemm_stream_act(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int cfg,
+                                int act, hipStream_t s) {
+  return stream_launch(x, ldx, w, y, ldy, M, N, K, cfg, 1, nullptr, true, s, false, nullptr, act);
 }
 
 extern "C" int k8s_ar_push_desc(int id, int N, int T, int mode, K8sPush* out);

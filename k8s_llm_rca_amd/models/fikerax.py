@@ -29,10 +29,9 @@ from typing import Dict, List, Optional, Tuple
 
 import torch
 
-from ..ops import moe as M
 from ..ops import norm as N
 from ..ops import seq_ops as S
-from ..ops.linear import linear, proj_f32out, proj_planes, swiglu_gemm
+from ..ops.linear import glu_proj, proj, proj_f32out, proj_planes
 from ..parallel.groups import ParallelContext, single
 
 TAIL_ALIGN = 32     # the rotated key part of a latent cache row is filled up to a multiple of this
@@ -378,7 +377,7 @@ class FikeraxModel:
     def _lightning(self, i: int, h: torch.Tensor, inp: S.SegStepInputs, state: torch.Tensor) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
         HV = c.heads * c.vdim
-        x = linear(h, L["w_in"])                                             # q | k | v | gate as activations
+        x = proj(h, L["w_in"])                                             # q | k | v | gate as activations
         o = S.decay_attention(x, c.heads, c.dim, c.vdim, L["decay"], state, inp.seg, silu=True)
         y = S.head_norm_gate(o, x[:, x.shape[1] - HV:], L["mem_norm"], 1, HV, self.cfg.norm_eps, self.dtype)
         return proj_planes(y, L["wo"])
@@ -398,7 +397,7 @@ class FikeraxModel:
         dn = proj_planes(h, L["w_in"])                                        # [., T, q_rank + KR + R] fp32
         cq = S.latent_norm(dn, L["dq_norm"], L["dkv_norm"], inp.slots, cache, c.q_rank, KR, self.cfg.norm_eps, self.dtype,
                            cache_t=cache_t, tail=R, tail_cs=cs)
-        q = linear(cq, L["w_uq"])                                             # [T, H (D + R)]
+        q = proj(cq, L["w_uq"])                                             # [T, H (D + R)]
         qr = S.rotated_tail(q, cs, H, D, c.tail) if R else None
         qa = torch.bmm(q.view(T, H, D + R)[:, :, :D].transpose(0, 1), L["uk"]).transpose(0, 1)    # [T, H, KR], head-major
         kw = dict(window=c.window, sink=L["sink"], head_major=True)
@@ -413,10 +412,7 @@ class FikeraxModel:
 
     def _dense(self, i: int, h: torch.Tensor) -> torch.Tensor:
         L = self.layers[i]
-        a = swiglu_gemm(h, L["w13"])                                          # one launch where a fused kernel takes the shape
-        if a is None:
-            a = M.glu_clamp(linear(h, L["w13"]), 1.0, math.inf, 0.0)          # silu(gate) * up
-        return proj_planes(a, L["w2"])
+        return proj_planes(glu_proj(h, L["w13"]), L["w2"])                    # silu(gate) * up
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[Optional[torch.Tensor]],
                 vts: List[Optional[torch.Tensor]], states: Optional[Dict[str, torch.Tensor]] = None,

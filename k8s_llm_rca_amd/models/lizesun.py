@@ -35,7 +35,7 @@ import torch
 
 from ..ops import norm as N
 from ..ops import seq_ops as S
-from ..ops.linear import linear, proj_f32out, proj_planes
+from ..ops.linear import proj, proj_f32out, proj_planes, relu_sq_proj
 from ..parallel.groups import ParallelContext, single
 
 
@@ -389,9 +389,9 @@ class LizesunModel:
                 keep = vmix["v"] = torch.empty(x.shape[0], G * V, dtype=torch.float32, device=x.device)
             else:
                 other = vmix["v"]
-        q = S.attn_prep(x[:, :H * D + G * (D + V)], L["bias"], H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], self.dtype, norm=True,
-                        q_w=L["q_w"], k_w=L["k_w"], eps=self.cfg.norm_eps, lam=L["lam"], v_other=other, v_keep=keep,
-                        vt=vts[ci])
+        q = S.attn_prep(x[:, :H * D + G * (D + V)], L["bias"], H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci],
+                        self.dtype, norm=True, q_w=L["q_w"], k_w=L["k_w"], eps=self.cfg.norm_eps, lam=L["lam"],
+                        v_other=other, v_keep=keep, vt=vts[ci])
         o = S.masked_attention(q, H, G, D, V, kcs[ci], vcs[ci], inp.seg, a.scale, softcap=a.softcap, chunk=a.chunk,
                                gate=x[:, H * D + G * (D + V):], vt=vts[ci])
         return proj_planes(o, L["wo"])
@@ -422,7 +422,7 @@ class LizesunModel:
     def _delta(self, li: int, h, inp: S.SegStepInputs, states) -> torch.Tensor:
         L, c = self.layers[li], self.cfg.layers[li].delta
         j, ra, rg = self.delta_of[li], L["ra"], L["rg"]
-        qkv = linear(h, L["w_qkv"])                                    # [T, 2 G D + H V]
+        qkv = proj(h, L["w_qkv"])                                    # [T, 2 G D + H V]
         qkv = S.short_conv(qkv, L["conv_w"], None, states[f"dconv{j}"], inp.seg, act=True)
         agb = proj_f32out(h, L["w_agb"])                               # [T, ra + rg + H] fp32
         dec = proj_f32out(self._act(agb[:, :ra]), L["w_a2"])           # [T, H D] fp32, before bias and softplus
@@ -457,7 +457,7 @@ class LizesunModel:
             else:
                 h = N.add_dyt(x, self._delta(li, h, inp, states), 1.0, None, 1.0, *after, out_dtype=dt)
             if spec.ff:
-                y = proj_planes(N.relu_sq(linear(h, L["w_up"])), L["w_down"])
+                y = proj_planes(relu_sq_proj(h, L["w_up"]), L["w_down"])
                 h = N.add_dyt(x, y, 1.0, None, 1.0, *nxt, out_dtype=dt)
             if layers_out is not None:
                 layers_out.append(x.clone())

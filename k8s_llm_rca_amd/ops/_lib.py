@@ -50,6 +50,7 @@ _SIGS = {
     "k8s_gemm_big_set_ws": [P],
     "k8s_gemm_big_claim_ws": [P],
     "k8s_gemm_big_tail_foreign": [],
+    "k8s_gemm_stream_act": [P, I, P, P, I, I, I, I, I, I, P],
     "k8s_gemm_stream_silu": [P, I, P, P, I, I, I, I, I, P],
     "k8s_gemm_stream_silu_norm": [P, I, P, I, P, P, P, F, P, P, I, I, I, I, I, P],
     "k8s_gemm_skinny_rope_norm": [P, I, P, I, P, P, P, F, P, P, I, I, I, I, P, P, P, P, P, I, I, I, P],

@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 import json
+import math
 import os
 from typing import Dict, List, Tuple
 
@@ -10,6 +11,8 @@ import torch.nn.functional as F
 
 from ..knobs import KNOBS
 from ._lib import check, lib, ptr, scratch, stream_ptr
+from .moe import glu_clamp
+from .norm import relu_sq
 
 SKINNY_MAX_M = KNOBS.skinny_max_m
 # measured on MI355X (tools/bench_kernels.py): the skinny kernel beats hipBLASLt
@@ -145,7 +148,8 @@ def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     M, K = x.shape
     N = w.shape[0]
     if (_enabled and 0 < M <= SKINNY_F32_MAX_M and M * N <= SKINNY_F32_MAX_MN and N * K <= SKINNY_MAX_NK
-            and K % 256 == 0 and N % 16 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.dtype == torch.bfloat16 and w.is_contiguous()):
+            and K % 256 == 0 and N % 16 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.dtype == torch.bfloat16 and w.is_contiguous()):
         out = torch.empty((M, N), dtype=torch.float32, device=x.device)
         check(lib().k8s_gemm_skinny_f32(ptr(x), x.stride(0), ptr(w), ptr(out), N, M, N, K, stream_ptr(x)),
               "gemm_skinny_f32")
@@ -153,23 +157,33 @@ def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return linear_f32out(x, w)
 
 
-PLANE_CFG = 14          # gemm_stream's LDS-DMA form with 4 stages
-PLANE_WGS = 256         # workgroups (64-column strips x K ranges) a product is cut into
+# -------------------------------------------------- products of a few rows by their shape
+# The stream kernel on 32-column strips (csrc/kernels/gemm_stream.hip): twice the workgroups of the 64-column form, so a
+# weight of 2k..8k rows puts one on each of the 256 compute units without cutting K.
+NARROW_WGS = 256        # strips one wave of workgroups holds; more of them lose to the wider strips
+NARROW_MAX_M = 128      # two 16-row fragments per wave
 
 
-def plane_splits(M: int, N: int, K: int) -> int:
-    """K ranges :func:`proj_planes` cuts a product of a few rows into (1: one plane).  A product this narrow has a
-    workgroup per 64 columns, and 2048 columns leave seven of eight compute units idle: K is cut until every one has a
-    range.  us with cold weights, hipBLASLt / the skinny kernel / planes (the consumer's reads not counted):
-    2048 x 2048, 1 / 16 / 64 rows 8.1 / 4.9 / 4.1, 8.3 / 6.2 / 4.6, 8.9 / 11.7 / 5.4;  K 8192 12.4 / 12.6 / 8.5,
-    12.5 / 17.5 / 9.2, 21.8 / 38 / 10.1, at 128 rows 20.8 / -- / 12.8.  Past 64 rows a short K loses it again to the planes'
-    reads (128 rows, K 2048: 8.8 / -- / 7.3 + 8 planes of a megabyte)."""
-    if N % 64 or not (0 < M <= 64 or (M <= 128 and K >= 4096)):
-        return 1
-    s = 8
-    while s > 1 and (N // 64 * s > PLANE_WGS or K < 128 * s or not stream_shape_ok(M, N, K, PLANE_CFG, s)):
+def _narrow_cfg(M: int) -> int:
+    """Stages of the 32-column form: 6 up to 32 rows, 4 above (us at 8192 x 2048, 6 / 4 stages: 1 row 10.0 / 10.4, 32 rows
+    10.2 / 10.6, 64 rows 11.4 / 11.1, 128 rows 14.7 / 13.7)."""
+    return 36 if M <= 32 else 34
+
+
+def plane_plan(M: int, N: int, K: int):
+    """(stream configuration, K ranges) of :func:`proj_planes`; one range: the product is not cut.  2048 columns are 32 or
+    64 strips for 256 compute units, so K is cut until each has a workgroup: four ranges of 32-column strips where K is
+    short, eight of 64-column strips from 4096 on.  us with cold weights at 1 / 16 / 64 / 128 rows: 2048 x 2048 hipBLASLt
+    8.1 / 8.3 / 8.9 / 8.8, the skinny kernel 4.9 / 6.2 / 11.7 / --, 64-column planes 4.2 / 4.5 / 5.5 / 7.2, 32-column
+    planes 4.1 / 4.4 / 4.8 / 6.6 and half as many to read;  2560 x 2048 32-column planes 5.0 / 5.3 / 6.8 / 10.0 against
+    10.5 / 11.7 / 12.5 / 15.9;  2048 x 8192 12.4 / 12.5 / 21.8 / 20.8, 12.6 / 17.5 / 38 / --, 64-column 8.7 / 9.2 / 10.0 /
+    12.8, 32-column 9.9 / 10.0 / 11.5 / 15.6."""
+    if not 0 < M <= NARROW_MAX_M:
+        return 14, 1
+    cfg, bn, s, most = (34, 32, 4, 320) if K < 4096 else (14, 64, 8, 256)
+    while s > 1 and (-(-N // bn) * s > most or K < 128 * s or not stream_shape_ok(M, N, K, cfg, s)):
         s //= 2
-    return s
+    return cfg, s
 
 
 def proj_planes(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -177,15 +191,87 @@ def proj_planes(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     consumers that read it once and add the planes on the way in.  S = 1 wherever the planes do not pay."""
     M, K = x.shape
     N = w.shape[0]
-    if (x.is_cuda and x.dtype == torch.bfloat16 == w.dtype and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and w.is_contiguous() and x.data_ptr() % 16 == 0 == w.data_ptr() % 16):
-        S = plane_splits(M, N, K)
+    if _few_ok(x, w):
+        cfg, S = plane_plan(M, N, K)
         if S > 1:
             out = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
-            check(lib().k8s_gemm_stream_part(ptr(x), x.stride(0), ptr(w), None, N, M, N, K, PLANE_CFG, S, ptr(out),
+            check(lib().k8s_gemm_stream_part(ptr(x), x.stride(0), ptr(w), None, N, M, N, K, cfg, S, ptr(out),
                                              stream_ptr(x)), "gemm_stream_part")
             return out
     return proj_f32out(x, w)[None]
+
+
+def _few_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (x.is_cuda and x.dtype == torch.bfloat16 == w.dtype and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.is_contiguous() and x.data_ptr() % 16 == 0 == w.data_ptr() % 16)
+
+
+def proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``x @ w.T`` as activations, with the 32-column stream form where it is the fastest: 17 to 128 rows (below, the skinny
+    kernel) and one wave of strips with the K it was measured at.  us at 17..32 / 64 / 128 rows, hipBLASLt / this:
+    8192 x 2048 12.3 / 10.2, 12.8 / 11.1, 15.6 / 13.7;  4736 x 2048 12.3 / 9.7, 12.9 / 10.7, 15.2 / 13.6;  2048 x 2048
+    9.2 / 8.3, 10.6 / 8.3, 10.5 / 10.6.  At 273 strips the second wave costs it the lead (8736 x 2048, 64 rows:
+    15.3 / 17.2)."""
+    M, K = x.shape
+    N = w.shape[0]
+    if (16 < M <= NARROW_MAX_M and 32 <= N <= 32 * NARROW_WGS and K <= 2048 and (N, K) not in _dispatch and _few_ok(x, w)
+            and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
+        return gemm_stream(x, w, _narrow_cfg(M), 1)
+    return linear(x, w)
+
+
+def big_tiles_fill(M: int, N: int, silu: bool) -> bool:
+    """Whether gemm_big's 256-row tiles fill the 256 compute units to four fifths over all their waves.  Then its fused
+    epilogue beats hipBLASLt and a pass over the result, otherwise the idle last wave costs more than the pass: us apart /
+    fused of SwiGLU 8192 x 2048 at 192 tiles 50 / 49, 256 65 / 56, 320 100 / 111, 384 106 / 110, 448 116 / 100, 512
+    124 / 106, 704 192 / 148, 4096 tiles 936 / 811, and of the squared relu 128 37 / 52, 192 52 / 44, 256 63 / 52, 320
+    83 / 100, 384 98 / 102, 448 112 / 96, 512 120 / 102, 2048 tiles 479 / 400."""
+    tiles = -(-M // 256) * -(-N // (128 if silu else 256))
+    return 5 * tiles >= 4 * 256 * -(-tiles // 256)
+
+
+def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``max(x @ w.T, 0)^2`` as activations.  In one launch for up to 128 rows over one wave of 32-column strips (us apart /
+    fused at 8192 x 2048: 1 row 10.5 / 9.8, 16 rows 12.9 / 10.1, 64 rows 15.5 / 11.0, 128 rows 17.9 / 13.9) and for prompts
+    whose tiles fill the card (:func:`big_tiles_fill`) or whose K is so short that the result's passes are what is paid
+    (1024 x 256 at 16384 rows: 31 / 16); the fused forms square the fp32 sum."""
+    M, K = x.shape
+    N = w.shape[0]
+    if _few_ok(x, w):
+        if (0 < M <= NARROW_MAX_M and N <= 32 * NARROW_WGS and K <= 2048 and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
+            out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+            check(lib().k8s_gemm_stream_act(ptr(x), x.stride(0), ptr(w), ptr(out), N, M, N, K, _narrow_cfg(M), 1,
+                                            stream_ptr(x)), "gemm_stream_act")
+            return out
+        if M > DISPATCH_MAX_M and big_shape_ok(M, N, K) and (K <= 512 or big_tiles_fill(M, N, False)):
+            return gemm_big(x, w, relu2=True)
+    return relu_sq(linear(x, w))
+
+
+def glu_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``silu(x @ Wg.T) * (x @ Wu.T)`` as activations (w = [Wg; Wu]): what a dispatch table says, then one launch by shape.
+    Up to 128 rows (us apart / fused at 1, 16, 64, 128 rows): up to 256 strips of 16 outputs the 32-row strips, except where
+    few weight bytes leave the skinny kernel ahead (4096 x 2048 11.4 / 9.9, 13.1 / 10.3, 15.8 / 11.1, 18.2 / 14.1;  2048 x
+    2048 7.7 / 9.3, 9.3 / 9.6, 14.8 / 10.4, 17.8 / 13.5;  640 x 384 6.1 / 3.3 .. 9.4 / 4.6); wider weights the 64-row strips
+    (6144 x 2048 14.2 / 12.9, 18.5 / 13.4, 19.4 / 14.5, 22.7 / 18.4), from 8192 on the register ring up to 32 rows (8192 x
+    2048 17.1 / 16.3, 22.5 / 16.3, then 21.3 / 17.3, 24.6 / 21.7).  Prompts: see :func:`big_tiles_fill`, or a short K
+    (640 x 384: always)."""
+    a = swiglu_gemm(x, w)
+    if a is not None:
+        return a
+    M, K = x.shape
+    I = w.shape[0] // 2
+    if _few_ok(x, w):
+        if 0 < M <= NARROW_MAX_M:
+            if I <= 16 * NARROW_WGS:
+                cfg = _narrow_cfg(M) if K <= 2048 and (M > 16 or I > 3072 or K <= 512) else 0
+            else:
+                cfg = 8 if M <= 32 and I >= 8192 and K % 512 == 0 else 14
+            if cfg and stream_shape_ok(M, 2 * I, K, cfg, 1) and I % (16 if cfg > 30 else 32) == 0:
+                return gemm_stream_silu(x, w, cfg)
+        elif M > DISPATCH_MAX_M and big_shape_ok(M, I, K, True) and (K <= 512 or big_tiles_fill(M, I, True)):
+            return gemm_big(x, w, silu=True)
+    return glu_clamp(linear(x, w), 1.0, math.inf, 0.0)
 
 
 def reserve_lib_workspace(dev: torch.device, claim_stream: int = None) -> None:
@@ -580,15 +666,17 @@ def big_shape_ok(M: int, N: int, K: int, silu: bool = False, splits: int = 1) ->
 
 
 def gemm_big(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None, silu: bool = False,
-             pipe: int = None, splits: int = 1) -> torch.Tensor:
+             pipe: int = None, splits: int = 1, relu2: bool = False) -> torch.Tensor:
     """``x @ w.T`` on the prefill-size MFMA kernel (csrc/kernels/gemm_big.hip:
     256 x 256 x 64 tiles, eight-phase ping-pong schedule, LDS-DMA staging;
     ``pipe`` = the VAR bits (1 = the ping-pong stagger, the default ``BIG_PIPE``;
     +2 static priority, +4 the 32x32x16-MFMA form)).  ``silu=True``: ``w`` is the gate_up weight
     [2I, K] and the result is ``silu(x @ Wg.T) * (x @ Wu.T)`` [M, I] -- the
     SwiGLU epilogue, with the unfused path's bf16 rounding of gate and up.
+    ``relu2=True``: ``max(x @ w.T, 0)^2``.
     ``splits`` > 1: K split over that many workgroups per tile (fp32 partials
     in the gemm_mid scratch, then a reduce launch)."""
+    assert not (relu2 and (silu or splits > 1))
     M, K = x.shape
     N = w.shape[0] // 2 if silu else w.shape[0]
     if not (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0
@@ -607,8 +695,8 @@ def gemm_big(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None, silu: b
         check(lib().k8s_gemm_big_split(ptr(x), x.stride(0), ptr(w), ptr(out), out.stride(0), M, N, K, var, splits,
                                        ptr(part), stream_ptr(x)), "gemm_big_split")
         return out
-    check(lib().k8s_gemm_big(ptr(x), x.stride(0), ptr(w), ptr(out), out.stride(0), M, N, K, int(silu), var,
-                             stream_ptr(x)), "gemm_big")
+    check(lib().k8s_gemm_big(ptr(x), x.stride(0), ptr(w), ptr(out), out.stride(0), M, N, K,
+                             3 if relu2 else int(silu), var, stream_ptr(x)), "gemm_big")
     return out
 
 
@@ -617,11 +705,12 @@ def stream_shape_ok(M: int, N: int, K: int, cfg: int, splits: int) -> bool:
     64-deep chunks, a slice of whole cfg-chunk loop trips, the 8-deep ring only
     up to two 16-row fragments per wave (M <= 128)."""
     # cfg 13..16: the LDS-DMA kernel with 3..6 stages (any chunk count); 23 / 24:
-    # the same on 128-column strips with 3 / 4 stages; 4 / 8: the register ring,
-    # whose loop has no partial trip
+    # the same on 128-column strips with 3 / 4 stages; 34 / 36: on 32-column strips
+    # with 4 / 6 stages (M <= 128); 4 / 8: the register ring, whose loop has no partial trip
     ok_cfg = (cfg == 4 or (cfg == 8 and M <= 128) or cfg == 13 or (cfg == 14 and M <= 192)
-              or (cfg in (15, 16) and M <= 64) or cfg == 23 or (cfg == 24 and M <= 192))
-    bn = 128 if cfg > 20 else 64
+              or (cfg in (15, 16) and M <= 64) or cfg == 23 or (cfg == 24 and M <= 192)
+              or (cfg in (34, 36) and M <= 128))
+    bn = 32 if cfg > 30 else 128 if cfg > 20 else 64
     return (ok_cfg and 0 < M <= 256 and N % bn == 0 and splits >= 1 and K % (64 * splits) == 0
             and (cfg > 10 or (K // splits // 64) % cfg == 0))
 

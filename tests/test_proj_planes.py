@@ -20,7 +20,7 @@ def rnd(*shape, seed=0):
 def test_planes_sum_to_the_product(n, k, m):
     x, w = rnd(m, k).to(BF), (rnd(n, k) * k ** -0.5).to(BF)
     y = L.proj_planes(x.cuda(), w.cuda())
-    assert y.dtype == torch.float32 and y.shape[1:] == (m, n) and y.shape[0] == L.plane_splits(m, n, k)
+    assert y.dtype == torch.float32 and y.shape[1:] == (m, n) and y.shape[0] == L.plane_plan(m, n, k)[1]
     want = x.double() @ w.double().T
     # fp32 sums of K terms of size K^(-1/2), in ranges
     assert float((y.double().sum(0).cpu() - want).abs().max()) < 4e-6 * k ** 0.5
