@@ -20,7 +20,7 @@
 namespace k8s {
 
 // ---------------------------------------------------------------------------
-// MFMA form (bf16): v_mfma_f32_16x16x32_bf16, one wave per work item, no LDS.
+// MFMA form (bf16): v_mfma_f32_16x16x32_bf16, one wave per work item.
 //
 // The latents are cached twice: c [pages][BS][R] (a key's R numbers contiguous:
 // the QK^T operand) and ct [pages][R][BS] (8 consecutive keys of one latent
@@ -34,12 +34,8 @@ namespace k8s {
 // the k-slots of the PV operand: P moves from accumulator to operand in place.
 //
 // Items ([n][4] int32: segment, first row, tokens, position of the first row's
-// token) are made on the host from the step's segments.  SPLIT (decode rows):
-// grid.y partitions of `part` keys write unnormalised partials which
-// latent_reduce merges -- the partition borders depend on the key index only,
-// never on the batch (with a window a row's partitions start at the one its first
-// visible key lies in).  Otherwise (prompt portions) a wave walks every key its
-// rows see and writes the gated, normalised output.
+// token) are made on the host from the step's segments: a wave walks every key its
+// rows see and writes the gated, normalised output.  Decode rows: token_attn.hip.
 //
 // NP: 32-number chunks of the cache row behind the latent (a score-only key part): row width R + 32 NP.
 constexpr float kLog2e = 1.4426950408889634f;
@@ -60,9 +56,6 @@ struct LatArgs {
   int window;             // 0: every key up to the row's own position
   uint16_t* out;          // element (t, h, c) at t * ost + h * osh + c
   long ost, osh;
-  float* part_o;          // [T][H][n_parts][R]
-  float* part_ml;         // [T][H][n_parts][2]
-  int n_parts, part;
   int H, HC, TPM, BS;
   float scale_log2;
 };
@@ -113,118 +106,6 @@ __device__ __forceinline__ void lat_softmax(const f32x4 (&s)[2], float scale_log
       for (int i = 0; i < 4; ++i) o[dt][i] *= ar[i];
   }
   l += psum;
-}
-
-template <int NR, int NP, int MT, bool SPLIT>
-__global__ void __launch_bounds__(256) latent_attn_mfma_kernel(LatArgs a) {
-  constexpr int R = NR * 32, ND = R / 16, NC = NR + NP, RW = R + 32 * NP;
-  const int lane = threadIdx.x & 63, r = lane & 15, h = lane >> 4;
-  // workgroups go round-robin over the 8 XCDs, each with its own L2: give every XCD a contiguous
-  // range of items (neighbouring token groups of the same sequences read the same latent pages)
-  const int per = gridDim.x >> 3;
-  const int blk = (gridDim.x & 7) == 0 ? (blockIdx.x & 7) * per + (blockIdx.x >> 3) : blockIdx.x;
-  const int item = blk * 4 + (threadIdx.x >> 6);
-  if (item >= a.n_items) return;
-  const int sg = a.items[item * 4], row0 = a.items[item * 4 + 1], ntok = a.items[item * 4 + 2],
-            pos0 = a.items[item * 4 + 3];
-  const int hc = blockIdx.z;
-  int k_begin = a.window > 0 ? max(0, pos0 - a.window + 1) : 0, k_end = pos0 + ntok;
-  if constexpr (SPLIT) {
-    const int p0 = (k_begin / a.part + blockIdx.y) * a.part;
-    k_begin = max(k_begin, p0);
-    k_end = min(k_end, p0 + a.part);
-    if (k_begin >= k_end) return;
-  }
-  // this lane's query row in every tile
-  const int tl = r / a.HC, hl = r - tl * a.HC, head = hc * a.HC + hl;
-  bf16x8 qf[MT][NC];
-  int limit[MT], lo[MT];
-  f32x4 o[MT][ND];
-  float m[MT], l[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int ti = mt * a.TPM + tl;
-    const bool valid = tl < a.TPM && ti < ntok && head < a.H;
-    limit[mt] = valid ? min(pos0 + ti + 1, k_end) : 0;
-    lo[mt] = max(k_begin, a.window > 0 ? pos0 + ti - a.window + 1 : 0);
-    const size_t rq = row0 + (valid ? ti : 0), hq = valid ? head : 0;
-#pragma unroll
-    for (int cc = 0; cc < NC; ++cc) {
-      qf[mt][cc] = ld16(cc < NR ? a.qa + rq * a.qst + hq * a.qsh + 32 * cc + 8 * h
-                                : a.qr + (rq * a.H + hq) * (32 * NP) + 32 * (cc - NR) + 8 * h);
-      if (!valid)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) qf[mt][cc][j] = (__bf16)0.f;
-    }
-#pragma unroll
-    for (int dt = 0; dt < ND; ++dt) o[mt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    m[mt] = (!SPLIT && a.sink && valid) ? a.sink[head] * kLog2e : -INFINITY;
-    l[mt] = 0.f;
-  }
-  const int* pages = a.bt + (size_t)sg * a.maxb;
-  for (int kb = k_begin & ~31; kb < k_end; kb += 32) {
-    const int page = pages[kb / a.BS], off = kb % a.BS;
-    const uint16_t* cp = a.c + (size_t)page * a.BS * RW;
-    const uint16_t* tp = a.ct + (size_t)page * R * a.BS;
-    bf16x8 kf[2][NC];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int key = off + 8 * (r >> 2) + 4 * t + (r & 3);
-#pragma unroll
-      for (int cc = 0; cc < NC; ++cc) kf[t][cc] = ld16(cp + (size_t)key * RW + 32 * cc + 8 * h);
-    }
-    const bool open = kb >= k_begin && kb + 32 <= k_end && kb + 31 <= pos0 &&
-                      (a.window <= 0 || kb >= pos0 + ntok - a.window);
-    bf16x8 pf[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      f32x4 s[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int cc = 0; cc < NC; ++cc)
-          s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][cc], qf[mt][cc], s[t], 0, 0, 0);
-      }
-      lat_softmax<ND>(s, a.scale_log2, open, kb, h, lo[mt], limit[mt], m[mt], l[mt], o[mt], pf[mt]);
-    }
-#pragma unroll
-    for (int dt = 0; dt < ND; ++dt) {
-      const bf16x8 vf = ld16(tp + (size_t)(16 * dt + r) * a.BS + off + 8 * h);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) o[mt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[mt], vf, o[mt][dt], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    float lt = l[mt];
-    lt += __shfl_xor(lt, 16, 64);
-    lt += __shfl_xor(lt, 32, 64);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int q = 4 * h + i;                       // the query row of accumulator element i
-      const int qtl = q / a.HC, qhl = q - qtl * a.HC, qhead = hc * a.HC + qhl, ti = mt * a.TPM + qtl;
-      const float lq = __shfl(lt, q, 64), mq = __shfl(m[mt], q, 64);
-      if (!(qtl < a.TPM && ti < ntok && qhead < a.H)) continue;
-      const size_t rh = (size_t)(row0 + ti) * a.H + qhead;
-      if constexpr (SPLIT) {
-        const size_t pi = rh * a.n_parts + blockIdx.y;
-#pragma unroll
-        for (int dt = 0; dt < ND; ++dt) a.part_o[pi * R + 16 * dt + r] = o[mt][dt][i];
-        if (r == 0) {
-          a.part_ml[pi * 2] = mq;
-          a.part_ml[pi * 2 + 1] = lq;
-        }
-      } else {
-        const float g = a.gate ? 1.f / (1.f + expf(-a.gate[(size_t)(row0 + ti) * a.ldg + qhead])) : 1.f;
-        const float ls = a.sink ? lq + __builtin_amdgcn_exp2f(a.sink[qhead] * kLog2e - mq) : lq;
-        const float sc = ls > 0.f ? g / ls : 0.f;
-        uint16_t* op = a.out + (size_t)(row0 + ti) * a.ost + (size_t)qhead * a.osh + r;
-#pragma unroll
-        for (int dt = 0; dt < ND; ++dt) op[16 * dt] = f2bf(o[mt][dt][i] * sc);
-      }
-    }
-  }
 }
 
 // Prompt portions: the four waves of a workgroup own four consecutive items of ONE
@@ -366,42 +247,11 @@ __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs 
   }
 }
 
-// Merge of the key partitions of decode rows: one workgroup per (row, head).
-// A row at position p has the partitions from the one its first visible key lies in to p / part.
-__global__ void __launch_bounds__(128) latent_reduce_kernel(const float* __restrict__ part_o,
-                                                            const float* __restrict__ part_ml,
-                                                            const int* __restrict__ positions,
-                                                            const float* __restrict__ gate, int ldg,
-                                                            uint16_t* __restrict__ out, int H, int R, int n_parts,
-                                                            int part, long ost, long osh, int window,
-                                                            const float* __restrict__ sink) {
-  const int row = blockIdx.x / H, head = blockIdx.x - row * H;
-  const size_t rh = (size_t)row * H + head;
-  const int pos = positions[row], lo = window > 0 ? max(0, pos - window + 1) : 0;
-  const int np = min(n_parts, pos / part - lo / part + 1);
-  const float sk = sink ? sink[head] * kLog2e : -INFINITY;
-  float mx = sk;
-  for (int p = 0; p < np; ++p) mx = fmaxf(mx, part_ml[(rh * n_parts + p) * 2]);
-  float lsum = sink ? exp2f(sk - mx) : 0.f;
-  for (int p = 0; p < np; ++p) lsum += exp2f(part_ml[(rh * n_parts + p) * 2] - mx) * part_ml[(rh * n_parts + p) * 2 + 1];
-  const float g = gate ? 1.f / (1.f + expf(-gate[(size_t)row * ldg + head])) : 1.f;
-  for (int c = threadIdx.x; c < R; c += 128) {
-    float acc = 0.f;
-    for (int p = 0; p < np; ++p)
-      acc = fmaf(exp2f(part_ml[(rh * n_parts + p) * 2] - mx), part_o[(rh * n_parts + p) * R + c], acc);
-    out[row * ost + head * osh + c] = f2bf(acc / lsum * g);
-  }
-}
-
 template <int NR, int NP>
-static int launch_lat_np(const LatArgs& a, int split, int mt2, int n_head_chunks, hipStream_t s) {
+static int launch_lat_np(const LatArgs& a, int n_head_chunks, hipStream_t s) {
   int nblk = (a.n_items + 3) / 4;
   if (nblk > 8) nblk = (nblk + 7) & ~7;   // a multiple of the XCD count (the kernels' item remap)
-  const dim3 grid(nblk, split ? a.n_parts : 1, n_head_chunks);
-  if (split) {
-    hipLaunchKernelGGL((latent_attn_mfma_kernel<NR, NP, 1, true>), grid, dim3(256), 0, s, a);
-    return (int)hipGetLastError();
-  }
+  const dim3 grid(nblk, 1, n_head_chunks);
   if (a.n_items % 4) return (int)hipErrorInvalidValue;   // prompt items come in fours per segment
   constexpr size_t lds = 2 * (size_t)(4 * NR + 2 * NP) * 64 * 16;  // two buffers of 2 (NR + NP) + R / 16 KiB
   // tiles per wave and waves per SIMD by register need: two tiles while two waves still fit a SIMD
@@ -415,11 +265,11 @@ static int launch_lat_np(const LatArgs& a, int split, int mt2, int n_head_chunks
 }
 
 template <int NR>
-static int launch_lat(const LatArgs& a, int np, int split, int mt2, int n_head_chunks, hipStream_t s) {
+static int launch_lat(const LatArgs& a, int np, int n_head_chunks, hipStream_t s) {
   switch (np) {
-    case 0: return launch_lat_np<NR, 0>(a, split, mt2, n_head_chunks, s);
-    case 1: return launch_lat_np<NR, 1>(a, split, mt2, n_head_chunks, s);
-    case 2: return launch_lat_np<NR, 2>(a, split, mt2, n_head_chunks, s);
+    case 0: return launch_lat_np<NR, 0>(a, n_head_chunks, s);
+    case 1: return launch_lat_np<NR, 1>(a, n_head_chunks, s);
+    case 2: return launch_lat_np<NR, 2>(a, n_head_chunks, s);
     default: return (int)hipErrorInvalidValue;
   }
 }
@@ -437,40 +287,32 @@ K8S_API int k8s_latent_attn_mfma_ok(int R, int RP) {
   }
 }
 
-// split = 1: decode rows (items of one token), partials + merge into out; `positions` [T] are the
-// rows' positions and n_rows the number of decode rows (the first rows of the step).
-// split = 0: prompt portions, items of up to tiles * (16 / min(H, 16)) tokens.
+// Items of up to k8s_latent_attn_mfma_ok() * (16 / min(H, 16)) tokens, in fours per segment.
 K8S_API int k8s_latent_attn_mfma(const void* qa, const void* c, const void* ct, const int* bt, int maxb,
-                                 const int* items, int n_items, const float* gate, int ldg, void* out,
-                                 float* part_o, float* part_ml, int n_parts, int part, const int* positions,
-                                 int n_rows, int H, int R, int BS, float scale, int split, int tiles,
-                                 hipStream_t s, long qst, long qsh, const void* qr, int RP, long ost, long osh,
+                                 const int* items, int n_items, const float* gate, int ldg, void* out, int H, int R,
+                                 int BS, float scale, hipStream_t s, long qst, long qsh, const void* qr, int RP, long ost, long osh,
                                  int window, const float* sink) {
   if (n_items <= 0) return 0;
-  if (!k8s_latent_attn_mfma_ok(R, RP) || BS % 32 || H <= 0 || (split && part % 32) || (RP && !qr) || window < 0 ||
+  if (!k8s_latent_attn_mfma_ok(R, RP) || BS % 32 || H <= 0 || (RP && !qr) || window < 0 ||
       qst % 8 || qsh % 8)
     return (int)hipErrorInvalidValue;
   k8s::LatArgs a;
   a.qst = qst; a.qsh = qsh; a.qr = (const uint16_t*)qr; a.ost = ost; a.osh = osh; a.window = window; a.sink = sink;
   a.qa = (const uint16_t*)qa; a.c = (const uint16_t*)c; a.ct = (const uint16_t*)ct; a.bt = bt; a.maxb = maxb;
   a.items = items; a.n_items = n_items; a.gate = gate; a.ldg = ldg; a.out = (uint16_t*)out;
-  a.part_o = part_o; a.part_ml = part_ml; a.n_parts = n_parts; a.part = part;
   a.H = H; a.HC = H < 16 ? H : 16; a.TPM = 16 / a.HC; a.BS = BS; a.scale_log2 = scale * k8s::kLog2e;
-  const int nhc = (H + a.HC - 1) / a.HC, mt2 = (!split && tiles == 2);
+  const int nhc = (H + a.HC - 1) / a.HC;
   int rc;
   switch (R / 32) {
-    case 1: rc = k8s::launch_lat<1>(a, RP / 32, split, mt2, nhc, s); break;
-    case 2: rc = k8s::launch_lat<2>(a, RP / 32, split, mt2, nhc, s); break;
-    case 3: rc = k8s::launch_lat<3>(a, RP / 32, split, mt2, nhc, s); break;
-    case 4: rc = k8s::launch_lat<4>(a, RP / 32, split, mt2, nhc, s); break;
-    case 6: rc = k8s::launch_lat<6>(a, RP / 32, split, mt2, nhc, s); break;
-    case 8: rc = k8s::launch_lat<8>(a, RP / 32, split, mt2, nhc, s); break;
-    case 12: rc = k8s::launch_lat<12>(a, RP / 32, split, mt2, nhc, s); break;
-    case 16: rc = k8s::launch_lat<16>(a, RP / 32, split, mt2, nhc, s); break;
+    case 1: rc = k8s::launch_lat<1>(a, RP / 32, nhc, s); break;
+    case 2: rc = k8s::launch_lat<2>(a, RP / 32, nhc, s); break;
+    case 3: rc = k8s::launch_lat<3>(a, RP / 32, nhc, s); break;
+    case 4: rc = k8s::launch_lat<4>(a, RP / 32, nhc, s); break;
+    case 6: rc = k8s::launch_lat<6>(a, RP / 32, nhc, s); break;
+    case 8: rc = k8s::launch_lat<8>(a, RP / 32, nhc, s); break;
+    case 12: rc = k8s::launch_lat<12>(a, RP / 32, nhc, s); break;
+    case 16: rc = k8s::launch_lat<16>(a, RP / 32, nhc, s); break;
     default: return (int)hipErrorInvalidValue;
   }
-  if (rc || !split) return rc;
-  hipLaunchKernelGGL(k8s::latent_reduce_kernel, dim3(n_rows * H), dim3(128), 0, s, part_o, part_ml, positions, gate, ldg,
-                     (uint16_t*)out, H, R, n_parts, part, ost, osh, window, sink);
-  return (int)hipGetLastError();
+  return rc;
 }

@@ -1,0 +1,489 @@
+// Attention of single tokens (decode rows) over paged keys, bf16 on v_mfma_f32_16x16x32_bf16: for the masked layers
+// (masked_attn.hip) and the latent ones (latent_attn.hip).
+//
+// One token has one position, so the tile of 16 query rows those kernels give to tokens goes to the HEADS that share a
+// key head here: up to 16 heads read a key's bytes once.  A workgroup owns (row, key head, part of the row's keys) and
+// its waves take the part's 32-key blocks in turn (wave w: blocks w, w + NW, ..), each with an online softmax of its own;
+// the waves' maxima, sums and outputs meet in LDS and are added in wave order.  A row whose keys fit one part is
+// finished there (sink, gate, rounding); otherwise token_merge_kernel joins the parts with the same arithmetic.  Blocks,
+// waves and parts follow from positions alone, so a row's bits do not depend on the step it is in.
+//
+// What bounds it: the chain row -> page -> keys -> scores -> join of some 5 us, and that one compute unit takes cold keys
+// in at 20 to 30 KB a us, far below its share of the caches' rate.  So parts are small (256 masked or 128 latent keys: 64
+// and 144 KB), and a merge of 3.5 us pays from the second part on.  16 heads over 2 of 128 / 16 heads over latents of
+// 256 + 64, us with the merge, and in brackets what a tile of 16 tokens per wave (masked) and a wave per 256 keys (latent)
+// took in engine steps of about that size: 1 row at 100 keys 5.3 / 8.5 (8.4 / 13.5), 8 rows at 1500 10.7 / 12.5 (26 / 36),
+// 64 rows at 400 12.3 / 14.3 (28 / 35).
+#include "common.h"
+#include "key_runs.h"
+
+namespace k8s {
+
+constexpr float kTokLog2e = 1.4426950408889634f;
+
+struct TokOut {
+  const float* sink;      // [H] or null
+  const float* gate;      // rows of stride gs, column h, or null
+  int gs;
+  uint16_t* out;          // element (row, h, c) at row * ost + h * osh + c
+  float* out32;           // the same in fp32 instead
+  long ost, osh;
+  float* po;              // [items][H][parts][V]: a part's unnormalised output
+  float* pml;             // [items][H][parts][2]: its maximum (log2 units) and denominator
+  int H, n_parts;
+};
+
+// 1 / denominator (sink included) times the gate; w: the factor of the outputs
+__device__ __forceinline__ float tok_finish(const TokOut& a, int row, int head, float m, float l, float& w) {
+  const float sk = a.sink ? a.sink[head] * kTokLog2e : -INFINITY;
+  const float M = fmaxf(m, sk);
+  w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+  const float L = l * w + (a.sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f);
+  const float g = a.gate ? 1.f / (1.f + expf(-a.gate[(size_t)row * a.gs + head])) : 1.f;
+  return L > 0.f ? g / L : 0.f;
+}
+
+__device__ __forceinline__ void tok_store4(const TokOut& a, int row, int head, int c, const f32x4& v) {
+  const size_t o = (size_t)row * a.ost + (size_t)head * a.osh + c;       // V, the strides: multiples of 16
+  if (a.out32)
+    *reinterpret_cast<f32x4*>(a.out32 + o) = v;
+  else
+    *reinterpret_cast<u16x4*>(a.out + o) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+}
+
+template <int NW, int V>
+struct TokLds {
+  static constexpr int P = V + 4;    // row pitch: the four rows a store instruction writes lie 16 banks apart
+  alignas(16) float o[NW][16][P];
+  float ml[NW][16][2];
+};
+
+// The waves' heads -> LDS -> out or a part.  m, l: of head lane & 15, l already summed over the lane quarters.
+// o[dt][i]: head 4 (lane >> 4) + i, column 16 dt + (lane & 15).  A wave without a block brings m = -inf and zeros.
+// Four columns a thread and every wave's numbers read at once: with a column a thread and a loop over the waves the join
+// was the larger part of the kernel (latent, 32 keys a part: 18.9 us).
+template <int NW, int ND>
+__device__ __forceinline__ void tok_join(TokLds<NW, ND * 16>& s, const TokOut& a, int row, int head0, int nh, int part,
+                                         float m, float l, const f32x4 (&o)[ND]) {
+  constexpr int V = ND * 16;
+  const int lane = threadIdx.x & 63, r = lane & 15, hq = lane >> 4, wv = threadIdx.x >> 6;
+  if (hq == 0) {
+    s.ml[wv][r][0] = m;
+    s.ml[wv][r][1] = l;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (4 * hq + i < nh) {
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt) s.o[wv][4 * hq + i][16 * dt + r] = o[dt][i];
+    }
+  __syncthreads();
+  for (int e = threadIdx.x; e < nh * (V / 4); e += 64 * NW) {
+    const int hh = e / (V / 4), c = 4 * (e % (V / 4)), head = head0 + hh;
+    float mw[NW], lw[NW];
+    f32x4 ow[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      mw[w] = s.ml[w][hh][0];
+      lw[w] = s.ml[w][hh][1];
+      ow[w] = *reinterpret_cast<const f32x4*>(&s.o[w][hh][c]);
+    }
+    float M = mw[0], L = 0.f;
+#pragma unroll
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, mw[w]);
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw[w] - M);   // -inf: no visible key
+      L = fmaf(lw[w], f, L);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] = fmaf(ow[w][k], f, acc[k]);
+    }
+    if (a.n_parts > 1) {
+      const size_t pi = ((size_t)blockIdx.x * a.H + head) * a.n_parts + part;
+      *reinterpret_cast<f32x4*>(a.po + pi * V + c) = acc;
+      if (c == 0) {
+        a.pml[pi * 2] = M;
+        a.pml[pi * 2 + 1] = L;
+      }
+    } else {
+      float w;
+      const float f = tok_finish(a, row, head, M, L, w);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] *= w * f;
+      tok_store4(a, row, head, c, acc);
+    }
+  }
+}
+
+// a part without keys
+__device__ __forceinline__ void tok_empty(const TokOut& a, int head0, int nh, int part) {
+  if ((int)threadIdx.x < nh) {
+    float* ml = a.pml + (((size_t)blockIdx.x * a.H + head0 + threadIdx.x) * a.n_parts + part) * 2;
+    ml[0] = -INFINITY;
+    ml[1] = 0.f;
+  }
+}
+
+// One workgroup per (row, head).  Group j of V / 4 threads adds the parts j, j + S, .. (S groups), the groups' sums are
+// added in order.  Nothing but the sum waits for anything: the first parts are on their way while the maxima arrive.
+__global__ void __launch_bounds__(256) token_merge_kernel(TokOut a, const int* __restrict__ items, int V) {
+  constexpr int U = 4;
+  __shared__ f32x4 sum[256];
+  const int it = blockIdx.x / a.H, head = blockIdx.x % a.H, lane = threadIdx.x & 63, np = a.n_parts;
+  const int row = items[it * 4 + 1], W = V / 4, S = 256 / W, j = threadIdx.x / W, c = threadIdx.x % W;
+  const size_t p0 = (size_t)blockIdx.x * np;
+  const f32x4* po = reinterpret_cast<const f32x4*>(a.po + p0 * V) + c;
+  const float* ml = a.pml + p0 * 2;
+  const bool on = j < S;
+  f32x4 v[U];
+  float mv[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int p = j + S * u;
+    const bool has = on && p < np;
+    v[u] = po[(size_t)(has ? p : 0) * W];
+    mv[u] = has ? ml[p * 2] : -INFINITY;
+  }
+  float M = -INFINITY, L = 0.f;
+  for (int p = lane; p < np; p += 64) M = fmaxf(M, ml[p * 2]);
+  M = wave_max(M);
+  for (int p = lane; p < np; p += 64) {
+    const float m = ml[p * 2];
+    if (m != -INFINITY) L = fmaf(ml[p * 2 + 1], __builtin_amdgcn_exp2f(m - M), L);
+  }
+  L = wave_sum(L);
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto add = [&](const f32x4& x, float m) {
+    if (m == -INFINITY) return;                            // a part without a visible key (its output was not written)
+    const float f = __builtin_amdgcn_exp2f(m - M);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[k] = fmaf(x[k], f, acc[k]);
+  };
+#pragma unroll
+  for (int u = 0; u < U; ++u) add(v[u], mv[u]);
+  if (on)
+    for (int p = j + S * U; p < np; p += S) add(po[(size_t)p * W], ml[p * 2]);
+  sum[threadIdx.x] = acc;
+  __syncthreads();
+  if (j > 0) return;
+  for (int g = 1; g < S; ++g) acc += sum[g * W + c];
+  float w;
+  const float f = tok_finish(a, row, head, M, L, w);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) acc[k] *= w * f;
+  tok_store4(a, row, head, 4 * c, acc);
+}
+
+__device__ __forceinline__ bf16x8 tld16(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
+
+// Scores p[8] (log2 units, keys 8 h .. 8 h + 7 of head lane & 15; -inf: not seen) -> the running maximum and sum, the
+// weights as the value product's operand; the output is rescaled only where a head's maximum moved.
+template <int ND>
+__device__ __forceinline__ void tok_softmax(const float (&p)[8], int hq, float& m, float& l, f32x4 (&o)[ND], bf16x8& pf) {
+  float cmax = p[0];
+#pragma unroll
+  for (int j = 1; j < 8; ++j) cmax = fmaxf(cmax, p[j]);
+  cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
+  cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+  const bool grow = cmax > m;
+  const float mn = grow ? cmax : m, ms = mn == -INFINITY ? 0.f : mn;
+  float ps = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float e = __builtin_amdgcn_exp2f(p[j] - ms);
+    ps += e;
+    pf[j] = (__bf16)e;
+  }
+  if (__any(grow)) {
+    const float alpha = __builtin_amdgcn_exp2f(m - ms);
+    l *= alpha;
+    m = mn;
+    float ai[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ai[i] = __shfl(alpha, 4 * hq + i, 64);
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[dt][i] *= ai[i];
+  }
+  l += ps;
+}
+
+struct MaskTokArgs {
+  const uint16_t* q;      // [T][H * D]
+  const uint16_t* kc;     // [pages][BS][G * D]
+  const uint16_t* vt;     // [pages][G * V][BS]
+  const int* bt;
+  int maxb;
+  const int* items;       // [rows][4]: segment, row, 1, position
+  int G, BS, chunk, window, keep_first, part_blocks, most;   // a part: part_blocks, or more where most parts are too few
+  float scale, softcap;
+  TokOut t;
+};
+
+// grid (rows, key heads x groups of 16 of their heads, parts); a part is a run of the row's list of 32-key blocks
+// (kept first tokens, then the window's or chunk's).
+template <int NDC, int NV, bool CAP>
+__global__ void __launch_bounds__(512) masked_attn_token_kernel(MaskTokArgs a) {
+  constexpr int D = NDC * 32, V = NV * 16, NW = 8;
+  __shared__ TokLds<NW, V> lds;
+  const int lane = threadIdx.x & 63, r = lane & 15, hq = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sg = a.items[blockIdx.x * 4], row = a.items[blockIdx.x * 4 + 1], pos = a.items[blockIdx.x * 4 + 3];
+  const int H = a.t.H, hpg = H / a.G, nhc = (hpg + 15) / 16, g = blockIdx.y / nhc, hc = blockIdx.y % nhc;
+  const int head0 = g * hpg + 16 * hc, nh = min(16, hpg - 16 * hc), NK = a.G * D, NVt = a.G * V;
+  const int keep = a.window > 0 ? a.keep_first : 0;
+  const KeyRuns k0 = key_runs(pos, a.chunk, a.window, a.keep_first);
+  const int lo_al = k0.lo & ~31, a_beg = k0.a0 & ~31;
+  const int a_end = a.window > 0 ? min(lo_al, (a.keep_first + 31) & ~31) : a_beg;
+  const int nblkA = max(0, (a_end - a_beg) >> 5), nblk = nblkA + ((pos - lo_al) >> 5) + 1;
+  const int pb = max(a.part_blocks, (nblk + a.most - 1) / a.most), b_lo = (int)blockIdx.z * pb;
+  const int nb = min(nblk, b_lo + pb) - b_lo;
+  if (nb <= 0) {                                           // the whole workgroup (parts of a longer row's step)
+    tok_empty(a.t, head0, nh, blockIdx.z);
+    return;
+  }
+  bf16x8 qf[NDC];
+  const uint16_t* qp = a.q + (size_t)row * H * D + (size_t)(head0 + min(r, nh - 1)) * D;
+#pragma unroll
+  for (int cc = 0; cc < NDC; ++cc) qf[cc] = tld16(qp + 32 * cc + 8 * hq);
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[NV];
+#pragma unroll
+  for (int dt = 0; dt < NV; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float sc2 = a.scale * kTokLog2e, cap2 = a.softcap * kTokLog2e, icap = a.softcap > 0.f ? a.scale / a.softcap : 0.f;
+  const int* pages = a.bt + (size_t)sg * a.maxb;
+  const int my = (nb - wv + NW - 1) / NW;                  // this wave's blocks (<= 0: none)
+  // lane i holds the first key, the page and the place in it of the wave's block base + i
+  int base = 0, kbv = 0, pgv = 0, ofv = 0;
+  auto fill = [&](int k) {
+    base = k;
+    const int bi = b_lo + wv + NW * (k + lane);
+    kbv = bi < nblkA ? a_beg + 32 * bi : lo_al + 32 * (bi - nblkA);
+    const int pi = kbv / a.BS;
+    ofv = kbv - pi * a.BS;
+    pgv = k + lane < my ? pages[pi] : 0;
+  };
+  fill(0);
+  bf16x8 kf[2][2][NDC], vf[2][NV];
+  int kb[2];
+  auto load = [&](int u, int k) {
+    if (k - base == 64) fill(k);
+    kb[u] = __shfl(kbv, k - base, 64);
+    const int page = __shfl(pgv, k - base, 64), off = __shfl(ofv, k - base, 64);
+    const uint16_t* kp = a.kc + ((size_t)page * a.BS + off) * NK + g * D + 8 * hq;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int cc = 0; cc < NDC; ++cc) kf[u][t][cc] = tld16(kp + (size_t)(8 * (r >> 2) + 4 * t + (r & 3)) * NK + 32 * cc);
+    const uint16_t* vp = a.vt + ((size_t)page * NVt + (size_t)g * V) * a.BS + off + 8 * hq;
+#pragma unroll
+    for (int dt = 0; dt < NV; ++dt) vf[u][dt] = tld16(vp + (size_t)(16 * dt + r) * a.BS);
+  };
+  if (my > 0) load(0, 0);
+  if (my > 1) load(1, 1);
+  const int cq_lo = a.chunk > 0 ? (pos / a.chunk) * a.chunk : 0, wq_lo = a.window > 0 ? pos - a.window + 1 : 0;
+  for (int k = 0; k < my; k += 2) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (k + u >= my) break;
+      float p[8];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int cc = 0; cc < NDC; ++cc) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[u][t][cc], qf[cc], s, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[4 * t + i] = s[i];
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = kb[u] + 8 * hq + j;
+        if (CAP) {                                         // cap tanh(x), tanh(x) = 1 - 2 / (1 + e^(2x)), in log2 units
+          const float e = __builtin_amdgcn_exp2f(fminf(p[j] * icap * (2.f * kTokLog2e), 60.f));
+          p[j] = cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + e));
+        } else {
+          p[j] *= sc2;
+        }
+        p[j] = key <= pos && key >= cq_lo && (key >= wq_lo || key < keep) ? p[j] : -INFINITY;
+      }
+      bf16x8 pf;
+      tok_softmax<NV>(p, hq, m, l, o, pf);
+#pragma unroll
+      for (int dt = 0; dt < NV; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, vf[u][dt], o[dt], 0, 0, 0);
+      if (k + u + 2 < my) load(u, k + u + 2);
+    }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  tok_join<NW, NV>(lds, a.t, row, head0, nh, blockIdx.z, m, l, o);
+}
+
+struct LatTokArgs {
+  const uint16_t* qa;     // element (row, h, c) at row * qst + h * qsh + c
+  long qst, qsh;
+  const uint16_t* qr;     // [T][H][32 NP]
+  const uint16_t* c;      // [pages][BS][R + 32 NP]
+  const uint16_t* ct;     // [pages][R][BS]
+  const int* bt;
+  int maxb;
+  const int* items;       // [rows][4]: segment, row, 1, position
+  int BS, window, part, most;   // a part: `part` keys, or more where most parts are too few
+  float scale_log2;
+  TokOut t;
+};
+
+// grid (rows, parts, groups of 16 heads); parts are ranges of the key index (a row's first one is that of its first
+// visible key).
+template <int NR, int NP, int NW>
+__global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a) {
+  constexpr int R = NR * 32, ND = R / 16, NC = NR + NP, RW = R + 32 * NP, NH = ND / 2;
+  __shared__ TokLds<NW, R> lds;
+  const int lane = threadIdx.x & 63, r = lane & 15, hq = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sg = a.items[blockIdx.x * 4], row = a.items[blockIdx.x * 4 + 1], pos = a.items[blockIdx.x * 4 + 3];
+  const int H = a.t.H, head0 = 16 * blockIdx.z, nh = min(16, H - head0);
+  const int lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  const int first = lo / a.part * a.part, part = max(a.part, ((pos + a.most - first) / a.most + 31) & ~31);
+  const int p0 = first + (int)blockIdx.y * part, k_begin = max(lo, p0), k_end = min(pos + 1, p0 + part);
+  if (k_begin >= k_end) {                                  // the whole workgroup
+    tok_empty(a.t, head0, nh, blockIdx.y);
+    return;
+  }
+  const int kb0 = k_begin & ~31, nb = (k_end - kb0 + 31) >> 5;
+  bf16x8 qf[NC];
+  const size_t hl = head0 + min(r, nh - 1);
+#pragma unroll
+  for (int cc = 0; cc < NC; ++cc)
+    qf[cc] = tld16(cc < NR ? a.qa + row * a.qst + hl * a.qsh + 32 * cc + 8 * hq
+                           : a.qr + ((size_t)row * H + hl) * (32 * NP) + 32 * (cc - NR) + 8 * hq);
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[ND];
+#pragma unroll
+  for (int dt = 0; dt < ND; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int* pages = a.bt + (size_t)sg * a.maxb;
+  for (int b = wv; b < nb; b += NW) {
+    const int kb = kb0 + 32 * b, page = pages[kb / a.BS], off = kb % a.BS;
+    const uint16_t* cp = a.c + (size_t)page * a.BS * RW;
+    const uint16_t* tp = a.ct + (size_t)page * R * a.BS + (size_t)r * a.BS + off + 8 * hq;
+    bf16x8 kf[2][NC], vf[ND];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc)
+        kf[t][cc] = tld16(cp + (size_t)(off + 8 * (r >> 2) + 4 * t + (r & 3)) * RW + 32 * cc + 8 * hq);
+#pragma unroll
+    for (int dt = 0; dt < NH; ++dt) vf[dt] = tld16(tp + (size_t)(16 * dt) * a.BS);
+    float p[8];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][cc], qf[cc], s, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = kb + 8 * hq + 4 * t + i;
+        p[4 * t + i] = key < k_end && key >= k_begin ? s[i] * a.scale_log2 : -INFINITY;
+      }
+    }
+    // the second half of the values takes the registers the keys leave
+#pragma unroll
+    for (int dt = NH; dt < ND; ++dt) vf[dt] = tld16(tp + (size_t)(16 * dt) * a.BS);
+    bf16x8 pf;
+    tok_softmax<ND>(p, hq, m, l, o, pf);
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, vf[dt], o[dt], 0, 0, 0);
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  tok_join<NW, ND>(lds, a.t, row, head0, nh, blockIdx.y, m, l, o);
+}
+
+template <int NDC, int NV>
+static int launch_mask_tok(const MaskTokArgs& a, int rows, hipStream_t s) {
+  const int hpg = a.t.H / a.G;
+  const dim3 grid(rows, a.G * ((hpg + 15) / 16), a.t.n_parts);
+  if (a.softcap > 0.f)
+    hipLaunchKernelGGL((masked_attn_token_kernel<NDC, NV, true>), grid, dim3(512), 0, s, a);
+  else
+    hipLaunchKernelGGL((masked_attn_token_kernel<NDC, NV, false>), grid, dim3(512), 0, s, a);
+  if (a.t.n_parts > 1)
+    hipLaunchKernelGGL(token_merge_kernel, dim3(rows * a.t.H), dim3(256), 0, s, a.t, a.items, NV * 16);
+  return (int)hipGetLastError();
+}
+
+template <int NR>
+static int launch_lat_tok(const LatTokArgs& a, int np, int rows, hipStream_t s) {
+  constexpr int NW = 4;
+  const dim3 grid(rows, a.t.n_parts, (a.t.H + 15) / 16);
+  switch (np) {
+    case 0: hipLaunchKernelGGL((latent_attn_token_kernel<NR, 0, NW>), grid, dim3(64 * NW), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((latent_attn_token_kernel<NR, 1, NW>), grid, dim3(64 * NW), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((latent_attn_token_kernel<NR, 2, NW>), grid, dim3(64 * NW), 0, s, a); break;
+    default: return (int)hipErrorInvalidValue;
+  }
+  if (a.t.n_parts > 1)
+    hipLaunchKernelGGL(token_merge_kernel, dim3(rows * a.t.H), dim3(256), 0, s, a.t, a.items, NR * 32);
+  return (int)hipGetLastError();
+}
+
+}  // namespace k8s
+
+using namespace k8s;
+
+K8S_API int k8s_masked_attn_mfma_ok(int H, int G, int D, int V);
+K8S_API int k8s_latent_attn_mfma_ok(int R, int RP);
+
+// items [rows][4]; n_parts > 1: po [rows][H][n_parts][V], pml [rows][H][n_parts][2]
+K8S_API int k8s_masked_attn_token(const void* q, const void* kc, const void* vt, const int* bt, int maxb,
+                                  const int* items, int rows, const float* sink, const float* gate, int gs, void* out,
+                                  int H, int G, int D, int V, int BS, int chunk, int window, int keep_first, float scale,
+                                  float softcap, hipStream_t s, int part_blocks, int most, int n_parts, float* pml,
+                                  float* po, int out_f32) {
+  if (rows <= 0) return 0;
+  if (!k8s_masked_attn_mfma_ok(H, G, D, V) || BS % 32 || chunk < 0 || window < 0 || keep_first < 0 || n_parts < 1 ||
+      part_blocks < 1 || most < 1 || n_parts > most || (n_parts > 1 && (!pml || !po)))
+    return (int)hipErrorInvalidValue;
+  MaskTokArgs a;
+  a.q = (const uint16_t*)q; a.kc = (const uint16_t*)kc; a.vt = (const uint16_t*)vt; a.bt = bt; a.maxb = maxb;
+  a.items = items; a.G = G; a.BS = BS; a.chunk = chunk; a.window = window; a.keep_first = keep_first;
+  a.part_blocks = part_blocks; a.most = most; a.scale = scale; a.softcap = softcap;
+  a.t.sink = sink; a.t.gate = gate; a.t.gs = gs; a.t.out = out_f32 ? nullptr : (uint16_t*)out;
+  a.t.out32 = out_f32 ? (float*)out : nullptr; a.t.ost = (long)H * V; a.t.osh = V; a.t.po = po; a.t.pml = pml;
+  a.t.H = H; a.t.n_parts = n_parts;
+  if (D == 96) return launch_mask_tok<3, 6>(a, rows, s);
+  if (D == 64 && V == 64) return launch_mask_tok<2, 4>(a, rows, s);
+  if (D == 64 && V == 128) return launch_mask_tok<2, 8>(a, rows, s);
+  if (D == 128 && V == 64) return launch_mask_tok<4, 4>(a, rows, s);
+  return launch_mask_tok<4, 8>(a, rows, s);
+}
+
+// items [rows][4]; n_parts > 1: po [rows][H][n_parts][R], pml [rows][H][n_parts][2]
+K8S_API int k8s_latent_attn_token(const void* qa, long qst, long qsh, const void* qr, int RP, const void* c, const void* ct,
+                                  const int* bt, int maxb, const int* items, int rows, const float* gate, int ldg,
+                                  const float* sink, void* out, long ost, long osh, float* po, float* pml, int n_parts,
+                                  int part, int most, int H, int R, int BS, int window, float scale, hipStream_t s) {
+  if (rows <= 0) return 0;
+  if (!k8s_latent_attn_mfma_ok(R, RP) || BS % 32 || H <= 0 || n_parts < 1 || n_parts > most || part <= 0 || part % 32 || (RP && !qr) ||
+      window < 0 || qst % 8 || qsh % 8 || (n_parts > 1 && (!pml || !po)))
+    return (int)hipErrorInvalidValue;
+  LatTokArgs a;
+  a.qa = (const uint16_t*)qa; a.qst = qst; a.qsh = qsh; a.qr = (const uint16_t*)qr; a.c = (const uint16_t*)c;
+  a.ct = (const uint16_t*)ct; a.bt = bt; a.maxb = maxb; a.items = items; a.BS = BS; a.window = window; a.part = part;
+  a.most = most;
+  a.scale_log2 = scale * kTokLog2e;
+  a.t.sink = sink; a.t.gate = gate; a.t.gs = ldg; a.t.out = (uint16_t*)out; a.t.out32 = nullptr; a.t.ost = ost;
+  a.t.osh = osh; a.t.po = po; a.t.pml = pml; a.t.H = H; a.t.n_parts = n_parts;
+  switch (R / 32) {
+    case 1: return launch_lat_tok<1>(a, RP / 32, rows, s);
+    case 2: return launch_lat_tok<2>(a, RP / 32, rows, s);
+    case 3: return launch_lat_tok<3>(a, RP / 32, rows, s);
+    case 4: return launch_lat_tok<4>(a, RP / 32, rows, s);
+    case 6: return launch_lat_tok<6>(a, RP / 32, rows, s);
+    case 8: return launch_lat_tok<8>(a, RP / 32, rows, s);
+    case 12: return launch_lat_tok<12>(a, RP / 32, rows, s);
+    case 16: return launch_lat_tok<16>(a, RP / 32, rows, s);
+    default: return (int)hipErrorInvalidValue;
+  }
+}

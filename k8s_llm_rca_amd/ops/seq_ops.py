@@ -25,8 +25,12 @@ import torch
 
 from ._lib import check, lib, ptr, scratch, stream_ptr, use_hip
 
-DECODE_PART = 256   # keys per partition of a decode row (split-KV); borders depend on the key index only
-WINDOW_DECODE_PART = 128   # the same where a window bounds a row's keys
+# Parts a single token's keys are cut into, a workgroup each (csrc/kernels/token_attn.hip).  us at parts of half the size /
+# this / twice: masked, 1 row at 200 keys 8.9 / 6.5 / 6.5, at 4000 9.1 / 10.5 / 14.4, 64 rows at 400 14.7 / 12.3 / 10.4, at
+# 1500 34.6 / 27.5 / 28.0;  latent, 1 row at 200 9.3 / 11.5 / 11.5, at 4000 15.7 / 14.1 / 15.8, 64 at 400 17.5 / 14.3 / 17.6.
+MASK_TOKEN_BLOCKS = 8    # 32-key blocks of the row's own list
+LATENT_PART = 128        # keys, from the part of the row's first visible key on
+TOKEN_PARTS = 64         # a row with more than so many of them has larger ones: the partial results stay bounded
 
 
 @dataclass
@@ -386,24 +390,23 @@ def latent_attention_mfma(qa: torch.Tensor, cache: torch.Tensor, cache_t: torch.
     L, st = lib(), stream_ptr(qa)
     bt, maxb = seg.block_tables, seg.block_tables.shape[1]
     gs = gate.stride(0) if gate is not None else 0
-    more = (qa.stride(0), qa.stride(1), ptr(qr), W - R, out.stride(0), out.stride(1), int(window), ptr(sink))
     if dec.shape[0]:
-        part = DECODE_PART
+        part = LATENT_PART
         n_parts = -(-kmax // part)
         if window > 0:      # a row's parts start at the one its first visible key lies in
-            part = WINDOW_DECODE_PART
-            n_parts = min(-(-kmax // part), (min(int(window), kmax) + part - 2) // part + 1)
-        nd = seg.n_single
-        part_o = scratch(nd * H * n_parts * R, torch.float32, qa.device)
-        part_ml = scratch(nd * H * n_parts * 2, torch.float32, qa.device)
-        check(L.k8s_latent_attn_mfma(ptr(qa), ptr(cache), ptr(cache_t), ptr(bt), maxb, ptr(dec), dec.shape[0],
-                                     ptr(gate), gs, ptr(out), ptr(part_o), ptr(part_ml), n_parts,
-                                     part, ptr(positions), nd, H, R, BS, float(scale), 1, 1, st, *more),
-              "latent_attn_mfma (decode)")
+            n_parts = min(n_parts, (min(int(window), kmax) + part - 2) // part + 1)
+        n_parts = min(n_parts, TOKEN_PARTS)
+        po = pml = None
+        if n_parts > 1:
+            po, pml = (scratch(dec.shape[0] * H * n_parts * n, torch.float32, qa.device) for n in (R, 2))
+        check(L.k8s_latent_attn_token(ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), W - R, ptr(cache), ptr(cache_t),
+                                      ptr(bt), maxb, ptr(dec), dec.shape[0], ptr(gate), gs, ptr(sink), ptr(out),
+                                      out.stride(0), out.stride(1), ptr(po), ptr(pml), n_parts, part, TOKEN_PARTS, H,
+                                      R, BS, int(window), float(scale), st), "latent_attn_token")
     if pre.shape[0]:
-        check(L.k8s_latent_attn_mfma(ptr(qa), ptr(cache), ptr(cache_t), ptr(bt), maxb, ptr(pre), pre.shape[0],
-                                     ptr(gate), gs, ptr(out), None, None, 1, DECODE_PART, None, 0,
-                                     H, R, BS, float(scale), 0, tiles, st, *more), "latent_attn_mfma (prefill)")
+        check(L.k8s_latent_attn_mfma(ptr(qa), ptr(cache), ptr(cache_t), ptr(bt), maxb, ptr(pre), pre.shape[0], ptr(gate),
+                                     gs, ptr(out), H, R, BS, float(scale), st, qa.stride(0), qa.stride(1), ptr(qr), W - R,
+                                     out.stride(0), out.stride(1), int(window), ptr(sink)), "latent_attn_mfma")
     return out
 
 
@@ -1030,7 +1033,23 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
             assert vt.is_contiguous() and vt.shape[1:] == (G * V, BS) and BS % 32 == 0
             items = seg.tile_items(WINDOW_TILE)
             n_items = items.shape[0]
-            # steps of few rows (decoding): a tile's key blocks are split over workgroups as well -- parts of
+            if T == seg.n_seg and maps == 1:
+                kmax = max(seg.pos0_host) + 1
+                nblk = -(-kmax // 32)
+                if window > 0:     # the window from a block's border on; + the kept blocks
+                    nblk = min(nblk, (int(window) + 62) // 32 + -(-int(keep_first) // 32))
+                if chunk > 0:
+                    nblk = min(nblk, (int(chunk) + 62) // 32)
+                n_parts, po, pml = min(-(-nblk // MASK_TOKEN_BLOCKS), TOKEN_PARTS), None, None
+                if n_parts > 1:
+                    po, pml = (scratch(T * H * n_parts * n, torch.float32, q.device) for n in (V, 2))
+                check(lib().k8s_masked_attn_token(ptr(q), ptr(kc), ptr(vt), ptr(seg.block_tables),
+                                                  seg.block_tables.shape[1], ptr(items), T, ptr(sink), ptr(gate), gs,
+                                                  ptr(out), H, G, D, V, BS, int(chunk), int(window), int(keep_first),
+                                                  float(scale), float(softcap), stream_ptr(q), MASK_TOKEN_BLOCKS,
+                                                  TOKEN_PARTS, n_parts, ptr(pml), ptr(po), int(out_f32)), "masked_attn_token")
+                return out
+            # steps of few rows: a tile's key blocks are split over workgroups as well -- parts of
             # MASK_PART_BLOCKS blocks of the tile's own block list (at most MASK_MAX_PARTS parts), then a merge
             # (more tiles than that only where they are single tokens: a prompt's parts would be all traffic)
             n_parts, pb, pml, po = 1, MASK_PART_BLOCKS, None, None
