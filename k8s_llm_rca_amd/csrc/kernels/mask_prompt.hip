@@ -1,0 +1,291 @@
+// Prompt portions of the masked attention (masked_attn.hip: causal, chunked, windowed with kept first tokens, sinks,
+// capped scores, output gates, score maps) with the heads of a key head as rows of one tile.
+//
+// A workgroup is 4 waves x 32 rows (token, head of the key head): 128 / heads tokens.  Keys go in blocks of 64 whose
+// 32-key halves do not cross a page (BS % 32 == 0), fetched into registers while the block before is computed and parked in LDS (two
+// buffers, one barrier per block), so a byte of K and V leaves the caches once per 128 rows.  v_mfma_f32_32x32x16_bf16,
+// swapped: S^T = K Q^T, a lane owns query row lane & 31; MFMA row rho of a 32-key half stands for key
+// 16 (reg >> 3) + 8 hi + (reg & 7), reg = (rho & 3) + 4 (rho >> 3), hi = (rho >> 2) & 1, so that a lane's score
+// registers 8 s .. 8 s + 7 are the weights operand of O^T = V^T P^T as they stand.  LDS rows are padded by 16 bytes: the
+// 16 rows a quarter wave reads 16 bytes of lie in different banks for D = 64, 96 and 128 alike.
+//
+// What bounds it: matrix and vector instructions of two waves a SIMD in turn (240 registers).  Eight prompts of 2048, 16
+// heads over 2 of 128, us: causal 245 = 561 TFLOP/s, a window of 1024 180 = 574, chunks of 1024 with capped scores 170 =
+// 405 (an exponential and a reciprocal more per score).  Tiles of 16 tokens x 2 heads a wave with operands from the caches
+// took 681, 485 and 418: every wave fetched its keys itself.
+#include "common.h"
+#include "key_runs.h"
+
+namespace k8s {
+
+struct MaskPromptArgs {
+  const uint16_t* q;      // [T][H M D]
+  const uint16_t* kc;     // [pages][BS][G M D]
+  const uint16_t* vt;     // [pages][G V][BS]
+  const int* bt;
+  int maxb;
+  const int* items;       // [n][4]: segment, first row, tokens (<= max(1, 128 / (H / G))), position of the first token
+  int n_items;
+  const float* sink;      // [H M] or null
+  const float* gate;      // rows of stride gs, column h, or null
+  int gs;
+  uint16_t* out;          // [T][H M V]
+  float* out32;           // the same in fp32 instead
+  int H, G, M, BS, chunk, window, keep_first;    // H: heads (each with M maps)
+  float scale, softcap;
+};
+
+__device__ __forceinline__ int mp_key(int reg, int hi) { return 16 * (reg >> 3) + 8 * hi + (reg & 7); }
+
+// HALF: BS is an odd multiple of 32, a block's halves may lie in two pages.
+template <int ND, int NV, int NW, bool CAP, bool HALF>
+__global__ void __launch_bounds__(64 * NW, 8 / NW) mask_prompt_kernel(MaskPromptArgs a) {
+  constexpr int D = ND * 16, V = NV * 32, TH = 64 * NW, KP = D * 2 + 16, VP = 144;
+  constexpr int KC = 64 * D / 8 / TH, VC = V * 8 / TH;      // 16-byte chunks per thread and block
+  static_assert(64 * D / 8 % TH == 0 && V * 8 % TH == 0, "whole chunks per thread");
+  constexpr float kLog2e = 1.4426950408889634f;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2][64 * KP + V * VP];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 31, hi = lane >> 5;
+  // key heads (and groups of 128 of their heads) next to each other, the last items first: they see the most keys
+  const int hpg = a.H / a.G, hw = min(hpg, 32 * NW), nhc = (hpg + hw - 1) / hw, per = a.G * a.M * nhc;
+  const int kh = blockIdx.x % per / nhc, hc = blockIdx.x % nhc, gv = kh / a.M, mp = kh % a.M;
+  const int item = a.n_items - 1 - blockIdx.x / per;
+  const int sg = a.items[item * 4], row0 = a.items[item * 4 + 1], ntok = a.items[item * 4 + 2],
+            pos0 = a.items[item * 4 + 3];
+  const int HM = a.H * a.M, NK = a.G * a.M * D, NVt = a.G * V;
+  const int grow = w * 32 + r, tt = grow / hw, hh = hc * hw + grow % hw, head = (gv * hpg + hh) * a.M + mp;
+  const bool valid = tt < ntok && hh < hpg;
+  const int pos = pos0 + tt, pos_last = pos0 + ntok - 1;
+  const int limit = valid ? pos : -1;                       // last visible key
+  const int cq_lo = a.chunk > 0 ? (pos / a.chunk) * a.chunk : 0;
+  const int wq_lo = a.window > 0 ? pos - a.window + 1 : 0;
+  const int keep = a.window > 0 ? a.keep_first : 0;
+  // the wave's first and last token: a block that both see whole needs no mask
+  const int wt0 = w * 32 / hw, wt1 = min(ntok - 1, (w * 32 + 31) / hw);
+  const bool full = (w * 32 + 31) / hw < ntok;              // every row of the wave is a token's
+  const int wp0 = pos0 + wt0, wp1 = pos0 + wt1;
+  const int cl_lo = a.chunk > 0 ? (wp1 / a.chunk) * a.chunk : 0, wl_lo = a.window > 0 ? wp1 - a.window + 1 : 0;
+  const int cw_lo = a.chunk > 0 ? (wp0 / a.chunk) * a.chunk : 0, ww_lo = a.window > 0 ? wp0 - a.window + 1 : 0;
+  // the tile's key blocks: kept first tokens [a_beg, a_end), then [lo_al, pos_last]
+  const KeyRuns k0 = key_runs(pos0, a.chunk, a.window, a.keep_first);
+  const int lo_al = k0.lo & ~63, a_beg = k0.a0 & ~63;
+  const int a_end = a.window > 0 ? min(lo_al, (a.keep_first + 63) & ~63) : a_beg;
+  const int nblkA = max(0, (a_end - a_beg) >> 6), nblk = nblkA + ((pos_last - lo_al) >> 6) + 1;
+  const int* pages = a.bt + (size_t)sg * a.maxb;
+  auto block_at = [&](int bi) { return bi < nblkA ? a_beg + 64 * bi : lo_al + 64 * (bi - nblkA); };
+
+  bf16x8 qf[ND];
+  const uint16_t* qp = a.q + (size_t)(row0 + (valid ? tt : 0)) * HM * D + (size_t)(valid ? head : mp) * D + 8 * hi;
+#pragma unroll
+  for (int s = 0; s < ND; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + 16 * s);
+  f32x16 o[NV];
+#pragma unroll
+  for (int dt = 0; dt < NV; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+  float m = a.sink && valid ? a.sink[head] * kLog2e : -INFINITY, l = 0.f;
+  // a scale that is not positive is applied before the mask and the maximum, a positive one in the exponent
+  const float sc1 = a.scale * kLog2e, sc2 = sc1 > 0.f ? sc1 : 1.f, cap2 = a.softcap * kLog2e, icap = CAP ? 2.f * kLog2e * a.scale / a.softcap : 0.f;
+
+  bf16x8 stg[KC + VC];
+  auto load = [&](int kb, int pg0, int pg1) {
+    const int of0 = kb % a.BS, of1 = HALF ? (kb + 32) % a.BS : 0;
+    const uint16_t* kp = a.kc + ((size_t)pg0 * a.BS + of0) * NK + kh * D;
+    const uint16_t* vp = a.vt + ((size_t)pg0 * NVt + (size_t)gv * V) * a.BS + of0;
+    const uint16_t* k1 = HALF ? a.kc + ((size_t)pg1 * a.BS + of1 - 32) * NK + kh * D : kp;
+    const uint16_t* v1 = HALF ? a.vt + ((size_t)pg1 * NVt + (size_t)gv * V) * a.BS + of1 - 32 : vp;
+#pragma unroll
+    for (int i = 0; i < KC; ++i) {
+      const int c = tid + TH * i, key = c / (D / 8);
+      stg[i] = *reinterpret_cast<const bf16x8*>((HALF && key >= 32 ? k1 : kp) + (size_t)key * NK + 8 * (c % (D / 8)));
+    }
+#pragma unroll
+    for (int i = 0; i < VC; ++i) {
+      const int c = tid + TH * i;
+      stg[KC + i] = *reinterpret_cast<const bf16x8*>((HALF && (c & 4) ? v1 : vp) + (size_t)(c >> 3) * a.BS + 8 * (c & 7));
+    }
+  };
+  // the pages of a block's halves (a second half past the last key reads the first's)
+  auto page0 = [&](int kb) { return pages[kb / a.BS]; };
+  auto page1 = [&](int kb) { return HALF ? pages[(kb + 32 <= pos_last ? kb + 32 : kb) / a.BS] : 0; };
+  auto park = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < KC; ++i) {
+      const int c = tid + TH * i;
+      *reinterpret_cast<bf16x8*>(lds[b] + (c / (D / 8)) * KP + 16 * (c % (D / 8))) = stg[i];
+    }
+#pragma unroll
+    for (int i = 0; i < VC; ++i) {
+      const int c = tid + TH * i;
+      *reinterpret_cast<bf16x8*>(lds[b] + 64 * KP + (c >> 3) * VP + 16 * (c & 7)) = stg[KC + i];
+    }
+  };
+  const int krow = mp_key((r & 3) + 4 * (r >> 3), (r >> 2) & 1);   // the key of this lane's MFMA row in a 32-key half
+  // the queries are there before the loop: its waits count the block loads alone
+#pragma unroll
+  for (int s = 0; s < ND; ++s) asm volatile("" ::"v"(qf[s]));
+  int kb_next = block_at(min(1, nblk - 1)), pg0 = page0(kb_next), pg1 = page1(kb_next);
+  {
+    const int kb = block_at(0);
+    load(kb, page0(kb), page1(kb));
+    park(0);
+  }
+  __syncthreads();
+  for (int bi = 0; bi < nblk; ++bi) {
+    const int kb = block_at(bi);
+    // the page of the block after the next, while this one is computed (the last ones are read again: every load is
+    // unconditional, so the count of loads in flight is known)
+    const int kb_after = block_at(min(bi + 2, nblk - 1)), pa0 = page0(kb_after), pa1 = page1(kb_after);
+    load(kb_next, pg0, pg1);
+    // a wave all of whose tokens come before the block, or after its window or chunk, has nothing to do
+    const bool live = wt0 < ntok && kb <= wp1 && kb + 63 >= cw_lo && (kb + 63 >= ww_lo || kb < keep);
+    if (live) {
+      const unsigned char *kl = lds[bi & 1], *vl = kl + 64 * KP;
+      f32x16 sc[2];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        const unsigned char* kr = kl + (32 * kt + krow) * KP + 16 * hi;
+        f32x16 acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+        for (int s = 0; s < ND; ++s)
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kr + 32 * s), qf[s], acc, 0, 0, 0);
+        sc[kt] = acc;
+      }
+      if (CAP) {                                            // cap tanh(x), tanh(x) = 1 - 2 / (1 + e^(2x)), in log2 units
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const float e = __builtin_amdgcn_exp2f(fminf(sc[kt][i] * icap, 60.f));
+            sc[kt][i] = cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + e));
+          }
+      } else if (!(sc1 > 0.f)) {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sc[kt][i] *= sc1;
+      }
+      if (!(full && kb + 63 <= wp0 && kb >= cl_lo && (kb >= wl_lo || kb + 64 <= keep))) {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int key = kb + 32 * kt + mp_key(i, hi);
+            const bool ok = key <= limit && key >= cq_lo && (key >= wq_lo || key < keep);
+            sc[kt][i] = ok ? sc[kt][i] : -INFINITY;
+          }
+      }
+      float cmax = sc[0][0];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) cmax = fmaxf(cmax, sc[kt][i]);
+      cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+      // the reference moves only where a row's maximum outgrows it by 2^8: weights up to 256, exact in the sums, and most
+      // blocks leave the outputs alone
+      const float mc = CAP ? cmax : cmax * sc2;
+      const bool upd = mc > m + 8.f;
+      const float mn = upd ? mc : m, sub = mn == -INFINITY ? 0.f : -mn;
+      bf16x8 pf[2][2];
+      float ps = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float x = sc[kt][8 * s + j], e = __builtin_amdgcn_exp2f(CAP ? x + sub : fmaf(x, sc2, sub));
+            ps += e;
+            pf[kt][s][j] = (__bf16)e;
+          }
+      if (__any(upd)) {
+        const float alpha = upd ? __builtin_amdgcn_exp2f(m - mn) : 1.f;
+        l *= alpha;
+        m = mn;
+#pragma unroll
+        for (int dt = 0; dt < NV; ++dt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+      }
+      l += ps;
+#pragma unroll
+      for (int dt = 0; dt < NV; ++dt) {
+        const unsigned char* vr = vl + (32 * dt + r) * VP + 16 * hi;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(vr + 64 * kt + 32 * s),
+                                                            pf[kt][s], o[dt], 0, 0, 0);
+      }
+    }
+    park((bi + 1) & 1);
+    kb_next = kb_after;
+    pg0 = pa0;
+    pg1 = pa1;
+    __syncthreads();
+  }
+  if (!valid) return;
+  l += __shfl_xor(l, 32, 64);
+  if (a.sink) l += __builtin_amdgcn_exp2f(a.sink[head] * kLog2e - m);
+  float f = 1.f / l;
+  if (a.gate) f *= 1.f / (1.f + __expf(-a.gate[(size_t)(row0 + tt) * a.gs + head]));
+  const size_t ob = (size_t)(row0 + tt) * HM * V + (size_t)head * V + 4 * hi;   // o[dt][i]: dim 32 dt + 8 (i >> 2) + 4 hi + (i & 3)
+#pragma unroll
+  for (int dt = 0; dt < NV; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+      const size_t oo = ob + 32 * dt + 2 * i;
+      if (a.out32)
+        *reinterpret_cast<f32x4*>(a.out32 + oo) = f32x4{o[dt][i] * f, o[dt][i + 1] * f, o[dt][i + 2] * f, o[dt][i + 3] * f};
+      else
+        *reinterpret_cast<u16x4*>(a.out + oo) =
+            u16x4{f2bf(o[dt][i] * f), f2bf(o[dt][i + 1] * f), f2bf(o[dt][i + 2] * f), f2bf(o[dt][i + 3] * f)};
+    }
+}
+
+template <int ND, int NV, int NW>
+static int launch_mp(const MaskPromptArgs& a, hipStream_t s) {
+  const int hpg = a.H / a.G, hw = hpg < 32 * NW ? hpg : 32 * NW;
+  const dim3 grid(a.n_items * a.G * a.M * ((hpg + hw - 1) / hw));
+#define K8S_MP(CAP, HALF) \
+  hipLaunchKernelGGL((mask_prompt_kernel<ND, NV, NW, CAP, HALF>), grid, dim3(64 * NW), 0, s, a)
+  if (a.softcap > 0.f) {
+    if (a.BS % 64) K8S_MP(true, true);
+    else K8S_MP(true, false);
+  } else {
+    if (a.BS % 64) K8S_MP(false, true);
+    else K8S_MP(false, false);
+  }
+#undef K8S_MP
+  return (int)hipGetLastError();
+}
+
+}  // namespace k8s
+
+using namespace k8s;
+
+K8S_API int k8s_masked_attn_mfma_ok(int H, int G, int D, int V);
+
+// Items of up to max(1, 128 / (H / G)) tokens.
+K8S_API int k8s_masked_attn_prompt(const void* q, const void* kc, const void* vt, const int* bt, int maxb, const int* items,
+                                   int n_items, const float* sink, const float* gate, int gs, void* out, int H, int G,
+                                   int D, int V, int BS, int chunk, int window, int keep_first, float scale, float softcap,
+                                   hipStream_t s, int maps, int out_f32) {
+  if (n_items <= 0) return 0;
+  if (!k8s_masked_attn_mfma_ok(H, G, D, V) || BS % 32 || chunk < 0 || window < 0 || keep_first < 0 || maps < 1)
+    return (int)hipErrorInvalidValue;
+  MaskPromptArgs a;
+  a.q = (const uint16_t*)q; a.kc = (const uint16_t*)kc; a.vt = (const uint16_t*)vt; a.bt = bt; a.maxb = maxb;
+  a.items = items; a.n_items = n_items; a.sink = sink; a.gate = gate; a.gs = gs;
+  a.out = out_f32 ? nullptr : (uint16_t*)out; a.out32 = out_f32 ? (float*)out : nullptr;
+  a.H = H; a.G = G; a.M = maps; a.BS = BS; a.chunk = chunk; a.window = window; a.keep_first = keep_first;
+  a.scale = scale; a.softcap = softcap;
+  if (D == 96) return launch_mp<6, 3, 4>(a, s);
+  if (D == 64 && V == 64) return launch_mp<4, 2, 4>(a, s);
+  if (D == 64 && V == 128) return launch_mp<4, 4, 4>(a, s);
+  if (D == 128 && V == 64) return launch_mp<8, 2, 4>(a, s);
+  return launch_mp<8, 4, 4>(a, s);
+}

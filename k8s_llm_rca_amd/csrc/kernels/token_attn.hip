@@ -31,6 +31,7 @@ struct TokOut {
   float* po;              // [items][H][parts][V]: a part's unnormalised output
   float* pml;             // [items][H][parts][2]: its maximum (log2 units) and denominator
   int H, n_parts;
+  int hs;                 // heads of one workgroup are hs apart (score maps: theirs lie [head][map])
 };
 
 // 1 / denominator (sink included) times the gate; w: the factor of the outputs
@@ -79,7 +80,7 @@ __device__ __forceinline__ void tok_join(TokLds<NW, ND * 16>& s, const TokOut& a
     }
   __syncthreads();
   for (int e = threadIdx.x; e < nh * (V / 4); e += 64 * NW) {
-    const int hh = e / (V / 4), c = 4 * (e % (V / 4)), head = head0 + hh;
+    const int hh = e / (V / 4), c = 4 * (e % (V / 4)), head = head0 + hh * a.hs;
     float mw[NW], lw[NW];
     f32x4 ow[NW];
 #pragma unroll
@@ -119,7 +120,7 @@ __device__ __forceinline__ void tok_join(TokLds<NW, ND * 16>& s, const TokOut& a
 // a part without keys
 __device__ __forceinline__ void tok_empty(const TokOut& a, int head0, int nh, int part) {
   if ((int)threadIdx.x < nh) {
-    float* ml = a.pml + (((size_t)blockIdx.x * a.H + head0 + threadIdx.x) * a.n_parts + part) * 2;
+    float* ml = a.pml + (((size_t)blockIdx.x * a.H + head0 + threadIdx.x * a.hs) * a.n_parts + part) * 2;
     ml[0] = -INFINITY;
     ml[1] = 0.f;
   }
@@ -211,8 +212,8 @@ __device__ __forceinline__ void tok_softmax(const float (&p)[8], int hq, float& 
 }
 
 struct MaskTokArgs {
-  const uint16_t* q;      // [T][H * D]
-  const uint16_t* kc;     // [pages][BS][G * D]
+  const uint16_t* q;      // [T][H * D] (H: heads x maps)
+  const uint16_t* kc;     // [pages][BS][G * maps * D]
   const uint16_t* vt;     // [pages][G * V][BS]
   const int* bt;
   int maxb;
@@ -222,7 +223,7 @@ struct MaskTokArgs {
   TokOut t;
 };
 
-// grid (rows, key heads x groups of 16 of their heads, parts); a part is a run of the row's list of 32-key blocks
+// grid (rows, key heads (x maps) x groups of 16 of their heads, parts); a part is a run of the row's list of 32-key blocks
 // (kept first tokens, then the window's or chunk's).
 template <int NDC, int NV, bool CAP>
 __global__ void __launch_bounds__(512) masked_attn_token_kernel(MaskTokArgs a) {
@@ -231,8 +232,9 @@ __global__ void __launch_bounds__(512) masked_attn_token_kernel(MaskTokArgs a) {
   const int lane = threadIdx.x & 63, r = lane & 15, hq = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sg = a.items[blockIdx.x * 4], row = a.items[blockIdx.x * 4 + 1], pos = a.items[blockIdx.x * 4 + 3];
-  const int H = a.t.H, hpg = H / a.G, nhc = (hpg + 15) / 16, g = blockIdx.y / nhc, hc = blockIdx.y % nhc;
-  const int head0 = g * hpg + 16 * hc, nh = min(16, hpg - 16 * hc), NK = a.G * D, NVt = a.G * V;
+  const int H = a.t.H, M = a.t.hs, hpg = H / (a.G * M), nhc = (hpg + 15) / 16, g = blockIdx.y / nhc, hc = blockIdx.y % nhc;
+  const int gv = g / M, head0 = (gv * hpg + 16 * hc) * M + g % M, nh = min(16, hpg - 16 * hc), NK = a.G * M * D,
+            NVt = a.G * V;
   const int keep = a.window > 0 ? a.keep_first : 0;
   const KeyRuns k0 = key_runs(pos, a.chunk, a.window, a.keep_first);
   const int lo_al = k0.lo & ~31, a_beg = k0.a0 & ~31;
@@ -245,7 +247,7 @@ __global__ void __launch_bounds__(512) masked_attn_token_kernel(MaskTokArgs a) {
     return;
   }
   bf16x8 qf[NDC];
-  const uint16_t* qp = a.q + (size_t)row * H * D + (size_t)(head0 + min(r, nh - 1)) * D;
+  const uint16_t* qp = a.q + (size_t)row * H * D + (size_t)(head0 + min(r, nh - 1) * M) * D;
 #pragma unroll
   for (int cc = 0; cc < NDC; ++cc) qf[cc] = tld16(qp + 32 * cc + 8 * hq);
   float m = -INFINITY, l = 0.f;
@@ -277,7 +279,7 @@ __global__ void __launch_bounds__(512) masked_attn_token_kernel(MaskTokArgs a) {
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int cc = 0; cc < NDC; ++cc) kf[u][t][cc] = tld16(kp + (size_t)(8 * (r >> 2) + 4 * t + (r & 3)) * NK + 32 * cc);
-    const uint16_t* vp = a.vt + ((size_t)page * NVt + (size_t)g * V) * a.BS + off + 8 * hq;
+    const uint16_t* vp = a.vt + ((size_t)page * NVt + (size_t)gv * V) * a.BS + off + 8 * hq;
 #pragma unroll
     for (int dt = 0; dt < NV; ++dt) vf[u][dt] = tld16(vp + (size_t)(16 * dt + r) * a.BS);
   };
@@ -402,8 +404,8 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
 
 template <int NDC, int NV>
 static int launch_mask_tok(const MaskTokArgs& a, int rows, hipStream_t s) {
-  const int hpg = a.t.H / a.G;
-  const dim3 grid(rows, a.G * ((hpg + 15) / 16), a.t.n_parts);
+  const int hpg = a.t.H / (a.G * a.t.hs);
+  const dim3 grid(rows, a.G * a.t.hs * ((hpg + 15) / 16), a.t.n_parts);
   if (a.softcap > 0.f)
     hipLaunchKernelGGL((masked_attn_token_kernel<NDC, NV, true>), grid, dim3(512), 0, s, a);
   else
@@ -440,18 +442,18 @@ K8S_API int k8s_masked_attn_token(const void* q, const void* kc, const void* vt,
                                   const int* items, int rows, const float* sink, const float* gate, int gs, void* out,
                                   int H, int G, int D, int V, int BS, int chunk, int window, int keep_first, float scale,
                                   float softcap, hipStream_t s, int part_blocks, int most, int n_parts, float* pml,
-                                  float* po, int out_f32) {
+                                  float* po, int maps, int out_f32) {
   if (rows <= 0) return 0;
   if (!k8s_masked_attn_mfma_ok(H, G, D, V) || BS % 32 || chunk < 0 || window < 0 || keep_first < 0 || n_parts < 1 ||
-      part_blocks < 1 || most < 1 || n_parts > most || (n_parts > 1 && (!pml || !po)))
+      part_blocks < 1 || maps < 1 || most < 1 || n_parts > most || (n_parts > 1 && (!pml || !po)))
     return (int)hipErrorInvalidValue;
   MaskTokArgs a;
   a.q = (const uint16_t*)q; a.kc = (const uint16_t*)kc; a.vt = (const uint16_t*)vt; a.bt = bt; a.maxb = maxb;
   a.items = items; a.G = G; a.BS = BS; a.chunk = chunk; a.window = window; a.keep_first = keep_first;
   a.part_blocks = part_blocks; a.most = most; a.scale = scale; a.softcap = softcap;
   a.t.sink = sink; a.t.gate = gate; a.t.gs = gs; a.t.out = out_f32 ? nullptr : (uint16_t*)out;
-  a.t.out32 = out_f32 ? (float*)out : nullptr; a.t.ost = (long)H * V; a.t.osh = V; a.t.po = po; a.t.pml = pml;
-  a.t.H = H; a.t.n_parts = n_parts;
+  a.t.out32 = out_f32 ? (float*)out : nullptr; a.t.ost = (long)H * maps * V; a.t.osh = V;
+  a.t.po = po; a.t.pml = pml; a.t.H = H * maps; a.t.n_parts = n_parts; a.t.hs = maps;
   if (D == 96) return launch_mask_tok<3, 6>(a, rows, s);
   if (D == 64 && V == 64) return launch_mask_tok<2, 4>(a, rows, s);
   if (D == 64 && V == 128) return launch_mask_tok<2, 8>(a, rows, s);
@@ -474,7 +476,7 @@ K8S_API int k8s_latent_attn_token(const void* qa, long qst, long qsh, const void
   a.most = most;
   a.scale_log2 = scale * kTokLog2e;
   a.t.sink = sink; a.t.gate = gate; a.t.gs = ldg; a.t.out = (uint16_t*)out; a.t.out32 = nullptr; a.t.ost = ost;
-  a.t.osh = osh; a.t.po = po; a.t.pml = pml; a.t.H = H; a.t.n_parts = n_parts;
+  a.t.osh = osh; a.t.po = po; a.t.pml = pml; a.t.H = H; a.t.n_parts = n_parts; a.t.hs = 1;
   switch (R / 32) {
     case 1: return launch_lat_tok<1>(a, RP / 32, rows, s);
     case 2: return launch_lat_tok<2>(a, RP / 32, rows, s);

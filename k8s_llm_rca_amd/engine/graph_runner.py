@@ -48,6 +48,9 @@ class _DecodeSegments(SegMeta):
     def attn_items(self, tokens_per_item: int) -> tuple:
         return self.items, self.items[:0], self.pos0_host[0] + 1
 
+    def mask_items(self, tokens_per_item: int) -> tuple:
+        return self.items, self.items[:0], self.pos0_host[0] + 1
+
     def tile_items(self, tokens_per_item: int) -> torch.Tensor:
         return self.items
 

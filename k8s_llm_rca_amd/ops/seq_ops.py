@@ -31,6 +31,11 @@ from ._lib import check, lib, ptr, scratch, stream_ptr, use_hip
 MASK_TOKEN_BLOCKS = 8    # 32-key blocks of the row's own list
 LATENT_PART = 128        # keys, from the part of the row's first visible key on
 TOKEN_PARTS = 64         # a row with more than so many of them has larger ones: the partial results stay bounded
+MASK_TILE_ROWS = 128     # (token, head) rows of one workgroup of the masked prompt kernel
+# A step's prompt rows up to which they are taken one by one as well (masked layers): the tiles of one sequence each walk all
+# their keys, the rows have them cut into parts.  us, prompt kernel / rows, 16 heads over 2: 8 rows at 0 / 500 / 2000 keys
+# 7.7 / 4.9, 20 / 11.5, 62 / 11.7;  128 rows 11.5 / 6.5, 25.7 / 25.7, 68 / 63;  256 rows 14.7 / 14.4, 29 / 49, 72 / 121.
+MASK_FEW_ROWS = 128
 
 
 @dataclass
@@ -87,6 +92,32 @@ class SegMeta:
             if self.row_seg.device.type == "cuda":
                 host = host.pin_memory()
             got = self._items[key] = host.to(self.row_seg.device, non_blocking=True)
+        return got
+
+    def mask_items(self, tokens_per_item: int) -> tuple:
+        """Work items of the masked attention, made once per step: (items of one token, tiles of at most
+        ``tokens_per_item``, most keys an item of one token sees).  The leading segments of one token are single items,
+        and so are all rows where no more than ``MASK_FEW_ROWS`` stand behind them."""
+        key = ("mask", tokens_per_item)
+        got = self._items.get(key)
+        if got is None:
+            n1 = 0
+            while n1 < self.n_seg and self.row0_host[n1 + 1] - self.row0_host[n1] == 1:
+                n1 += 1
+            if self.row0_host[-1] - n1 <= MASK_FEW_ROWS:
+                n1 = self.n_seg
+            it, kmax, n = [], 0, 0
+            for s in range(self.n_seg):
+                a, b, p0 = self.row0_host[s], self.row0_host[s + 1], self.pos0_host[s]
+                step = 1 if s < n1 else tokens_per_item
+                it += [(s, r, min(step, b - r), p0 + r - a) for r in range(a, b, step)]
+                if s < n1:
+                    kmax, n = max(kmax, p0 + b - a), len(it)
+            host = torch.from_numpy(np.asarray(it, dtype=np.int32).reshape(-1, 4))
+            if self.row_seg.device.type == "cuda":
+                host = host.pin_memory()
+            both = host.to(self.row_seg.device, non_blocking=True)
+            got = self._items[key] = (both[:n], both[n:], kmax)
         return got
 
     def chunk_ranges(self, rows: int, min_rows: int) -> Optional[tuple]:
@@ -1031,10 +1062,11 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
         gs = gate.stride(0) if gate is not None else 0
         if vt is not None and masked_mfma_ok(H, G, D, V, q.dtype, q.device):
             assert vt.is_contiguous() and vt.shape[1:] == (G * V, BS) and BS % 32 == 0
-            items = seg.tile_items(WINDOW_TILE)
-            n_items = items.shape[0]
-            if T == seg.n_seg and maps == 1:
-                kmax = max(seg.pos0_host) + 1
+            common = (ptr(sink), ptr(gate), gs, ptr(out), H, G, D, V, BS, int(chunk), int(window), int(keep_first),
+                      float(scale), float(softcap), stream_ptr(q))
+            bt, maxb = seg.block_tables, seg.block_tables.shape[1]
+            rows, tiles, kmax = seg.mask_items(max(1, MASK_TILE_ROWS // (H // G)))
+            if rows.shape[0]:
                 nblk = -(-kmax // 32)
                 if window > 0:     # the window from a block's border on; + the kept blocks
                     nblk = min(nblk, (int(window) + 62) // 32 + -(-int(keep_first) // 32))
@@ -1042,35 +1074,13 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
                     nblk = min(nblk, (int(chunk) + 62) // 32)
                 n_parts, po, pml = min(-(-nblk // MASK_TOKEN_BLOCKS), TOKEN_PARTS), None, None
                 if n_parts > 1:
-                    po, pml = (scratch(T * H * n_parts * n, torch.float32, q.device) for n in (V, 2))
-                check(lib().k8s_masked_attn_token(ptr(q), ptr(kc), ptr(vt), ptr(seg.block_tables),
-                                                  seg.block_tables.shape[1], ptr(items), T, ptr(sink), ptr(gate), gs,
-                                                  ptr(out), H, G, D, V, BS, int(chunk), int(window), int(keep_first),
-                                                  float(scale), float(softcap), stream_ptr(q), MASK_TOKEN_BLOCKS,
-                                                  TOKEN_PARTS, n_parts, ptr(pml), ptr(po), int(out_f32)), "masked_attn_token")
-                return out
-            # steps of few rows: a tile's key blocks are split over workgroups as well -- parts of
-            # MASK_PART_BLOCKS blocks of the tile's own block list (at most MASK_MAX_PARTS parts), then a merge
-            # (more tiles than that only where they are single tokens: a prompt's parts would be all traffic)
-            n_parts, pb, pml, po = 1, MASK_PART_BLOCKS, None, None
-            if n_items <= WINDOW_SPLIT_ITEMS or (n_items <= 4 * WINDOW_SPLIT_ITEMS and T <= 2 * n_items):
-                kmax = max(p + b - a for p, a, b in zip(seg.pos0_host, seg.row0_host[:-1], seg.row0_host[1:]))
-                nblk = -(-kmax // 32) + 1                  # an upper bound of any tile's blocks
-                if window > 0:     # a tile's span: the window, its 16 tokens, a block's alignment; + the kept blocks
-                    nblk = min(nblk, (int(window) + 45) // 32 + 1 + -(-int(keep_first) // 32))
-                if chunk > 0:
-                    nblk = min(nblk, (int(chunk) + 45) // 32 + 1)
-                most = MASK_MAX_PARTS if n_items <= WINDOW_SPLIT_ITEMS else max(1, 1024 // n_items)
-                pb = max(MASK_PART_BLOCKS, -(-nblk // most))
-                n_parts = -(-nblk // pb)
-                if n_parts > 1:
-                    pml = scratch(n_items * n_parts * HQ * 32, torch.float32, q.device)
-                    po = scratch(n_items * n_parts * 16 * HQ * V, torch.float32, q.device)
-            check(lib().k8s_masked_attn_mfma(ptr(q), ptr(kc), ptr(vt), ptr(seg.block_tables),
-                                             seg.block_tables.shape[1], ptr(items), n_items, ptr(sink),
-                                             ptr(gate), gs, ptr(out), H, G, D, V, BS, int(chunk), int(window),
-                                             int(keep_first), float(scale), float(softcap), stream_ptr(q), pb, n_parts,
-                                             ptr(pml), ptr(po), int(maps), int(out_f32)), "masked_attn_mfma")
+                    po, pml = (scratch(rows.shape[0] * HQ * n_parts * n, torch.float32, q.device) for n in (V, 2))
+                check(lib().k8s_masked_attn_token(ptr(q), ptr(kc), ptr(vt), ptr(bt), maxb, ptr(rows), rows.shape[0],
+                                                  *common, MASK_TOKEN_BLOCKS, TOKEN_PARTS, n_parts, ptr(pml), ptr(po),
+                                                  int(maps), int(out_f32)), "masked_attn_token")
+            if tiles.shape[0]:
+                check(lib().k8s_masked_attn_prompt(ptr(q), ptr(kc), ptr(vt), ptr(bt), maxb, ptr(tiles), tiles.shape[0],
+                                                   *common, int(maps), int(out_f32)), "masked_attn_prompt")
             return out
         assert vc is not None          # the vector-pipe kernel reads token-major values
         parts, po, pml = _rows_parts(seg, T, HQ, H // G, V, q.device, int(chunk), int(window), int(keep_first))
@@ -1111,10 +1121,6 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
             o = o * torch.sigmoid(gate[a:e, :HQ])[:, :, None]
         out[a:e] = o.reshape(n, HQ * V).to(out.dtype)
     return out
-
-
-MASK_PART_BLOCKS = 4    # 32-key blocks per part when a step of few rows is split over the keys too
-MASK_MAX_PARTS = 32
 
 
 def masked_mfma_ok(H: int, G: int, D: int, V: int, dtype, device) -> bool:

@@ -1,0 +1,66 @@
+"""Masked attention of prompt portions on the matrix cores (tiles of 128 token-head rows over 64-key blocks) in a step with
+single tokens in front, against 64 bits: every mask, page sizes whose blocks cross pages, odd head counts, score maps."""
+import math
+
+import pytest
+import torch
+
+from k8s_llm_rca_amd.ops import seq_ops as S
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+LENS, POS0 = [1, 1, 170, 33, 1, 129], [0, 300, 0, 95, 200, 64]      # two single tokens in front, one among the portions
+
+
+def meta(n_pages, pages):
+    row0 = [0]
+    for n in LENS:
+        row0.append(row0[-1] + n)
+
+    def i32(v):
+        return torch.tensor(v, dtype=torch.int32, device="cuda")
+    return S.SegMeta(len(LENS), i32([s for s, n in enumerate(LENS) for _ in range(n)]), i32(row0), i32(POS0),
+                     i32([0] * len(LENS)), i32([pages] * len(LENS)), row0, list(POS0), [0] * len(LENS))
+
+
+@pytest.mark.parametrize("H,G,D,V,maps,BS", [(16, 2, 128, 128, 1, 64), (3, 3, 64, 64, 1, 32), (20, 1, 96, 96, 1, 96),
+                                             (6, 2, 64, 128, 2, 64), (131, 1, 64, 64, 1, 128), (5, 1, 128, 64, 1, 32)])
+@pytest.mark.parametrize("kw", [dict(), dict(window=70, keep_first=20), dict(window=1), dict(window=130, keep_first=70),
+                                dict(chunk=50, softcap=6.0), dict(chunk=100, window=33, keep_first=3),
+                                dict(scale=-0.05), dict(scale=0.0)])
+def test_prompts(H, G, D, V, maps, BS, kw):
+    kw = dict(kw)
+    n, HQ = 320, H * maps
+    g = torch.Generator().manual_seed(D + H)
+    scale = kw.pop("scale", D ** -0.5)
+    N = -(-n // BS)
+    pages = torch.randperm(N, generator=g).tolist()
+    k, v = torch.randn(n, G * maps, D, generator=g).to(BF), torch.randn(n, G, V, generator=g).to(BF)
+    kc, vt = torch.zeros(N, BS, G * maps * D, dtype=BF), torch.zeros(N, G * V, BS, dtype=BF)
+    for i in range(n):
+        kc[pages[i // BS], i % BS], vt[pages[i // BS], :, i % BS] = k[i].reshape(-1), v[i].reshape(-1)
+    T, m = sum(LENS), meta(N, pages)
+    assert [x.shape[0] > 0 for x in m.mask_items(max(1, 128 // (H // G)))[:2]] == [True, True]
+    q = (2 * torch.randn(T, HQ, D, generator=g)).to(BF)
+    sink, gate = torch.randn(HQ, generator=g), torch.randn(T, HQ + 1, generator=g)
+    got = {f32: S.masked_attention(q.view(T, -1).cuda(), H, G, D, V, kc.cuda(), None, m, scale, sink=sink.cuda(),
+                                   gate=gate.cuda()[:, 1:], vt=vt.cuda(), maps=maps, out_f32=f32, **kw) for f32 in (0, 1)}
+    assert torch.equal(got[1].to(BF), got[0])
+    qi = torch.cat([p + torch.arange(x) for p, x in zip(POS0, LENS)])[:, None]
+    kp = torch.arange(n)[None]
+    vis = kp <= qi
+    if "chunk" in kw:
+        vis &= qi // kw["chunk"] == kp // kw["chunk"]
+    if "window" in kw:
+        vis &= (qi - kp < kw["window"]) | (kp < kw.get("keep_first", 0))
+    rep = H // G
+    kk = k.double().view(n, G, maps, D).repeat_interleave(rep, 1).reshape(n, HQ, D)
+    vv = v.double().repeat_interleave(rep, 1).repeat_interleave(maps, 1)
+    s = torch.bmm(q.double().transpose(0, 1), kk.permute(1, 2, 0).contiguous()) * scale           # [HQ, T, n]
+    if "softcap" in kw:
+        s = kw["softcap"] * torch.tanh(s / kw["softcap"])
+    s = s.masked_fill(~vis[None], -math.inf)
+    p = torch.softmax(torch.cat([s, sink.double()[:, None, None].expand(HQ, T, 1)], -1), -1)[..., :-1]
+    want = torch.bmm(p, vv.transpose(0, 1).contiguous()).transpose(0, 1) * torch.sigmoid(gate[:, 1:].double())[..., None]
+    # the weights are rounded to bf16 (2^-9 each, of both signs) before they meet the values, the result once more
+    assert float((got[1].double().cpu().view(T, HQ, V) - want).abs().max()) < 2.0 ** -7 * float(want.abs().max())

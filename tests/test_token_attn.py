@@ -109,6 +109,22 @@ def test_latent(H, R, P, window, extras):
         assert torch.equal(run([r])[0], got[r]) and torch.equal(run([r, 13], head_major=False)[0], got[r])
 
 
+def test_score_maps():
+    """Two maps a head: each map against its own key head, both against the head's values."""
+    g = torch.Generator().manual_seed(5)
+    H, G, D, V, M, n = 6, 2, 64, 128, 2, 640
+    k, v = torch.randn(n, G, M, D, generator=g).to(BF), torch.randn(n, G, V, generator=g).to(BF)
+    q = torch.randn(3, H, M, D, generator=g).to(BF)
+    pos, dev = [0, 257, 639], "cuda"
+    kc, vt = k.view(10, BS, -1).to(dev), v.view(10, BS, -1).transpose(1, 2).contiguous().to(dev)
+    got = S.masked_attention(q.view(3, -1).to(dev), H, G, D, V, kc, None, meta(pos, list(range(10))), 0.125, vt=vt, maps=M,
+                             out_f32=True).view(3, H, M, V)
+    for t, p in enumerate(pos):
+        s = torch.einsum("hmd,jhmd->hmj", q[t].double(), k[:p + 1].double().repeat_interleave(H // G, 1)) * 0.125
+        want = torch.einsum("hmj,jhv->hmv", torch.softmax(s, -1), v[:p + 1].double().repeat_interleave(H // G, 1))
+        close(got[t], want)
+
+
 @pytest.mark.parametrize("most", [1, 3, 5])
 def test_rows_of_more_keys_than_parts(most, monkeypatch):
     """Parts grow where the count is bounded; the same result as unbounded."""
