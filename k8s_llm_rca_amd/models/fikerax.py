@@ -398,8 +398,7 @@ class FikeraxModel:
         cq = S.latent_norm(dn, L["dq_norm"], L["dkv_norm"], inp.slots, cache, c.q_rank, KR, self.cfg.norm_eps, self.dtype,
                            cache_t=cache_t, tail=R, tail_cs=cs)
         q = proj(cq, L["w_uq"])                                             # [T, H (D + R)]
-        qr = S.rotated_tail(q, cs, H, D, c.tail) if R else None
-        qa = torch.bmm(q.view(T, H, D + R)[:, :, :D].transpose(0, 1), L["uk"]).transpose(0, 1)    # [T, H, KR], head-major
+        qa, qr = S.latent_queries(q, L["uk"], cs, H, D, c.tail)               # [T, H, KR] head-major, [T, H, tail]
         kw = dict(window=c.window, sink=L["sink"], head_major=True)
         if cache_t is not None:
             o = S.latent_attention_mfma(qa, cache, cache_t, None, inp.seg, inp.positions, c.scale, qr=qr, **kw)
@@ -407,7 +406,7 @@ class FikeraxModel:
             o = S.latent_attention(qa.float(), cache, None, inp.seg, c.scale, self.dtype,
                                    qr=qr.float() if qr is not None else None, **kw)
         ov = torch.empty(T, H, V, dtype=self.dtype, device=h.device)
-        torch.bmm(o.transpose(0, 1), L["uv_t"], out=ov.transpose(0, 1))       # written token-major: W_o reads it as it is
+        S.head_proj(o, L["uv_t"], ov)                                         # written token-major: W_o reads it as it is
         return proj_planes(ov.view(T, H * V), L["wo"])
 
     def _dense(self, i: int, h: torch.Tensor) -> torch.Tensor:

@@ -374,10 +374,6 @@ class LizesunModel:
         return n + sum(size(t) for t in (self.embed, self.lm_head, self.final_norm))
 
     # -------------------------------------------------------------- forward
-    def _act(self, x32: torch.Tensor) -> torch.Tensor:
-        """A column slice of an fp32 GEMM result as the next GEMM's operand."""
-        return x32.to(self.dtype).contiguous()
-
     def _chunk_attention(self, li: int, h, inp: S.SegStepInputs, kcs, vcs, vts, vmix: dict) -> torch.Tensor:
         L, a = self.layers[li], self.cfg.layers[li].attn
         ci = self.cache_of[li]
@@ -425,8 +421,8 @@ class LizesunModel:
         qkv = proj(h, L["w_qkv"])                                    # [T, 2 G D + H V]
         qkv = S.short_conv(qkv, L["conv_w"], None, states[f"dconv{j}"], inp.seg, act=True)
         agb = proj_f32out(h, L["w_agb"])                               # [T, ra + rg + H] fp32
-        dec = proj_f32out(self._act(agb[:, :ra]), L["w_a2"])           # [T, H D] fp32, before bias and softplus
-        gate = proj_f32out(self._act(agb[:, ra:ra + rg]), L["w_g2"])   # [T, H V] fp32, before the sigmoid
+        # [T, H D] before bias and softplus, [T, H V] before the sigmoid, both fp32
+        dec, gate = S.low_rank_pair(agb, 0, L["w_a2"], ra, L["w_g2"], self.dtype)
         o = S.gated_delta(qkv, c.heads, c.kv_heads, c.dim, c.vdim, dec, L["rate"], L["dt_bias"], agb[:, ra + rg:],
                           states[f"delta{j}"], inp.seg)
         o = S.head_norm_gate(o, gate, L["delta_norm"], c.heads, c.vdim, self.cfg.norm_eps, self.dtype)

@@ -358,6 +358,64 @@ def rotated_tail(q: torch.Tensor, cs: torch.Tensor, H: int, N: int, pad: int) ->
     return out
 
 
+# Rows up to which small products run on the vector pipes (csrc/kernels/small_proj.hip).  us, library / this, at 1, 16, 64,
+# 128 rows: 16 heads 128 -> 256 with the rotated part 7.3 / 3.1, 7.3 / 4.7, 9.1 / 5.5, 9.6 / 7.2;  256 -> 128 6.9 / 3.4,
+# 6.3 / 5.2, 6.5 / 5.6, 7.4 / 6.9;  two of 64 -> 2048 with their roundings 12.2 / 2.5, 11.8 / 3.6, 12.4 / 4.0, 12.2 / 5.5.
+SMALL_PROJ_ROWS = 128
+
+
+def _small_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return use_hip(x) and 0 < x.shape[0] <= SMALL_PROJ_ROWS and w.dtype == torch.bfloat16 and w.is_contiguous()
+
+
+def head_proj(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+    """``out[t, h] = x[t, h] @ w[h]`` of ``x`` [T, H, K] and ``w`` [H, K, N] (the strides of ``x`` and ``out`` [T, H, N]
+    but the last are free): a kernel of one launch for few rows of bf16, the library's batched product otherwise."""
+    T, H, K = x.shape
+    N = w.shape[2]
+    if (_small_rows(x, w) and x.dtype == torch.bfloat16 == out.dtype and x.stride(2) == 1 == out.stride(2) and K % 8 == 0
+            and K <= 1024 and N % 64 == 0):
+        check(lib().k8s_head_proj(ptr(x), x.stride(0), x.stride(1), ptr(w), ptr(out), out.stride(0), out.stride(1), T, H, K,
+                                  N, None, None, 0, 0, stream_ptr(x)), "head_proj")
+    else:
+        torch.bmm(x.transpose(0, 1), w, out=out.transpose(0, 1))
+    return out
+
+
+def latent_queries(q: torch.Tensor, uk: torch.Tensor, cs: Optional[torch.Tensor], H: int, D: int, pad: int) -> tuple:
+    """A latent layer's queries from its heads ``q`` [T, H (D + R)]: (their first D entries in latent space by ``uk``
+    [H, D, KR], [T, H, KR] and head-major in memory; the R entries behind rotated by ``cs`` as :func:`rotated_tail` has
+    them, None without ``cs``)."""
+    T, KR = q.shape[0], uk.shape[2]
+    x = q.view(T, H, -1)
+    R = x.shape[2] - D
+    if _small_rows(q, uk) and q.dtype == torch.bfloat16 and q.is_contiguous() and D % 8 == 0 and D <= 1024 and KR % 64 == 0:
+        qa = torch.empty(H, T, KR, dtype=q.dtype, device=q.device).transpose(0, 1)
+        qr = None
+        if R:
+            assert cs.dtype == torch.float32 and cs.is_contiguous() and cs.shape == (T, R) and pad >= R and pad % 2 == 0
+            qr = torch.empty(T, H, pad, dtype=q.dtype, device=q.device)
+        check(lib().k8s_head_proj(ptr(q), x.stride(0), x.stride(1), ptr(uk), ptr(qa), qa.stride(0), qa.stride(1), T, H, D,
+                                  KR, ptr(cs), ptr(qr), R, pad if R else 0, stream_ptr(q)), "head_proj")
+        return qa, qr
+    qr = rotated_tail(q, cs, H, D, pad) if R else None
+    return torch.bmm(x[:, :, :D].transpose(0, 1), uk).transpose(0, 1), qr
+
+
+def low_rank_pair(x: torch.Tensor, c0: int, w0: torch.Tensor, c1: int, w1: torch.Tensor, dtype) -> tuple:
+    """``x[:, c:c + K] @ w.T`` in fp32 for two column ranges of fp32 rows, rounded to the activations' ``dtype`` first."""
+    from .linear import proj_f32out
+    T, (N0, K0), (N1, K1) = x.shape[0], w0.shape, w1.shape
+    if (_small_rows(x, w0) and _small_rows(x, w1) and dtype == torch.bfloat16 and x.dtype == torch.float32
+            and x.stride(1) == 1 and all(k % 32 == 0 and 0 < k <= 1024 for k in (K0, K1))
+            and w0.data_ptr() % 16 == 0 == w1.data_ptr() % 16):
+        a, b = (torch.empty(T, n, dtype=torch.float32, device=x.device) for n in (N0, N1))
+        check(lib().k8s_low_rank_pair(ptr(x), x.stride(0), T, c0, K0, ptr(w0), N0, ptr(a), c1, K1, ptr(w1), N1, ptr(b),
+                                      stream_ptr(x)), "low_rank_pair")
+        return a, b
+    return tuple(proj_f32out(x[:, c:c + w.shape[1]].to(dtype).contiguous(), w) for c, w in ((c0, w0), (c1, w1)))
+
+
 ROWS_PART = 128     # visible keys per part of the vector-pipe attention
 ROWS_HEADS = 8      # heads of one key head per workgroup of it
 ROWS_FILL = 512     # workgroups from which it walks a row's parts itself
