@@ -96,6 +96,35 @@ __global__ void __launch_bounds__(256) embed_scale_dyt_kernel(const int* __restr
   }
 }
 
+// The same with four neighbouring columns per thread (16384 rows of 2048 106 -> 50 us, one row 10.3 -> 2.4).
+__device__ __forceinline__ f32x4 ldd4(const float* p, size_t i) { return *reinterpret_cast<const f32x4*>(p + i); }
+__device__ __forceinline__ f32x4 ldd4(const uint16_t* p, size_t i) {
+  const u16x4 v = *reinterpret_cast<const u16x4*>(p + i);
+  return f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
+}
+template <typename TE, typename TA>
+__global__ void __launch_bounds__(512) embed_scale_dyt4_kernel(const int* __restrict__ ids, const TE* __restrict__ embed,
+                                                               float scale, float* __restrict__ x, float alpha,
+                                                               const float* __restrict__ w, const float* __restrict__ b,
+                                                               TA* __restrict__ out, int W) {
+  const size_t o = (size_t)blockIdx.x * W, src = (size_t)ids[blockIdx.x] * W;
+  for (int c = 4 * threadIdx.x; c < W; c += 4 * blockDim.x) {
+    f32x4 v = ldd4(embed, src + c), wv = f32x4{0.f, 0.f, 0.f, 0.f}, bv = wv;
+    if (w) {
+      wv = ldd4(w, c);
+      bv = ldd4(b, c);
+    }
+    float r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] *= scale;
+      r[k] = fmaf(tanhf(alpha * v[k]), wv[k], bv[k]);
+    }
+    *reinterpret_cast<f32x4*>(x + o + c) = v;
+    if (w) st4(out, o + c, r);
+  }
+}
+
 template <typename TA>
 __global__ void __launch_bounds__(256) relu_sq_kernel(const TA* __restrict__ u, TA* __restrict__ out, size_t n) {
   for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) {
@@ -161,9 +190,15 @@ K8S_API int k8s_embed_scale_dyt(const int* ids, const void* embed, int edt, floa
                                 const float* w, const float* b, void* out, int odt, int T, int W, hipStream_t s) {
   if (T <= 0 || W <= 0) return 0;
   if ((w == nullptr) != (out == nullptr) || (w && !b)) return (int)hipErrorInvalidValue;
-#define K8S_EMB(TE, TA)                                                                                         \
-  hipLaunchKernelGGL((embed_scale_dyt_kernel<TE, TA>), dim3(T), dim3(256), 0, s, ids, (const TE*)embed, scale, x, \
-                     alpha, w, b, (TA*)out, W)
+  const bool by4 = W % 4 == 0 && (((uintptr_t)embed | (uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)out) & 15) == 0;
+  const int t4 = (W / 4 + 63) / 64 * 64;
+#define K8S_EMB(TE, TA)                                                                                                 \
+  if (by4)                                                                                                              \
+    hipLaunchKernelGGL((embed_scale_dyt4_kernel<TE, TA>), dim3(T), dim3(t4 > 512 ? 512 : t4), 0, s, ids,                \
+                       (const TE*)embed, scale, x, alpha, w, b, (TA*)out, W);                                           \
+  else                                                                                                                  \
+    hipLaunchKernelGGL((embed_scale_dyt_kernel<TE, TA>), dim3(T), dim3(256), 0, s, ids, (const TE*)embed, scale, x,     \
+                       alpha, w, b, (TA*)out, W)
   if (edt == 0 && odt == 0) {
     K8S_EMB(uint16_t, uint16_t);
   } else if (edt == 0) {

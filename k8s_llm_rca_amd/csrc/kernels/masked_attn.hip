@@ -194,16 +194,20 @@ __device__ __forceinline__ void write_values(const float* __restrict__ x, int qs
   for (int k = 1; k < nr; ++k) run = run && slots[r0 + k] == s0 + k;
   for (int c = tid; c < NV; c += threads) {
     const float vb = bias ? bias[v_col + c] : 0.f;
-    float v[TR];
+    float v[TR], vo[TR];
 #pragma unroll
-    for (int k = 0; k < TR; ++k) v[k] = k < nr ? sum_planes(x + (size_t)(r0 + k) * qs + v_col + c, pstep, TR == 1 ? planes : 1) + vb : 0.f;
+    for (int k = 0; k < TR; ++k) {
+      const int kk = min(k, nr - 1);
+      v[k] = sum_planes(x + (size_t)(r0 + kk) * qs + v_col + c, pstep, TR == 1 ? planes : 1) + vb;
+      vo[k] = MIX && v_other ? v_other[(size_t)(r0 + kk) * NV + c] : 0.f;
+    }
     if (MIX) {
 #pragma unroll
       for (int k = 0; k < TR; ++k)
         if (k < nr) {
           const size_t o = (size_t)(r0 + k) * NV + c;
           if (v_keep) v_keep[o] = v[k];
-          if (v_other) v[k] = (1.f - lam) * v[k] + lam * v_other[o];
+          if (v_other) v[k] = (1.f - lam) * v[k] + lam * vo[k];
         }
     }
     if (vt && run) {
@@ -262,12 +266,19 @@ __global__ void __launch_bounds__(256) attn_prep_pairs_kernel(const float* __res
   write_values<TA, TR, false>(x, qs, r0, nr, NV, v_col, nullptr, slots, vc, vt, BS, tid, 256, 0.f, nullptr, nullptr);
 }
 
+// four neighbours of a float array of any alignment
+__device__ __forceinline__ f32x4 any4(const float* p) {
+  f32x4 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
 // The preparation with rotation halves (i with i + rot / 2), biases and a norm per head behind the rotation, cos | sin from
 // the table:  D / 8 neighbouring lanes (a power of two) hold a head, each two groups of four entries -- rotated ones and
 // their partners, or eight neighbours behind the rotated part -- so the rotation needs no exchange, the norm a few
 // cross-lane sums, and every access is 16 bytes.  16 heads of 128 over 2 with values mixed across layers, 16384 rows: 226 us
-// (attn_prep_kernel: a row's heads through LDS, a double-precision angle per pair where they are rotated) -> 134 us, one
-// row 15 -> 4.9 us.  TR = 1 (few rows): threads of their own for the values, so that a row is one pass of loads.
+// (attn_prep_kernel: a row's heads through LDS, a double-precision angle per pair where they are rotated) -> 73 us, one
+// row 15 -> 3.0 us.  TR = 1 (few rows): threads of their own for the values, so that a row is one pass of loads.
 template <typename TA, int TR, bool MIX>
 __global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(const float* __restrict__ x, int qs, int H, int G, int NV, int D,
                                                              int v_col, const float* __restrict__ bias,
@@ -287,11 +298,19 @@ __global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(co
     const int a = turn ? 4 * j : 8 * j, b = turn ? a + half : a + 4;
     const float* p = x + (size_t)r * qs + u * D;
     f32x4 va = sum_planes4(p + a, pstep, TR == 1 ? planes : 1), vb = sum_planes4(p + b, pstep, TR == 1 ? planes : 1);
+    // the norm's weights with the row (entry by entry behind the norm they were half of the time)
+    const float* w = u < H ? q_w : k_w;
+    f32x4 wa = f32x4{1.f, 1.f, 1.f, 1.f}, wb = wa;
+    if (w) {
+      wa = any4(w + a);
+      wb = any4(w + b);
+    }
     if (bias) {
+      const f32x4 ba = any4(bias + u * D + a), bb = any4(bias + u * D + b);
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        va[k] += bias[u * D + a + k];
-        vb[k] += bias[u * D + b + k];
+        va[k] += ba[k];
+        vb[k] += bb[k];
       }
     }
     if (turn) {
@@ -312,11 +331,10 @@ __global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(co
       for (int o = 1; o < lph; o <<= 1) ss += __shfl_xor(ss, o, 64);
       rn = 1.f / sqrtf(ss / (float)D + eps);
     }
-    const float* w = u < H ? q_w : k_w;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      va[k] *= rn * (w ? w[a + k] : 1.f);
-      vb[k] *= rn * (w ? w[b + k] : 1.f);
+      va[k] *= rn * wa[k];
+      vb[k] *= rn * wb[k];
     }
     if (u < H) {
       const size_t o = ((size_t)r * H + u) * D;

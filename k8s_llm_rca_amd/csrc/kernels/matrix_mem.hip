@@ -423,27 +423,79 @@ __global__ void __launch_bounds__(256) head_norm_sigmoid_kernel(const float* __r
   }
 }
 
+// Four neighbouring gates (VG: one aligned access).
+template <bool VG>
+__device__ __forceinline__ f32x4 gates4(const float* p) {
+  if (VG) return *reinterpret_cast<const f32x4*>(p);
+  return f32x4{p[0], p[1], p[2], p[3]};
+}
+template <bool VG>
+__device__ __forceinline__ f32x4 gates4(const uint16_t* p) {
+  if (!VG) return f32x4{bf2f(p[0]), bf2f(p[1]), bf2f(p[2]), bf2f(p[3])};
+  const u16x4 v = *reinterpret_cast<const u16x4*>(p);
+  return f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
+}
+__device__ __forceinline__ void put4(float* p, const f32x4& v) { *reinterpret_cast<f32x4*>(p) = v; }
+__device__ __forceinline__ void put4(uint16_t* p, const f32x4& v) {
+  *reinterpret_cast<u16x4*>(p) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+}
+
+// The same for V = 4 L (L lanes of a wave per head) without sub and with 16-byte accesses: results, gates and weights are
+// asked for together, the norm is a few cross-lane sums.  16384 rows of 16 heads of 128, fp32 gates, us: a wave per head
+// with a column a lane 127, this 60 (335 MB).
+template <typename TA, typename TG, int L>
+__global__ void __launch_bounds__(256) head_norm_lanes_kernel(const float* __restrict__ o, const TG* __restrict__ gate,
+                                                              int gs, const float* __restrict__ w, int wh,
+                                                              TA* __restrict__ out, int n_rh, int H, float eps,
+                                                              const float* __restrict__ mul, float oscale) {
+  constexpr int V = 4 * L;
+  const int rh = (blockIdx.x * 256 + threadIdx.x) / L, c = 4 * (threadIdx.x % L);
+  if (rh >= n_rh) return;                                  // whole groups of lanes
+  const int r = rh / H, h = rh - r * H;
+  f32x4 u = *reinterpret_cast<const f32x4*>(o + (size_t)rh * V + c), g = f32x4{0.f, 0.f, 0.f, 0.f},
+        wv = f32x4{1.f, 1.f, 1.f, 1.f};
+  if (gate) g = gates4<true>(gate + (size_t)r * gs + (size_t)h * V + c);
+  if (w) wv = *reinterpret_cast<const f32x4*>(w + (size_t)h * wh + c);
+  const float mu = mul ? mul[rh] : 1.f;
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) ss = fmaf(u[k] * mu, u[k] * mu, ss);
+#pragma unroll
+  for (int d = 1; d < L; d <<= 1) ss += __shfl_xor(ss, d, 64);
+  const float rn = mu * oscale / sqrtf(ss / (float)V + eps);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) u[k] = u[k] * rn * wv[k] * (gate ? sigmoid_f(g[k]) : 1.f);
+  put4(out + (size_t)rh * V + c, u);
+}
+
 // The same with one norm over a whole row of V (a multiple of 4): a workgroup per row, four neighbouring entries per
-// thread and round, the row in registers between the sum of squares and the output.
+// thread and round; the row, its gates and weights are asked for together and stay in registers.  16384 rows of 2048, bf16
+// gates, us: gates one by one behind the sum 93, this 57 (268 MB); one row 3.0, now 2.5.  VG: gates by 8 or 16 bytes.
 constexpr int kRowRounds = 4;
-template <typename TA, typename TG>
+template <typename TA, typename TG, bool VG>
 __global__ void __launch_bounds__(1024) row_norm_sigmoid_kernel(const float* __restrict__ o, const TG* __restrict__ gate,
                                                                 int gs, const float* __restrict__ w,
                                                                 TA* __restrict__ out, int V, float eps) {
   __shared__ float red[16];
   const size_t row = (size_t)blockIdx.x * V;
   const int step = 4 * blockDim.x;
-  f32x4 v[kRowRounds];
+  f32x4 v[kRowRounds], g[kRowRounds], wv[kRowRounds];
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < kRowRounds; ++k) {
     const int c = 4 * threadIdx.x + k * step;
     if (c < V) {
       v[k] = *reinterpret_cast<const f32x4*>(o + row + c);
+      if (gate) g[k] = gates4<VG>(gate + (size_t)blockIdx.x * gs + c);
+      if (w) wv[k] = f32x4{w[c], w[c + 1], w[c + 2], w[c + 3]};
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kRowRounds; ++k)
+    if (4 * (int)threadIdx.x + k * step < V) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) ss = fmaf(v[k][i], v[k][i], ss);
     }
-  }
   const float rn = 1.f / sqrtf(block_sum(ss, red) / (float)V + eps);
 #pragma unroll
   for (int k = 0; k < kRowRounds; ++k) {
@@ -451,15 +503,11 @@ __global__ void __launch_bounds__(1024) row_norm_sigmoid_kernel(const float* __r
     if (c < V) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float u = v[k][i] * rn;
-        if (w) u *= w[c + i];
-        if (gate) u *= 1.f / (1.f + __expf(-ldx(gate, (size_t)blockIdx.x * gs + c + i)));
-        v[k][i] = u;
+        v[k][i] *= rn;
+        if (w) v[k][i] *= wv[k][i];
+        if (gate) v[k][i] *= 1.f / (1.f + __expf(-g[k][i]));
       }
-      if constexpr (sizeof(TA) == 4)
-        *reinterpret_cast<f32x4*>(out + row + c) = v[k];
-      else
-        *reinterpret_cast<u16x4*>(out + row + c) = u16x4{f2bf(v[k][0]), f2bf(v[k][1]), f2bf(v[k][2]), f2bf(v[k][3])};
+      put4(out + row + c, v[k]);
     }
   }
 }
@@ -468,11 +516,28 @@ template <typename TA, typename TG>
 static int launch_head_norm(const float* o, const void* gate, int gs, const float* w, int wh, void* out, int T, int H,
                             int V, float eps, hipStream_t s, const float* mul, int sub, float lam, float oscale) {
   const int n_rh = T * H;
-  if (H == 1 && !mul && !sub && oscale == 1.f && V % 4 == 0 && V >= 256 && V <= 4 * 1024 * kRowRounds &&
-      (((uintptr_t)o | (uintptr_t)out) & 15) == 0) {
+  const bool rows16 = (((uintptr_t)o | (uintptr_t)out) & 15) == 0;
+  const bool vg = gate == nullptr || (gs % 4 == 0 && (uintptr_t)gate % (4 * sizeof(TG)) == 0);
+  if (H == 1 && !mul && !sub && oscale == 1.f && V % 4 == 0 && V >= 256 && V <= 4 * 1024 * kRowRounds && rows16) {
     const int want = (V / 4 + 63) / 64 * 64;
-    hipLaunchKernelGGL((row_norm_sigmoid_kernel<TA, TG>), dim3(T), dim3(want > 1024 ? 1024 : want), 0, s, o,
-                       (const TG*)gate, gs, w, (TA*)out, V, eps);
+    const dim3 b(want > 1024 ? 1024 : want);
+    if (vg)
+      hipLaunchKernelGGL((row_norm_sigmoid_kernel<TA, TG, true>), dim3(T), b, 0, s, o, (const TG*)gate, gs, w, (TA*)out, V,
+                         eps);
+    else
+      hipLaunchKernelGGL((row_norm_sigmoid_kernel<TA, TG, false>), dim3(T), b, 0, s, o, (const TG*)gate, gs, w, (TA*)out,
+                         V, eps);
+  } else if (!sub && (V == 64 || V == 128 || V == 256) && rows16 && vg && ((uintptr_t)w & 15) == 0 && wh % 4 == 0) {
+#define K8S_HL(L)                                                                                                 \
+  hipLaunchKernelGGL((head_norm_lanes_kernel<TA, TG, L>), dim3((unsigned)(((size_t)n_rh * L + 255) / 256)), dim3(256), 0, s, \
+                     o, (const TG*)gate, gs, w, wh, (TA*)out, n_rh, H, eps, mul, oscale)
+    if (V == 64)
+      K8S_HL(16);
+    else if (V == 128)
+      K8S_HL(32);
+    else
+      K8S_HL(64);
+#undef K8S_HL
   } else {
     hipLaunchKernelGGL((head_norm_sigmoid_kernel<TA, TG>), dim3((n_rh + 3) / 4), dim3(256), 0, s, o, (const TG*)gate, gs,
                        w, wh, (TA*)out, n_rh, H, V, eps, mul, sub, lam, oscale);
