@@ -133,11 +133,12 @@ int build_plan(const Key& k, size_t ws_limit, Plan* out) {
 
 // ws: device scratch of ws_bytes (reused by every call on the stream; must
 // outlive any HIP graph that captured a call).  f32out: Y is fp32 (the lm_head's
-// logits, B9: sampling reads fp32 logits), else bf16.
+// logits, B9: sampling reads fp32 logits), else bf16; 2: fp32, alpha times the
+// product added to what y holds (the fp32 residual of a layer).
 K8S_API int k8s_blaslt_gemm2(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, void* ws,
-                             size_t ws_bytes, hipStream_t s, int f32out) {
-  if (M <= 0 || N <= 0 || K <= 0 || ldx < K || ldy < N) return (int)hipErrorInvalidValue;
-  const Key key{M, N, K, ldx, ldy, f32out ? 1 : 0};
+                             size_t ws_bytes, hipStream_t s, int f32out, float alpha) {
+  if (M <= 0 || N <= 0 || K <= 0 || ldx < K || ldy < N || f32out < 0 || f32out > 2) return (int)hipErrorInvalidValue;
+  const Key key{M, N, K, ldx, ldy, f32out};
   Plan* plan;
   {
     std::lock_guard<std::mutex> g(g_mu);
@@ -152,7 +153,7 @@ K8S_API int k8s_blaslt_gemm2(const void* x, int ldx, const void* w, void* y, int
     plan = &it->second;
   }
   if (plan->ws > ws_bytes) return 1300;
-  const float alpha = 1.f, beta = 0.f;
+  const float beta = f32out == 2 ? 1.f : 0.f;
   hipblasStatus_t st = hipblasLtMatmul(g_handle, plan->desc, &alpha, w, plan->a, x, plan->b, &beta, y, plan->c, y,
                                        plan->c, &plan->algo, ws, plan->ws, s);
   return st == HIPBLAS_STATUS_SUCCESS ? 0 : 1400 + (int)st;
@@ -160,7 +161,7 @@ K8S_API int k8s_blaslt_gemm2(const void* x, int ldx, const void* w, void* y, int
 
 K8S_API int k8s_blaslt_gemm(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, void* ws,
                             size_t ws_bytes, hipStream_t s) {
-  return k8s_blaslt_gemm2(x, ldx, w, y, ldy, M, N, K, ws, ws_bytes, s, 0);
+  return k8s_blaslt_gemm2(x, ldx, w, y, ldy, M, N, K, ws, ws_bytes, s, 0, 1.f);
 }
 
 K8S_API int k8s_blaslt_num_plans() {

@@ -31,7 +31,7 @@ import torch
 
 from ..ops import norm as N
 from ..ops import seq_ops as S
-from ..ops.linear import glu_proj, proj, proj_f32out, proj_planes
+from ..ops.linear import glu_proj, proj, proj_add, proj_f32out, proj_planes
 from ..parallel.groups import ParallelContext, single
 
 TAIL_ALIGN = 32     # the rotated key part of a latent cache row is filled up to a multiple of this
@@ -380,7 +380,7 @@ class FikeraxModel:
         x = proj(h, L["w_in"])                                             # q | k | v | gate as activations
         o = S.decay_attention(x, c.heads, c.dim, c.vdim, L["decay"], state, inp.seg, silu=True)
         y = S.head_norm_gate(o, x[:, x.shape[1] - HV:], L["mem_norm"], 1, HV, self.cfg.norm_eps, self.dtype)
-        return proj_planes(y, L["wo"])
+        return y
 
     def _attention(self, i: int, h: torch.Tensor, inp: S.SegStepInputs, tables, kc, vc, vt) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
@@ -388,7 +388,7 @@ class FikeraxModel:
         q = S.attn_prep(x, L["b_in"], c.heads, c.kv_heads, c.dim, c.vdim, inp.positions, inp.slots, kc, vc, self.dtype,
                         norm="head", eps=self.cfg.norm_eps, rope=self.ropes[i], rope_cs=self._table(i, inp, tables), vt=vt)
         o = S.masked_attention(q, c.heads, c.kv_heads, c.dim, c.vdim, kc, vc, inp.seg, c.scale, window=c.window, vt=vt)
-        return proj_planes(o, L["wo"])
+        return o
 
     def _latent_attention(self, i: int, h: torch.Tensor, inp: S.SegStepInputs, tables, cache, cache_t) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
@@ -407,11 +407,7 @@ class FikeraxModel:
                                    qr=qr.float() if qr is not None else None, **kw)
         ov = torch.empty(T, H, V, dtype=self.dtype, device=h.device)
         S.head_proj(o, L["uv_t"], ov)                                         # written token-major: W_o reads it as it is
-        return proj_planes(ov.view(T, H * V), L["wo"])
-
-    def _dense(self, i: int, h: torch.Tensor) -> torch.Tensor:
-        L = self.layers[i]
-        return proj_planes(glu_proj(h, L["w13"]), L["w2"])                    # silu(gate) * up
+        return ov.view(T, H * V)
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[Optional[torch.Tensor]],
                 vts: List[Optional[torch.Tensor]], states: Optional[Dict[str, torch.Tensor]] = None,
@@ -439,12 +435,20 @@ class FikeraxModel:
                 y = self._attention(i, h, inp, tables, kcs[ci], vcs[ci], vts[ci])
             else:
                 y = self._latent_attention(i, h, inp, tables, kcs[ci], vts[ci])
+            w = L["wo"]
             if spec.ff:
-                h = N.hyper_step(x, y, one, mix1, inn=one, nw=L["norm2"], eps=eps, out_dtype=dt)
-                y = self._dense(i, h)
+                y = proj_add(x[:, 0], y, w)
+                h = (N.hyper_read(x, None, L["norm2"], eps, dt) if y is None
+                     else N.hyper_step(x, y, one, mix1, inn=one, nw=L["norm2"], eps=eps, out_dtype=dt))
+                y, w = glu_proj(h, L["w13"]), L["w2"]                            # silu(gate) * up
+            # (a pass that reads the embedding once more adds the product too)
+            y = proj_planes(y, w) if into.get("again") else proj_add(x[:, 0], y, w)
             if layers_out is not None:
-                layers_out.append(x[:, 0] + y.sum(0))
-            h = N.hyper_step(x, y, one, mix1, **into)
+                layers_out.append(x[:, 0].clone() if y is None else x[:, 0] + y.sum(0))
+            if y is not None:
+                h = N.hyper_step(x, y, one, mix1, **into)
+            elif into:
+                h = N.hyper_read(x, None, into["nw"], eps, dt)
         return proj_f32out(N.hyper_read(x, inp.logits_idx, self.final_norm, eps, dt), self.head)
 
 

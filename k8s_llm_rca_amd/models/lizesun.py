@@ -35,7 +35,7 @@ import torch
 
 from ..ops import norm as N
 from ..ops import seq_ops as S
-from ..ops.linear import proj, proj_f32out, proj_planes, relu_sq_proj
+from ..ops.linear import proj, proj_add, proj_f32out, relu_sq_proj
 from ..parallel.groups import ParallelContext, single
 
 
@@ -390,7 +390,7 @@ class LizesunModel:
                         v_other=other, v_keep=keep, vt=vts[ci])
         o = S.masked_attention(q, H, G, D, V, kcs[ci], vcs[ci], inp.seg, a.scale, softcap=a.softcap, chunk=a.chunk,
                                gate=x[:, H * D + G * (D + V):], vt=vts[ci])
-        return proj_planes(o, L["wo"])
+        return o
 
     def _parallel(self, li: int, h, inp: S.SegStepInputs, kcs, vcs, vts, states, tables: dict):
         L, spec = self.layers[li], self.cfg.layers[li]
@@ -413,7 +413,7 @@ class LizesunModel:
                                  states[f"memn{j}"], states[f"memm{j}"], inp.seg, defer_scale=True)
         orr = S.head_norm_gate(o, xr[:, 2 * hd + hv:2 * hd + 2 * hv], L["mem_norm"], b.heads, b.vdim,
                                self.cfg.norm_eps, self.dtype, mul=mul)
-        return proj_planes(ol, L["wo_l"]), proj_planes(orr, L["wo_r"])
+        return ol, orr
 
     def _delta(self, li: int, h, inp: S.SegStepInputs, states) -> torch.Tensor:
         L, c = self.layers[li], self.cfg.layers[li].delta
@@ -426,7 +426,7 @@ class LizesunModel:
         o = S.gated_delta(qkv, c.heads, c.kv_heads, c.dim, c.vdim, dec, L["rate"], L["dt_bias"], agb[:, ra + rg:],
                           states[f"delta{j}"], inp.seg)
         o = S.head_norm_gate(o, gate, L["delta_norm"], c.heads, c.vdim, self.cfg.norm_eps, self.dtype)
-        return proj_planes(o, L["wo"])
+        return o
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[torch.Tensor],
                 vts: List[Optional[torch.Tensor]], states: Dict[str, torch.Tensor],
@@ -444,16 +444,18 @@ class LizesunModel:
         for li, (spec, L) in enumerate(zip(cfg.layers, self.layers)):
             nxt = self.layers[li + 1]["norm1"] if li + 1 < nl else (1.0, None, None)   # the final norm: wanted rows only
             after = L["norm2"] if spec.ff else nxt
-            if spec.kind == "attention":
-                h = N.add_dyt(x, self._chunk_attention(li, h, inp, kcs, vcs, vts, vmix), 1.0, None, 1.0, *after,
-                              out_dtype=dt)
-            elif spec.kind == "parallel":
-                yl, yr = self._parallel(li, h, inp, kcs, vcs, vts, states, tables)
-                h = N.add_dyt(x, yl, spec.left_scale, yr, spec.right_scale, *after, out_dtype=dt)
+            if spec.kind == "parallel":
+                ol, orr = self._parallel(li, h, inp, kcs, vcs, vts, states, tables)
+                yl = proj_add(x, ol, L["wo_l"], spec.left_scale)
+                yr = proj_add(x, orr, L["wo_r"], spec.right_scale)
+                add = (yl, spec.left_scale, yr, spec.right_scale) if yl is not None else (yr, spec.right_scale, None, 1.0)
+                h = N.add_dyt(x, *add, *after, out_dtype=dt)
             else:
-                h = N.add_dyt(x, self._delta(li, h, inp, states), 1.0, None, 1.0, *after, out_dtype=dt)
+                o = (self._chunk_attention(li, h, inp, kcs, vcs, vts, vmix) if spec.kind == "attention"
+                     else self._delta(li, h, inp, states))
+                h = N.add_dyt(x, proj_add(x, o, L["wo"]), 1.0, None, 1.0, *after, out_dtype=dt)
             if spec.ff:
-                y = proj_planes(relu_sq_proj(h, L["w_up"]), L["w_down"])
+                y = proj_add(x, relu_sq_proj(h, L["w_up"]), L["w_down"])
                 h = N.add_dyt(x, y, 1.0, None, 1.0, *nxt, out_dtype=dt)
             if layers_out is not None:
                 layers_out.append(x.clone())

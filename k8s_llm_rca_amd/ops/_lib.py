@@ -59,7 +59,7 @@ _SIGS = {
     "k8s_splitk_addnorm": [P, I, P, P, P, I, I, I, F, P],
     "k8s_gemm_mid_num_cfgs": [],
     "k8s_blaslt_gemm": [P, I, P, P, I, I, I, I, P, ctypes.c_size_t, P],
-    "k8s_blaslt_gemm2": [P, I, P, P, I, I, I, I, P, ctypes.c_size_t, P, I],
+    "k8s_blaslt_gemm2": [P, I, P, P, I, I, I, I, P, ctypes.c_size_t, P, I, F],
     "k8s_blaslt_num_plans": [],
     "k8s_blaslt_tune": [P, I, P, P, I, I, I, I, P, ctypes.c_size_t, I, I, P, P],
     "k8s_blaslt_clear_tuning": [],
