@@ -1,0 +1,11 @@
+// Scalar functions of the recurrent layers' gates, fp32.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace k8s {
+
+__device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+__device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
+__device__ __forceinline__ float logsigmoid_f(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
+
+}  // namespace k8s

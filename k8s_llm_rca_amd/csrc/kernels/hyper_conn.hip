@@ -79,6 +79,7 @@ constexpr int kMaxStreams = 16;   // the form for any count: one column per thre
 // S streams at compile time (S > 0) or S_ <= kMaxStreams of them (S == 0).
 // y: fp32 rows [yp][T][W] whose planes are summed, or (inv given) rows of yp in expert order weighted by ew [T][K].
 // out / mix: this sublayer's; in / nw: the next one's (h null: nothing reads the streams next).
+// rs (optional) [T][rn]: y is divided by sqrt(sum(rs) / rw + reps), the root mean square of an operand that was not normed.
 // eid (optional) [T]: token ids whose rows of emb, times es, are added to every stream.
 template <int S, int VEC, typename TY, typename TA>
 __global__ void __launch_bounds__(1024) hyper_step_kernel(float* __restrict__ x, const TY* __restrict__ y,
@@ -87,7 +88,8 @@ __global__ void __launch_bounds__(1024) hyper_step_kernel(float* __restrict__ x,
                                                          const float* __restrict__ mix, const float* __restrict__ in,
                                                          const float* __restrict__ nw, float eps, TA* __restrict__ h,
                                                          int W, int S_, const int* __restrict__ eid,
-                                                         const TA* __restrict__ emb, float es, int yp) {
+                                                         const TA* __restrict__ emb, float es, int yp,
+                                                         const float* __restrict__ rs, int rn, float rw, float reps) {
   extern __shared__ float u[];
   __shared__ float red[16];
   constexpr int SM = S > 0 ? S : kMaxStreams;
@@ -97,7 +99,12 @@ __global__ void __launch_bounds__(1024) hyper_step_kernel(float* __restrict__ x,
   float w0[VEC];
   first_weights<VEC>(nw, W, h != nullptr, w0);
   const size_t e0 = eid ? (size_t)eid[t] * W : 0;
-  float ss = 0.f;
+  float ss = 0.f, ys = 1.f;
+  if (rs) {                                                // every wave by itself
+    float sum = 0.f;
+    for (int i = threadIdx.x & 63; i < rn; i += 64) sum += rs[t * rn + i];
+    ys = 1.f / sqrtf(wave_sum(sum) / rw + reps);
+  }
   for (int c = threadIdx.x * VEC; c < W; c += blockDim.x * VEC) {
     float xv[SM][VEC], yv[VEC];
 #pragma unroll
@@ -125,6 +132,10 @@ __global__ void __launch_bounds__(1024) hyper_step_kernel(float* __restrict__ x,
 #pragma unroll
         for (int k = 0; k < VEC; ++k) yv[k] += pv[k];
       }
+    }
+    if (rs) {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) yv[k] *= ys;
     }
     float uv[VEC], av[VEC];
 #pragma unroll
@@ -235,11 +246,12 @@ static bool hyper_row_ok(int W) { return W > 0 && (size_t)W * sizeof(float) <= 6
 template <int VEC, typename TY, typename TA>
 static void hyper_step_launch(float* x, const void* y, const int* inv, const float* ew, int K, const float* out,
                               const float* mix, const float* in, const float* nw, float eps, void* h, int T, int S,
-                              int W, const int* eid, const void* emb, float es, int yp, hipStream_t s) {
+                              int W, const int* eid, const void* emb, float es, int yp, const float* rs, int rn, float rw,
+                              float reps, hipStream_t s) {
   const dim3 g(T), b(hyper_threads(T, W, VEC));
 #define K8S_HS(SS)                                                                                              \
   hipLaunchKernelGGL((hyper_step_kernel<SS, VEC, TY, TA>), g, b, W * sizeof(float), s, x, (const TY*)y, inv, ew, K, \
-                     out, mix, in, nw, eps, (TA*)h, W, S, eid, (const TA*)emb, es, yp)
+                     out, mix, in, nw, eps, (TA*)h, W, S, eid, (const TA*)emb, es, yp, rs, rn, rw, reps)
   switch (S) {
     case 1: K8S_HS(1); break;
     case 2: K8S_HS(2); break;
@@ -257,20 +269,21 @@ using namespace k8s;
 // ydt / hdt / edt: 0 bf16, 1 fp32.  inv null: y is fp32 [yp][T][W].  emb has the type of h.
 K8S_API int k8s_hyper_step(float* x, const void* y, int ydt, const int* inv, const float* ew, int K, const float* out,
                            const float* mix, const float* in, const float* nw, float eps, void* h, int hdt, int T, int S,
-                           int W, hipStream_t s, const int* eid, const void* emb, float es, int yp) {
+                           int W, hipStream_t s, const int* eid, const void* emb, float es, int yp, const float* rs, int rn, float rw,
+                           float reps) {
   if (T <= 0) return 0;
   if (!hyper_row_ok(W) || S < 1 || S > kMaxStreams || !y || !out || !mix || (h && (!in || !nw)) ||
-      yp < 1 || (inv && (!ew || K < 1 || yp != 1)) || (!inv && ydt != 1) || (eid && !emb))
+      yp < 1 || (inv && (!ew || K < 1 || yp != 1)) || (!inv && ydt != 1) || (eid && !emb) || (rs && (rn < 1 || !(rw > 0.f))))
     return (int)hipErrorInvalidValue;
 #define K8S_HY(VEC)                                                                                               \
   if (ydt == 0 && hdt == 0)                                                                                       \
-    hyper_step_launch<VEC, uint16_t, uint16_t>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, s);         \
+    hyper_step_launch<VEC, uint16_t, uint16_t>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, rs, rn, rw, reps, s);         \
   else if (ydt == 0)                                                                                              \
-    hyper_step_launch<VEC, uint16_t, float>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, s);            \
+    hyper_step_launch<VEC, uint16_t, float>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, rs, rn, rw, reps, s);            \
   else if (hdt == 0)                                                                                              \
-    hyper_step_launch<VEC, float, uint16_t>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, s);            \
+    hyper_step_launch<VEC, float, uint16_t>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, rs, rn, rw, reps, s);            \
   else                                                                                                            \
-    hyper_step_launch<VEC, float, float>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, s)
+    hyper_step_launch<VEC, float, float>(x, y, inv, ew, K, out, mix, in, nw, eps, h, T, S, W, eid, emb, es, yp, rs, rn, rw, reps, s)
   if (W % 4 == 0 && S <= 4) {
     K8S_HY(4);
   } else {

@@ -31,6 +31,7 @@
 // (the carry kernels then turn cs / cx into every chunk's START state and advance the slot's state)
 // MODE 2: the chunk again from its start state, writing the outputs.
 #include "common.h"
+#include "gates.h"
 
 namespace k8s {
 
@@ -46,10 +47,6 @@ template <>
 __device__ __forceinline__ void stx<float>(float* p, size_t i, float v) { p[i] = v; }
 template <>
 __device__ __forceinline__ void stx<uint16_t>(uint16_t* p, size_t i, float v) { p[i] = f2bf(v); }
-
-__device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
-__device__ __forceinline__ float logsigmoid_f(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
 constexpr int kMemTb = 16;     // tokens per batch
 constexpr int kMemVb = 64;     // state columns per workgroup

@@ -378,9 +378,8 @@ class FikeraxModel:
         L, c = self.layers[i], self.cfg.layers[i].mix
         HV = c.heads * c.vdim
         x = proj(h, L["w_in"])                                             # q | k | v | gate as activations
-        o = S.decay_attention(x, c.heads, c.dim, c.vdim, L["decay"], state, inp.seg, silu=True)
-        y = S.head_norm_gate(o, x[:, x.shape[1] - HV:], L["mem_norm"], 1, HV, self.cfg.norm_eps, self.dtype)
-        return y
+        return S.decay_layer(x, c.heads, c.dim, c.vdim, L["decay"], state, inp.seg, x[:, x.shape[1] - HV:], L["mem_norm"],
+                             self.cfg.norm_eps, self.dtype)
 
     def _attention(self, i: int, h: torch.Tensor, inp: S.SegStepInputs, tables, kc, vc, vt) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
@@ -429,26 +428,29 @@ class FikeraxModel:
             if r + 1 < len(self.runs):
                 j, add = self.runs[r + 1]
                 into = dict(inn=one, nw=self.layers[j]["norm1"], eps=eps, out_dtype=dt, again=again if add else None)
+            rms = None                                     # what the residual's pass makes up for behind the projection
             if spec.kind == "lightning":
-                y = self._lightning(i, h, inp, states[f"mem{self.state_of[r]}"])
+                y, rms = self._lightning(i, h, inp, states[f"mem{self.state_of[r]}"])
             elif spec.kind == "attention":
                 y = self._attention(i, h, inp, tables, kcs[ci], vcs[ci], vts[ci])
             else:
                 y = self._latent_attention(i, h, inp, tables, kcs[ci], vts[ci])
             w = L["wo"]
             if spec.ff:
-                y = proj_add(x[:, 0], y, w)
+                y = proj_add(x[:, 0], y, w) if rms is None else proj_planes(y, w)
                 h = (N.hyper_read(x, None, L["norm2"], eps, dt) if y is None
-                     else N.hyper_step(x, y, one, mix1, inn=one, nw=L["norm2"], eps=eps, out_dtype=dt))
-                y, w = glu_proj(h, L["w13"]), L["w2"]                            # silu(gate) * up
+                     else N.hyper_step(x, y, one, mix1, inn=one, nw=L["norm2"], eps=eps, out_dtype=dt, rms=rms))
+                y, w, rms = glu_proj(h, L["w13"]), L["w2"], None                 # silu(gate) * up
             # (a pass that reads the embedding once more adds the product too)
-            y = proj_planes(y, w) if into.get("again") else proj_add(x[:, 0], y, w)
-            if layers_out is not None:
-                layers_out.append(x[:, 0].clone() if y is None else x[:, 0] + y.sum(0))
+            y = proj_planes(y, w) if into.get("again") or rms is not None else proj_add(x[:, 0], y, w)
             if y is not None:
-                h = N.hyper_step(x, y, one, mix1, **into)
+                h = N.hyper_step(x, y, one, mix1, rms=rms, **into)
             elif into:
                 h = N.hyper_read(x, None, into["nw"], eps, dt)
+            if layers_out is not None:
+                # (the residual in front of the embedding that a further pass adds)
+                layers_out.append(x[:, 0] - self.embed[inp.input_ids.long()].float() * cfg.embed_scale if into.get("again")
+                                  else x[:, 0].clone())
         return proj_f32out(N.hyper_read(x, inp.logits_idx, self.final_norm, eps, dt), self.head)
 
 

@@ -408,11 +408,8 @@ class LizesunModel:
         ol = S.masked_attention(q, H, G, D, V, kcs[ci], vcs[ci], inp.seg, a.scale, window=a.window,
                                 keep_first=a.keep_first, sink=L["sink"], vt=vts[ci])
         xr = x[:, nl:]
-        hd, hv = b.heads * b.dim, b.heads * b.vdim
-        o, mul = S.matrix_memory(xr, b.heads, b.dim, b.vdim, L["gate_bias"], b.gate_cap, states[f"mem{j}"],
-                                 states[f"memn{j}"], states[f"memm{j}"], inp.seg, defer_scale=True)
-        orr = S.head_norm_gate(o, xr[:, 2 * hd + hv:2 * hd + 2 * hv], L["mem_norm"], b.heads, b.vdim,
-                               self.cfg.norm_eps, self.dtype, mul=mul)
+        orr = S.memory_layer(xr, b.heads, b.dim, b.vdim, L["gate_bias"], b.gate_cap, states[f"mem{j}"], states[f"memn{j}"],
+                             states[f"memm{j}"], inp.seg, L["mem_norm"], self.cfg.norm_eps, self.dtype)
         return ol, orr
 
     def _delta(self, li: int, h, inp: S.SegStepInputs, states) -> torch.Tensor:
@@ -423,10 +420,8 @@ class LizesunModel:
         agb = proj_f32out(h, L["w_agb"])                               # [T, ra + rg + H] fp32
         # [T, H D] before bias and softplus, [T, H V] before the sigmoid, both fp32
         dec, gate = S.low_rank_pair(agb, 0, L["w_a2"], ra, L["w_g2"], self.dtype)
-        o = S.gated_delta(qkv, c.heads, c.kv_heads, c.dim, c.vdim, dec, L["rate"], L["dt_bias"], agb[:, ra + rg:],
-                          states[f"delta{j}"], inp.seg)
-        o = S.head_norm_gate(o, gate, L["delta_norm"], c.heads, c.vdim, self.cfg.norm_eps, self.dtype)
-        return o
+        return S.delta_layer(qkv, c.heads, c.kv_heads, c.dim, c.vdim, dec, L["rate"], L["dt_bias"], agb[:, ra + rg:],
+                             states[f"delta{j}"], inp.seg, gate, L["delta_norm"], self.cfg.norm_eps, self.dtype)
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[torch.Tensor],
                 vts: List[Optional[torch.Tensor]], states: Dict[str, torch.Tensor],

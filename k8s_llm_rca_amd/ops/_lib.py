@@ -96,6 +96,9 @@ _SIGS = {
     "k8s_latent_attn_mfma_ok": [I, I],
     "k8s_latent_attn_mfma": [P, P, P, P, I, P, I, P, I, P, I, I, I, F, P, L, L, P, I, L, L, I, P],
     "k8s_latent_attn_token": [P, L, L, P, I, P, P, P, I, P, I, P, I, P, P, L, L, P, P, I, I, I, I, I, I, I, F, P],
+    "k8s_delta_step": [P, I, P, P, P, P, I, P, P, P, P, I, P, I, P, I, I, I, I, I, F, F, P],
+    "k8s_memory_step": [P, I, P, F, P, P, P, P, P, P, I, P, I, P, I, I, I, I, I, F, F, P],
+    "k8s_decay_step": [P, I, I, P, P, P, P, P, I, P, P, P, I, I, I, I, P],
     "k8s_head_proj": [P, L, L, P, P, L, L, I, I, I, I, P, P, I, I, P],
     "k8s_low_rank_pair": [P, I, I, I, I, P, I, P, I, I, P, I, P, P],
     "k8s_masked_attn_prompt": [P, P, P, P, I, P, I, P, P, I, P, I, I, I, I, I, I, I, I, F, F, P, I, I],
@@ -139,7 +142,7 @@ _SIGS = {
     "k8s_gated_delta_tiles": [P, I, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, F, P, P, I, P, P],
     "k8s_head_norm_gate": [P, P, I, P, I, P, I, I, I, F, I, P, P, I, F, F, I],
     "k8s_ssd_scan": [P, I, P, I, I, P, I, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, I, P, P, I, P, P, P],
-    "k8s_hyper_step": [P, P, I, P, P, I, P, P, P, P, F, P, I, I, I, I, P, P, P, F, I],
+    "k8s_hyper_step": [P, P, I, P, P, I, P, P, P, P, F, P, I, I, I, I, P, P, P, F, I, P, I, F, F],
     "k8s_hyper_embed": [P, P, I, F, P, I, P, P, F, P, I, I, I, P],
     "k8s_hyper_read": [P, P, I, I, P, P, F, P, I, I, P],
     "k8s_walks": [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P, P, P, P],

@@ -355,17 +355,19 @@ def hyper_embed(ids: torch.Tensor, embed: torch.Tensor, scale: float, x: torch.T
 
 def hyper_step(x: torch.Tensor, y: torch.Tensor, out: torch.Tensor, mix: torch.Tensor, experts: Optional[tuple] = None,
                inn: Optional[torch.Tensor] = None, nw: Optional[torch.Tensor] = None, eps: float = 0.0,
-               out_dtype=None, again: Optional[tuple] = None) -> Optional[torch.Tensor]:
+               out_dtype=None, again: Optional[tuple] = None, rms: Optional[tuple] = None) -> Optional[torch.Tensor]:
     """In place on the streams ``x`` [T, S, W]: ``x_r <- sum_s mix[s, r] x_s + out[r] y`` (all at once from the old ones).
     ``y``: fp32 rows [T, W] or planes [S, T, W] of them that are summed (:func:`..ops.linear.proj_planes`), or with ``experts = (inv, w)`` the experts' output rows in expert order, joined on the way in
     as ``sum_k w[t, k] y[inv[t K + k]]`` (``inv`` from :func:`..ops.moe.align`, ``w`` [T, K] fp32).  With ``inn, nw`` also
     returns the next sublayer's input ``rms(sum_s inn[s] x_s) * nw`` of the new streams as activations.  ``again =
     (ids, embed, scale)``: the embedding output ``embed[ids] * scale`` is added to every stream as well, in front of that
-    read."""
+    read.  ``rms = (ss, width, eps)``: ``y`` is divided by ``sqrt(sum(ss[t]) / width + eps)`` first, ``ss`` [T, n] fp32."""
     T, S, W = x.shape
     read = nw is not None
     ids, embed, escale = again if again is not None else (None, None, 0.0)
+    ss, width, reps = rms if rms is not None else (None, 1.0, 0.0)
     if use_hip(x):
+        assert ss is None or (ss.dtype == torch.float32 and ss.is_contiguous() and ss.dim() == 2 and ss.shape[0] == T)
         assert x.dtype == torch.float32 and x.is_contiguous() and y.is_contiguous() and y.shape[-1] == W
         yp = y.shape[0] if y.dim() == 3 else 1
         assert out.dtype == mix.dtype == torch.float32 and out.numel() == S and mix.is_contiguous() and mix.numel() == S * S
@@ -386,13 +388,16 @@ def hyper_step(x: torch.Tensor, y: torch.Tensor, out: torch.Tensor, mix: torch.T
             h = torch.empty(T, W, dtype=out_dtype, device=x.device)
         check(lib().k8s_hyper_step(ptr(x), ptr(y), _odt(y.dtype), ptr(inv), ptr(ew), K, ptr(out), ptr(mix), ptr(inn),
                                    ptr(nw), float(eps), ptr(h), _odt(out_dtype) if read else 1, T, S, W, stream_ptr(x),
-                                   ptr(ids), ptr(embed), float(escale), yp), "hyper_step")
+                                   ptr(ids), ptr(embed), float(escale), yp, ptr(ss), ss.shape[1] if ss is not None else 0,
+                                   float(width), float(reps)), "hyper_step")
         return h
     if experts is not None:
         inv, ew = experts
         y = (y.float()[inv.long()].view(T, ew.shape[1], W) * ew[:, :, None]).sum(1)
     elif y.dim() == 3:
         y = y.sum(0)
+    if ss is not None:
+        y = y * torch.rsqrt(ss.sum(1, keepdim=True) / width + reps)
     x.copy_(torch.einsum("sr,tsw->trw", mix, x) + out[None, :, None] * y[:, None])
     if again is not None:
         x += (embed[ids.long()].float() * escale)[:, None]

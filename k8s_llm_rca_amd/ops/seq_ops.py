@@ -1389,3 +1389,80 @@ def matrix_memory(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tens
             out[r] = (torch.einsum("hdv,hd->hv", S, q[r]) / den[:, None]).reshape(-1)
         state[sl], nstate[sl], mstate[sl] = S, n, m
     return (out, None) if defer_scale else out
+
+
+# ------------------------------------------------------------------ one token per sequence through a matrix state
+# (csrc/kernels/state_step.hip): the state update with its gates, norm and output gate in one launch.  us, token-by-token
+# kernel with its gate and norm passes / this, 16 heads of 128 x 128 at 1 / 8 / 64 / 256 sequences: delta rule 14.1 / 7.1,
+# 16.6 / 7.3, 49.5 / 27.2, 181 / 111;  matrix memory 17.0 / 7.3, 20.7 / 6.7, 54.4 / 30.3, 181 / 109;  decaying attention
+# 9.4 / 5.8, 11.0 / 6.0, 40.1 / 28.4, 142 / 107 (the states' bytes, in and out: 0.4, 3.4, 27, 109).
+def _step_ok(x: torch.Tensor, seg: SegMeta, D: int, V: int, gate: torch.Tensor, w: Optional[torch.Tensor]) -> bool:
+    return (use_hip(x) and seg.n_seg == x.shape[0] and seg.row0_host[-1] == seg.n_seg and D in (64, 128) and V in (64, 128)
+            and min(b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:])) == 1
+            and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0
+            and gate.stride(1) == 1 and gate.stride(0) % 4 == 0 and gate.data_ptr() % 16 == 0
+            and (w is None or (w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0)))
+
+
+def delta_layer(qkv: torch.Tensor, H: int, G: int, D: int, V: int, a: torch.Tensor, rate: torch.Tensor,
+                dt_bias: torch.Tensor, beta: torch.Tensor, state: torch.Tensor, seg: SegMeta, gate: torch.Tensor,
+                w: Optional[torch.Tensor], eps: float, out_dtype) -> torch.Tensor:
+    """:func:`gated_delta`, then :func:`head_norm_gate` over each head."""
+    if (_step_ok(qkv, seg, D, V, gate, w) and gate.dtype == torch.float32 and out_dtype == qkv.dtype
+            and qkv.is_contiguous()):
+        T = qkv.shape[0]
+        assert qkv.shape[1] == 2 * G * D + H * V and H % G == 0 and state.is_contiguous() and state.shape[1:] == (H, D, V)
+        assert a.dtype == torch.float32 and a.is_contiguous() and a.shape == (T, H * D)
+        assert beta.dtype == torch.float32 and beta.stride(1) == 1 and beta.shape[1] >= H and gate.shape[1] >= H * V
+        assert rate.dtype == dt_bias.dtype == torch.float32 and rate.numel() == H and dt_bias.numel() == H * D
+        assert w is None or w.numel() in (V, H * V)
+        out = torch.empty(T, H * V, dtype=out_dtype, device=qkv.device)
+        check(lib().k8s_delta_step(ptr(qkv), _dt(qkv.dtype), ptr(a), ptr(rate), ptr(dt_bias), ptr(beta), beta.stride(0),
+                                   ptr(state), ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(gate), gate.stride(0), ptr(w),
+                                   V if w is not None and w.numel() == H * V else 0, ptr(out), T, H, G, D, V, float(eps),
+                                   float(UNIT_EPS), stream_ptr(qkv)), "delta_step")
+        return out
+    o = gated_delta(qkv, H, G, D, V, a, rate, dt_bias, beta, state, seg)
+    return head_norm_gate(o, gate, w, H, V, eps, out_dtype)
+
+
+def memory_layer(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tensor, cap: float, state: torch.Tensor,
+                 nstate: torch.Tensor, mstate: torch.Tensor, seg: SegMeta, w: Optional[torch.Tensor], eps: float,
+                 out_dtype) -> torch.Tensor:
+    """:func:`matrix_memory`, then :func:`head_norm_gate` over each head with the gates that stand behind the values."""
+    gate = x[:, 2 * H * D + H * V:2 * H * (D + V)]
+    if _step_ok(x, seg, D, V, gate, w):
+        T = x.shape[0]
+        assert x.dtype == torch.float32 and x.shape[1] == 2 * H * (D + V) + 2 * H
+        assert gate_bias.dtype == torch.float32 and gate_bias.numel() == 2 * H and (w is None or w.numel() in (V, H * V))
+        assert state.is_contiguous() and state.shape[1:] == (H, D, V) and nstate.is_contiguous()
+        assert nstate.shape[1:] == (H, D) and mstate.is_contiguous() and mstate.shape[1:] == (H,)
+        out = torch.empty(T, H * V, dtype=out_dtype, device=x.device)
+        check(lib().k8s_memory_step(ptr(x), x.stride(0), ptr(gate_bias), float(cap), ptr(state), ptr(nstate), ptr(mstate),
+                                    ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(gate), gate.stride(0), ptr(w),
+                                    V if w is not None and w.numel() == H * V else 0, ptr(out), _dt(out_dtype), T, H, D, V,
+                                    float(eps), float(DEN_EPS), stream_ptr(x)), "memory_step")
+        return out
+    o, mul = matrix_memory(x, H, D, V, gate_bias, cap, state, nstate, mstate, seg, defer_scale=True)
+    return head_norm_gate(o, gate, w, H, V, eps, out_dtype, mul=mul)
+
+
+def decay_layer(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor, state: torch.Tensor, seg: SegMeta,
+                gate: torch.Tensor, w: torch.Tensor, eps: float, out_dtype) -> tuple:
+    """:func:`decay_attention` with silu, then one norm over all heads, its weight and the gates: (y, None), or for steps of
+    single tokens (y without the division by the row's root mean square, (sums of squares [T, H], H V, eps)), which
+    :func:`.norm.hyper_step` makes up for behind the output projection."""
+    if (_step_ok(x, seg, D, V, gate, w) and gate.dtype == x.dtype == out_dtype and w.numel() == H * V):
+        T = x.shape[0]
+        assert x.shape[1] >= H * (2 * D + V) and gate.shape[1] >= H * V
+        assert decay.dtype == torch.float32 and decay.numel() == H
+        assert state.is_contiguous() and state.dtype == torch.float32 and state.shape[1:] == (H, D, V)
+        out = torch.empty(T, H * V, dtype=out_dtype, device=x.device)
+        ss = torch.empty(T, H, dtype=torch.float32, device=x.device)
+        check(lib().k8s_decay_step(ptr(x), x.stride(0), _dt(x.dtype), ptr(decay), ptr(state), ptr(seg.seg_pos0),
+                                   ptr(seg.seg_slot), ptr(gate), gate.stride(0), ptr(w), ptr(out), ptr(ss), T, H, D, V,
+                                   stream_ptr(x)), "decay_step")
+        return out, (ss, H * V, eps)
+    o = decay_attention(x, H, D, V, decay, state, seg, silu=True)
+    return head_norm_gate(o, gate, w, 1, H * V, eps, out_dtype), None
+
