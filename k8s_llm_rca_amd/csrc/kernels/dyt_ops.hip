@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256) add_dyt4_kernel(float* __restrict__ x, co
                                                        const float* __restrict__ y2, float sy2, float alpha,
                                                        const float* __restrict__ w, const float* __restrict__ b,
                                                        TA* __restrict__ out, size_t n4, int W, int yp, int yp2) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
     const size_t e = i * 4;
     const int c = (int)(e % (size_t)W);
     f32x4 xv = *reinterpret_cast<const f32x4*>(x + e);
@@ -169,11 +169,15 @@ K8S_API int k8s_add_dyt(float* x, const float* y, float sy, const float* y2, flo
   if ((w == nullptr) != (out == nullptr) || (w && !b) || (y2 && !y) || yp < 1 || yp2 < 1) return (int)hipErrorInvalidValue;
   const size_t n = (size_t)T * W;
   if (W % 4 == 0) {
+    // few rows: a wave per workgroup, so that more compute units take the planes in (one row, eight planes of 2048:
+    // 4.4 -> 3.8 us in a reply step)
+    const int th = n / 4 <= 64 * 1024 ? 64 : 256;
+    const int g4 = th == 64 ? (int)((n / 4 + 63) / 64) : grid_for(n / 4);
     if (odt == 0)
-      hipLaunchKernelGGL((add_dyt4_kernel<uint16_t>), dim3(grid_for(n / 4)), dim3(256), 0, s, x, y, sy, y2, sy2, alpha, w,
+      hipLaunchKernelGGL((add_dyt4_kernel<uint16_t>), dim3(g4), dim3(th), 0, s, x, y, sy, y2, sy2, alpha, w,
                          b, (uint16_t*)out, n / 4, W, yp, yp2);
     else
-      hipLaunchKernelGGL((add_dyt4_kernel<float>), dim3(grid_for(n / 4)), dim3(256), 0, s, x, y, sy, y2, sy2, alpha, w, b,
+      hipLaunchKernelGGL((add_dyt4_kernel<float>), dim3(g4), dim3(th), 0, s, x, y, sy, y2, sy2, alpha, w, b,
                          (float*)out, n / 4, W, yp, yp2);
   } else {
     if (odt == 0)

@@ -180,7 +180,7 @@ __device__ __forceinline__ void sta4<uint16_t>(uint16_t* p, size_t i, const f32x
 }
 
 // The value columns of TR rows from r0 (nr of them exist) to their pages: row-major, and a column of TR rows whose slots
-// are TR aligned neighbours of one page to the transposed page in one store.  MIX: kept as projected (v_keep) and mixed
+// are neighbours of one page to the transposed page in one store.  MIX: kept as projected (v_keep) and mixed
 // with another layer's (v_other) on the way, where these are given.
 template <typename TA, int TR, bool MIX>
 __device__ __forceinline__ void write_values(const float* __restrict__ x, int qs, int r0, int nr, int NV, int v_col,
@@ -190,7 +190,7 @@ __device__ __forceinline__ void write_values(const float* __restrict__ x, int qs
                                              int planes = 1, size_t pstep = 0) {
   if (NV == 0) return;
   const int s0 = slots[r0];
-  bool run = TR > 1 && nr == TR && s0 >= 0 && s0 % TR == 0 && BS % TR == 0;    // then a page holds all TR
+  bool run = TR > 1 && nr == TR && s0 >= 0 && s0 % BS + TR <= BS;              // then a page holds all TR
   for (int k = 1; k < nr; ++k) run = run && slots[r0 + k] == s0 + k;
   for (int c = tid; c < NV; c += threads) {
     const float vb = bias ? bias[v_col + c] : 0.f;
@@ -213,8 +213,10 @@ __device__ __forceinline__ void write_values(const float* __restrict__ x, int qs
     if (vt && run) {
       const int page = s0 / BS;
       TA* o = vt + ((size_t)page * NV + c) * BS + (s0 - page * BS);
+      TA t[TR];
 #pragma unroll
-      for (int k = 0; k + 4 <= TR; k += 4) sta4(o, k, f32x4{v[k], v[k + 1], v[k + 2], v[k + 3]});
+      for (int k = 0; k < TR; ++k) sta(t, k, v[k]);
+      __builtin_memcpy(o, t, sizeof(t));                   // of any alignment: a sequence's rows start anywhere in a tile
     } else if (vt) {
 #pragma unroll
       for (int k = 0; k < TR; ++k) {
@@ -234,7 +236,7 @@ __device__ __forceinline__ void write_values(const float* __restrict__ x, int qs
 
 // The preparation where a row's entries do not meet beyond their rotation pair (2i, 2i + 1): no norm, no bias,
 // cos | sin from the table.  A thread takes four neighbouring entries -- two pairs -- at a time straight from
-// memory to memory (no LDS).  A workgroup takes TR rows; value column c of TR rows whose slots are TR aligned
+// memory to memory (no LDS).  A workgroup takes TR rows; value column c of TR rows whose slots are
 // neighbours of one page goes to the transposed page in one store.
 template <typename TA, int TR>
 __global__ void __launch_bounds__(256) attn_prep_pairs_kernel(const float* __restrict__ x, int qs, int NQ, int NK, int NV,
@@ -278,9 +280,12 @@ __device__ __forceinline__ f32x4 any4(const float* p) {
 // their partners, or eight neighbours behind the rotated part -- so the rotation needs no exchange, the norm a few
 // cross-lane sums, and every access is 16 bytes.  16 heads of 128 over 2 with values mixed across layers, 16384 rows: 226 us
 // (attn_prep_kernel: a row's heads through LDS, a double-precision angle per pair where they are rotated) -> 73 us, one
-// row 15 -> 3.0 us.  TR = 1 (few rows): threads of their own for the values, so that a row is one pass of loads.
+// row 15 -> 3.0 us.  TR = 1 (few rows): a row over several
+// workgroups, its values in some of their own: one pass of loads, and one compute unit does not take all its planes in
+// (one row, four planes: 5.2 -> 4.1 us in a reply step).
+constexpr int kPrepRow = 128;
 template <typename TA, int TR, bool MIX>
-__global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(const float* __restrict__ x, int qs, int H, int G, int NV, int D,
+__global__ void __launch_bounds__(256) attn_prep_half_kernel(const float* __restrict__ x, int qs, int H, int G, int NV, int D,
                                                              int v_col, const float* __restrict__ bias,
                                                              const int* __restrict__ slots, TA* __restrict__ kc,
                                                              TA* __restrict__ vc, TA* __restrict__ vt, int BS,
@@ -291,8 +296,10 @@ __global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(co
                                                              float* __restrict__ v_keep, int planes, size_t pstep) {
   const int r0 = blockIdx.x * TR, tid = threadIdx.x, half = rot >> 1, lph = D >> 3, units = H + G;
   const int nr = min(TR, T - r0), n = units * lph;
-  const int heads = TR == 1 ? min((int)blockDim.x - 64, (n + 63) & ~63) : 256;      // threads of the heads
-  for (int i = tid; i < nr * n && tid < heads; i += heads) {
+  // TR = 1: the first workgroups of a row have its heads, 128 threads each, the others its values
+  const int hb = TR == 1 ? (n + kPrepRow - 1) / kPrepRow : 1, heads = TR == 1 ? hb * kPrepRow : 256;
+  const int at = TR == 1 ? (int)blockIdx.y * kPrepRow + tid : tid;
+  for (int i = at; i < nr * n && at < heads; i += heads) {
     const int rr = i / n, u = (i - rr * n) / lph, j = i & (lph - 1), r = r0 + rr;
     const bool turn = 8 * j < rot;
     const int a = turn ? 4 * j : 8 * j, b = turn ? a + half : a + 4;
@@ -351,9 +358,9 @@ __global__ void __launch_bounds__(TR == 1 ? 1024 : 256) attn_prep_half_kernel(co
   }
   if (TR > 1)
     write_values<TA, TR, MIX>(x, qs, r0, nr, NV, v_col, bias, slots, vc, vt, BS, tid, 256, lam, v_other, v_keep);
-  else if (tid >= heads)
-    write_values<TA, TR, MIX>(x, qs, r0, nr, NV, v_col, bias, slots, vc, vt, BS, tid - heads, blockDim.x - heads, lam,
-                              v_other, v_keep, planes, pstep);
+  else if (at >= heads)
+    write_values<TA, TR, MIX>(x, qs, r0, nr, NV, v_col, bias, slots, vc, vt, BS, at - heads,
+                              (gridDim.y - hb) * kPrepRow, lam, v_other, v_keep, planes, pstep);
 }
 
 
@@ -429,10 +436,9 @@ K8S_API int k8s_attn_prep_half(const float* x, int qs, int H, int G, int D, int 
       NV < 0 || v_col < 0 || BS < 1 || (G > 0 && !kc) || (NV > 0 && !vc && !vt) || norm < 0 || norm > 1 ||
       planes < 1 || (planes > 1 && (T > 1024 || pstep % 4)) || ((uintptr_t)x & 15) || ((uintptr_t)cs & 15))
     return (int)hipErrorInvalidValue;
-  const int one = (H + G) * (D / 8), want = (one + 63) / 64 * 64 + (NV + 63) / 64 * 64;     // threads of a row's one pass
-  const int row_threads = want < 128 ? 128 : (want > 1024 ? 1024 : want);
+  const int row_groups = ((H + G) * (D / 8) + kPrepRow - 1) / kPrepRow + (NV + kPrepRow - 1) / kPrepRow;
 #define K8S_PH(TA, TR, MIX)                                                                                             \
-  hipLaunchKernelGGL((attn_prep_half_kernel<TA, TR, MIX>), dim3((T + TR - 1) / TR), dim3(TR == 1 ? row_threads : 256), 0, s, x, qs, H, G, NV, D, \
+  hipLaunchKernelGGL((attn_prep_half_kernel<TA, TR, MIX>), dim3((T + TR - 1) / TR, TR == 1 ? row_groups : 1), dim3(TR == 1 ? kPrepRow : 256), 0, s, x, qs, H, G, NV, D, \
                      v_col, bias, slots, (TA*)kc, (TA*)vc, (TA*)vt, BS, (TA*)q_out, rot, cs, norm, q_w, k_w, eps, T, lam, \
                      v_other, v_keep, planes, pstep)
 #define K8S_PH_T(TA)                                   \

@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(PLANES ? 512 : 256) latent_norm_kernel(const f
 
 // The same for many rows: two rows a wave, eight a workgroup, norms by cross-lane sums, every row in registers between
 // its sums and its results.  What the row-by-row kernel waits for is the transposed pages, two bytes of a line per token
-// and column: here a column's eight tokens, where they are aligned neighbours of a page, are one store of 16 bytes.
+// and column: here a column's eight tokens, where they are neighbours of a page, are one store of 16 bytes.
 // 16384 rows of 768 + 256 + 64: 52 us row by row, 30 here (130 MB).  Row pitch and parts multiples of 4, QR <= 2048,
 // KR <= 1024, 16-byte rows.
 constexpr int kLnRows = 8;
@@ -384,20 +384,14 @@ __global__ void __launch_bounds__(256) latent_norm_rows_kernel(const float* __re
   if (!cache_t) return;
   __syncthreads();
   const int s0 = slots[t0];
-  bool run = nr == kLnRows && s0 >= 0 && s0 % kLnRows == 0 && BS % kLnRows == 0;     // then a page holds all of them
+  bool run = nr == kLnRows && s0 >= 0 && s0 % BS + kLnRows <= BS;                    // then a page holds all of them
   for (int k = 1; k < nr; ++k) run = run && slots[t0 + k] == s0 + k;
   for (int c = threadIdx.x; c < KR; c += 256) {
     if (run) {
       TA v[kLnRows];
 #pragma unroll
       for (int k = 0; k < kLnRows; ++k) v[k] = tile[k * KR + c];
-      TA* o = cache_t + ((size_t)(s0 / BS) * KR + c) * BS + s0 % BS;
-#pragma unroll
-      for (int k = 0; k < kLnRows; k += 16 / (int)sizeof(TA)) {
-        f32x4 raw;
-        __builtin_memcpy(&raw, v + k, 16);
-        *reinterpret_cast<f32x4*>(o + k) = raw;
-      }
+      __builtin_memcpy(cache_t + ((size_t)(s0 / BS) * KR + c) * BS + s0 % BS, v, sizeof(v));   // of any alignment
     } else {
       for (int k = 0; k < nr; ++k) {
         const int sl = slots[t0 + k];

@@ -24,8 +24,8 @@ def test_forms(T, dt, H, G, D, V, rot, v_is_k, keep, other):
     x = rnd(T, width + 4)
     slots = torch.randperm(pages * BS, generator=g)[:T].to(torch.int32)
     if T > 1000:
-        slots[:512] = torch.arange(512, dtype=torch.int32) + 64       # runs of aligned neighbours among scattered ones
-        slots[512:] = torch.arange(T - 512, dtype=torch.int32) + 64 + 512
+        slots[:512] = torch.arange(512, dtype=torch.int32) + 64       # runs of neighbours, aligned and not
+        slots[512:] = torch.arange(T - 512, dtype=torch.int32) + 64 + 512 + 3
     slots[T // 2] = -1
     pos = torch.randint(0, 5000, (T,), generator=g).to(torch.int32)
     bias, q_w, k_w, v_other = rnd(width), rnd(D), rnd(D), rnd(T, NV)
