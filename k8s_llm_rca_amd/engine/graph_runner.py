@@ -317,7 +317,7 @@ class GraphRunnerMixin:
                               block_tables=flat[8 * B:].view(B, width), row0_host=list(range(B + 1)),
                               pos0_host=[width * self.kv.block_size - 1] * B, slot_host=[0] * B, n_single=B)
         seg.items = flat[4 * B:8 * B].view(B, 4)
-        inp = SegStepInputs(ids, pos, slots, seg, torch.arange(B, device=self.device))
+        inp = SegStepInputs(ids, pos, slots, seg, None)
         states = self.states.t if self.states is not None else {}
         if self._graph_pool is None:
             self._graph_pool = torch.cuda.graph_pool_handle()

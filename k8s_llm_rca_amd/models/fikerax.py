@@ -428,6 +428,8 @@ class FikeraxModel:
             if r + 1 < len(self.runs):
                 j, add = self.runs[r + 1]
                 into = dict(inn=one, nw=self.layers[j]["norm1"], eps=eps, out_dtype=dt, again=again if add else None)
+            elif inp.logits_idx is None:                   # every row is wanted: the last write-back reads the head's input
+                into = dict(inn=one, nw=self.final_norm, eps=eps, out_dtype=dt)
             rms = None                                     # what the residual's pass makes up for behind the projection
             if spec.kind == "lightning":
                 y, rms = self._lightning(i, h, inp, states[f"mem{self.state_of[r]}"])
@@ -451,7 +453,9 @@ class FikeraxModel:
                 # (the residual in front of the embedding that a further pass adds)
                 layers_out.append(x[:, 0] - self.embed[inp.input_ids.long()].float() * cfg.embed_scale if into.get("again")
                                   else x[:, 0].clone())
-        return proj_f32out(N.hyper_read(x, inp.logits_idx, self.final_norm, eps, dt), self.head)
+        if inp.logits_idx is not None:
+            h = N.hyper_read(x, inp.logits_idx, self.final_norm, eps, dt)
+        return proj_f32out(h, self.head)
 
 
 def random_tensors(cfg: FikeraxConfig, seed: int = 0, device="cpu") -> Dict[str, torch.Tensor]:

@@ -437,7 +437,9 @@ class LizesunModel:
         vmix: dict = {}
         tables: dict = {}
         for li, (spec, L) in enumerate(zip(cfg.layers, self.layers)):
-            nxt = self.layers[li + 1]["norm1"] if li + 1 < nl else (1.0, None, None)   # the final norm: wanted rows only
+            # (the final norm reads the wanted rows only, or with the last layer where every row is wanted)
+            nxt = (self.layers[li + 1]["norm1"] if li + 1 < nl
+                   else (1.0, None, None) if inp.logits_idx is not None else self.final_norm)
             after = L["norm2"] if spec.ff else nxt
             if spec.kind == "parallel":
                 ol, orr = self._parallel(li, h, inp, kcs, vcs, vts, states, tables)
@@ -454,8 +456,9 @@ class LizesunModel:
                 h = N.add_dyt(x, y, 1.0, None, 1.0, *nxt, out_dtype=dt)
             if layers_out is not None:
                 layers_out.append(x.clone())
-        xr = x.index_select(0, inp.logits_idx).contiguous()
-        h = N.add_dyt(xr, None, 1.0, None, 1.0, *self.final_norm, out_dtype=dt)
+        if inp.logits_idx is not None or not nl:
+            xr = x.index_select(0, inp.logits_idx).contiguous() if inp.logits_idx is not None else x
+            h = N.add_dyt(xr, None, 1.0, None, 1.0, *self.final_norm, out_dtype=dt)
         return proj_f32out(h, self.lm_head)
 
 

@@ -560,7 +560,7 @@ class SegStepInputs:
     positions: torch.Tensor        # [T] int32
     slots: torch.Tensor            # [T] int32 cache slot (page * BS + offset) of every row
     seg: SegMeta
-    logits_idx: torch.Tensor       # [n] int64 rows whose logits are needed
+    logits_idx: Optional[torch.Tensor]   # [n] int64 rows whose logits are needed (None, captured steps: every row, in order)
 
 
 def short_conv(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], tail: torch.Tensor, seg: SegMeta,
