@@ -161,7 +161,7 @@ class LLMEngine(SchedulerMixin, StepExecMixin, GraphRunnerMixin, SamplerMixin):
         self._mask_ver = -1
         self._graphs: Dict[tuple, tuple] = {}
         self._graph_pool = None
-        # graphs of models in the segment layout: (rows, block-table width) -> (graph, static input, logits)
+        # graphs of models in the segment layout: (rows, block-table width, weight loads) -> (graph, static input, logits, step)
         self._seg_graphs: Dict[tuple, tuple] = {}
         self._seg_seen: Dict[tuple, int] = {}
         self._seg_stream = None

@@ -263,11 +263,11 @@ class GraphRunnerMixin:
         pages, work items -- is read from one static buffer that each step fills with one copy.  The logits are copied
         out: what a step returns stays the caller's."""
         B, BS = len(decode), self.kv.block_size
-        if B > max(self.cfg.graph_batch_sizes) or len(set(id(s) for s, _ in decode)) != B:
-            return None
+        if B > max(self.cfg.graph_batch_sizes) or len(set(id(s) for s, _ in decode)) != B or KNOBS.sync_debug:
+            return None                        # (a capture has no room for the synchronisation behind every launch)
         pages = max(s.n_cached + j for s, j in decode) // BS + 1
         width = 1 << (pages - 1).bit_length() if pages <= 8 else -(-pages // 8) * 8 if pages <= 128 else -(-pages // 32) * 32
-        key = (B, width)
+        key = (B, width, self.model.loads)
         got = self._seg_graphs.pop(key, None)
         if got is None:
             if len(self._seg_seen) > 4096:

@@ -204,6 +204,7 @@ class FikeraxModel:
     step_layout = "segments"   # the engine packs steps as segments (ops.seq_ops.SegStepInputs)
     graph_capturable = False
     segment_graphs = True      # steps of single tokens replay HIP graphs (engine/graph_runner.py)
+    loads = 0                  # times weights were loaded: a graph reads those it was captured with
 
     def __init__(self, cfg: FikeraxConfig, device, dtype=torch.bfloat16, pc: Optional[ParallelContext] = None,
                  seed: int = 0, init: bool = True):
@@ -322,6 +323,7 @@ class FikeraxModel:
         """Build the fused device layout from checkpoint tensors (``get(name)`` -> tensor; names of the
         safetensors file: ``embed``, ``l<i>.norm1``, ``l<i>.mix.q``, ``l<i>.mlp.gate`` ...)."""
         cfg, dev, dt = self.cfg, self.device, self.dtype
+        self.loads += 1
 
         def put(*names, dtype=dt):
             ts = [get(n) for n in names]

@@ -78,3 +78,31 @@ def test_generation_with_and_without_graphs(model):
         texts.append(done)
         assert (eng.stats["graph_steps"] > 0) == graphs
     assert texts[0] == texts[1] and len(texts[0]) == 3
+
+
+@pytest.mark.parametrize("model", ["tiny-fikerax", "tiny-lizesun"])
+def test_weights_loaded_after_capture_are_used(model):
+    """A graph reads the weights it was captured with: new ones are captured anew; rows without wanted logits replay too."""
+    engines = [engine(model, torch.bfloat16, graphs) for graphs in (True, False)]
+    sids = [eng.new_sequence() for eng in engines]
+    for n in (9, *[1] * 8):
+        a, b = (eng.feed([(s, list(range(n)), [n - 1])]) for eng, s in zip(engines, sids))
+        assert torch.equal(a, b)
+    assert engines[0].stats["captures"] == 1
+    for eng in engines:
+        eng.model._random_init(11)
+    for _ in range(8):
+        a, b = (eng.feed([(s, [5], [0])]) for eng, s in zip(engines, sids))
+        assert torch.equal(a, b)
+    assert engines[0].stats["captures"] == 2
+    a, b = (eng.feed([(s, [5], [])]) for eng, s in zip(engines, sids))
+    assert a.shape == b.shape and a.shape[0] == 0
+
+
+def test_a_check_behind_every_launch_runs_steps_eagerly(monkeypatch):
+    monkeypatch.setattr(G.KNOBS, "sync_debug", True)
+    eng = engine("tiny-fikerax", torch.bfloat16, True)
+    sid = eng.new_sequence()
+    for _ in range(6):
+        eng.feed([(sid, [3], [0])])
+    assert eng.stats["captures"] == 0
