@@ -419,6 +419,7 @@ def low_rank_pair(x: torch.Tensor, c0: int, w0: torch.Tensor, c1: int, w1: torch
 ROWS_PART = 128     # visible keys per part of the vector-pipe attention
 ROWS_HEADS = 8      # heads of one key head per workgroup of it
 ROWS_FILL = 512     # workgroups from which it walks a row's parts itself
+ROWS_SCRATCH = 1 << 28      # floats of partial results past which it does so as well (1 GiB)
 
 
 def _rows_parts(seg: SegMeta, T: int, heads: int, per_key: int, V: int, dev, chunk: int = 0, window: int = 0,
@@ -437,7 +438,7 @@ def _rows_parts(seg: SegMeta, T: int, heads: int, per_key: int, V: int, dev, chu
     if window > 0:
         most = min(most, window + keep_first)
     parts = -(-most // ROWS_PART)
-    if parts <= 1:
+    if parts <= 1 or T * heads * parts * (V + 2) > ROWS_SCRATCH:
         return 0, None, None
     return (parts, scratch(T * heads * parts * V, torch.float32, dev), scratch(T * heads * parts * 2, torch.float32, dev))
 
@@ -578,7 +579,7 @@ def short_conv(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], tail
         d = _dt(x.dtype)
         items = seg.tile_items(WINDOW_TILE)      # rows in tiles of one segment: metadata once per tile
         lens = [b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:])]
-        one = items.shape[0] == seg.n_seg and min(lens) > 0      # a tile per segment
+        one = items.shape[0] == seg.n_seg and min(lens, default=0) > 0      # a tile per segment
         check(lib().k8s_short_conv(ptr(x), x.stride(0), d, ptr(w), ptr(b), ptr(tail), ptr(seg.row_seg),
                                    ptr(seg.seg_row0), ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(out), T, seg.n_seg, C,
                                    taps, int(act), d, stream_ptr(x), ptr(items), items.shape[0], int(one)), "short_conv")
@@ -1398,7 +1399,7 @@ def matrix_memory(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tens
 # 9.4 / 5.8, 11.0 / 6.0, 40.1 / 28.4, 142 / 107 (the states' bytes, in and out: 0.4, 3.4, 27, 109).
 def _step_ok(x: torch.Tensor, seg: SegMeta, D: int, V: int, gate: torch.Tensor, w: Optional[torch.Tensor]) -> bool:
     return (use_hip(x) and seg.n_seg == x.shape[0] and seg.row0_host[-1] == seg.n_seg and D in (64, 128) and V in (64, 128)
-            and min(b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:])) == 1
+            and min((b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:])), default=0) == 1
             and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0
             and gate.stride(1) == 1 and gate.stride(0) % 4 == 0 and gate.data_ptr() % 16 == 0
             and (w is None or (w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0)))

@@ -102,3 +102,17 @@ def test_latent_rows(H, R, P, window):
     p = weights(s, vis[:, None], sink)
     want = torch.einsum("thj,jr->thr", p, c[:, :R].double()) * torch.sigmoid(gate[rows].double())[..., None]
     assert float((full[rows].double().cpu() - want).abs().max()) < 2e-5 * float(want.abs().max())
+
+
+def test_partial_results_stay_bounded(monkeypatch):
+    """Past ROWS_SCRATCH floats of partial results a workgroup walks its row's parts itself: the same bits."""
+    n, H, D, dev = 300, 4, 16, torch.device("cuda")
+    g = torch.Generator().manual_seed(2)
+    q, kc, vc = (torch.randn(*s, generator=g).to(dev) for s in ((3, H * D), (11, BS, D), (11, BS, D)))
+    seg = meta([3], [n], [list(range(11))[:10]], dev)
+    args = (q, H, 1, D, D, kc, vc, seg, D ** -0.5)
+    assert S._rows_parts(seg, 3, H, H, D, dev)[0] == 3
+    a = S.masked_attention(*args)
+    monkeypatch.setattr(S, "ROWS_SCRATCH", 3 * H * 3 * (D + 2) - 1)
+    assert S._rows_parts(seg, 3, H, H, D, dev)[0] == 0
+    assert torch.equal(a, S.masked_attention(*args))
