@@ -59,11 +59,33 @@ def select_gemm(M: int, N: int, K: int, x_ok_layout: bool = True, out_contig: bo
     return KIND_LIB, 0, 1
 
 
+# fp32 products of a few rows (csrc/kernels/few_rows_f32.hip).  Up to 8 rows, for wide weights up to 5: each row is read by
+# every workgroup, so past that a wide weight is no faster.  us, library / this at 1, 2, 4, 8 rows: 2048 x 2048 12.0 / 4.9,
+# 12.1 / 5.2, 12.1 / 5.8, 12.2 / 7.1;  2048 x 8192 22.9 / 12.5, 23.3 / 12.7, 22.9 / 13.5, 23.3 / 17.2;  3072 x 768 7.2 / 3.8,
+# 8.4 / 4.1, 8.3 / 4.4, 7.3 / 5.3;  16384 x 2048 31.7 / 20.7, 32.0 / 20.7, 31.8 / 24.1, 32.2 / 30.8;  8192 x 2048 at 5, 6, 8
+# rows 16.2 / 14.9, 16.2 / 16.2, 16.4 / 17.5.  (16384 x 2048 at 20.7 is 6.5 TB/s: part of the weights stays in the caches.)
+FEW_F32_ROWS = 8
+FEW_F32_WIDE = 8192, 5
+
+
+def _few_f32_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    (M, K), N = x.shape, w.shape[0]
+    return (x.is_cuda and w.is_cuda and x.dtype == torch.float32 == w.dtype
+            and 0 < M <= (FEW_F32_WIDE[1] if N >= FEW_F32_WIDE[0] else FEW_F32_ROWS) and N > 0 and K > 0 and K % 4 == 0
+            and w.dim() == 2 and w.shape[1] == K and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.stride(0) >= K and x.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
-    """``x @ w.T`` for ``x`` [M, K] and ``w`` [N, K] (bf16)."""
+    """``x @ w.T`` for ``x`` [M, K] and ``w`` [N, K]."""
     M, K = x.shape
     N = w.shape[0]
     if not (x.is_cuda and x.dtype == torch.bfloat16):
+        if out is None and _few_f32_ok(x, w):
+            out = torch.empty((M, N), dtype=torch.float32, device=x.device)
+            check(lib().k8s_few_rows_f32(ptr(x), x.stride(0), ptr(w), ptr(out), M, N, K, stream_ptr(x)), "few_rows_f32")
+            return out
         return lib_gemm(x, w, out)
     layout = x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
     kind, cfg, splits = select_gemm(M, N, K, layout, out is None or out.is_contiguous())
