@@ -1,7 +1,7 @@
 // Small products of a few rows (reply steps), on the vector pipes: a matrix of a quarter megabyte a head or less, whose
 // time is the launch and one trip to memory.
 //
-// head_proj:  out[t][h][n] = sum_k a[t][h][k] w[h][k][n], bf16 with fp32 sums (a latent layer's query into latent space,
+// head_proj:  out[t][h][n] = sum_k a[t][h][k] w[h][k][n], bf16 or fp32 with fp32 sums (a latent layer's query into latent space,
 //   its output out of it), and, in the same launch, the rotated key part's queries: the RD entries behind a[t][h][0 .. K)
 //   turned in neighbouring pairs by cs [t][RD] (cos | sin), filled up with zeros to RP.
 // low_rank_pair:  out_i[t][n] = sum_k bf16(x[t][c_i + k]) w_i[n][k] for two column ranges of the same fp32 rows.
@@ -12,31 +12,52 @@
 
 namespace k8s {
 
+template <typename TX>
 struct HeadProjArgs {
-  const uint16_t* a;      // element (t, h, k) at t * ast + h * ash + k
+  const TX* a;            // element (t, h, k) at t * ast + h * ash + k
   long ast, ash;
-  const uint16_t* w;      // [H][K][N]
-  uint16_t* out;          // element (t, h, n) at t * ost + h * osh + n
+  const TX* w;            // [H][K][N]
+  TX* out;                // element (t, h, n) at t * ost + h * osh + n
   long ost, osh;
   int T, H, K, N;
   const float* cs;
-  uint16_t* qr;           // [T][H][RP] or null
+  TX* qr;                 // [T][H][RP] or null
   int RD, RP;
 };
 
+__device__ __forceinline__ float ldx(const uint16_t* p) { return bf2f(*p); }
+__device__ __forceinline__ float ldx(const float* p) { return *p; }
+__device__ __forceinline__ void stx(uint16_t* p, float v) { *p = f2bf(v); }
+__device__ __forceinline__ void stx(float* p, float v) { *p = v; }
+// two neighbouring weights as they lie in memory
+template <typename TX>
+struct Pair;
+template <>
+struct Pair<uint16_t> {
+  uint32_t v;
+  __device__ __forceinline__ float lo() const { return bf2f((uint16_t)v); }
+  __device__ __forceinline__ float hi() const { return bf2f((uint16_t)(v >> 16)); }
+};
+template <>
+struct alignas(8) Pair<float> {
+  float a, b;
+  __device__ __forceinline__ float lo() const { return a; }
+  __device__ __forceinline__ float hi() const { return b; }
+};
+
 // U: weight rows in flight per thread
-template <int TR, int U>
-__global__ void __launch_bounds__(256) head_proj_kernel(HeadProjArgs a) {
+template <int TR, int U, typename TX>
+__global__ void __launch_bounds__(256) head_proj_kernel(HeadProjArgs<TX> a) {
   extern __shared__ float smem[];                          // [K][TR], then [8][TR][64]
   const int tid = threadIdx.x, c = 2 * (tid & 31), kg = tid >> 5, n0 = blockIdx.x * 64, h = blockIdx.y;
   const int t0 = blockIdx.z * TR, nt = min(TR, a.T - t0), KG = a.K / 8;
-  const uint16_t* wp = a.w + ((size_t)h * a.K + (size_t)kg * KG) * a.N + n0 + c;
-  uint32_t wv[U];
+  const TX* wp = a.w + ((size_t)h * a.K + (size_t)kg * KG) * a.N + n0 + c;
+  Pair<TX> wv[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) wv[u] = *reinterpret_cast<const uint32_t*>(wp + (size_t)min(u, KG - 1) * a.N);
+  for (int u = 0; u < U; ++u) wv[u] = *reinterpret_cast<const Pair<TX>*>(wp + (size_t)min(u, KG - 1) * a.N);
   for (int e = tid; e < a.K * TR; e += 256) {
     const int k = e % a.K, t = e / a.K;
-    smem[k * TR + t] = t < nt ? bf2f(a.a[(size_t)(t0 + t) * a.ast + (size_t)h * a.ash + k]) : 0.f;
+    smem[k * TR + t] = t < nt ? ldx(a.a + (size_t)(t0 + t) * a.ast + (size_t)h * a.ash + k) : 0.f;
   }
   if (a.qr && blockIdx.x == 0) {
     const int hp = a.RP >> 1, half = a.RD >> 1;
@@ -44,14 +65,14 @@ __global__ void __launch_bounds__(256) head_proj_kernel(HeadProjArgs a) {
       const int t = t0 + e / hp, i = e % hp;
       float x = 0.f, y = 0.f;
       if (i < half) {
-        const uint16_t* p = a.a + (size_t)t * a.ast + (size_t)h * a.ash + a.K + 2 * i;
-        const float u = bf2f(p[0]), v = bf2f(p[1]), co = a.cs[(size_t)t * a.RD + i], si = a.cs[(size_t)t * a.RD + half + i];
+        const TX* p = a.a + (size_t)t * a.ast + (size_t)h * a.ash + a.K + 2 * i;
+        const float u = ldx(p), v = ldx(p + 1), co = a.cs[(size_t)t * a.RD + i], si = a.cs[(size_t)t * a.RD + half + i];
         x = u * co - v * si;
         y = v * co + u * si;
       }
-      uint16_t* q = a.qr + ((size_t)t * a.H + h) * a.RP + 2 * i;
-      q[0] = f2bf(x);
-      q[1] = f2bf(y);
+      TX* q = a.qr + ((size_t)t * a.H + h) * a.RP + 2 * i;
+      stx(q, x);
+      stx(q + 1, y);
     }
   }
   __syncthreads();
@@ -59,12 +80,12 @@ __global__ void __launch_bounds__(256) head_proj_kernel(HeadProjArgs a) {
   for (int k0 = 0; k0 < KG; k0 += U) {
     if (k0 > 0) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) wv[u] = *reinterpret_cast<const uint32_t*>(wp + (size_t)min(k0 + u, KG - 1) * a.N);
+      for (int u = 0; u < U; ++u) wv[u] = *reinterpret_cast<const Pair<TX>*>(wp + (size_t)min(k0 + u, KG - 1) * a.N);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (k0 + u < KG) {
-        const float w0 = bf2f((uint16_t)wv[u]), w1 = bf2f((uint16_t)(wv[u] >> 16));
+        const float w0 = wv[u].lo(), w1 = wv[u].hi();
         const float* xs = smem + (kg * KG + k0 + u) * TR;
 #pragma unroll
         for (int t = 0; t < TR; ++t) {
@@ -84,7 +105,7 @@ __global__ void __launch_bounds__(256) head_proj_kernel(HeadProjArgs a) {
     float v = 0.f;
 #pragma unroll
     for (int g = 0; g < 8; ++g) v += smem[g * TR * 64 + e];
-    a.out[(size_t)(t0 + e / 64) * a.ost + (size_t)h * a.osh + n0 + e % 64] = f2bf(v);
+    stx(a.out + (size_t)(t0 + e / 64) * a.ost + (size_t)h * a.osh + n0 + e % 64, v);
   }
 }
 
@@ -149,24 +170,30 @@ using namespace k8s;
     __VA_ARGS__;                  \
   }
 
-// K % 8 == 0 up to 1024, N % 64 == 0; qr null: no rotated part.
-K8S_API int k8s_head_proj(const void* x, long ast, long ash, const void* w, void* out, long ost, long osh, int T, int H,
-                          int K, int N, const float* cs, void* qr, int RD, int RP, hipStream_t s) {
-  if (T <= 0) return 0;
-  if (H < 1 || K < 8 || K % 8 || K > 1024 || N < 64 || N % 64 || (uintptr_t)w % 4 ||
-      (qr && (RD < 0 || RD % 2 || RP % 2 || RP < RD || (RD && !cs))))
-    return (int)hipErrorInvalidValue;
-  HeadProjArgs a{(const uint16_t*)x, ast, ash, (const uint16_t*)w, (uint16_t*)out, ost, osh, T, H, K, N, cs, (uint16_t*)qr,
-                 RD, RP};
+template <typename TX>
+static int head_proj_launch(const void* x, long ast, long ash, const void* w, void* out, long ost, long osh, int T, int H,
+                            int K, int N, const float* cs, void* qr, int RD, int RP, hipStream_t s) {
+  HeadProjArgs<TX> a{(const TX*)x, ast, ash, (const TX*)w, (TX*)out, ost, osh, T, H, K, N, cs, (TX*)qr, RD, RP};
   K8S_TR(K > 128 && T > 4 ? 4 : T, {
     const size_t lds = sizeof(float) * TR * (K > 512 ? K : 512);
     const dim3 grid(N / 64, H, (T + TR - 1) / TR);
     if (K <= 128)
-      hipLaunchKernelGGL((head_proj_kernel<TR, 16>), grid, dim3(256), lds, s, a);
+      hipLaunchKernelGGL((head_proj_kernel<TR, 16, TX>), grid, dim3(256), lds, s, a);
     else
-      hipLaunchKernelGGL((head_proj_kernel<TR, 32>), grid, dim3(256), lds, s, a);
+      hipLaunchKernelGGL((head_proj_kernel<TR, 32, TX>), grid, dim3(256), lds, s, a);
   });
   return (int)hipGetLastError();
+}
+
+// K % 8 == 0 up to 1024, N % 64 == 0; qr null: no rotated part.  dt: 0 bf16, 1 fp32.
+K8S_API int k8s_head_proj(const void* x, long ast, long ash, const void* w, void* out, long ost, long osh, int T, int H,
+                          int K, int N, const float* cs, void* qr, int RD, int RP, int dt, hipStream_t s) {
+  if (T <= 0) return 0;
+  if (H < 1 || K < 8 || K % 8 || K > 1024 || N < 64 || N % 64 || dt < 0 || dt > 1 || (uintptr_t)w % (dt ? 8 : 4) ||
+      (qr && (RD < 0 || RD % 2 || RP % 2 || RP < RD || (RD && !cs))))
+    return (int)hipErrorInvalidValue;
+  return (dt ? head_proj_launch<float> : head_proj_launch<uint16_t>)(x, ast, ash, w, out, ost, osh, T, H, K, N, cs, qr, RD,
+                                                                     RP, s);
 }
 
 // K0, K1 % 32 == 0 up to 1024; weights 16-byte aligned.

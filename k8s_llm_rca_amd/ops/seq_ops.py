@@ -360,7 +360,8 @@ def rotated_tail(q: torch.Tensor, cs: torch.Tensor, H: int, N: int, pad: int) ->
 
 # Rows up to which small products run on the vector pipes (csrc/kernels/small_proj.hip).  us, library / this, at 1, 16, 64,
 # 128 rows: 16 heads 128 -> 256 with the rotated part 7.3 / 3.1, 7.3 / 4.7, 9.1 / 5.5, 9.6 / 7.2;  256 -> 128 6.9 / 3.4,
-# 6.3 / 5.2, 6.5 / 5.6, 7.4 / 6.9;  two of 64 -> 2048 with their roundings 12.2 / 2.5, 11.8 / 3.6, 12.4 / 4.0, 12.2 / 5.5.
+# 6.3 / 5.2, 6.5 / 5.6, 7.4 / 6.9, in fp32 6.5 / 3.4, 6.6 / 5.1, 11.9 / 5.8, 20 / 8.1 and 9.5 / 4.4, 8.5 / 5.7, 11.4 / 6.8,
+# 18.8 / 9.3;  two of 64 -> 2048 with their roundings 12.2 / 2.5, 11.8 / 3.6, 12.4 / 4.0, 12.2 / 5.5.
 SMALL_PROJ_ROWS = 128
 
 
@@ -368,15 +369,21 @@ def _small_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     return use_hip(x) and 0 < x.shape[0] <= SMALL_PROJ_ROWS and w.dtype == torch.bfloat16 and w.is_contiguous()
 
 
+def _small_heads(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (use_hip(x) and 0 < x.shape[0] <= SMALL_PROJ_ROWS and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float32)
+            and w.is_contiguous() and w.data_ptr() % 8 == 0
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+
+
 def head_proj(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """``out[t, h] = x[t, h] @ w[h]`` of ``x`` [T, H, K] and ``w`` [H, K, N] (the strides of ``x`` and ``out`` [T, H, N]
-    but the last are free): a kernel of one launch for few rows of bf16, the library's batched product otherwise."""
+    but the last are free): a kernel of one launch for few rows, the library's batched product otherwise."""
     T, H, K = x.shape
     N = w.shape[2]
-    if (_small_rows(x, w) and x.dtype == torch.bfloat16 == out.dtype and x.stride(2) == 1 == out.stride(2) and K % 8 == 0
+    if (_small_heads(x, w) and x.dtype == out.dtype and x.stride(2) == 1 == out.stride(2) and K % 8 == 0
             and K <= 1024 and N % 64 == 0):
         check(lib().k8s_head_proj(ptr(x), x.stride(0), x.stride(1), ptr(w), ptr(out), out.stride(0), out.stride(1), T, H, K,
-                                  N, None, None, 0, 0, stream_ptr(x)), "head_proj")
+                                  N, None, None, 0, 0, _dt(x.dtype), stream_ptr(x)), "head_proj")
     else:
         torch.bmm(x.transpose(0, 1), w, out=out.transpose(0, 1))
     return out
@@ -389,14 +396,14 @@ def latent_queries(q: torch.Tensor, uk: torch.Tensor, cs: Optional[torch.Tensor]
     T, KR = q.shape[0], uk.shape[2]
     x = q.view(T, H, -1)
     R = x.shape[2] - D
-    if _small_rows(q, uk) and q.dtype == torch.bfloat16 and q.is_contiguous() and D % 8 == 0 and D <= 1024 and KR % 64 == 0:
+    if _small_heads(q, uk) and q.is_contiguous() and D % 8 == 0 and D <= 1024 and KR % 64 == 0:
         qa = torch.empty(H, T, KR, dtype=q.dtype, device=q.device).transpose(0, 1)
         qr = None
         if R:
             assert cs.dtype == torch.float32 and cs.is_contiguous() and cs.shape == (T, R) and pad >= R and pad % 2 == 0
             qr = torch.empty(T, H, pad, dtype=q.dtype, device=q.device)
         check(lib().k8s_head_proj(ptr(q), x.stride(0), x.stride(1), ptr(uk), ptr(qa), qa.stride(0), qa.stride(1), T, H, D,
-                                  KR, ptr(cs), ptr(qr), R, pad if R else 0, stream_ptr(q)), "head_proj")
+                                  KR, ptr(cs), ptr(qr), R, pad if R else 0, _dt(q.dtype), stream_ptr(q)), "head_proj")
         return qa, qr
     qr = rotated_tail(q, cs, H, D, pad) if R else None
     return torch.bmm(x[:, :, :D].transpose(0, 1), uk).transpose(0, 1), qr

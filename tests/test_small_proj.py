@@ -12,28 +12,31 @@ def rnd(*shape, seed=0):
     return torch.randn(*shape, generator=torch.Generator().manual_seed(seed + sum(shape)))
 
 
-def close(got, want):
-    assert got.dtype == BF and got.shape == want.shape
-    assert bool(((got.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * float(want.abs().max())).all())
+def close(got, want, dt=BF):
+    """One rounding of the result, and fp32 sums."""
+    assert got.dtype == dt and got.shape == want.shape
+    ulp = 2.0 ** -8 if dt == BF else 2.0 ** -24
+    assert bool(((got.double().cpu() - want).abs() <= ulp * want.abs() + 1e-5 * float(want.abs().max())).all())
 
 
 @pytest.mark.parametrize("T", [1, 3, 4, 5, 8, 9, 64, 128, 129])
 @pytest.mark.parametrize("H,D,R,KR,pad", [(16, 128, 64, 256, 64), (3, 40, 6, 64, 32), (2, 200, 0, 128, 0), (5, 8, 32, 192, 64)])
-def test_heads(T, H, D, R, KR, pad):
-    q, uk = rnd(T, H * (D + R)).to(BF), (rnd(H, D, KR) * D ** -0.5).to(BF)
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_heads(T, H, D, R, KR, pad, dt):
+    q, uk = rnd(T, H * (D + R)).to(dt), (rnd(H, D, KR) * D ** -0.5).to(dt)
     cs = rnd(T, R) if R else None
     qa, qr = S.latent_queries(q.cuda(), uk.cuda(), cs.cuda() if R else None, H, D, pad)
     x = q.view(T, H, D + R)
-    close(qa, torch.bmm(x[:, :, :D].double().transpose(0, 1), uk.double()).transpose(0, 1))
+    close(qa, torch.bmm(x[:, :, :D].double().transpose(0, 1), uk.double()).transpose(0, 1), dt)
     assert qa.transpose(0, 1).is_contiguous()
     if R:
         assert torch.equal(qr, S.rotated_tail(q.cuda(), cs.cuda(), H, D, pad))
     else:
         assert qr is None
     # out of latent space: head-major in, token-major out
-    uv = (rnd(H, KR, 64) * KR ** -0.5).to(BF)
-    out = torch.empty(T, H, 64, dtype=BF, device="cuda")
-    close(S.head_proj(qa, uv.cuda(), out), torch.bmm(qa.double().cpu().transpose(0, 1), uv.double()).transpose(0, 1))
+    uv = (rnd(H, KR, 64) * KR ** -0.5).to(dt)
+    out = torch.empty(T, H, 64, dtype=dt, device="cuda")
+    close(S.head_proj(qa, uv.cuda(), out), torch.bmm(qa.double().cpu().transpose(0, 1), uv.double()).transpose(0, 1), dt)
 
 
 @pytest.mark.parametrize("T", [1, 4, 7, 64, 128, 129])
