@@ -11,7 +11,8 @@
 //
 // tile_*_kernel, one workgroup per (tile, head), all tiles at once: Q G, K G, (K G_(j,15])^T, P, T = (I + A)^-1 diag(beta)
 // and G_15 into a workspace.  The products over (j, i] are formed by multiplying decays, never as ratios or exponentials of
-// differences, so that they hold for any decay; T by forward substitution.
+// differences, so that they hold for any decay; T by forward substitution.  A value that is not finite reaches its own and
+// later tokens, never earlier ones (lower_rows), as token by token.
 // tile_state_kernel, one workgroup per (segment, head, 64 columns), walks the tiles of its segment.  A wave holds the state
 // of 16 columns in accumulators: tile dt, rows d = 16 dt + 4 hq + i, column r (lane = 16 hq + r).  A contraction may take
 // its index in any order that both operands agree on, so register i of accumulator dt IS the second operand of the step
@@ -259,6 +260,27 @@ __global__ void __launch_bounds__(256) tile_memory_kernel(TileArgs p) {
   w[W::p + tid] = s;
 }
 
+// Whether none of this lane's four numbers is infinite or NaN.
+__device__ __forceinline__ bool finite4(const f32x4& v) {
+  const float z = (v[0] * 0.f + v[1] * 0.f) + (v[2] * 0.f + v[3] * 0.f);
+  return z == z;
+}
+
+// c + A B for a lower triangular A [16][16] (af: its operand), row i from the rows of B up to i alone: a zero above the
+// diagonal times a number that is not finite would be NaN in the rows of earlier tokens.
+__device__ __forceinline__ f32x4 lower_rows(const f32x4& af, const f32x4& b, const f32x4& c, int hq) {
+  f32x4 out = c;
+#pragma unroll 1
+  for (int i = 0; i < kTs; ++i) {
+    f32x4 t = c;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t = __builtin_amdgcn_mfma_f32_16x16x4f32(af[e], 4 * hq + e <= i ? b[e] : 0.f, t, 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = 4 * hq + e == i ? t[e] : out[e];
+  }
+  return out;
+}
+
 template <int D, int KIND, typename TA>
 __global__ void __launch_bounds__(256) tile_state_kernel(TileArgs p) {
   using W = TileWs<D, KIND>;
@@ -335,7 +357,7 @@ __global__ void __launch_bounds__(256) tile_state_kernel(TileArgs p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) U = __builtin_amdgcn_mfma_f32_16x16x4f32(tf[i], R[i], U, 0, 0, 0);
     }
-    const f32x4 pf = *reinterpret_cast<const f32x4*>(b + oP + r * LT + 4 * hq);
+    const f32x4 pf = *reinterpret_cast<const f32x4*>(b + oP + r * LT + 4 * hq), Oq = O;
 #pragma unroll
     for (int i = 0; i < 4; ++i) O = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[i], U[i], O, 0, 0, 0);
 #pragma unroll
@@ -346,6 +368,12 @@ __global__ void __launch_bounds__(256) tile_state_kernel(TileArgs p) {
       for (int i = 0; i < 4; ++i) S[dt][i] *= ef[i];
 #pragma unroll
       for (int i = 0; i < 4; ++i) S[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(tf[i], U[i], S[dt], 0, 0, 0);
+    }
+    // Rare: the two triangular products row by row (the state takes in every token either way).  Behind the state's own
+    // products, off the chain from tile to tile.
+    if (__any(!finite4(U) || (KIND == 0 && !finite4(R)))) {
+      if (KIND == 0) U = lower_rows(*reinterpret_cast<const f32x4*>(b + oI + r * LT + 4 * hq), R, f32x4{0.f, 0.f, 0.f, 0.f}, hq);
+      O = lower_rows(*reinterpret_cast<const f32x4*>(b + oP + r * LT + 4 * hq), U, Oq, hq);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

@@ -118,3 +118,43 @@ def test_matrix_memory_in_tiles(H, D, V, lens, pos0, slots, cap):
     rel = 16 * 2.0 ** -24 * math.sqrt(max(lens)) + 2 * max(lens) * cap * 2.0 ** -24
     for got, e in zip(std, end):
         assert float((got.double().cpu() - e).abs().max()) < rel * float(e.abs().max())
+
+
+@gpu
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("rule,what", [("delta", w) for w in ("v", "q", "k", "decay", "beta")] +
+                         [("memory", w) for w in ("v", "q", "k")])
+@pytest.mark.parametrize("D,V", [(64, 72), (128, 16)])
+def test_what_is_not_finite_reaches_no_earlier_token(rule, what, value, D, V):
+    """Tokens in front of a value that is not finite keep their bits, and so do the other head and the other sequence; from
+    it on outputs and state are finite where they are token by token."""
+    H, lens, pos0, slots = 2, (37, 20), (4, 0), (1, 0)
+    T, g = sum(lens), torch.Generator().manual_seed(D)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g)
+    width = 2 * H * D + H * V + (H * V + 2 * H if rule == "memory" else 0)
+    x, a, beta, state, extra = rnd(T, width), rnd(T, H * D), rnd(T, H), rnd(2, H, D, V), [rnd(2, H, D), rnd(2, H)]
+
+    def run(dev, t=None):
+        xs, st, ex = x.clone(), state.clone().to(dev), [e.clone().to(dev) for e in extra]
+        al, bl = a.clone(), beta.clone()
+        if t is not None:       # of head 1: the last entry of its vector
+            dst, col = {"q": (xs, 2 * D - 1), "k": (xs, 2 * H * D - 1), "v": (xs, 2 * H * D + 2 * V - 1),
+                        "decay": (al, 2 * D - 1), "beta": (bl, 1)}[what]
+            dst[t, col] = value
+        m = seg_meta(lens, pos0, slots, dev)
+        if rule == "delta":
+            o = S.gated_delta(xs.to(dev), H, H, D, V, al.to(dev), torch.ones(H).to(dev), torch.zeros(H * D).to(dev),
+                              bl.to(dev), st, m)
+        else:
+            o = S.matrix_memory(xs.to(dev), H, D, V, torch.zeros(2 * H).to(dev), 5.0, st, *ex, m)
+        return o.view(T, H, V).cpu(), st.cpu()
+    clean, end = run("cuda")
+    for t in (5, 15, 30, 36):
+        got, st = run("cuda", t)
+        want, wst = run("cpu", t)
+        assert torch.equal(got[:t], clean[:t]) and torch.equal(got[lens[0]:], clean[lens[0]:])
+        assert torch.equal(got[:, 0], clean[:, 0]) and torch.equal(st[0], end[0])
+        assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+        assert torch.equal(torch.isfinite(st), torch.isfinite(wst))
