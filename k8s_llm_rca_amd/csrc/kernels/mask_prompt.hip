@@ -9,10 +9,16 @@
 // registers 8 s .. 8 s + 7 are the weights operand of O^T = V^T P^T as they stand.  LDS rows are padded by 16 bytes: the
 // 16 rows a quarter wave reads 16 bytes of lie in different banks for D = 64, 96 and 128 alike.
 //
+// Zero weights times values that are not finite are NaN in rows that do not see their keys.  A tile that ends with a result
+// that is not finite walks its keys once more (CARE): in blocks that some token does not see whole, such values are parked
+// as zeros, and added behind the walk where they are seen.  (Looking at every block's values on the way cost 3.5 %.)
+//
 // What bounds it: matrix and vector instructions of two waves a SIMD in turn (240 registers).  Eight prompts of 2048, 16
 // heads over 2 of 128, us: causal 245 = 561 TFLOP/s, a window of 1024 180 = 574, chunks of 1024 with capped scores 170 =
 // 405 (an exponential and a reciprocal more per score).  Tiles of 16 tokens x 2 heads a wave with operands from the caches
 // took 681, 485 and 418: every wave fetched its keys itself.
+#include <type_traits>
+
 #include "common.h"
 #include "key_runs.h"
 
@@ -35,16 +41,20 @@ struct MaskPromptArgs {
   float scale, softcap;
 };
 
+// of a pair of bf16 numbers: bits 15 and 31 set where one is infinite or NaN (an exponent of ones)
+__device__ __forceinline__ uint32_t mp_wild(uint32_t v) { return ((v & 0x7f807f80u) + 0x00800080u) & 0x80008000u; }
+
 __device__ __forceinline__ int mp_key(int reg, int hi) { return 16 * (reg >> 3) + 8 * hi + (reg & 7); }
 
 // HALF: BS is an odd multiple of 32, a block's halves may lie in two pages.
 template <int ND, int NV, int NW, bool CAP, bool HALF>
-__global__ void __launch_bounds__(64 * NW, 8 / NW) mask_prompt_kernel(MaskPromptArgs a) {
+__global__ void __launch_bounds__(64 * NW, ND == 4 && NV == 2 ? 3 : 2) mask_prompt_kernel(MaskPromptArgs a) {
   constexpr int D = ND * 16, V = NV * 32, TH = 64 * NW, KP = D * 2 + 16, VP = 144;
   constexpr int KC = 64 * D / 8 / TH, VC = V * 8 / TH;      // 16-byte chunks per thread and block
   static_assert(64 * D / 8 % TH == 0 && V * 8 % TH == 0, "whole chunks per thread");
   constexpr float kLog2e = 1.4426950408889634f;
   __shared__ __attribute__((aligned(16))) unsigned char lds[2][64 * KP + V * VP];
+  __shared__ int wild[NW];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 31, hi = lane >> 5;
   // key heads (and groups of 128 of their heads) next to each other, the last items first: they see the most keys
   const int hpg = a.H / a.G, hw = min(hpg, 32 * NW), nhc = (hpg + hw - 1) / hw, per = a.G * a.M * nhc;
@@ -79,11 +89,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) mask_prompt_kernel(MaskPrompt
 #pragma unroll
   for (int s = 0; s < ND; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + 16 * s);
   f32x16 o[NV];
-#pragma unroll
-  for (int dt = 0; dt < NV; ++dt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
-  float m = a.sink && valid ? a.sink[head] * kLog2e : -INFINITY, l = 0.f;
+  float m, l;
   // a scale that is not positive is applied before the mask and the maximum, a positive one in the exponent
   const float sc1 = a.scale * kLog2e, sc2 = sc1 > 0.f ? sc1 : 1.f, cap2 = a.softcap * kLog2e, icap = CAP ? 2.f * kLog2e * a.scale / a.softcap : 0.f;
 
@@ -108,7 +114,18 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) mask_prompt_kernel(MaskPrompt
   // the pages of a block's halves (a second half past the last key reads the first's)
   auto page0 = [&](int kb) { return pages[kb / a.BS]; };
   auto page1 = [&](int kb) { return HALF ? pages[(kb + 32 <= pos_last ? kb + 32 : kb) / a.BS] : 0; };
-  auto park = [&](int b) {
+  const int tl_lo = a.chunk > 0 ? (pos_last / a.chunk) * a.chunk : 0, tw_lo = a.window > 0 ? pos_last - a.window + 1 : 0;
+  auto open = [&](int kb) { return kb + 63 <= pos0 && kb >= tl_lo && (kb >= tw_lo || kb + 64 <= keep); };
+  auto park = [&](int b, int kb, auto care) {
+    if constexpr (decltype(care)::value) {
+      if (!open(kb)) {
+        uint32_t x[4 * VC];
+        __builtin_memcpy(x, stg + KC, sizeof(x));
+#pragma unroll
+        for (int i = 0; i < 4 * VC; ++i) x[i] &= ~((mp_wild(x[i]) >> 15) * 0xffffu);
+        __builtin_memcpy(stg + KC, x, sizeof(x));
+      }
+    }
 #pragma unroll
     for (int i = 0; i < KC; ++i) {
       const int c = tid + TH * i;
@@ -124,111 +141,149 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) mask_prompt_kernel(MaskPrompt
   // the queries are there before the loop: its waits count the block loads alone
 #pragma unroll
   for (int s = 0; s < ND; ++s) asm volatile("" ::"v"(qf[s]));
-  int kb_next = block_at(min(1, nblk - 1)), pg0 = page0(kb_next), pg1 = page1(kb_next);
-  {
-    const int kb = block_at(0);
-    load(kb, page0(kb), page1(kb));
-    park(0);
-  }
-  __syncthreads();
-  for (int bi = 0; bi < nblk; ++bi) {
-    const int kb = block_at(bi);
-    // the page of the block after the next, while this one is computed (the last ones are read again: every load is
-    // unconditional, so the count of loads in flight is known)
-    const int kb_after = block_at(min(bi + 2, nblk - 1)), pa0 = page0(kb_after), pa1 = page1(kb_after);
-    load(kb_next, pg0, pg1);
-    // a wave all of whose tokens come before the block, or after its window or chunk, has nothing to do
-    const bool live = wt0 < ntok && kb <= wp1 && kb + 63 >= cw_lo && (kb + 63 >= ww_lo || kb < keep);
-    if (live) {
-      const unsigned char *kl = lds[bi & 1], *vl = kl + 64 * KP;
-      f32x16 sc[2];
+  auto walk = [&](auto care) {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        const unsigned char* kr = kl + (32 * kt + krow) * KP + 16 * hi;
-        f32x16 acc;
+    for (int dt = 0; dt < NV; ++dt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+      for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+    m = a.sink && valid ? a.sink[head] * kLog2e : -INFINITY;
+    l = 0.f;
+    int kb_next = block_at(min(1, nblk - 1)), pg0 = page0(kb_next), pg1 = page1(kb_next);
+    {
+      const int kb = block_at(0);
+      load(kb, page0(kb), page1(kb));
+      park(0, kb, care);
+    }
+    __syncthreads();
+    for (int bi = 0; bi < nblk; ++bi) {
+      const int kb = block_at(bi);
+      // the page of the block after the next, while this one is computed (the last ones are read again: every load is
+      // unconditional, so the count of loads in flight is known)
+      const int kb_after = block_at(min(bi + 2, nblk - 1)), pa0 = page0(kb_after), pa1 = page1(kb_after);
+      load(kb_next, pg0, pg1);
+      // a wave all of whose tokens come before the block, or after its window or chunk, has nothing to do
+      const bool live = wt0 < ntok && kb <= wp1 && kb + 63 >= cw_lo && (kb + 63 >= ww_lo || kb < keep);
+      if (live) {
+        const unsigned char *kl = lds[bi & 1], *vl = kl + 64 * KP;
+        f32x16 sc[2];
 #pragma unroll
-        for (int s = 0; s < ND; ++s)
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kr + 32 * s), qf[s], acc, 0, 0, 0);
-        sc[kt] = acc;
-      }
-      if (CAP) {                                            // cap tanh(x), tanh(x) = 1 - 2 / (1 + e^(2x)), in log2 units
+        for (int kt = 0; kt < 2; ++kt) {
+          const unsigned char* kr = kl + (32 * kt + krow) * KP + 16 * hi;
+          f32x16 acc;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+          for (int s = 0; s < ND; ++s)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kr + 32 * s), qf[s], acc, 0, 0, 0);
+          sc[kt] = acc;
+        }
+        if (CAP) {                                            // cap tanh(x), tanh(x) = 1 - 2 / (1 + e^(2x)), in log2 units
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const float e = __builtin_amdgcn_exp2f(fminf(sc[kt][i] * icap, 60.f));
+              sc[kt][i] = cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + e));
+            }
+        } else if (!(sc1 > 0.f)) {
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc[kt][i] *= sc1;
+        }
+        if (!(full && kb + 63 <= wp0 && kb >= cl_lo && (kb >= wl_lo || kb + 64 <= keep))) {
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const int key = kb + 32 * kt + mp_key(i, hi);
+              const bool ok = key <= limit && key >= cq_lo && (key >= wq_lo || key < keep);
+              sc[kt][i] = ok ? sc[kt][i] : -INFINITY;
+            }
+        }
+        float cmax = sc[0][0];
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const float e = __builtin_amdgcn_exp2f(fminf(sc[kt][i] * icap, 60.f));
-            sc[kt][i] = cap2 * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + e));
-          }
-      } else if (!(sc1 > 0.f)) {
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) sc[kt][i] *= sc1;
-      }
-      if (!(full && kb + 63 <= wp0 && kb >= cl_lo && (kb >= wl_lo || kb + 64 <= keep))) {
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int key = kb + 32 * kt + mp_key(i, hi);
-            const bool ok = key <= limit && key >= cq_lo && (key >= wq_lo || key < keep);
-            sc[kt][i] = ok ? sc[kt][i] : -INFINITY;
-          }
-      }
-      float cmax = sc[0][0];
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) cmax = fmaxf(cmax, sc[kt][i]);
-      cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
-      // the reference moves only where a row's maximum outgrows it by 2^8: weights up to 256, exact in the sums, and most
-      // blocks leave the outputs alone
-      const float mc = CAP ? cmax : cmax * sc2;
-      const bool upd = mc > m + 8.f;
-      const float mn = upd ? mc : m, sub = mn == -INFINITY ? 0.f : -mn;
-      bf16x8 pf[2][2];
-      float ps = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float x = sc[kt][8 * s + j], e = __builtin_amdgcn_exp2f(CAP ? x + sub : fmaf(x, sc2, sub));
-            ps += e;
-            pf[kt][s][j] = (__bf16)e;
-          }
-      if (__any(upd)) {
-        const float alpha = upd ? __builtin_amdgcn_exp2f(m - mn) : 1.f;
-        l *= alpha;
-        m = mn;
-#pragma unroll
-        for (int dt = 0; dt < NV; ++dt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
-      }
-      l += ps;
-#pragma unroll
-      for (int dt = 0; dt < NV; ++dt) {
-        const unsigned char* vr = vl + (32 * dt + r) * VP + 16 * hi;
+          for (int i = 0; i < 16; ++i) cmax = fmaxf(cmax, sc[kt][i]);
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+        // the reference moves only where a row's maximum outgrows it by 2^8: weights up to 256, exact in the sums, and most
+        // blocks leave the outputs alone
+        const float mc = CAP ? cmax : cmax * sc2;
+        const bool upd = mc > m + 8.f;
+        const float mn = upd ? mc : m, sub = mn == -INFINITY ? 0.f : -mn;
+        bf16x8 pf[2][2];
+        float ps = 0.f;
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
           for (int s = 0; s < 2; ++s)
-            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(vr + 64 * kt + 32 * s),
-                                                            pf[kt][s], o[dt], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float x = sc[kt][8 * s + j], e = __builtin_amdgcn_exp2f(CAP ? x + sub : fmaf(x, sc2, sub));
+              ps += e;
+              pf[kt][s][j] = (__bf16)e;
+            }
+        if (__any(upd)) {
+          const float alpha = upd ? __builtin_amdgcn_exp2f(m - mn) : 1.f;
+          l *= alpha;
+          m = mn;
+#pragma unroll
+          for (int dt = 0; dt < NV; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+        }
+        l += ps;
+#pragma unroll
+        for (int dt = 0; dt < NV; ++dt) {
+          const unsigned char* vr = vl + (32 * dt + r) * VP + 16 * hi;
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+              o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(vr + 64 * kt + 32 * s),
+                                                              pf[kt][s], o[dt], 0, 0, 0);
+        }
       }
+      park((bi + 1) & 1, kb_next, care);
+      kb_next = kb_after;
+      pg0 = pa0;
+      pg1 = pa1;
+      __syncthreads();
     }
-    park((bi + 1) & 1);
-    kb_next = kb_after;
-    pg0 = pa0;
-    pg1 = pa1;
-    __syncthreads();
-  }
+  };
+  walk(std::false_type{});
+  float z = 0.f;
+#pragma unroll
+  for (int dt = 0; dt < NV; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z = fmaf(o[dt][i], 0.f, z);
+  const bool any = __any(z != z);
+  if (lane == 0) wild[w] = any;
+  __syncthreads();
+  bool care = false;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) care |= wild[i] != 0;
+  if (care) walk(std::true_type{});
   if (!valid) return;
   l += __shfl_xor(l, 32, 64);
+  if (care) {                                               // (a weight above zero leaves infinity and NaN what they are)
+    for (int bi = 0; bi < nblk; ++bi) {
+      const int kb = block_at(bi);
+      if (open(kb)) continue;
+      for (int key = kb; key < min(kb + 64, limit + 1); ++key) {
+        if (key < cq_lo || (key < wq_lo && key >= keep)) continue;
+        const uint16_t* vp = a.vt + ((size_t)pages[key / a.BS] * NVt + (size_t)gv * V + 4 * hi) * a.BS + key % a.BS;
+#pragma unroll
+        for (int dt = 0; dt < NV; ++dt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const uint16_t v = vp[(size_t)(32 * dt + 8 * (i >> 2) + (i & 3)) * a.BS];
+            if (mp_wild(v)) o[dt][i] += bf2f(v);
+          }
+      }
+    }
+  }
   if (a.sink) l += __builtin_amdgcn_exp2f(a.sink[head] * kLog2e - m);
   float f = 1.f / l;
   if (a.gate) f *= 1.f / (1.f + __expf(-a.gate[(size_t)(row0 + tt) * a.gs + head]));

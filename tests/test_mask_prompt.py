@@ -64,3 +64,44 @@ def test_prompts(H, G, D, V, maps, BS, kw):
     want = torch.bmm(p, vv.transpose(0, 1).contiguous()).transpose(0, 1) * torch.sigmoid(gate[:, 1:].double())[..., None]
     # the weights are rounded to bf16 (2^-9 each, of both signs) before they meet the values, the result once more
     assert float((got[1].double().cpu().view(T, HQ, V) - want).abs().max()) < 2.0 ** -7 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("H,G,D,V,BS", [(8, 1, 128, 128, 64), (2, 2, 64, 64, 32), (4, 2, 96, 96, 96)])
+@pytest.mark.parametrize("kw", [dict(), dict(window=50, keep_first=7), dict(chunk=40, softcap=9.0)])
+def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(H, G, D, V, BS, kw, value):
+    """One entry of one key's value, of a key at every place in a block: rows that do not see the key keep their bits, and so
+    do all other columns; keys that nobody has written are not read into the sums either."""
+    n, lead = 240, 60
+    g = torch.Generator().manual_seed(BS)
+    N = -(-n // BS)
+    kc, v = torch.randn(N, BS, G * D, generator=g).to(BF).cuda(), torch.randn(N * BS, G, V, generator=g).to(BF)
+    q, T = torch.randn(n - lead, H * D, generator=g).to(BF).cuda(), n - lead
+
+    def i32(x):
+        return torch.tensor(x, dtype=torch.int32, device="cuda")
+    m = S.SegMeta(1, i32([0] * T), i32([0, T]), i32([lead]), i32([0]), i32([list(range(N))]), [0, T], [lead], [0])
+    assert m.mask_items(max(1, 128 // (H // G)))[1].shape[0] > 0
+
+    def run(keys):
+        vx = v.clone()
+        vx[n:] = value
+        for t in keys:
+            vx[t, -1, V - 3] = value
+        vt = vx.view(N, BS, G * V).transpose(1, 2).contiguous().cuda()
+        return S.masked_attention(q, H, G, D, V, kc, None, m, D ** -0.5, vt=vt, out_f32=True, **kw).view(T, H, V)
+    clean = run([])
+    assert bool(torch.isfinite(clean).all())
+    pos = torch.arange(lead, n, device="cuda")
+    for keys in ([3], [70], [127], [128], [191], [239], [64, 160]):
+        got, sees = run(keys), torch.zeros(T, dtype=torch.bool, device="cuda")
+        for t in keys:
+            s = pos >= t
+            if "chunk" in kw:
+                s &= pos // kw["chunk"] == t // kw["chunk"]
+            if "window" in kw:
+                s &= (pos - t < kw["window"]) | (t < kw["keep_first"])
+            sees |= s
+        hit = torch.zeros_like(got, dtype=torch.bool)
+        hit[sees, (G - 1) * (H // G):, V - 3] = True
+        assert bool((got[~hit] == clean[~hit]).all()) and not bool(torch.isfinite(got[hit]).any())
