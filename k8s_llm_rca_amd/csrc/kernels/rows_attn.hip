@@ -65,11 +65,11 @@ struct RowsArgs {
   int n_parts;
 };
 
-// (m, l) and the outputs of a further part; the running maximum may be -inf, the part's is finite
+// (m, l) and the outputs of a further part; both maxima may be -inf (no key yet, a part whose scores all are)
 __device__ __forceinline__ void ra_join(float& m, float& l, float mp, float lp, float& a, float& b) {
-  const float mn = fmaxf(m, mp);
-  a = expf(m - mn);
-  b = expf(mp - mn);
+  const float mn = fmaxf(m, mp), ms = mn == -INFINITY ? 0.f : mn;
+  a = expf(m - ms);
+  b = expf(mp - ms);
   l = fmaf(l, a, __fmul_rn(lp, b));
   m = mn;
 }
@@ -165,8 +165,8 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
     __syncthreads();
     for (int h = wv; h < nh; h += 4) {              // the part's softmax, a wave per head
       const float s0 = sp[h * kRaKeys + lane], s1 = sp[h * kRaKeys + 64 + lane];
-      const float mp = wave_max(fmaxf(s0, s1));     // finite: a part holds a visible key
-      const float e0 = expf(s0 - mp), e1 = expf(s1 - mp);
+      const float mp = wave_max(fmaxf(s0, s1)), ms = mp == -INFINITY ? 0.f : mp;
+      const float e0 = expf(s0 - ms), e1 = expf(s1 - ms);
       sp[h * kRaKeys + lane] = e0;
       sp[h * kRaKeys + 64 + lane] = e1;
       const float lp = wave_sum(e0 + e1);
@@ -180,11 +180,10 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
       float op[kRaHeads];
 #pragma unroll
       for (int k = 0; k < kRaHeads; ++k) op[k] = 0.f;
-      const int nk4 = (nk + 3) & ~3;                // (weights past nk are zero, their slots repeat the last)
-      for (int j = 0; j < nk4; j += 4) {
+      auto four = [&](int j, int n) {               // keys j .. j + n of the part
         float v[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = rld(vbase, (size_t)ss[j + e] * p.vs);
+        for (int e = 0; e < 4; ++e) v[e] = e < n ? rld(vbase, (size_t)ss[j + e] * p.vs) : 0.f;
 #pragma unroll
         for (int k = 0; k < kRaHeads; ++k) {
           const int h = hs + k * tpc;
@@ -194,7 +193,10 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
             for (int e = 0; e < 4; ++e) op[k] = fmaf(w[e], v[e], op[k]);
           }
         }
-      }
+      };
+      const int nk4 = nk & ~3;
+      for (int j = 0; j < nk4; j += 4) four(j, 4);
+      if (nk4 < nk) four(nk4, nk - nk4);            // (weights past nk are zero, and zero times an infinity would be NaN)
 #pragma unroll
       for (int k = 0; k < kRaHeads; ++k) {
         const int h = hs + k * tpc;

@@ -116,3 +116,32 @@ def test_partial_results_stay_bounded(monkeypatch):
     monkeypatch.setattr(S, "ROWS_SCRATCH", 3 * H * 3 * (D + 2) - 1)
     assert S._rows_parts(seg, 3, H, H, D, dev)[0] == 0
     assert torch.equal(a, S.masked_attention(*args))
+
+
+@pytest.mark.parametrize("alone", [True, False])
+@pytest.mark.parametrize("n", [1, 3, 130, 258])
+def test_infinite_keys_and_values(n, alone):
+    """An infinite value of the last visible key makes its column infinite, and keys whose scores are all minus infinity weigh
+    nothing beside others -- by themselves, in a part of their own or as a whole part in front."""
+    H, D, pages, dev = 2, 8, 10, "cuda"
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(n, H * D, generator=g) for _ in range(3))
+    q[:, ::D] = 1.0
+    k[:128, ::D] = -math.inf                              # rows up to 127 see nothing else
+    v[n - 1, 3] = math.inf
+    kc, vc = torch.zeros(pages, BS, H * D), torch.zeros(pages, BS, H * D)
+    kc.view(-1, H * D)[:n], vc.view(-1, H * D)[:n] = k, v
+    first = n - 1 if alone else 0
+    got = S.masked_attention(q[first:].to(dev), H, H, D, D, kc.to(dev), vc.to(dev),
+                             meta([n - first], [first], list(range(pages)), dev), 1.0, sink=torch.zeros(H).to(dev))
+    s = torch.einsum("thd,nhd->thn", q.double().nan_to_num(0).view(n, H, D), k.double().view(n, H, D).clamp(-1e300, 1e300))
+    p = weights(s.masked_fill(s < -1e200, -math.inf), (torch.arange(n)[None] <= torch.arange(n)[:, None])[:, None], torch.zeros(H))
+    want = torch.einsum("thn,nhd->thd", p, v.double().nan_to_num(0, 0, 0).view(n, H, D)).reshape(n, -1)
+    if n > 128:
+        want[n - 1, 3] = math.inf
+        assert torch.equal(torch.isinf(got.cpu()), torch.isinf(want[first:]))
+    else:                                                 # a weight of zero: the column is not a number, the others are zero
+        want[n - 1, 3] = math.nan
+        assert torch.equal(torch.isnan(got.cpu()), torch.isnan(want[first:]))
+    ok = torch.isfinite(want[first:])
+    assert float((got.cpu().double() - want[first:])[ok].abs().max()) < 1e-5
