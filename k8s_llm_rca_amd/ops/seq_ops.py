@@ -992,8 +992,9 @@ def attn_prep(qkv: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D
     activations.  ``G = 0``: only queries (a layer that reads another layer's pages).  ``qkv`` [S, T, ..]: the sum of its
     planes (:func:`.linear.proj_planes`)."""
     planes, pstep = 1, 0
+    by16 = all(t is None or t.data_ptr() % 16 == 0 for t in (kc, rope_cs))      # (attn_prep_half)
     if qkv.dim() == 3:
-        if qkv.shape[0] > 1 and use_hip(qkv) and norm in (False, None, True, "head") and not q_temp and 8 <= D <= 512 \
+        if qkv.shape[0] > 1 and use_hip(qkv) and by16 and norm in (False, None, True, "head") and not q_temp and 8 <= D <= 512 \
                 and D & (D - 1) == 0 and (rope is None or (rope_cs is not None and not rope.pairs and rope.dims % 8 == 0)) \
                 and not (rope is None and rot_dims) and qkv.stride(1) % 4 == 0 and qkv.data_ptr() % 16 == 0 \
                 and qkv.stride(0) % 4 == 0 and qkv.shape[1] <= 1024 and (norm or bias is not None):
@@ -1033,7 +1034,7 @@ def attn_prep(qkv: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D
                                             ptr(vt), BS, ptr(q_out), _dt(out_dtype), int(rot_dims), ptr(rope_cs), T,
                                             stream_ptr(qkv)), "attn_prep_pairs")
             return q_out
-        if (mode < 2 and not tq_every and 8 <= D <= 512 and D & (D - 1) == 0
+        if (mode < 2 and by16 and not tq_every and 8 <= D <= 512 and D & (D - 1) == 0
                 and qkv.stride(0) % 4 == 0 and qkv.data_ptr() % 16 == 0 and rot_dims % 8 == 0
                 and (rot_dims == 0 or (rope is not None and not rope.pairs and rope_cs is not None))):
             # a head's entries meet in its rotation and its norm alone: a few lanes per head, no LDS
@@ -1404,10 +1405,12 @@ def matrix_memory(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tens
 # kernel with its gate and norm passes / this, 16 heads of 128 x 128 at 1 / 8 / 64 / 256 sequences: delta rule 14.1 / 7.1,
 # 16.6 / 7.3, 49.5 / 27.2, 181 / 111;  matrix memory 17.0 / 7.3, 20.7 / 6.7, 54.4 / 30.3, 181 / 109;  decaying attention
 # 9.4 / 5.8, 11.0 / 6.0, 40.1 / 28.4, 142 / 107 (the states' bytes, in and out: 0.4, 3.4, 27, 109).
-def _step_ok(x: torch.Tensor, seg: SegMeta, D: int, V: int, gate: torch.Tensor, w: Optional[torch.Tensor]) -> bool:
+def _step_ok(x: torch.Tensor, seg: SegMeta, D: int, V: int, state: torch.Tensor, gate: torch.Tensor,
+             w: Optional[torch.Tensor]) -> bool:
+    """Whether a step is one token each and rows, states, gates and weights can be read by 16 bytes."""
     return (use_hip(x) and seg.n_seg == x.shape[0] and seg.row0_host[-1] == seg.n_seg and D in (64, 128) and V in (64, 128)
             and min((b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:])), default=0) == 1
-            and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0
+            and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and state.data_ptr() % 16 == 0
             and gate.stride(1) == 1 and gate.stride(0) % 4 == 0 and gate.data_ptr() % 16 == 0
             and (w is None or (w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0)))
 
@@ -1416,7 +1419,7 @@ def delta_layer(qkv: torch.Tensor, H: int, G: int, D: int, V: int, a: torch.Tens
                 dt_bias: torch.Tensor, beta: torch.Tensor, state: torch.Tensor, seg: SegMeta, gate: torch.Tensor,
                 w: Optional[torch.Tensor], eps: float, out_dtype) -> torch.Tensor:
     """:func:`gated_delta`, then :func:`head_norm_gate` over each head."""
-    if (_step_ok(qkv, seg, D, V, gate, w) and gate.dtype == torch.float32 and out_dtype == qkv.dtype
+    if (_step_ok(qkv, seg, D, V, state, gate, w) and gate.dtype == torch.float32 and out_dtype == qkv.dtype
             and qkv.is_contiguous()):
         T = qkv.shape[0]
         assert qkv.shape[1] == 2 * G * D + H * V and H % G == 0 and state.is_contiguous() and state.shape[1:] == (H, D, V)
@@ -1439,7 +1442,7 @@ def memory_layer(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tenso
                  out_dtype) -> torch.Tensor:
     """:func:`matrix_memory`, then :func:`head_norm_gate` over each head with the gates that stand behind the values."""
     gate = x[:, 2 * H * D + H * V:2 * H * (D + V)]
-    if _step_ok(x, seg, D, V, gate, w):
+    if _step_ok(x, seg, D, V, state, gate, w):
         T = x.shape[0]
         assert x.dtype == torch.float32 and x.shape[1] == 2 * H * (D + V) + 2 * H
         assert gate_bias.dtype == torch.float32 and gate_bias.numel() == 2 * H and (w is None or w.numel() in (V, H * V))
@@ -1460,7 +1463,7 @@ def decay_layer(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor, st
     """:func:`decay_attention` with silu, then one norm over all heads, its weight and the gates: (y, None), or for steps of
     single tokens (y without the division by the row's root mean square, (sums of squares [T, H], H V, eps)), which
     :func:`.norm.hyper_step` makes up for behind the output projection."""
-    if (_step_ok(x, seg, D, V, gate, w) and gate.dtype == x.dtype == out_dtype and w.numel() == H * V):
+    if (_step_ok(x, seg, D, V, state, gate, w) and gate.dtype == x.dtype == out_dtype and w.numel() == H * V):
         T = x.shape[0]
         assert x.shape[1] >= H * (2 * D + V) and gate.shape[1] >= H * V
         assert decay.dtype == torch.float32 and decay.numel() == H
