@@ -13,6 +13,7 @@ import os
 import threading
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _build
 from ..knobs import KNOBS, push_native
@@ -230,6 +231,19 @@ def check(rc: int, name: str) -> None:
             torch.cuda.synchronize()
         except RuntimeError as e:
             raise RuntimeError(f"{name}: device fault surfaced at sync: {e}") from e
+
+
+def unwatched(*tensors) -> bool:
+    """Whether a kernel launched by address does all that torch's operator would with these tensors: neither autograd (either
+    direction), ``torch.func``, tracing, compiling, a torch mode, a tensor subclass nor autocast has a part in the call.
+    Kernels that took a torch operator's place ask this and leave the others to the operator."""
+    f = torch._C._functorch.peek_interpreter_stack
+    if (f() is not None or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch.jit.is_tracing() or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")):
+        return False
+    grad = torch.is_grad_enabled()
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and not (grad and t.requires_grad)
+               and forward_ad.unpack_dual(t).tangent is None for t in tensors)
 
 
 def use_hip(*tensors) -> bool:

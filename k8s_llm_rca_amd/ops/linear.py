@@ -10,7 +10,7 @@ import torch
 import torch.nn.functional as F
 
 from ..knobs import KNOBS
-from ._lib import check, lib, ptr, scratch, stream_ptr
+from ._lib import check, lib, ptr, scratch, stream_ptr, unwatched
 from .moe import glu_clamp
 from .norm import relu_sq
 
@@ -70,11 +70,11 @@ FEW_F32_WIDE = 8192, 5
 
 def _few_f32_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     (M, K), N = x.shape, w.shape[0]
-    return (x.is_cuda and w.is_cuda and x.dtype == torch.float32 == w.dtype
+    return (x.is_cuda and w.is_cuda and x.dtype == torch.float32 == w.dtype and unwatched(x, w)
             and 0 < M <= (FEW_F32_WIDE[1] if N >= FEW_F32_WIDE[0] else FEW_F32_ROWS) and N > 0 and K > 0 and K % 4 == 0
             and w.dim() == 2 and w.shape[1] == K and w.is_contiguous() and w.data_ptr() % 16 == 0
             and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.stride(0) >= K and x.data_ptr() % 16 == 0
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+            and x.stride(0) < 2 ** 31)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:

@@ -23,7 +23,7 @@ import numpy as np
 
 import torch
 
-from ._lib import check, lib, ptr, scratch, stream_ptr, use_hip
+from ._lib import check, lib, ptr, scratch, stream_ptr, unwatched, use_hip
 
 # Parts a single token's keys are cut into, a workgroup each (csrc/kernels/token_attn.hip).  us at parts of half the size /
 # this / twice: masked, 1 row at 200 keys 8.9 / 6.5 / 6.5, at 4000 9.1 / 10.5 / 14.4, 64 rows at 400 14.7 / 12.3 / 10.4, at
@@ -371,8 +371,7 @@ def _small_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def _small_heads(x: torch.Tensor, w: torch.Tensor) -> bool:
     return (use_hip(x) and 0 < x.shape[0] <= SMALL_PROJ_ROWS and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float32)
-            and w.is_contiguous() and w.data_ptr() % 8 == 0
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+            and unwatched(x, w) and w.is_contiguous() and w.data_ptr() % 8 == 0)
 
 
 def head_proj(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:

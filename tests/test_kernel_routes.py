@@ -2,7 +2,9 @@
 import pytest
 import torch
 
+from k8s_llm_rca_amd.ops import linear as L
 from k8s_llm_rca_amd.ops import seq_ops as S
+from k8s_llm_rca_amd.ops._lib import unwatched
 
 BF = torch.bfloat16
 gpu = pytest.mark.gpu
@@ -60,3 +62,56 @@ def test_unaligned_states_and_pages_give_the_same():
         pages.append([t.float() for t in (q, kc, vc)])
     for p, q in zip(*pages):
         assert float((p - q).abs().max()) <= 2.0 ** -7 * float(q.abs().max())
+
+
+def test_calls_that_something_watches():
+    """Every way in which torch has more to do with an operator than its numbers."""
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    x, w, seen = torch.randn(2, 4), torch.nn.Parameter(torch.randn(3, 4)), []
+
+    def look(*_):
+        seen.append(unwatched(x))
+        return x
+    assert unwatched(x, w.detach()) and not unwatched(x, w)
+    with torch.no_grad():
+        assert unwatched(x, w)
+    with forward_ad.dual_level():
+        assert unwatched(x, w.detach()) and not unwatched(forward_ad.make_dual(x, x), w.detach())
+    torch.func.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    torch.jit.trace(look, (x,), check_trace=False)
+    torch.set_autocast_enabled("cuda", True)              # (torch.autocast is off without a device)
+    look()
+    torch.set_autocast_enabled("cuda", False)
+    with TorchDispatchMode():
+        look()
+    with TorchFunctionMode():
+        look()
+    seen.append(unwatched(x.as_subclass(type("Sub", (torch.Tensor,), {}))))
+    assert len(seen) >= 7 and not any(seen)
+
+
+@gpu
+def test_transforms_of_products_in_fp32():
+    """Tangents, batched calls, traces and casts of fp32 products are torch's own, as of its operators."""
+    from torch.autograd import forward_ad
+    g = torch.Generator().manual_seed(1)
+    x, w, t = (torch.randn(*s, generator=g).cuda() for s in ((4, 64), (96, 64), (4, 64)))
+    q, uk, tq = (torch.randn(*s, generator=g).cuda() for s in ((4, 2 * 64), (2, 64, 64), (4, 2 * 64)))
+    calls = [(lambda a: L.linear(a, w), lambda a: a @ w.T, x, t),
+             (lambda a: S.latent_queries(a, uk, None, 2, 64, 0)[0],
+              lambda a: torch.bmm(a.view(-1, 2, 64).transpose(0, 1), uk).transpose(0, 1), q, tq)]
+    for f, ref, a, da in calls:
+        with forward_ad.dual_level():
+            d = forward_ad.unpack_dual(f(forward_ad.make_dual(a, da))).tangent
+        assert d is not None and torch.allclose(d, ref(da), atol=1e-4)
+        assert torch.allclose(torch.func.vmap(f)(torch.stack([a, da])), torch.stack([ref(a), ref(da)]), atol=1e-4)
+        assert torch.allclose(torch.func.jvp(f, (a,), (da,))[1], ref(da), atol=1e-4)
+        assert torch.allclose(torch.jit.trace(f, (a,), check_trace=False)(da), ref(da), atol=1e-4)
+        with torch.autocast("cuda", dtype=BF):
+            assert f(a).dtype == BF
+        v = a.clone().requires_grad_()
+        f(v).sum().backward()
+        assert torch.allclose(v.grad, torch.autograd.grad(ref(v).sum(), v)[0], atol=1e-4)
