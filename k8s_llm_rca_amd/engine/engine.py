@@ -41,7 +41,7 @@ from ..models.config import ModelConfig, get_config
 from ..models.registry import OWN_CONFIG as _OWN_CONFIG
 from ..ops import attention as A
 from ..parallel.groups import ParallelContext, single
-from .graph_runner import GraphRunnerMixin
+from .graph_runner import GraphRunnerMixin, SegGraphCache
 from .kv_cache import KVPool
 from .kv_manager import KVCacheManager
 from .sampler import SamplerMixin
@@ -161,10 +161,10 @@ class LLMEngine(SchedulerMixin, StepExecMixin, GraphRunnerMixin, SamplerMixin):
         self._mask_ver = -1
         self._graphs: Dict[tuple, tuple] = {}
         self._graph_pool = None
-        # graphs of models in the segment layout: (rows, block-table width, weight loads) -> (graph, static input, logits, step)
-        self._seg_graphs: Dict[tuple, tuple] = {}
-        self._seg_seen: Dict[tuple, int] = {}
-        self._seg_stream = None
+        # graphs of models in the segment layout: (rows, block-table width) -> (graph, static input, logits, step)
+        self._seg = SegGraphCache()
+        self._seg_loads = 0
+        self._seg_stream = self._seg_pool = None
         self._static = None
         self._pf_ws = None  # prefill split-KV partials (allocated on first split step)
         # multi-token decode items (a short chunk's tokens read their shared keys

@@ -34,12 +34,53 @@ from .types import PART_MIN, SPEC, InFlight, Request, Sequence, _LazySample, _sp
 log = logging.getLogger("k8s_llm_rca_amd.engine.engine")
 
 
-# Steps of a shape that run eagerly before it is captured (they also leave nothing to be set up inside the capture).  A
-# capture costs 2 to 4 ms, a replay saves 0.4 to 0.5 ms of a step (fikerax-1b, 1 / 7 / 64 rows: 1.14 / 1.20 / 1.85 ms of
-# which the host's launches take most -> 0.71 / 0.88 / 1.38; lizesun-1b, 8 layers: 1.17 / 1.27 / 1.66 -> 0.77 / 0.87 / 1.10),
-# so a shape that came three times is taken to come ten times more.
-SEG_GRAPH_AFTER = 3
+# A capture takes 1.1 to 1.4 ms in place of an eager step, a replay saves 0.4 to 0.5 ms (fikerax-1b, 1 / 7 / 64 rows: 1.14 /
+# 1.20 / 1.85 ms of which the host's launches take most -> 0.71 / 0.88 / 1.38; lizesun-1b, 8 layers: 1.17 / 1.27 / 1.66 ->
+# 0.77 / 0.87 / 1.10).  Generation of 64 replies, ms of an engine's second round, eager / captured whenever a shape had come
+# three times / paid for by replays: a reply ends every second step 222 / 272 / 235 (8 captures, none in later rounds), every
+# fourth 422 / 371 / 363; 24 replies of 4 to 200 tokens 255 / 164 / 164.
+SEG_GRAPH_AFTER = 3     # eager steps of a shape before it is captured (they leave nothing to be set up inside the capture)
 SEG_GRAPHS = 32         # graphs an engine keeps (least recently replayed ones go)
+SEG_PRICE = 3           # replays that pay for a capture
+SEG_AHEAD = 8           # captures an engine makes before replays have paid for them
+SEG_LONG = 64           # eager steps of a shape after which it is captured on no account but its own
+
+
+class SegGraphCache:
+    """Which shapes of steps have a graph, and which are worth one.  A batch that shrinks and grows runs through many shapes
+    of a few steps each, so captures are paid for by replays: an engine is never more than ``SEG_AHEAD`` captures behind
+    what eager steps alone would have taken, but for one per ``SEG_LONG`` eager steps of a shape.  A graph that gives way
+    to others has to be earned again."""
+
+    def __init__(self):
+        self.graphs: Dict[tuple, tuple] = {}       # least recently replayed first
+        self.seen: Dict[tuple, int] = {}           # eager steps of a shape without a graph
+        self.credit = SEG_AHEAD * SEG_PRICE        # replays
+
+    def get(self, key: tuple) -> Optional[tuple]:
+        """The graph of a shape, for a replay."""
+        got = self.graphs.pop(key, None)
+        if got is not None:
+            self.graphs[key] = got
+            self.credit = min(self.credit + 1, SEG_GRAPHS * SEG_PRICE)
+        return got
+
+    def worth(self, key: tuple) -> bool:
+        """Counts a step of a shape without a graph: whether to capture it."""
+        if len(self.seen) > 4096:
+            self.seen.clear()
+        n = self.seen[key] = self.seen.get(key, 0) + 1
+        return n > SEG_GRAPH_AFTER and (self.credit >= SEG_PRICE or n > SEG_LONG)
+
+    def room(self) -> bool:
+        return len(self.graphs) < SEG_GRAPHS
+
+    def put(self, key: tuple, graph: tuple) -> None:
+        while not self.room():
+            self.graphs.pop(next(iter(self.graphs)))
+        self.graphs[key] = graph
+        self.seen.pop(key, None)
+        self.credit = max(0, self.credit - SEG_PRICE)
 
 
 class _DecodeSegments(SegMeta):
@@ -267,14 +308,15 @@ class GraphRunnerMixin:
             return None                        # (a capture has no room for the synchronisation behind every launch)
         pages = max(s.n_cached + j for s, j in decode) // BS + 1
         width = 1 << (pages - 1).bit_length() if pages <= 8 else -(-pages // 8) * 8 if pages <= 128 else -(-pages // 32) * 32
-        key = (B, width, self.model.loads)
-        got = self._seg_graphs.pop(key, None)
-        if got is None:
-            if len(self._seg_seen) > 4096:
-                self._seg_seen.clear()
-            n = self._seg_seen[key] = self._seg_seen.get(key, 0) + 1
-            if n <= SEG_GRAPH_AFTER:
-                return None
+        cache, key = self._seg, (B, width)
+        if self._seg_loads != self.model.loads:       # other weights: no graph of the old ones is replayed any more
+            if cache.graphs:
+                torch.cuda.current_stream(self.device).synchronize()
+                cache.graphs.clear()
+            self._seg_loads = self.model.loads
+        got = cache.get(key)
+        if got is None and not cache.worth(key):
+            return None
         flat = np.zeros(8 * B + B * width, dtype=np.int32)
         ids, pos, slots, slot = flat[:4 * B].reshape(4, B)
         items, bt = flat[4 * B:8 * B].reshape(B, 4), flat[8 * B:].reshape(B, width)
@@ -290,11 +332,13 @@ class GraphRunnerMixin:
             bt[i, :n] = s.blocks[:n]
         host = torch.from_numpy(flat).pin_memory()
         if got is None:
+            if not cache.room():
+                torch.cuda.current_stream(self.device).synchronize()       # the last replay of the one that goes may still run
             got = self._seg_capture(B, width, host)
+            cache.put(key, got)
         else:
             got[1].copy_(host, non_blocking=True)
         self._trace_mark()
-        self._seg_graphs[key] = got            # now the most recently replayed one
         graph, _, out, _ = got
         graph.replay()
         if sample_idx == list(range(B)):
@@ -307,9 +351,6 @@ class GraphRunnerMixin:
         step is kept with the graph: every tensor in it is read by each replay, the row offsets too, which no copy fills."""
         t0 = time.perf_counter()
         cur = torch.cuda.current_stream(self.device)
-        while len(self._seg_graphs) >= SEG_GRAPHS:
-            cur.synchronize()                  # its last replay may still run
-            self._seg_graphs.pop(next(iter(self._seg_graphs)))
         flat = host.to(self.device, non_blocking=True)
         ids, pos, slots, slot = flat[:4 * B].view(4, B).unbind(0)
         rows = torch.arange(B + 1, dtype=torch.int32, device=self.device)
@@ -319,8 +360,8 @@ class GraphRunnerMixin:
         seg.items = flat[4 * B:8 * B].view(B, 4)
         inp = SegStepInputs(ids, pos, slots, seg, None)
         states = self.states.t if self.states is not None else {}
-        if self._graph_pool is None:
-            self._graph_pool = torch.cuda.graph_pool_handle()
+        if not self._seg.graphs:                   # (a pool goes with the last graph that holds it)
+            self._seg_pool = torch.cuda.graph_pool_handle()
         if self._seg_stream is None:
             self._seg_stream = torch.cuda.Stream(self.device)
         graph = torch.cuda.CUDAGraph()
@@ -331,7 +372,7 @@ class GraphRunnerMixin:
         self._seg_stream.wait_stream(cur)
         try:
             with torch.cuda.stream(self._seg_stream):
-                graph.capture_begin(pool=self._graph_pool, capture_error_mode="thread_local")
+                graph.capture_begin(pool=self._seg_pool, capture_error_mode="thread_local")
                 try:
                     out = self.model.forward(inp, *self.kv.tensors(), states)
                 finally:

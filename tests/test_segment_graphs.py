@@ -106,3 +106,15 @@ def test_a_check_behind_every_launch_runs_steps_eagerly(monkeypatch):
     for _ in range(6):
         eng.feed([(sid, [3], [0])])
     assert eng.stats["captures"] == 0
+
+
+def test_many_shapes_in_rotation_are_not_captured_again_and_again(monkeypatch):
+    monkeypatch.setattr(G, "SEG_GRAPHS", 2)
+    engines = [engine("tiny-fikerax", torch.bfloat16, graphs) for graphs in (True, False)]
+    sids = [[e.new_sequence() for _ in range(5)] for e in engines]
+    for i in range(60):                                   # batches of 5, 4, 3, 2, 1, 5, ..
+        k = 5 - i % 5
+        a, b = (e.feed([(s, [7 + i], [0]) for s in ss[:k]]) for e, ss in zip(engines, sids))
+        assert torch.equal(a, b)
+    st = engines[0].stats
+    assert st["captures"] * G.SEG_PRICE <= st["graph_steps"] + G.SEG_PRICE * G.SEG_AHEAD and len(engines[0]._seg.graphs) <= 2
