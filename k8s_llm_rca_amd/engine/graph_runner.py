@@ -10,6 +10,7 @@ per (rows, block-table width): see :meth:`GraphRunnerMixin._seg_graph_step`.
 """
 from __future__ import annotations
 
+import contextlib
 import json
 import logging
 import math
@@ -44,6 +45,7 @@ SEG_GRAPHS = 32         # graphs an engine keeps (least recently replayed ones g
 SEG_PRICE = 3           # replays that pay for a capture
 SEG_AHEAD = 8           # captures an engine makes before replays have paid for them
 SEG_LONG = 64           # eager steps of a shape after which it is captured on no account but its own
+SEG_BACKOFF = 256       # steps of a shape between a capture that failed and the next try
 
 
 class SegGraphCache:
@@ -56,6 +58,7 @@ class SegGraphCache:
         self.graphs: Dict[tuple, tuple] = {}       # least recently replayed first
         self.seen: Dict[tuple, int] = {}           # eager steps of a shape without a graph
         self.credit = SEG_AHEAD * SEG_PRICE        # replays
+        self.off = False                           # a capture could not be ended
 
     def get(self, key: tuple) -> Optional[tuple]:
         """The graph of a shape, for a replay."""
@@ -67,6 +70,8 @@ class SegGraphCache:
 
     def worth(self, key: tuple) -> bool:
         """Counts a step of a shape without a graph: whether to capture it."""
+        if self.off:
+            return False
         if len(self.seen) > 4096:
             self.seen.clear()
         n = self.seen[key] = self.seen.get(key, 0) + 1
@@ -81,6 +86,9 @@ class SegGraphCache:
         self.graphs[key] = graph
         self.seen.pop(key, None)
         self.credit = max(0, self.credit - SEG_PRICE)
+
+    def failed(self, key: tuple) -> None:
+        self.seen[key] = -SEG_BACKOFF
 
 
 class _DecodeSegments(SegMeta):
@@ -302,7 +310,8 @@ class GraphRunnerMixin:
         and how many cache pages the attention's grids are laid out for (the width of the block tables: a power of two up to
         8 pages, then in steps of 8, past 128 of 32); everything else a step's kernels need -- tokens, positions, cache and state slots,
         pages, work items -- is read from one static buffer that each step fills with one copy.  The logits are copied
-        out: what a step returns stays the caller's."""
+        out: what a step returns stays the caller's.  A capture that fails -- it takes memory beside the allocator's free
+        blocks -- has run nothing, so the step runs eagerly."""
         B, BS = len(decode), self.kv.block_size
         if B > max(self.cfg.graph_batch_sizes) or len(set(id(s) for s, _ in decode)) != B or KNOBS.sync_debug:
             return None                        # (a capture has no room for the synchronisation behind every launch)
@@ -334,7 +343,12 @@ class GraphRunnerMixin:
         if got is None:
             if not cache.room():
                 torch.cuda.current_stream(self.device).synchronize()       # the last replay of the one that goes may still run
-            got = self._seg_capture(B, width, host)
+            try:
+                got = self._seg_capture(B, width, host)
+            except Exception as e:                 # (what is wrong with the step itself shows again in the eager one)
+                log.warning("capture of a step of %d rows failed, the step runs eagerly: %s", B, e)
+                cache.failed(key)
+                return None
             cache.put(key, got)
         else:
             got[1].copy_(host, non_blocking=True)
@@ -375,8 +389,15 @@ class GraphRunnerMixin:
                 graph.capture_begin(pool=self._seg_pool, capture_error_mode="thread_local")
                 try:
                     out = self.model.forward(inp, *self.kv.tensors(), states)
-                finally:
-                    graph.capture_end()
+                except BaseException:
+                    self._seg.off = True           # until the capture has ended
+                    with contextlib.suppress(RuntimeError):        # (the first error is the one to report)
+                        graph.capture_end()
+                        self._seg.off = False
+                    raise
+                self._seg.off = True
+                graph.capture_end()
+                self._seg.off = False
         finally:
             if gc_was_on:
                 gc.enable()

@@ -1,4 +1,4 @@
-"""Which shapes of steps an engine captures: paid for by replays, earned again after giving way."""
+"""Which shapes of steps an engine captures: paid for by replays, earned again after giving way, not retried after a failure."""
 import random
 
 from k8s_llm_rca_amd.engine import graph_runner as G
@@ -51,3 +51,14 @@ def test_a_lonely_shape_comes_to_its_graph_without_credit():
     c = G.SegGraphCache()
     c.credit = 0
     assert drive(c, [(5, 1)] * 200) == [1, 199 - G.SEG_LONG, G.SEG_LONG]
+
+
+def test_a_failed_capture_is_not_tried_again_at_once():
+    c = G.SegGraphCache()
+    while not c.worth((1, 1)):
+        pass
+    c.failed((1, 1))
+    assert not any(c.worth((1, 1)) for _ in range(G.SEG_BACKOFF))
+    assert drive(c, [(2, 1)] * 10)[0] == 1
+    c.off = True
+    assert not any(c.worth((3, 1)) for _ in range(1000))

@@ -108,6 +108,36 @@ def test_a_check_behind_every_launch_runs_steps_eagerly(monkeypatch):
     assert eng.stats["captures"] == 0
 
 
+@pytest.mark.parametrize("model", ["tiny-fikerax", "tiny-lizesun"])
+def test_a_capture_that_fails_leaves_the_step_to_the_eager_path(model, monkeypatch):
+    """An error that only a capture meets (memory, say): the same logits, no further try at once, and captures of other
+    shapes as before."""
+    engines = [engine(model, torch.bfloat16, graphs) for graphs in (True, False)]
+    eng, forward = engines[0], engines[0].model.forward
+
+    def fails(inp, *a, **k):
+        out = forward(inp, *a, **k)
+        if torch.cuda.is_current_stream_capturing():
+            raise torch.OutOfMemoryError("no memory for a capture")
+        return out
+    monkeypatch.setattr(eng.model, "forward", fails)
+    sids = [[e.new_sequence() for _ in range(2)] for e in engines]
+
+    def step(n, k=1):
+        a, b = (e.feed([(s, list(range(n)), [n - 1]) for s in ss[:k]]) for e, ss in zip(engines, sids))
+        assert torch.equal(a, b)
+    for n in (9, *[1] * 8):
+        step(n)
+    assert eng.stats["captures"] == 0 == eng.stats["graph_steps"] and not eng._seg.off
+    monkeypatch.setattr(eng.model, "forward", forward)
+    for _ in range(8):
+        step(1)
+    assert eng.stats["captures"] == 0                     # (the shape that failed waits)
+    for n in (9, *[1] * 8):
+        step(n, 2)
+    assert eng.stats["captures"] == 1 and eng.stats["graph_steps"] > 0
+
+
 def test_many_shapes_in_rotation_are_not_captured_again_and_again(monkeypatch):
     monkeypatch.setattr(G, "SEG_GRAPHS", 2)
     engines = [engine("tiny-fikerax", torch.bfloat16, graphs) for graphs in (True, False)]
