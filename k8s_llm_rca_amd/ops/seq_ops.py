@@ -30,7 +30,8 @@ from ._lib import check, lib, ptr, scratch, stream_ptr, unwatched, use_hip
 # 1500 34.6 / 27.5 / 28.0;  latent, 1 row at 200 9.3 / 11.5 / 11.5, at 4000 15.7 / 14.1 / 15.8, 64 at 400 17.5 / 14.3 / 17.6.
 MASK_TOKEN_BLOCKS = 8    # 32-key blocks of the row's own list
 LATENT_PART = 128        # keys, from the part of the row's first visible key on
-TOKEN_PARTS = 64         # a row with more than so many of them has larger ones: the partial results stay bounded
+TOKEN_PARTS = 64         # a row with more than so many of them has larger ones
+TOKEN_SCRATCH = 1 << 28  # floats of partial results (1 GiB): a step of more takes its rows in groups
 MASK_TILE_ROWS = 128     # (token, head) rows of one workgroup of the masked prompt kernel
 # A step's prompt rows up to which they are taken one by one as well (masked layers): the tiles of one sequence each walk all
 # their keys, the rows have them cut into parts.  us, prompt kernel / rows, 16 heads over 2: 8 rows at 0 / 500 / 2000 keys
@@ -465,6 +466,15 @@ def _latent_out(qa: torch.Tensor, dtype, head_major: bool) -> torch.Tensor:
     return torch.empty(T, H, R, dtype=dtype, device=qa.device)
 
 
+def _token_groups(rows: torch.Tensor, heads: int, parts: int, V: int) -> tuple:
+    """Items of single tokens [n, 4] in groups whose partial results fit ``TOKEN_SCRATCH``, and scratch for the largest of
+    them: outputs, maxima and sums (None, None: one part, nothing to join)."""
+    if parts == 1:
+        return [rows], None, None
+    per = min(rows.shape[0], max(1, TOKEN_SCRATCH // (heads * parts * (V + 2))))
+    return (rows.split(per), *(scratch(per * heads * parts * n, torch.float32, rows.device) for n in (V, 2)))
+
+
 def latent_attention_mfma(qa: torch.Tensor, cache: torch.Tensor, cache_t: torch.Tensor, gate: Optional[torch.Tensor],
                           seg: SegMeta, positions: torch.Tensor, scale: float, qr: Optional[torch.Tensor] = None,
                           window: int = 0, sink: Optional[torch.Tensor] = None, head_major: bool = False) -> torch.Tensor:
@@ -492,13 +502,12 @@ def latent_attention_mfma(qa: torch.Tensor, cache: torch.Tensor, cache_t: torch.
         if window > 0:      # a row's parts start at the one its first visible key lies in
             n_parts = min(n_parts, (min(int(window), kmax) + part - 2) // part + 1)
         n_parts = min(n_parts, TOKEN_PARTS)
-        po = pml = None
-        if n_parts > 1:
-            po, pml = (scratch(dec.shape[0] * H * n_parts * n, torch.float32, qa.device) for n in (R, 2))
-        check(L.k8s_latent_attn_token(ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), W - R, ptr(cache), ptr(cache_t),
-                                      ptr(bt), maxb, ptr(dec), dec.shape[0], ptr(gate), gs, ptr(sink), ptr(out),
-                                      out.stride(0), out.stride(1), ptr(po), ptr(pml), n_parts, part, TOKEN_PARTS, H,
-                                      R, BS, int(window), float(scale), st), "latent_attn_token")
+        groups, po, pml = _token_groups(dec, H, n_parts, R)
+        for it in groups:
+            check(L.k8s_latent_attn_token(ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), W - R, ptr(cache), ptr(cache_t),
+                                          ptr(bt), maxb, ptr(it), it.shape[0], ptr(gate), gs, ptr(sink), ptr(out),
+                                          out.stride(0), out.stride(1), ptr(po), ptr(pml), n_parts, part, TOKEN_PARTS, H,
+                                          R, BS, int(window), float(scale), st), "latent_attn_token")
     if pre.shape[0]:
         check(L.k8s_latent_attn_mfma(ptr(qa), ptr(cache), ptr(cache_t), ptr(bt), maxb, ptr(pre), pre.shape[0], ptr(gate),
                                      gs, ptr(out), H, R, BS, float(scale), st, qa.stride(0), qa.stride(1), ptr(qr), W - R,
@@ -1140,12 +1149,12 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
                     nblk = min(nblk, (int(window) + 62) // 32 + -(-int(keep_first) // 32))
                 if chunk > 0:
                     nblk = min(nblk, (int(chunk) + 62) // 32)
-                n_parts, po, pml = min(-(-nblk // MASK_TOKEN_BLOCKS), TOKEN_PARTS), None, None
-                if n_parts > 1:
-                    po, pml = (scratch(rows.shape[0] * HQ * n_parts * n, torch.float32, q.device) for n in (V, 2))
-                check(lib().k8s_masked_attn_token(ptr(q), ptr(kc), ptr(vt), ptr(bt), maxb, ptr(rows), rows.shape[0],
-                                                  *common, MASK_TOKEN_BLOCKS, TOKEN_PARTS, n_parts, ptr(pml), ptr(po),
-                                                  int(maps), int(out_f32)), "masked_attn_token")
+                n_parts = min(-(-nblk // MASK_TOKEN_BLOCKS), TOKEN_PARTS)
+                groups, po, pml = _token_groups(rows, HQ, n_parts, V)
+                for it in groups:
+                    check(lib().k8s_masked_attn_token(ptr(q), ptr(kc), ptr(vt), ptr(bt), maxb, ptr(it), it.shape[0],
+                                                      *common, MASK_TOKEN_BLOCKS, TOKEN_PARTS, n_parts, ptr(pml), ptr(po),
+                                                      int(maps), int(out_f32)), "masked_attn_token")
             if tiles.shape[0]:
                 check(lib().k8s_masked_attn_prompt(ptr(q), ptr(kc), ptr(vt), ptr(bt), maxb, ptr(tiles), tiles.shape[0],
                                                    *common, int(maps), int(out_f32)), "masked_attn_prompt")

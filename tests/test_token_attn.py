@@ -144,3 +144,23 @@ def test_rows_of_more_keys_than_parts(most, monkeypatch):
     monkeypatch.setattr(S, "TOKEN_PARTS", most)
     for a, b in zip(run(), want):
         close(a, b.double().cpu())
+
+
+def test_partial_results_within_a_bound(monkeypatch):
+    """A step whose partial results pass the bound takes its rows in groups: the same bits, no allocation past the bound."""
+    H, G, D, n = 8, 2, 64, len(ENDS)
+    g = torch.Generator().manual_seed(9)
+    q, kc, vt = (torch.randn(*s, generator=g).to(BF).cuda() for s in ((n, H * D), (24, BS, G * D), (24, G * D, BS)))
+    qa, c, ct = (torch.randn(*s, generator=g).to(BF).cuda() for s in ((n, H, D), (24, BS, D), (24, D, BS)))
+    m, sizes, scratch = meta(ENDS, list(range(24))), [], S.scratch
+    monkeypatch.setattr(S, "scratch", lambda shape, *a: (sizes.append(shape), scratch(shape, *a))[1])
+
+    def run():
+        sizes.clear()
+        return (S.masked_attention(q, H, G, D, D, kc, None, m, 0.1, vt=vt),
+                S.latent_attention_mfma(qa, c, ct, None, m, m.seg_pos0, 0.1), max(sizes))
+    a, b, _ = run()
+    for limit in (1, 40000, 10 ** 5, 10 ** 9):
+        monkeypatch.setattr(S, "TOKEN_SCRATCH", limit)
+        x, y, most = run()
+        assert torch.equal(x, a) and torch.equal(y, b) and most <= max(limit, H * 11 * D)
