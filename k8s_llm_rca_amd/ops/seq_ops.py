@@ -1267,13 +1267,42 @@ def _mat_tiles(seg: SegMeta, kind: int, H: int, D: int, V: int):
     V 128; token by token or in chunks -> tiles, us):  delta rule, one sequence of 16 / 17 / 129 tokens 21 -> 21 / 23 -> 19 /
     165 -> 29, 64 of 17 tokens 72 -> 52;  memory, one of 17 / 33 / 129 tokens 23 -> 27 / 30 -> 28 / 73 -> 29, 64 of 17 tokens
     68 -> 48 -- its own steps are cheaper, so that few sequences need two tiles before the tiles' launch pays."""
-    per = lib().k8s_tile_state_ws(kind, D)
+    per = lib().k8s_tile_state_ws(kind, D)      # floats per (tile, head)
     few = seg.n_seg * H * -(-V // 64) < MAT_FILL_GROUPS
     cr = seg.chunk_ranges(MAT_TILE, 2 * MAT_TILE if kind == 1 and few else MAT_TILE) if per else None
     return None if cr is None else (*cr, cr[0].shape[0] * H * per + 256)
 
 
 UNIT_EPS = 1e-6     # q and k of the delta rule: x / sqrt(sum(x^2) + UNIT_EPS)
+
+
+MAT_SCRATCH = 1 << 28   # floats of the tiles' workspace (1 GiB): a step of more goes in several ones
+
+
+def _mat_pieces(seg: SegMeta, tiles: int, floats: int) -> list:
+    """A step whose ``tiles`` take ``floats`` of workspace as several steps, cut at tile borders: [(first row, end, SegMeta)].
+    A sequence that is cut goes on from its slot, as it does from one portion of a prompt to the next."""
+    dev, out = seg.row_seg.device, []
+    most = max(2, MAT_SCRATCH * tiles // floats)
+    todo = [(s, a, b) for s, (a, b) in enumerate(zip(seg.row0_host[:-1], seg.row0_host[1:])) if b > a]
+    while todo:
+        take, left = [], most
+        while todo and left and not (take and take[-1][0] == todo[0][0]):
+            s, a, b = todo.pop(0)
+            n = min(b - a, left * MAT_TILE)
+            take.append((s, a, a + n))
+            left -= -(-n // MAT_TILE)
+            if a + n < b:
+                todo.insert(0, (s, a + n, b))
+        r0 = [0]
+        for _, a, b in take:
+            r0.append(r0[-1] + b - a)
+        pos = [seg.pos0_host[s] + a - seg.row0_host[s] for s, a, _ in take]
+        slots = [seg.slot_host[s] for s, _, _ in take]
+        i32 = [torch.tensor(v, dtype=torch.int32, device=dev)
+               for v in ([i for i, (_, a, b) in enumerate(take) for _ in range(a, b)], r0, pos, slots, [[0]] * len(take))]
+        out.append((take[0][1], take[-1][2], SegMeta(len(take), *i32, r0, pos, slots)))
+    return out
 
 
 def gated_delta(qkv: torch.Tensor, H: int, G: int, D: int, V: int, a: torch.Tensor, rate: torch.Tensor,
@@ -1295,6 +1324,9 @@ def gated_delta(qkv: torch.Tensor, H: int, G: int, D: int, V: int, a: torch.Tens
         got = _mat_tiles(seg, 0, H, D, V)
         if got is not None:
             tiles, t0, n = got
+            if n > MAT_SCRATCH and tiles.shape[0] > 2:
+                return torch.cat([gated_delta(qkv[i:j], H, G, D, V, a[i:j], rate, dt_bias, beta[i:j], state, m)
+                                  for i, j, m in _mat_pieces(seg, tiles.shape[0], n)])
             ws = scratch(n, torch.float32, qkv.device)
             check(lib().k8s_gated_delta_tiles(ptr(qkv), _dt(qkv.dtype), ptr(a), ptr(rate), ptr(dt_bias), ptr(beta),
                                               beta.stride(0), ptr(state), ptr(seg.seg_row0), ptr(seg.seg_pos0),
@@ -1359,12 +1391,16 @@ def matrix_memory(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tens
         assert gate_bias.dtype == torch.float32 and gate_bias.numel() == 2 * H
         assert state.is_contiguous() and state.shape[1:] == (H, D, V) and nstate.is_contiguous()
         assert nstate.shape[1:] == (H, D) and mstate.is_contiguous() and mstate.shape[1:] == (H,)
+        got = _mat_tiles(seg, 1, H, D, V)
+        if got is not None and got[2] > MAT_SCRATCH and got[0].shape[0] > 2:
+            parts = [matrix_memory(x[i:j], H, D, V, gate_bias, cap, state, nstate, mstate, m, defer_scale)
+                     for i, j, m in _mat_pieces(seg, got[0].shape[0], got[2])]
+            return tuple(torch.cat(t) for t in zip(*parts)) if defer_scale else torch.cat(parts)
         ab = scratch(T * H * 3, torch.float32, x.device)
         nq = scratch(T * H, torch.float32, x.device)
         mul = scratch((T, H), torch.float32, x.device)
         # other sizes, long portions: chunks in parallel (end states from zero, a carry over the chunks, the chunks again
         # from their start states); short ones token by token
-        got = _mat_tiles(seg, 1, H, D, V)
         cr = _mat_chunks(seg, H, V) if got is None else None
         chunks, c0, cs, cx, cdec, nch, tws = None, None, None, None, None, 0, None
         if got is not None:

@@ -158,3 +158,45 @@ def test_what_is_not_finite_reaches_no_earlier_token(rule, what, value, D, V):
         assert torch.equal(got[:, 0], clean[:, 0]) and torch.equal(st[0], end[0])
         assert torch.equal(torch.isfinite(got), torch.isfinite(want))
         assert torch.equal(torch.isfinite(st), torch.isfinite(wst))
+
+
+def test_pieces_of_a_step():
+    """Cut at tile borders, each row once and in order, no sequence twice in a piece, no piece past its tiles."""
+    lens, pos0, slots = (40, 1, 0, 100, 16, 7), (3, 0, 0, 9, 0, 5), (5, 4, 3, 2, 1, 0)
+    seg = seg_meta(lens, pos0, slots, "cpu")
+    for most in (2, 3, 4, 7, 100):
+        at, seen = 0, {s: p for s, p in zip(slots, pos0)}
+        for i, j, m in S._mat_pieces(seg, 100, S.MAT_SCRATCH * 100 // most):
+            assert i == at and j - i == m.row0_host[-1] and len(set(m.slot_host)) == m.n_seg == len(m.pos0_host)
+            assert m.seg_row0.tolist() == m.row0_host and m.seg_pos0.tolist() == m.pos0_host
+            assert m.seg_slot.tolist() == m.slot_host and len(m.row_seg) == j - i
+            n = [b - a for a, b in zip(m.row0_host[:-1], m.row0_host[1:])]
+            assert sum(-(-k // 16) for k in n) <= most
+            for s, p, k in zip(m.slot_host, m.pos0_host, n):
+                assert p == seen[s]
+                seen[s] += k
+            at = j
+        assert at == sum(lens) and all(seen[s] == p + n for s, p, n in zip(slots, pos0, lens))
+
+
+@gpu
+@pytest.mark.parametrize("tiles", [2, 3, 5])
+def test_workspace_within_a_bound(tiles, monkeypatch):
+    """A step past the bound goes in several, to the results of the whole one."""
+    H, D, V, lens, pos0, slots = 2, 64, 64, (100, 17, 1, 45), (0, 4, 3, 9), (3, 0, 2, 1)
+    T, g = sum(lens), torch.Generator().manual_seed(2)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).cuda()
+    x, a, beta, xm, gb = rnd(T, 2 * H * D + H * V), rnd(T, H * D), rnd(T, H + 2), rnd(T, 2 * H * (D + V) + 2 * H), rnd(2 * H)
+    states, m = [rnd(4, H, D, V), rnd(4, H, D, V), rnd(4, H, D), rnd(4, H)], seg_meta(lens, pos0, slots, "cuda")
+
+    def run():
+        st = [s.clone() for s in states]
+        return [S.gated_delta(x, H, H, D, V, a, torch.ones(H).cuda(), torch.zeros(H * D).cuda(), beta[:, 2:], st[0], m),
+                *S.matrix_memory(xm, H, D, V, gb, 9.0, *st[1:], m, defer_scale=True), *st]
+    want = run()
+    assert S._mat_tiles(m, 0, H, D, V)[0].shape[0] == 13
+    monkeypatch.setattr(S, "MAT_SCRATCH", S._mat_tiles(m, 0, H, D, V)[2] * tiles // 13 + 1)
+    for p, q in zip(run(), want):
+        assert float((p - q).abs().max()) < 1e-5 * float(q.abs().max())
