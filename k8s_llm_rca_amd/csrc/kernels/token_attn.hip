@@ -41,7 +41,7 @@ __device__ __forceinline__ float tok_finish(const TokOut& a, int row, int head, 
   w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
   const float L = l * w + (a.sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f);
   const float g = a.gate ? 1.f / (1.f + expf(-a.gate[(size_t)row * a.gs + head])) : 1.f;
-  return L > 0.f ? g / L : 0.f;
+  return L == 0.f ? 0.f : g / L;                           // (NaN stays NaN)
 }
 
 __device__ __forceinline__ void tok_store4(const TokOut& a, int row, int head, int c, const f32x4& v) {
@@ -150,8 +150,8 @@ __global__ void __launch_bounds__(256) token_merge_kernel(TokOut a, const int* _
   for (int p = lane; p < np; p += 64) M = fmaxf(M, ml[p * 2]);
   M = wave_max(M);
   for (int p = lane; p < np; p += 64) {
-    const float m = ml[p * 2];
-    if (m != -INFINITY) L = fmaf(ml[p * 2 + 1], __builtin_amdgcn_exp2f(m - M), L);
+    const float m = ml[p * 2];                             // -inf: no visible key, or no score that is a number
+    L = fmaf(ml[p * 2 + 1], m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M), L);
   }
   L = wave_sum(L);
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};

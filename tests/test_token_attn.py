@@ -164,3 +164,23 @@ def test_partial_results_within_a_bound(monkeypatch):
         monkeypatch.setattr(S, "TOKEN_SCRATCH", limit)
         x, y, most = run()
         assert torch.equal(x, a) and torch.equal(y, b) and most <= max(limit, H * 11 * D)
+
+
+@pytest.mark.parametrize("sink", [False, True])
+def test_a_query_that_is_not_a_number(sink):
+    """All scores NaN: the row's result is, in one part and in many, and no other row's."""
+    H, G, D, n = 4, 2, 64, len(ENDS)
+    g = torch.Generator().manual_seed(5)
+    q, kc, vt = (torch.randn(*s, generator=g).to(BF).cuda() for s in ((n, H * D), (24, BS, G * D), (24, G * D, BS)))
+    qa, c, ct = (torch.randn(*s, generator=g).to(BF).cuda() for s in ((n, H, D), (24, BS, D), (24, D, BS)))
+    m, s = meta(ENDS, list(range(24))), torch.zeros(H).cuda() if sink else None
+
+    def run():
+        return (S.masked_attention(q, H, G, D, D, kc, None, m, 0.1, vt=vt, sink=s).view(n, H, D),
+                S.latent_attention_mfma(qa, c, ct, None, m, m.seg_pos0, 0.1, sink=s))
+    clean, bad = run(), [1, 7, 13]
+    q[bad, :D], qa[bad, 0, 3] = math.nan, math.nan
+    hit = torch.zeros(n, H, dtype=torch.bool, device="cuda")
+    hit[bad, 0] = True
+    for x, y in zip(run(), clean):
+        assert bool(torch.isnan(x[hit]).all()) and torch.equal(x[~hit], y[~hit])
