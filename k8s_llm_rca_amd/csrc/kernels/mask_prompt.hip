@@ -9,6 +9,9 @@
 // registers 8 s .. 8 s + 7 are the weights operand of O^T = V^T P^T as they stand.  LDS rows are padded by 16 bytes: the
 // 16 rows a quarter wave reads 16 bytes of lie in different banks for D = 64, 96 and 128 alike.
 //
+// Few tiles behind many keys: a tile's blocks are cut into parts, a workgroup each, whose outputs a second kernel joins
+// (n_parts; 500 rows at 8000 keys, 16 heads over 2 of 128: 211 -> 62 us).
+//
 // Zero weights times values that are not finite are NaN in rows that do not see their keys.  A tile that ends with a result
 // that is not finite walks its keys once more (CARE): in blocks that some token does not see whole, such values are parked
 // as zeros, and added behind the walk where they are seen.  (Looking at every block's values on the way cost 3.5 %.)
@@ -39,6 +42,10 @@ struct MaskPromptArgs {
   float* out32;           // the same in fp32 instead
   int H, G, M, BS, chunk, window, keep_first;    // H: heads (each with M maps)
   float scale, softcap;
+  // few tiles: a tile's blocks are split over grid.y workgroups of part_blocks each, whose results a merge joins
+  int n_parts, part_blocks, row_base;            // row_base: the first tile's first row
+  float* po;              // [rows][H M][n_parts][V]
+  float* pml;             // [rows][H M][n_parts][2]
 };
 
 // of a pair of bf16 numbers: bits 15 and 31 set where one is infinite or NaN (an exponent of ones)
@@ -81,6 +88,15 @@ __global__ void __launch_bounds__(64 * NW, ND == 4 && NV == 2 ? 3 : 2) mask_prom
   const int lo_al = k0.lo & ~63, a_beg = k0.a0 & ~63;
   const int a_end = a.window > 0 ? min(lo_al, (a.keep_first + 63) & ~63) : a_beg;
   const int nblkA = max(0, (a_end - a_beg) >> 6), nblk = nblkA + ((pos_last - lo_al) >> 6) + 1;
+  const int b_lo = blockIdx.y * a.part_blocks, b_hi = (int)blockIdx.y == a.n_parts - 1 ? nblk : min(nblk, b_lo + a.part_blocks);
+  const size_t part = (((size_t)(row0 + tt - a.row_base) * HM + head) * a.n_parts + blockIdx.y);
+  if (b_lo >= b_hi) {                                       // the whole workgroup: a part without blocks
+    if (valid && hi == 0) {
+      a.pml[part * 2] = -INFINITY;
+      a.pml[part * 2 + 1] = 0.f;
+    }
+    return;
+  }
   const int* pages = a.bt + (size_t)sg * a.maxb;
   auto block_at = [&](int bi) { return bi < nblkA ? a_beg + 64 * bi : lo_al + 64 * (bi - nblkA); };
 
@@ -146,20 +162,20 @@ __global__ void __launch_bounds__(64 * NW, ND == 4 && NV == 2 ? 3 : 2) mask_prom
     for (int dt = 0; dt < NV; ++dt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
-    m = a.sink && valid ? a.sink[head] * kLog2e : -INFINITY;
+    m = a.sink && valid && a.n_parts == 1 ? a.sink[head] * kLog2e : -INFINITY;
     l = 0.f;
-    int kb_next = block_at(min(1, nblk - 1)), pg0 = page0(kb_next), pg1 = page1(kb_next);
+    int kb_next = block_at(min(b_lo + 1, b_hi - 1)), pg0 = page0(kb_next), pg1 = page1(kb_next);
     {
-      const int kb = block_at(0);
+      const int kb = block_at(b_lo);
       load(kb, page0(kb), page1(kb));
-      park(0, kb, care);
+      park(b_lo & 1, kb, care);
     }
     __syncthreads();
-    for (int bi = 0; bi < nblk; ++bi) {
+    for (int bi = b_lo; bi < b_hi; ++bi) {
       const int kb = block_at(bi);
       // the page of the block after the next, while this one is computed (the last ones are read again: every load is
       // unconditional, so the count of loads in flight is known)
-      const int kb_after = block_at(min(bi + 2, nblk - 1)), pa0 = page0(kb_after), pa1 = page1(kb_after);
+      const int kb_after = block_at(min(bi + 2, b_hi - 1)), pa0 = page0(kb_after), pa1 = page1(kb_after);
       load(kb_next, pg0, pg1);
       // a wave all of whose tokens come before the block, or after its window or chunk, has nothing to do
       const bool live = wt0 < ntok && kb <= wp1 && kb + 63 >= cw_lo && (kb + 63 >= ww_lo || kb < keep);
@@ -268,7 +284,7 @@ __global__ void __launch_bounds__(64 * NW, ND == 4 && NV == 2 ? 3 : 2) mask_prom
   if (!valid) return;
   l += __shfl_xor(l, 32, 64);
   if (care) {                                               // (a weight above zero leaves infinity and NaN what they are)
-    for (int bi = 0; bi < nblk; ++bi) {
+    for (int bi = b_lo; bi < b_hi; ++bi) {
       const int kb = block_at(bi);
       if (open(kb)) continue;
       for (int key = kb; key < min(kb + 64, limit + 1); ++key) {
@@ -283,6 +299,19 @@ __global__ void __launch_bounds__(64 * NW, ND == 4 && NV == 2 ? 3 : 2) mask_prom
           }
       }
     }
+  }
+  if (a.n_parts > 1) {
+    if (hi == 0) {
+      a.pml[part * 2] = m;
+      a.pml[part * 2 + 1] = l;
+    }
+    float* po = a.po + part * V + 4 * hi;
+#pragma unroll
+    for (int dt = 0; dt < NV; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; i += 4)
+        *reinterpret_cast<f32x4*>(po + 32 * dt + 2 * i) = f32x4{o[dt][i], o[dt][i + 1], o[dt][i + 2], o[dt][i + 3]};
+    return;
   }
   if (a.sink) l += __builtin_amdgcn_exp2f(a.sink[head] * kLog2e - m);
   float f = 1.f / l;
@@ -301,10 +330,71 @@ __global__ void __launch_bounds__(64 * NW, ND == 4 && NV == 2 ? 3 : 2) mask_prom
     }
 }
 
+// Joins the parts of a (row, head).  S threads share four of its columns (W such groups to a row), each takes every S-th part;
+// theirs are joined in order.  S = 1 where the parts are few; eight for the many parts of few rows.
+template <int S>
+__global__ void __launch_bounds__(256) mask_prompt_merge_kernel(MaskPromptArgs a, size_t n4, int W) {
+  constexpr float kLog2e = 1.4426950408889634f;
+  __shared__ f32x4 sacc[S > 1 ? 256 : 1];
+  __shared__ float sml[S > 1 ? 256 : 1][2];
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) / S;
+  const int s = threadIdx.x % S, HM = a.H * a.M, n = a.n_parts;
+  const bool on = i < n4;
+  const size_t rh = (on ? i : 0) / W, row = a.row_base + rh / HM;
+  const int head = rh % HM, c = (on ? i : 0) - rh * W;
+  const float* ml = a.pml + rh * n * 2;
+  const f32x4* po = reinterpret_cast<const f32x4*>(a.po) + rh * n * W + c;
+  float M = -INFINITY, L = 0.f;
+#pragma unroll 8
+  for (int p = s; p < n; p += S) M = fmaxf(M, ml[2 * p]);
+  if (S == 1 && a.sink) M = fmaxf(M, a.sink[head] * kLog2e);
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float Ms = M == -INFINITY ? 0.f : M;
+#pragma unroll 8
+  for (int p = s; p < n; p += S) {
+    const float l = ml[2 * p + 1], f = __builtin_amdgcn_exp2f(ml[2 * p] - Ms);
+    const f32x4 v = po[(size_t)p * W];
+    L = fmaf(l, f, L);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[k] = l == 0.f ? acc[k] : fmaf(v[k], f, acc[k]);   // (l 0: a part this row sees no key of)
+  }
+  if (S > 1) {
+    sacc[threadIdx.x] = acc;
+    sml[threadIdx.x][0] = M;
+    sml[threadIdx.x][1] = L;
+    __syncthreads();
+    if (s > 0) return;
+    if (a.sink) M = fmaxf(M, a.sink[head] * kLog2e);
+#pragma unroll
+    for (int k = 1; k < S; ++k) M = fmaxf(M, sml[threadIdx.x + k][0]);
+  }
+  if (!on) return;
+  const float Mt = M == -INFINITY ? 0.f : M;
+  if (S > 1) {
+    L = 0.f;
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      const float f = __builtin_amdgcn_exp2f(sml[threadIdx.x + k][0] - Mt), l = sml[threadIdx.x + k][1];
+      L = fmaf(l, f, L);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[j] = l == 0.f ? acc[j] : fmaf(sacc[threadIdx.x + k][j], f, acc[j]);
+    }
+  }
+  if (a.sink) L += __builtin_amdgcn_exp2f(a.sink[head] * kLog2e - Mt);
+  float f = 1.f / L;
+  if (a.gate) f *= 1.f / (1.f + __expf(-a.gate[row * a.gs + head]));
+  const size_t o = (row * HM + head) * W * 4 + 4 * c;
+  if (a.out32)
+    *reinterpret_cast<f32x4*>(a.out32 + o) = f32x4{acc[0] * f, acc[1] * f, acc[2] * f, acc[3] * f};
+  else
+    *reinterpret_cast<u16x4*>(a.out + o) = u16x4{f2bf(acc[0] * f), f2bf(acc[1] * f), f2bf(acc[2] * f), f2bf(acc[3] * f)};
+}
+
 template <int ND, int NV, int NW>
-static int launch_mp(const MaskPromptArgs& a, hipStream_t s) {
+static int launch_mp(const MaskPromptArgs& a, int rows, hipStream_t s) {
   const int hpg = a.H / a.G, hw = hpg < 32 * NW ? hpg : 32 * NW;
-  const dim3 grid(a.n_items * a.G * a.M * ((hpg + hw - 1) / hw));
+  const dim3 grid(a.n_items * a.G * a.M * ((hpg + hw - 1) / hw), a.n_parts);
 #define K8S_MP(CAP, HALF) \
   hipLaunchKernelGGL((mask_prompt_kernel<ND, NV, NW, CAP, HALF>), grid, dim3(64 * NW), 0, s, a)
   if (a.softcap > 0.f) {
@@ -315,6 +405,12 @@ static int launch_mp(const MaskPromptArgs& a, hipStream_t s) {
     else K8S_MP(false, false);
   }
 #undef K8S_MP
+  if (a.n_parts == 1) return (int)hipGetLastError();
+  const size_t n4 = (size_t)rows * a.H * a.M * NV * 8;
+  if (a.n_parts <= 8)
+    hipLaunchKernelGGL(mask_prompt_merge_kernel<1>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, a, n4, NV * 8);
+  else
+    hipLaunchKernelGGL(mask_prompt_merge_kernel<8>, dim3((unsigned)((n4 + 31) / 32)), dim3(256), 0, s, a, n4, NV * 8);
   return (int)hipGetLastError();
 }
 
@@ -324,13 +420,17 @@ using namespace k8s;
 
 K8S_API int k8s_masked_attn_mfma_ok(int H, int G, int D, int V);
 
-// Items of up to max(1, 128 / (H / G)) tokens.
+// Items of up to max(1, 128 / (H / G)) tokens.  n_parts > 1: the items are the rows row_base .. row_base + rows of the step,
+// each tile's list of 64-key blocks is cut into parts of part_blocks (the last part takes what is left);
+// po [rows][H maps][n_parts][V], pml [.. ][2].
 K8S_API int k8s_masked_attn_prompt(const void* q, const void* kc, const void* vt, const int* bt, int maxb, const int* items,
                                    int n_items, const float* sink, const float* gate, int gs, void* out, int H, int G,
                                    int D, int V, int BS, int chunk, int window, int keep_first, float scale, float softcap,
-                                   hipStream_t s, int maps, int out_f32) {
+                                   hipStream_t s, int maps, int out_f32, int n_parts, int part_blocks, int row_base, int rows,
+                                   float* po, float* pml) {
   if (n_items <= 0) return 0;
-  if (!k8s_masked_attn_mfma_ok(H, G, D, V) || BS % 32 || chunk < 0 || window < 0 || keep_first < 0 || maps < 1)
+  if (!k8s_masked_attn_mfma_ok(H, G, D, V) || BS % 32 || chunk < 0 || window < 0 || keep_first < 0 || maps < 1 ||
+      n_parts < 1 || (n_parts > 1 && (part_blocks < 1 || rows < 1 || row_base < 0 || !po || !pml)))
     return (int)hipErrorInvalidValue;
   MaskPromptArgs a;
   a.q = (const uint16_t*)q; a.kc = (const uint16_t*)kc; a.vt = (const uint16_t*)vt; a.bt = bt; a.maxb = maxb;
@@ -338,9 +438,10 @@ K8S_API int k8s_masked_attn_prompt(const void* q, const void* kc, const void* vt
   a.out = out_f32 ? nullptr : (uint16_t*)out; a.out32 = out_f32 ? (float*)out : nullptr;
   a.H = H; a.G = G; a.M = maps; a.BS = BS; a.chunk = chunk; a.window = window; a.keep_first = keep_first;
   a.scale = scale; a.softcap = softcap;
-  if (D == 96) return launch_mp<6, 3, 4>(a, s);
-  if (D == 64 && V == 64) return launch_mp<4, 2, 4>(a, s);
-  if (D == 64 && V == 128) return launch_mp<4, 4, 4>(a, s);
-  if (D == 128 && V == 64) return launch_mp<8, 2, 4>(a, s);
-  return launch_mp<8, 4, 4>(a, s);
+  a.n_parts = n_parts; a.part_blocks = n_parts > 1 ? part_blocks : 1 << 30; a.row_base = row_base; a.po = po; a.pml = pml;
+  if (D == 96) return launch_mp<6, 3, 4>(a, rows, s);
+  if (D == 64 && V == 64) return launch_mp<4, 2, 4>(a, rows, s);
+  if (D == 64 && V == 128) return launch_mp<4, 4, 4>(a, rows, s);
+  if (D == 128 && V == 64) return launch_mp<8, 2, 4>(a, rows, s);
+  return launch_mp<8, 4, 4>(a, rows, s);
 }

@@ -97,8 +97,8 @@ class _DecodeSegments(SegMeta):
     def attn_items(self, tokens_per_item: int) -> tuple:
         return self.items, self.items[:0], self.pos0_host[0] + 1
 
-    def mask_items(self, tokens_per_item: int) -> tuple:
-        return self.items, self.items[:0], self.pos0_host[0] + 1
+    def mask_items(self, tokens_per_item: int, by_rows: bool = False) -> tuple:
+        return self.items, self.items[:0]
 
     def tile_items(self, tokens_per_item: int) -> torch.Tensor:
         return self.items

@@ -95,30 +95,43 @@ class SegMeta:
             got = self._items[key] = host.to(self.row_seg.device, non_blocking=True)
         return got
 
-    def mask_items(self, tokens_per_item: int) -> tuple:
-        """Work items of the masked attention, made once per step: (items of one token, tiles of at most
-        ``tokens_per_item``, most keys an item of one token sees).  The leading segments of one token are single items,
-        and so are all rows where no more than ``MASK_FEW_ROWS`` stand behind them."""
-        key = ("mask", tokens_per_item)
+    def _once(self, key: tuple, make):
         got = self._items.get(key)
         if got is None:
-            n1 = 0
-            while n1 < self.n_seg and self.row0_host[n1 + 1] - self.row0_host[n1] == 1:
-                n1 += 1
-            if self.row0_host[-1] - n1 <= MASK_FEW_ROWS:
-                n1 = self.n_seg
-            it, kmax, n = [], 0, 0
+            got = self._items[key] = make()
+        return got
+
+    def _behind(self, first: int, end: Optional[int] = None):
+        """(rows, position of the first) of the segments from ``first`` to ``end``."""
+        return ((b - a, p) for a, b, p in zip(self.row0_host[first:-1], self.row0_host[first + 1:], self.pos0_host[first:end]))
+
+    def singles(self) -> int:
+        """How many segments of one token stand in front (made once per step, as what follows)."""
+        return self._once(("singles",), lambda: next((i for i, (n, _) in enumerate(self._behind(0)) if n != 1), self.n_seg))
+
+    def most_keys(self, first: int, end: int) -> int:
+        """Most keys that a row of the segments from ``first`` to ``end`` sees."""
+        return self._once(("most", first, end), lambda: max((p + n for n, p in self._behind(first, end)), default=0))
+
+    def mask_items(self, tokens_per_item: int, by_rows: bool = False) -> tuple:
+        """Work items of the masked attention, made once per step: (items of one token, tiles of at most
+        ``tokens_per_item``).  The leading segments of one token are single items, and with ``by_rows`` all rows are."""
+        key = ("mask", tokens_per_item, by_rows)
+        got = self._items.get(key)
+        if got is None:
+            n1 = self.n_seg if by_rows else self.singles()
+            it, n = [], 0
             for s in range(self.n_seg):
                 a, b, p0 = self.row0_host[s], self.row0_host[s + 1], self.pos0_host[s]
                 step = 1 if s < n1 else tokens_per_item
                 it += [(s, r, min(step, b - r), p0 + r - a) for r in range(a, b, step)]
                 if s < n1:
-                    kmax, n = max(kmax, p0 + b - a), len(it)
+                    n = len(it)
             host = torch.from_numpy(np.asarray(it, dtype=np.int32).reshape(-1, 4))
             if self.row_seg.device.type == "cuda":
                 host = host.pin_memory()
             both = host.to(self.row_seg.device, non_blocking=True)
-            got = self._items[key] = (both[:n], both[n:], kmax)
+            got = self._items[key] = (both[:n], both[n:])
         return got
 
     def chunk_ranges(self, rows: int, min_rows: int) -> Optional[tuple]:
@@ -1141,23 +1154,39 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
             assert vt.is_contiguous() and vt.shape[1:] == (G * V, BS) and BS % 32 == 0
             common = (ptr(sink), ptr(gate), gs, ptr(out), H, G, D, V, BS, int(chunk), int(window), int(keep_first),
                       float(scale), float(softcap), stream_ptr(q))
-            bt, maxb = seg.block_tables, seg.block_tables.shape[1]
-            rows, tiles, kmax = seg.mask_items(max(1, MASK_TILE_ROWS // (H // G)))
-            if rows.shape[0]:
+            tpi = max(1, MASK_TILE_ROWS // (H // G))
+            def row_parts(kmax: int) -> int:      # parts of a row of so many keys: 32-key blocks
                 nblk = -(-kmax // 32)
                 if window > 0:     # the window from a block's border on; + the kept blocks
                     nblk = min(nblk, (int(window) + 62) // 32 + -(-int(keep_first) // 32))
                 if chunk > 0:
                     nblk = min(nblk, (int(chunk) + 62) // 32)
-                n_parts = min(-(-nblk // MASK_TOKEN_BLOCKS), TOKEN_PARTS)
+                return min(-(-nblk // MASK_TOKEN_BLOCKS), TOKEN_PARTS)
+            n1, end = seg.singles(), seg.n_seg
+            tmax, row0 = seg.most_keys(n1, end), seg.row0_host[n1]
+            few = T - row0 <= MASK_FEW_ROWS
+            rows, tiles = seg.mask_items(tpi, few)
+            bt, maxb = seg.block_tables, seg.block_tables.shape[1]
+            if rows.shape[0]:
+                n_parts = row_parts(seg.most_keys(0, end if few else n1))
                 groups, po, pml = _token_groups(rows, HQ, n_parts, V)
                 for it in groups:
                     check(lib().k8s_masked_attn_token(ptr(q), ptr(kc), ptr(vt), ptr(bt), maxb, ptr(it), it.shape[0],
                                                       *common, MASK_TOKEN_BLOCKS, TOKEN_PARTS, n_parts, ptr(pml), ptr(po),
                                                       int(maps), int(out_f32)), "masked_attn_token")
             if tiles.shape[0]:
+                nblk = -(-tmax // 64)
+                if window > 0:     # the first token's window from a block's border to the last token; + the kept blocks
+                    nblk = min(nblk, (int(window) + tpi + 125) // 64 + -(-int(keep_first) // 64))
+                if chunk > 0:
+                    nblk = min(nblk, (int(chunk) + tpi + 125) // 64)
+                n_parts, pb = _tile_parts(tiles.shape[0] * G * maps * -(-(H // G) // MASK_TILE_ROWS), nblk)
+                po = pml = None
+                if n_parts > 1:
+                    po, pml = (scratch((T - row0) * HQ * n_parts * n, torch.float32, q.device) for n in (V, 2))
                 check(lib().k8s_masked_attn_prompt(ptr(q), ptr(kc), ptr(vt), ptr(bt), maxb, ptr(tiles), tiles.shape[0],
-                                                   *common, int(maps), int(out_f32)), "masked_attn_prompt")
+                                                   *common, int(maps), int(out_f32), n_parts, pb, row0, T - row0, ptr(po),
+                                                   ptr(pml)), "masked_attn_prompt")
             return out
         assert vc is not None          # the vector-pipe kernel reads token-major values
         parts, po, pml = _rows_parts(seg, T, HQ, H // G, V, q.device, int(chunk), int(window), int(keep_first))
@@ -1198,6 +1227,25 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
             o = o * torch.sigmoid(gate[a:e, :HQ])[:, :, None]
         out[a:e] = o.reshape(n, HQ * V).to(out.dtype)
     return out
+
+
+# Prompt tiles cut over their keys where few of them would leave the chip idle behind a long context.  us, whole / cut, 16
+# heads over 2 of 128: 200 rows at 1000 keys 39 / 21, at 2000 62 / 26, at 8000 205 / 40;  1200 rows 64 / 50, 87 / 61, 227 /
+# 136;  4 over 4 of 64 at 8000, 500 rows 242 / 24 (tiles of 16 tokens, cut over 32 parts, 74).  The more workgroups there are
+# already, the longer a part has to be to pay for its share of the results' way to the merge: 16 over 2, 1200 rows in a window
+# of 1024 (150 workgroups, 18 blocks) 37 whole, 41 in two parts;  32 over 8, 800 rows from 0 (200, 13) 30 / 35;  500 rows in
+# the window (128, 18) 46 / 37.
+MASK_TILE_FILL = 512     # workgroups the chip holds at once
+MASK_TILE_BLOCKS = 4     # 64-key blocks of a part at least, and a fifteenth of the workgroups
+
+
+def _tile_parts(groups: int, nblk: int) -> tuple:
+    """(parts a tile's keys are cut into, 64-key blocks of a part) for a launch of ``groups`` workgroups without a cut."""
+    n = min(MASK_TILE_FILL // groups, nblk // max(MASK_TILE_BLOCKS, groups // 15))
+    if n < 2:
+        return 1, 0
+    pb = -(-nblk // n)
+    return -(-nblk // pb), pb
 
 
 def masked_mfma_ok(H: int, G: int, D: int, V: int, dtype, device) -> bool:

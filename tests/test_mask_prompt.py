@@ -69,9 +69,11 @@ def test_prompts(H, G, D, V, maps, BS, kw):
 @pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
 @pytest.mark.parametrize("H,G,D,V,BS", [(8, 1, 128, 128, 64), (2, 2, 64, 64, 32), (4, 2, 96, 96, 96)])
 @pytest.mark.parametrize("kw", [dict(), dict(window=50, keep_first=7), dict(chunk=40, softcap=9.0)])
-def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(H, G, D, V, BS, kw, value):
+@pytest.mark.parametrize("way", ["tiles", "parts"])
+def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(H, G, D, V, BS, kw, value, way, monkeypatch):
     """One entry of one key's value, of a key at every place in a block: rows that do not see the key keep their bits, and so
     do all other columns; keys that nobody has written are not read into the sums either."""
+    monkeypatch.setattr(S, "MASK_TILE_BLOCKS", 1 if way == "parts" else 1000)
     n, lead = 240, 60
     g = torch.Generator().manual_seed(BS)
     N = -(-n // BS)
@@ -81,7 +83,6 @@ def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(H, G, D, V
     def i32(x):
         return torch.tensor(x, dtype=torch.int32, device="cuda")
     m = S.SegMeta(1, i32([0] * T), i32([0, T]), i32([lead]), i32([0]), i32([list(range(N))]), [0, T], [lead], [0])
-    assert m.mask_items(max(1, 128 // (H // G)))[1].shape[0] > 0
 
     def run(keys):
         vx = v.clone()
@@ -105,3 +106,23 @@ def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(H, G, D, V
         hit = torch.zeros_like(got, dtype=torch.bool)
         hit[sees, (G - 1) * (H // G):, V - 3] = True
         assert bool((got[~hit] == clean[~hit]).all()) and not bool(torch.isfinite(got[hit]).any())
+
+
+@pytest.mark.parametrize("H,G,D,V,maps,BS", [(16, 2, 128, 128, 1, 64), (6, 2, 64, 128, 2, 64), (131, 1, 64, 64, 1, 128),
+                                             (5, 1, 128, 64, 1, 32)])
+@pytest.mark.parametrize("kw", [dict(), dict(window=130, keep_first=70), dict(chunk=100, window=33, keep_first=3),
+                                dict(chunk=50, softcap=6.0), dict(scale=0.0)])
+def test_tiles_cut_over_their_keys(H, G, D, V, maps, BS, kw, monkeypatch):
+    """The same against 64 bits with every 64-key block of a tile in a part of its own."""
+    monkeypatch.setattr(S, "MASK_TILE_BLOCKS", 1)
+    monkeypatch.setattr(S, "MASK_TILE_FILL", 1 << 20)
+    test_prompts(H, G, D, V, maps, BS, kw)
+
+
+def test_parts_of_a_tile():
+    """No block is left out, no part is empty where the list is longest, and a full chip is not cut."""
+    for groups in (1, 7, 26, 255, 256, 257, 512, 5000):
+        for nblk in (1, 7, 8, 9, 31, 125, 1000):
+            n, pb = S._tile_parts(groups, nblk)
+            assert n == 1 or (n * pb >= nblk > (n - 1) * pb and pb >= S.MASK_TILE_BLOCKS and n * groups <= S.MASK_TILE_FILL)
+    assert S._tile_parts(26, 125)[0] > 8 and S._tile_parts(257, 1000) == (1, 0)
