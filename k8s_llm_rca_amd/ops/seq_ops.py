@@ -33,10 +33,15 @@ LATENT_PART = 128        # keys, from the part of the row's first visible key on
 TOKEN_PARTS = 64         # a row with more than so many of them has larger ones
 TOKEN_SCRATCH = 1 << 28  # floats of partial results (1 GiB): a step of more takes its rows in groups
 MASK_TILE_ROWS = 128     # (token, head) rows of one workgroup of the masked prompt kernel
-# A step's prompt rows up to which they are taken one by one as well (masked layers): the tiles of one sequence each walk all
-# their keys, the rows have them cut into parts.  us, prompt kernel / rows, 16 heads over 2: 8 rows at 0 / 500 / 2000 keys
-# 7.7 / 4.9, 20 / 11.5, 62 / 11.7;  128 rows 11.5 / 6.5, 25.7 / 25.7, 68 / 63;  256 rows 14.7 / 14.4, 29 / 49, 72 / 121.
-MASK_FEW_ROWS = 128
+# A step's prompt rows are taken one by one as well (masked layers) while the keys and values they read stay within so many
+# bytes, and they and their parts within two rounds of workgroups: the rows have their keys cut into parts, and a tile's way
+# from keys to results is longer, but it reads them once for 128 (row, head) pairs (so two rows may read four times as much).
+# us, tiles / rows:  16 heads over 2 of 128, 16 / 64 / 128 rows at 0 keys 11 / 7, 11 / 8, 12 / 8, at 500 20 / 13, 20 / 17,
+# 22 / 26, at 2000 18 / 14, 21 / 36, 24 / 63, 2 rows at 30000 26 / 21;  16 over 16, 8 / 32 / 64 rows at 0 keys 10 / 8, 9 / 9,
+# 9 / 16, at 500 18 / 13, 17 / 38, 18 / 70, at 8000 25 / 111, 24 / 387, 28 / 760;  4 over 4 of 64, 8 / 32 rows at 2000 16 / 11,
+# 14 / 22;  8 over 1 of 64, 64 / 128 / 256 / 300 rows at 0 9 / 8, 10 / 7, 12 / 8, 13 / 16.
+MASK_ROW_BYTES = 32 << 20
+MASK_ROW_GROUPS = 512
 
 
 @dataclass
@@ -112,6 +117,16 @@ class SegMeta:
     def most_keys(self, first: int, end: int) -> int:
         """Most keys that a row of the segments from ``first`` to ``end`` sees."""
         return self._once(("most", first, end), lambda: max((p + n for n, p in self._behind(first, end)), default=0))
+
+    def keys_behind(self, first: int, most: int) -> int:
+        """Keys that the rows of the segments from ``first`` on see, each row its own, ``most`` of them at most."""
+        def count():
+            total = 0
+            for n, p in self._behind(first):
+                low = max(0, min(n, most - p))      # rows that see all of theirs: p + 1, p + 2 ..
+                total += low * p + low * (low + 1) // 2 + (n - low) * most
+            return total
+        return self._once(("behind", first, most), count)
 
     def mask_items(self, tokens_per_item: int, by_rows: bool = False) -> tuple:
         """Work items of the masked attention, made once per step: (items of one token, tiles of at most
@@ -1162,9 +1177,11 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
                 if chunk > 0:
                     nblk = min(nblk, (int(chunk) + 62) // 32)
                 return min(-(-nblk // MASK_TOKEN_BLOCKS), TOKEN_PARTS)
-            n1, end = seg.singles(), seg.n_seg
+            per_row, n1, end = G * maps * -(-(H // G) // 16), seg.singles(), seg.n_seg
             tmax, row0 = seg.most_keys(n1, end), seg.row0_host[n1]
-            few = T - row0 <= MASK_FEW_ROWS
+            most = min(int(chunk) or 1 << 30, int(window) + int(keep_first) if window > 0 else 1 << 30)
+            few = (row0 == T or (T - row0) * per_row * row_parts(tmax) <= MASK_ROW_GROUPS
+                   and (1 - 1.5 / (T - row0)) * seg.keys_behind(n1, most) * per_row * (D + V) * 2 <= MASK_ROW_BYTES)
             rows, tiles = seg.mask_items(tpi, few)
             bt, maxb = seg.block_tables, seg.block_tables.shape[1]
             if rows.shape[0]:

@@ -73,6 +73,7 @@ def test_prompts(H, G, D, V, maps, BS, kw):
 def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(H, G, D, V, BS, kw, value, way, monkeypatch):
     """One entry of one key's value, of a key at every place in a block: rows that do not see the key keep their bits, and so
     do all other columns; keys that nobody has written are not read into the sums either."""
+    monkeypatch.setattr(S, "MASK_ROW_BYTES", -1)
     monkeypatch.setattr(S, "MASK_TILE_BLOCKS", 1 if way == "parts" else 1000)
     n, lead = 240, 60
     g = torch.Generator().manual_seed(BS)
@@ -126,3 +127,11 @@ def test_parts_of_a_tile():
             n, pb = S._tile_parts(groups, nblk)
             assert n == 1 or (n * pb >= nblk > (n - 1) * pb and pb >= S.MASK_TILE_BLOCKS and n * groups <= S.MASK_TILE_FILL)
     assert S._tile_parts(26, 125)[0] > 8 and S._tile_parts(257, 1000) == (1, 0)
+
+
+@pytest.mark.parametrize("most", [1 << 30, 40, 5])
+def test_keys_that_rows_see(most):
+    m = S.SegMeta(3, *[None] * 5, [0, 1, 31, 40], [9, 0, 37], [0] * 3)
+    assert [m.keys_behind(f, most) for f in (0, 1, 3)] == [
+        sum(min(p + i + 1, most) for p, n in list(zip([9, 0, 37], [1, 30, 9]))[f:] for i in range(n)) for f in (0, 1, 3)]
+    assert m.singles() == 1
