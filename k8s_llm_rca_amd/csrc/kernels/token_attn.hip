@@ -225,9 +225,9 @@ struct MaskTokArgs {
 
 // grid (rows, key heads (x maps) x groups of 16 of their heads, parts); a part is a run of the row's list of 32-key blocks
 // (kept first tokens, then the window's or chunk's).
-template <int NDC, int NV, bool CAP>
-__global__ void __launch_bounds__(512) masked_attn_token_kernel(MaskTokArgs a) {
-  constexpr int D = NDC * 32, V = NV * 16, NW = 8;
+template <int NDC, int NV, bool CAP, int NW>
+__global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs a) {
+  constexpr int D = NDC * 32, V = NV * 16;
   __shared__ TokLds<NW, V> lds;
   const int lane = threadIdx.x & 63, r = lane & 15, hq = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -402,17 +402,31 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
   tok_join<NW, ND>(lds, a.t, row, head0, nh, blockIdx.y, m, l, o);
 }
 
-template <int NDC, int NV>
-static int launch_mask_tok(const MaskTokArgs& a, int rows, hipStream_t s) {
+template <int NDC, int NV, int NW>
+static int launch_mask_tok_nw(const MaskTokArgs& a, int rows, hipStream_t s) {
   const int hpg = a.t.H / (a.G * a.t.hs);
   const dim3 grid(rows, a.G * a.t.hs * ((hpg + 15) / 16), a.t.n_parts);
   if (a.softcap > 0.f)
-    hipLaunchKernelGGL((masked_attn_token_kernel<NDC, NV, true>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((masked_attn_token_kernel<NDC, NV, true, NW>), grid, dim3(64 * NW), 0, s, a);
   else
-    hipLaunchKernelGGL((masked_attn_token_kernel<NDC, NV, false>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((masked_attn_token_kernel<NDC, NV, false, NW>), grid, dim3(64 * NW), 0, s, a);
   if (a.t.n_parts > 1)
     hipLaunchKernelGGL(token_merge_kernel, dim3(rows * a.t.H), dim3(256), 0, s, a.t, a.items, NV * 16);
   return (int)hipGetLastError();
+}
+
+// Waves by the sizes of a head and by whether heads share keys, by nothing that changes from step to step (a row's bits):
+// eight, so that a part's blocks are on their way together;  four with 64 + 64 numbers a key, whose registers let more
+// workgroups onto a compute unit;  two where every head has keys of its own, for its many workgroups.  us at 1 / 64 rows,
+// eight waves / this / tiles of 16 tokens:  16 heads over 16 of 128, 1 key 3.8 / 3.8 / 6.6 and 12.9 / 8.0 / 7.3, 200 keys
+// 6.6 / 7.5 / 20 and 28 / 24 / 32, 4000 keys 11.1 / 12.2 / 37 and 480 / 399 / 442;  12 over 6 of 64 at 4000 keys 64 rows
+// 122 / 78 / 94;  4 over 4 of 64 8.5 / 8.7 / 25 and 75 / 45 / 65.
+template <int NDC, int NV>
+static int launch_mask_tok(const MaskTokArgs& a, int rows, hipStream_t s) {
+  if constexpr (NDC == 2 && NV == 4)
+    return launch_mask_tok_nw<NDC, NV, 4>(a, rows, s);
+  else
+    return a.t.H > a.G * a.t.hs ? launch_mask_tok_nw<NDC, NV, 8>(a, rows, s) : launch_mask_tok_nw<NDC, NV, 2>(a, rows, s);
 }
 
 template <int NR>
