@@ -387,11 +387,39 @@ def rotated_tail(q: torch.Tensor, cs: torch.Tensor, H: int, N: int, pad: int) ->
     return out
 
 
-# Rows up to which small products run on the vector pipes (csrc/kernels/small_proj.hip).  us, library / this, at 1, 16, 64,
-# 128 rows: 16 heads 128 -> 256 with the rotated part 7.3 / 3.1, 7.3 / 4.7, 9.1 / 5.5, 9.6 / 7.2;  256 -> 128 6.9 / 3.4,
-# 6.3 / 5.2, 6.5 / 5.6, 7.4 / 6.9, in fp32 6.5 / 3.4, 6.6 / 5.1, 11.9 / 5.8, 20 / 8.1 and 9.5 / 4.4, 8.5 / 5.7, 11.4 / 6.8,
-# 18.8 / 9.3;  two of 64 -> 2048 with their roundings 12.2 / 2.5, 11.8 / 3.6, 12.4 / 4.0, 12.2 / 5.5.
+# Rows up to which small products run on the vector pipes (csrc/kernels/small_proj.hip), within :func:`_few_heads` and
+# :func:`_few_ranks`.
 SMALL_PROJ_ROWS = 128
+
+
+def _few_heads(T: int, H: int, K: int, N: int, fp32: bool) -> bool:
+    """Whether ``T`` rows of ``H`` products K -> N are quicker on the vector pipes than the library's batched product: while
+    the multiply-adds hide behind one trip to memory, and while a thread's share of K (an eighth, in turn) is short.  us,
+    library / this, bf16 (fp32):  16 heads 128 -> 256 at 1, 16, 64, 128 rows 5.3 / 3.0, 5.2 / 4.5, 6.2 / 5.1, 7.4 / 6.7
+    (6.5 / 3.2, 6.5 / 5.0, 11.7 / 5.6, 19.7 / 7.9), 256 -> 128 7.1 / 3.6, 6.2 / 5.2, 6.4 / 5.6, 7.4 / 6.9 (9.4 / 4.2, 8.4 /
+    5.5, 11.3 / 6.7, 18.6 / 8.9);  64 heads 128 -> 128 at 16, 32, 64 rows 5.0 / 4.6, 4.9 / 5.1, 5.5 / 6.7;  128 heads 64 ->
+    256 at 8, 16 4.8 / 4.2, 4.8 / 5.3;  512 -> 128 at 1, 8, 16 of 4 heads 9.5 / 5.3, 9.6 / 7.8, 7.0 / 7.9 (12.1 / 6.4, 12.4 /
+    8.8, 10.8 / 8.8);  128 -> 512 of 4 at 4, 8 3.6 / 3.3, 3.6 / 4.2;  512 -> 512 of 16 at 1, 16 6.7 / 7.1, 6.8 / 10.3;  256 ->
+    64 of 4 at 2, 8 4.4 / 4.3, 4.4 / 4.7;  640 and 1024 entries: never."""
+    m = T * H * K * N
+    if N > 256:
+        return T <= 4 and K <= 128 and m <= 1 << 24
+    if K > 256:
+        return N <= 128 and K <= 512 and (m <= 1 << 26 if fp32 else T <= 8)
+    if 2 * N < K and not fp32:
+        return T <= 2
+    most = (1 << 26 if fp32 else 1 << 25) if K >= 128 else 1 << 24
+    if T >= 4 * H and (K < 128 or K * N >= 1 << 15):     # (the library takes the longer the more rows a head has)
+        most *= 2
+    return m <= most
+
+
+def _few_ranks(T: int, K0: int, N0: int, K1: int, N1: int) -> bool:
+    """The same for two products of low rank.  us, two roundings and two products / this:  64 -> 2048 at 1, 16, 128 rows
+    11.9 / 2.3, 11.5 / 3.4, 11.8 / 5.3, 64 -> 8192 at 128 16.8 / 14.9;  256 -> 8192 at 32, 64 18.5 / 15.2, 19.5 / 24.6;  512
+    -> 2048 at 4, 8, 16, 64 10.4 / 8.3, 10.7 / 13.0, 11.4 / 13.0, 20.2 / 15.3;  1024 -> 2048 at 2, 64 11.7 / 14.4, 29.5 / 27.6."""
+    K = max(K0, K1)
+    return T * (K0 * N0 + K1 * N1) <= 1 << 27 and (K <= 256 or K <= 512 and not 4 < T < 64)
 
 
 def _small_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -408,8 +436,8 @@ def head_proj(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tens
     but the last are free): a kernel of one launch for few rows, the library's batched product otherwise."""
     T, H, K = x.shape
     N = w.shape[2]
-    if (_small_heads(x, w) and x.dtype == out.dtype and x.stride(2) == 1 == out.stride(2) and K % 8 == 0
-            and K <= 1024 and N % 64 == 0):
+    if (_small_heads(x, w) and x.dtype == out.dtype and x.stride(2) == 1 == out.stride(2) and K % 8 == 0 and N % 64 == 0
+            and _few_heads(T, H, K, N, x.dtype == torch.float32)):
         check(lib().k8s_head_proj(ptr(x), x.stride(0), x.stride(1), ptr(w), ptr(out), out.stride(0), out.stride(1), T, H, K,
                                   N, None, None, 0, 0, _dt(x.dtype), stream_ptr(x)), "head_proj")
     else:
@@ -424,7 +452,8 @@ def latent_queries(q: torch.Tensor, uk: torch.Tensor, cs: Optional[torch.Tensor]
     T, KR = q.shape[0], uk.shape[2]
     x = q.view(T, H, -1)
     R = x.shape[2] - D
-    if _small_heads(q, uk) and q.is_contiguous() and D % 8 == 0 and D <= 1024 and KR % 64 == 0:
+    if (_small_heads(q, uk) and q.is_contiguous() and D % 8 == 0 and KR % 64 == 0
+            and _few_heads(T, H, D, KR, q.dtype == torch.float32)):
         qa = torch.empty(H, T, KR, dtype=q.dtype, device=q.device).transpose(0, 1)
         qr = None
         if R:
@@ -442,7 +471,7 @@ def low_rank_pair(x: torch.Tensor, c0: int, w0: torch.Tensor, c1: int, w1: torch
     from .linear import proj_f32out
     T, (N0, K0), (N1, K1) = x.shape[0], w0.shape, w1.shape
     if (_small_rows(x, w0) and _small_rows(x, w1) and dtype == torch.bfloat16 and x.dtype == torch.float32
-            and x.stride(1) == 1 and all(k % 32 == 0 and 0 < k <= 1024 for k in (K0, K1))
+            and x.stride(1) == 1 and all(k % 32 == 0 and k > 0 for k in (K0, K1)) and _few_ranks(T, K0, N0, K1, N1)
             and w0.data_ptr() % 16 == 0 == w1.data_ptr() % 16):
         a, b = (torch.empty(T, n, dtype=torch.float32, device=x.device) for n in (N0, N1))
         check(lib().k8s_low_rank_pair(ptr(x), x.stride(0), T, c0, K0, ptr(w0), N0, ptr(a), c1, K1, ptr(w1), N1, ptr(b),

@@ -115,3 +115,17 @@ def test_transforms_of_products_in_fp32():
         v = a.clone().requires_grad_()
         f(v).sum().backward()
         assert torch.allclose(v.grad, torch.autograd.grad(ref(v).sum(), v)[0], atol=1e-4)
+
+
+def test_sizes_of_small_products():
+    """The vector pipes take what they were measured faster at, over heads and sizes: (rows, heads, K, N) in bf16."""
+    for case, fast in {(1, 16, 128, 256): 1, (64, 16, 128, 256): 1, (128, 16, 128, 256): 1, (128, 16, 256, 128): 1,
+                       (16, 128, 128, 512): 0, (64, 32, 64, 512): 0, (1, 8, 1024, 1024): 0, (16, 4, 1024, 64): 0,
+                       (64, 64, 512, 512): 0, (2, 16, 512, 512): 0, (64, 64, 128, 128): 0, (16, 64, 128, 128): 1,
+                       (64, 64, 64, 64): 1, (128, 128, 64, 64): 0, (8, 16, 512, 128): 1, (16, 4, 512, 128): 0}.items():
+        assert S._few_heads(*case, False) == bool(fast), case
+    for case, fast in {(128, 16, 256, 256): 1, (16, 16, 512, 128): 1, (16, 128, 512, 128): 0, (128, 16, 256, 128): 1}.items():
+        assert S._few_heads(*case, True) == bool(fast), case
+    for case, fast in {(128, 64, 2048, 64, 2048): 1, (128, 128, 4096, 256, 4096): 0, (16, 1024, 8192, 1024, 8192): 0,
+                       (64, 512, 2048, 512, 2048): 1, (16, 512, 2048, 512, 2048): 0, (1, 512, 2048, 512, 2048): 1, (32, 256, 8192, 256, 8192): 1}.items():
+        assert S._few_ranks(*case) == bool(fast), case
