@@ -160,6 +160,13 @@ SKINNY_F32_MAX_M = 32
 # at fewer rows (us, hipBLASLt / skinny: 8192 x 2048 at 16 rows 13.0 / 10.9, at 32 12.9 / 15.4; 8736 x 2048 at 7 / 16 / 32
 # 14.2 / 12.2, 14.2 / 14.4, 14.3 / 21.2; 2560 x 2048 at 32 9.8 / 8.0)
 SKINNY_F32_MAX_MN = 144 * 1024
+# ... where K is long; the rows of a short one are little to read (8192 x 1024 at 32 rows 11.9 / 9.3, x 512 at 24 9.4 / 6.7)
+SKINNY_F32_SHORT_K, SKINNY_F32_SHORT_MN = 1024, 256 * 1024
+
+
+def _skinny_f32(M: int, N: int, K: int) -> bool:
+    return (_enabled and 0 < M <= SKINNY_F32_MAX_M and N * K <= SKINNY_MAX_NK and K % 256 == 0 and N % 16 == 0
+            and M * N <= (SKINNY_F32_SHORT_MN if K <= SKINNY_F32_SHORT_K else SKINNY_F32_MAX_MN))
 
 
 def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -169,8 +176,7 @@ def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return linear(x, w)
     M, K = x.shape
     N = w.shape[0]
-    if (_enabled and 0 < M <= SKINNY_F32_MAX_M and M * N <= SKINNY_F32_MAX_MN and N * K <= SKINNY_MAX_NK
-            and K % 256 == 0 and N % 16 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+    if (_skinny_f32(M, N, K) and x.stride(1) == 1 and x.stride(0) % 8 == 0
             and w.dtype == torch.bfloat16 and w.is_contiguous()):
         out = torch.empty((M, N), dtype=torch.float32, device=x.device)
         check(lib().k8s_gemm_skinny_f32(ptr(x), x.stride(0), ptr(w), ptr(out), N, M, N, K, stream_ptr(x)),
@@ -199,9 +205,19 @@ def plane_plan(M: int, N: int, K: int):
     8.1 / 8.3 / 8.9 / 8.8, the skinny kernel 4.9 / 6.2 / 11.7 / --, 64-column planes 4.2 / 4.5 / 5.5 / 7.2, 32-column
     planes 4.1 / 4.4 / 4.8 / 6.6 and half as many to read;  2560 x 2048 32-column planes 5.0 / 5.3 / 6.8 / 10.0 against
     10.5 / 11.7 / 12.5 / 15.9;  2048 x 8192 12.4 / 12.5 / 21.8 / 20.8, 12.6 / 17.5 / 38 / --, 64-column 8.7 / 9.2 / 10.0 /
-    12.8, 32-column 9.9 / 10.0 / 11.5 / 15.6."""
+    12.8, 32-column 9.9 / 10.0 / 11.5 / 15.6.
+
+    Up to 16 rows the skinny kernel leaves the planes only where K is long for the columns, up to 32 where it is more than a
+    strip or two.  us with the pass behind, skinny / planes:  1024 x 512 at 1 / 16 rows 4.8 / 5.6, 5.5 / 6.1, x 1536 6.6 /
+    6.4, 7.7 / 6.8;  2048 x 1024 5.7 / 6.1, 6.8 / 6.4;  4096 x 1024 6.2 / 7.6, 7.3 / 7.9, x 3072 10.6 / 13.3, 12.0 / 12.5, x
+    6144 16.0 / 15.3, 18.6 / 15.5, x 8192 18.8 / 22.7, 22.1 / 22.5;  5120 x 1024 7.2 / 8.5, 9.2 / 9.0, x 2048 10.5 / 10.9,
+    13.3 / 11.7;  2048 x 256 at 24 rows 5.6 / 6.1."""
     if not 0 < M <= NARROW_MAX_M:
         return 14, 1
+    if _skinny_f32(M, N, K):
+        long_k = (1024 if M > 8 else 1536) if N <= 2048 else 1536 if N > 4096 else 3072 if M > 8 else 4096
+        if K <= 256 if M > 16 else K < long_k or N * K >= 1 << 25:
+            return 14, 1
     cfg, bn, s, most = (34, 32, 4, 320) if K < 4096 else (14, 64, 8, 256)
     while s > 1 and (-(-N // bn) * s > most or K < 128 * s or not stream_shape_ok(M, N, K, cfg, s)):
         s //= 2
@@ -255,11 +271,12 @@ def proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     kernel) and one wave of strips with the K it was measured at.  us at 17..32 / 64 / 128 rows, hipBLASLt / this:
     8192 x 2048 12.3 / 10.2, 12.8 / 11.1, 15.6 / 13.7;  4736 x 2048 12.3 / 9.7, 12.9 / 10.7, 15.2 / 13.6;  2048 x 2048
     9.2 / 8.3, 10.6 / 8.3, 10.5 / 10.6.  At 273 strips the second wave costs it the lead (8736 x 2048, 64 rows:
-    15.3 / 17.2)."""
+    15.3 / 17.2);  a long K over few strips does where the library cuts it (1024 x 2048 at 24 / 128 rows 8.1 / 9.0, 8.4 /
+    10.3, 2048 x 2048 11.1 / 9.2, 11.4 / 13.0)."""
     M, K = x.shape
     N = w.shape[0]
     if (16 < M <= NARROW_MAX_M and 32 <= N <= 32 * NARROW_WGS and K <= 2048 and (N, K) not in _dispatch and _few_ok(x, w)
-            and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
+            and (K < 1536 or N > 2048 or M <= 64 and N * K >= 9 << 18) and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
         return gemm_stream(x, w, _narrow_cfg(M), 1)
     return linear(x, w)
 
@@ -278,11 +295,15 @@ def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``max(x @ w.T, 0)^2`` as activations.  In one launch for up to 128 rows over one wave of 32-column strips (us apart /
     fused at 8192 x 2048: 1 row 10.5 / 9.8, 16 rows 12.9 / 10.1, 64 rows 15.5 / 11.0, 128 rows 17.9 / 13.9) and for prompts
     whose tiles fill the card (:func:`big_tiles_fill`) or whose K is so short that the result's passes are what is paid
-    (1024 x 256 at 16384 rows: 31 / 16); the fused forms square the fp32 sum."""
+    (1024 x 256 at 16384 rows: 31 / 16); the fused forms square the fp32 sum.  Not for few rows of up to 4096 columns: the
+    strips are half the card, and the skinny kernel and its pass are quicker (2048 x 2048 at 1, 8, 16 rows 6.6 / 9.2, 7.4 /
+    9.2, 8.0 / 9.2, x 1024 5.0 / 5.7, 5.7 / 5.9, 6.0 / 5.9, x 512 4.4 / 4.4, 4.9 / 4.7, 5.2 / 4.6)."""
     M, K = x.shape
     N = w.shape[0]
     if _few_ok(x, w):
-        if (0 < M <= NARROW_MAX_M and N <= 32 * NARROW_WGS and K <= 2048 and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
+        skinny = N <= 4096 and K > 512 and M <= (8 if K <= 1536 else 16)
+        if (0 < M <= NARROW_MAX_M and N <= 32 * NARROW_WGS and K <= 2048 and not skinny
+                and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
             out = torch.empty((M, N), dtype=x.dtype, device=x.device)
             check(lib().k8s_gemm_stream_act(ptr(x), x.stride(0), ptr(w), ptr(out), N, M, N, K, _narrow_cfg(M), 1,
                                             stream_ptr(x)), "gemm_stream_act")

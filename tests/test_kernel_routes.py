@@ -129,3 +129,12 @@ def test_sizes_of_small_products():
     for case, fast in {(128, 64, 2048, 64, 2048): 1, (128, 128, 4096, 256, 4096): 0, (16, 1024, 8192, 1024, 8192): 0,
                        (64, 512, 2048, 512, 2048): 1, (16, 512, 2048, 512, 2048): 0, (1, 512, 2048, 512, 2048): 1, (32, 256, 8192, 256, 8192): 1}.items():
         assert S._few_ranks(*case) == bool(fast), case
+
+
+def test_products_of_few_rows_by_shape():
+    """Planes and narrow strips where they were measured faster: (rows, columns, K)."""
+    for case, cut in {(1, 2048, 2048): 1, (1, 2048, 1024): 0, (16, 1024, 512): 0, (24, 2048, 512): 1, (24, 2048, 256): 0,
+                      (1, 4096, 1024): 0, (8, 3072, 3072): 0, (16, 5120, 2048): 1, (17, 4096, 1024): 1, (8, 2560, 4096): 1, (8, 4096, 8192): 0,
+                      (1, 2048, 8192): 1, (64, 2560, 1024): 1}.items():
+        assert (L.plane_plan(*case)[1] > 1) == bool(cut), case
+    assert L._skinny_f32(32, 8192, 1024) and not L._skinny_f32(32, 8192, 2048) and L._skinny_f32(17, 8192, 2048)
