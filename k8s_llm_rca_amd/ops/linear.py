@@ -291,13 +291,26 @@ def big_tiles_fill(M: int, N: int, silu: bool) -> bool:
     return 5 * tiles >= 4 * 256 * -(-tiles // 256)
 
 
+SHORT_K = 512       # up to here what is paid is the result's way through memory, not the tiles
+
+
+def big_fused(M: int, N: int, K: int, silu: bool) -> bool:
+    """Whether a prompt's product takes gemm_big's fused epilogue (N: result columns, of SwiGLU half the weight's rows): a
+    short K once the product is large enough to outweigh a wave of tiles that takes 10 to 17 us whatever it holds, a longer
+    one where the tiles fill the card.  us apart / fused of the squared relu, M x N in millions: K 128 at 2.5 (256 x 10000)
+    11.1 / 10.8, 3.2 (1280 x 2500) 12.4 / 11.3, 0.6 (512 x 1200) 7.5 / 10.4;  K 256 at 2.6 12.7 / 12.7, 3.8 15.0 / 13.3;  K
+    512 at 3.2 16.7 / 17.8, 5.1 21.4 / 18.4, 0.3 8.1 / 15.8."""
+    if K <= SHORT_K:
+        return M * N * (2 if silu else 1) >= (1 << 21) + 4096 * K
+    return big_tiles_fill(M, N, silu)
+
+
 def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``max(x @ w.T, 0)^2`` as activations.  In one launch for up to 128 rows over one wave of 32-column strips (us apart /
     fused at 8192 x 2048: 1 row 10.5 / 9.8, 16 rows 12.9 / 10.1, 64 rows 15.5 / 11.0, 128 rows 17.9 / 13.9) and for prompts
-    whose tiles fill the card (:func:`big_tiles_fill`) or whose K is so short that the result's passes are what is paid
-    (1024 x 256 at 16384 rows: 31 / 16); the fused forms square the fp32 sum.  Not for few rows of up to 4096 columns: the
-    strips are half the card, and the skinny kernel and its pass are quicker (2048 x 2048 at 1, 8, 16 rows 6.6 / 9.2, 7.4 /
-    9.2, 8.0 / 9.2, x 1024 5.0 / 5.7, 5.7 / 5.9, 6.0 / 5.9, x 512 4.4 / 4.4, 4.9 / 4.7, 5.2 / 4.6)."""
+    (:func:`big_fused`); the fused forms square the fp32 sum.  Not for few rows of up to 4096 columns: the strips are half the
+    card, and the skinny kernel and its pass are quicker (2048 x 2048 at 1, 8, 16 rows 6.6 / 9.2, 7.4 / 9.2, 8.0 / 9.2, x 1024
+    5.0 / 5.7, 5.7 / 5.9, 6.0 / 5.9, x 512 4.4 / 4.4, 4.9 / 4.7, 5.2 / 4.6)."""
     M, K = x.shape
     N = w.shape[0]
     if _few_ok(x, w):
@@ -308,7 +321,7 @@ def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             check(lib().k8s_gemm_stream_act(ptr(x), x.stride(0), ptr(w), ptr(out), N, M, N, K, _narrow_cfg(M), 1,
                                             stream_ptr(x)), "gemm_stream_act")
             return out
-        if M > DISPATCH_MAX_M and big_shape_ok(M, N, K) and (K <= 512 or big_tiles_fill(M, N, False)):
+        if M > DISPATCH_MAX_M and big_shape_ok(M, N, K) and big_fused(M, N, K, False):
             return gemm_big(x, w, relu2=True)
     return relu_sq(linear(x, w))
 
@@ -319,8 +332,7 @@ def glu_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     few weight bytes leave the skinny kernel ahead (4096 x 2048 11.4 / 9.9, 13.1 / 10.3, 15.8 / 11.1, 18.2 / 14.1;  2048 x
     2048 7.7 / 9.3, 9.3 / 9.6, 14.8 / 10.4, 17.8 / 13.5;  640 x 384 6.1 / 3.3 .. 9.4 / 4.6); wider weights the 64-row strips
     (6144 x 2048 14.2 / 12.9, 18.5 / 13.4, 19.4 / 14.5, 22.7 / 18.4), from 8192 on the register ring up to 32 rows (8192 x
-    2048 17.1 / 16.3, 22.5 / 16.3, then 21.3 / 17.3, 24.6 / 21.7).  Prompts: see :func:`big_tiles_fill`, or a short K
-    (640 x 384: always)."""
+    2048 17.1 / 16.3, 22.5 / 16.3, then 21.3 / 17.3, 24.6 / 21.7).  Prompts: :func:`big_fused`."""
     a = swiglu_gemm(x, w)
     if a is not None:
         return a
@@ -334,7 +346,7 @@ def glu_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
                 cfg = 8 if M <= 32 and I >= 8192 and K % 512 == 0 else 14
             if cfg and stream_shape_ok(M, 2 * I, K, cfg, 1) and I % (16 if cfg > 30 else 32) == 0:
                 return gemm_stream_silu(x, w, cfg)
-        elif M > DISPATCH_MAX_M and big_shape_ok(M, I, K, True) and (K <= 512 or big_tiles_fill(M, I, True)):
+        elif M > DISPATCH_MAX_M and big_shape_ok(M, I, K, True) and big_fused(M, I, K, True):
             return gemm_big(x, w, silu=True)
     return glu_clamp(linear(x, w), 1.0, math.inf, 0.0)
 

@@ -50,9 +50,11 @@ def test_glu_of_few_rows(m, i, k):
 
 
 @pytest.mark.parametrize("m,n,k,fused", [(1345, 8192, 2048, False), (1345, 10240, 2048, True), (16384, 256, 256, True),
-                                         (300, 1024, 384, True), (300, 1024, 640, False), (513, 768, 256, True)])
+                                         (300, 1024, 384, False), (300, 1024, 640, False), (513, 768, 256, False),
+                                         (5000, 768, 256, True), (4000, 1024, 512, False), (4200, 1024, 512, True)])
 def test_prompt_rows(m, n, k, fused):
-    assert (k <= 512 or L.big_tiles_fill(m, n, False)) == fused
+    assert L.big_fused(m, n, k, False) == fused == L.big_fused(m, n // 2, k, True) or k > 512
+    assert L.big_fused(m, n, k, False) == fused
     x, w = operands(m, n, k)
     want = x.double() @ w.double().T
     close(L.relu_sq_proj(x, w), want.clamp_min(0) ** 2, 3.1)
