@@ -1355,12 +1355,30 @@ def _mat_chunks(seg: SegMeta, H: int, V: int):
 MAT_TILE = 16       # tokens per tile of the matrix-core form
 
 
+def _long_and_few(seg: SegMeta, H: int, D: int, V: int) -> bool:
+    """Whether the matrix memory of a step is a long serial chain beside a nearly idle chip.  The tiles walk a sequence at 0.9
+    (D 16) to 2.1 us (D 128) a tile in a workgroup per head and 64 columns; chunks of 64 tokens run beside each other, until
+    they too fill the chip, with 4 D bytes of state per thread.  us chunks / tiles at 1000, 2000, 4000 tokens, by workgroups:
+    D 32, 4 73 / 79, 98 / 142, 148 / 279, 32 86 / 89, 127 / 160, 218 / 299, 64 100 / 93, 167 / 167;  D 64, 8 96 / 102, 136 /
+    193, 233 / 368, 16 111 / 108, 187 / 198, 342 / 378, 32 160 / 114, 295 / 207;  D 128, 4 183 / 148, 212 / 280, 327 / 536, 8
+    190 / 152, 274 / 284, 506 / 541, 16 249 / 156, 453 / 288;  D 16, 8 102 / 70, 129 / 127, 191 / 241, 32 110 / 74, 170 / 136,
+    312 / 252."""
+    longest = max(b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:]))
+    if longest < (2048 if D < 32 else 1024 if D <= 64 else 1792):
+        return False
+    groups = H * -(-V // 64) * (seg.row0_host[-1] / longest)     # short sequences beside it count by their tokens
+    return groups <= (1024 // D if D >= 32 else 16)
+
+
 def _mat_tiles(seg: SegMeta, kind: int, H: int, D: int, V: int):
     """(tiles, first tile of every segment, floats of workspace) for the matrix-core form of the delta rule (``kind`` 0) or
     the matrix memory (1), or None: no portion is long enough, or no form for ``D``.  Where the line lies (16 heads, D 64,
     V 128; token by token or in chunks -> tiles, us):  delta rule, one sequence of 16 / 17 / 129 tokens 21 -> 21 / 23 -> 19 /
     165 -> 29, 64 of 17 tokens 72 -> 52;  memory, one of 17 / 33 / 129 tokens 23 -> 27 / 30 -> 28 / 73 -> 29, 64 of 17 tokens
-    68 -> 48 -- its own steps are cheaper, so that few sequences need two tiles before the tiles' launch pays."""
+    68 -> 48 -- its own steps are cheaper, so that few sequences need two tiles before the tiles' launch pays, and long ones of
+    few heads go in chunks (:func:`_long_and_few`)."""
+    if kind == 1 and _long_and_few(seg, H, D, V):
+        return None
     per = lib().k8s_tile_state_ws(kind, D)      # floats per (tile, head)
     few = seg.n_seg * H * -(-V // 64) < MAT_FILL_GROUPS
     cr = seg.chunk_ranges(MAT_TILE, 2 * MAT_TILE if kind == 1 and few else MAT_TILE) if per else None
