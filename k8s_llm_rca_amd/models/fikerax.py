@@ -447,14 +447,15 @@ class FikeraxModel:
                 y, w, rms = glu_proj(h, L["w13"]), L["w2"], None                 # silu(gate) * up
             # (a pass that reads the embedding once more adds the product too)
             y = proj_planes(y, w) if into.get("again") or rms is not None else proj_add(x[:, 0], y, w)
+            if layers_out is not None and into.get("again"):   # the residual in front of the embedding added once more
+                before = x.clone()
+                N.hyper_step(before, y, one, mix1, rms=rms)
             if y is not None:
                 h = N.hyper_step(x, y, one, mix1, rms=rms, **into)
             elif into:
                 h = N.hyper_read(x, None, into["nw"], eps, dt)
             if layers_out is not None:
-                # (the residual in front of the embedding that a further pass adds)
-                layers_out.append(x[:, 0] - self.embed[inp.input_ids.long()].float() * cfg.embed_scale if into.get("again")
-                                  else x[:, 0].clone())
+                layers_out.append(before[:, 0] if into.get("again") else x[:, 0].clone())
         if inp.logits_idx is not None:
             h = N.hyper_read(x, inp.logits_idx, self.final_norm, eps, dt)
         return proj_f32out(h, self.head)

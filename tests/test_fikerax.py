@@ -586,6 +586,22 @@ def test_layers_match_after_every_run(backend):
         assert e < (1e-5 if dt == torch.float32 else 0.03), (i, e)
 
 
+def test_the_residual_in_front_of_a_repeated_pass_is_not_rounded_again():
+    """What is handed out behind the pass before a repeated one is the residual itself, as without the loop."""
+    layers = [(lat(), 40), (lig(), 0), (att(), 36), (lig(), 0)]
+    outs = []
+    for loop in ((1, 4, 2), None):
+        d = config(layers, loop=loop)
+        eng = engine(d, weights(d, 1), ("cpu", torch.float32))
+        got, fw = [], eng.model.forward
+        eng.model.forward = lambda *a, **k: fw(*a, layers_out=got, **k)
+        eng.feed([(eng.new_sequence(), toks(45, d["vocab"], 2), [])])
+        outs.append(got)
+    assert [len(o) for o in outs] == [7, 4]
+    for a, b in zip(outs[0], outs[1]):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("backend", BACKENDS)
 @pytest.mark.parametrize("cuts", [(), (70,), (30, 2, 2, 17, 3, 5), (69,), (1, 68), (2,) * 35])
 def test_prefill_decode_and_portions_agree_with_oracle(backend, cuts):
