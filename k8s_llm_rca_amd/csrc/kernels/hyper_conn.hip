@@ -50,7 +50,8 @@ __device__ __forceinline__ void stv<4, uint16_t>(uint16_t* p, size_t i, const fl
 }
 
 // this thread's first columns of the norm's weight, asked for with the row itself: behind the sum they would be a second
-// trip to memory (one row of 2048 in a reply step: 4.6 -> 4.3 us)
+// trip to memory.  (One row of 2048: 4.2 to 4.6 us in a traced reply step with this and with the load behind the sum, so it
+// gains nothing there; 2.65 against 2.54 where all of it lies in the caches.)
 template <int VEC>
 __device__ __forceinline__ void first_weights(const float* __restrict__ w, int W, bool on, float (&w0)[VEC]) {
 #pragma unroll

@@ -17,8 +17,9 @@
 // as zeros, and added behind the walk where they are seen.  (Looking at every block's values on the way cost 3.5 %.)
 //
 // What bounds it: matrix and vector instructions of two waves a SIMD in turn (240 registers).  Eight prompts of 2048, 16
-// heads over 2 of 128, us: causal 245 = 561 TFLOP/s, a window of 1024 180 = 574, chunks of 1024 with capped scores 170 =
-// 405 (an exponential and a reciprocal more per score).  Tiles of 16 tokens x 2 heads a wave with operands from the caches
+// heads over 2 of 128, us alone in a loop: causal 230 = 598 TFLOP/s, a window of 1024 175 = 590, chunks of 1024 with capped
+// scores 168 = 410 (an exponential and a reciprocal more per score);  between a prompt's other kernels, whose traffic has
+// taken the caches, the latter two 190 to 220 and 183 to 186.  Tiles of 16 tokens x 2 heads a wave with operands from the caches
 // took 681, 485 and 418: every wave fetched its keys itself.
 #include <type_traits>
 

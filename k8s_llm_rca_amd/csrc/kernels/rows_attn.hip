@@ -280,7 +280,8 @@ K8S_API int k8s_masked_attn_rows(const void* q, const void* kc, const void* vc, 
   if (T <= 0) return 0;
   if (maps < 1) return (int)hipErrorInvalidValue;
   const int HQ = H * maps;
-  // (a row's queries and outputs: at most 64 KB and 8192 numbers)
+  // the sizes callers may count on, all within this kernel's LDS: 8192 outputs a row; queries, 64 scores and two sums a head
+  // in 64 KB
   if (H < 1 || G < 1 || H % G || D < 1 || V < 1 || HQ * V > 8192 || chunk < 0 || window < 0 || keep_first < 0 ||
       (size_t)(HQ * D + HQ * 64 + 2 * HQ) * sizeof(float) > 64 * 1024 || (n_parts > 0 && (!po || !pml)))
     return (int)hipErrorInvalidValue;
@@ -331,7 +332,8 @@ K8S_API int k8s_latent_attn_rows(const float* qa, const void* cache, const int* 
   if (n_rows <= 0) return 0;
   if (H <= 0 || R <= 0 || R > 2048 || RP < 0 || (RP && !qr) || window < 0 || (n_parts > 0 && (!po || !pml)))
     return (int)hipErrorInvalidValue;
-  // (the widest cache rows: as many heads' queries as make 2048 numbers, 32 keys and their scores within 160 KB)
+  // the sizes callers may count on, all within this kernel's LDS: the queries of as many heads as make 2048 numbers beside 32
+  // cache rows and their scores in 160 KB
   const size_t hg = 2048 / R < H ? (2048 / R < 64 ? 2048 / R : 64) : (H < 64 ? H : 64);
   if ((hg * (R + RP) + 32 * (size_t)(R + RP + 1) + 35 * hg) * sizeof(float) > 160 * 1024) return (int)hipErrorInvalidValue;
   RowsArgs p{};

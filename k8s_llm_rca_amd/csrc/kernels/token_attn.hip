@@ -9,10 +9,10 @@
 // waves and parts follow from positions alone, so a row's bits do not depend on the step it is in.
 //
 // What bounds it: the chain row -> page -> keys -> scores -> join of some 5 us, and that one compute unit takes cold keys
-// in at 20 to 30 KB a us, far below its share of the caches' rate.  So parts are small (256 masked or 128 latent keys: 64
-// and 144 KB), and a merge of 3.5 us pays from the second part on.  16 heads over 2 of 128 / 16 heads over latents of
-// 256 + 64, us with the merge, and in brackets what a tile of 16 tokens per wave (masked) and a wave per 256 keys (latent)
-// took in engine steps of about that size: 1 row at 100 keys 5.3 / 8.5 (8.4 / 13.5), 8 rows at 1500 10.7 / 12.5 (26 / 36),
+// in at 20 to 30 KB a us, far below its share of the caches' rate.  So parts are small (256 masked or 128 latent keys: 128
+// KB of keys and values and 144 KB), and a merge of 3.5 us pays from the second part on.  16 heads over 2 of 128 / 16 heads
+// over latents of 256 + 64, us with the merge, and in brackets what a tile of 16 tokens per wave (masked) and a wave per 256
+// keys (latent) took in engine steps of about that size: 1 row at 100 keys 5.3 / 8.5 (8.4 / 13.5), 8 rows at 1500 10.7 / 12.5 (26 / 36),
 // 64 rows at 400 12.3 / 14.3 (28 / 35).
 #include "common.h"
 #include "key_runs.h"

@@ -246,7 +246,8 @@ def _few_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 # Rows from which an output projection is added to the residual by the product itself, so that the norm behind it reads one
 # fp32 row instead of two and writes none.  us, product + residual and norm apart / together: K 8192 at 5000 rows 164 / 170,
-# 8102 246 / 231, 16384 509 / 465, 24730 856 / 800;  K 2048 at 2000 35 / 33, 8102 100 / 91, 16384 194 / 169, 24730 357 / 313.
+# 8102 246 / 231, 16384 509 / 465, 24730 856 / 800;  K 2048 at 2000 35 / 33, 8102 100 / 91, 16384 194 / 169, 24730 357 / 313
+# (2048 columns; at 256 to 5120 columns and 6200 to 32000 rows nothing is slower together).
 ADD_ROWS = 6144
 
 

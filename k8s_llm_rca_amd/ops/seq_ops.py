@@ -1560,7 +1560,8 @@ def matrix_memory(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tens
 # (csrc/kernels/state_step.hip): the state update with its gates, norm and output gate in one launch.  us, token-by-token
 # kernel with its gate and norm passes / this, 16 heads of 128 x 128 at 1 / 8 / 64 / 256 sequences: delta rule 14.1 / 7.1,
 # 16.6 / 7.3, 49.5 / 27.2, 181 / 111;  matrix memory 17.0 / 7.3, 20.7 / 6.7, 54.4 / 30.3, 181 / 109;  decaying attention
-# 9.4 / 5.8, 11.0 / 6.0, 40.1 / 28.4, 142 / 107 (the states' bytes, in and out: 0.4, 3.4, 27, 109).
+# 9.4 / 5.8, 11.0 / 6.0, 40.1 / 28.4, 142 / 107.  The states' bytes, in and out, take 0.4, 3.4, 27 and 109
+# at the rate of a large copy; of 268 MB the caches hold a part from one call to the next.
 def _step_ok(x: torch.Tensor, seg: SegMeta, D: int, V: int, state: torch.Tensor, gate: torch.Tensor,
              w: Optional[torch.Tensor]) -> bool:
     """Whether a step is one token each and rows, states, gates and weights can be read by 16 bytes."""
