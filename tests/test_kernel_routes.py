@@ -64,6 +64,28 @@ def test_unaligned_states_and_pages_give_the_same():
         assert float((p - q).abs().max()) <= 2.0 ** -7 * float(q.abs().max())
 
 
+def test_head_products_that_do_not_fit_are_refused(monkeypatch):
+    """Weights of other heads, other sizes or another device go to torch's batched product, as before there was a kernel; a
+    launch by address would read past them."""
+    monkeypatch.setattr(S, "use_hip", lambda *t: True)
+    monkeypatch.setattr(S, "lib", lambda: pytest.fail("launched"))
+    monkeypatch.setattr(S, "rotated_tail", lambda *a: None)
+    x, out = torch.zeros(2, 4, 16), torch.zeros(2, 4, 64)
+    assert S._small_heads(x, torch.zeros(4, 16, 64), 4, 16, out)
+    for w in (torch.zeros(3, 16, 64), torch.zeros(4, 8, 64), torch.zeros(4, 24, 64), torch.zeros(8, 16, 64)):
+        with pytest.raises(RuntimeError):
+            S.head_proj(x, w, out)
+        with pytest.raises(RuntimeError):
+            S.latent_queries(x.view(2, 64), w, None, 4, 16, 0)
+    with pytest.raises(RuntimeError):
+        S.latent_queries(torch.zeros(2, 48), torch.zeros(4, 16, 64), None, 4, 16, 0)      # rows shorter than their heads
+    assert not S._small_heads(x, torch.empty(4, 16, 64, device="meta"), 4, 16, out)
+    for bad in (torch.zeros(1, 4, 64), torch.zeros(2, 4, 128)):
+        S.head_proj(x, torch.zeros(4, 16, 64), bad)                                        # (torch sizes it anew)
+    with pytest.raises(RuntimeError):
+        S.head_proj(x, torch.zeros(4, 16, 64), torch.zeros(2, 4, 64, requires_grad=True))
+
+
 def test_calls_that_something_watches():
     """Every way in which torch has more to do with an operator than its numbers."""
     from torch.autograd import forward_ad
