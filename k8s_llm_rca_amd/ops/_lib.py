@@ -233,17 +233,23 @@ def check(rc: int, name: str) -> None:
             raise RuntimeError(f"{name}: device fault surfaced at sync: {e}") from e
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
 def unwatched(*tensors) -> bool:
     """Whether a kernel launched by address does all that torch's operator would with these tensors: neither autograd (either
     direction), ``torch.func``, tracing, compiling, a torch mode, a tensor subclass nor autocast has a part in the call.
-    Kernels that took a torch operator's place ask this and leave the others to the operator."""
-    f = torch._C._functorch.peek_interpreter_stack
-    if (f() is not None or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch.jit.is_tracing() or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")):
+    Kernels that took a torch operator's place ask this and leave the others to the operator: once the sizes fit, since it
+    takes 1.3 us of the host, and before strides and addresses, which such tensors need not have."""
+    C = torch._C
+    if (C._functorch.peek_interpreter_stack() is not None or C._len_torch_dispatch_stack() or C._len_torch_function_stack()
+            or C._get_tracing_state() is not None or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")):
         return False
-    grad = torch.is_grad_enabled()
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and not (grad and t.requires_grad)
-               and forward_ad.unpack_dual(t).tangent is None for t in tensors)
+    grad, dual = torch.is_grad_enabled(), forward_ad._current_level >= 0
+    for t in tensors:
+        if type(t) not in _PLAIN or (grad and t.requires_grad) or (dual and forward_ad.unpack_dual(t).tangent is not None):
+            return False
+    return True
 
 
 def use_hip(*tensors) -> bool:

@@ -70,9 +70,9 @@ FEW_F32_WIDE = 8192, 5
 
 def _few_f32_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     (M, K), N = x.shape, w.shape[0]
-    return (x.is_cuda and w.is_cuda and x.dtype == torch.float32 == w.dtype and unwatched(x, w)
+    return (x.is_cuda and w.is_cuda and x.dtype == torch.float32 == w.dtype
             and 0 < M <= (FEW_F32_WIDE[1] if N >= FEW_F32_WIDE[0] else FEW_F32_ROWS) and N > 0 and K > 0 and K % 4 == 0
-            and w.dim() == 2 and w.shape[1] == K and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and w.dim() == 2 and w.shape[1] == K and unwatched(x, w) and w.is_contiguous() and w.data_ptr() % 16 == 0
             and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.stride(0) >= K and x.data_ptr() % 16 == 0
             and x.stride(0) < 2 ** 31)
 

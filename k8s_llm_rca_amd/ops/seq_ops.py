@@ -427,11 +427,12 @@ def _small_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def _small_heads(x: torch.Tensor, w: torch.Tensor, H: int, K: int, *out) -> bool:
-    """Whether the products of ``H`` heads with ``w`` [H, K, N] may be launched by address: all else is for the library's
-    batched product, which refuses what does not fit."""
+    """Whether the products of ``H`` heads with ``w`` [H, K, N] may be launched by address and are quicker so: all else is for
+    the library's batched product, which refuses what does not fit."""
     return (use_hip(x) and 0 < x.shape[0] <= SMALL_PROJ_ROWS and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float32)
-            and w.shape[:2] == (H, K) and w.device == x.device and unwatched(x, w, *out) and w.is_contiguous()
-            and w.data_ptr() % 8 == 0)
+            and w.shape[:2] == (H, K) and w.device == x.device and K % 8 == 0 and w.shape[2] % 64 == 0
+            and _few_heads(x.shape[0], H, K, w.shape[2], x.dtype == torch.float32) and unwatched(x, w, *out)
+            and w.is_contiguous() and w.data_ptr() % 8 == 0)
 
 
 def head_proj(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
@@ -440,8 +441,7 @@ def head_proj(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tens
     T, H, K = x.shape
     N = w.shape[2]
     if (_small_heads(x, w, H, K, out) and x.dtype == out.dtype and out.shape == (T, H, N) and out.device == x.device
-            and x.stride(2) == 1 == out.stride(2) and K % 8 == 0 and N % 64 == 0
-            and _few_heads(T, H, K, N, x.dtype == torch.float32)):
+            and x.stride(2) == 1 == out.stride(2)):
         check(lib().k8s_head_proj(ptr(x), x.stride(0), x.stride(1), ptr(w), ptr(out), out.stride(0), out.stride(1), T, H, K,
                                   N, None, None, 0, 0, _dt(x.dtype), stream_ptr(x)), "head_proj")
     else:
@@ -456,8 +456,7 @@ def latent_queries(q: torch.Tensor, uk: torch.Tensor, cs: Optional[torch.Tensor]
     T, KR = q.shape[0], uk.shape[2]
     x = q.view(T, H, -1)
     R = x.shape[2] - D
-    if (_small_heads(q, uk, H, D) and R >= 0 and q.is_contiguous() and D % 8 == 0 and KR % 64 == 0
-            and _few_heads(T, H, D, KR, q.dtype == torch.float32)):
+    if _small_heads(q, uk, H, D) and R >= 0 and q.is_contiguous():
         qa = torch.empty(H, T, KR, dtype=q.dtype, device=q.device).transpose(0, 1)
         qr = None
         if R:
