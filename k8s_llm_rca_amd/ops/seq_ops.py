@@ -430,7 +430,7 @@ def _small_heads(x: torch.Tensor, w: torch.Tensor, H: int, K: int, *out) -> bool
     """Whether the products of ``H`` heads with ``w`` [H, K, N] may be launched by address and are quicker so: all else is for
     the library's batched product, which refuses what does not fit."""
     return (use_hip(x) and 0 < x.shape[0] <= SMALL_PROJ_ROWS and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float32)
-            and w.shape[:2] == (H, K) and w.device == x.device and K % 8 == 0 and w.shape[2] % 64 == 0
+            and w.shape[:2] == (H, K) and w.numel() > 0 and w.device == x.device and K % 8 == 0 and w.shape[2] % 64 == 0
             and _few_heads(x.shape[0], H, K, w.shape[2], x.dtype == torch.float32) and unwatched(x, w, *out)
             and w.is_contiguous() and w.data_ptr() % 8 == 0)
 

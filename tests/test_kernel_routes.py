@@ -80,6 +80,8 @@ def test_head_products_that_do_not_fit_are_refused(monkeypatch):
     with pytest.raises(RuntimeError):
         S.latent_queries(torch.zeros(2, 48), torch.zeros(4, 16, 64), None, 4, 16, 0)      # rows shorter than their heads
     assert not S._small_heads(x, torch.empty(4, 16, 64, device="meta"), 4, 16, out)
+    assert not S.head_proj(x[:, :, :0], torch.zeros(4, 0, 64), torch.ones(2, 4, 64)).any()        # a sum of nothing
+    assert S.head_proj(x, torch.zeros(4, 16, 0), out[:, :, :0]).numel() == 0
     for bad in (torch.zeros(1, 4, 64), torch.zeros(2, 4, 128)):
         S.head_proj(x, torch.zeros(4, 16, 64), bad)                                        # (torch sizes it anew)
     with pytest.raises(RuntimeError):
