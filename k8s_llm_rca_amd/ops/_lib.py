@@ -234,6 +234,8 @@ def check(rc: int, name: str) -> None:
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+_transforms, _tracing, _autocast = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state, torch.is_autocast_enabled
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
 
 
 def unwatched(*tensors) -> bool:
@@ -241,9 +243,8 @@ def unwatched(*tensors) -> bool:
     direction), ``torch.func``, tracing, compiling, a torch mode, a tensor subclass nor autocast has a part in the call.
     Kernels that took a torch operator's place ask this and leave the others to the operator: once the sizes fit, since it
     takes 1.3 us of the host, and before strides and addresses, which such tensors need not have."""
-    C = torch._C
-    if (C._functorch.peek_interpreter_stack() is not None or C._len_torch_dispatch_stack() or C._len_torch_function_stack()
-            or C._get_tracing_state() is not None or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")):
+    if (_transforms() is not None or _dispatch_modes() or _function_modes() or _tracing() is not None
+            or torch.compiler.is_compiling() or _autocast("cuda")):
         return False
     grad, dual = torch.is_grad_enabled(), forward_ad._current_level >= 0
     for t in tensors:

@@ -1,6 +1,7 @@
 """Projection GEMMs: hand-written skinny MFMA GEMM for decode shapes, hipBLASLt otherwise."""
 from __future__ import annotations
 
+import functools
 import json
 import math
 import os
@@ -212,9 +213,12 @@ def plane_plan(M: int, N: int, K: int):
     6.4, 7.7 / 6.8;  2048 x 1024 5.7 / 6.1, 6.8 / 6.4;  4096 x 1024 6.2 / 7.6, 7.3 / 7.9, x 3072 10.6 / 13.3, 12.0 / 12.5, x
     6144 16.0 / 15.3, 18.6 / 15.5, x 8192 18.8 / 22.7, 22.1 / 22.5;  5120 x 1024 7.2 / 8.5, 9.2 / 9.0, x 2048 10.5 / 10.9,
     13.3 / 11.7;  2048 x 256 at 24 rows 5.6 / 6.1."""
-    if not 0 < M <= NARROW_MAX_M:
-        return 14, 1
-    if _skinny_f32(M, N, K):
+    return _plane_plan(M, N, K, _enabled) if 0 < M <= NARROW_MAX_M else (14, 1)
+
+
+@functools.lru_cache(maxsize=4096)      # (asked for every product of a step; 1.2 us of the host worked out, 0.2 looked up)
+def _plane_plan(M: int, N: int, K: int, skinny: bool):
+    if skinny and _skinny_f32(M, N, K):
         long_k = (1024 if M > 8 else 1536) if N <= 2048 else 1536 if N > 4096 else 3072 if M > 8 else 4096
         if K <= 256 if M > 16 else K < long_k or N * K >= 1 << 25:
             return 14, 1

@@ -106,27 +106,29 @@ class SegMeta:
             got = self._items[key] = make()
         return got
 
-    def _behind(self, first: int, end: Optional[int] = None):
-        """(rows, position of the first) of the segments from ``first`` to ``end``."""
-        return ((b - a, p) for a, b, p in zip(self.row0_host[first:-1], self.row0_host[first + 1:], self.pos0_host[first:end]))
-
     def singles(self) -> int:
-        """How many segments of one token stand in front (made once per step, as what follows)."""
-        return self._once(("singles",), lambda: next((i for i, (n, _) in enumerate(self._behind(0)) if n != 1), self.n_seg))
+        """How many segments of one token stand in front."""
+        r = self.row0_host
+        for i in range(self.n_seg):
+            if r[i + 1] - r[i] != 1:
+                return i
+        return self.n_seg
 
     def most_keys(self, first: int, end: int) -> int:
         """Most keys that a row of the segments from ``first`` to ``end`` sees."""
-        return self._once(("most", first, end), lambda: max((p + n for n, p in self._behind(first, end)), default=0))
+        r, most = self.row0_host, 0
+        for i in range(first, end):
+            most = max(most, self.pos0_host[i] + r[i + 1] - r[i])
+        return most
 
     def keys_behind(self, first: int, most: int) -> int:
         """Keys that the rows of the segments from ``first`` on see, each row its own, ``most`` of them at most."""
-        def count():
-            total = 0
-            for n, p in self._behind(first):
-                low = max(0, min(n, most - p))      # rows that see all of theirs: p + 1, p + 2 ..
-                total += low * p + low * (low + 1) // 2 + (n - low) * most
-            return total
-        return self._once(("behind", first, most), count)
+        r, total = self.row0_host, 0
+        for i in range(first, self.n_seg):
+            n, p = r[i + 1] - r[i], self.pos0_host[i]
+            low = max(0, min(n, most - p))          # rows that see all of theirs: p + 1, p + 2 ..
+            total += low * p + low * (low + 1) // 2 + (n - low) * most
+        return total
 
     def mask_items(self, tokens_per_item: int, by_rows: bool = False) -> tuple:
         """Work items of the masked attention, made once per step: (items of one token, tiles of at most
@@ -429,9 +431,10 @@ def _small_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
 def _small_heads(x: torch.Tensor, w: torch.Tensor, H: int, K: int, *out) -> bool:
     """Whether the products of ``H`` heads with ``w`` [H, K, N] may be launched by address and are quicker so: all else is for
     the library's batched product, which refuses what does not fit."""
-    return (use_hip(x) and 0 < x.shape[0] <= SMALL_PROJ_ROWS and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float32)
-            and w.shape[:2] == (H, K) and w.numel() > 0 and w.device == x.device and K % 8 == 0 and w.shape[2] % 64 == 0
-            and _few_heads(x.shape[0], H, K, w.shape[2], x.dtype == torch.float32) and unwatched(x, w, *out)
+    T, (HW, KW, N), dt = x.shape[0], w.shape, x.dtype
+    return (use_hip(x) and 0 < T <= SMALL_PROJ_ROWS and dt == w.dtype and (dt == torch.bfloat16 or dt == torch.float32)
+            and HW == H > 0 and KW == K > 0 and N > 0 and w.device == x.device and K % 8 == 0 and N % 64 == 0
+            and _few_heads(T, H, K, N, dt == torch.float32) and unwatched(x, w, *out)
             and w.is_contiguous() and w.data_ptr() % 8 == 0)
 
 
@@ -532,7 +535,7 @@ def _token_groups(rows: torch.Tensor, heads: int, parts: int, V: int) -> tuple:
     if parts == 1:
         return [rows], None, None
     per = min(rows.shape[0], max(1, TOKEN_SCRATCH // (heads * parts * (V + 2))))
-    return (rows.split(per), *(scratch(per * heads * parts * n, torch.float32, rows.device) for n in (V, 2)))
+    return ([rows] if per == rows.shape[0] else rows.split(per), *(scratch(per * heads * parts * n, torch.float32, rows.device) for n in (V, 2)))
 
 
 def latent_attention_mfma(qa: torch.Tensor, cache: torch.Tensor, cache_t: torch.Tensor, gate: Optional[torch.Tensor],
@@ -1060,7 +1063,7 @@ def attn_prep(qkv: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D
     activations.  ``G = 0``: only queries (a layer that reads another layer's pages).  ``qkv`` [S, T, ..]: the sum of its
     planes (:func:`.linear.proj_planes`)."""
     planes, pstep = 1, 0
-    by16 = all(t is None or t.data_ptr() % 16 == 0 for t in (kc, rope_cs))      # (attn_prep_half)
+    by16 = (kc is None or kc.data_ptr() % 16 == 0) and (rope_cs is None or rope_cs.data_ptr() % 16 == 0)    # (attn_prep_half)
     if qkv.dim() == 3:
         if qkv.shape[0] > 1 and use_hip(qkv) and by16 and norm in (False, None, True, "head") and not q_temp and 8 <= D <= 512 \
                 and D & (D - 1) == 0 and (rope is None or (rope_cs is not None and not rope.pairs and rope.dims % 8 == 0)) \
@@ -1201,40 +1204,22 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
             assert vt.is_contiguous() and vt.shape[1:] == (G * V, BS) and BS % 32 == 0
             common = (ptr(sink), ptr(gate), gs, ptr(out), H, G, D, V, BS, int(chunk), int(window), int(keep_first),
                       float(scale), float(softcap), stream_ptr(q))
-            tpi = max(1, MASK_TILE_ROWS // (H // G))
-            def row_parts(kmax: int) -> int:      # parts of a row of so many keys: 32-key blocks
-                nblk = -(-kmax // 32)
-                if window > 0:     # the window from a block's border on; + the kept blocks
-                    nblk = min(nblk, (int(window) + 62) // 32 + -(-int(keep_first) // 32))
-                if chunk > 0:
-                    nblk = min(nblk, (int(chunk) + 62) // 32)
-                return min(-(-nblk // MASK_TOKEN_BLOCKS), TOKEN_PARTS)
-            per_row, n1, end = G * maps * -(-(H // G) // 16), seg.singles(), seg.n_seg
-            tmax, row0 = seg.most_keys(n1, end), seg.row0_host[n1]
-            most = min(int(chunk) or 1 << 30, int(window) + int(keep_first) if window > 0 else 1 << 30)
-            few = (row0 == T or (T - row0) * per_row * row_parts(tmax) <= MASK_ROW_GROUPS
-                   and (1 - 1.5 / (T - row0)) * seg.keys_behind(n1, most) * per_row * (D + V) * 2 <= MASK_ROW_BYTES)
-            rows, tiles = seg.mask_items(tpi, few)
+            rows, r_parts, tiles, t_parts, pb, row0 = seg._once(
+                ("mask plan", H, G, D, V, chunk, window, keep_first, maps),
+                lambda: _mask_plan(seg, H, G, D, V, int(chunk), int(window), int(keep_first), int(maps)))
             bt, maxb = seg.block_tables, seg.block_tables.shape[1]
             if rows.shape[0]:
-                n_parts = row_parts(seg.most_keys(0, end if few else n1))
-                groups, po, pml = _token_groups(rows, HQ, n_parts, V)
+                groups, po, pml = _token_groups(rows, HQ, r_parts, V)
                 for it in groups:
                     check(lib().k8s_masked_attn_token(ptr(q), ptr(kc), ptr(vt), ptr(bt), maxb, ptr(it), it.shape[0],
-                                                      *common, MASK_TOKEN_BLOCKS, TOKEN_PARTS, n_parts, ptr(pml), ptr(po),
+                                                      *common, MASK_TOKEN_BLOCKS, TOKEN_PARTS, r_parts, ptr(pml), ptr(po),
                                                       int(maps), int(out_f32)), "masked_attn_token")
             if tiles.shape[0]:
-                nblk = -(-tmax // 64)
-                if window > 0:     # the first token's window from a block's border to the last token; + the kept blocks
-                    nblk = min(nblk, (int(window) + tpi + 125) // 64 + -(-int(keep_first) // 64))
-                if chunk > 0:
-                    nblk = min(nblk, (int(chunk) + tpi + 125) // 64)
-                n_parts, pb = _tile_parts(tiles.shape[0] * G * maps * -(-(H // G) // MASK_TILE_ROWS), nblk)
                 po = pml = None
-                if n_parts > 1:
-                    po, pml = (scratch((T - row0) * HQ * n_parts * n, torch.float32, q.device) for n in (V, 2))
+                if t_parts > 1:
+                    po, pml = (scratch((T - row0) * HQ * t_parts * n, torch.float32, q.device) for n in (V, 2))
                 check(lib().k8s_masked_attn_prompt(ptr(q), ptr(kc), ptr(vt), ptr(bt), maxb, ptr(tiles), tiles.shape[0],
-                                                   *common, int(maps), int(out_f32), n_parts, pb, row0, T - row0, ptr(po),
+                                                   *common, int(maps), int(out_f32), t_parts, pb, row0, T - row0, ptr(po),
                                                    ptr(pml)), "masked_attn_prompt")
             return out
         assert vc is not None          # the vector-pipe kernel reads token-major values
@@ -1295,6 +1280,37 @@ def _tile_parts(groups: int, nblk: int) -> tuple:
         return 1, 0
     pb = -(-nblk // n)
     return -(-nblk // pb), pb
+
+
+def _mask_plan(seg: SegMeta, H: int, G: int, D: int, V: int, chunk: int, window: int, keep_first: int, maps: int) -> tuple:
+    """How a step's rows are shared out, made once per step and kind of layer (5 us of the host): (items of one token, parts
+    of their keys; tiles, parts of theirs, 64-key blocks of a part, the first tile's first row)."""
+    def row_parts(kmax: int) -> int:      # parts of a row of so many keys: 32-key blocks
+        nblk = -(-kmax // 32)
+        if window > 0:     # the window from a block's border on; + the kept blocks
+            nblk = min(nblk, (window + 62) // 32 + -(-keep_first // 32))
+        if chunk > 0:
+            nblk = min(nblk, (chunk + 62) // 32)
+        return min(-(-nblk // MASK_TOKEN_BLOCKS), TOKEN_PARTS)
+
+    tpi, hpg, T = max(1, MASK_TILE_ROWS // (H // G)), H // G, seg.row0_host[-1]
+    per_row, n1, end = G * maps * -(-hpg // 16), seg.singles(), seg.n_seg
+    tmax, row0 = seg.most_keys(n1, end), seg.row0_host[n1]
+    most = min(chunk or 1 << 30, window + keep_first if window > 0 else 1 << 30)
+    few = (row0 == T or (T - row0) * per_row * row_parts(tmax) <= MASK_ROW_GROUPS
+           and (1 - 1.5 / (T - row0)) * seg.keys_behind(n1, most) * per_row * (D + V) * 2 <= MASK_ROW_BYTES)
+    rows, tiles = seg.mask_items(tpi, few)
+    r_parts, t_parts, pb = 1, 1, 0
+    if rows.shape[0]:
+        r_parts = row_parts(seg.most_keys(0, end if few else n1))
+    if tiles.shape[0]:
+        nblk = -(-tmax // 64)
+        if window > 0:     # the first token's window from a block's border to the last token; + the kept blocks
+            nblk = min(nblk, (window + tpi + 125) // 64 + -(-keep_first // 64))
+        if chunk > 0:
+            nblk = min(nblk, (chunk + tpi + 125) // 64)
+        t_parts, pb = _tile_parts(tiles.shape[0] * G * maps * -(-hpg // MASK_TILE_ROWS), nblk)
+    return rows, r_parts, tiles, t_parts, pb, row0
 
 
 def masked_mfma_ok(H: int, G: int, D: int, V: int, dtype, device) -> bool:
