@@ -79,6 +79,15 @@ int k8s_gemm_big_rope(const void* x, int ldx, const void* w, void* qkv, int ldq,
                       hipStream_t s);
 int k8s_gemm_stream_silu(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int cfg,
                          hipStream_t s);
+int k8s_gemm_rows(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int nf, int ranges, int out,
+                  hipStream_t s);
+int k8s_gemm_rows_rope(const void* x, int ldx, const void* w, void* qkv, int ldq, int M, int N, int K, int nf, const int* pos,
+                       const float* cos_sin, const int* slots, void* kc, void* vc, int nq, int nkv, int BS, hipStream_t s);
+int k8s_gemm_rows_norm(const void* x, int x_stride, const float* part, int splits, const void* res_in, void* res_out,
+                       const void* norm_w, float eps, const void* w, void* y, int ldy, int M, int N, int K, int nf,
+                       const int* pos, const float* cos_sin, const int* slots, void* kc, void* vc, int nq, int nkv, int BS,
+                       hipStream_t s);
+int k8s_gemm_stream_reduce(const float* part, int splits, void* y, int ldy, int M, int N, hipStream_t s);
 int k8s_gemm_stream_push(const void* x, int ldx, const void* w, int M, int N, int K, int cfg, int splits, void* part,
                          int ar_id, int mode, hipStream_t s);
 int k8s_ar_push_addnorm_bf16(int id, void* res, const void* w, void* y, int T, int H, float eps, int mode, int S,
@@ -94,11 +103,12 @@ int k8s_gemm_stream_silu_norm(const void* x, int x_stride, const float* part, in
 }
 
 // kind: 0 hipBLASLt, 1 skinny, 2 gemm_mid (cfg, splits), 3 single-expert grouped (splits),
-// 4 gemm_stream (cfg = ring depth, splits), 5 gemm_big (cfg = schedule variant, splits);
+// 4 gemm_stream (cfg = ring depth, splits), 5 gemm_big (cfg = schedule variant, splits),
+// 6 gemm_rows (cfg = fragments of a workgroup, splits);
 // fuse: 1 -- a split-K o / down projection may leave its partials to the next norm;
-// 2 (gate_up, kinds 4 / 5 with one K split) -- the SwiGLU-epilogue form, which
+// 2 (gate_up, kinds 4 / 5 / 6 with one K split) -- the SwiGLU-epilogue form, which
 // writes act directly (gu is never written, no silu_mul launch);
-// 3 (qkv, kind 1) -- the skinny kernel's RoPE / KV-write epilogue (no rope_kv launch);
+// 3 (qkv, kinds 1 / 6) -- the kernel's RoPE / KV-write epilogue (no rope_kv launch);
 // 4 (qkv, kind 5) -- gemm_big's RoPE / KV-write epilogue (prefill sizes)
 struct K8sGemmSel {
   int kind, cfg, splits, fuse;
@@ -183,11 +193,11 @@ constexpr int kD = 128;
 // partials in the kind's scratch for the following norm to reduce
 // (k8s_splitk_addnorm); deferred() tells the caller where they are.
 bool deferred(const K8sGemmSel& g, bool defer) {
-  return defer && g.fuse && g.splits > 1 && (g.kind == 2 || g.kind == 3 || g.kind == 4 || g.kind == 5);
+  return defer && g.fuse && g.splits > 1 && g.kind >= 2 && g.kind <= 6;
 }
 
 const void* part_of(const K8sLlamaStep& s, const K8sGemmSel& g) {
-  return (g.kind == 2 || g.kind == 4 || g.kind == 5) ? s.mid_part : s.grp_part;
+  return g.kind == 3 ? s.grp_part : s.mid_part;
 }
 
 int gemm(const K8sLlamaStep& s, const K8sGemmSel& g, const void* x, int ldx, const void* w, void* y, int ldy, int M,
@@ -209,6 +219,11 @@ int gemm(const K8sLlamaStep& s, const K8sGemmSel& g, const void* x, int ldx, con
         return (d ? k8s_gemm_big_part : k8s_gemm_big_split)(x, ldx, w, y, ldy, M, N, K, g.cfg, g.splits, s.mid_part,
                                                             st);
       return k8s_gemm_big(x, ldx, w, y, ldy, M, N, K, 0, g.cfg, st);
+    case 6: {
+      if (g.splits == 1) return k8s_gemm_rows(x, ldx, w, y, ldy, M, N, K, g.cfg, 1, 0, st);
+      const int rc = k8s_gemm_rows(x, ldx, w, s.mid_part, N, M, N, K, g.cfg, g.splits, 1, st);
+      return rc || d ? rc : k8s_gemm_stream_reduce((const float*)s.mid_part, g.splits, y, ldy, M, N, st);
+    }
     default:
       return k8s_blaslt_gemm(x, ldx, w, y, ldy, M, N, K, s.blaslt_ws, s.blaslt_ws_bytes, st);
   }
@@ -253,16 +268,21 @@ K8S_API int k8s_llama_layers(const K8sLlamaStep* sp, hipStream_t st) {
   // current / other residual buffer (norm_fuse ping-pong, see K8sLlamaStep)
   void* rc = s.residual;
   void* ro = s.res2;
-  const bool nf_qkv = !tp && (s.norm_fuse & 1) && s.sel[0].kind == 1 && s.sel[0].fuse == 3;
-  const bool nf_gu = !tp && (s.norm_fuse & 2) && s.sel[2].kind == 4 && s.sel[2].fuse == 2;
+  const bool nf_qkv = !tp && (s.norm_fuse & 1) && (s.sel[0].kind == 1 || s.sel[0].kind == 6) && s.sel[0].fuse == 3;
+  const bool nf_gu = !tp && (s.norm_fuse & 2) && (s.sel[2].kind == 4 || s.sel[2].kind == 6) && s.sel[2].fuse == 2;
   for (int l = 0; l < s.L; ++l) {
     if (nf_qkv) {  // input norm + qkv GEMM + RoPE / KV write in one launch
       const bool first = l == 0;
       const float* part = pend ? (const float*)part_of(s, s.sel[3]) : nullptr;
-      K8S_TRY(k8s_gemm_skinny_rope_norm(first ? rc : (pend ? nullptr : s.prev), H, part, s.sel[3].splits,
-                                        first ? nullptr : rc, first ? nullptr : ro, s.in_norm[l], s.eps, s.wqkv[l],
-                                        qkv, ld_qkv, T, ld_qkv, H, s.pos, s.cos_sin, s.slots, s.kc[l], s.vc[l], s.nq,
-                                        s.nkv, s.BS, st));
+      const void* in = first ? rc : (pend ? nullptr : s.prev);
+      if (s.sel[0].kind == 6)
+        K8S_TRY(k8s_gemm_rows_norm(in, H, part, s.sel[3].splits, first ? nullptr : rc, first ? nullptr : ro, s.in_norm[l],
+                                   s.eps, s.wqkv[l], qkv, ld_qkv, T, ld_qkv, H, s.sel[0].cfg, s.pos, s.cos_sin, s.slots,
+                                   s.kc[l], s.vc[l], s.nq, s.nkv, s.BS, st));
+      else
+        K8S_TRY(k8s_gemm_skinny_rope_norm(in, H, part, s.sel[3].splits, first ? nullptr : rc, first ? nullptr : ro,
+                                          s.in_norm[l], s.eps, s.wqkv[l], qkv, ld_qkv, T, ld_qkv, H, s.pos, s.cos_sin,
+                                          s.slots, s.kc[l], s.vc[l], s.nq, s.nkv, s.BS, st));
       if (!first) {
         void* t = rc;
         rc = ro;
@@ -288,6 +308,9 @@ K8S_API int k8s_llama_layers(const K8sLlamaStep* sp, hipStream_t st) {
     } else if (s.sel[0].kind == 5 && s.sel[0].fuse == 4) {  // prefill-size qkv, RoPE / KV write in the epilogue
       K8S_TRY(k8s_gemm_big_rope(s.y, H, s.wqkv[l], qkv, ld_qkv, T, ld_qkv, H, s.pos, s.cos_sin, s.slots, s.kc[l],
                                 s.vc[l], s.nq, s.nkv, s.BS, s.sel[0].cfg, st));
+    } else if (s.sel[0].kind == 6 && s.sel[0].fuse == 3) {
+      K8S_TRY(k8s_gemm_rows_rope(s.y, H, s.wqkv[l], qkv, ld_qkv, T, ld_qkv, H, s.sel[0].cfg, s.pos, s.cos_sin, s.slots,
+                                 s.kc[l], s.vc[l], s.nq, s.nkv, s.BS, st));
     } else if (s.sel[0].kind == 1 && s.sel[0].fuse == 3) {  // skinny qkv with the RoPE / KV-write epilogue
       K8S_TRY(k8s_gemm_skinny_rope(s.y, H, s.wqkv[l], qkv, ld_qkv, T, ld_qkv, H, s.pos, s.cos_sin, s.slots, s.kc[l],
                                    s.vc[l], s.nq, s.nkv, s.BS, st));
@@ -321,9 +344,14 @@ K8S_API int k8s_llama_layers(const K8sLlamaStep* sp, hipStream_t st) {
       K8S_TRY(k8s_ar_allreduce_bf16(s.ar_id, s.obuf, s.obuf, n_out, s.ar_mode, st));
     if (nf_gu) {  // post-attention norm + gate_up + SwiGLU in one launch
       const bool dp = deferred(s.sel[1], true);
-      K8S_TRY(k8s_gemm_stream_silu_norm(dp ? nullptr : s.obuf, H, dp ? (const float*)part_of(s, s.sel[1]) : nullptr,
-                                        s.sel[1].splits, rc, ro, s.post_norm[l], s.eps, s.wgu[l], s.act, s.I, T, s.I,
-                                        H, s.sel[2].cfg, st));
+      const float* part = dp ? (const float*)part_of(s, s.sel[1]) : nullptr;
+      if (s.sel[2].kind == 6)
+        K8S_TRY(k8s_gemm_rows_norm(dp ? nullptr : s.obuf, H, part, s.sel[1].splits, rc, ro, s.post_norm[l], s.eps, s.wgu[l],
+                                   s.act, s.I, T, s.I, H, s.sel[2].cfg, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0,
+                                   st));
+      else
+        K8S_TRY(k8s_gemm_stream_silu_norm(dp ? nullptr : s.obuf, H, part, s.sel[1].splits, rc, ro, s.post_norm[l], s.eps,
+                                          s.wgu[l], s.act, s.I, T, s.I, H, s.sel[2].cfg, st));
       void* t = rc;
       rc = ro;
       ro = t;
@@ -337,6 +365,8 @@ K8S_API int k8s_llama_layers(const K8sLlamaStep* sp, hipStream_t st) {
       // gate_up done above
     } else if (s.sel[2].fuse == 2 && s.sel[2].kind == 5) {  // gate_up + SwiGLU in one launch: gu is never written
       K8S_TRY(k8s_gemm_big(s.y, H, s.wgu[l], s.act, s.I, T, s.I, H, 1, s.sel[2].cfg, st));
+    } else if (s.sel[2].fuse == 2 && s.sel[2].kind == 6) {
+      K8S_TRY(k8s_gemm_rows(s.y, H, s.wgu[l], s.act, s.I, T, s.I, H, s.sel[2].cfg, 1, 2, st));
     } else if (s.sel[2].fuse == 2 && s.sel[2].kind == 4) {
       K8S_TRY(k8s_gemm_stream_silu(s.y, H, s.wgu[l], s.act, s.I, T, s.I, H, s.sel[2].cfg, st));
     } else {

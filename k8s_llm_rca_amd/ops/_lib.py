@@ -37,6 +37,10 @@ _SIGS = {
     "k8s_attn_prefill": [P, I, P, P, P, I, P, P, P, P, P, P, P, P, I, P, P, P, P, I, P, P, I, I, I, F, P, I, P],
     "k8s_sample": [P, I, I, I, I, P, P, P, P, P, I, P, P, P, P, P, P, I, P, P, P, I],
     "k8s_gemm_skinny": [P, I, P, P, I, I, I, I, P],
+    "k8s_gemm_rows": [P, I, P, P, I, I, I, I, I, I, I, P],
+    "k8s_gemm_stream_reduce": [P, I, P, I, I, I, P],
+    "k8s_gemm_rows_rope": [P, I, P, P, I, I, I, I, I, P, P, P, P, P, I, I, I, P],
+    "k8s_gemm_rows_norm": [P, I, P, I, P, P, P, F, P, P, I, I, I, I, I, P, P, P, P, P, I, I, I, P],
     "k8s_gemm_skinny_f32": [P, I, P, P, I, I, I, I, P],
     "k8s_few_rows_f32": [P, I, P, P, I, I, I, P],
     "k8s_gemm_skinny_rope": [P, I, P, P, I, I, I, I, P, P, P, P, P, I, I, I, P],

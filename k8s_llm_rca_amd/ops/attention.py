@@ -96,6 +96,11 @@ def skinny_rope_ok(M: int, N: int, K: int, nq: int, nkv: int) -> bool:
     return _skinny_rope and 0 < M <= 16 and K % 256 == 0 and N == (nq + 2 * nkv) * HEAD_DIM
 
 
+def rows_rope_ok(N: int, nq: int, nkv: int) -> bool:
+    """The row-streaming kernel's rotating form takes the qkv projection (heads of 128, whole)."""
+    return _skinny_rope and N == (nq + 2 * nkv) * HEAD_DIM
+
+
 def linear_rope_kv(y: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, cos_sin: torch.Tensor,
                    slots: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: torch.Tensor, nq: int,
                    nkv: int) -> torch.Tensor:
@@ -109,7 +114,7 @@ def linear_rope_kv(y: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, co
     N = w.shape[0]
     if _fuse_qkv and use_hip(y) and y.dtype == torch.bfloat16 and slots is not None:
         layout = y.stride(1) == 1 and y.stride(0) % 8 == 0 and w.is_contiguous()
-        kind, cfg, splits = LIN.select_gemm(M, N, K, layout, True)
+        kind, cfg, splits = LIN.select_gemm(M, N, K, layout, True, LIN.rows_ok(y, w))
         if kind == LIN.KIND_SKINNY and layout and skinny_rope_ok(M, N, K, nq, nkv):
             qkv = torch.empty((M, N), dtype=y.dtype, device=y.device)
             BS = k_cache.shape[2]
@@ -117,16 +122,26 @@ def linear_rope_kv(y: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, co
                                              ptr(cos_sin), ptr(slots), ptr(k_cache), ptr(v_cache), nq, nkv, BS,
                                              stream_ptr(y)), "gemm_skinny_rope")
             return qkv
+        if kind == LIN.KIND_ROWS and splits == 1 and LIN.rows_ok(y, w) and rows_rope_ok(N, nq, nkv):
+            qkv = torch.empty((M, N), dtype=y.dtype, device=y.device)
+            check(lib().k8s_gemm_rows_rope(ptr(y), y.stride(0), ptr(w), ptr(qkv), N, M, N, K, cfg, ptr(positions),
+                                           ptr(cos_sin), ptr(slots), ptr(k_cache), ptr(v_cache), nq, nkv, k_cache.shape[2],
+                                           stream_ptr(y)), "gemm_rows_rope")
+            return qkv
         if layout and N == (nq + 2 * nkv) * HEAD_DIM and LIN.rope_choice(M, N, K):
             # the prefill-size qkv GEMM with RoPE + the paged KV write in its epilogue
             return LIN.gemm_big_rope(y, w, positions, cos_sin, slots, k_cache, v_cache, nq, nkv)
-        if kind in (LIN.KIND_STREAM, LIN.KIND_MID, LIN.KIND_BIG) and splits > 1:
+        if kind in (LIN.KIND_STREAM, LIN.KIND_MID, LIN.KIND_BIG, LIN.KIND_ROWS) and splits > 1:
             qkv = torch.empty((M, N), dtype=y.dtype, device=y.device)
             part = LIN._scratch(y.device, splits * M * N)
-            fn = {LIN.KIND_STREAM: lib().k8s_gemm_stream_part, LIN.KIND_MID: lib().k8s_gemm_mid_part,
-                  LIN.KIND_BIG: lib().k8s_gemm_big_part}[kind]
-            check(fn(ptr(y), y.stride(0), ptr(w), ptr(qkv), N, M, N, K, cfg, splits, ptr(part), stream_ptr(y)),
-                  "qkv gemm (split-K partials)")
+            if kind == LIN.KIND_ROWS:
+                check(lib().k8s_gemm_rows(ptr(y), y.stride(0), ptr(w), ptr(part), N, M, N, K, cfg, splits, LIN.ROWS_F32,
+                                          stream_ptr(y)), "qkv gemm (K ranges)")
+            else:
+                fn = {LIN.KIND_STREAM: lib().k8s_gemm_stream_part, LIN.KIND_MID: lib().k8s_gemm_mid_part,
+                      LIN.KIND_BIG: lib().k8s_gemm_big_part}[kind]
+                check(fn(ptr(y), y.stride(0), ptr(w), ptr(qkv), N, M, N, K, cfg, splits, ptr(part), stream_ptr(y)),
+                      "qkv gemm (split-K partials)")
             BS = k_cache.shape[2]
             assert positions.dtype == torch.int32 and cos_sin.dtype == torch.float32 and slots.dtype == torch.int32
             assert k_cache.shape[1] == nkv and v_cache.shape[2] == HEAD_DIM and v_cache.shape[3] == BS

@@ -68,6 +68,7 @@ _fuse_splitk = KNOBS.fuse_splitk
 # (csrc/kernels/norm_prologue.h; bit-identical, two launches fewer per layer)
 _norm_fuse = KNOBS.norm_fuse
 NORM_FUSE_MAX_T = 4
+NORM_FUSE_MAX_H = 4096      # norm_prologue.h: 256 threads, two 16-byte pieces each
 # (Round 3 also carried a row-chunked o / down GEMM with each chunk's
 # all-reduce on a side stream, and the prefill attention on a side stream beside
 # the decode attention: both measured as losses -- profiles/r3/ab/tp_overlap_*,
@@ -203,10 +204,12 @@ class LlamaExecutor:
             fuse = 2 if fused else int(_fuse_splitk)
             if i == 0 and kind == LIN.KIND_SKINNY and A.skinny_rope_ok(T, N, K, m.nq, m.nkv):
                 fuse = 3  # RoPE + KV write in the qkv GEMM's epilogue
+            elif i == 0 and kind == LIN.KIND_ROWS and splits == 1 and A.rows_rope_ok(N, m.nq, m.nkv):
+                fuse = 3
             elif i == 0 and N == (m.nq + 2 * m.nkv) * m.D and LIN.rope_choice(T, N, K):
                 kind, cfg, splits, fuse = LIN.KIND_BIG, LIN.BIG_PIPE, 1, 4  # gemm_big's RoPE + KV-write epilogue
             sels.append((kind, cfg, splits, fuse))
-            if kind in (LIN.KIND_MID, LIN.KIND_STREAM, LIN.KIND_BIG) and splits > 1:
+            if kind in (LIN.KIND_MID, LIN.KIND_STREAM, LIN.KIND_BIG, LIN.KIND_ROWS) and splits > 1:
                 need_mid = max(need_mid, splits * T * N)
             elif kind == LIN.KIND_GRP:
                 need_grp = max(need_grp, splits * T * N if splits > 1 else 1)
@@ -273,10 +276,11 @@ class LlamaExecutor:
             st.grp_offs = LIN.grp_offsets(dev, T).data_ptr()
         # fused norms (TP = 1): mirrors llama_exec.hip's nf_qkv / nf_gu conditions
         nf = 0
-        if _norm_fuse and self._car is None and m.nf_flags is None and T <= NORM_FUSE_MAX_T:
-            if st.sel[0].kind == LIN.KIND_SKINNY and st.sel[0].fuse == 3:
+        if _norm_fuse and self._car is None and m.nf_flags is None and T <= NORM_FUSE_MAX_T and H <= NORM_FUSE_MAX_H:
+            if st.sel[0].kind in (LIN.KIND_SKINNY, LIN.KIND_ROWS) and st.sel[0].fuse == 3:
                 nf |= 1
-            if st.sel[2].kind == LIN.KIND_STREAM and st.sel[2].fuse == 2 and st.sel[2].cfg in (4, 8):
+            if st.sel[2].fuse == 2 and (st.sel[2].kind == LIN.KIND_ROWS
+                                        or st.sel[2].kind == LIN.KIND_STREAM and st.sel[2].cfg in (4, 8)):
                 nf |= 2
         st.norm_fuse = nf
         res2 = scratch((T, H), dt, dev) if nf else None

@@ -28,15 +28,89 @@ def set_skinny(enabled: bool) -> None:
     _enabled = enabled
 
 
-KIND_LIB, KIND_SKINNY, KIND_MID, KIND_GRP, KIND_STREAM, KIND_BIG = 0, 1, 2, 3, 4, 5
+KIND_LIB, KIND_SKINNY, KIND_MID, KIND_GRP, KIND_STREAM, KIND_BIG, KIND_ROWS = 0, 1, 2, 3, 4, 5, 6
+
+# -------------------------------------------------- products of up to 32 rows (csrc/kernels/gemm_rows.hip)
+ROWS_MAX_M = 32
+ROWS_BF16, ROWS_F32, ROWS_SILU, ROWS_RELU2 = 0, 1, 2, 3
 
 
-def select_gemm(M: int, N: int, K: int, x_ok_layout: bool = True, out_contig: bool = True) -> Tuple[int, int, int]:
+def rows_shape_ok(M: int, N: int, K: int, nf: int, ranges: int, out: int = ROWS_F32) -> bool:
+    """What csrc/kernels/gemm_rows.hip accepts; ``N``: result columns."""
+    return (0 < M <= ROWS_MAX_M and nf in ((1, 2, 4) if M <= 16 else (2, 4)) and N > 0 and K > 0
+            and N % ((8 if out == ROWS_SILU else 16) * nf) == 0 and ranges >= 1 and (ranges == 1 or out == ROWS_F32)
+            and K % (4 * ranges * (64 if nf == 4 or M > 16 else 128)) == 0)
+
+
+@functools.lru_cache(maxsize=4096)
+def rows_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = False):
+    """(16-row fragments of a workgroup, K ranges) with which the row-streaming kernel takes a product, or None: another
+    kernel is the quicker one or the shape does not fit.  ``N``: result columns; ``planes``: K ranges may stay apart.
+
+    Up to 16 rows it is the quickest at all sizes from 128 x 512 to 128256 x 4096, at 0.53 to 0.97 of the time before with
+    cold weights, but for one row of a K of 8192 (bf16 of 4096 / 8192 / 16384 columns 14.4 / 26.6 / 49.8 us before, 15.1 /
+    29.0 / 56.6), which the skinny kernel keeps.  Up to 32 rows X is half of what it reads: from 8192 columns on (us at 32
+    rows before / this: 8192 x 2048 10.3 / 9.0, 16384 x 4096 42.0 / 26.9; 4096 x 2048 9.2 / 10.0 in fp32, 4096 x 8192 20.8 /
+    26.8), and of these not where K is 1536 or 3072, at which the library is at its best (28672 x 3072 46.2 / 49.6); planes
+    up to a K of 2048 (2048 x 2048 with the pass behind 0.93, 2560 x 4096 1.10, 1088 x 8192 1.06 of the time before).
+
+    The fragments and ranges are those of the least work on the busiest compute unit: a workgroup streams 16 nf x K / ranges
+    weights and X of M rows (2.5 % of a fragment's time each row), and 256 of them run at once.  Four fragments, whose loads
+    cover 128 bytes of a row instead of 256, cost a tenth more.  Over the measured sizes this is within 0.6 % of the best
+    choice on average.  K is cut only where one fragment a workgroup would leave more than a quarter of the compute units
+    idle, and not for a K of up to 1024 (2048 x 1024 whole / cut 5.1 / 5.0 us with the pass behind)."""
+    big = N * (2 if out == ROWS_SILU else 1)
+    if not 0 < M <= ROWS_MAX_M or big < 128 or K < 512:
+        return None
+    if M > 16 and not ((K <= 1024 or K % 2048 == 0) and (K <= 2048 if planes else big >= 8192)):
+        return None
+    if M == 1 and K == 8192 and out != ROWS_F32:
+        return None
+    strips = -(-big // (16 if M <= 16 else 32))
+    cut = planes and (K > 1024 or M > 16) and 4 * strips < 3 * 256 * -(-strips // 256)
+    best = None
+    for nf in (1, 2, 4):
+        for ranges in (1, 2, 4, 8) if cut else (1,):
+            if not rows_shape_ok(M, N, K, nf, ranges, out):
+                continue
+            wgs = big // (16 * nf) * ranges
+            waves = -(-wgs // 256) if wgs <= 6 * 256 else wgs / 256
+            cost = (waves * (nf * K / ranges * (1 + 0.025 * M / nf) * (1.1 if nf == 4 else 1) + 50)
+                    + (ranges * M * N / 512 if planes else 0))
+            if best is None or cost < best[0]:
+                best = cost, nf, ranges
+    return best and best[1:]
+
+
+def rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Layout and alignment the row-streaming kernel needs (16-byte loads of both)."""
+    return (x.is_cuda and x.dtype == torch.bfloat16 == w.dtype and x.shape[1] == w.shape[1] and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and w.is_contiguous() and x.data_ptr() % 16 == 0 == w.data_ptr() % 16)
+
+
+def gemm_rows(x: torch.Tensor, w: torch.Tensor, nf: int, out_kind: int = ROWS_BF16, ranges: int = 1,
+              out: torch.Tensor = None) -> torch.Tensor:
+    """``x @ w.T`` of up to 32 rows on the row-streaming kernel: bf16, fp32 (with ``ranges`` as planes [ranges, M, N]),
+    SwiGLU (w = [Wg; Wu]) or squared relu."""
+    M, K = x.shape
+    N = w.shape[0] // (2 if out_kind == ROWS_SILU else 1)
+    if out is None:
+        out = torch.empty((ranges, M, N) if ranges > 1 else (M, N), device=x.device,
+                          dtype=torch.float32 if out_kind == ROWS_F32 else x.dtype)
+    check(lib().k8s_gemm_rows(ptr(x), x.stride(0), ptr(w), ptr(out), out.stride(-2), M, N, K, nf, ranges, out_kind,
+                              stream_ptr(x)), "gemm_rows")
+    return out
+
+
+def select_gemm(M: int, N: int, K: int, x_ok_layout: bool = True, out_contig: bool = True,
+                rows: bool = True) -> Tuple[int, int, int]:
     """(kind, cfg, splits) :func:`linear` runs for a contiguous bf16 ``x`` [M, K]
     and ``w`` [N, K] on the GPU -- the measured dispatch table first, then the
-    skinny kernel's default range, else hipBLASLt.  Also used by the native
-    layer executor (ops/layer_exec.py) so both paths pick the same kernel."""
+    row-streaming kernel and the skinny kernel's default range, else hipBLASLt.  Also used by the native
+    layer executor (ops/layer_exec.py) so both paths pick the same kernel.
+    ``rows``: x and w lie as the row-streaming kernel needs them."""
     forced_skinny = False
+    rows = rows and x_ok_layout
     if _dispatch and M <= DISPATCH_MAX_M:
         ent = _lookup(N, K, M)
         if ent is not None:
@@ -47,6 +121,8 @@ def select_gemm(M: int, N: int, K: int, x_ok_layout: bool = True, out_contig: bo
                 return KIND_GRP, 0, splits
             if kind == "stream" and x_ok_layout and out_contig and stream_shape_ok(M, N, K, cfg, splits):
                 return KIND_STREAM, cfg, splits
+            if kind == "rows" and rows and rows_shape_ok(M, N, K, cfg, splits):
+                return KIND_ROWS, cfg, splits
             if kind == "lib":
                 return KIND_LIB, 0, 1
             forced_skinny = kind == "skinny" and M <= 128
@@ -54,6 +130,10 @@ def select_gemm(M: int, N: int, K: int, x_ok_layout: bool = True, out_contig: bo
         big_splits = _big_pick(M, N, K)
         if big_splits:
             return KIND_BIG, BIG_PIPE, big_splits
+    if rows and not forced_skinny:
+        plan = rows_plan(M, N, K)
+        if plan is not None:
+            return KIND_ROWS, plan[0], 1
     if (_enabled and (M == 1 or forced_skinny or (M <= SKINNY_MAX_M and N * K <= SKINNY_MAX_NK))
             and x_ok_layout and K % 256 == 0 and N % 16 == 0):
         return KIND_SKINNY, 0, 1
@@ -89,7 +169,17 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torch.
             return out
         return lib_gemm(x, w, out)
     layout = x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
-    kind, cfg, splits = select_gemm(M, N, K, layout, out is None or out.is_contiguous())
+    kind, cfg, splits = select_gemm(M, N, K, layout, out is None or out.is_contiguous(), rows_ok(x, w) and (out is None or out.stride(1) == 1))
+    if kind == KIND_ROWS:
+        if splits == 1:
+            return gemm_rows(x, w, cfg, out=out)
+        part = _scratch(x.device, splits * M * N)
+        check(lib().k8s_gemm_rows(ptr(x), x.stride(0), ptr(w), ptr(part), N, M, N, K, cfg, splits, ROWS_F32, stream_ptr(x)),
+              "gemm_rows")
+        if out is None:
+            out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        check(lib().k8s_gemm_stream_reduce(ptr(part), splits, ptr(out), out.stride(0), M, N, stream_ptr(x)), "gemm_reduce")
+        return out
     if kind == KIND_MID:
         return gemm_mid(x, w, cfg, splits, out)
     if kind == KIND_GRP:
@@ -144,6 +234,9 @@ def linear_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             and w.is_contiguous():
         M, K = x.shape
         N = w.shape[0]
+        plan = rows_plan(M, N, K, ROWS_F32) if rows_ok(x, w) else None
+        if plan is not None:
+            return gemm_rows(x, w, plan[0], ROWS_F32)
         out = torch.empty((M, N), dtype=torch.float32, device=x.device)
         if M == 0:  # a step whose chunks all end mid-prompt samples no row
             return out
@@ -177,6 +270,9 @@ def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return linear(x, w)
     M, K = x.shape
     N = w.shape[0]
+    plan = rows_plan(M, N, K, ROWS_F32) if rows_ok(x, w) else None
+    if plan is not None:
+        return gemm_rows(x, w, plan[0], ROWS_F32)
     if (_skinny_f32(M, N, K) and x.stride(1) == 1 and x.stride(0) % 8 == 0
             and w.dtype == torch.bfloat16 and w.is_contiguous()):
         out = torch.empty((M, N), dtype=torch.float32, device=x.device)
@@ -200,7 +296,8 @@ def _narrow_cfg(M: int) -> int:
 
 
 def plane_plan(M: int, N: int, K: int):
-    """(stream configuration, K ranges) of :func:`proj_planes`; one range: the product is not cut.  2048 columns are 32 or
+    """(stream configuration, K ranges) of :func:`proj_planes`, (ROWS_CFG + fragments, K ranges) where the row-streaming kernel
+    takes it; one range: the product is not cut.  The other forms: 2048 columns are 32 or
     64 strips for 256 compute units, so K is cut until each has a workgroup: four ranges of 32-column strips where K is
     short, eight of 64-column strips from 4096 on.  us with cold weights at 1 / 16 / 64 / 128 rows: 2048 x 2048 hipBLASLt
     8.1 / 8.3 / 8.9 / 8.8, the skinny kernel 4.9 / 6.2 / 11.7 / --, 64-column planes 4.2 / 4.5 / 5.5 / 7.2, 32-column
@@ -213,7 +310,13 @@ def plane_plan(M: int, N: int, K: int):
     6.4, 7.7 / 6.8;  2048 x 1024 5.7 / 6.1, 6.8 / 6.4;  4096 x 1024 6.2 / 7.6, 7.3 / 7.9, x 3072 10.6 / 13.3, 12.0 / 12.5, x
     6144 16.0 / 15.3, 18.6 / 15.5, x 8192 18.8 / 22.7, 22.1 / 22.5;  5120 x 1024 7.2 / 8.5, 9.2 / 9.0, x 2048 10.5 / 10.9,
     13.3 / 11.7;  2048 x 256 at 24 rows 5.6 / 6.1."""
+    plan = rows_plan(M, N, K, ROWS_F32, True)
+    if plan is not None:
+        return ROWS_CFG + plan[0], plan[1]
     return _plane_plan(M, N, K, _enabled) if 0 < M <= NARROW_MAX_M else (14, 1)
+
+
+ROWS_CFG = 100      # past every stream configuration
 
 
 @functools.lru_cache(maxsize=4096)      # (asked for every product of a step; 1.2 us of the host worked out, 0.2 looked up)
@@ -235,6 +338,10 @@ def proj_planes(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     N = w.shape[0]
     if _few_ok(x, w):
         cfg, S = plane_plan(M, N, K)
+        if cfg > ROWS_CFG and K == w.shape[1]:
+            return gemm_rows(x, w, cfg - ROWS_CFG, ROWS_F32, S).view(S, M, N)
+        if cfg > ROWS_CFG:
+            cfg, S = _plane_plan(M, N, K, _enabled)
         if S > 1:
             out = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
             check(lib().k8s_gemm_stream_part(ptr(x), x.stride(0), ptr(w), None, N, M, N, K, cfg, S, ptr(out),
@@ -281,7 +388,7 @@ def proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     M, K = x.shape
     N = w.shape[0]
     if (16 < M <= NARROW_MAX_M and 32 <= N <= 32 * NARROW_WGS and K <= 2048 and (N, K) not in _dispatch and _few_ok(x, w)
-            and (K < 1536 or N > 2048 or M <= 64 and N * K >= 9 << 18) and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
+            and rows_plan(M, N, K) is None and (K < 1536 or N > 2048 or M <= 64 and N * K >= 9 << 18) and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
         return gemm_stream(x, w, _narrow_cfg(M), 1)
     return linear(x, w)
 
@@ -319,6 +426,9 @@ def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     M, K = x.shape
     N = w.shape[0]
     if _few_ok(x, w):
+        plan = rows_plan(M, N, K, ROWS_RELU2) if K == w.shape[1] else None
+        if plan is not None:
+            return gemm_rows(x, w, plan[0], ROWS_RELU2)
         skinny = N <= 4096 and K > 512 and M <= (8 if K <= 1536 else 16)
         if (0 < M <= NARROW_MAX_M and N <= 32 * NARROW_WGS and K <= 2048 and not skinny
                 and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
@@ -344,6 +454,9 @@ def glu_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     M, K = x.shape
     I = w.shape[0] // 2
     if _few_ok(x, w):
+        plan = rows_plan(M, I, K, ROWS_SILU) if w.shape == (2 * I, K) else None
+        if plan is not None:
+            return gemm_rows(x, w, plan[0], ROWS_SILU)
         if 0 < M <= NARROW_MAX_M:
             if I <= 16 * NARROW_WGS:
                 cfg = _narrow_cfg(M) if K <= 2048 and (M > 16 or I > 3072 or K <= 512) else 0
@@ -709,6 +822,8 @@ def swiglu_choice(M: int, N2: int, K: int):
         kind, cfg, splits = select_gemm(M, N2, K)
         if kind == KIND_STREAM and splits == 1:
             return KIND_STREAM, cfg, 1
+        if kind == KIND_ROWS and splits == 1 and (N2, K) in _dispatch and rows_shape_ok(M, N2 // 2, K, cfg, 1, ROWS_SILU):
+            return KIND_ROWS, cfg, 1
     return None
 
 
@@ -736,6 +851,8 @@ def swiglu_gemm(y: torch.Tensor, w_gu: torch.Tensor):
         return None
     if ch[0] == KIND_BIG:
         return gemm_big(y, w_gu, silu=True, pipe=ch[1])
+    if ch[0] == KIND_ROWS:
+        return gemm_rows(y, w_gu, ch[1], ROWS_SILU)
     return gemm_stream_silu(y, w_gu, ch[1])
 
 
@@ -882,7 +999,7 @@ def reserve_dispatch_scratch(dev: torch.device) -> None:
     for key, rows in _dispatch.items():
         n = key[-2]
         for m, kind, _, splits in rows:
-            if kind in ("mid", "stream") and splits > 1:  # both use the gemm_mid partial buffer
+            if kind in ("mid", "stream", "rows") and splits > 1:  # all use the gemm_mid partial buffer
                 need_mid = max(need_mid, m * n * splits)
             elif kind == "grp" and splits > 1:
                 need_grp = max(need_grp, m * n * splits)

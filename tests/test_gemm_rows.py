@@ -1,0 +1,158 @@
+"""The row-streaming product (csrc/kernels/gemm_rows.hip) at the edges of its forms, and the rule that picks it."""
+import pytest
+import torch
+
+from k8s_llm_rca_amd.ops import attention as A
+from k8s_llm_rca_amd.ops import linear as L
+from k8s_llm_rca_amd.ops._lib import lib, ptr, stream_ptr
+
+BF = torch.bfloat16
+gpu = pytest.mark.gpu
+
+
+def operands(m, n, k):
+    g = torch.Generator().manual_seed(m * 7 + n + k)
+    return torch.randn(m, k, generator=g).to(BF).cuda(), (torch.randn(n, k, generator=g) * k ** -0.5).to(BF).cuda()
+
+
+#: K a wave's one chunk, two, three (odd) and seven; strips: one, and one short of and past what a card runs at once
+SHAPES = [(16, 512), (32, 1024), (64, 1536), (4080, 512), (4128, 512), (128, 3584), (256, 2048)]
+
+
+@gpu
+@pytest.mark.parametrize("n,k", SHAPES)
+@pytest.mark.parametrize("m", [1, 3, 4, 15, 16, 17, 31, 32])
+@pytest.mark.parametrize("nf", [1, 2, 4])
+def test_forms_against_float64(m, n, k, nf):
+    x, w = operands(m, n, k)
+    want = x.double() @ w.double().T
+    ran = 0
+    for ranges in (1, 2, 4):
+        if not L.rows_shape_ok(m, n, k, nf, ranges):
+            continue
+        ran += 1
+        buf = torch.full((ranges * m * n + 64,), 7.0, device="cuda")           # nothing is written behind the planes
+        y = buf[:ranges * m * n].view(ranges, m, n)
+        L.gemm_rows(x, w, nf, L.ROWS_F32, ranges, out=y)
+        # fp32 sums of K terms of size K^(-1/2), in chunks, waves and ranges
+        assert float((y.double().sum(0) - want).abs().max()) < 4e-6 * k ** 0.5
+        assert bool((buf[ranges * m * n:] == 7.0).all())
+    if not L.rows_shape_ok(m, n, k, nf, 1):
+        assert lib().k8s_gemm_rows(ptr(x), k, ptr(w), ptr(x), n, m, n, k, nf, 1, 0, stream_ptr(x)) != 0
+        return
+    ldy = n + 24
+    wide = torch.full((m, ldy), 7.0, device="cuda", dtype=BF)
+    y = L.gemm_rows(x, w, nf, out=wide[:, :n])
+    assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()) and bool((wide[:, n:] == 7.0).all())
+    r = L.gemm_rows(x, w, nf, L.ROWS_RELU2)
+    assert bool(((r.double() - want.clamp_min(0) ** 2).abs() <= 2.0 ** -8 * want.clamp_min(0) ** 2 + 1e-4).all())
+    if n % (16 * nf) == 0 and L.rows_shape_ok(m, n // 2, k, nf, 1, L.ROWS_SILU):
+        # the separate pass's rounding of gate and up: the same bits as from the plain form
+        g, u = y[:, :n // 2].float(), y[:, n // 2:].float()
+        a = L.gemm_rows(x, w, nf, L.ROWS_SILU).float()
+        assert torch.allclose(a, torch.nn.functional.silu(g) * u, rtol=2.0 ** -8, atol=1e-6)
+
+
+@gpu
+def test_rows_of_infinities_stay_by_themselves():
+    for m, nf in ((5, 1), (16, 2), (20, 4)):
+        x, w = operands(m, 256, 1024)
+        clean = L.gemm_rows(x, w, nf)
+        x[2, 100] = float("inf")
+        w2 = w.clone()
+        w2[7, 3] = float("nan")
+        y = L.gemm_rows(x, w2, nf)
+        keep = [i for i in range(m) if i != 2]
+        cols = [i for i in range(256) if i != 7]
+        assert torch.equal(y[keep][:, cols], clean[keep][:, cols])
+        assert bool(torch.isinf(y[2, cols]).all()) and bool(torch.isnan(y[:, 7]).all())
+
+
+@gpu
+@pytest.mark.parametrize("m,nf", [(1, 1), (3, 2), (16, 4), (17, 2), (32, 4)])
+@pytest.mark.parametrize("nq,nkv", [(32, 8), (3, 1)])
+def test_rotating_form_is_product_and_rope(m, nf, nq, nkv):
+    K, BS, NB = 1024, 64, 4
+    N = (nq + 2 * nkv) * 128
+    x, w = operands(m, N, K)
+    cs = A.rope_cos_sin(4096, 500000.0, device="cuda")
+    pos = torch.randint(0, 4000, (m,), device="cuda", dtype=torch.int32)
+    slots = torch.randperm(NB * BS, device="cuda")[:m].int()
+    if m > 1:
+        slots[1] = -1
+    kc, vc = torch.zeros(NB, nkv, BS, 128, device="cuda", dtype=BF), torch.zeros(NB, nkv, 128, BS, device="cuda", dtype=BF)
+    kc2, vc2 = kc.clone(), vc.clone()
+    ref = L.gemm_rows(x, w, nf)
+    A.rope_kv_write(ref, pos, cs, slots, kc, vc, nq, nkv)
+    out = torch.empty_like(ref)
+    assert lib().k8s_gemm_rows_rope(ptr(x), K, ptr(w), ptr(out), N, m, N, K, nf, ptr(pos), ptr(cs), ptr(slots), ptr(kc2),
+                                    ptr(vc2), nq, nkv, BS, stream_ptr(x)) == 0
+    assert torch.equal(out, ref) and torch.equal(kc2, kc) and torch.equal(vc2, vc)
+
+
+@gpu
+@pytest.mark.parametrize("m", [1, 3, 4])
+@pytest.mark.parametrize("mode", ["first", "add", "part"])
+@pytest.mark.parametrize("H,nf", [(512, 1), (1536, 2), (4096, 4)])
+def test_norm_in_front_is_norm_and_product(m, mode, H, nf):
+    I, eps, nq, nkv, BS = 512, 1e-5, 6, 1, 64
+    g = torch.Generator(device="cuda").manual_seed(m + H)
+    res, x = (torch.randn(m, H, device="cuda", generator=g).to(BF) for _ in range(2))
+    part = torch.randn(4, m, H, device="cuda", generator=g) * 0.5
+    nw = (torch.rand(H, device="cuda", generator=g) + 0.5).to(BF)
+    w = (torch.randn(2 * I, H, device="cuda", generator=g) * 0.02).to(BF)
+    y, r = torch.empty(m, H, device="cuda", dtype=BF), res.clone()
+    s = stream_ptr(x)
+    if mode == "part":
+        assert lib().k8s_splitk_addnorm(ptr(part), 4, ptr(r), ptr(nw), ptr(y), m, H, H, eps, s) == 0
+    else:
+        assert lib().k8s_rmsnorm(ptr(x), ptr(r) if mode == "add" else None, ptr(nw), ptr(y), m, H, H, H, eps, s) == 0
+    src = (ptr(x) if mode != "part" else None, H, ptr(part) if mode == "part" else None, 4,
+           ptr(res) if mode != "first" else None)
+    new = torch.full_like(res, float("nan"))
+    dst = ptr(new) if mode != "first" else None
+    act = torch.empty(m, I, device="cuda", dtype=BF)
+    assert lib().k8s_gemm_rows_norm(*src, dst, ptr(nw), eps, ptr(w), ptr(act), I, m, I, H, nf, None, None, None, None, None,
+                                    0, 0, 0, s) == 0
+    assert torch.equal(act, L.gemm_rows(y, w, nf, L.ROWS_SILU)) and (mode == "first" or torch.equal(new, r))
+    N = (nq + 2 * nkv) * 128
+    w = (torch.randn(N, H, device="cuda", generator=g) * 0.02).to(BF)
+    cs, pos = A.rope_cos_sin(64, 500000.0, device="cuda"), torch.arange(m, device="cuda", dtype=torch.int32)
+    pages = [torch.zeros(2, nkv, *d, device="cuda", dtype=BF) for d in ((BS, 128), (128, BS)) for _ in range(2)]
+    outs = [torch.empty(m, N, device="cuda", dtype=BF) for _ in range(2)]
+    assert lib().k8s_gemm_rows_rope(ptr(y), H, ptr(w), ptr(outs[0]), N, m, N, H, nf, ptr(pos), ptr(cs), ptr(pos),
+                                    ptr(pages[0]), ptr(pages[2]), nq, nkv, BS, s) == 0
+    assert lib().k8s_gemm_rows_norm(*src, dst, ptr(nw), eps, ptr(w), ptr(outs[1]), N, m, N, H, nf, ptr(pos), ptr(cs), ptr(pos),
+                                    ptr(pages[1]), ptr(pages[3]), nq, nkv, BS, s) == 0
+    assert torch.equal(*outs) and torch.equal(*pages[:2]) and torch.equal(*pages[2:])
+
+
+def test_rule_gives_what_the_kernel_takes():
+    """Every plan fits the kernel; past its rows and sizes there is none."""
+    for out in (L.ROWS_BF16, L.ROWS_F32, L.ROWS_SILU, L.ROWS_RELU2):
+        for m in (0, 1, 7, 16, 17, 32, 33):
+            for n in (8, 16, 100, 128, 264, 1088, 2048, 2576, 5120, 8192, 28672, 128256):
+                for k in (256, 512, 768, 1024, 1536, 2048, 4096, 8192, 14336):
+                    for planes in ((False, True) if out == L.ROWS_F32 else (False,)):
+                        p = L.rows_plan(m, n, k, out, planes)
+                        assert p is None or L.rows_shape_ok(m, n, k, p[0], p[1], out), (out, m, n, k, p)
+                        if m in (0, 33) or k < 512 or n % 8:
+                            assert p is None
+    assert L.rows_plan(1, 2048, 2048, L.ROWS_F32, True)[1] > 1 == L.rows_plan(1, 4096, 4096, L.ROWS_F32, True)[1]
+    assert L.rows_plan(1, 8192, 8192) is None and L.rows_plan(24, 4096, 4096) is None and L.rows_plan(24, 8192, 2048)
+
+
+@gpu
+def test_operands_the_kernel_cannot_read_go_elsewhere():
+    """Rows that do not start on 16 bytes, a transposed weight: the same values as before, by another kernel."""
+    x, w = operands(5, 512, 1024)
+    want = x.double() @ w.double().T
+    odd = torch.empty(5, 1032, device="cuda", dtype=BF)[:, 4:1028]
+    odd.copy_(x)
+    flat = torch.empty(512 * 1024 + 4, device="cuda", dtype=BF)[4:].view(512, 1024)
+    flat.copy_(w)
+    for a, b in ((odd, w), (x, flat), (x, w.t().contiguous().t())):
+        assert not L.rows_ok(a, b)
+        for f in (L.linear, L.proj):
+            assert bool(((f(a, b).double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
+        assert float((L.proj_planes(a, b).double().sum(0) - want).abs().max()) < 4e-6 * 32
