@@ -132,6 +132,28 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// The sums over the wave of V values a lane (V a power of two up to 64), halving the values with the distance; lane l is left
+// with the sum of value l / (64 / V).  V - 1 + 6 - log2 V exchanges instead of 6 V.
+template <int V, int O = 32>
+__device__ __forceinline__ float wave_sums(const float (&v)[V]) {
+  if constexpr (V == 1) {
+    float a = v[0];
+#pragma unroll
+    for (int o = O; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+    return a;
+  } else {
+    const bool up = threadIdx.x & O;
+    float h[V / 2];
+#pragma unroll
+    for (int i = 0; i < V / 2; ++i) {
+      const float a = v[i], b = v[i + V / 2];
+      const float other = up ? a : b, mine = up ? b : a;
+      h[i] = mine + __shfl_xor(other, O, 64);
+    }
+    return wave_sums<V / 2, O / 2>(h);
+  }
+}
+
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));

@@ -13,28 +13,6 @@ namespace k8s {
 
 constexpr int kFewN = 4;       // rows of w per workgroup
 
-// The sums over the wave of V values a lane (V a power of two up to 64), halving the values with the distance; lane l is left
-// with the sum of value l / (64 / V).  V - 1 + 6 - log2 V exchanges instead of 6 V.
-template <int V, int O = 32>
-__device__ __forceinline__ float wave_sums(const float (&v)[V]) {
-  if constexpr (V == 1) {
-    float a = v[0];
-#pragma unroll
-    for (int o = O; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
-    return a;
-  } else {
-    const bool up = threadIdx.x & O;
-    float h[V / 2];
-#pragma unroll
-    for (int i = 0; i < V / 2; ++i) {
-      const float a = v[i], b = v[i + V / 2];
-      const float other = up ? a : b, mine = up ? b : a;
-      h[i] = mine + __shfl_xor(other, O, 64);
-    }
-    return wave_sums<V / 2, O / 2>(h);
-  }
-}
-
 template <int M>
 __global__ void __launch_bounds__(256) few_rows_f32_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w,
                                                            float* __restrict__ y, int N, int K) {

@@ -30,8 +30,9 @@ from typing import Dict, List, Optional, Tuple
 import torch
 
 from ..ops import norm as N
+from ..ops import row_step as R
 from ..ops import seq_ops as S
-from ..ops.linear import glu_proj, proj, proj_add, proj_f32out, proj_planes
+from ..ops.linear import proj, proj_add, proj_f32out, proj_planes
 from ..parallel.groups import ParallelContext, single
 
 TAIL_ALIGN = 32     # the rotated key part of a latent cache row is filled up to a multiple of this
@@ -376,29 +377,29 @@ class FikeraxModel:
             tables[id(rope)] = S.rope_table(inp.positions, rope)
         return tables[id(rope)]
 
-    def _lightning(self, i: int, h: torch.Tensor, inp: S.SegStepInputs, state: torch.Tensor) -> torch.Tensor:
+    def _lightning(self, i: int, h, inp: S.SegStepInputs, state: torch.Tensor) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
         HV = c.heads * c.vdim
-        x = proj(h, L["w_in"])                                             # q | k | v | gate as activations
+        x = R.proj(h, L["w_in"])                                           # q | k | v | gate as activations
         return S.decay_layer(x, c.heads, c.dim, c.vdim, L["decay"], state, inp.seg, x[:, x.shape[1] - HV:], L["mem_norm"],
                              self.cfg.norm_eps, self.dtype)
 
-    def _attention(self, i: int, h: torch.Tensor, inp: S.SegStepInputs, tables, kc, vc, vt) -> torch.Tensor:
+    def _attention(self, i: int, h, inp: S.SegStepInputs, tables, kc, vc, vt) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
-        x = proj_planes(h, L["w_in"])
+        x = R.proj_planes(h, L["w_in"])
         q = S.attn_prep(x, L["b_in"], c.heads, c.kv_heads, c.dim, c.vdim, inp.positions, inp.slots, kc, vc, self.dtype,
                         norm="head", eps=self.cfg.norm_eps, rope=self.ropes[i], rope_cs=self._table(i, inp, tables), vt=vt)
         o = S.masked_attention(q, c.heads, c.kv_heads, c.dim, c.vdim, kc, vc, inp.seg, c.scale, window=c.window, vt=vt)
         return o
 
-    def _latent_attention(self, i: int, h: torch.Tensor, inp: S.SegStepInputs, tables, cache, cache_t) -> torch.Tensor:
+    def _latent_attention(self, i: int, h, inp: S.SegStepInputs, tables, cache, cache_t) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
-        T, H, D, R, V, KR = h.shape[0], c.heads, c.dim, c.rot_dim, c.vdim, c.kv_rank
+        T, H, D, V, KR = inp.input_ids.shape[0], c.heads, c.dim, c.vdim, c.kv_rank
         cs = self._table(i, inp, tables)
-        dn = proj_planes(h, L["w_in"])                                        # [., T, q_rank + KR + R] fp32
+        dn = R.proj_planes(h, L["w_in"])                                      # [., T, q_rank + KR + rot_dim] fp32
         cq = S.latent_norm(dn, L["dq_norm"], L["dkv_norm"], inp.slots, cache, c.q_rank, KR, self.cfg.norm_eps, self.dtype,
-                           cache_t=cache_t, tail=R, tail_cs=cs)
-        q = proj(cq, L["w_uq"])                                             # [T, H (D + R)]
+                           cache_t=cache_t, tail=c.rot_dim, tail_cs=cs)
+        q = proj(cq, L["w_uq"])                                             # [T, H (D + rot_dim)]
         qa, qr = S.latent_queries(q, L["uk"], cs, H, D, c.tail)               # [T, H, KR] head-major, [T, H, tail]
         kw = dict(window=c.window, sink=L["sink"], head_major=True)
         if cache_t is not None:
@@ -406,7 +407,7 @@ class FikeraxModel:
         else:
             o = S.latent_attention(qa.float(), cache, None, inp.seg, c.scale, self.dtype,
                                    qr=qr.float() if qr is not None else None, **kw)
-        ov = torch.empty(T, H, V, dtype=self.dtype, device=h.device)
+        ov = torch.empty(T, H, V, dtype=self.dtype, device=o.device)
         S.head_proj(o, L["uv_t"], ov)                                         # written token-major: W_o reads it as it is
         return ov.view(T, H * V)
 
@@ -426,12 +427,12 @@ class FikeraxModel:
         for r, (i, _) in enumerate(self.runs):
             spec, L, ci = cfg.layers[i], self.layers[i], self.cache_of[r]
             # the write-back of the run's last sublayer also reads the next run's input
-            into: dict = {}
+            nxt: Optional[dict] = None
             if r + 1 < len(self.runs):
                 j, add = self.runs[r + 1]
-                into = dict(inn=one, nw=self.layers[j]["norm1"], eps=eps, out_dtype=dt, again=again if add else None)
+                nxt = dict(nw=self.layers[j]["norm1"], again=again if add else None)
             elif inp.logits_idx is None:                   # every row is wanted: the last write-back reads the head's input
-                into = dict(inn=one, nw=self.final_norm, eps=eps, out_dtype=dt)
+                nxt = dict(nw=self.final_norm)
             rms = None                                     # what the residual's pass makes up for behind the projection
             if spec.kind == "lightning":
                 y, rms = self._lightning(i, h, inp, states[f"mem{self.state_of[r]}"])
@@ -439,26 +440,32 @@ class FikeraxModel:
                 y = self._attention(i, h, inp, tables, kcs[ci], vcs[ci], vts[ci])
             else:
                 y = self._latent_attention(i, h, inp, tables, kcs[ci], vts[ci])
+            x = R.residual(h, x)
             w = L["wo"]
             if spec.ff:
                 y = proj_add(x[:, 0], y, w) if rms is None else proj_planes(y, w)
                 h = (N.hyper_read(x, None, L["norm2"], eps, dt) if y is None
-                     else N.hyper_step(x, y, one, mix1, inn=one, nw=L["norm2"], eps=eps, out_dtype=dt, rms=rms))
-                y, w, rms = glu_proj(h, L["w13"]), L["w2"], None                 # silu(gate) * up
+                     else R.step(x, y, one, mix1, L["norm2"], eps, dt, rms=rms))
+                y, w, rms = R.glu_proj(h, L["w13"]), L["w2"], None               # silu(gate) * up
+                x = R.residual(h, x)
             # (a pass that reads the embedding once more adds the product too)
-            y = proj_planes(y, w) if into.get("again") or rms is not None else proj_add(x[:, 0], y, w)
-            if layers_out is not None and into.get("again"):   # the residual in front of the embedding added once more
-                before = x.clone()
-                N.hyper_step(before, y, one, mix1, rms=rms)
-            if y is not None:
-                h = N.hyper_step(x, y, one, mix1, rms=rms, **into)
-            elif into:
-                h = N.hyper_read(x, None, into["nw"], eps, dt)
-            if layers_out is not None:
-                layers_out.append(before[:, 0] if into.get("again") else x[:, 0].clone())
+            embeds = nxt is not None and nxt.get("again")
+            y = proj_planes(y, w) if embeds or rms is not None else proj_add(x[:, 0], y, w)
+            if layers_out is not None:                     # the residual in front of the embedding added once more
+                after = x.clone()
+                if y is not None:
+                    N.hyper_step(after, y, one, mix1, rms=rms)
+                layers_out.append(after[:, 0])
+            if y is None:
+                h = N.hyper_read(x, None, nxt["nw"], eps, dt) if nxt else None
+            elif nxt:
+                h = R.step(x, y, one, mix1, eps=eps, out_dtype=dt, rms=rms, **nxt)
+            else:
+                N.hyper_step(x, y, one, mix1, rms=rms)
         if inp.logits_idx is not None:
             h = N.hyper_read(x, inp.logits_idx, self.final_norm, eps, dt)
-        return proj_f32out(h, self.head)
+            return proj_f32out(h, self.head)
+        return R.proj_f32out(h, self.head)
 
 
 def random_tensors(cfg: FikeraxConfig, seed: int = 0, device="cpu") -> Dict[str, torch.Tensor]:

@@ -34,8 +34,9 @@ from typing import Dict, List, Optional, Tuple
 import torch
 
 from ..ops import norm as N
+from ..ops import row_step as R
 from ..ops import seq_ops as S
-from ..ops.linear import proj, proj_add, proj_f32out, relu_sq_proj
+from ..ops.linear import proj_add, proj_f32out
 from ..parallel.groups import ParallelContext, single
 
 
@@ -380,7 +381,7 @@ class LizesunModel:
         L, a = self.layers[li], self.cfg.layers[li].attn
         ci = self.cache_of[li]
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
-        x = proj_f32out(h, L["w_in"])                                  # [T, H D + G D + G V + H] fp32
+        x = R.proj_f32out(h, L["w_in"])                                # [T, H D + G D + G V + H] fp32
         keep = other = None
         if a.v_mix:
             if li == self.vmix_first:
@@ -400,7 +401,7 @@ class LizesunModel:
         ci, j = self.cache_of[li], self.mem_of[li]
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
         nl = H * D + G * (D + V)
-        x = proj_f32out(h, L["w_in"])                                  # left q | k | v, right q | k | v | g | i | f
+        x = R.proj_f32out(h, L["w_in"])                                # left q | k | v, right q | k | v | g | i | f
         key = (a.rot_dims, a.rot_base)
         rope = self.ropes.get(key)
         if rope is not None and key not in tables:                     # cos | sin of the step's positions, made once
@@ -417,9 +418,9 @@ class LizesunModel:
     def _delta(self, li: int, h, inp: S.SegStepInputs, states) -> torch.Tensor:
         L, c = self.layers[li], self.cfg.layers[li].delta
         j, ra, rg = self.delta_of[li], L["ra"], L["rg"]
-        qkv = proj(h, L["w_qkv"])                                    # [T, 2 G D + H V]
+        qkv = R.proj(h, L["w_qkv"], keep=True)                       # [T, 2 G D + H V]
         qkv = S.short_conv(qkv, L["conv_w"], None, states[f"dconv{j}"], inp.seg, act=True)
-        agb = proj_f32out(h, L["w_agb"])                               # [T, ra + rg + H] fp32
+        agb = R.proj_f32out(h, L["w_agb"])                             # [T, ra + rg + H] fp32
         # [T, H D] before bias and softplus, [T, H V] before the sigmoid, both fp32
         dec, gate = S.low_rank_pair(agb, 0, L["w_a2"], ra, L["w_g2"], self.dtype)
         return S.delta_layer(qkv, c.heads, c.kv_heads, c.dim, c.vdim, dec, L["rate"], L["dt_bias"], agb[:, ra + rg:],
@@ -445,23 +446,28 @@ class LizesunModel:
             after = L["norm2"] if spec.ff else nxt
             if spec.kind == "parallel":
                 ol, orr = self._parallel(li, h, inp, kcs, vcs, vts, states, tables)
+                x = R.residual(h, x)
                 yl = proj_add(x, ol, L["wo_l"], spec.left_scale)
                 yr = proj_add(x, orr, L["wo_r"], spec.right_scale)
                 add = (yl, spec.left_scale, yr, spec.right_scale) if yl is not None else (yr, spec.right_scale, None, 1.0)
-                h = N.add_dyt(x, *add, *after, out_dtype=dt)
+                h = R.dyt_step(x, *add, *after, out_dtype=dt)
             else:
                 o = (self._chunk_attention(li, h, inp, kcs, vcs, vts, vmix) if spec.kind == "attention"
                      else self._delta(li, h, inp, states))
-                h = N.add_dyt(x, proj_add(x, o, L["wo"]), 1.0, None, 1.0, *after, out_dtype=dt)
+                x = R.residual(h, x)
+                h = R.dyt_step(x, proj_add(x, o, L["wo"]), 1.0, None, 1.0, *after, out_dtype=dt)
             if spec.ff:
-                y = proj_add(x, relu_sq_proj(h, L["w_up"]), L["w_down"])
-                h = N.add_dyt(x, y, 1.0, None, 1.0, *nxt, out_dtype=dt)
+                u = R.relu_sq_proj(h, L["w_up"])
+                x = R.residual(h, x)
+                h = R.dyt_step(x, proj_add(x, u, L["w_down"]), 1.0, None, 1.0, *nxt, out_dtype=dt)
             if layers_out is not None:
+                if isinstance(h, R.RowStep):
+                    h = h.read()                                       # the residual as it is behind this layer
                 layers_out.append(x.clone())
         if inp.logits_idx is not None or not nl:
             xr = x.index_select(0, inp.logits_idx).contiguous() if inp.logits_idx is not None else x
             h = N.add_dyt(xr, None, 1.0, None, 1.0, *self.final_norm, out_dtype=dt)
-        return proj_f32out(h, self.lm_head)
+        return R.proj_f32out(h, self.lm_head)
 
 
 def random_tensors(cfg: LizesunConfig, seed: int = 0, device="cpu") -> Dict[str, torch.Tensor]:

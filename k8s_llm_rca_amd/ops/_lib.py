@@ -41,6 +41,8 @@ _SIGS = {
     "k8s_gemm_stream_reduce": [P, I, P, I, I, I, P],
     "k8s_gemm_rows_rope": [P, I, P, P, I, I, I, I, I, P, P, P, P, P, I, I, I, P],
     "k8s_gemm_rows_norm": [P, I, P, I, P, P, P, F, P, P, I, I, I, I, I, P, P, P, P, P, I, I, I, P],
+    "k8s_gemm_row_step_rms": [P, P, P, I, P, I, F, F, P, P, F, P, F, P, P, P, I, I, I, I, I, P],
+    "k8s_gemm_row_step_dyt": [P, P, P, I, F, P, I, F, F, P, P, P, P, P, I, I, I, I, I, P],
     "k8s_gemm_skinny_f32": [P, I, P, P, I, I, I, I, P],
     "k8s_few_rows_f32": [P, I, P, P, I, I, I, P],
     "k8s_gemm_skinny_rope": [P, I, P, P, I, I, I, I, P, P, P, P, P, I, I, I, P],

@@ -1,0 +1,154 @@
+"""A residual's pass that is not made yet, for the product that stands behind it (csrc/kernels/gemm_row_step.hip).
+
+With one row the pass (:func:`..ops.norm.hyper_step` with one stream, :func:`..ops.norm.add_dyt`) is a launch of 3 to 4 us
+in which the chip waits; the kernel makes the row in every workgroup of the product instead, under the weights' way from
+memory.  A model asks for its next sublayer's input with :func:`step` / :func:`dyt_step`, which return either the activations
+(the residual updated in place) or a :class:`RowStep`; the products below take both, and :func:`residual` says where the
+residual is afterwards."""
+from typing import Optional
+
+import torch
+
+from . import linear as L
+from . import norm as N
+from ._lib import check, lib, ptr, stream_ptr, use_hip
+
+MAX_K, COLS, PLANES, SUMS = 2048, 512, 4, 64     # what the kernel takes (kStepMaxK, kStepCols, kStepPlanes, kStepSums)
+
+
+def plan(n: int, k: int, out_kind: int, planes: bool = False):
+    """(16-row fragments a workgroup, K ranges) with which one row's product takes its residual pass in front, or None.
+    ``n``: result columns.  Wherever the row-streaming kernel takes one row and a wave can ask for its whole share at once;
+    the fragments of the least work on the busiest of 256 compute units, two where that is the same (us of one / two: 8192
+    SwiGLU 13.4 / 12.8, 8192 8.0 / 7.4, 32768 23.6 / 23.3, 8736 9.6 / 10.3, 2304 4.4 / 5.4).  K is cut in two only where half
+    of the units would stay idle (1088 columns whole / cut 4.0 / 3.7, 2560 4.5 / 5.2)."""
+    if (("silu", 2 * n, k) if out_kind == L.ROWS_SILU else (n, k)) in L.dispatch_table():
+        return None                              # another kernel was measured for this weight
+    if L.rows_plan(1, n, k, out_kind, planes) is None or k > MAX_K or k % COLS:
+        return None
+    half = out_kind == L.ROWS_SILU
+    fits = [nf for nf in (2, 1) if n % ((8 if half else 16) * nf) == 0]
+    if not fits:
+        return None
+    wgs = {nf: n // ((8 if half else 16) * nf) for nf in fits}
+    nf = min(fits, key=lambda f: -(-wgs[f] // 256) * f)
+    ranges = 2 if planes and wgs[nf] < 128 and k % (2 * COLS) == 0 else 1
+    return nf, ranges
+
+
+class RowStep:
+    """``x``: the fp32 residual [1, W], replaced by a new tensor when a product has made the pass; ``h``: its activations,
+    once somebody has them."""
+
+    def __init__(self, x: torch.Tensor, act: int, launch, read):
+        self.x, self.h, self._act, self._launch, self._read = x, None, act, launch, read
+
+    def read(self) -> torch.Tensor:
+        """The activations by the separate pass, the residual updated in place."""
+        if self.h is None:
+            if self._launch is None:
+                raise RuntimeError("the pass was made in front of a product that did not keep its activations")
+            self.h = self._read()
+        return self.h
+
+    def product(self, w: torch.Tensor, out_kind: int, plain, planes: bool = False, keep: bool = False):
+        """``plain(h, w)`` with the pass in front where the kernel takes it.  ``keep``: ``h`` is read again afterwards."""
+        n, k = w.shape[0] // (2 if out_kind == L.ROWS_SILU else 1), w.shape[1]
+        p = (plan(n, k, out_kind, planes) if self.h is None and self._launch is not None
+             and out_kind in (L.ROWS_BF16, L.ROWS_F32, self._act) else None)
+        if (p is None or w.dtype != torch.bfloat16 or not w.is_contiguous() or w.data_ptr() % 16 or k != self.x.shape[1]
+                or w.device != self.x.device or w.shape[0] % 2 and out_kind == L.ROWS_SILU):
+            return plain(self.read(), w)
+        out = torch.empty((p[1], 1, n) if planes else (1, n), device=w.device,
+                          dtype=torch.float32 if out_kind == L.ROWS_F32 else w.dtype)
+        x_out = torch.empty_like(self.x)
+        h = torch.empty(1, k, dtype=w.dtype, device=w.device) if keep else None
+        self._launch(x_out, h, w, out, n, k, p[0], p[1], out_kind)
+        self.x, self.h, self._launch = x_out, h, None
+        return out
+
+
+def residual(h, x: torch.Tensor) -> torch.Tensor:
+    """The residual behind a product of ``h``: ``x`` itself, or where the pass put it."""
+    return h.x.view(x.shape) if isinstance(h, RowStep) else x
+
+
+def _one_row(x: torch.Tensor, y: Optional[torch.Tensor], out_dtype) -> bool:
+    W = x.shape[-1]
+    return (use_hip(x) and x.shape[0] == 1 and x.numel() == W and COLS <= W <= MAX_K and W % COLS == 0 and y is not None
+            and out_dtype == torch.bfloat16 and x.dtype == torch.float32 and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and _planes_ok(y, W))
+
+
+def _planes_ok(y: torch.Tensor, W: int) -> bool:
+    return (y.dtype == torch.float32 and y.is_contiguous() and y.data_ptr() % 16 == 0 and y.shape[-2:] == (1, W)
+            and y.dim() <= 3 and y.numel() <= PLANES * W)
+
+
+def _fp32_row(t: torch.Tensor, W: int) -> bool:
+    return t.dtype == torch.float32 and t.is_contiguous() and t.numel() == W and t.data_ptr() % 16 == 0
+
+
+def step(x: torch.Tensor, y: torch.Tensor, one: torch.Tensor, mix: torch.Tensor, nw: torch.Tensor, eps: float, out_dtype,
+         again: Optional[tuple] = None, rms: Optional[tuple] = None):
+    """:func:`..ops.norm.hyper_step` on one stream that is only added to (``one``, ``mix``: ones; ``x`` [T, 1, W])."""
+    def read():
+        return N.hyper_step(x, y, one, mix, inn=one, nw=nw, eps=eps, out_dtype=out_dtype, again=again, rms=rms)
+
+    W = x.shape[-1]
+    ids, embed, escale = again if again is not None else (None, None, 0.0)
+    ss, width, reps = rms if rms is not None else (None, 1.0, 0.0)
+    if not (_one_row(x, y, out_dtype) and x.shape[1] == 1 and _fp32_row(nw, W)
+            and (ss is None or ss.dtype == torch.float32 and ss.is_contiguous() and ss.shape[0] == 1 and 0 < ss.numel() <= SUMS)
+            and (ids is None or ids.dtype == torch.int32 and ids.numel() == 1 and embed.dtype == out_dtype
+                 and embed.is_contiguous() and embed.shape[1] == W and embed.data_ptr() % 8 == 0)):
+        return read()
+
+    def launch(x_out, h, w, out, n, k, nf, ranges, kind):
+        check(lib().k8s_gemm_row_step_rms(ptr(x), ptr(x_out), ptr(y), y.shape[0] if y.dim() == 3 else 1, ptr(ss),
+                                          ss.numel() if ss is not None else 0, float(width), float(reps), ptr(ids), ptr(embed),
+                                          float(escale), ptr(nw), float(eps), ptr(h), ptr(w), ptr(out), n, k, nf, ranges, kind,
+                                          stream_ptr(x)), "gemm_row_step_rms")
+
+    return RowStep(x.view(1, W), L.ROWS_SILU, launch, read)
+
+
+def dyt_step(x: torch.Tensor, y: Optional[torch.Tensor], sy: float, y2: Optional[torch.Tensor], sy2: float, alpha: float,
+             w: Optional[torch.Tensor], b: Optional[torch.Tensor], out_dtype):
+    """:func:`..ops.norm.add_dyt`."""
+    def read():
+        return N.add_dyt(x, y, sy, y2, sy2, alpha, w, b, out_dtype=out_dtype)
+
+    W = x.shape[-1]
+    if not (w is not None and _one_row(x, y, out_dtype) and (y2 is None or _planes_ok(y2, W)) and _fp32_row(w, W)
+            and _fp32_row(b, W)):
+        return read()
+
+    def launch(x_out, h, wt, out, n, k, nf, ranges, kind):
+        yp, yp2 = (t.shape[0] if t is not None and t.dim() == 3 else 1 for t in (y, y2))
+        check(lib().k8s_gemm_row_step_dyt(ptr(x), ptr(x_out), ptr(y), yp, float(sy), ptr(y2), yp2, float(sy2), float(alpha),
+                                          ptr(w), ptr(b), ptr(h), ptr(wt), ptr(out), n, k, nf, ranges, kind, stream_ptr(x)),
+              "gemm_row_step_dyt")
+
+    return RowStep(x, L.ROWS_RELU2, launch, read)
+
+
+# ------------------------------------------------------------------------- products of activations, or of what makes them
+def proj(h, w: torch.Tensor, keep: bool = False) -> torch.Tensor:
+    return h.product(w, L.ROWS_BF16, L.proj, keep=keep) if isinstance(h, RowStep) else L.proj(h, w)
+
+
+def proj_f32out(h, w: torch.Tensor) -> torch.Tensor:
+    return h.product(w, L.ROWS_F32, L.proj_f32out) if isinstance(h, RowStep) else L.proj_f32out(h, w)
+
+
+def proj_planes(h, w: torch.Tensor) -> torch.Tensor:
+    return h.product(w, L.ROWS_F32, L.proj_planes, planes=True) if isinstance(h, RowStep) else L.proj_planes(h, w)
+
+
+def glu_proj(h, w: torch.Tensor) -> torch.Tensor:
+    return h.product(w, L.ROWS_SILU, L.glu_proj) if isinstance(h, RowStep) else L.glu_proj(h, w)
+
+
+def relu_sq_proj(h, w: torch.Tensor) -> torch.Tensor:
+    return h.product(w, L.ROWS_RELU2, L.relu_sq_proj) if isinstance(h, RowStep) else L.relu_sq_proj(h, w)
