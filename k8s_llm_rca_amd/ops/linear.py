@@ -206,6 +206,34 @@ _blaslt_ws = {}
 _native_lib_gemm = KNOBS.native_blaslt
 
 
+_lib_tuned: Dict[Tuple[int, int], List[Tuple[int, int]]] = {}    # rows (from, to) of weights with a measured solution
+
+
+def row_cut(M: int, N: int, K: int, tuned: bool = False) -> int:
+    """Rows of a library product that go into a launch of their own because their 256 x 256 tiles are whole waves of the 256
+    compute units (the rest follows in a second one), or 0.  For some tiles more than whole waves the library takes a wave
+    more, or smaller tiles for all of them.  us whole / cut:  2048 x 2048 added to fp32 at 17000 rows (2.09 waves) 172 / 150,
+    24730 (3.03) 246 / 218;  2048 x 8192 at 16500 641 / 434, 24730 743 / 639, but 20000 (2.47) 726 / 542 and 22000 (2.69)
+    765 / 579;  8192 x 2048 in bf16 at 2100 (1.12) 85 / 64, 12000 (5.88) 389 / 295, 24730 629 / 592, 3300 (1.62) 94 / 95;
+    2560 x 2048 at 27000 (4.14) 313 / 261, 22000 (3.36) 218 / 246;  4096 x 14336 at 4123 (1.06) 730 / 367.  So up to 0.15 of
+    a wave whatever the shape, further where the columns divide a wave and are many or K is long.  Over 92 random sizes of 18
+    weights 0.88 of the time (0.50 to 1.12, six of them past 1.02).  ``tuned``: a call that takes measured solutions, which
+    stay with the rows they were measured for."""
+    nt = -(-N // 256)
+    full, over = divmod(-(-M // 256) * nt, 256)
+    if full < 1 or not over or tuned and any(lo <= M <= hi for lo, hi in _lib_tuned.get((N, K), ())):
+        return 0
+    most = 0.15
+    if 256 % nt == 0 and N % 256 == 0 and (nt >= 32 or K >= 4096 and full > 1):
+        most = 1.0 if full > 1 else 0.5
+    return full * 256 // nt * 256 if over <= most * 256 else 0
+
+
+def _row_parts(M: int, N: int, K: int, tuned: bool = False) -> Tuple[Tuple[int, int], ...]:
+    cut = row_cut(M, N, K, tuned)
+    return ((0, cut), (cut, M)) if 0 < cut < M else ((0, M),)
+
+
 def lib_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
     """``x @ w.T`` on hipBLASLt (bf16, fp32 accumulate)."""
     if (_native_lib_gemm and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
@@ -219,8 +247,9 @@ def lib_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torc
         ws = _blaslt_ws.get(x.device)
         if ws is None:
             ws = _blaslt_ws[x.device] = torch.empty(BLASLT_WS_BYTES, dtype=torch.uint8, device=x.device)
-        check(lib().k8s_blaslt_gemm(ptr(x), x.stride(0), ptr(w), ptr(out), out.stride(0), M, N, K, ptr(ws),
-                                    BLASLT_WS_BYTES, stream_ptr(x)), "blaslt_gemm")
+        for a, b in _row_parts(M, N, K, True):
+            check(lib().k8s_blaslt_gemm(ptr(x[a:]), x.stride(0), ptr(w), ptr(out[a:]), out.stride(0), b - a, N, K, ptr(ws),
+                                        BLASLT_WS_BYTES, stream_ptr(x)), "blaslt_gemm")
         return out
     if out is None:
         return F.linear(x, w)
@@ -243,8 +272,9 @@ def linear_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         ws = _blaslt_ws.get(x.device)
         if ws is None:
             ws = _blaslt_ws[x.device] = torch.empty(BLASLT_WS_BYTES, dtype=torch.uint8, device=x.device)
-        check(lib().k8s_blaslt_gemm2(ptr(x), x.stride(0), ptr(w), ptr(out), N, M, N, K, ptr(ws), BLASLT_WS_BYTES,
-                                     stream_ptr(x), 1, 1.0), "blaslt_gemm_f32out")
+        for a, b in _row_parts(M, N, K):
+            check(lib().k8s_blaslt_gemm2(ptr(x[a:]), x.stride(0), ptr(w), ptr(out[a:]), N, b - a, N, K, ptr(ws),
+                                         BLASLT_WS_BYTES, stream_ptr(x), 1, 1.0), "blaslt_gemm_f32out")
         return out
     return x.float() @ w.float().t()
 
@@ -373,8 +403,9 @@ def proj_add(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, scale: float = 1
     ws = _blaslt_ws.get(x.device)
     if ws is None:
         ws = _blaslt_ws[x.device] = torch.empty(BLASLT_WS_BYTES, dtype=torch.uint8, device=x.device)
-    check(lib().k8s_blaslt_gemm2(ptr(x), x.stride(0), ptr(w), ptr(r), N, M, N, K, ptr(ws), BLASLT_WS_BYTES, stream_ptr(x), 2,
-                                 float(scale)), "blaslt_gemm_add")
+    for a, b in _row_parts(M, N, K):
+        check(lib().k8s_blaslt_gemm2(ptr(x[a:]), x.stride(0), ptr(w), ptr(r[a:]), N, b - a, N, K, ptr(ws), BLASLT_WS_BYTES,
+                                     stream_ptr(x), 2, float(scale)), "blaslt_gemm_add")
     return None
 
 
@@ -564,6 +595,7 @@ def load_lib_algos(path: str) -> int:
         N, K = (int(v) for v in key.split(","))
         for M, idx in sorted(ladder.items(), key=lambda kv: int(kv[0])):
             if lib().k8s_blaslt_set_algo(int(M), N, K, int(idx)) == 0:
+                _lib_tuned.setdefault((N, K), []).append((int(M), 1 << 30))
                 n += 1
     # bucketed form (tools/blaslt_tune_buckets.py): [lo, hi, solution] per (N, K),
     # each verified on the engine's own call path at the bucket's ends and middle
@@ -571,12 +603,14 @@ def load_lib_algos(path: str) -> int:
         N, K = (int(v) for v in key.split(","))
         for lo, hi, idx in rows:
             if lib().k8s_blaslt_set_algo_range(int(lo), int(hi), N, K, int(idx)) == 0:
+                _lib_tuned.setdefault((N, K), []).append((int(lo), int(hi)))
                 n += 1
     return n
 
 
 def clear_lib_tuning() -> None:
     lib().k8s_blaslt_clear_tuning()
+    _lib_tuned.clear()
 
 
 # ------------------------------------------------------- measured dispatch

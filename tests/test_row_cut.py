@@ -1,0 +1,44 @@
+"""Library products of which whole waves of tiles go into a launch of their own (ops/linear.py: row_cut)."""
+import pytest
+import torch
+
+from k8s_llm_rca_amd.ops import linear as L
+
+BF = torch.bfloat16
+
+
+def test_cut_is_whole_waves_of_tiles():
+    for n, k in [(2048, 2048), (2048, 8192), (8192, 2048), (2560, 2048), (8736, 2048), (3072, 768), (384, 384), (100, 64),
+                 (65536, 512), (70000, 512)]:
+        nt = -(-n // 256)
+        for m in list(range(1, 700, 37)) + [1024, 2047, 2049, 4123, 8192, 8193, 16500, 24576, 24730, 32768]:
+            cut = L.row_cut(m, n, k)
+            assert 0 <= cut < m and cut % 256 == 0
+            assert cut // 256 * nt <= -(-m // 256) * nt // 256 * 256          # no more tiles than the whole waves hold
+            parts = L._row_parts(m, n, k)
+            assert parts[0][0] == 0 and parts[-1][1] == m and all(a < b for a, b in parts)
+    assert L.row_cut(24730, 2048, 2048) == 24576 and L.row_cut(20000, 2048, 2048) == 0
+    assert L.row_cut(20000, 2048, 8192) == 16384 and L.row_cut(16384, 2048, 8192) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(2049, 8192, 512), (4100, 4096, 256), (8450, 2048, 384)])
+def test_cut_products_against_float64(m, n, k):
+    assert L.row_cut(m, n, k)
+    g = torch.Generator().manual_seed(m)
+    wide = torch.randn(m, k + 64, generator=g).to(BF).cuda()
+    x, w = wide[:, :k], (torch.randn(n, k, generator=g) * k ** -0.5).to(BF).cuda()      # rows apart
+    want = x.double() @ w.double().T
+    buf = torch.full((m + 1, n), 7.0, device="cuda")
+    y = L.linear_f32out(x, w)
+    assert float((y.double() - want).abs().max()) < 4e-6 * k ** 0.5                       # fp32 sums of K terms of K^(-1/2)
+    r = buf[:m]
+    old, L.ADD_ROWS = L.ADD_ROWS, 0
+    try:
+        assert L.proj_add(r, x, w, 0.5) is None
+    finally:
+        L.ADD_ROWS = old
+    assert float((r.double() - 7.0 - 0.5 * want).abs().max()) < 4e-6 * k ** 0.5 and bool((buf[m] == 7.0).all())
+    out = torch.full((m, n + 16), 3.0, device="cuda", dtype=BF)
+    b = L.lib_gemm(x, w, out[:, :n])
+    assert bool(((b.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()) and bool((out[:, n:] == 3.0).all())
