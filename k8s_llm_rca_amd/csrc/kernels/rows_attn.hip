@@ -19,7 +19,8 @@
 namespace k8s {
 
 constexpr int kRaKeys = 128;    // keys of a part
-constexpr int kRaHeads = 8;     // heads of a workgroup
+constexpr int kRaHeads = 8;     // heads of a workgroup that walks all parts
+constexpr int kRaFew = 2;       // of one that has a single part
 
 template <typename T>
 __device__ __forceinline__ float rld(const T* p, size_t i);
@@ -75,11 +76,15 @@ __device__ __forceinline__ void ra_join(float& m, float& l, float mp, float lp, 
 }
 __device__ __forceinline__ float ra_join_out(float o, float a, float op, float b) { return fmaf(o, a, __fmul_rn(op, b)); }
 
-template <typename TQ, typename TC, typename TO, bool VEC>
+// PART: a workgroup has one part (p.po).  Few of them run then, each a chain of latencies, so that all the registers are its
+// own: every value of the part is asked for before the scores, and 16 pieces of a key at a time instead of 4.  The sums are
+// those of the other form.
+template <typename TQ, typename TC, typename TO, bool VEC, bool PART>
 __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
+  constexpr int NH = PART ? kRaFew : kRaHeads;
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int D = p.D1 + p.D2, V = p.V, hpg = p.H / (p.G * p.M);
-  const int HB = min(hpg, kRaHeads), nhb = (hpg + HB - 1) / HB, nvb = (V + 255) / 256;
+  const int HB = min(hpg, NH), nhb = (hpg + HB - 1) / HB, nvb = (V + 255) / 256;
   float* sq = sm;                                   // [HB][D4]
   const int D4 = (D + 3) & ~3;
   float* sp = sq + HB * D4;                         // [HB][128]
@@ -94,7 +99,7 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
   auto head = [&](int i) { return (g * hpg + hb * HB + i) * p.M + gm % p.M; };
   const int sg = p.row_seg[r], pos = p.seg_pos0[sg] + r - p.seg_row0[sg];
   const KeyRuns kr = key_runs(pos, p.chunk, p.window, p.keep_first);
-  const int x_lo = p.po ? blockIdx.z * kRaKeys : 0, x_hi = p.po ? min(kr.total, x_lo + kRaKeys) : kr.total;
+  const int x_lo = PART ? blockIdx.z * kRaKeys : 0, x_hi = PART ? min(kr.total, x_lo + kRaKeys) : kr.total;
   if (x_lo >= x_hi) return;
   const int* bt = p.bt + (size_t)sg * p.maxb;
   for (int i = tid; i < nh * D; i += 256) {
@@ -107,11 +112,11 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
   const bool own = hs < tpc;
   const TC* kbase = (const TC*)p.kc + (size_t)gm * D;
   const TC* vbase = (const TC*)p.vc + (size_t)g * V + v0 + col;
-  float m[kRaHeads], l[kRaHeads], o[kRaHeads];      // of head hs + k tpc
+  float m[NH], l[NH], o[NH];      // of head hs + k tpc
 #pragma unroll
-  for (int k = 0; k < kRaHeads; ++k) {
+  for (int k = 0; k < NH; ++k) {
     const int h = hs + k * tpc;
-    const bool on = own && h < nh && p.sink && !p.po;
+    const bool on = own && h < nh && p.sink && !PART;
     m[k] = on ? p.sink[head(h)] : -INFINITY;
     l[k] = on ? 1.f : 0.f;
     o[k] = 0.f;
@@ -124,21 +129,28 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
       ss[tid] = bt[j / p.BS] * p.BS + j % p.BS;
     }
     __syncthreads();
+    TC vall[PART ? kRaKeys : 1];
+    if constexpr (PART) {
+      if (own) {
+#pragma unroll
+        for (int j = 0; j < kRaKeys; ++j) vall[j] = vbase[(size_t)ss[j] * p.vs];      // (past nk: the last one again)
+      }
+    }
     {  // scores: a wave has 64 keys and every other head
       const int x = (wv & 1) * 64 + lane, h0 = wv >> 1;
       if ((wv & 1) * 64 < nk && h0 < nh) {
         const TC* kp = kbase + (size_t)ss[x] * p.ks;
         const float* q0 = sq + h0 * D4;
-        const float* qh[4];
+        const float* qh[NH / 2];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) qh[k] = h0 + 2 * k < nh ? q0 + 2 * k * D4 : q0;
-        float a[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < NH / 2; ++k) qh[k] = h0 + 2 * k < nh ? q0 + 2 * k * D4 : q0;
+        float a[NH / 2] = {};
         if (VEC) {
-#pragma unroll 4
+#pragma unroll (PART ? 16 : 4)
           for (int d = 0; d < D; d += 4) {
             const f32x4 kv = rld4(kp + d);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
+            for (int k = 0; k < NH / 2; ++k) {
               const f32x4 qv = *reinterpret_cast<const f32x4*>(qh[k] + d);
 #pragma unroll
               for (int e = 0; e < 4; ++e) a[k] = fmaf(qv[e], kv[e], a[k]);
@@ -148,11 +160,11 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
           for (int d = 0; d < D; ++d) {
             const float kv = rld(kp, d);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) a[k] = fmaf(qh[k][d], kv, a[k]);
+            for (int k = 0; k < NH / 2; ++k) a[k] = fmaf(qh[k][d], kv, a[k]);
           }
         }
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < NH / 2; ++k)
           if (h0 + 2 * k < nh) {
             float s = a[k] * p.scale;
             if (p.softcap > 0.f) s = p.softcap * tanhf(s / p.softcap);
@@ -177,15 +189,12 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
     }
     __syncthreads();
     if (own) {
-      float op[kRaHeads];
+      float op[NH];
 #pragma unroll
-      for (int k = 0; k < kRaHeads; ++k) op[k] = 0.f;
-      auto four = [&](int j, int n) {               // keys j .. j + n of the part
-        float v[4];
+      for (int k = 0; k < NH; ++k) op[k] = 0.f;
+      auto with = [&](int j, const float (&v)[4]) {  // keys j .. j + 3 of the part
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = e < n ? rld(vbase, (size_t)ss[j + e] * p.vs) : 0.f;
-#pragma unroll
-        for (int k = 0; k < kRaHeads; ++k) {
+        for (int k = 0; k < NH; ++k) {
           const int h = hs + k * tpc;
           if (h < nh) {
             const f32x4 w = *reinterpret_cast<const f32x4*>(sp + h * kRaKeys + j);
@@ -194,14 +203,32 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
           }
         }
       };
-      const int nk4 = nk & ~3;
-      for (int j = 0; j < nk4; j += 4) four(j, 4);
-      if (nk4 < nk) four(nk4, nk - nk4);            // (weights past nk are zero, and zero times an infinity would be NaN)
+      // (weights past nk are zero, and zero times an infinity would be NaN)
+      if constexpr (PART) {
 #pragma unroll
-      for (int k = 0; k < kRaHeads; ++k) {
+        for (int j = 0; j < kRaKeys; j += 4)
+          if (j < nk) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = j + e < nk ? rld(vall + j + e, 0) : 0.f;
+            with(j, v);
+          }
+      } else {
+        auto four = [&](int j, int n) {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = e < n ? rld(vbase, (size_t)ss[j + e] * p.vs) : 0.f;
+          with(j, v);
+        };
+        const int nk4 = nk & ~3;
+        for (int j = 0; j < nk4; j += 4) four(j, 4);
+        if (nk4 < nk) four(nk4, nk - nk4);
+      }
+#pragma unroll
+      for (int k = 0; k < NH; ++k) {
         const int h = hs + k * tpc;
         if (h < nh) {
-          if (p.po) {
+          if constexpr (PART) {
             const size_t at = ((size_t)blockIdx.x * p.H + head(h)) * p.n_parts + blockIdx.z;
             p.po[at * V + v0 + col] = op[k];
             if (col == 0 && vb == 0) {
@@ -217,9 +244,9 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
       }
     }
   }
-  if (p.po || !own) return;
+  if (PART || !own) return;
 #pragma unroll
-  for (int k = 0; k < kRaHeads; ++k) {
+  for (int k = 0; k < NH; ++k) {
     const int h = hs + k * tpc;
     if (h < nh) {
       const int hh = head(h);
@@ -252,12 +279,13 @@ __global__ void __launch_bounds__(256) rows_attn_merge_kernel(RowsArgs p) {
 
 template <typename TQ, typename TC, typename TO>
 static int launch_rows(const RowsArgs& p, int T, hipStream_t s) {
-  const int D = p.D1 + p.D2, hpg = p.H / (p.G * p.M), HB = hpg < kRaHeads ? hpg : kRaHeads;
+  const int D = p.D1 + p.D2, hpg = p.H / (p.G * p.M), most = p.po ? kRaFew : kRaHeads, HB = hpg < most ? hpg : most;
   const size_t lds = sizeof(float) * ((size_t)HB * ((D + 3) / 4 * 4) + HB * kRaKeys + 2 * HB + kRaKeys);
   const dim3 grid(T, p.G * p.M * ((hpg + HB - 1) / HB) * ((p.V + 255) / 256), p.po ? p.n_parts : 1);
   // four numbers of a key at a time where every key starts on such a border
   const bool vec = D % 4 == 0 && p.ks % 4 == 0 && ((uintptr_t)p.kc & (4 * sizeof(TC) - 1)) == 0;
-  auto k = vec ? rows_attn_kernel<TQ, TC, TO, true> : rows_attn_kernel<TQ, TC, TO, false>;
+  auto k = p.po ? (vec ? rows_attn_kernel<TQ, TC, TO, true, true> : rows_attn_kernel<TQ, TC, TO, false, true>)
+                : (vec ? rows_attn_kernel<TQ, TC, TO, true, false> : rows_attn_kernel<TQ, TC, TO, false, false>);
   if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
     return (int)hipGetLastError();
   hipLaunchKernelGGL(k, grid, dim3(256), lds, s, p);

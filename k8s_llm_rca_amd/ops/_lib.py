@@ -45,6 +45,7 @@ _SIGS = {
     "k8s_gemm_row_step_dyt": [P, P, P, I, F, P, I, F, F, P, P, P, P, P, I, I, I, I, I, P],
     "k8s_gemm_skinny_f32": [P, I, P, P, I, I, I, I, P],
     "k8s_few_rows_f32": [P, I, P, P, I, I, I, P],
+    "k8s_few_rows_glu_f32": [P, I, P, P, I, I, I, P],
     "k8s_gemm_skinny_rope": [P, I, P, P, I, I, I, I, P, P, P, P, P, I, I, I, P],
     "k8s_gemm_mid": [P, I, P, P, I, I, I, I, I, I, P, P],
     "k8s_gemm_mid_part": [P, I, P, P, I, I, I, I, I, I, P, P],

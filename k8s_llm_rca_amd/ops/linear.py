@@ -497,6 +497,10 @@ def glu_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
                 return gemm_stream_silu(x, w, cfg)
         elif M > DISPATCH_MAX_M and big_shape_ok(M, I, K, True) and big_fused(M, I, K, True):
             return gemm_big(x, w, silu=True)
+    if w.shape[0] == 2 * I and _few_f32_ok(x, w):
+        out = torch.empty((M, I), dtype=torch.float32, device=x.device)
+        check(lib().k8s_few_rows_glu_f32(ptr(x), x.stride(0), ptr(w), ptr(out), M, I, K, stream_ptr(x)), "few_rows_glu_f32")
+        return out
     return glu_clamp(linear(x, w), 1.0, math.inf, 0.0)
 
 

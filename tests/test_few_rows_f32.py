@@ -62,3 +62,17 @@ def test_infinities_stay_in_their_row():
     x[1, 7] = float("inf")
     y = L.linear(x, w)
     assert torch.isfinite(y[[0, 2]]).all() and torch.isinf(y[1]).all()
+
+
+@pytest.mark.parametrize("n,k", [(1, 4), (3, 8), (127, 1028), (1024, 2048), (4095, 260), (4096, 64)])
+def test_gated_unit_is_product_and_pass(n, k):
+    """The products' sums and the pass's arithmetic: the same bits, also where a sum is not finite."""
+    x, w = operands(8, 2 * n, k)
+    w *= k ** -0.5
+    w[n - 1, 0] = float("nan")
+    w[2 * n - 1, k - 1] = float("inf")
+    most = 8 if 2 * n < 8192 else 5
+    for m in range(1, most + 1):
+        want = L.glu_clamp(L.linear(x[:m], w), 1.0, float("inf"), 0.0)
+        got = L.glu_proj(x[:m], w)
+        assert torch.equal(got.nan_to_num(7.0, 8.0, 9.0), want.nan_to_num(7.0, 8.0, 9.0))
