@@ -10,7 +10,7 @@
 //
 // GLU: w = [N gate rows; N up rows], y = g sigmoid(g) u of both (glu_clamp_kernel's arithmetic without its limits): a workgroup
 // takes two rows of each, so that the two rows of sums are not written, read and launched for again (8192 x 2048 at two
-// rows: 20.4 + 4.7 us -> @GLU@).
+// rows: 20.4 + 4.7 us -> 20.8 in a traced step).
 #include "common.h"
 
 namespace k8s {
