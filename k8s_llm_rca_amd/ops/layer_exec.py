@@ -68,6 +68,9 @@ _fuse_splitk = KNOBS.fuse_splitk
 # (csrc/kernels/norm_prologue.h; bit-identical, two launches fewer per layer)
 _norm_fuse = KNOBS.norm_fuse
 NORM_FUSE_MAX_T = 4
+# of the row-streaming kernel (us of the norm's launch and the product / of the fused form: 6144 x 4096 with the rotation at 1,
+# 2, 4 rows 15 / 11.8, 15 / 14.2, 15 / 18.4, 28672 x 4096 SwiGLU 40 / 36.3, 40.5 / 38.4, 40 / 44)
+NORM_FUSE_ROWS_T = 2
 NORM_FUSE_MAX_H = 4096      # norm_prologue.h: 256 threads, two 16-byte pieces each
 # (Round 3 also carried a row-chunked o / down GEMM with each chunk's
 # all-reduce on a side stream, and the prefill attention on a side stream beside
@@ -277,11 +280,16 @@ class LlamaExecutor:
         # fused norms (TP = 1): mirrors llama_exec.hip's nf_qkv / nf_gu conditions
         nf = 0
         if _norm_fuse and self._car is None and m.nf_flags is None and T <= NORM_FUSE_MAX_T and H <= NORM_FUSE_MAX_H:
-            if st.sel[0].kind in (LIN.KIND_SKINNY, LIN.KIND_ROWS) and st.sel[0].fuse == 3:
+            rows = LIN.KIND_ROWS if T <= NORM_FUSE_ROWS_T else -1
+            if st.sel[0].kind in (LIN.KIND_SKINNY, rows) and st.sel[0].fuse == 3:
                 nf |= 1
-            if st.sel[2].fuse == 2 and (st.sel[2].kind == LIN.KIND_ROWS
+            if st.sel[2].fuse == 2 and (st.sel[2].kind == rows
                                         or st.sel[2].kind == LIN.KIND_STREAM and st.sel[2].cfg in (4, 8)):
                 nf |= 2
+                # every workgroup makes the rows, so as few of them as there are (28672 x 4096 at 1, 2, 4 rows, us on one /
+                # two / four fragments 40.0 / 38.8 / 36.3, 46.9 / 43.3 / 38.4, 60.2 / 53.0 / 44.0; without the norm one: 35.7)
+                if st.sel[2].kind == LIN.KIND_ROWS and LIN.rows_shape_ok(T, m.inter, H, 4, 1, LIN.ROWS_SILU):
+                    st.sel[2].cfg = 4
         st.norm_fuse = nf
         res2 = scratch((T, H), dt, dev) if nf else None
         st.res2 = ptr(res2)

@@ -156,3 +156,40 @@ def test_operands_the_kernel_cannot_read_go_elsewhere():
         for f in (L.linear, L.proj):
             assert bool(((f(a, b).double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
         assert float((L.proj_planes(a, b).double().sum(0) - want).abs().max()) < 4e-6 * 32
+
+
+@gpu
+def test_executor_with_the_norms_in_front_of_both_products():
+    """One and two rows: the norm in front of the rotated and the gated product, the latter on the widest strips (whatever the
+    table says); three and four: apart.  The same bits as all apart, and as without the executor."""
+    from k8s_llm_rca_amd.models.config import get_config
+    from k8s_llm_rca_amd.models.llama import LlamaModel
+    from k8s_llm_rca_amd.ops import layer_exec as LX
+    from tests.test_tp_gpu import _prefill_inputs
+    keys = [(1536, 512), (2048, 512), (512, 1024)]
+    saved, fuse0 = {k: L._dispatch.get(k) for k in keys}, LX._norm_fuse
+    try:
+        L._dispatch[(1536, 512)] = L._dispatch[(2048, 512)] = [(16, "rows", 1, 1)]
+        L._dispatch[(512, 1024)] = [(16, "rows", 1, 2)]
+        m = LlamaModel(get_config("tiny-llama", n_layers=2, init_std=0.08), "cuda:0", BF, None, seed=4)
+        for T in (1, 2, 3, 4):
+            got = {}
+            for mode in ("fused", "apart", "python"):
+                LX._norm_fuse = mode == "fused"
+                LX.set_enabled(mode != "python")
+                inp, kc, vc = _prefill_inputs(m, T, seed=T)
+                got[mode] = m.forward(inp, kc, vc).float().cpu(), kc.float().cpu()
+                if mode == "fused":
+                    assert m._exec.st.norm_fuse == (3 if T <= LX.NORM_FUSE_ROWS_T else 0)
+                    assert m._exec.st.sel[2].cfg == (4 if T <= LX.NORM_FUSE_ROWS_T else 1)
+            for a, b in zip(got["fused"], got["apart"]):
+                assert torch.equal(a, b)
+            for a, b in zip(got["fused"], got["python"]):
+                assert torch.equal(a, b)
+    finally:
+        LX._norm_fuse = fuse0
+        LX.set_enabled(True)
+        for k, v in saved.items():
+            L._dispatch.pop(k, None)
+            if v is not None:
+                L._dispatch[k] = v
