@@ -588,9 +588,8 @@ __global__ void __launch_bounds__(256) big_reduce_kernel(const float* __restrict
 // sum the wrong slices.  So the workspace belongs to ONE stream: the first
 // launch that uses it claims it (g_tail_owner), and a launch on any other
 // stream runs without the split tail (whole-tile last wave: slower, never
-// wrong).  k8s_gemm_big_set_ws releases the claim.    The engine
-// claims it explicitly for its compute stream at init (k8s_gemm_big_claim_ws,
-// ADVICE r5), so a short-lived stream that happens to launch first (a capture's
+// wrong).  k8s_gemm_big_set_ws releases the claim.  The engine
+// claims it explicitly for its compute stream at init (k8s_gemm_big_claim_ws), so a short-lived stream that happens to launch first (a capture's
 // warm-up, a tuning side stream) can no longer take it; claims are serialised
 // by g_tail_mu, so two host threads never both own it.
 constexpr int kTailUnits = 256;
@@ -602,16 +601,24 @@ static long g_tail_foreign[16] = {};  // launches that skipped the tail (another
 static std::mutex g_tail_mu;
 
 // (tail tiles r, split S) for T tiles of nt K-tiles on 256 CUs: the last partial
-// wave's r tiles in r x S units (S in {4, 2}: r S <= 256, nt % (2 S) == 0, >= 8 K-tiles each).
+// wave's r tiles in r x S units (S in {4, 2}: r S <= 256, nt % (2 S) == 0, >= 8 K-tiles each),
+// or whole (r = 0) where that is no slower.  A whole tile takes some nt us; a split one nt / S, 12 us
+// for the partials' way out and back through the ticket, and 1 / 12 us for each of the r S units, whose
+// 256 KB share the memory (us past the full waves, split / whole: K 2048 at 8, 32, 64 tiles in four 23 / 32,
+// 31 / 34, 41 / 36, at 96, 128 in two 38 / 33, 47 / 35; K 4096 at 16, 64 in four 32 / 62, 53 / 63, at 96, 112 in
+// two 58 / 65, 70 / 59; K 1024 at 128 in two 38 / 21; K 8192 at 32 in four 53 / 117).
 static void tail_plan(int T, int nt, int& r, int& S) {
   r = T % 256;
   S = 1;
   if (r == 0) return;
-  for (int c : {4, 2})
-    if (r * c <= kTailUnits && nt % (2 * c) == 0 && nt / c >= 8) {
+  int best = 12 * nt;
+  for (int c : {4, 2}) {
+    const int cost = 12 * nt / c + 144 + r * c;
+    if (r * c <= kTailUnits && nt % (2 * c) == 0 && nt / c >= 8 && cost < best) {
       S = c;
-      break;
+      best = cost;
     }
+  }
   if (S == 1) r = 0;
 }
 

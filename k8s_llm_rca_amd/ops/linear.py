@@ -424,14 +424,17 @@ def proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return linear(x, w)
 
 
-def big_tiles_fill(M: int, N: int, silu: bool) -> bool:
-    """Whether gemm_big's 256-row tiles fill the 256 compute units to four fifths over all their waves.  Then its fused
-    epilogue beats hipBLASLt and a pass over the result, otherwise the idle last wave costs more than the pass: us apart /
-    fused of SwiGLU 8192 x 2048 at 192 tiles 50 / 49, 256 65 / 56, 320 100 / 111, 384 106 / 110, 448 116 / 100, 512
-    124 / 106, 704 192 / 148, 4096 tiles 936 / 811, and of the squared relu 128 37 / 52, 192 52 / 44, 256 63 / 52, 320
-    83 / 100, 384 98 / 102, 448 112 / 96, 512 120 / 102, 2048 tiles 479 / 400."""
+def big_tiles_fill(M: int, N: int, silu: bool, K: int = 4096) -> bool:
+    """Whether gemm_big's 256-row tiles fill the 256 compute units far enough over all their waves.  Then its fused epilogue
+    beats hipBLASLt and a pass over the result, otherwise the idle last wave costs more than the pass: up to a K of 1024 from
+    half on, up to 2048 from seven tenths, else from four fifths.  us fused / apart at waves of tiles:  squared relu 8192 x
+    2048 at 0.50 38.6 / 36.8, 0.75 42 / 48, 1.00 49 / 60, 1.12 77 / 72, 1.38 82 / 90, 1.50 83 / 96, 2.12 123 / 128, 2.38
+    127 / 141, 5.00 226 / 282, 8192 x 1024 at 0.38 24.0 / 23.6, 0.50 24.9 / 25.3, 1.12 48 / 53;  SwiGLU 8192 x 2048 at 0.75
+    48.4 / 48.7, 1.25 96 / 86, 1.50 97 / 99, 2.25 138 / 135, 2.50 137 / 154, 4.25 227 / 239, 6144 x 2048 at 1.31 85 / 81, 1.50
+    85 / 89, 8192 x 4096 at 1.50 153 / 148, 2.50 239 / 248."""
     tiles = -(-M // 256) * -(-N // (128 if silu else 256))
-    return 5 * tiles >= 4 * 256 * -(-tiles // 256)
+    tenths = 5 if K <= 1024 else 7 if K <= 2048 else 8
+    return 10 * tiles >= tenths * 256 * -(-tiles // 256)
 
 
 SHORT_K = 512       # up to here what is paid is the result's way through memory, not the tiles
@@ -445,7 +448,7 @@ def big_fused(M: int, N: int, K: int, silu: bool) -> bool:
     512 at 3.2 16.7 / 17.8, 5.1 21.4 / 18.4, 0.3 8.1 / 15.8."""
     if K <= SHORT_K:
         return M * N * (2 if silu else 1) >= (1 << 21) + 4096 * K
-    return big_tiles_fill(M, N, silu)
+    return big_tiles_fill(M, N, silu, K)
 
 
 def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
