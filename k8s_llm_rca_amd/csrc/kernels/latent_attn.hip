@@ -39,6 +39,7 @@ namespace k8s {
 //
 // NP: 32-number chunks of the cache row behind the latent (a score-only key part): row width R + 32 NP.
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr int kBatch = 8;      // fragments that are read from LDS at once
 
 struct LatArgs {
   const uint16_t* qa;     // element (t, h, c) at t * qst + h * qsh + c
@@ -59,6 +60,8 @@ struct LatArgs {
   int H, HC, TPM, BS;
   float scale_log2;
 };
+
+typedef __attribute__((address_space(3))) void lds_void_t;
 
 __device__ __forceinline__ bf16x8 ld16(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
@@ -111,18 +114,23 @@ __device__ __forceinline__ void lat_softmax(const f32x4 (&s)[2], float scale_log
 // Prompt portions: the four waves of a workgroup own four consecutive items of ONE
 // segment (the host pads every segment's items to a multiple of four with empty
 // ones), so they read the same keys.  A chunk's operand fragments do not depend on
-// the item: kf[t][cc] and vf[dt] are loaded from global memory once per workgroup
-// (a quarter by each wave), parked in LDS in fragment order -- slot f holds the 64
-// lanes' 16 bytes, so writes and reads are conflict-free -- and read back by all
-// four waves.  Two buffers: chunk i + 1 is fetched into registers while chunk i
-// is computed, and written after it; one barrier per chunk.
+// the item: kf[t][cc] and vf[dt] go from global memory to LDS once per workgroup, without
+// a register between (a quarter by each wave), in fragment order -- slot f holds the 64
+// lanes' 16 bytes, so reads are conflict-free -- and are read by all
+// four waves.  Two buffers: chunk i + 1 is asked for when chunk i begins and its page number
+// one chunk earlier; one barrier per chunk.
+//
+// What bounds it: one tile of 16 rows uses a fragment once, so a wave waits for LDS between its batches, and beside 576
+// cycles of matrix instructions a chunk has some 480 of softmax.  16384 rows of 16 heads over a window of 1024 keys, R 256 +
+// 64: 596 us with fragments through registers and two reads in flight, 550 with LDS-DMA, batches of eight and the page number
+// early (4 and 12 a batch the same); 3517 and 4351 rows 107 -> 96 and 183 -> 157.  Two tiles a wave, one wave a SIMD: 669.
 template <int NR, int NP, int MT, int OCC>
 __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs a) {
   constexpr int R = NR * 32, ND = R / 16, NC = NR + NP, RW = R + 32 * NP, NF = 2 * NC + ND, NFW = (NF + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   bf16x8* frag = reinterpret_cast<bf16x8*>(lds_raw);          // [2][NF][64]
   __shared__ int kend_s[4], kbeg_s[4];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, h = lane >> 4;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, h = lane >> 4;
   // ... and the LAST items of the range first: they see the most keys, so the short ones fill the tail
   const int per = gridDim.x >> 3;
   const int blk = (gridDim.x & 7) == 0 ? (blockIdx.x & 7) * per + (per - 1 - (blockIdx.x >> 3))
@@ -166,65 +174,82 @@ __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs 
     l[mt] = 0.f;
   }
   const int* pages = a.bt + (size_t)sg * a.maxb;
-  // this wave's share of a chunk's fragments: f = wv + 4 i
-  bf16x8 pre[NFW];
-  auto fetch = [&](int kb) {
-    const int page = pages[kb / a.BS], off = kb % a.BS;
+  // this wave's share of a chunk's fragments, f = wv + 4 i, straight into LDS (lane l's 16 bytes at 16 l of the slot)
+  auto fetch = [&](int kb, int page, int buf) {
+    const int off = kb % a.BS;
     const uint16_t* cp = a.c + (size_t)page * a.BS * RW;
     const uint16_t* tp = a.ct + (size_t)page * R * a.BS;
 #pragma unroll
     for (int i = 0; i < NFW; ++i) {
       const int f = wv + 4 * i;
+      if (NF % 4 && f >= NF) continue;
+      const uint16_t* src;
       if (f < 2 * NC) {
         const int t = f / NC, cc = f - t * NC;
-        const int key = off + 8 * (r >> 2) + 4 * t + (r & 3);
-        pre[i] = ld16(cp + (size_t)key * RW + 32 * cc + 8 * h);
-      } else if (NF % 4 == 0 || f < NF) {
-        const int dt = f - 2 * NC;
-        pre[i] = ld16(tp + (size_t)(16 * dt + r) * a.BS + off + 8 * h);
+        src = cp + (size_t)(off + 8 * (r >> 2) + 4 * t + (r & 3)) * RW + 32 * cc + 8 * h;
+      } else {
+        src = tp + (size_t)(16 * (f - 2 * NC) + r) * a.BS + off + 8 * h;
       }
+      __builtin_amdgcn_global_load_lds(src, (lds_void_t*)(frag + ((size_t)buf * NF + f) * 64), 16, 0, 0);
     }
   };
-  auto park = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < NFW; ++i)
-      if (NF % 4 == 0 || wv + 4 * i < NF) frag[((size_t)buf * NF + wv + 4 * i) * 64 + lane] = pre[i];
+  auto landed = [&]() {                                       // this wave's share is there; then every wave's
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
   };
+  auto page_of = [&](int kb) { return pages[min(kb, k_end - 1) / a.BS]; };
+  int page = 0;
   if (k_beg < k_end) {
-    fetch(k_beg);
-    park(0);
+    fetch(k_beg, page_of(k_beg), 0);
+    page = page_of(k_beg + 32);
   }
+  // The fragments in the order of their use: keys (both tiles in turn), then values; batches of kBatch, the next one asked for
+  // once the first of a batch is there -- the compiler waits for all LDS reads in flight where LDS-DMA is about.
+  auto slot = [](int j) { return j < 2 * NC ? (j & 1) * NC + (j >> 1) : j; };
   int buf = 0;
   for (int kb = k_beg; kb < k_end; kb += 32, buf ^= 1) {
-    __syncthreads();
-    const bool more = kb + 32 < k_end;
-    if (more) fetch(kb + 32);
+    landed();                                                 // (and nobody reads the other buffer any more)
+    if (kb + 32 < k_end) fetch(kb + 32, page, buf ^ 1);
+    page = page_of(kb + 64);                                  // there with that chunk
     const bf16x8* fb = frag + (size_t)buf * NF * 64 + lane;
+    const bool open = kb + 31 <= pos0 && (a.window <= 0 || kb >= pos0 + ntok - a.window);
     f32x4 s[MT][2];
+    bf16x8 pf[MT], fr[2][kBatch];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int mt = 0; mt < MT; ++mt) s[mt][0] = s[mt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto read = [&](int b) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) s[mt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < kBatch; ++i)
+        if (b * kBatch + i < NF) fr[b & 1][i] = fb[slot(b * kBatch + i) * 64];
+    };
+    read(0);
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) {
-        const bf16x8 kf = fb[(t * NC + cc) * 64];
+    for (int b = 0; b * kBatch < NF; ++b) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          s[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[mt][cc], s[mt][t], 0, 0, 0);
+      for (int i = 0; i < kBatch; ++i) {
+        const int j = b * kBatch + i;
+        if (j >= NF) continue;
+        if (j == 2 * NC) {
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+            lat_softmax<ND>(s[mt], a.scale_log2, open, kb, h, lo[mt], limit[mt], m[mt], l[mt], o[mt], pf[mt]);
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          if (j < 2 * NC)
+            s[mt][j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fr[b & 1][i], qf[mt][j >> 1], s[mt][j & 1], 0, 0, 0);
+          else
+            o[mt][j - 2 * NC] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[mt], fr[b & 1][i], o[mt][j - 2 * NC], 0, 0, 0);
+        }
+        if (i == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+          if ((b + 1) * kBatch < NF) read(b + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
-    const bool open = kb + 31 <= pos0 && (a.window <= 0 || kb >= pos0 + ntok - a.window);
-    bf16x8 pf[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-      lat_softmax<ND>(s[mt], a.scale_log2, open, kb, h, lo[mt], limit[mt], m[mt], l[mt], o[mt], pf[mt]);
-#pragma unroll
-    for (int dt = 0; dt < ND; ++dt) {
-      const bf16x8 vf = fb[(2 * NC + dt) * 64];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) o[mt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[mt], vf, o[mt][dt], 0, 0, 0);
-    }
-    if (more) park(buf ^ 1);
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
