@@ -154,7 +154,7 @@ __device__ __forceinline__ void set_chunk(f32x16& v, const f32x4& t) {
 template <int MODE, int SH>
 __device__ __forceinline__ int w_row(int tn, int h, int slab, int rho, int N) {
   if constexpr (SH == 16) {
-    if constexpr (MODE == 0 || MODE == 3)  // lane group g of the fragment pair <- columns 8g .. 8g+7
+    if constexpr (MODE == 0 || MODE >= 3)  // lane group g of the fragment pair <- columns 8g .. 8g+7
       return tn * BN + 128 * h + 32 * slab + 8 * ((rho >> 2) & 3) + 4 * (rho >> 4) + (rho & 3);
     else if constexpr (MODE == 1)  // fragment 0: gate rows, fragment 1: the up rows of the same act columns
       return (rho >> 4 ? N : 0) + tn * 128 + 64 * h + 16 * slab + (rho & 15);
@@ -164,7 +164,7 @@ __device__ __forceinline__ int w_row(int tn, int h, int slab, int rho, int N) {
     // 32x32 accumulator: register r of lane half hh holds fragment row
     // (r & 3) + 8 (r >> 2) + 4 hh; rho -> (r, hh)
     const int r = (rho & 3) + 4 * (rho >> 3), hh = (rho >> 2) & 1;
-    if constexpr (MODE == 0 || MODE == 3)  // lane half hh <- columns 16 hh .. 16 hh + 15 (register order)
+    if constexpr (MODE == 0 || MODE >= 3)  // lane half hh <- columns 16 hh .. 16 hh + 15 (register order)
       return tn * BN + 128 * h + 32 * slab + 16 * hh + r;
     else if constexpr (MODE == 1)  // registers 0-7: gate of act columns 8 hh .. +7, registers 8-15: their up rows
       return (r >= 8 ? N : 0) + tn * 128 + 64 * h + 16 * slab + 8 * hh + (r & 7);
@@ -181,13 +181,15 @@ struct RopeArgs {
   uint16_t* kc;          // [blocks][nkv][BS][128]
   uint16_t* vc;          // [blocks][nkv][128][BS]
   int nq, nkv, BS;
+  float scale;           // MODE 4
 };
 
 // MODE 0: plain (N output columns = W rows); MODE 1: SwiGLU (N = I output
 // act columns, W has 2I rows, I = N); MODE 2: the qkv projection with RoPE on q
 // and k and the paged K / V write in the epilogue (N = (nq + 2 nkv) 128; the
 // rope_kv_kernel's arithmetic and rounding: bit-identical to GEMM + k8s_rope_kv);
-// MODE 3: MODE 0 with max(., 0)^2 of every output.
+// MODE 3: MODE 0 with max(., 0)^2 of every output;
+// MODE 4: y is fp32 and scale times the product is added to it.
 // VAR bit 0: ping-pong stagger of waves
 // 4-7; bit 1: s_setprio(1) around the MFMA clusters; bit 2: the 32x32x16 MFMA
 // (1 = the default).
@@ -524,6 +526,15 @@ __global__ void __launch_bounds__(512, 1) gemm_big_kernel(const uint16_t* __rest
             }
           }
         }
+      } else if (MODE == 4) {
+        float* o = reinterpret_cast<float*>(y) + (size_t)m * ldy + tn * BN + 128 * qw + 32 * wc + NV * fhi;
+#pragma unroll
+        for (int e = 0; e < NV; e += 4) {
+          f32x4 t = *reinterpret_cast<const f32x4*>(o + e);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) t[c] = fmaf(ra.scale, v[e + c], t[c]);
+          *reinterpret_cast<f32x4*>(o + e) = t;
+        }
       } else if (MODE == 0 || MODE == 3) {
         uint16_t* o = y + (size_t)m * ldy + tn * BN + 128 * qw + 32 * wc + NV * fhi;
 #pragma unroll
@@ -680,7 +691,7 @@ static int big_launch(const void* x, int ldx, const void* w, void* y, int ldy, i
   using namespace k8s::big;
   if (M <= 0) return 0;
   if (splits < 1 || K % (2 * BK * splits) || K < 2 * BK || ldx % 8 || ldx < K || ldy < N || N <= 0 ||
-      (mode != 1 && N % BN) || (mode == 1 && N % 128) || mode < 0 || mode > 3 ||
+      (mode != 1 && N % BN) || (mode == 1 && N % 128) || mode < 0 || mode > 4 ||
       ((uintptr_t)x % 16) || ((uintptr_t)w % 16) || (mode != 1 && (ldy % 8 || (uintptr_t)y % 16)) ||
       (mode == 1 && (ldy % 4 || (uintptr_t)y % 8)) || (splits > 1 && (mode != 0 || part == nullptr)))
     return (int)hipErrorInvalidValue;
@@ -700,6 +711,8 @@ static int big_launch(const void* x, int ldx, const void* w, void* y, int ldy, i
   } else if (mode == 2) {
     rc = (var & 4) ? launch<2, 5>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s)
                    : launch<2, 1>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s);
+  } else if (mode == 4) {
+    rc = launch<4, 1>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s);
   } else {
     rc = (var & 4) ? launch<3, 5>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s)
                    : launch<3, 1>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s);
@@ -775,6 +788,7 @@ K8S_API long k8s_gemm_big_tail_foreign() {
 // aligned x / w / y (8 for y in mode 1); y row stride ldy >= N.
 K8S_API int k8s_gemm_big(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int mode,
                          int var, hipStream_t s) {
+  if (mode == 4) return (int)hipErrorInvalidValue;       // k8s_gemm_big_add
   return big_launch(x, ldx, w, y, ldy, M, N, K, mode, var, 1, nullptr, true, s);
 }
 
@@ -790,6 +804,17 @@ K8S_API int k8s_gemm_big_rope(const void* x, int ldx, const void* w, void* qkv, 
     return (int)hipErrorInvalidValue;
   g_rope = RopeArgs{pos, cos_sin, slots, (uint16_t*)kc, (uint16_t*)vc, nq, nkv, BS};
   const int rc = big_launch(x, ldx, w, qkv, ldq, M, N, K, 2, var, 1, nullptr, true, s);
+  g_rope = RopeArgs{};
+  return rc;
+}
+
+// r[M][N] (fp32, rows ldr apart) += scale * (x . w^T).  N % 256 == 0, ldr % 8 == 0, r 16-byte aligned.
+K8S_API int k8s_gemm_big_add(const void* x, int ldx, const void* w, float* r, int ldr, int M, int N, int K, float scale,
+                             hipStream_t s) {
+  using namespace k8s::big;
+  g_rope = RopeArgs{};
+  g_rope.scale = scale;
+  const int rc = big_launch(x, ldx, w, r, ldr, M, N, K, 4, 1, 1, nullptr, true, s);
   g_rope = RopeArgs{};
   return rc;
 }

@@ -392,6 +392,20 @@ def _few_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 ADD_ROWS = 6144
 
 
+def big_add_pays(M: int, N: int, K: int) -> bool:
+    """Whether gemm_big adds a product to an fp32 residual quicker than the library: where its 256-row tiles all but fill their
+    waves, one or two of them or a long K.  us library / gemm_big at waves of tiles:  2048 x 8192 at 0.78 198 / 173, 1.00
+    207 / 196, 1.47 316 / 337, 2.00 412 / 405, 3.00 620 / 596, 4.00 826 / 788;  2048 x 2048 at 0.78 66 / 59, 1.00 70 / 65,
+    1.12 87 / 104, 2.00 130 / 127, 3.00 202 / 205, 4.00 267 / 283;  4096 x 4096 at 2.00 219 / 209, 2.25 254 / 292, 4.00
+    447 / 448;  2048 x 14336 at 1.00 345 / 332, 4096 x 8192 at 6.00 1207 / 1158;  1024 x 8192 at 0.50 116 / 127."""
+    if N % 256 or K % 128 or K < 2048:
+        return False
+    tiles = -(-M // 256) * (N // 256)
+    if tiles <= 256:
+        return tiles >= 196
+    return (tiles <= 512 or K >= 8192) and 100 * tiles >= 95 * 256 * -(-tiles // 256)
+
+
 def proj_add(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, scale: float = 1.0):
     """``r += scale * (x @ w.T)`` on an fp32 residual ``r`` [M, N] where that pays (the result is then None), else the
     product as :func:`proj_planes` leaves it, which the caller's next pass adds."""
@@ -404,6 +418,10 @@ def proj_add(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, scale: float = 1
     if ws is None:
         ws = _blaslt_ws[x.device] = torch.empty(BLASLT_WS_BYTES, dtype=torch.uint8, device=x.device)
     for a, b in _row_parts(M, N, K):
+        if big_add_pays(b - a, N, K) and r.data_ptr() % 16 == 0:
+            check(lib().k8s_gemm_big_add(ptr(x[a:]), x.stride(0), ptr(w), ptr(r[a:]), N, b - a, N, K, float(scale),
+                                         stream_ptr(x)), "gemm_big_add")
+            continue
         check(lib().k8s_blaslt_gemm2(ptr(x[a:]), x.stride(0), ptr(w), ptr(r[a:]), N, b - a, N, K, ptr(ws), BLASLT_WS_BYTES,
                                      stream_ptr(x), 2, float(scale)), "blaslt_gemm_add")
     return None

@@ -1,4 +1,5 @@
-"""Library products of which whole waves of tiles go into a launch of their own (ops/linear.py: row_cut)."""
+"""Library products of which whole waves of tiles go into a launch of their own (ops/linear.py: row_cut), and those that
+gemm_big adds to the residual."""
 import pytest
 import torch
 
@@ -42,3 +43,23 @@ def test_cut_products_against_float64(m, n, k):
     out = torch.full((m, n + 16), 3.0, device="cuda", dtype=BF)
     b = L.lib_gemm(x, w, out[:, :n])
     assert bool(((b.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()) and bool((out[:, n:] == 3.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,lda", [(6200, 2048, 2048, 2048), (6144, 2304, 2048, 2112), (50100, 256, 2048, 2048),
+                                       (8191, 2048, 2048, 2056), (200, 512, 256, 256), (1, 256, 128, 128)])
+def test_gemm_big_adds_to_the_residual(m, n, k, lda):
+    g = torch.Generator().manual_seed(m + n)
+    x = torch.randn(m, lda, generator=g).to(BF).cuda()[:, :k]
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(BF).cuda()
+    want = x.double() @ w.double().T
+    buf = torch.randn(m + 1, n, generator=g).cuda()
+    before = buf.clone()
+    L.check(L.lib().k8s_gemm_big_add(L.ptr(x), lda, L.ptr(w), L.ptr(buf), n, m, n, k, 0.5, L.stream_ptr(x)), "add")
+    assert float((buf[:m].double() - before[:m].double() - 0.5 * want).abs().max()) < 4e-6 * k ** 0.5
+    assert torch.equal(buf[m], before[m])
+    if m >= L.ADD_ROWS and k >= 2048:
+        assert L.big_add_pays(m, n, k)
+        r = before[:m].clone()
+        assert L.proj_add(r, x, w, 0.5) is None and torch.equal(r, buf[:m])
+    assert L.lib().k8s_gemm_big_add(L.ptr(x), lda, L.ptr(w), L.ptr(buf), n, m, n - 128, k, 0.5, L.stream_ptr(x)) != 0
