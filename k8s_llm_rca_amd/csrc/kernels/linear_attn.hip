@@ -72,9 +72,18 @@ __device__ __forceinline__ bf16x8 lds16(const uint16_t* p) { return *reinterpret
 struct Blk {
   uint2 r[4];
 };
-__device__ __forceinline__ void blk_load(Blk& b, const uint16_t* p, size_t xs, int t, int n) {
+// p: the block's first row (the same for all lanes), off: this thread's row t and column in bytes from there.  A whole block of
+// 64 rows needs no look at n.
+__device__ __forceinline__ void blk_load(Blk& b, const uint16_t* p, uint32_t off, int xs, int t, int n) {
+  const char* q = reinterpret_cast<const char*>(p);
+  if (n >= kLaTok) {
 #pragma unroll
-  for (int k = 0; k < 4; ++k) b.r[k] = t + k < n ? *reinterpret_cast<const uint2*>(p + (t + k) * xs) : uint2{0u, 0u};
+    for (int k = 0; k < 4; ++k) b.r[k] = *reinterpret_cast<const uint2*>(q + (size_t)k * xs * 2 + off);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      b.r[k] = t + k < n ? *reinterpret_cast<const uint2*>(q + (size_t)k * xs * 2 + off) : uint2{0u, 0u};
+  }
 }
 template <bool SILU>
 __device__ __forceinline__ void blk_act(Blk& b) {
@@ -116,8 +125,13 @@ constexpr int la_lds_bytes(bool outputs) {
   return 2 * (trow(D) + trow(16 * NW) + (outputs ? kLaTok * ld + k_or_p : 0));
 }
 
-template <int D, int NW, int MODE, bool SILU>
-__global__ void __launch_bounds__(64 * NW, 2) decay_attn_mfma_kernel(LinArgs a) {
+// TWO: 128 registers, so that two workgroups of eight waves share a compute unit, where there are more than 256 of them: this
+// thread's numbers are made anew in every block, unknown to the optimizer, or the addresses of all the tiles would take the
+// registers.  Alone on its unit a workgroup is the slower for it (16 heads of 128, one workgroup a unit 131 / 148 us); 64
+// portions of 256 to 512 rows 239 - 254 -> 217 - 242 by run, 8 of 2048 cut into 512 workgroups 223 - 226 -> 198 - 221, seven of
+// 351 to 701 93 - 97 -> 72 - 77.
+template <int D, int NW, int MODE, bool SILU, bool TWO>
+__global__ void __launch_bounds__(64 * NW, TWO ? 4 : 2) decay_attn_mfma_kernel(LinArgs a) {
   constexpr int NT = 64 * NW, VB = 16 * NW, ND = D / 16, NC = D / 32, LD = D + kLaPad, LP = kLaTok + kLaPad;
   constexpr int KB = (16 * (D / 4) + NT - 1) / NT, VBK = (16 * (VB / 4) + NT - 1) / NT;   // blocks per thread
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -153,7 +167,7 @@ __global__ void __launch_bounds__(64 * NW, 2) decay_attn_mfma_kernel(LinArgs a) 
 #pragma unroll
   for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) S[dt][i] = (!fresh && vok) ? st[(size_t)(16 * dt + 4 * hq + i) * V + vcol] : 0.f;
+    for (int i = 0; i < 4; ++i) S[dt][i] = (!fresh && vok) ? (st + (size_t)(16 * dt + i) * V)[(uint32_t)(4 * hq * V + vcol)] : 0.f;
   Blk bq[MODE != 1 ? KB : 1], bk[KB], bv[VBK];
   const int qo = hh * D, ko = (H + hh) * D, vo = 2 * H * D + hh * V + v0;
   auto fetch = [&](int t0) {
@@ -163,18 +177,22 @@ __global__ void __launch_bounds__(64 * NW, 2) decay_attn_mfma_kernel(LinArgs a) 
     for (int b = 0; b < KB; ++b) {
       const int e = tid + b * NT, t = e / (D / 4) * 4, c = e % (D / 4) * 4;
       if ((16 * (D / 4)) % NT == 0 || t < kLaTok) {
-        if (MODE != 1) blk_load(bq[b], xp + qo + c, a.xs, t, n);
-        blk_load(bk[b], xp + ko + c, a.xs, t, n);
+        const uint32_t off = 2u * ((uint32_t)t * a.xs + c);
+        if (MODE != 1) blk_load(bq[b], xp + qo, off, a.xs, t, n);
+        blk_load(bk[b], xp + ko, off, a.xs, t, n);
       }
     }
 #pragma unroll
     for (int b = 0; b < VBK; ++b) {
       const int e = tid + b * NT, t = e / (VB / 4) * 4, c = e % (VB / 4) * 4;
-      blk_load(bv[b], xp + vo + c, a.xs, t, v0 + c < V ? n : 0);
+      blk_load(bv[b], xp + vo, 2u * ((uint32_t)t * a.xs + c), a.xs, t, V % VB == 0 || v0 + c < V ? n : 0);
     }
   };
   fetch(r0);
   for (int t0 = r0; t0 < r1; t0 += kLaTok) {
+    int tid = threadIdx.x;
+    if constexpr (TWO) asm volatile("" : "+v"(tid));
+    const int r = tid & 15, hq = (tid & 63) >> 4;
     const int nb = min(kLaTok, r1 - t0);
     __syncthreads();                                        // the previous block's tiles are read no more
 #pragma unroll
@@ -297,15 +315,18 @@ __global__ void __launch_bounds__(64 * NW, 2) decay_attn_mfma_kernel(LinArgs a) 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int tk = 16 * t + 4 * hq + i;
-          if (tk < nb) a.o[(size_t)(t0 + tk) * H * V + (size_t)hh * V + vcol] = O[t][i];
+          float* orow = a.o + (size_t)(t0 + 16 * t + i) * H * V + (size_t)hh * V + v0;
+          if (tk < nb) orow[(uint32_t)(4 * hq * H * V + 16 * wv + r)] = O[t][i];
         }
     }
   }
   if (MODE != 2 && vok) {
+    uint32_t at = 4 * hq * V + vcol;
+    asm volatile("" : "+v"(at));                            // not kept in registers through the walk
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) st[(size_t)(16 * dt + 4 * hq + i) * V + vcol] = S[dt][i];
+      for (int i = 0; i < 4; ++i) (st + (size_t)(16 * dt + i) * V)[at] = S[dt][i];
   }
 }
 
@@ -334,7 +355,9 @@ __global__ void __launch_bounds__(256) decay_carry_kernel(const float* __restric
 template <int D, int NW, int MODE, bool SILU>
 static int launch_la(const LinArgs& a, int items, hipStream_t s) {
   constexpr int lds = la_lds_bytes<D, NW>(MODE != 1);
-  auto k = decay_attn_mfma_kernel<D, NW, MODE, SILU>;
+  auto k = decay_attn_mfma_kernel<D, NW, MODE, SILU, false>;
+  if constexpr (D == 128 && NW == 8)
+    if ((long)items * a.H * ((a.V + 127) / 128) > 256) k = decay_attn_mfma_kernel<D, NW, MODE, SILU, true>;
   if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds))
     return (int)hipGetLastError();
   hipLaunchKernelGGL(k, dim3(items, a.H, (a.V + 16 * NW - 1) / (16 * NW)), dim3(64 * NW), lds, s, a);

@@ -838,9 +838,8 @@ def decay_attention(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor
         longest = max(b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:]))
         mfma = longest >= LIN_MFMA_ROWS and decay_mfma_ok(D, V, x.dtype, x.device) and x.stride(0) % 4 == 0
         if mfma:
-            ranges = max(1, LIN_GROUPS // (H * -(-V // 128)))      # as many as give the chip a workgroup per unit
-            rows = max(LIN_CHUNK, -(-T // (64 * ranges)) * 64)
-            cr = seg.chunk_ranges(rows, rows)                       # (None: no portion is longer than a range)
+            rows = _lin_rows(T, seg.n_seg, H, D, V)
+            cr = seg.chunk_ranges(rows, rows) if rows else None     # (None: no portion is longer than a range)
         else:
             cr = seg.chunk_ranges(SSM_CHUNK, 2 * SSM_CHUNK) if seg.n_seg * H * V * 8 < SEQ_FILL_LANES else None
         chunks, c0, cs, nch = None, None, None, 0
@@ -874,6 +873,19 @@ def decay_attention(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor
 LIN_MFMA_ROWS = 17      # rows of a step's longest portion from which the matrix-core form runs
 LIN_CHUNK = 128         # rows at least per range where ranges of a portion run in parallel
 LIN_GROUPS = 256        # workgroups (ranges x heads x 128 value columns) a step is cut into
+
+
+def _lin_rows(T: int, n_seg: int, H: int, D: int, V: int) -> int:
+    """Rows of a range, 0: portions stay whole.  As many ranges as give the chip a workgroup per unit; of the form that two
+    workgroups of a unit share (csrc/kernels/linear_attn.hip) two, where the portions are not one or a few long ones, whose
+    carry walks all of them (us of 16 heads of 128 at 256 / 512 workgroups: 8 x 2048 rows 223 - 231 / 198 - 221, 7 of 351 to
+    701 91 / 72 - 77, 1 x 4000 73 / 76), and none where the portions are 256 workgroups by themselves (16 x 1024 131 / 194)."""
+    per, groups = H * -(-V // 128), LIN_GROUPS
+    if D == 128 and V > 64:
+        if n_seg * per >= LIN_GROUPS:
+            return 0
+        groups *= 2 if n_seg >= 4 else 1
+    return max(LIN_CHUNK, -(-T // (64 * max(1, groups // per))) * 64)
 
 
 def decay_mfma_ok(D: int, V: int, dtype, device) -> bool:
