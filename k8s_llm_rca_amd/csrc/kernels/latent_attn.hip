@@ -115,15 +115,18 @@ __device__ __forceinline__ void lat_softmax(const f32x4 (&s)[2], float scale_log
 // segment (the host pads every segment's items to a multiple of four with empty
 // ones), so they read the same keys.  A chunk's operand fragments do not depend on
 // the item: kf[t][cc] and vf[dt] go from global memory to LDS once per workgroup, without
-// a register between (a quarter by each wave), in fragment order -- slot f holds the 64
-// lanes' 16 bytes, so reads are conflict-free -- and are read by all
-// four waves.  Two buffers: chunk i + 1 is asked for when chunk i begins and its page number
+// a register between (a quarter by each wave) -- slot f holds the 64
+// lanes' 16 bytes, row by row, a row's four pieces swapped so that reads are
+// conflict-free -- and are read by all four waves.  Two buffers: chunk i + 1 is asked for when chunk i begins and its page number
 // one chunk earlier; one barrier per chunk.
 //
 // What bounds it: one tile of 16 rows uses a fragment once, so a wave waits for LDS between its batches, and beside 576
 // cycles of matrix instructions a chunk has some 480 of softmax.  16384 rows of 16 heads over a window of 1024 keys, R 256 +
 // 64: 596 us with fragments through registers and two reads in flight, 550 with LDS-DMA, batches of eight and the page number
-// early (4 and 12 a batch the same); 3517 and 4351 rows 107 -> 96 and 183 -> 157.  Two tiles a wave, one wave a SIMD: 669.
+// early (4 and 12 a batch the same), 453 with a row's 64 bytes in four lanes that follow each other (in fragment order they
+// lie 16 apart and each is a lookup of its own in the first-level cache); 3517 and 4351 rows 107 -> 96 -> 87 and 183 -> 157
+// -> 149.  Not quicker: two tiles a wave and one wave a SIMD (669 before the last change), eight waves to a workgroup that
+// share the keys of 8 items (495: all wait at one barrier), a row's 128 bytes in eight lanes (465).
 template <int NR, int NP, int MT, int OCC>
 __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs a) {
   constexpr int R = NR * 32, ND = R / 16, NC = NR + NP, RW = R + 32 * NP, NF = 2 * NC + ND, NFW = (NF + 3) / 4;
@@ -174,7 +177,10 @@ __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs 
     l[mt] = 0.f;
   }
   const int* pages = a.bt + (size_t)sg * a.maxb;
-  // this wave's share of a chunk's fragments, f = wv + 4 i, straight into LDS (lane l's 16 bytes at 16 l of the slot)
+  // this wave's share of a chunk's fragments, f = wv + 4 i, straight into LDS (lane l's 16 bytes at 16 l of the slot): four
+  // lanes take a row's 64 bytes, in an order that spreads a column of eight rows over all banks; a fragment's lane reads at
+  const int lr = lane >> 2, lh = (lane & 3) ^ ((lr >> 1) & 3);
+  const int at = 4 * r + (h ^ ((r >> 1) & 3));
   auto fetch = [&](int kb, int page, int buf) {
     const int off = kb % a.BS;
     const uint16_t* cp = a.c + (size_t)page * a.BS * RW;
@@ -186,9 +192,9 @@ __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs 
       const uint16_t* src;
       if (f < 2 * NC) {
         const int t = f / NC, cc = f - t * NC;
-        src = cp + (size_t)(off + 8 * (r >> 2) + 4 * t + (r & 3)) * RW + 32 * cc + 8 * h;
+        src = cp + (size_t)(off + 8 * (lr >> 2) + 4 * t + (lr & 3)) * RW + 32 * cc + 8 * lh;
       } else {
-        src = tp + (size_t)(16 * (f - 2 * NC) + r) * a.BS + off + 8 * h;
+        src = tp + (size_t)(16 * (f - 2 * NC) + lr) * a.BS + off + 8 * lh;
       }
       __builtin_amdgcn_global_load_lds(src, (lds_void_t*)(frag + ((size_t)buf * NF + f) * 64), 16, 0, 0);
     }
@@ -213,7 +219,7 @@ __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs 
     landed();                                                 // (and nobody reads the other buffer any more)
     if (kb + 32 < k_end) fetch(kb + 32, page, buf ^ 1);
     page = page_of(kb + 64);                                  // there with that chunk
-    const bf16x8* fb = frag + (size_t)buf * NF * 64 + lane;
+    const bf16x8* fb = frag + (size_t)buf * NF * 64 + at;
     const bool open = kb + 31 <= pos0 && (a.window <= 0 || kb >= pos0 + ntok - a.window);
     f32x4 s[MT][2];
     bf16x8 pf[MT], fr[2][kBatch];
