@@ -3,14 +3,17 @@
 // heads share a cache row of W = R + RP numbers, which is the key, and whose first R numbers are the value.
 //
 // A row's visible keys are cut into parts of 128 by their place in its own key range.  Within a part the scores of up to
-// eight heads (two where a workgroup has one part) of one key head meet in LDS -- a lane has one key and up to four heads, so that a key's numbers are read once
-// for them -- then their softmax, then a thread walks the part's keys for one value column and the heads again.  Parts are
+// eight heads (two where a workgroup has one part) of one key head meet in LDS -- four (two) lanes beside each other have a
+// key, so that they read the same 16 bytes of it, and a quarter (half) of the heads each -- then their softmax, then a thread walks the part's keys for one value column and the heads again.  Parts are
 // joined in order with fixed multiply-adds, by the workgroup itself where there are rows enough to fill the chip, by a
 // second kernel where few rows are spread over a workgroup per part: both do the same arithmetic, so a row's result does
 // not depend on how the prompt was cut or on what else is in the step.
 //
-// What bounds it: the scores (one lane reads a whole key, 16 bytes at a time) and latency at few rows, for which reason the
-// heads and the parts are spread over workgroups.  fp32, 16 heads over 2 of 128, two rows at 340 keys: 980 us (a
+// What bounds it: the scores -- lookups of the first-level cache, one for every key that four neighbouring lanes read -- and
+// latency at few rows, for which reason the heads and the parts are spread over workgroups.  622 rows of two prompts, 16
+// heads, 256 + 64 numbers and 2 key heads of 128, median of both: a lane a key, four keys in four lanes, 150 us; three
+// workgroups a compute unit by their registers and 16 values on their way 126; two lanes a key 106; four lanes a key, two
+// keys each, and four workgroups 98 (one register spilled; three without a spill 105).  fp32, 16 heads over 2 of 128, two rows at 340 keys: 980 us (a
 // workgroup per row, all heads one after the other, the scores formed twice) -> 28 us; 666 rows of two prompts: 1451 ->
 // 122 us; latent (16 heads, 256 + 64 numbers): 706 -> 39 and 719 -> 196 us.
 #include "common.h"
@@ -21,6 +24,7 @@ namespace k8s {
 constexpr int kRaKeys = 128;    // keys of a part
 constexpr int kRaHeads = 8;     // heads of a workgroup that walks all parts
 constexpr int kRaFew = 2;       // of one that has a single part
+constexpr int kRaAsk = 16;     // values of a column asked for together where a workgroup walks all parts
 
 template <typename T>
 __device__ __forceinline__ float rld(const T* p, size_t i);
@@ -80,15 +84,15 @@ __device__ __forceinline__ float ra_join_out(float o, float a, float op, float b
 // own: every value of the part is asked for before the scores, and 16 pieces of a key at a time instead of 4; and two heads a
 // workgroup, for with eight the multiply-adds and LDS reads of one compute unit are as long as the chain.  The sums are
 // those of the other form.  Reply steps of two rows at 340 keys, both forms, median of a trace: 35.8 us -> 31.3 (registers)
-// -> 16.9 (two heads).
+// -> 16.9 (two heads) -> 14.5 (two lanes a key).
 template <typename TQ, typename TC, typename TO, bool VEC, bool PART>
-__global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
+__global__ void __launch_bounds__(256, PART ? 1 : 4) rows_attn_kernel(RowsArgs p) {
   constexpr int NH = PART ? kRaFew : kRaHeads;
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int D = p.D1 + p.D2, V = p.V, hpg = p.H / (p.G * p.M);
   const int HB = min(hpg, NH), nhb = (hpg + HB - 1) / HB, nvb = (V + 255) / 256;
   float* sq = sm;                                   // [HB][D4]
-  const int D4 = (D + 3) & ~3;
+  const int D4 = ((D + 3) & ~3) + 4;                // (neighbouring heads' rows in different banks)
   float* sp = sq + HB * D4;                         // [HB][128]
   float* sl = sp + HB * kRaKeys;                    // [HB][2]: m, l of the part
   int* ss = reinterpret_cast<int*>(sl + 2 * HB);    // [128]: cache slots
@@ -138,42 +142,55 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
         for (int j = 0; j < kRaKeys; ++j) vall[j] = vbase[(size_t)ss[j] * p.vs];      // (past nk: the last one again)
       }
     }
-    {  // scores: a wave has 64 keys and every other head
-      const int x = (wv & 1) * 64 + lane, h0 = wv >> 1;
-      if ((wv & 1) * 64 < nk && h0 < nh) {
-        const TC* kp = kbase + (size_t)ss[x] * p.ks;
+    {  // scores: HL lanes beside each other have a key (KX of them), each every HL-th head
+      constexpr int HL = PART ? 2 : 4, KW = 64 / HL, KX = kRaKeys / (4 * KW), HP = NH / HL;
+      const int x = wv * KW + lane / HL, h0 = lane % HL;
+      if (wv * KW < nk && h0 < nh) {
+        const TC* kp[KX];
+#pragma unroll
+        for (int i = 0; i < KX; ++i) kp[i] = kbase + (size_t)ss[x + 4 * KW * i] * p.ks;
         const float* q0 = sq + h0 * D4;
-        const float* qh[NH / 2];
+        const float* qh[HP];
 #pragma unroll
-        for (int k = 0; k < NH / 2; ++k) qh[k] = h0 + 2 * k < nh ? q0 + 2 * k * D4 : q0;
-        float a[NH / 2] = {};
+        for (int k = 0; k < HP; ++k) qh[k] = h0 + HL * k < nh ? q0 + HL * k * D4 : q0;
+        float a[HP][KX] = {};
         if (VEC) {
-#pragma unroll (PART ? 16 : 4)
+#pragma unroll (PART ? 16 : 2)
           for (int d = 0; d < D; d += 4) {
-            const f32x4 kv = rld4(kp + d);
+            f32x4 kv[KX];
 #pragma unroll
-            for (int k = 0; k < NH / 2; ++k) {
+            for (int i = 0; i < KX; ++i) kv[i] = rld4(kp[i] + d);
+#pragma unroll
+            for (int k = 0; k < HP; ++k) {
               const f32x4 qv = *reinterpret_cast<const f32x4*>(qh[k] + d);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) a[k] = fmaf(qv[e], kv[e], a[k]);
+              for (int i = 0; i < KX; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a[k][i] = fmaf(qv[e], kv[i][e], a[k][i]);
             }
           }
         } else {
-          for (int d = 0; d < D; ++d) {
-            const float kv = rld(kp, d);
+          for (int d = 0; d < D; ++d)
 #pragma unroll
-            for (int k = 0; k < NH / 2; ++k) a[k] = fmaf(qh[k][d], kv, a[k]);
-          }
+            for (int i = 0; i < KX; ++i) {
+              const float kv = rld(kp[i], d);
+#pragma unroll
+              for (int k = 0; k < HP; ++k) a[k][i] = fmaf(qh[k][d], kv, a[k][i]);
+            }
         }
 #pragma unroll
-        for (int k = 0; k < NH / 2; ++k)
-          if (h0 + 2 * k < nh) {
-            float s = a[k] * p.scale;
-            if (p.softcap > 0.f) s = p.softcap * tanhf(s / p.softcap);
-            sp[(h0 + 2 * k) * kRaKeys + x] = x < nk ? s : -INFINITY;
-          }
+        for (int k = 0; k < HP; ++k)
+#pragma unroll
+          for (int i = 0; i < KX; ++i)
+            if (h0 + HL * k < nh) {
+              float s = a[k][i] * p.scale;
+              if (p.softcap > 0.f) s = p.softcap * tanhf(s / p.softcap);
+              const int xi = x + 4 * KW * i;
+              sp[(h0 + HL * k) * kRaKeys + xi] = xi < nk ? s : -INFINITY;
+            }
       } else if (h0 < nh) {
-        for (int h = h0; h < nh; h += 2) sp[h * kRaKeys + x] = -INFINITY;
+        for (int h = h0; h < nh; h += HL)
+          for (int i = 0; i < KX; ++i) sp[h * kRaKeys + x + 4 * KW * i] = -INFINITY;
       }
     }
     __syncthreads();
@@ -223,7 +240,15 @@ __global__ void __launch_bounds__(256) rows_attn_kernel(RowsArgs p) {
           with(j, v);
         };
         const int nk4 = nk & ~3;
-        for (int j = 0; j < nk4; j += 4) four(j, 4);
+        int j4 = 0;
+        for (; j4 + kRaAsk <= nk4; j4 += kRaAsk) {          // their values on their way together
+          float v[kRaAsk / 4][4];
+#pragma unroll
+          for (int e = 0; e < kRaAsk; ++e) v[e / 4][e % 4] = rld(vbase, (size_t)ss[j4 + e] * p.vs);
+#pragma unroll
+          for (int e = 0; e < kRaAsk; e += 4) with(j4 + e, v[e / 4]);
+        }
+        for (; j4 < nk4; j4 += 4) four(j4, 4);
         if (nk4 < nk) four(nk4, nk - nk4);
       }
 #pragma unroll
@@ -282,7 +307,7 @@ __global__ void __launch_bounds__(256) rows_attn_merge_kernel(RowsArgs p) {
 template <typename TQ, typename TC, typename TO>
 static int launch_rows(const RowsArgs& p, int T, hipStream_t s) {
   const int D = p.D1 + p.D2, hpg = p.H / (p.G * p.M), most = p.po ? kRaFew : kRaHeads, HB = hpg < most ? hpg : most;
-  const size_t lds = sizeof(float) * ((size_t)HB * ((D + 3) / 4 * 4) + HB * kRaKeys + 2 * HB + kRaKeys);
+  const size_t lds = sizeof(float) * ((size_t)HB * ((D + 3) / 4 * 4 + 4) + HB * kRaKeys + 2 * HB + kRaKeys);
   const dim3 grid(T, p.G * p.M * ((hpg + HB - 1) / HB) * ((p.V + 255) / 256), p.po ? p.n_parts : 1);
   // four numbers of a key at a time where every key starts on such a border
   const bool vec = D % 4 == 0 && p.ks % 4 == 0 && ((uintptr_t)p.kc & (4 * sizeof(TC) - 1)) == 0;

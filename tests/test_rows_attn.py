@@ -145,3 +145,21 @@ def test_infinite_keys_and_values(n, alone):
         assert torch.equal(torch.isnan(got.cpu()), torch.isnan(want[first:]))
     ok = torch.isfinite(want[first:])
     assert float((got.cpu().double() - want[first:])[ok].abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("H", [1, 2, 4, 5, 7])
+def test_keys_of_neighbouring_lanes(H):
+    """Every count of keys in a part, heads that do not fill the lanes of a key."""
+    n, D, dev = 700, 8, torch.device("cuda")
+    g = torch.Generator().manual_seed(H)
+    q, k, v = (torch.randn(n, h * D, generator=g) for h in (H, 1, 1))
+    kc, vc = torch.full((22, BS, D), math.nan), torch.full((22, BS, D), math.nan)      # (slots without a key are not read)
+    kc.view(-1, D)[:n], vc.view(-1, D)[:n] = k, v
+    seg = meta([n], [0], list(range(22)), dev)
+    got = S.masked_attention(q.to(dev), H, 1, D, D, seg=seg, kc=kc.to(dev), vc=vc.to(dev), scale=D ** -0.5)
+    rows = torch.arange(0, 270)
+    vis = torch.arange(n)[None] <= rows[:, None]
+    s = torch.einsum("thd,jd->thj", q.double().view(n, H, D)[rows], k.double()) * D ** -0.5
+    want = torch.einsum("thj,jv->thv", weights(s, vis[:, None], None), v.double())
+    # fp32 sums of 8 and up to 270 terms
+    assert float((got.cpu().double().view(n, H, D)[rows] - want).abs().max()) < 2e-5 * float(want.abs().max())
