@@ -9,7 +9,7 @@
 // waves and parts follow from positions alone, so a row's bits do not depend on the step it is in.
 //
 // What bounds it: the chain row -> page -> keys -> scores -> join of some 5 us, and that one compute unit takes cold keys
-// in at 20 to 30 KB a us, far below its share of the caches' rate.  So parts are small (256 masked or 128 latent keys: 128
+// in at 20 to 30 KB a us (as fragments; tok_turn), far below its share of the caches' rate.  So parts are small (256 masked or 128 latent keys: 128
 // KB of keys and values and 144 KB), and a merge of 3.5 us pays from the second part on.  16 heads over 2 of 128 / 16 heads
 // over latents of 256 + 64, us with the merge, and in brackets what a tile of 16 tokens per wave (masked) and a wave per 256
 // keys (latent) took in engine steps of about that size: 1 row at 100 keys 5.3 / 8.5 (8.4 / 13.5), 8 rows at 1500 10.7 / 12.5 (26 / 36),
@@ -178,6 +178,20 @@ __global__ void __launch_bounds__(256) token_merge_kernel(TokOut a, const int* _
 
 __device__ __forceinline__ bf16x8 tld16(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
+// Keys and values are loaded with lane 4 r + h at piece h of row r, so that four lanes beside each other read 64 bytes of a
+// line; the fragment wants them in lane 16 h + r (from: 4 (4 r + h), the byte address of the lane that has this lane's).
+// Loaded where the fragment wants them, four neighbours read four rows and each is a lookup of its own in the first-level
+// cache: in reply steps 7 rows at 800 keys 8.7 -> 6.7 us masked, 9.6 -> 7.9 latent, 5 rows at 1200 8.5 -> 7.1; one row and
+// 64 rows at 512 as before (4.4 - 6, 12.6, 15 us).
+__device__ __forceinline__ bf16x8 tok_turn(bf16x8 v, int from) {
+  int w[4];
+  __builtin_memcpy(w, &v, 16);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_ds_bpermute(from, w[i]);
+  __builtin_memcpy(&v, w, 16);
+  return v;
+}
+
 // Scores p[8] (log2 units, keys 8 h .. 8 h + 7 of head lane & 15; -inf: not seen) -> the running maximum and sum, the
 // weights as the value product's operand; the output is rescaled only where a head's maximum moved.
 template <int ND>
@@ -268,20 +282,21 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
     pgv = k + lane < my ? pages[pi] : 0;
   };
   fill(0);
+  const int lr = lane >> 2, lh = lane & 3, from = 4 * (4 * r + hq);
   bf16x8 kf[2][2][NDC], vf[2][NV];
   int kb[2];
   auto load = [&](int u, int k) {
     if (k - base == 64) fill(k);
     kb[u] = __shfl(kbv, k - base, 64);
     const int page = __shfl(pgv, k - base, 64), off = __shfl(ofv, k - base, 64);
-    const uint16_t* kp = a.kc + ((size_t)page * a.BS + off) * NK + g * D + 8 * hq;
+    const uint16_t* kp = a.kc + ((size_t)page * a.BS + off) * NK + g * D + 8 * lh;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int cc = 0; cc < NDC; ++cc) kf[u][t][cc] = tld16(kp + (size_t)(8 * (r >> 2) + 4 * t + (r & 3)) * NK + 32 * cc);
-    const uint16_t* vp = a.vt + ((size_t)page * NVt + (size_t)gv * V) * a.BS + off + 8 * hq;
+      for (int cc = 0; cc < NDC; ++cc) kf[u][t][cc] = tld16(kp + (size_t)(8 * (lr >> 2) + 4 * t + (lr & 3)) * NK + 32 * cc);
+    const uint16_t* vp = a.vt + ((size_t)page * NVt + (size_t)gv * V) * a.BS + off + 8 * lh;
 #pragma unroll
-    for (int dt = 0; dt < NV; ++dt) vf[u][dt] = tld16(vp + (size_t)(16 * dt + r) * a.BS);
+    for (int dt = 0; dt < NV; ++dt) vf[u][dt] = tld16(vp + (size_t)(16 * dt + lr) * a.BS);
   };
   if (my > 0) load(0, 0);
   if (my > 1) load(1, 1);
@@ -295,7 +310,7 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
       for (int t = 0; t < 2; ++t) {
         f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int cc = 0; cc < NDC; ++cc) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[u][t][cc], qf[cc], s, 0, 0, 0);
+        for (int cc = 0; cc < NDC; ++cc) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tok_turn(kf[u][t][cc], from), qf[cc], s, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) p[4 * t + i] = s[i];
       }
@@ -313,7 +328,7 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
       bf16x8 pf;
       tok_softmax<NV>(p, hq, m, l, o, pf);
 #pragma unroll
-      for (int dt = 0; dt < NV; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, vf[u][dt], o[dt], 0, 0, 0);
+      for (int dt = 0; dt < NV; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, tok_turn(vf[u][dt], from), o[dt], 0, 0, 0);
       if (k + u + 2 < my) load(u, k + u + 2);
     }
   }
@@ -365,16 +380,17 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
 #pragma unroll
   for (int dt = 0; dt < ND; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int* pages = a.bt + (size_t)sg * a.maxb;
+  const int lr = lane >> 2, lh = lane & 3, from = 4 * (4 * r + hq);
   for (int b = wv; b < nb; b += NW) {
     const int kb = kb0 + 32 * b, page = pages[kb / a.BS], off = kb % a.BS;
     const uint16_t* cp = a.c + (size_t)page * a.BS * RW;
-    const uint16_t* tp = a.ct + (size_t)page * R * a.BS + (size_t)r * a.BS + off + 8 * hq;
+    const uint16_t* tp = a.ct + (size_t)page * R * a.BS + (size_t)lr * a.BS + off + 8 * lh;
     bf16x8 kf[2][NC], vf[ND];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc)
-        kf[t][cc] = tld16(cp + (size_t)(off + 8 * (r >> 2) + 4 * t + (r & 3)) * RW + 32 * cc + 8 * hq);
+        kf[t][cc] = tld16(cp + (size_t)(off + 8 * (lr >> 2) + 4 * t + (lr & 3)) * RW + 32 * cc + 8 * lh);
 #pragma unroll
     for (int dt = 0; dt < NH; ++dt) vf[dt] = tld16(tp + (size_t)(16 * dt) * a.BS);
     float p[8];
@@ -382,7 +398,7 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
     for (int t = 0; t < 2; ++t) {
       f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][cc], qf[cc], s, 0, 0, 0);
+      for (int cc = 0; cc < NC; ++cc) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tok_turn(kf[t][cc], from), qf[cc], s, 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int key = kb + 8 * hq + 4 * t + i;
@@ -395,7 +411,7 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
     bf16x8 pf;
     tok_softmax<ND>(p, hq, m, l, o, pf);
 #pragma unroll
-    for (int dt = 0; dt < ND; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, vf[dt], o[dt], 0, 0, 0);
+    for (int dt = 0; dt < ND; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, tok_turn(vf[dt], from), o[dt], 0, 0, 0);
   }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
