@@ -419,6 +419,7 @@ class FikeraxModel:
         :meth:`state_spec`.  ``layers_out`` (debugging): receives the residual after every layer run."""
         cfg, eps, dt = self.cfg, self.cfg.norm_eps, self.dtype
         T, one = inp.input_ids.shape[0], self.one
+        idx = S.wanted_rows(inp)
         mix1 = one.view(1, 1)
         tables: Dict[int, torch.Tensor] = {}
         again = (inp.input_ids, self.embed, cfg.embed_scale)
@@ -431,7 +432,7 @@ class FikeraxModel:
             if r + 1 < len(self.runs):
                 j, add = self.runs[r + 1]
                 nxt = dict(nw=self.layers[j]["norm1"], again=again if add else None)
-            elif inp.logits_idx is None:                   # every row is wanted: the last write-back reads the head's input
+            elif idx is None:                              # every row is wanted: the last write-back reads the head's input
                 nxt = dict(nw=self.final_norm)
             rms = None                                     # what the residual's pass makes up for behind the projection
             if spec.kind == "lightning":
@@ -462,8 +463,8 @@ class FikeraxModel:
                 h = R.step(x, y, one, mix1, eps=eps, out_dtype=dt, rms=rms, **nxt)
             else:
                 N.hyper_step(x, y, one, mix1, rms=rms)
-        if inp.logits_idx is not None:
-            h = N.hyper_read(x, inp.logits_idx, self.final_norm, eps, dt)
+        if idx is not None:
+            h = N.hyper_read(x, idx, self.final_norm, eps, dt)
             return proj_f32out(h, self.head)
         return R.proj_f32out(h, self.head)
 

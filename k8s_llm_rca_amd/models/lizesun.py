@@ -434,6 +434,7 @@ class LizesunModel:
         :meth:`state_spec`.  ``layers_out`` (debugging): receives a copy of the residual after every layer."""
         cfg, dt = self.cfg, self.dtype
         T, W, nl = inp.input_ids.shape[0], cfg.hidden, cfg.n_layers
+        idx = S.wanted_rows(inp)
         x = torch.empty(T, W, dtype=torch.float32, device=self.device)
         first = self.layers[0]["norm1"] if nl else (1.0, None, None)
         h = N.embed_scale_dyt(inp.input_ids, self.embed, cfg.embed_scale, x, *first, out_dtype=dt)
@@ -442,7 +443,7 @@ class LizesunModel:
         for li, (spec, L) in enumerate(zip(cfg.layers, self.layers)):
             # (the final norm reads the wanted rows only, or with the last layer where every row is wanted)
             nxt = (self.layers[li + 1]["norm1"] if li + 1 < nl
-                   else (1.0, None, None) if inp.logits_idx is not None else self.final_norm)
+                   else (1.0, None, None) if idx is not None else self.final_norm)
             after = L["norm2"] if spec.ff else nxt
             if spec.kind == "parallel":
                 ol, orr = self._parallel(li, h, inp, kcs, vcs, vts, states, tables)
@@ -464,8 +465,8 @@ class LizesunModel:
                 if isinstance(h, R.RowStep):
                     h = h.read()                                       # the residual as it is behind this layer
                 layers_out.append(x.clone())
-        if inp.logits_idx is not None or not nl:
-            xr = x.index_select(0, inp.logits_idx).contiguous() if inp.logits_idx is not None else x
+        if idx is not None or not nl:
+            xr = x.index_select(0, idx).contiguous() if idx is not None else x
             h = N.add_dyt(xr, None, 1.0, None, 1.0, *self.final_norm, out_dtype=dt)
         return R.proj_f32out(h, self.lm_head)
 

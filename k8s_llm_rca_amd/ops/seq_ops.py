@@ -642,6 +642,13 @@ class SegStepInputs:
     logits_idx: Optional[torch.Tensor]   # [n] int64 rows whose logits are needed (None, captured steps: every row, in order)
 
 
+def wanted_rows(inp: SegStepInputs) -> Optional[torch.Tensor]:
+    """``logits_idx``, or None where that is every row: with one row the head may take another product than behind a row that
+    was picked (ops/row_step.py), and a step's bits are the same captured (None) and not."""
+    idx = inp.logits_idx
+    return None if idx is not None and inp.input_ids.shape[0] == 1 == idx.numel() else idx
+
+
 def short_conv(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], tail: torch.Tensor, seg: SegMeta,
                act: bool = True) -> torch.Tensor:
     """Causal per-channel convolution with bias and SiLU: ``out_t = act(b + sum_j w[:, j] x_(t - taps + 1 + j))``

@@ -2,9 +2,12 @@
 import pytest
 import torch
 
+from k8s_llm_rca_amd.engine.engine import EngineConfig, LLMEngine
+from k8s_llm_rca_amd.models.registry import get_any_config
 from k8s_llm_rca_amd.ops import linear as L
 from k8s_llm_rca_amd.ops import norm as N
 from k8s_llm_rca_amd.ops import row_step as R
+from k8s_llm_rca_amd.ops import seq_ops as S
 
 BF = torch.bfloat16
 gpu = pytest.mark.gpu
@@ -151,3 +154,32 @@ def test_captured_and_repeated():
         g.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(out, eager))
+
+
+def test_the_only_row_is_every_row():
+    def rows(t, idx):
+        ids = torch.zeros(t, dtype=torch.int32)
+        return S.wanted_rows(S.SegStepInputs(ids, ids, ids, None, idx))
+
+    some = torch.tensor([0])
+    assert rows(1, some) is None and rows(1, None) is None and rows(2, None) is None
+    assert rows(2, some) is some and rows(1, some[:0]) is not None and rows(1, some.repeat(2)).numel() == 2
+
+
+@gpu
+@pytest.mark.parametrize("model", ["fikerax-1b", "lizesun-1b"])
+def test_one_row_has_the_same_bits_captured_and_not(model):
+    """At widths that the kernel takes: the head behind the last pass, and behind the row picked from the residual."""
+    over = {"layers": get_any_config(model).layers[:3]} if model == "lizesun-1b" else {}
+
+    def logits(graphs):
+        eng = LLMEngine(EngineConfig(model=model, model_overrides=over, device="cuda", dtype=BF, num_blocks=16, block_size=64,
+                                     max_context=512, state_slots=2, use_graphs=graphs, prefix_sharing=False, seed=3))
+        sid = eng.new_sequence()
+        out = [eng.feed([(sid, [5, 6, 7], [2])])] + [eng.feed([(sid, [11 * i], [0])]).clone() for i in range(8)]
+        torch.cuda.synchronize()
+        return out, eng.stats["graph_steps"]
+
+    (want, none), (got, some) = logits(False), logits(True)
+    assert not none and some >= 4
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
