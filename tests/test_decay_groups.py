@@ -16,9 +16,22 @@ def test_ranges():
             assert S._lin_rows(5000, n_seg, H, 128, 200) % 64 == 0
 
 
+def test_ranges_follow_the_lengths():
+    """However many short portions are beside it, a long one is cut as it is alone."""
+    def rows(lens, H=16):
+        return S._lin_rows(sum(lens), len(lens), H, 128, 128, max(lens))
+
+    assert rows([4000]) == rows([1] * 15 + [4000]) == rows([1] * 63 + [4000]) == 256
+    assert rows([4000] + [40] * 15) == 320 and rows([1] * 3 + [4000]) == 256
+    assert 0 < rows([512] * 63 + [4096]) < 4096 and 0 < rows([512] * 31 + [2048]) < 2048
+    assert rows([1024] * 16) == rows([512] * 15 + [1024]) == rows([1] * 32 + [300]) == 0      # nothing to wait for
+    assert rows([1000] * 4) == 256 and rows([1000] * 5) == 192                               # two workgroups a unit
+    assert rows([1] * 15 + [512], 64) == 0 and rows([1] * 15 + [768], 64) == 256
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("lens,V,silu", [([70] * 18, 128, False), ([64, 1, 130, 65] * 5, 128, True), ([300] * 6, 128, False),
-                                         ([129] * 9, 144, True), ([600] * 4, 128, True)])
+                                         ([129] * 9, 144, True), ([600] * 5, 128, True), ([1] * 15 + [900], 128, True)])
 def test_more_than_a_workgroup_a_unit(lens, V, silu):
     H, D, dev = 16, 128, "cuda"
     g = torch.Generator().manual_seed(sum(lens) + V)
@@ -33,7 +46,7 @@ def test_more_than_a_workgroup_a_unit(lens, V, silu):
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
     seg = S.SegMeta(n, i32([s for s, k in enumerate(lens) for _ in range(k)]), i32(row0), i32(pos0), i32(list(range(n))),
                     i32([[0]] * n), row0, pos0, list(range(n)))
-    rows = S._lin_rows(T, n, H, D, V)
+    rows = S._lin_rows(T, n, H, D, V, max(lens))
     groups = (sum(-(-k // rows) for k in lens) if rows and max(lens) > rows else n) * H * -(-V // 128)
     assert groups > 256
     state = start.to(dev)
