@@ -775,9 +775,10 @@ K8S_API int k8s_gemm_stream_part(const void* x, int ldx, const void* w, void* y,
   return stream_launch(x, ldx, w, y, ldy, M, N, K, cfg, splits, part, false, s);
 }
 
-// y[M][N] (bf16) = the sum of fp32 planes [splits][M][N].
+// y[M][N] (bf16) = the sum of fp32 planes [splits][M][N]; 16-byte loads and stores.
 K8S_API int k8s_gemm_stream_reduce(const float* part, int splits, void* y, int ldy, int M, int N, hipStream_t s) {
-  if (M <= 0 || N <= 0 || N % 8 || ldy < N || ldy % 8 || splits < 1 || !part) return (int)hipErrorInvalidValue;
+  if (M <= 0 || N <= 0 || N % 8 || ldy < N || ldy % 8 || splits < 1 || !part || !y || (((uintptr_t)part | (uintptr_t)y) & 15))
+    return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(gemm_stream_reduce_kernel, dim3((M * N / 8 + 255) / 256), dim3(256), 0, s, part, splits, (uint16_t*)y,
                      ldy, M, N);
   return (int)hipGetLastError();

@@ -103,12 +103,13 @@ def gemm_rows(x: torch.Tensor, w: torch.Tensor, nf: int, out_kind: int = ROWS_BF
 
 
 def select_gemm(M: int, N: int, K: int, x_ok_layout: bool = True, out_contig: bool = True,
-                rows: bool = True) -> Tuple[int, int, int]:
+                rows: bool = True, out_wide: bool = True) -> Tuple[int, int, int]:
     """(kind, cfg, splits) :func:`linear` runs for a contiguous bf16 ``x`` [M, K]
     and ``w`` [N, K] on the GPU -- the measured dispatch table first, then the
     row-streaming kernel and the skinny kernel's default range, else hipBLASLt.  Also used by the native
     layer executor (ops/layer_exec.py) so both paths pick the same kernel.
-    ``rows``: x and w lie as the row-streaming kernel needs them."""
+    ``rows``: x and w lie as the row-streaming kernel needs them; ``out_wide``: the result can be stored by 16 bytes, as the
+    sum of K ranges is."""
     forced_skinny = False
     rows = rows and x_ok_layout
     if _dispatch and M <= DISPATCH_MAX_M:
@@ -121,7 +122,7 @@ def select_gemm(M: int, N: int, K: int, x_ok_layout: bool = True, out_contig: bo
                 return KIND_GRP, 0, splits
             if kind == "stream" and x_ok_layout and out_contig and stream_shape_ok(M, N, K, cfg, splits):
                 return KIND_STREAM, cfg, splits
-            if kind == "rows" and rows and rows_shape_ok(M, N, K, cfg, splits):
+            if kind == "rows" and rows and (splits == 1 or out_wide) and rows_shape_ok(M, N, K, cfg, splits):
                 return KIND_ROWS, cfg, splits
             if kind == "lib":
                 return KIND_LIB, 0, 1
@@ -169,7 +170,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torch.
             return out
         return lib_gemm(x, w, out)
     layout = x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
-    kind, cfg, splits = select_gemm(M, N, K, layout, out is None or out.is_contiguous(), rows_ok(x, w) and (out is None or out.stride(1) == 1))
+    rows = rows_ok(x, w) and (out is None or out.stride(1) == 1)
+    wide = out is None or out.stride(0) % 8 == 0 == out.data_ptr() % 16
+    kind, cfg, splits = select_gemm(M, N, K, layout, out is None or out.is_contiguous(), rows, wide)
     if kind == KIND_ROWS:
         if splits == 1:
             return gemm_rows(x, w, cfg, out=out)

@@ -159,6 +159,29 @@ def test_operands_the_kernel_cannot_read_go_elsewhere():
 
 
 @gpu
+@pytest.mark.parametrize("m", [24, 32])
+@pytest.mark.parametrize("ld,first", [(512, 0), (519, 0), (520, 0), (520, 4)])
+def test_sums_of_ranges_only_where_they_can_be_stored(m, ld, first, monkeypatch):
+    """A table's K ranges end in 16-byte stores: a result with other rows or another start is left to another kernel."""
+    n, k = 512, 1024
+    monkeypatch.setitem(L._dispatch, (n, k), [(32, "rows", 2, 2)])
+    x, w = operands(m, n, k)
+    want = x.double() @ w.double().T
+    buf = torch.full((m * ld + 16,), 7.0, device="cuda", dtype=BF)
+    out = buf[first:first + m * ld].view(m, ld)[:, :n]
+    ranges = ld % 8 == 0 == first % 8
+    assert (L.select_gemm(m, n, k, True, True, True, ranges) == (L.KIND_ROWS, 2, 2)) == ranges
+    L.linear(x, w, out=out)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
+    kept = torch.ones_like(buf, dtype=torch.bool)
+    kept[first:first + m * ld].view(m, ld)[:, :n] = False
+    assert bool((buf[kept] == 7.0).all())
+    part = torch.zeros(2, m, n, device="cuda")
+    s = stream_ptr(x)
+    assert (lib().k8s_gemm_stream_reduce(ptr(part), 2, ptr(out), ld, m, n, s) == 0) == ranges
+
+
+@gpu
 def test_executor_with_the_norms_in_front_of_both_products():
     """One and two rows: the norm in front of the rotated and the gated product, the latter on the widest strips (whatever the
     table says); three and four: apart.  The same bits as all apart, and as without the executor."""
