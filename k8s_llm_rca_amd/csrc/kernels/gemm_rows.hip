@@ -232,9 +232,12 @@ static int rows_launch(const void* x, int ldx, const void* w, void* y, int ldy, 
                        const RowsRope& rp, const NormIn& nin, hipStream_t s) {
   const bool halves = out == kRowsSilu || out == kRowsRope;
   const int strip = (halves ? 8 : 16) * NF, cols = out == kRowsRope ? N / 2 : N;   // rope: columns counted as pairs
-  if (M <= 0 || M > 16 * MT || (NORM && M > kNormMaxRows) || N <= 0 || N % (out == kRowsRope ? 128 : 1) || cols % strip || ranges < 1 || ldx % 8 || K <= 0 ||
-      K % (ranges * kRowsWaves * CH) || (ranges > 1 && out != kRowsF32) || ldy < N || (ranges > 1 && ldy != N))
+  if (M <= 0 || M > 16 * MT || (NORM && M > kNormMaxRows) || N <= 0 || N % (out == kRowsRope ? 128 : 1) || cols % strip ||
+      ranges < 1 || K <= 0 || K % (ranges * kRowsWaves * CH) || (ranges > 1 && out != kRowsF32) || ldy < N ||
+      (ranges > 1 && ldy != N) || !w || !y || ((uintptr_t)w & 15))
     return (int)hipErrorInvalidValue;
+  if (!NORM && (!x || ((uintptr_t)x & 15) || ldx % 8 || (M > 1 && ldx < K))) return (int)hipErrorInvalidValue;
+  if (out == kRowsRope && rp.slots && (!rp.kc || !rp.vc)) return (int)hipErrorInvalidValue;
   const dim3 g(cols / strip, ranges), b(kRowsWaves * 64);
   const size_t lds = NORM ? (size_t)M * K * 2 : 0;
 #define K8S_ROWS(OUT)                                                                                                   \
@@ -286,7 +289,7 @@ using namespace k8s;
 
 // nf: 16-row fragments of a workgroup, 1 (up to 16 rows), 2 or 4; ranges > 1: fp32 planes [ranges][M][N].
 // out: 0 bf16, 1 fp32, 2 silu(x . w[0:N]^T) * (x . w[N:2N]^T), 3 max(., 0)^2.  K: whole chunks for each of four waves
-// (128 entries, 64 where nf is 4 or there are more than 16 rows).
+// (128 entries, 64 where nf is 4 or there are more than 16 rows).  x (its rows too) and w lie on 16 bytes.
 K8S_API int k8s_gemm_rows(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int nf, int ranges,
                           int out, hipStream_t s) {
   if (out < kRowsBf16 || out > kRowsRelu2) return (int)hipErrorInvalidValue;
@@ -309,7 +312,9 @@ K8S_API int k8s_gemm_rows_norm(const void* x, int x_stride, const float* part, i
                                const void* norm_w, float eps, const void* w, void* y, int ldy, int M, int N, int K, int nf,
                                const int* pos, const float* cos_sin, const int* slots, void* kc, void* vc, int nq, int nkv,
                                int BS, hipStream_t s) {
+  auto off = [](const void* p) { return ((uintptr_t)p & 15) != 0; };
   if (M <= 0 || M > kNormMaxRows || K % 8 || K / 8 > 256 * kNormMaxChunks || !norm_w || (!x && !part) ||
+      off(x) || off(part) || off(res_in) || off(res_out) || off(norm_w) || (!part && (x_stride % 8 || (M > 1 && x_stride < K))) ||
       (part && (splits < 1 || !res_in)) || (res_in && (!res_out || res_out == res_in)) ||
       (pos && (N != (nq + 2 * nkv) * 128 || !cos_sin || BS <= 0)))
     return (int)hipErrorInvalidValue;

@@ -876,13 +876,14 @@ def _big_pick(M: int, N: int, K: int, silu: bool = False) -> int:
 _stream_silu = KNOBS.stream_silu
 
 
-def swiglu_choice(M: int, N2: int, K: int):
+def swiglu_choice(M: int, N2: int, K: int, rows: bool = True):
     """(kind, cfg, splits) of the SwiGLU-epilogue gate_up GEMM for ``M`` rows of
-    a [N2 = 2I, K] gate_up weight, or ``None`` (gate_up GEMM + silu_mul)."""
+    a [N2 = 2I, K] gate_up weight, or ``None`` (gate_up GEMM + silu_mul).
+    ``rows``: as in :func:`select_gemm`."""
     if _big_pick(M, N2, K, silu=True):
         return KIND_BIG, BIG_PIPE, 1
     if _stream_silu and _dispatch and M <= DISPATCH_MAX_M and (N2 // 2) % 64 == 0:
-        kind, cfg, splits = select_gemm(M, N2, K)
+        kind, cfg, splits = select_gemm(M, N2, K, rows=rows)
         if kind == KIND_STREAM and splits == 1:
             return KIND_STREAM, cfg, 1
         if kind == KIND_ROWS and splits == 1 and (N2, K) in _dispatch and rows_shape_ok(M, N2 // 2, K, cfg, 1, ROWS_SILU):
@@ -909,7 +910,7 @@ def swiglu_gemm(y: torch.Tensor, w_gu: torch.Tensor):
     if not (y.is_cuda and y.dtype == torch.bfloat16 and y.stride(1) == 1 and y.stride(0) % 8 == 0
             and w_gu.is_contiguous()):
         return None
-    ch = swiglu_choice(M, w_gu.shape[0], K)
+    ch = swiglu_choice(M, w_gu.shape[0], K, rows_ok(y, w_gu))
     if ch is None:
         return None
     if ch[0] == KIND_BIG:

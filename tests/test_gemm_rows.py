@@ -159,6 +159,31 @@ def test_operands_the_kernel_cannot_read_go_elsewhere():
 
 
 @gpu
+def test_gated_operands_the_kernel_cannot_read_go_elsewhere(monkeypatch):
+    """The gated form of a table entry, on operands that do not start on 16 bytes; and what the entry points refuse."""
+    m, i, k = 5, 256, 1024
+    monkeypatch.setitem(L._dispatch, (2 * i, k), [(32, "rows", 2, 1)])
+    x, w = operands(m, 2 * i, k)
+    assert L.swiglu_choice(m, 2 * i, k) == (L.KIND_ROWS, 2, 1) and L.swiglu_gemm(x, w) is not None
+    want = L.glu_proj(x, w)
+    odd = torch.empty(m, k + 8, device="cuda", dtype=BF)[:, 4:k + 4]
+    odd.copy_(x)
+    flat = torch.empty(2 * i * k + 4, device="cuda", dtype=BF)[4:].view(2 * i, k)
+    flat.copy_(w)
+    for a, b in ((odd, w), (x, flat)):
+        assert L.swiglu_gemm(a, b) is None
+        # the plain product's sums in another order: a bf16 bit of gate and up
+        assert torch.allclose(L.glu_proj(a, b).float(), want.float(), rtol=2.0 ** -6, atol=2.0 ** -9)
+    s, y = stream_ptr(x), torch.empty(m, 2 * i, device="cuda", dtype=BF)
+    ok = [ptr(x), k, ptr(w), ptr(y), 2 * i, m, 2 * i, k, 2, 1, 0, s]
+    assert lib().k8s_gemm_rows(*ok) == 0
+    for at, bad in ((0, None), (0, ptr(odd)), (1, k - 8), (1, k + 4), (2, None), (2, ptr(flat)), (3, None), (4, 2 * i - 16)):
+        assert lib().k8s_gemm_rows(*ok[:at], bad, *ok[at + 1:]) != 0
+    one = ok[:5] + [1] + ok[6:]
+    assert lib().k8s_gemm_rows(*one[:1], 0, *one[2:]) == 0                 # one row has no stride
+
+
+@gpu
 @pytest.mark.parametrize("m", [24, 32])
 @pytest.mark.parametrize("ld,first", [(512, 0), (519, 0), (520, 0), (520, 4)])
 def test_sums_of_ranges_only_where_they_can_be_stored(m, ld, first, monkeypatch):
