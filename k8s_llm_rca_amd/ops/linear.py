@@ -47,12 +47,19 @@ def rows_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = False
     """(16-row fragments of a workgroup, K ranges) with which the row-streaming kernel takes a product, or None: another
     kernel is the quicker one or the shape does not fit.  ``N``: result columns; ``planes``: K ranges may stay apart.
 
-    Up to 16 rows it is the quickest at all sizes from 128 x 512 to 128256 x 4096, at 0.53 to 0.97 of the time before with
-    cold weights, but for one row of a K of 8192 (bf16 of 4096 / 8192 / 16384 columns 14.4 / 26.6 / 49.8 us before, 15.1 /
-    29.0 / 56.6), which the skinny kernel keeps.  Up to 32 rows X is half of what it reads: from 8192 columns on (us at 32
-    rows before / this: 8192 x 2048 10.3 / 9.0, 16384 x 4096 42.0 / 26.9; 4096 x 2048 9.2 / 10.0 in fp32, 4096 x 8192 20.8 /
-    26.8), and of these not where K is 1536 or 3072, at which the library is at its best (28672 x 3072 46.2 / 49.6); planes
-    up to a K of 2048 (2048 x 2048 with the pass behind 0.93, 2560 x 4096 1.10, 1088 x 8192 1.06 of the time before).
+    Up to 16 rows it is the quickest at the sizes from 128 x 512 to 128256 x 4096, at 0.53 to 0.97 of the time before with
+    cold weights.  Up to 32 rows X is half of what it reads: from 8192 columns on (us at 32 rows before / this: 8192 x 2048
+    10.3 / 9.0, 16384 x 4096 42.0 / 26.9; 4096 x 2048 9.2 / 10.0 in fp32, 4096 x 8192 20.8 / 26.8), and of these where K is
+    up to 1024 or a multiple of 2048 (1280 to 3584 0.61 to 1.07 of the time before, by shape); planes up to a K of 2048
+    (2048 x 2048 with the pass behind 0.93, 2560 x 4096 1.10, 1088 x 8192 1.06 of the time before); and not past 40960
+    columns of a K from 8192 on with 25 rows or more, where X is most of it (57344 x 8192 188 / 202, gated 57344 x 12288 280 / 299).
+
+    Rows of W that are a multiple of 16 KB apart, and no others, cost up to a third of the rate until there are columns
+    enough (they likely fall on few of the memory's channels).  us before / this at a K of 7168, 8192, 8704 and one row 48.6 /
+    38.5, 52.1 / 57.9, 62.3 / 46.0 (16384 columns);  at 32 rows of 8192 x 8192 31.4 / 35.2, 16384 x 8192 54.7 / 67.5, 28672 x
+    8192 115 / 100, 16384 x 16384 96.7 / 119.6, 28672 x 16384 167 / 175;  at 8 rows of 8192 x 16384 56.5 / 61.4, 16384 x 8192
+    67.6 / 56.1, 8192 x 8192 30.8 / 31.3.  So one row of a K of 8192 stays with the skinny kernel, a K of 16384 and, past 16
+    rows, of 8192 with the library up to three times as many columns.
 
     The fragments and ranges are those of the least work on the busiest compute unit: a workgroup streams 16 nf x K / ranges
     weights and X of M rows (2.5 % of a fragment's time each row), and 256 of them run at once.  Four fragments, whose loads
@@ -65,6 +72,10 @@ def rows_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = False
     if M > 16 and not ((K <= 1024 or K % 2048 == 0) and (K <= 2048 if planes else big >= 8192)):
         return None
     if M == 1 and K == 8192 and out != ROWS_F32:
+        return None
+    if K % (8192 if M > 16 else 16384) == 0 and 8192 <= big < 3 * K and (M > 1 or out == ROWS_F32):
+        return None
+    if M > 24 and K >= 8192 and big > 40960:
         return None
     strips = -(-big // (16 if M <= 16 else 32))
     cut = planes and (K > 1024 or M > 16) and 4 * strips < 3 * 256 * -(-strips // 256)

@@ -142,6 +142,20 @@ def test_rule_gives_what_the_kernel_takes():
     assert L.rows_plan(1, 8192, 8192) is None and L.rows_plan(24, 4096, 4096) is None and L.rows_plan(24, 8192, 2048)
 
 
+def test_rows_of_weights_on_the_same_channels():
+    """A K of 16 KB a row: another kernel is the quicker one until the columns are many; neighbouring K are taken."""
+    for out in (L.ROWS_BF16, L.ROWS_F32, L.ROWS_RELU2):
+        for m in (17, 24, 32):
+            assert L.rows_plan(m, 8192, 8192, out) is None and L.rows_plan(m, 16384, 8192, out) is None
+            assert L.rows_plan(m, 28672, 8192, out) and L.rows_plan(m, 16384, 6144, out) and L.rows_plan(m, 16384, 10240, out)
+            assert L.rows_plan(m, 28672, 16384, out) is None
+        assert L.rows_plan(8, 16384, 8192, out) and L.rows_plan(8, 4096, 16384, out)
+        assert L.rows_plan(8, 8192, 16384, out) is None and L.rows_plan(16, 28672, 16384, out) is None
+    assert L.rows_plan(32, 8192, 8192, L.ROWS_SILU) is None and L.rows_plan(32, 14336, 8192, L.ROWS_SILU)
+    assert L.rows_plan(1, 8192, 16384) and L.rows_plan(1, 8192, 16384, L.ROWS_F32) is None
+    assert L.rows_plan(24, 57344, 8192) and L.rows_plan(25, 57344, 8192) is None
+
+
 @gpu
 def test_operands_the_kernel_cannot_read_go_elsewhere():
     """Rows that do not start on 16 bytes, a transposed weight: the same values as before, by another kernel."""
