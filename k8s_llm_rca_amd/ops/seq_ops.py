@@ -901,7 +901,8 @@ def _lin_rows(T: int, n_seg: int, H: int, D: int, V: int, longest: Optional[int]
     per, groups = H * -(-V // 128), LIN_GROUPS
     longest = -(-T // n_seg) if longest is None else longest
     if D == 128 and V > 64:
-        if n_seg * per >= LIN_GROUPS and longest <= T * per // LIN_GROUPS + LIN_WALK[n_seg * per > 2 * LIN_GROUPS]:
+        past = longest - LIN_WALK[n_seg * per > 2 * LIN_GROUPS]
+        if n_seg * per >= LIN_GROUPS and past * LIN_GROUPS <= T * per:
             return 0
         groups *= 2 if T >= 5 * longest else 1
     return max(LIN_CHUNK, -(-T // (64 * max(1, groups // per))) * 64)
