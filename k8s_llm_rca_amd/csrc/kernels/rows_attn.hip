@@ -3,28 +3,29 @@
 // heads share a cache row of W = R + RP numbers, which is the key, and whose first R numbers are the value.
 //
 // A row's visible keys are cut into parts of 128 by their place in its own key range.  Within a part the scores of up to
-// eight heads (two where a workgroup has one part) of one key head meet in LDS -- four (two) lanes beside each other have a
-// key, so that they read the same 16 bytes of it, and a quarter (half) of the heads each -- then their softmax, then a thread walks the part's keys for one value column and the heads again.  Parts are
-// joined in order with fixed multiply-adds, by the workgroup itself where there are rows enough to fill the chip, by a
-// second kernel where few rows are spread over a workgroup per part: both do the same arithmetic, so a row's result does
-// not depend on how the prompt was cut or on what else is in the step.
+// eight heads (two where workgroups are few) of one key head meet in LDS -- four (two) lanes beside each other have a
+// key, so that they read the same 16 bytes of it, and a quarter (half) of the heads each -- then their softmax, then a
+// thread walks the part's keys for one value column and the heads again.  Parts are joined in order with fixed
+// multiply-adds, by the workgroup itself where there are rows enough to fill the chip, by a second kernel where few rows are
+// spread over a workgroup per part: both do the same arithmetic, so a row's result does not depend on how the prompt was cut
+// or on what else is in the step.
 //
 // What bounds it: the scores -- lookups of the first-level cache, one for every key that four neighbouring lanes read -- and
 // latency at few rows, for which reason the heads and the parts are spread over workgroups.  622 rows of two prompts, 16
 // heads, 256 + 64 numbers and 2 key heads of 128, median of both: a lane a key, four keys in four lanes, 150 us; three
 // workgroups a compute unit by their registers and 16 values on their way 126; two lanes a key 106; four lanes a key, two
-// keys each, and four workgroups 98 (one register spilled; three without a spill 105).  fp32, 16 heads over 2 of 128, two rows at 340 keys: 980 us (a
-// workgroup per row, all heads one after the other, the scores formed twice) -> 28 us; 666 rows of two prompts: 1451 ->
-// 122 us; latent (16 heads, 256 + 64 numbers): 706 -> 39 and 719 -> 196 us.
+// keys each, and four workgroups 98 (one register spilled; three without a spill 105).  fp32, 16 heads over 2 of 128, two
+// rows at 340 keys: 980 us (a workgroup per row, all heads one after the other, the scores formed twice) -> 28 us; 666 rows
+// of two prompts: 1451 -> 122 us; latent (16 heads, 256 + 64 numbers): 706 -> 39 and 719 -> 196 us.
 #include "common.h"
 #include "key_runs.h"
 
 namespace k8s {
 
 constexpr int kRaKeys = 128;    // keys of a part
-constexpr int kRaHeads = 8;     // heads of a workgroup that walks all parts
-constexpr int kRaFew = 2;       // of one that has a single part
-constexpr int kRaAsk = 16;     // values of a column asked for together where a workgroup walks all parts
+constexpr int kRaHeads = 8;     // heads of a workgroup
+constexpr int kRaFew = 2;       // of one that has a single part, where few of them run
+constexpr int kRaAsk = 16;      // values of a column asked for together with eight heads
 
 template <typename T>
 __device__ __forceinline__ float rld(const T* p, size_t i);
@@ -80,14 +81,18 @@ __device__ __forceinline__ void ra_join(float& m, float& l, float mp, float lp, 
 }
 __device__ __forceinline__ float ra_join_out(float o, float a, float op, float b) { return fmaf(o, a, __fmul_rn(op, b)); }
 
-// PART: a workgroup has one part (p.po).  Few of them run then, each a chain of latencies, so that all the registers are its
-// own: every value of the part is asked for before the scores, and 16 pieces of a key at a time instead of 4; and two heads a
-// workgroup, for with eight the multiply-adds and LDS reads of one compute unit are as long as the chain.  The sums are
-// those of the other form.  Reply steps of two rows at 340 keys, both forms, median of a trace: 35.8 us -> 31.3 (registers)
-// -> 16.9 (two heads) -> 14.5 (two lanes a key).
-template <typename TQ, typename TC, typename TO, bool VEC, bool PART>
-__global__ void __launch_bounds__(256, PART ? 1 : 4) rows_attn_kernel(RowsArgs p) {
-  constexpr int NH = PART ? kRaFew : kRaHeads;
+// PART: a workgroup has one part (p.po).  FEW: and there are few of them, each a chain of latencies, so that all the registers
+// are its own: every value of the part is asked for before the scores, and 16 pieces of a key at a time instead of 2; and two
+// heads a workgroup, for with eight the multiply-adds and LDS reads of one compute unit are as long as the chain.  The sums are
+// those of the other forms.  Reply steps of two rows at 340 keys, both attentions, median of a trace: 35.8 us -> 31.3
+// (registers) -> 16.9 (two heads) -> 14.5 (two lanes a key).
+// Few: up to 512 workgroups of two heads over fp32 pages and 256 over bf16 ones, which need more registers: what runs at
+// once.  Past that they go in turns and read each key four times as often.  us with the merge, eight heads / two, 16 heads
+// over 2 of 128: 7 rows at 800 keys (392) 25.7 / 23.6 fp32, 26.1 / 28.4 bf16; 12 at 700 (576) 25.6 / 28.6, 25.4 / 36.0; 32 heads
+// over 2 of 64: 32 rows at 500 (2048) 23.4 / 44.7, 23.3 / 77.0; 4 at 500 (256) 21.3 / 19.6, 22.1 / 20.3.
+template <typename TQ, typename TC, typename TO, bool VEC, bool PART, bool FEW>
+__global__ void __launch_bounds__(256, FEW ? 1 : 4) rows_attn_kernel(RowsArgs p) {
+  constexpr int NH = FEW ? kRaFew : kRaHeads;
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int D = p.D1 + p.D2, V = p.V, hpg = p.H / (p.G * p.M);
   const int HB = min(hpg, NH), nhb = (hpg + HB - 1) / HB, nvb = (V + 255) / 256;
@@ -135,15 +140,15 @@ __global__ void __launch_bounds__(256, PART ? 1 : 4) rows_attn_kernel(RowsArgs p
       ss[tid] = bt[j / p.BS] * p.BS + j % p.BS;
     }
     __syncthreads();
-    TC vall[PART ? kRaKeys : 1];
-    if constexpr (PART) {
+    TC vall[FEW ? kRaKeys : 1];
+    if constexpr (FEW) {
       if (own) {
 #pragma unroll
         for (int j = 0; j < kRaKeys; ++j) vall[j] = vbase[(size_t)ss[j] * p.vs];      // (past nk: the last one again)
       }
     }
     {  // scores: HL lanes beside each other have a key (KX of them), each every HL-th head
-      constexpr int HL = PART ? 2 : 4, KW = 64 / HL, KX = kRaKeys / (4 * KW), HP = NH / HL;
+      constexpr int HL = FEW ? 2 : 4, KW = 64 / HL, KX = kRaKeys / (4 * KW), HP = NH / HL;
       const int x = wv * KW + lane / HL, h0 = lane % HL;
       if (wv * KW < nk && h0 < nh) {
         const TC* kp[KX];
@@ -155,7 +160,7 @@ __global__ void __launch_bounds__(256, PART ? 1 : 4) rows_attn_kernel(RowsArgs p
         for (int k = 0; k < HP; ++k) qh[k] = h0 + HL * k < nh ? q0 + HL * k * D4 : q0;
         float a[HP][KX] = {};
         if (VEC) {
-#pragma unroll (PART ? 16 : 2)
+#pragma unroll (FEW ? 16 : 2)
           for (int d = 0; d < D; d += 4) {
             f32x4 kv[KX];
 #pragma unroll
@@ -223,7 +228,7 @@ __global__ void __launch_bounds__(256, PART ? 1 : 4) rows_attn_kernel(RowsArgs p
         }
       };
       // (weights past nk are zero, and zero times an infinity would be NaN)
-      if constexpr (PART) {
+      if constexpr (FEW) {
 #pragma unroll
         for (int j = 0; j < kRaKeys; j += 4)
           if (j < nk) {
@@ -306,13 +311,18 @@ __global__ void __launch_bounds__(256) rows_attn_merge_kernel(RowsArgs p) {
 
 template <typename TQ, typename TC, typename TO>
 static int launch_rows(const RowsArgs& p, int T, hipStream_t s) {
-  const int D = p.D1 + p.D2, hpg = p.H / (p.G * p.M), most = p.po ? kRaFew : kRaHeads, HB = hpg < most ? hpg : most;
+  const int D = p.D1 + p.D2, hpg = p.H / (p.G * p.M), z = p.po ? p.n_parts : 1;
+  auto groups = [&](int most) { return p.G * p.M * ((hpg + most - 1) / most) * ((p.V + 255) / 256); };
+  const bool few = p.po && (long)T * groups(kRaFew) * z <= (sizeof(TC) == 4 ? 512 : 256);
+  const int most = few ? kRaFew : kRaHeads, HB = hpg < most ? hpg : most;
   const size_t lds = sizeof(float) * ((size_t)HB * ((D + 3) / 4 * 4 + 4) + HB * kRaKeys + 2 * HB + kRaKeys);
-  const dim3 grid(T, p.G * p.M * ((hpg + HB - 1) / HB) * ((p.V + 255) / 256), p.po ? p.n_parts : 1);
+  const dim3 grid(T, groups(most), z);
   // four numbers of a key at a time where every key starts on such a border
   const bool vec = D % 4 == 0 && p.ks % 4 == 0 && ((uintptr_t)p.kc & (4 * sizeof(TC) - 1)) == 0;
-  auto k = p.po ? (vec ? rows_attn_kernel<TQ, TC, TO, true, true> : rows_attn_kernel<TQ, TC, TO, false, true>)
-                : (vec ? rows_attn_kernel<TQ, TC, TO, true, false> : rows_attn_kernel<TQ, TC, TO, false, false>);
+  auto k = few    ? (vec ? rows_attn_kernel<TQ, TC, TO, true, true, true> : rows_attn_kernel<TQ, TC, TO, false, true, true>)
+           : p.po ? (vec ? rows_attn_kernel<TQ, TC, TO, true, true, false> : rows_attn_kernel<TQ, TC, TO, false, true, false>)
+                  : (vec ? rows_attn_kernel<TQ, TC, TO, true, false, false>
+                         : rows_attn_kernel<TQ, TC, TO, false, false, false>);
   if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
     return (int)hipGetLastError();
   hipLaunchKernelGGL(k, grid, dim3(256), lds, s, p);

@@ -55,6 +55,8 @@ def test_masked_rows(H, G, D, V, maps, dt, kw):
     rows = [0, 127, 128, 129, 255, 256, 383, 384, 511, 640, 699]
     for r in rows:                                      # alone: a workgroup per part
         assert torch.equal(run(r, r + 1)[0], full[r])
+    for a, b in ((600, 624), (100, 160), (690, 700)):   # workgroups with eight heads of a part, and on both sides of the line
+        assert torch.equal(run(a, b), full[a:b])
     qi, kp = torch.arange(n)[:, None], torch.arange(n)[None]
     vis = kp <= qi
     if kw.get("chunk"):
@@ -96,6 +98,8 @@ def test_latent_rows(H, R, P, window):
     rows = [0, 127, 128, 129, 256, 399]
     for r in rows:
         assert torch.equal(run(r, r + 1)[0], full[r])
+    for a, b in ((320, 360), (396, 400)):
+        assert torch.equal(run(a, b), full[a:b])
     s = torch.einsum("thr,jr->thj", torch.cat([qa, qr], -1).double()[rows] if P else qa.double()[rows], c.double()) * scale
     dist = torch.tensor(rows)[:, None] - torch.arange(n)[None]
     vis = (dist >= 0) & (dist < window) if window else dist >= 0
