@@ -35,6 +35,22 @@ ROWS_MAX_M = 32
 ROWS_BF16, ROWS_F32, ROWS_SILU, ROWS_RELU2 = 0, 1, 2, 3
 
 
+def _rows_channels(M: int, big: int, K: int, out: int, planes: bool) -> bool:
+    """Whether rows of W that are a multiple of 16 KB apart make another kernel the quicker one.  They, and no others, cost up
+    to a third of the rate until there are columns enough (they likely fall on few of the memory's channels).  us before /
+    with the row-streaming kernel, bf16:  one row of 16384 x 7168, 8192, 8704 48.6 / 38.5, 52.1 / 57.9, 62.3 / 46.0;  8 rows
+    of 6144 x 8192 1.06, 9216 x 8192 1.12, 15360 x 8192 1.05 of the time before, but 4096 x 8192 0.87, 16384 x 8192 0.83, and
+    gated 0.9 at all columns;  8192 x 16384 56.5 / 61.4;  32 rows of 8192 x 8192 31.4 / 35.2, 16384 x 8192 54.7 / 67.5, 28672
+    x 8192 115 / 100, 16384 x 16384 96.7 / 119.6, 28672 x 16384 167 / 175."""
+    if K % 8192:
+        return False
+    if M == 1 and out != ROWS_F32:
+        return K == 8192                 # (16384 and more: 0.72 to 0.88 of the skinny kernel's time)
+    if M > 16 or K % 16384 == 0:
+        return 8192 <= big < 3 * K
+    return out != ROWS_SILU and (8192 if planes or out == ROWS_RELU2 else 5119) < big < 2 * K
+
+
 def rows_shape_ok(M: int, N: int, K: int, nf: int, ranges: int, out: int = ROWS_F32) -> bool:
     """What csrc/kernels/gemm_rows.hip accepts; ``N``: result columns."""
     return (0 < M <= ROWS_MAX_M and nf in ((1, 2, 4) if M <= 16 else (2, 4)) and N > 0 and K > 0
@@ -47,19 +63,19 @@ def rows_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = False
     """(16-row fragments of a workgroup, K ranges) with which the row-streaming kernel takes a product, or None: another
     kernel is the quicker one or the shape does not fit.  ``N``: result columns; ``planes``: K ranges may stay apart.
 
-    Up to 16 rows it is the quickest at the sizes from 128 x 512 to 128256 x 4096, at 0.53 to 0.97 of the time before with
-    cold weights.  Up to 32 rows X is half of what it reads: from 8192 columns on (us at 32 rows before / this: 8192 x 2048
+    Up to 16 rows it is the quickest at sizes from 128 x 512 to 128256 x 4096, at 0.53 to 0.97 of the time before with cold
+    weights.  Up to 32 rows X is half of what it reads: from 8192 columns on (us at 32 rows before / this: 8192 x 2048
     10.3 / 9.0, 16384 x 4096 42.0 / 26.9; 4096 x 2048 9.2 / 10.0 in fp32, 4096 x 8192 20.8 / 26.8), and of these where K is
     up to 1024 or a multiple of 2048 (1280 to 3584 0.61 to 1.07 of the time before, by shape); planes up to a K of 2048
     (2048 x 2048 with the pass behind 0.93, 2560 x 4096 1.10, 1088 x 8192 1.06 of the time before); and not past 40960
-    columns of a K from 8192 on with 25 rows or more, where X is most of it (57344 x 8192 188 / 202, gated 57344 x 12288 280 / 299).
+    columns of a K from 8192 on with 25 rows or more, where X is most of it (57344 x 8192 188 / 202, gated 57344 x 12288
+    280 / 299).
 
-    Rows of W that are a multiple of 16 KB apart, and no others, cost up to a third of the rate until there are columns
-    enough (they likely fall on few of the memory's channels).  us before / this at a K of 7168, 8192, 8704 and one row 48.6 /
-    38.5, 52.1 / 57.9, 62.3 / 46.0 (16384 columns);  at 32 rows of 8192 x 8192 31.4 / 35.2, 16384 x 8192 54.7 / 67.5, 28672 x
-    8192 115 / 100, 16384 x 16384 96.7 / 119.6, 28672 x 16384 167 / 175;  at 8 rows of 8192 x 16384 56.5 / 61.4, 16384 x 8192
-    67.6 / 56.1, 8192 x 8192 30.8 / 31.3.  So one row of a K of 8192 stays with the skinny kernel, a K of 16384 and, past 16
-    rows, of 8192 with the library up to three times as many columns.
+    Where K is no multiple of 512, only four fragments with loads of 128 bytes fit up to 16 rows, and few workgroups are left:
+    us before / this at 2560 x 1280 and 1 row 4.2 / 6.2, 2048 x 3840 and 4 rows 9.0 / 13.9, 128 x 768 and 16 rows 3.0 / 4.8,
+    but 8192 x 1280 0.9 to 1.0 (one row 1.02 to 1.08), 16384 x 1280 0.6 to 0.8 of the time before, gated from 2048 columns on
+    0.7 to 1.04.  Planes that cannot be cut lose to those that can: 2048 x 768 at 32 rows 1.14, 128 x 3584 at 16 rows 1.12.
+    Little more columns than a wave of workgroups has: 8736 x 4096 at 32 rows 1.15, 9216 x 12288 at 16 1.10, 4112 x 12288 1.14.
 
     The fragments and ranges are those of the least work on the busiest compute unit: a workgroup streams 16 nf x K / ranges
     weights and X of M rows (2.5 % of a fragment's time each row), and 256 of them run at once.  Four fragments, whose loads
@@ -71,9 +87,14 @@ def rows_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = False
         return None
     if M > 16 and not ((K <= 1024 or K % 2048 == 0) and (K <= 2048 if planes else big >= 8192)):
         return None
-    if M == 1 and K == 8192 and out != ROWS_F32:
+    if M <= 16 and K % 512 and big < (4096 if out == ROWS_SILU else 8192 + (M == 1)):
         return None
-    if K % (8192 if M > 16 else 16384) == 0 and 8192 <= big < 3 * K and (M > 1 or out == ROWS_F32):
+    if planes and (M > 16 and K % 512 or M > 8 and K > 2048 and K % 1024 and big < 1024):
+        return None
+    if _rows_channels(M, big, K, out, planes):
+        return None
+    if out != ROWS_SILU and (8192 < big <= 10240 and (M > 8 and K > 6144 or M > 16 and K > 2048 and big < 9216)
+                             or 4096 < big < 4608 and M > 8 and K >= 8192):
         return None
     if M > 24 and K >= 8192 and big > 40960:
         return None

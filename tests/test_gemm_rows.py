@@ -149,11 +149,28 @@ def test_rows_of_weights_on_the_same_channels():
             assert L.rows_plan(m, 8192, 8192, out) is None and L.rows_plan(m, 16384, 8192, out) is None
             assert L.rows_plan(m, 28672, 8192, out) and L.rows_plan(m, 16384, 6144, out) and L.rows_plan(m, 16384, 10240, out)
             assert L.rows_plan(m, 28672, 16384, out) is None
-        assert L.rows_plan(8, 16384, 8192, out) and L.rows_plan(8, 4096, 16384, out)
+        assert L.rows_plan(8, 16384, 8192, out) and L.rows_plan(8, 4096, 8192, out) and L.rows_plan(8, 4096, 16384, out)
+        assert L.rows_plan(8, 9216, 8192, out) is None and L.rows_plan(8, 9216, 6144, out)
         assert L.rows_plan(8, 8192, 16384, out) is None and L.rows_plan(16, 28672, 16384, out) is None
+    assert L.rows_plan(8, 6144, 8192) is None and L.rows_plan(8, 4608, 8192, L.ROWS_SILU)
     assert L.rows_plan(32, 8192, 8192, L.ROWS_SILU) is None and L.rows_plan(32, 14336, 8192, L.ROWS_SILU)
     assert L.rows_plan(1, 8192, 16384) and L.rows_plan(1, 8192, 16384, L.ROWS_F32) is None
     assert L.rows_plan(24, 57344, 8192) and L.rows_plan(25, 57344, 8192) is None
+
+
+def test_few_workgroups_are_left_to_other_kernels():
+    """Four fragments are all that fits where K is no multiple of 512: taken with columns enough."""
+    for k in (768, 1280, 1792, 2816, 3840):
+        for m in (1, 4, 16):
+            for n in (128, 1088, 2560, 4096):
+                assert L.rows_plan(m, n, k) is None and L.rows_plan(m, n, k, L.ROWS_F32, True) is None
+                assert L.rows_plan(m, n, k, L.ROWS_RELU2) is None
+            assert L.rows_plan(m, 16384, k) and L.rows_plan(m, 2560, k, L.ROWS_SILU)
+        assert L.rows_plan(1, 8192, k) is None and L.rows_plan(2, 8192, k)
+        assert L.rows_plan(32, 2048, k, L.ROWS_F32, True) is None
+    assert L.rows_plan(16, 2560, 1024) and L.rows_plan(32, 2048, 1024, L.ROWS_F32, True)
+    assert L.rows_plan(16, 128, 3584, L.ROWS_F32, True) is None and L.rows_plan(8, 128, 3584, L.ROWS_F32, True)
+    assert L.rows_plan(32, 8736, 4096) is None and L.rows_plan(32, 8736, 2048) and L.rows_plan(16, 8736, 4096)
 
 
 @gpu
