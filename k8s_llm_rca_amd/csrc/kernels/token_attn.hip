@@ -9,11 +9,11 @@
 // waves and parts follow from positions alone, so a row's bits do not depend on the step it is in.
 //
 // What bounds it: the chain row -> page -> keys -> scores -> join of some 5 us, and that one compute unit takes cold keys
-// in at 20 to 30 KB a us (as fragments; tok_turn), far below its share of the caches' rate.  So parts are small (256 masked or 128 latent keys: 128
-// KB of keys and values and 144 KB), and a merge of 3.5 us pays from the second part on.  16 heads over 2 of 128 / 16 heads
-// over latents of 256 + 64, us with the merge, and in brackets what a tile of 16 tokens per wave (masked) and a wave per 256
-// keys (latent) took in engine steps of about that size: 1 row at 100 keys 5.3 / 8.5 (8.4 / 13.5), 8 rows at 1500 10.7 / 12.5 (26 / 36),
-// 64 rows at 400 12.3 / 14.3 (28 / 35).
+// in at 20 to 30 KB a us (as fragments; tok_turn), far below its share of the caches' rate.  So parts are small (256 masked
+// or 128 latent keys: 128 KB of keys and values and 144 KB), and a merge of 3.5 us pays from the second part on.  16 heads
+// over 2 of 128 / 16 heads over latents of 256 + 64, us with the merge, and in brackets what a tile of 16 tokens per wave
+// (masked) and a wave per 256 keys (latent) took in engine steps of about that size, all with fragments' loads: 1 row at 100
+// keys 5.3 / 8.5 (8.4 / 13.5), 8 rows at 1500 10.7 / 12.5 (26 / 36), 64 rows at 400 12.3 / 14.3 (28 / 35).
 #include "common.h"
 #include "key_runs.h"
 
@@ -178,19 +178,28 @@ __global__ void __launch_bounds__(256) token_merge_kernel(TokOut a, const int* _
 
 __device__ __forceinline__ bf16x8 tld16(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
-// Keys and values are loaded with lane 4 r + h at piece h of row r, so that four lanes beside each other read 64 bytes of a
-// line; the fragment wants them in lane 16 h + r (from: 4 (4 r + h), the byte address of the lane that has this lane's).
+// TURN: keys and values are loaded with lane 4 r + h at piece h of row r, so that four lanes beside each other read 64 bytes of
+// a line; the fragment wants them in lane 16 h + r (from: 4 (4 r + h), the byte address of the lane that has this lane's).
 // Loaded where the fragment wants them, four neighbours read four rows and each is a lookup of its own in the first-level
-// cache: in reply steps 7 rows at 800 keys 8.7 -> 6.7 us masked, 9.6 -> 7.9 latent, 5 rows at 1200 8.5 -> 7.1; one row and
-// 64 rows at 512 as before (4.4 - 6, 12.6, 15 us).
+// cache.  That counts where a compute unit has one or two workgroups, each a chain of such loads; where others run meanwhile
+// the exchanges through LDS cost more than the lookups.  us with the merge, as fragments / turned, in a replayed chain:
+// masked, 16 heads over 2 of 128, 7 rows at 1000 keys 11.2 / 9.6, 64 at 2000 35 / 35; 16 over 16 of 64, 16 rows at 200 (256
+// workgroups) 6.3 / 6.0, 32 at 200 (512) 8.1 / 7.3, 16 at 512 (768) 13.0 / 13.9, 64 at 512 30 / 34; 8 over 8 of 64 + 128 7.4 / 7.7
+// and of 128 + 128 8.2 / 8.4 at 4 and 7 rows.  Latent, 16 heads of 256 + 64, 7 rows at 1000 12.3 / 10.8, 32 at 512 (160) 13.9 /
+// 12.4, 16 at 2000 (256) 13.6 / 13.9, 64 at 512 (320) 18.6 / 19.3; of 512 + 64 18.3 / 15.4, 39 / 41 at 64 rows; of 64 + 32 7.5 / 7.7.
+template <bool TURN>
 __device__ __forceinline__ bf16x8 tok_turn(bf16x8 v, int from) {
-  int w[4];
-  __builtin_memcpy(w, &v, 16);
+  if constexpr (TURN) {
+    int w[4];
+    __builtin_memcpy(w, &v, 16);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_ds_bpermute(from, w[i]);
-  __builtin_memcpy(&v, w, 16);
+    for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_ds_bpermute(from, w[i]);
+    __builtin_memcpy(&v, w, 16);
+  }
   return v;
 }
+
+constexpr int kTurnMasked = 512, kTurnLatent = 256, kTurnLong = 192;      // workgroups up to which it pays (kTurnLong: R > 256)
 
 // Scores p[8] (log2 units, keys 8 h .. 8 h + 7 of head lane & 15; -inf: not seen) -> the running maximum and sum, the
 // weights as the value product's operand; the output is rescaled only where a head's maximum moved.
@@ -239,7 +248,7 @@ struct MaskTokArgs {
 
 // grid (rows, key heads (x maps) x groups of 16 of their heads, parts); a part is a run of the row's list of 32-key blocks
 // (kept first tokens, then the window's or chunk's).
-template <int NDC, int NV, bool CAP, int NW>
+template <int NDC, int NV, bool CAP, int NW, bool TURN>
 __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs a) {
   constexpr int D = NDC * 32, V = NV * 16;
   __shared__ TokLds<NW, V> lds;
@@ -282,7 +291,7 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
     pgv = k + lane < my ? pages[pi] : 0;
   };
   fill(0);
-  const int lr = lane >> 2, lh = lane & 3, from = 4 * (4 * r + hq);
+  const int lr = TURN ? lane >> 2 : r, lh = TURN ? lane & 3 : hq, from = 4 * (4 * r + hq);
   bf16x8 kf[2][2][NDC], vf[2][NV];
   int kb[2];
   auto load = [&](int u, int k) {
@@ -310,7 +319,8 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
       for (int t = 0; t < 2; ++t) {
         f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int cc = 0; cc < NDC; ++cc) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tok_turn(kf[u][t][cc], from), qf[cc], s, 0, 0, 0);
+        for (int cc = 0; cc < NDC; ++cc)
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tok_turn<TURN>(kf[u][t][cc], from), qf[cc], s, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) p[4 * t + i] = s[i];
       }
@@ -328,7 +338,8 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
       bf16x8 pf;
       tok_softmax<NV>(p, hq, m, l, o, pf);
 #pragma unroll
-      for (int dt = 0; dt < NV; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, tok_turn(vf[u][dt], from), o[dt], 0, 0, 0);
+      for (int dt = 0; dt < NV; ++dt)
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, tok_turn<TURN>(vf[u][dt], from), o[dt], 0, 0, 0);
       if (k + u + 2 < my) load(u, k + u + 2);
     }
   }
@@ -353,7 +364,7 @@ struct LatTokArgs {
 
 // grid (rows, parts, groups of 16 heads); parts are ranges of the key index (a row's first one is that of its first
 // visible key).
-template <int NR, int NP, int NW>
+template <int NR, int NP, int NW, bool TURN>
 __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a) {
   constexpr int R = NR * 32, ND = R / 16, NC = NR + NP, RW = R + 32 * NP, NH = ND / 2;
   __shared__ TokLds<NW, R> lds;
@@ -380,7 +391,7 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
 #pragma unroll
   for (int dt = 0; dt < ND; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int* pages = a.bt + (size_t)sg * a.maxb;
-  const int lr = lane >> 2, lh = lane & 3, from = 4 * (4 * r + hq);
+  const int lr = TURN ? lane >> 2 : r, lh = TURN ? lane & 3 : hq, from = 4 * (4 * r + hq);
   for (int b = wv; b < nb; b += NW) {
     const int kb = kb0 + 32 * b, page = pages[kb / a.BS], off = kb % a.BS;
     const uint16_t* cp = a.c + (size_t)page * a.BS * RW;
@@ -398,7 +409,8 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
     for (int t = 0; t < 2; ++t) {
       f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tok_turn(kf[t][cc], from), qf[cc], s, 0, 0, 0);
+      for (int cc = 0; cc < NC; ++cc)
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tok_turn<TURN>(kf[t][cc], from), qf[cc], s, 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int key = kb + 8 * hq + 4 * t + i;
@@ -411,7 +423,8 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
     bf16x8 pf;
     tok_softmax<ND>(p, hq, m, l, o, pf);
 #pragma unroll
-    for (int dt = 0; dt < ND; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, tok_turn(vf[dt], from), o[dt], 0, 0, 0);
+    for (int dt = 0; dt < ND; ++dt)
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, tok_turn<TURN>(vf[dt], from), o[dt], 0, 0, 0);
   }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
@@ -422,10 +435,13 @@ template <int NDC, int NV, int NW>
 static int launch_mask_tok_nw(const MaskTokArgs& a, int rows, hipStream_t s) {
   const int hpg = a.t.H / (a.G * a.t.hs);
   const dim3 grid(rows, a.G * a.t.hs * ((hpg + 15) / 16), a.t.n_parts);
-  if (a.softcap > 0.f)
-    hipLaunchKernelGGL((masked_attn_token_kernel<NDC, NV, true, NW>), grid, dim3(64 * NW), 0, s, a);
-  else
-    hipLaunchKernelGGL((masked_attn_token_kernel<NDC, NV, false, NW>), grid, dim3(64 * NW), 0, s, a);
+  auto k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, false>
+                           : masked_attn_token_kernel<NDC, NV, false, NW, false>;
+  if constexpr (NV == 2 * NDC && (NDC == 2 || NW == 8))      // keys as long as values, heads that share keys or are of 64
+    if ((long)rows * grid.y * grid.z <= kTurnMasked)
+      k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, true>
+                          : masked_attn_token_kernel<NDC, NV, false, NW, true>;
+  hipLaunchKernelGGL(k, grid, dim3(64 * NW), 0, s, a);
   if (a.t.n_parts > 1)
     hipLaunchKernelGGL(token_merge_kernel, dim3(rows * a.t.H), dim3(256), 0, s, a.t, a.items, NV * 16);
   return (int)hipGetLastError();
@@ -445,14 +461,22 @@ static int launch_mask_tok(const MaskTokArgs& a, int rows, hipStream_t s) {
     return a.t.H > a.G * a.t.hs ? launch_mask_tok_nw<NDC, NV, 8>(a, rows, s) : launch_mask_tok_nw<NDC, NV, 2>(a, rows, s);
 }
 
-template <int NR>
-static int launch_lat_tok(const LatTokArgs& a, int np, int rows, hipStream_t s) {
+template <int NR, int NP>
+static void launch_lat_tok_np(const LatTokArgs& a, int rows, hipStream_t s) {
   constexpr int NW = 4;
   const dim3 grid(rows, a.t.n_parts, (a.t.H + 15) / 16);
+  auto k = latent_attn_token_kernel<NR, NP, NW, false>;
+  if constexpr (NR >= 6)
+    if ((long)rows * grid.y * grid.z <= (NR > 8 ? kTurnLong : kTurnLatent)) k = latent_attn_token_kernel<NR, NP, NW, true>;
+  hipLaunchKernelGGL(k, grid, dim3(64 * NW), 0, s, a);
+}
+
+template <int NR>
+static int launch_lat_tok(const LatTokArgs& a, int np, int rows, hipStream_t s) {
   switch (np) {
-    case 0: hipLaunchKernelGGL((latent_attn_token_kernel<NR, 0, NW>), grid, dim3(64 * NW), 0, s, a); break;
-    case 1: hipLaunchKernelGGL((latent_attn_token_kernel<NR, 1, NW>), grid, dim3(64 * NW), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((latent_attn_token_kernel<NR, 2, NW>), grid, dim3(64 * NW), 0, s, a); break;
+    case 0: launch_lat_tok_np<NR, 0>(a, rows, s); break;
+    case 1: launch_lat_tok_np<NR, 1>(a, rows, s); break;
+    case 2: launch_lat_tok_np<NR, 2>(a, rows, s); break;
     default: return (int)hipErrorInvalidValue;
   }
   if (a.t.n_parts > 1)

@@ -73,6 +73,7 @@ def test_masked(H, G, D, V, kw, extras):
     for r in (0, 3, 9, 10, 12):              # alone (fewer parts in the step, or none) and beside a long row: the same bits
         assert torch.equal(run([r])[0], got[r]) and torch.equal(run([r, 13])[0], got[r])
     assert torch.equal(run(every, out_f32=True).to(BF), got)
+    assert torch.equal(run(every * 40), got.repeat(40, 1))      # past the workgroups that load by lines: the same bits
 
 
 @pytest.mark.parametrize("H,R,P", [(16, 256, 64), (5, 32, 0), (20, 64, 32), (16, 512, 64), (3, 384, 0), (33, 128, 32)])
@@ -107,6 +108,7 @@ def test_latent(H, R, P, window, extras):
     close(got, want)
     for r in (0, 3, 6, 9, 12):
         assert torch.equal(run([r])[0], got[r]) and torch.equal(run([r, 13], head_major=False)[0], got[r])
+    assert torch.equal(run(every * 20), got.repeat(20, 1, 1))
 
 
 def test_score_maps():
