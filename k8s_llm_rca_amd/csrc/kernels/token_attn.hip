@@ -199,7 +199,7 @@ __device__ __forceinline__ bf16x8 tok_turn(bf16x8 v, int from) {
   return v;
 }
 
-constexpr int kTurnMasked = 512, kTurnLatent = 256, kTurnLong = 192;      // workgroups up to which it pays (kTurnLong: R > 256)
+constexpr int kTurnMasked = 512, kTurnLatent = 255, kTurnLong = 192;      // workgroups up to which it pays (kTurnLong: R > 256)
 
 // Scores p[8] (log2 units, keys 8 h .. 8 h + 7 of head lane & 15; -inf: not seen) -> the running maximum and sum, the
 // weights as the value product's operand; the output is rescaled only where a head's maximum moved.
