@@ -842,10 +842,10 @@ def decay_attention(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor
         # long portions: chunks in parallel (end states from zero, a carry over the chunks, the chunks
         # again from their start states); short ones token by token.  On the matrix cores a portion goes in
         # blocks of 64 tokens, and its chunks are ranges of several blocks
-        longest = max(b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:]))
-        mfma = longest >= LIN_MFMA_ROWS and decay_mfma_ok(D, V, x.dtype, x.device) and x.stride(0) % 4 == 0
+        lens = [b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:])]
+        mfma = max(lens) >= LIN_MFMA_ROWS and decay_mfma_ok(D, V, x.dtype, x.device) and x.stride(0) % 4 == 0
         if mfma:
-            rows = _lin_rows(T, seg.n_seg, H, D, V, longest)
+            rows = _lin_rows(T, seg.n_seg, H, D, V, lens)
             cr = seg.chunk_ranges(rows, rows) if rows else None     # (None: no portion is longer than a range)
         else:
             cr = seg.chunk_ranges(SSM_CHUNK, 2 * SSM_CHUNK) if seg.n_seg * H * V * 8 < SEQ_FILL_LANES else None
@@ -885,27 +885,28 @@ LIN_GROUPS = 256        # workgroups (ranges x heads x 128 value columns) a step
 LIN_WALK = 768, 512     # rows the longest portion may walk past the chip's share, with up to 512 workgroups and with more
 
 
-def _lin_rows(T: int, n_seg: int, H: int, D: int, V: int, longest: Optional[int] = None) -> int:
-    """Rows of a range, 0: portions stay whole.  As many ranges as give the chip a workgroup per unit; of the form that two
-    workgroups of a unit share (csrc/kernels/linear_attn.hip) two, where no portion has more than a fifth of the rows: the
-    carry walks all ranges of a portion (us of 16 heads of 128 at 256 / 512 workgroups: 31 x 512 + 2048 rows 363 / 299, 7 of
-    351 to 701 88 / 78, 5 x 1000 107 / 83, but 4 x 1000 64 / 71, 4 x 600 54 / 60, 1 x 4000 67 / 75, 15 single rows + 4000
-    198 / 282).
+def _lin_rows(T: int, n_seg: int, H: int, D: int, V: int, lens: Optional[List[int]] = None) -> int:
+    """Rows of a range, 0: portions stay whole.  ``lens``: the portions' rows (without them they are taken as equal).  As many
+    ranges as give the chip a workgroup per unit;  of the form that two workgroups of a unit share
+    (csrc/kernels/linear_attn.hip) two, where no portion has more than a fifth of the rows, as the carry walks all ranges of a
+    portion, and one each would be ranges of 512 rows or more than 256 of them (us of 16 heads of 128 at 256 / 512
+    workgroups: 31 x 512 + 2048 rows 363 / 299, 7 of 351 to 701 88 / 78, 5 x 1000 107 / 83, but 4 x 1000 64 / 71, 4 x 600 54 /
+    60, 1 x 4000 67 / 75, 15 single rows + 4000 198 / 282;  of 4 heads 16 x 1024 65 / 74, 5 x 2000 51 / 60).
 
-    Whole, where the portions are 256 workgroups or more by themselves and the ``longest`` (without it they are taken as
-    equal) is not left walking alone: up to ``LIN_WALK`` rows past T H / 256, which is what a unit gets of the step, and
-    fewer of them where not all workgroups run at once (whole / cut: 16 x 1024 117 / 184, 15 x 512 + 1024 107 / 167, 15 x
-    300 + 1000 106 / 128, 31 single rows + 768 133 / 140, of 64 heads 15 + 512 175 / 188;  past the line 31 x 512 + 2048
-    378 / 299, 63 x 512 + 3072 850 / 549, 15 x 300 + 1500 157 / 139, 63 single rows + 1000 222 / 198, 15 + 4000 412 / 198, of
-    64 heads 15 + 768 259 / 215)."""
-    per, groups = H * -(-V // 128), LIN_GROUPS
-    longest = -(-T // n_seg) if longest is None else longest
+    Whole, where the portions are 256 workgroups or more by themselves and the longest is not left walking alone: up to
+    ``LIN_WALK`` rows past T H / 256, which is what a unit gets of the step, and fewer of them where not all workgroups run at
+    once (whole / cut: 16 x 1024 117 / 184, 15 x 512 + 1024 107 / 167, 15 x 300 + 1000 106 / 128, 31 single rows + 768 133 /
+    140, of 64 heads 15 + 512 175 / 188;  past the line 31 x 512 + 2048 378 / 299, 63 x 512 + 3072 850 / 549, 15 x 300 + 1500
+    157 / 139, 63 single rows + 1000 222 / 198, 15 + 4000 412 / 198, of 64 heads 15 + 768 259 / 215)."""
+    per, lens = H * -(-V // 128), lens or [-(-T // n_seg)] * n_seg
+    rows, longest = max(LIN_CHUNK, -(-T // (64 * max(1, LIN_GROUPS // per))) * 64), max(lens)
     if D == 128 and V > 64:
         past = longest - LIN_WALK[n_seg * per > 2 * LIN_GROUPS]
         if n_seg * per >= LIN_GROUPS and past * LIN_GROUPS <= T * per:
             return 0
-        groups *= 2 if T >= 5 * longest else 1
-    return max(LIN_CHUNK, -(-T // (64 * max(1, groups // per))) * 64)
+        if T >= 5 * longest and (rows >= 512 or per * sum(-(-n // rows) for n in lens if n > rows) > LIN_GROUPS):
+            rows = max(LIN_CHUNK, -(-T // (64 * max(1, 2 * LIN_GROUPS // per))) * 64)
+    return rows
 
 
 def decay_mfma_ok(D: int, V: int, dtype, device) -> bool:

@@ -19,13 +19,14 @@ def test_ranges():
 def test_ranges_follow_the_lengths():
     """However many short portions are beside it, a long one is cut as it is alone."""
     def rows(lens, H=16):
-        return S._lin_rows(sum(lens), len(lens), H, 128, 128, max(lens))
+        return S._lin_rows(sum(lens), len(lens), H, 128, 128, lens)
 
     assert rows([4000]) == rows([1] * 15 + [4000]) == rows([1] * 63 + [4000]) == 256
     assert rows([4000] + [40] * 15) == 320 and rows([1] * 3 + [4000]) == 256
     assert 0 < rows([512] * 63 + [4096]) < 4096 and 0 < rows([512] * 31 + [2048]) < 2048
     assert rows([1024] * 16) == rows([512] * 15 + [1024]) == rows([1] * 32 + [300]) == 0      # nothing to wait for
     assert rows([1000] * 4) == 256 and rows([1000] * 5) == 192                               # two workgroups a unit
+    assert rows([1024] * 16, 4) == 256 and rows([2000] * 5, 4) == 192 and rows([2048] * 8) == 512
     assert rows([1] * 15 + [512], 64) == 0 and rows([1] * 15 + [768], 64) == 256
 
 
@@ -46,7 +47,7 @@ def test_more_than_a_workgroup_a_unit(lens, V, silu):
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
     seg = S.SegMeta(n, i32([s for s, k in enumerate(lens) for _ in range(k)]), i32(row0), i32(pos0), i32(list(range(n))),
                     i32([[0]] * n), row0, pos0, list(range(n)))
-    rows = S._lin_rows(T, n, H, D, V, max(lens))
+    rows = S._lin_rows(T, n, H, D, V, lens)
     groups = (sum(-(-k // rows) for k in lens) if rows and max(lens) > rows else n) * H * -(-V // 128)
     assert groups > 256
     state = start.to(dev)
