@@ -39,6 +39,7 @@ struct LinArgs {
   float* cs;
   float* o;
   int H, V;
+  int two;               // launch the form of which two workgroups share a compute unit, where there is one
 };
 
 // dec^n by repeated squaring
@@ -125,7 +126,7 @@ constexpr int la_lds_bytes(bool outputs) {
   return 2 * (trow(D) + trow(16 * NW) + (outputs ? kLaTok * ld + k_or_p : 0));
 }
 
-// TWO: 128 registers, so that two workgroups of eight waves share a compute unit, where there are more than 256 of them: this
+// TWO: 128 registers, so that two workgroups of eight waves share a compute unit, where the caller finds enough of them: this
 // thread's numbers are made anew in every block, unknown to the optimizer, or the addresses of all the tiles would take the
 // registers.  Alone on its unit a workgroup is the slower for it (16 heads of 128, one workgroup a unit 131 / 148 us); 64
 // portions of 256 to 512 rows 239 - 254 -> 217 - 242 by run, 8 of 2048 cut into 512 workgroups 223 - 226 -> 198 - 221, seven of
@@ -357,7 +358,7 @@ static int launch_la(const LinArgs& a, int items, hipStream_t s) {
   constexpr int lds = la_lds_bytes<D, NW>(MODE != 1);
   auto k = decay_attn_mfma_kernel<D, NW, MODE, SILU, false>;
   if constexpr (D == 128 && NW == 8)
-    if ((long)items * a.H * ((a.V + 127) / 128) > 256) k = decay_attn_mfma_kernel<D, NW, MODE, SILU, true>;
+    if (a.two) k = decay_attn_mfma_kernel<D, NW, MODE, SILU, true>;
   if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds))
     return (int)hipGetLastError();
   hipLaunchKernelGGL(k, dim3(items, a.H, (a.V + 16 * NW - 1) / (16 * NW)), dim3(64 * NW), lds, s, a);
@@ -392,7 +393,7 @@ K8S_API int k8s_decay_attn_mfma_ok(int D, int V) {
 
 K8S_API int k8s_decay_attn_mfma(const void* x, int xs, int silu, const float* decay, float* state, const int* seg_row0,
                                 const int* seg_pos0, const int* seg_slot, float* o, int n_seg, int H, int D, int V,
-                                hipStream_t s, const int* items, int n_items, const int* seg_item0, float* cs) {
+                                hipStream_t s, const int* items, int n_items, const int* seg_item0, float* cs, int two) {
   if (n_seg <= 0) return 0;
   if (!k8s_decay_attn_mfma_ok(D, V) || H < 1 || xs % 4 || ((uintptr_t)x & 7) || xs < H * (2 * D + V) ||
       (n_items > 0 && (!items || !seg_item0 || !cs)))
@@ -410,6 +411,7 @@ K8S_API int k8s_decay_attn_mfma(const void* x, int xs, int silu, const float* de
   a.o = o;
   a.H = H;
   a.V = V;
+  a.two = two;
 #define K8S_LA(DD)                                                                    \
   return silu ? launch_la_v<DD, true>(a, n_seg, n_items, seg_item0, s)                \
               : launch_la_v<DD, false>(a, n_seg, n_items, seg_item0, s)

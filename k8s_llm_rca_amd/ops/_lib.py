@@ -131,7 +131,7 @@ _SIGS = {
     "k8s_selective_scan": [P, I, P, P, P, I, I, P, P, P, I, P, P, P, P, P, I, I, I, I, P, P, I, P, P, P],
     "k8s_decay_attn": [P, I, I, I, P, P, P, P, P, P, I, I, I, I, P, P, I, P, P],
     "k8s_decay_attn_mfma_ok": [I, I],
-    "k8s_decay_attn_mfma": [P, I, I, P, P, P, P, P, P, I, I, I, I, P, P, I, P, P],
+    "k8s_decay_attn_mfma": [P, I, I, P, P, P, P, P, P, I, I, I, I, P, P, I, P, P, I],
     "k8s_retention": [P, I, P, P, P, P, P, P, P, I, I, I, I, I, F, F, I, P, I, P, P, I, P, P],
     "k8s_window_kv_write": [P, I, I, I, I, P, P, P, I, I, P, P, I],
     "k8s_window_attn_mfma_ok": [I, I, I, I],

@@ -857,7 +857,8 @@ def decay_attention(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor
         if mfma:
             check(lib().k8s_decay_attn_mfma(ptr(x), x.stride(0), int(silu), ptr(decay), ptr(state), ptr(seg.seg_row0),
                                             ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(out), seg.n_seg, H, D, V,
-                                            stream_ptr(x), ptr(chunks), nch, ptr(c0), ptr(cs)), "decay_attn_mfma")
+                                            stream_ptr(x), ptr(chunks), nch, ptr(c0), ptr(cs),
+                                            int(_lin_two(lens, rows if cr is not None else 0, H, V))), "decay_attn_mfma")
             return out
         check(lib().k8s_decay_attn(ptr(x), x.stride(0), _dt(x.dtype), int(silu), ptr(decay), ptr(state),
                                    ptr(seg.seg_row0), ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(out), seg.n_seg, H, D, V,
@@ -907,6 +908,16 @@ def _lin_rows(T: int, n_seg: int, H: int, D: int, V: int, lens: Optional[List[in
         if T >= 5 * longest and (rows >= 512 or per * sum(-(-n // rows) for n in lens if n > rows) > LIN_GROUPS):
             rows = max(LIN_CHUNK, -(-T // (64 * max(1, 2 * LIN_GROUPS // per))) * 64)
     return rows
+
+
+def _lin_two(lens: List[int], rows: int, H: int, V: int) -> bool:
+    """Whether two workgroups of :func:`decay_attention` share a compute unit (heads of 128; ``rows``: of a range, 0: portions
+    whole): where there are more than 256.  With fewer than 16 heads' columns those of a block (64 rows) or less, reply
+    tokens above all, do not count: they end before the others meet (us counted / not: 8 heads, 48 single rows + 16 x 1000
+    178 / 140, 63 + 600 112 / 100; 16 heads 24 + 8 x 1000 177 / 208, 31 + 768 134 / 158, 15 + 4000 195 / 206)."""
+    per = H * -(-V // 128)
+    least = 0 if per >= 16 else 64
+    return per * sum(n // rows + (n % rows > least) if rows else n > least for n in lens) > LIN_GROUPS
 
 
 def decay_mfma_ok(D: int, V: int, dtype, device) -> bool:

@@ -30,6 +30,13 @@ def test_ranges_follow_the_lengths():
     assert rows([1] * 15 + [512], 64) == 0 and rows([1] * 15 + [768], 64) == 256
 
 
+def test_two_workgroups_a_unit():
+    assert S._lin_two([1024] * 17, 0, 16, 128) and not S._lin_two([1024] * 16, 0, 16, 128)
+    assert S._lin_two([1] * 15 + [4000], 256, 16, 128) and not S._lin_two([4000], 256, 16, 128)
+    assert not S._lin_two([1] * 48 + [1000] * 16, 256, 4, 128) and S._lin_two([1000] * 17, 256, 4, 128)   # single rows
+    assert not S._lin_two([64] * 100, 0, 4, 128) and S._lin_two([65] * 100, 0, 4, 128)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("lens,V,silu", [([70] * 18, 128, False), ([64, 1, 130, 65] * 5, 128, True), ([300] * 6, 128, False),
                                          ([129] * 9, 144, True), ([600] * 5, 128, True), ([1] * 15 + [900], 128, True)])
@@ -49,7 +56,7 @@ def test_more_than_a_workgroup_a_unit(lens, V, silu):
                     i32([[0]] * n), row0, pos0, list(range(n)))
     rows = S._lin_rows(T, n, H, D, V, lens)
     groups = (sum(-(-k // rows) for k in lens) if rows and max(lens) > rows else n) * H * -(-V // 128)
-    assert groups > 256
+    assert groups > 256 and S._lin_two(lens, rows if rows and max(lens) > rows else 0, H, V)
     state = start.to(dev)
     xd = x.to(dev)
     got = S.decay_attention(xd, H, D, V, decay.to(dev), state, seg, silu=silu)
