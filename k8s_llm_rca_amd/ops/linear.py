@@ -251,16 +251,22 @@ def row_cut(M: int, N: int, K: int, tuned: bool = False) -> int:
     24730 (3.03) 246 / 218;  2048 x 8192 at 16500 641 / 434, 24730 743 / 639, but 20000 (2.47) 726 / 542 and 22000 (2.69)
     765 / 579;  8192 x 2048 in bf16 at 2100 (1.12) 85 / 64, 12000 (5.88) 389 / 295, 24730 629 / 592, 3300 (1.62) 94 / 95;
     2560 x 2048 at 27000 (4.14) 313 / 261, 22000 (3.36) 218 / 246;  4096 x 14336 at 4123 (1.06) 730 / 367.  So up to 0.15 of
-    a wave whatever the shape, further where the columns divide a wave and are many or K is long.  Over 92 random sizes of 18
-    weights 0.88 of the time (0.50 to 1.12, six of them past 1.02).  ``tuned``: a call that takes measured solutions, which
-    stay with the rows they were measured for."""
+    a wave where the columns are up to 24 tiles that they nearly fill (past that the tiles of a row leave too little to gain:
+    28672 x 256 at 1704 43 / 67, 8736 x 4096 at 11027 685 / 778, 1088 x 512 at 14181 35 / 43) or divide a wave;  further where
+    they divide it and are many or K is long, past two waves (three of tiles of which a wave is two rows) and with a K from
+    1024 on (32768 x 4096 at 540, 1.5 waves, 150 / 177, x 1024 at 1109, 2.5, 95 / 110, 8192 x 512 at 19744 186 / 207).  What
+    the library takes for a size is not to be foreseen: over 452 random sizes that this cuts 0.89 of the time, 32 of them past
+    1.02 (8192 x 384 at 2284 30 / 37, 2560 x 14336 at 19632 1128 / 1350).  ``tuned``: a call that takes measured solutions,
+    which stay with the rows they were measured for."""
     nt = -(-N // 256)
     full, over = divmod(-(-M // 256) * nt, 256)
     if full < 1 or not over or tuned and any(lo <= M <= hi for lo, hi in _lib_tuned.get((N, K), ())):
         return 0
     most = 0.15
-    if 256 % nt == 0 and N % 256 == 0 and (nt >= 32 or K >= 4096 and full > 1):
-        most = 1.0 if full > 1 else 0.5
+    if 256 % nt == 0 and N % 256 == 0:
+        most = 1.0 if full > 1 + (nt > 64) and K >= 1024 and (nt >= 32 or K >= 4096) else most
+    elif nt > 24 or 10 * N < 9 * 256 * nt:
+        return 0
     return full * 256 // nt * 256 if over <= most * 256 else 0
 
 

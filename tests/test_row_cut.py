@@ -19,6 +19,11 @@ def test_cut_is_whole_waves_of_tiles():
             parts = L._row_parts(m, n, k)
             assert parts[0][0] == 0 and parts[-1][1] == m and all(a < b for a, b in parts)
     assert L.row_cut(24730, 2048, 2048) == 24576 and L.row_cut(20000, 2048, 2048) == 0
+    assert L.row_cut(540, 32768, 4096) == L.row_cut(1061, 32768, 4096) == 0 and L.row_cut(1600, 32768, 4096) == 1536
+    assert L.row_cut(19744, 8192, 512) == 0 and L.row_cut(19744, 8192, 2048) and L.row_cut(2100, 8192, 512) == 2048
+    for m, n, k in ((1704, 28672, 256), (11027, 8736, 4096), (14181, 1088, 512)):
+        assert L.row_cut(m, n, k) == 0
+    assert L.row_cut(27000, 2560, 2048) and L.row_cut(6341, 2576, 2048)
     assert L.row_cut(20000, 2048, 8192) == 16384 and L.row_cut(16384, 2048, 8192) == 0
 
 
