@@ -485,16 +485,21 @@ def proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def big_tiles_fill(M: int, N: int, silu: bool, K: int = 4096) -> bool:
     """Whether gemm_big's 256-row tiles fill the 256 compute units far enough over all their waves.  Then its fused epilogue
-    beats hipBLASLt and a pass over the result, otherwise the idle last wave costs more than the pass: up to a K of 1024 from
-    half on, up to 2048 past the first wave from seven tenths (within it least is to be had: SwiGLU at 0.75 48.4 / 48.7), else
-    from four fifths.  us fused / apart at waves of tiles:  squared relu 8192 x
-    2048 at 0.50 38.6 / 36.8, 0.75 42 / 48, 1.00 49 / 60, 1.12 77 / 72, 1.38 82 / 90, 1.50 83 / 96, 2.12 123 / 128, 2.38
-    127 / 141, 5.00 226 / 282, 8192 x 1024 at 0.38 24.0 / 23.6, 0.50 24.9 / 25.3, 1.12 48 / 53;  SwiGLU 8192 x 2048 at
-    1.25 96 / 86, 1.50 97 / 99, 2.25 138 / 135, 2.50 137 / 154, 4.25 227 / 239, 6144 x 2048 at 1.31 85 / 81, 1.50
-    85 / 89, 8192 x 4096 at 1.50 153 / 148, 2.50 239 / 248."""
-    tiles = -(-M // 256) * -(-N // (128 if silu else 256))
-    tenths = 5 if K <= 1024 else 7 if K <= 2048 and tiles > 256 else 8
-    return 10 * tiles >= tenths * 256 * -(-tiles // 256)
+    beats hipBLASLt and a pass over the result, otherwise the idle last wave costs more than the pass: from four fifths, and
+    where the rows themselves (not whole tiles of them, which the library takes smaller) fill half up to a K of 1024, or past
+    the first wave seven tenths up to 2048 (within it least is to be had: SwiGLU at 0.75 48.4 / 48.7).  us fused / apart at
+    waves of tiles:  squared relu 8192 x 2048 at 0.50 38.6 / 36.8, 0.75 42 / 48, 1.00 49 / 60, 1.12 77 / 72, 1.38 82 / 90, 1.50
+    83 / 96, 2.12 123 / 128, 2.38 127 / 141, 5.00 226 / 282, 8192 x 1024 at 0.38 24.0 / 23.6, 0.50 24.9 / 25.3, 1.12 48 / 53;
+    SwiGLU 8192 x 2048 at 1.25 96 / 86, 1.50 97 / 99, 2.25 138 / 135, 2.50 137 / 154, 4.25 227 / 239, 6144 x 2048 at 1.31 85 /
+    81, 1.50 85 / 89, 8192 x 4096 at 1.50 153 / 148, 2.50 239 / 248;  with rows that end early in a tile, SwiGLU 8192 x 1024 at
+    274 rows (0.50 waves, 0.27 of rows) 28 / 22, 16384 x 2048 at 537 (1.50, 1.05) 95 / 89.  Over 256 random sizes between the
+    first line and the others 0.84 of the time, none past 1.02."""
+    cols = -(-N // (128 if silu else 256))
+    tiles = -(-M // 256) * cols
+    units = 256 * -(-tiles // 256)
+    if 10 * tiles >= 8 * units:
+        return True
+    return (K <= 1024 or K <= 2048 and tiles > 256) and 10 * M * cols >= (5 if K <= 1024 else 7) * 256 * units
 
 
 SHORT_K = 512       # up to here what is paid is the result's way through memory, not the tiles

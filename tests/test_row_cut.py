@@ -68,3 +68,12 @@ def test_gemm_big_adds_to_the_residual(m, n, k, lda):
         r = before[:m].clone()
         assert L.proj_add(r, x, w, 0.5) is None and torch.equal(r, buf[:m])
     assert L.lib().k8s_gemm_big_add(L.ptr(x), lda, L.ptr(w), L.ptr(buf), n, m, n - 128, k, 0.5, L.stream_ptr(x)) != 0
+
+
+def test_fused_epilogues_count_rows_not_tiles():
+    """Past the general line a fused epilogue wants the rows to fill the waves, not tiles that end early."""
+    for silu, n in ((True, 8192), (False, 16384)):
+        assert not L.big_tiles_fill(274, n, silu, 1024) and L.big_tiles_fill(512, n, silu, 1024)
+        assert not L.big_tiles_fill(537, 2 * n, silu, 2048) and L.big_tiles_fill(768, 2 * n, silu, 2048)
+        assert L.big_tiles_fill(1, 4 * n, silu, 1024)                        # whole waves of tiles, as ever
+        assert not L.big_tiles_fill(768, 2 * n, silu, 4096)
