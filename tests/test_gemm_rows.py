@@ -1,4 +1,7 @@
 """The row-streaming product (csrc/kernels/gemm_rows.hip) at the edges of its forms, and the rule that picks it."""
+import json
+import os
+
 import pytest
 import torch
 
@@ -171,6 +174,21 @@ def test_few_workgroups_are_left_to_other_kernels():
     assert L.rows_plan(16, 2560, 1024) and L.rows_plan(32, 2048, 1024, L.ROWS_F32, True)
     assert L.rows_plan(16, 128, 3584, L.ROWS_F32, True) is None and L.rows_plan(8, 128, 3584, L.ROWS_F32, True)
     assert L.rows_plan(32, 8736, 4096) is None and L.rows_plan(32, 8736, 2048) and L.rows_plan(16, 8736, 4096)
+
+
+def test_tables_take_the_kernel_where_it_was_the_quicker():
+    seen = 0
+    for name in os.listdir(L.DATA_DIR):
+        if not name.startswith("gemm_dispatch_"):
+            continue
+        with open(os.path.join(L.DATA_DIR, name)) as f:
+            shapes = json.load(f)["shapes"]
+        for key, rows in shapes.items():
+            for r in (r for r in rows if r["kind"] == "rows"):
+                n, k = (int(v) for v in key.split(","))
+                seen += 1
+                assert r["t_us"] < r["lib_us"] and L.rows_shape_ok(r["m"], n, k, r["cfg"], r["splits"]), (name, key, r)
+    assert seen
 
 
 @gpu
