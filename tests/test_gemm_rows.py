@@ -130,6 +130,29 @@ def test_norm_in_front_is_norm_and_product(m, mode, H, nf):
     assert torch.equal(*outs) and torch.equal(*pages[:2]) and torch.equal(*pages[2:])
 
 
+@gpu
+@pytest.mark.parametrize("m", [1, 2, 4])
+@pytest.mark.parametrize("planes", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("H,nf", [(512, 1), (4096, 4)])
+def test_norm_in_front_of_any_count_of_planes(m, planes, H, nf):
+    """Up to four planes are asked for in front of the weights (past the last: it again), more are read behind them."""
+    I, eps = 512, 1e-5
+    g = torch.Generator(device="cuda").manual_seed(m + H + planes)
+    res = torch.randn(m, H, device="cuda", generator=g).to(BF)
+    buf = torch.full((planes * m * H + 64,), float("nan"), device="cuda")                 # behind the last plane: not read
+    part = buf[:planes * m * H].view(planes, m, H)
+    part.copy_(torch.randn(planes, m, H, device="cuda", generator=g) * 0.5)
+    nw = (torch.rand(H, device="cuda", generator=g) + 0.5).to(BF)
+    w = (torch.randn(2 * I, H, device="cuda", generator=g) * 0.02).to(BF)
+    y, r = torch.empty(m, H, device="cuda", dtype=BF), res.clone()
+    s = stream_ptr(res)
+    assert lib().k8s_splitk_addnorm(ptr(part), planes, ptr(r), ptr(nw), ptr(y), m, H, H, eps, s) == 0
+    new, act = torch.full_like(res, float("nan")), torch.empty(m, I, device="cuda", dtype=BF)
+    assert lib().k8s_gemm_rows_norm(None, H, ptr(part), planes, ptr(res), ptr(new), ptr(nw), eps, ptr(w), ptr(act), I, m, I, H,
+                                    nf, None, None, None, None, None, 0, 0, 0, s) == 0
+    assert torch.equal(new, r) and torch.equal(act, L.gemm_rows(y, w, nf, L.ROWS_SILU))
+
+
 def test_rule_gives_what_the_kernel_takes():
     """Every plan fits the kernel; past its rows and sizes there is none."""
     for out in (L.ROWS_BF16, L.ROWS_F32, L.ROWS_SILU, L.ROWS_RELU2):

@@ -77,3 +77,32 @@ def test_fused_epilogues_count_rows_not_tiles():
         assert not L.big_tiles_fill(537, 2 * n, silu, 2048) and L.big_tiles_fill(768, 2 * n, silu, 2048)
         assert L.big_tiles_fill(1, 4 * n, silu, 1024)                        # whole waves of tiles, as ever
         assert not L.big_tiles_fill(768, 2 * n, silu, 4096)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(4300, 4096, 2048), (200, 4096, 2048), (1540, 4096, 8192), (1, 256, 8192)])
+def test_gemm_big_adds_tiles_that_are_split(m, n, k):
+    """A last wave in slices of K: the last to arrive adds the sum of all to the residual, once."""
+    g = torch.Generator().manual_seed(m + k)
+    x = torch.randn(m, k + 8, generator=g).to(BF).cuda()[:, :k]
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(BF).cuda()
+    want = x.double() @ w.double().T
+    before = torch.randn(m + 1, n, generator=g).cuda()
+
+    def add():
+        r = before.clone()
+        L.check(L.lib().k8s_gemm_big_add(L.ptr(x), k + 8, L.ptr(w), L.ptr(r), n, m, n, k, 0.5, L.stream_ptr(x)), "add")
+        return r
+
+    dev = torch.device("cuda", torch.cuda.current_device())
+    try:
+        L.reserve_big_ws(dev, enable=False)
+        whole = add()
+        L.reserve_big_ws(dev, enable=True)              # (the next launch claims the slices' memory for its stream)
+        split = [add() for _ in range(3)]
+    finally:
+        L.reserve_big_ws(dev)
+    assert all(torch.equal(s, split[0]) for s in split) and not torch.equal(split[0], whole)
+    for r in (whole, split[0]):
+        assert float((r[:m].double() - before[:m].double() - 0.5 * want).abs().max()) < 4e-6 * k ** 0.5
+        assert torch.equal(r[m], before[m])
