@@ -120,6 +120,11 @@ def rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.stride(0) % 8 == 0 and w.is_contiguous() and x.data_ptr() % 16 == 0 == w.data_ptr() % 16)
 
 
+def _rows_choice(x: torch.Tensor, w: torch.Tensor, M: int, N: int, K: int, out: int):
+    """:func:`rows_plan` of operands that lie as the kernel needs them (asked last: prompts pay for one comparison)."""
+    return rows_plan(M, N, K, out) if 0 < M <= ROWS_MAX_M and rows_ok(x, w) else None
+
+
 def gemm_rows(x: torch.Tensor, w: torch.Tensor, nf: int, out_kind: int = ROWS_BF16, ranges: int = 1,
               out: torch.Tensor = None) -> torch.Tensor:
     """``x @ w.T`` of up to 32 rows on the row-streaming kernel: bf16, fp32 (with ``ranges`` as planes [ranges, M, N]),
@@ -202,7 +207,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torch.
             return out
         return lib_gemm(x, w, out)
     layout = x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
-    rows = rows_ok(x, w) and (out is None or out.stride(1) == 1)
+    rows = M <= ROWS_MAX_M and rows_ok(x, w) and (out is None or out.stride(1) == 1)
     wide = out is None or out.stride(0) % 8 == 0 == out.data_ptr() % 16
     kind, cfg, splits = select_gemm(M, N, K, layout, out is None or out.is_contiguous(), rows, wide)
     if kind == KIND_ROWS:
@@ -271,6 +276,8 @@ def row_cut(M: int, N: int, K: int, tuned: bool = False) -> int:
 
 
 def _row_parts(M: int, N: int, K: int, tuned: bool = False) -> Tuple[Tuple[int, int], ...]:
+    if M * N < 256 << 16:                # less than a wave
+        return ((0, M),)
     cut = row_cut(M, N, K, tuned)
     return ((0, cut), (cut, M)) if 0 < cut < M else ((0, M),)
 
@@ -288,8 +295,9 @@ def lib_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torc
         ws = _blaslt_ws.get(x.device)
         if ws is None:
             ws = _blaslt_ws[x.device] = torch.empty(BLASLT_WS_BYTES, dtype=torch.uint8, device=x.device)
+        ldx, ldo = x.stride(0), out.stride(0)
         for a, b in _row_parts(M, N, K, True):
-            check(lib().k8s_blaslt_gemm(ptr(x[a:]), x.stride(0), ptr(w), ptr(out[a:]), out.stride(0), b - a, N, K, ptr(ws),
+            check(lib().k8s_blaslt_gemm(ptr(x) + 2 * a * ldx, ldx, ptr(w), ptr(out) + 2 * a * ldo, ldo, b - a, N, K, ptr(ws),
                                         BLASLT_WS_BYTES, stream_ptr(x)), "blaslt_gemm")
         return out
     if out is None:
@@ -304,7 +312,7 @@ def linear_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             and w.is_contiguous():
         M, K = x.shape
         N = w.shape[0]
-        plan = rows_plan(M, N, K, ROWS_F32) if rows_ok(x, w) else None
+        plan = _rows_choice(x, w, M, N, K, ROWS_F32)
         if plan is not None:
             return gemm_rows(x, w, plan[0], ROWS_F32)
         out = torch.empty((M, N), dtype=torch.float32, device=x.device)
@@ -313,8 +321,9 @@ def linear_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         ws = _blaslt_ws.get(x.device)
         if ws is None:
             ws = _blaslt_ws[x.device] = torch.empty(BLASLT_WS_BYTES, dtype=torch.uint8, device=x.device)
+        ldx = x.stride(0)
         for a, b in _row_parts(M, N, K):
-            check(lib().k8s_blaslt_gemm2(ptr(x[a:]), x.stride(0), ptr(w), ptr(out[a:]), N, b - a, N, K, ptr(ws),
+            check(lib().k8s_blaslt_gemm2(ptr(x) + 2 * a * ldx, ldx, ptr(w), ptr(out) + 4 * a * N, N, b - a, N, K, ptr(ws),
                                          BLASLT_WS_BYTES, stream_ptr(x), 1, 1.0), "blaslt_gemm_f32out")
         return out
     return x.float() @ w.float().t()
@@ -341,7 +350,7 @@ def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return linear(x, w)
     M, K = x.shape
     N = w.shape[0]
-    plan = rows_plan(M, N, K, ROWS_F32) if rows_ok(x, w) else None
+    plan = _rows_choice(x, w, M, N, K, ROWS_F32)
     if plan is not None:
         return gemm_rows(x, w, plan[0], ROWS_F32)
     if (_skinny_f32(M, N, K) and x.stride(1) == 1 and x.stride(0) % 8 == 0
@@ -381,7 +390,7 @@ def plane_plan(M: int, N: int, K: int):
     6.4, 7.7 / 6.8;  2048 x 1024 5.7 / 6.1, 6.8 / 6.4;  4096 x 1024 6.2 / 7.6, 7.3 / 7.9, x 3072 10.6 / 13.3, 12.0 / 12.5, x
     6144 16.0 / 15.3, 18.6 / 15.5, x 8192 18.8 / 22.7, 22.1 / 22.5;  5120 x 1024 7.2 / 8.5, 9.2 / 9.0, x 2048 10.5 / 10.9,
     13.3 / 11.7;  2048 x 256 at 24 rows 5.6 / 6.1."""
-    plan = rows_plan(M, N, K, ROWS_F32, True)
+    plan = rows_plan(M, N, K, ROWS_F32, True) if M <= ROWS_MAX_M else None
     if plan is not None:
         return ROWS_CFG + plan[0], plan[1]
     return _plane_plan(M, N, K, _enabled) if 0 < M <= NARROW_MAX_M else (14, 1)
@@ -458,13 +467,14 @@ def proj_add(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, scale: float = 1
     ws = _blaslt_ws.get(x.device)
     if ws is None:
         ws = _blaslt_ws[x.device] = torch.empty(BLASLT_WS_BYTES, dtype=torch.uint8, device=x.device)
+    ldx = x.stride(0)
     for a, b in _row_parts(M, N, K):
-        if big_add_pays(b - a, N, K) and r.data_ptr() % 16 == 0:
-            check(lib().k8s_gemm_big_add(ptr(x[a:]), x.stride(0), ptr(w), ptr(r[a:]), N, b - a, N, K, float(scale),
-                                         stream_ptr(x)), "gemm_big_add")
+        xa, ra = ptr(x) + 2 * a * ldx, ptr(r) + 4 * a * N
+        if big_add_pays(b - a, N, K) and ra % 16 == 0:
+            check(lib().k8s_gemm_big_add(xa, ldx, ptr(w), ra, N, b - a, N, K, float(scale), stream_ptr(x)), "gemm_big_add")
             continue
-        check(lib().k8s_blaslt_gemm2(ptr(x[a:]), x.stride(0), ptr(w), ptr(r[a:]), N, b - a, N, K, ptr(ws), BLASLT_WS_BYTES,
-                                     stream_ptr(x), 2, float(scale)), "blaslt_gemm_add")
+        check(lib().k8s_blaslt_gemm2(xa, ldx, ptr(w), ra, N, b - a, N, K, ptr(ws), BLASLT_WS_BYTES, stream_ptr(x), 2,
+                                     float(scale)), "blaslt_gemm_add")
     return None
 
 
@@ -525,7 +535,7 @@ def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     M, K = x.shape
     N = w.shape[0]
     if _few_ok(x, w):
-        plan = rows_plan(M, N, K, ROWS_RELU2) if K == w.shape[1] else None
+        plan = rows_plan(M, N, K, ROWS_RELU2) if M <= ROWS_MAX_M and K == w.shape[1] else None
         if plan is not None:
             return gemm_rows(x, w, plan[0], ROWS_RELU2)
         skinny = N <= 4096 and K > 512 and M <= (8 if K <= 1536 else 16)
@@ -553,7 +563,7 @@ def glu_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     M, K = x.shape
     I = w.shape[0] // 2
     if _few_ok(x, w):
-        plan = rows_plan(M, I, K, ROWS_SILU) if w.shape == (2 * I, K) else None
+        plan = rows_plan(M, I, K, ROWS_SILU) if M <= ROWS_MAX_M and w.shape == (2 * I, K) else None
         if plan is not None:
             return gemm_rows(x, w, plan[0], ROWS_SILU)
         if 0 < M <= NARROW_MAX_M:
@@ -953,7 +963,7 @@ def swiglu_gemm(y: torch.Tensor, w_gu: torch.Tensor):
     if not (y.is_cuda and y.dtype == torch.bfloat16 and y.stride(1) == 1 and y.stride(0) % 8 == 0
             and w_gu.is_contiguous()):
         return None
-    ch = swiglu_choice(M, w_gu.shape[0], K, rows_ok(y, w_gu))
+    ch = swiglu_choice(M, w_gu.shape[0], K, M <= ROWS_MAX_M and rows_ok(y, w_gu))
     if ch is None:
         return None
     if ch[0] == KIND_BIG:

@@ -75,7 +75,7 @@ def residual(h, x: torch.Tensor) -> torch.Tensor:
 
 def _one_row(x: torch.Tensor, y: Optional[torch.Tensor], out_dtype) -> bool:
     W = x.shape[-1]
-    return (use_hip(x) and x.shape[0] == 1 and x.numel() == W and COLS <= W <= MAX_K and W % COLS == 0 and y is not None
+    return (x.shape[0] == 1 and use_hip(x) and x.numel() == W and COLS <= W <= MAX_K and W % COLS == 0 and y is not None
             and out_dtype == torch.bfloat16 and x.dtype == torch.float32 and x.is_contiguous() and x.data_ptr() % 16 == 0
             and _planes_ok(y, W))
 

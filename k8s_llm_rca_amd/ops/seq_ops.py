@@ -842,11 +842,10 @@ def decay_attention(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor
         # long portions: chunks in parallel (end states from zero, a carry over the chunks, the chunks
         # again from their start states); short ones token by token.  On the matrix cores a portion goes in
         # blocks of 64 tokens, and its chunks are ranges of several blocks
-        lens = [b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:])]
-        mfma = max(lens) >= LIN_MFMA_ROWS and decay_mfma_ok(D, V, x.dtype, x.device) and x.stride(0) % 4 == 0
+        lens, longest = seg._once("lens", lambda: _lens(seg))
+        mfma = longest >= LIN_MFMA_ROWS and decay_mfma_ok(D, V, x.dtype, x.device) and x.stride(0) % 4 == 0
         if mfma:
-            rows = _lin_rows(T, seg.n_seg, H, D, V, lens)
-            cr = seg.chunk_ranges(rows, rows) if rows else None     # (None: no portion is longer than a range)
+            cr, two = seg._once(("decay", H, D, V, LIN_GROUPS), lambda: _lin_plan(seg, T, lens, H, D, V))
         else:
             cr = seg.chunk_ranges(SSM_CHUNK, 2 * SSM_CHUNK) if seg.n_seg * H * V * 8 < SEQ_FILL_LANES else None
         chunks, c0, cs, nch = None, None, None, 0
@@ -858,7 +857,7 @@ def decay_attention(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor
             check(lib().k8s_decay_attn_mfma(ptr(x), x.stride(0), int(silu), ptr(decay), ptr(state), ptr(seg.seg_row0),
                                             ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(out), seg.n_seg, H, D, V,
                                             stream_ptr(x), ptr(chunks), nch, ptr(c0), ptr(cs),
-                                            int(_lin_two(lens, rows if cr is not None else 0, H, V))), "decay_attn_mfma")
+                                            two), "decay_attn_mfma")
             return out
         check(lib().k8s_decay_attn(ptr(x), x.stride(0), _dt(x.dtype), int(silu), ptr(decay), ptr(state),
                                    ptr(seg.seg_row0), ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(out), seg.n_seg, H, D, V,
@@ -908,6 +907,18 @@ def _lin_rows(T: int, n_seg: int, H: int, D: int, V: int, lens: Optional[List[in
         if T >= 5 * longest and (rows >= 512 or per * sum(-(-n // rows) for n in lens if n > rows) > LIN_GROUPS):
             rows = max(LIN_CHUNK, -(-T // (64 * max(1, 2 * LIN_GROUPS // per))) * 64)
     return rows
+
+
+def _lens(seg: SegMeta) -> tuple:
+    lens = [b - a for a, b in zip(seg.row0_host[:-1], seg.row0_host[1:])]
+    return lens, max(lens)
+
+
+def _lin_plan(seg: SegMeta, T: int, lens: List[int], H: int, D: int, V: int) -> tuple:
+    """(ranges as :meth:`SegMeta.chunk_ranges` gives them or None, whether two workgroups share a unit)."""
+    rows = _lin_rows(T, seg.n_seg, H, D, V, lens)
+    cut = seg.chunk_ranges(rows, rows) if rows else None       # (None: no portion is longer than a range)
+    return cut, int(_lin_two(lens, rows if cut is not None else 0, H, V))
 
 
 def _lin_two(lens: List[int], rows: int, H: int, V: int) -> bool:

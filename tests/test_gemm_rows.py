@@ -279,6 +279,18 @@ def test_sums_of_ranges_only_where_they_can_be_stored(m, ld, first, monkeypatch)
 
 
 @gpu
+def test_prompts_do_not_pay_for_the_rule(monkeypatch):
+    """Past the kernel's rows neither the operands nor the rule are looked at: a small prompt's step is host time."""
+    def asked(*a, **k):
+        raise AssertionError("asked")
+    x, w = operands(L.ROWS_MAX_M + 1, 512, 1024)
+    monkeypatch.setattr(L, "rows_ok", asked)
+    monkeypatch.setattr(L, "row_cut", asked)
+    for f in (L.linear, L.linear_f32out, L.proj_f32out, L.proj_planes, L.relu_sq_proj, L.glu_proj):
+        f(x, w)
+
+
+@gpu
 def test_executor_with_the_norms_in_front_of_both_products():
     """One and two rows: the norm in front of the rotated and the gated product, the latter on the widest strips (whatever the
     table says); three and four: apart.  The same bits as all apart, and as without the executor."""
