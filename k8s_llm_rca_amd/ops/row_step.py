@@ -75,7 +75,7 @@ def residual(h, x: torch.Tensor) -> torch.Tensor:
 
 def _one_row(x: torch.Tensor, y: Optional[torch.Tensor], out_dtype) -> bool:
     W = x.shape[-1]
-    return (x.shape[0] == 1 and use_hip(x) and x.numel() == W and COLS <= W <= MAX_K and W % COLS == 0 and y is not None
+    return (use_hip(x) and x.numel() == W and COLS <= W <= MAX_K and W % COLS == 0 and y is not None
             and out_dtype == torch.bfloat16 and x.dtype == torch.float32 and x.is_contiguous() and x.data_ptr() % 16 == 0
             and _planes_ok(y, W))
 
@@ -92,6 +92,9 @@ def _fp32_row(t: torch.Tensor, W: int) -> bool:
 def step(x: torch.Tensor, y: torch.Tensor, one: torch.Tensor, mix: torch.Tensor, nw: torch.Tensor, eps: float, out_dtype,
          again: Optional[tuple] = None, rms: Optional[tuple] = None):
     """:func:`..ops.norm.hyper_step` on one stream that is only added to (``one``, ``mix``: ones; ``x`` [T, 1, W])."""
+    if x.shape[0] != 1:                              # (before anything else: prompts pay for one comparison)
+        return N.hyper_step(x, y, one, mix, inn=one, nw=nw, eps=eps, out_dtype=out_dtype, again=again, rms=rms)
+
     def read():
         return N.hyper_step(x, y, one, mix, inn=one, nw=nw, eps=eps, out_dtype=out_dtype, again=again, rms=rms)
 
@@ -116,6 +119,9 @@ def step(x: torch.Tensor, y: torch.Tensor, one: torch.Tensor, mix: torch.Tensor,
 def dyt_step(x: torch.Tensor, y: Optional[torch.Tensor], sy: float, y2: Optional[torch.Tensor], sy2: float, alpha: float,
              w: Optional[torch.Tensor], b: Optional[torch.Tensor], out_dtype):
     """:func:`..ops.norm.add_dyt`."""
+    if x.shape[0] != 1:
+        return N.add_dyt(x, y, sy, y2, sy2, alpha, w, b, out_dtype=out_dtype)
+
     def read():
         return N.add_dyt(x, y, sy, y2, sy2, alpha, w, b, out_dtype=out_dtype)
 

@@ -183,3 +183,16 @@ def test_one_row_has_the_same_bits_captured_and_not(model):
     (want, none), (got, some) = logits(False), logits(True)
     assert not none and some >= 4
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_more_rows_do_not_pay_for_the_rule(monkeypatch):
+    """From two rows on neither operand is looked at: a small prompt's step is host time."""
+    def asked(*a, **k):
+        raise AssertionError("asked")
+    monkeypatch.setattr(R, "_one_row", asked)
+    monkeypatch.setattr(R, "use_hip", asked)
+    monkeypatch.setattr(N, "hyper_step", lambda *a, **k: "apart")
+    monkeypatch.setattr(N, "add_dyt", lambda *a, **k: "apart")
+    x, y, w = torch.randn(2, 1, 512), torch.randn(2, 512), torch.ones(512)
+    assert R.step(x, y, w, w, w, 1e-6, BF) == "apart"
+    assert R.dyt_step(x[:, 0], y, 1.0, None, 1.0, 0.5, w, w, BF) == "apart"
