@@ -600,9 +600,10 @@ __global__ void __launch_bounds__(256) big_reduce_kernel(const float* __restrict
 // launch that uses it claims it (g_tail_owner), and a launch on any other
 // stream runs without the split tail (whole-tile last wave: slower, never
 // wrong).  k8s_gemm_big_set_ws releases the claim.  The engine
-// claims it explicitly for its compute stream at init (k8s_gemm_big_claim_ws), so a short-lived stream that happens to launch first (a capture's
-// warm-up, a tuning side stream) can no longer take it; claims are serialised
-// by g_tail_mu, so two host threads never both own it.
+// claims it explicitly for its compute stream at init (k8s_gemm_big_claim_ws),
+// so a short-lived stream that happens to launch first (a capture's warm-up, a
+// tuning side stream) can no longer take it; claims are serialised by g_tail_mu,
+// so two host threads never both own it.
 constexpr int kTailUnits = 256;
 constexpr size_t kTailWsBytes = (size_t)kTailUnits * BM * BN * 4 + kTailUnits * 4;
 static void* g_tail_ws[16] = {};

@@ -210,7 +210,8 @@ static int row_step_any(int norm, int out, const RowStep& a, const void* w, void
 
 static bool row_step_ok(const RowStep& a, const void* w, const void* y, int N, int K, int nf, int ranges, int out) {
   auto off = [](const void* p, int n) { return ((uintptr_t)p % n) != 0; };
-  return a.x && a.x_out && a.x_out != a.x && a.y && a.yp >= 1 && a.yp <= kStepPlanes && a.w && w && y && N > 0 && K >= kStepCols && K <= kStepMaxK &&
+  return a.x && a.x_out && a.x_out != a.x && a.y && a.yp >= 1 && a.yp <= kStepPlanes && a.w && w && y && N > 0 &&
+         K >= kStepCols && K <= kStepMaxK &&
          ranges >= 1 && K % (kStepCols * ranges) == 0 && (nf == 1 || nf == 2) && (ranges == 1 || out == kStepF32) &&
          !off(a.x, 16) && !off(a.x_out, 16) && !off(a.y, 16) && !off(a.y2, 16) && !off(a.w, 16) && !off(a.b, 16) &&
          !off(a.h_out, 8) && !off(a.emb, 8) && !off(w, 16);
@@ -240,7 +241,8 @@ K8S_API int k8s_gemm_row_step_dyt(const float* x, float* x_out, const float* y, 
   RowStep a{};
   a.x = x, a.x_out = x_out, a.y = y, a.yp = yp, a.sy = sy, a.y2 = y2, a.yp2 = yp2, a.sy2 = sy2, a.alpha = alpha;
   a.w = nw, a.b = nb, a.h_out = (uint16_t*)h_out;
-  if (!row_step_ok(a, w, out, N, K, nf, ranges, kind) || !nb || (y2 && (yp2 < 1 || yp2 > kStepPlanes))) return (int)hipErrorInvalidValue;
+  if (!row_step_ok(a, w, out, N, K, nf, ranges, kind) || !nb || (y2 && (yp2 < 1 || yp2 > kStepPlanes)))
+    return (int)hipErrorInvalidValue;
   return nf == 1 ? row_step_any<2>(kStepDyt, kind, a, w, out, N, K, ranges, s)
                  : row_step_any<4>(kStepDyt, kind, a, w, out, N, K, ranges, s);
 }

@@ -186,7 +186,8 @@ __device__ __forceinline__ bf16x8 tld16(const uint16_t* p) { return *reinterpret
 // masked, 16 heads over 2 of 128, 7 rows at 1000 keys 11.2 / 9.6, 64 at 2000 35 / 35; 16 over 16 of 64, 16 rows at 200 (256
 // workgroups) 6.3 / 6.0, 32 at 200 (512) 8.1 / 7.3, 16 at 512 (768) 13.0 / 13.9, 64 at 512 30 / 34; 8 over 8 of 64 + 128 7.4 / 7.7
 // and of 128 + 128 8.2 / 8.4 at 4 and 7 rows.  Latent, 16 heads of 256 + 64, 7 rows at 1000 12.3 / 10.8, 32 at 512 (160) 13.9 /
-// 12.4, 16 at 2000 (256) 13.6 / 13.9, 64 at 512 (320) 18.6 / 19.3; of 512 + 64 18.3 / 15.4, 39 / 41 at 64 rows; of 64 + 32 7.5 / 7.7.
+// 12.4, 16 at 2000 (256) 13.6 / 13.9, 64 at 512 (320) 18.6 / 19.3; of 512 + 64 18.3 / 15.4, 39 / 41 at 64 rows; of 64 + 32
+// 7.5 / 7.7.
 template <bool TURN>
 __device__ __forceinline__ bf16x8 tok_turn(bf16x8 v, int from) {
   if constexpr (TURN) {
@@ -521,8 +522,8 @@ K8S_API int k8s_latent_attn_token(const void* qa, long qst, long qsh, const void
                                   const float* sink, void* out, long ost, long osh, float* po, float* pml, int n_parts,
                                   int part, int most, int H, int R, int BS, int window, float scale, hipStream_t s) {
   if (rows <= 0) return 0;
-  if (!k8s_latent_attn_mfma_ok(R, RP) || BS % 32 || H <= 0 || n_parts < 1 || n_parts > most || part <= 0 || part % 32 || (RP && !qr) ||
-      window < 0 || qst % 8 || qsh % 8 || (n_parts > 1 && (!pml || !po)))
+  if (!k8s_latent_attn_mfma_ok(R, RP) || BS % 32 || H <= 0 || n_parts < 1 || n_parts > most || part <= 0 || part % 32 ||
+      (RP && !qr) || window < 0 || qst % 8 || qsh % 8 || (n_parts > 1 && (!pml || !po)))
     return (int)hipErrorInvalidValue;
   LatTokArgs a;
   a.qa = (const uint16_t*)qa; a.qst = qst; a.qsh = qsh; a.qr = (const uint16_t*)qr; a.c = (const uint16_t*)c;

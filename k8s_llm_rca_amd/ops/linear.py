@@ -488,7 +488,8 @@ def proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     M, K = x.shape
     N = w.shape[0]
     if (16 < M <= NARROW_MAX_M and 32 <= N <= 32 * NARROW_WGS and K <= 2048 and (N, K) not in _dispatch and _few_ok(x, w)
-            and rows_plan(M, N, K) is None and (K < 1536 or N > 2048 or M <= 64 and N * K >= 9 << 18) and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
+            and rows_plan(M, N, K) is None and (K < 1536 or N > 2048 or M <= 64 and N * K >= 9 << 18)
+            and stream_shape_ok(M, N, K, _narrow_cfg(M), 1)):
         return gemm_stream(x, w, _narrow_cfg(M), 1)
     return linear(x, w)
 

@@ -66,7 +66,9 @@ def test_rms_pass_in_front(n, k, planes, rn, add):
     nw = (1 + 0.1 * torch.randn(k, generator=g)).cuda()
     one = torch.ones(1, device="cuda")
     ss = (torch.rand(1, rn, generator=g) * 100).cuda() if rn else None
-    again = (torch.tensor([3], dtype=torch.int32, device="cuda"), torch.randn(5, k, generator=g).to(BF).cuda(), 4.5) if add else None
+    again = None
+    if add:
+        again = torch.tensor([3], dtype=torch.int32, device="cuda"), torch.randn(5, k, generator=g).to(BF).cuda(), 4.5
     kw = dict(again=again, rms=(ss, 2048.0, 1e-5) if rn else None)
     x1 = x0.clone()
     h = N.hyper_step(x1, y, one, one.view(1, 1), inn=one, nw=nw, eps=1e-5, out_dtype=BF, **kw)
