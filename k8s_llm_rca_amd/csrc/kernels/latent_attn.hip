@@ -39,7 +39,6 @@ namespace k8s {
 //
 // NP: 32-number chunks of the cache row behind the latent (a score-only key part): row width R + 32 NP.
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr int kBatch = 8;      // fragments that are read from LDS at once
 
 struct LatArgs {
   const uint16_t* qa;     // element (t, h, c) at t * qst + h * qsh + c
@@ -127,9 +126,13 @@ __device__ __forceinline__ void lat_softmax(const f32x4 (&s)[2], float scale_log
 // lie 16 apart and each is a lookup of its own in the first-level cache); 3517 and 4351 rows 107 -> 96 -> 87 and 183 -> 157
 // -> 149.  Not quicker: two tiles a wave and one wave a SIMD (669 before the last change), eight waves to a workgroup that
 // share the keys of 8 items (495: all wait at one barrier), a row's 128 bytes in eight lanes (465).
+// With two tiles (R up to 128) a fragment is used twice and more workgroups share a compute unit, so that registers count: us
+// through registers / batches of 8 / 4 / 2: 16 heads of R 64, two of 4000 rows 208 / 247 / 234 / 187; 24 heads of 96, 3000 rows
+// behind 1000 199 / 270 / 185 / 184; 16 heads of 96 + 64, 16 of 700 73 / 68 / 65 / 57.
 template <int NR, int NP, int MT, int OCC>
 __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs a) {
   constexpr int R = NR * 32, ND = R / 16, NC = NR + NP, RW = R + 32 * NP, NF = 2 * NC + ND, NFW = (NF + 3) / 4;
+  constexpr int BATCH = MT > 1 ? 2 : 8;                       // fragments that are read from LDS at once
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   bf16x8* frag = reinterpret_cast<bf16x8*>(lds_raw);          // [2][NF][64]
   __shared__ int kend_s[4], kbeg_s[4];
@@ -211,7 +214,7 @@ __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs 
     fetch(k_beg, page_of(k_beg), 0);
     page = page_of(k_beg + 32);
   }
-  // The fragments in the order of their use: keys (both tiles in turn), then values; batches of kBatch, the next one asked for
+  // The fragments in the order of their use: keys (both tiles in turn), then values; batches, the next one asked for
   // once the first of a batch is there -- the compiler waits for all LDS reads in flight where LDS-DMA is about.
   auto slot = [](int j) { return j < 2 * NC ? (j & 1) * NC + (j >> 1) : j; };
   int buf = 0;
@@ -222,20 +225,20 @@ __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs 
     const bf16x8* fb = frag + (size_t)buf * NF * 64 + at;
     const bool open = kb + 31 <= pos0 && (a.window <= 0 || kb >= pos0 + ntok - a.window);
     f32x4 s[MT][2];
-    bf16x8 pf[MT], fr[2][kBatch];
+    bf16x8 pf[MT], fr[2][BATCH];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) s[mt][0] = s[mt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto read = [&](int b) {
 #pragma unroll
-      for (int i = 0; i < kBatch; ++i)
-        if (b * kBatch + i < NF) fr[b & 1][i] = fb[slot(b * kBatch + i) * 64];
+      for (int i = 0; i < BATCH; ++i)
+        if (b * BATCH + i < NF) fr[b & 1][i] = fb[slot(b * BATCH + i) * 64];
     };
     read(0);
 #pragma unroll
-    for (int b = 0; b * kBatch < NF; ++b) {
+    for (int b = 0; b * BATCH < NF; ++b) {
 #pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        const int j = b * kBatch + i;
+      for (int i = 0; i < BATCH; ++i) {
+        const int j = b * BATCH + i;
         if (j >= NF) continue;
         if (j == 2 * NC) {
 #pragma unroll
@@ -251,7 +254,7 @@ __global__ void __launch_bounds__(256, OCC) latent_attn_mfma_lds_kernel(LatArgs 
         }
         if (i == 0) {
           __builtin_amdgcn_sched_barrier(0);
-          if ((b + 1) * kBatch < NF) read(b + 1);
+          if ((b + 1) * BATCH < NF) read(b + 1);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
