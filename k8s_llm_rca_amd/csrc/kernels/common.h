@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define K8S_API extern "C" __attribute__((visibility("default")))
 
 namespace k8s {
@@ -129,6 +131,21 @@ __device__ __forceinline__ float sum_planes(const float* p, size_t step, int n) 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// The wave's sum in its last lane (only), on the vector pipe alone: no trip through LDS for an exchange.
+__device__ __forceinline__ float wave_sum_dpp(float v) {
+  auto add = [&](auto ctrl, auto rows) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, decltype(rows)::value, 0xf, false));
+  };
+  using std::integral_constant;
+  add(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});   // lanes 1, 2, 4, 8 before, within rows of 16
+  add(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});   // the row before's last lane, into rows 1 and 3
+  add(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});   // lane 31, into rows 2 and 3
   return v;
 }
 

@@ -39,6 +39,17 @@ struct RowsRope {
   int nq, nkv, BS;
 };
 
+// How x comes: as it is; normed by every workgroup (NormIn); or the product's rows are divided by the root mean square of what
+// x was made from (RowScale), whose sums of squares a gemm_step (gemm_step.hip) left in parts.
+enum RowsIn { kRowsPlain = 0, kRowsNorm = 1, kRowsScaled = 2 };
+constexpr int kRowsParts = 256;          // parts of a row's sum of squares, at most: four a lane
+
+struct RowScale {
+  const float* part;     // [M][parts]
+  int parts;             // a multiple of 4
+  float width, eps;
+};
+
 // LDS of one wave: what its lanes wrote is there for its other lanes
 __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -52,11 +63,14 @@ constexpr int rows_lds(int MT, int NF, int CH) { return 16 * NF * (CH > 32 * MT 
 // grid (strips, K ranges); K range of kslice = 4 waves x whole chunks.  Forms of two halves (SwiGLU: gate and up rows, rope:
 // entries d and d + 64 of a head) take 8 NF rows of each.  NORM: x is the normed row block that the workgroup makes itself
 // (norm_prologue.h) while its first weights are on their way; the row's own loads are asked for in front of them (6144 x 4096
-// rotated 13.5 -> 11.6 us, 28672 x 4096 SwiGLU 39.4 -> 37.6, on four fragments instead of one 36.3).
-template <int MT, int NF, int CH, int OUT, bool NORM>
+// rotated 13.5 -> 11.6 us, 28672 x 4096 SwiGLU 39.4 -> 37.6, on four fragments instead of one 36.3).  Scaled: a wave sums the
+// parts of up to four rows, asked for in front of the weights, and every sum is multiplied before it is rounded or stored.
+template <int MT, int NF, int CH, int OUT, int IN>
 __global__ void __launch_bounds__(kRowsWaves * 64, 2)
     gemm_rows_kernel(const uint16_t* __restrict__ x, int ldx, const uint16_t* __restrict__ w, void* __restrict__ y, int ldy,
-                     int M, int N, int K, int kslice, RowsRope rp, NormIn nin) {
+                     int M, int N, int K, int kslice, RowsRope rp, NormIn nin, RowScale rsc) {
+  constexpr bool NORM = IN == kRowsNorm, SCALED = IN == kRowsScaled;
+  static_assert(!SCALED || MT == 1);
   constexpr bool kHalves = OUT == kRowsSilu || OUT == kRowsRope;
   constexpr int HR = 8 * NF;            // rows of a half
   constexpr int PP = CH / 8;            // 16-byte pieces of a row's chunk
@@ -135,6 +149,13 @@ __global__ void __launch_bounds__(kRowsWaves * 64, 2)
   NormRow nrow;
   u16x8 nwv[kNormMaxChunks];
   if constexpr (NORM) norm_ask(nrow, nwv, 0, M, nin);
+  f32x4 pv[SCALED ? 4 : 1];
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)                                   // (past the last row or part: the last ones again, not used)
+      pv[q] = *reinterpret_cast<const f32x4*>(rsc.part + (size_t)min(wv + kRowsWaves * q, M - 1) * rsc.parts +
+                                              min(4 * lane, rsc.parts - 4));
+  }
   __builtin_amdgcn_sched_barrier(0);
   load_w(0, 0);
   __builtin_amdgcn_sched_barrier(0);
@@ -145,6 +166,15 @@ __global__ void __launch_bounds__(kRowsWaves * 64, 2)
   if constexpr (NORM) {
     __shared__ float nscr[16];
     norm_rows_to_lds<true>(k8s_norm_lds, M, nin, blockIdx.x == 0 && blockIdx.y == 0, nscr, nrow, nwv);
+  }
+  __shared__ float factor[SCALED ? 16 : 1];
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float ss = wave_sum_dpp(4 * lane < rsc.parts ? pv[q][0] + pv[q][1] + pv[q][2] + pv[q][3] : 0.f);
+      if (lane == 63) factor[wv + kRowsWaves * q] = 1.f / sqrtf(ss / rsc.width + rsc.eps);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
   if (nch > 1) {
     int c = 0;
@@ -179,6 +209,7 @@ __global__ void __launch_bounds__(kRowsWaves * 64, 2)
     float t = p[0];
 #pragma unroll
     for (int q = 1; q < kRowsWaves; ++q) t += p[q * WL / 2];
+    if constexpr (SCALED) t *= factor[m];
     return t;
   };
   uint16_t* yb = reinterpret_cast<uint16_t*>(y);
@@ -227,9 +258,10 @@ __global__ void __launch_bounds__(kRowsWaves * 64, 2)
   }
 }
 
-template <int MT, int NF, int CH, bool NORM>
+template <int MT, int NF, int CH, int IN>
 static int rows_launch(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int ranges, int out,
-                       const RowsRope& rp, const NormIn& nin, hipStream_t s) {
+                       const RowsRope& rp, const NormIn& nin, const RowScale& rsc, hipStream_t s) {
+  constexpr bool NORM = IN == kRowsNorm;
   const bool halves = out == kRowsSilu || out == kRowsRope;
   const int strip = (halves ? 8 : 16) * NF, cols = out == kRowsRope ? N / 2 : N;   // rope: columns counted as pairs
   if (M <= 0 || M > 16 * MT || (NORM && M > kNormMaxRows) || N <= 0 || N % (out == kRowsRope ? 128 : 1) || cols % strip ||
@@ -241,12 +273,19 @@ static int rows_launch(const void* x, int ldx, const void* w, void* y, int ldy, 
   const dim3 g(cols / strip, ranges), b(kRowsWaves * 64);
   const size_t lds = NORM ? (size_t)M * K * 2 : 0;
 #define K8S_ROWS(OUT)                                                                                                   \
-  hipLaunchKernelGGL((gemm_rows_kernel<MT, NF, CH, OUT, NORM>), g, b, lds, s, (const uint16_t*)x, ldx, (const uint16_t*)w, y, \
-                     ldy, M, N, K, K / ranges, rp, nin)
+  hipLaunchKernelGGL((gemm_rows_kernel<MT, NF, CH, OUT, IN>), g, b, lds, s, (const uint16_t*)x, ldx, (const uint16_t*)w, y, \
+                     ldy, M, N, K, K / ranges, rp, nin, rsc)
   if constexpr (NORM) {
     switch (out) {
       case kRowsSilu: K8S_ROWS(kRowsSilu); break;
       case kRowsRope: K8S_ROWS(kRowsRope); break;
+      default: return (int)hipErrorInvalidValue;
+    }
+  } else if constexpr (IN == kRowsScaled) {
+    switch (out) {
+      case kRowsBf16: K8S_ROWS(kRowsBf16); break;
+      case kRowsF32: K8S_ROWS(kRowsF32); break;
+      case kRowsSilu: K8S_ROWS(kRowsSilu); break;
       default: return (int)hipErrorInvalidValue;
     }
   } else {
@@ -263,17 +302,17 @@ static int rows_launch(const void* x, int ldx, const void* w, void* y, int ldy, 
   return (int)hipGetLastError();
 }
 
-template <bool NORM>
+template <int IN>
 static int rows_any(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int nf, int ranges, int out,
-                    const RowsRope& rp, const NormIn& nin, hipStream_t s) {
-#define K8S_ROWS_AS(MT, NF, CH) return rows_launch<MT, NF, CH, NORM>(x, ldx, w, y, ldy, M, N, K, ranges, out, rp, nin, s)
+                    const RowsRope& rp, const NormIn& nin, const RowScale& rsc, hipStream_t s) {
+#define K8S_ROWS_AS(MT, NF, CH) return rows_launch<MT, NF, CH, IN>(x, ldx, w, y, ldy, M, N, K, ranges, out, rp, nin, rsc, s)
   if (M <= 16) {
     switch (nf) {
       case 1: K8S_ROWS_AS(1, 1, 128);
       case 2: K8S_ROWS_AS(1, 2, 128);
       case 4: K8S_ROWS_AS(1, 4, 64);
     }
-  } else if constexpr (!NORM) {
+  } else if constexpr (IN == kRowsPlain) {
     switch (nf) {
       case 2: K8S_ROWS_AS(2, 2, 64);
       case 4: K8S_ROWS_AS(2, 4, 64);
@@ -293,7 +332,16 @@ using namespace k8s;
 K8S_API int k8s_gemm_rows(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int nf, int ranges,
                           int out, hipStream_t s) {
   if (out < kRowsBf16 || out > kRowsRelu2) return (int)hipErrorInvalidValue;
-  return rows_any<false>(x, ldx, w, y, ldy, M, N, K, nf, ranges, out, RowsRope{}, NormIn{}, s);
+  return rows_any<kRowsPlain>(x, ldx, w, y, ldy, M, N, K, nf, ranges, out, RowsRope{}, NormIn{}, RowScale{}, s);
+}
+
+// The same for up to 16 rows, row m divided by sqrt(sum(part[m]) / width + eps).  out: 0 bf16, 1 fp32, 2 SwiGLU.
+K8S_API int k8s_gemm_rows_scaled(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int nf, int ranges,
+                                 int out, const float* part, int parts, float width, float eps, hipStream_t s) {
+  if (!part || ((uintptr_t)part & 15) || parts < 4 || parts % 4 || parts > kRowsParts || M > 16 || !(width > 0.f))
+    return (int)hipErrorInvalidValue;
+  return rows_any<kRowsScaled>(x, ldx, w, y, ldy, M, N, K, nf, ranges, out, RowsRope{}, NormIn{},
+                               RowScale{part, parts, width, eps}, s);
 }
 
 // qkv = x . w^T (w = [q heads; k heads; v heads] x 128 rows) with q and k rotated and k, v written to their pages: what
@@ -303,7 +351,7 @@ K8S_API int k8s_gemm_rows_rope(const void* x, int ldx, const void* w, void* qkv,
                                int BS, hipStream_t s) {
   if (N != (nq + 2 * nkv) * 128 || !pos || !cos_sin || BS <= 0) return (int)hipErrorInvalidValue;
   const RowsRope rp{pos, cos_sin, slots, (uint16_t*)kc, (uint16_t*)vc, nq, nkv, BS};
-  return rows_any<false>(x, ldx, w, qkv, ldq, M, N, K, nf, 1, kRowsRope, rp, NormIn{}, s);
+  return rows_any<kRowsPlain>(x, ldx, w, qkv, ldq, M, N, K, nf, 1, kRowsRope, rp, NormIn{}, RowScale{}, s);
 }
 
 // The SwiGLU (pos null) or rotating form on X = rmsnorm(x [or the planes `part`] + res_in) * norm_w, made by every workgroup
@@ -321,5 +369,5 @@ K8S_API int k8s_gemm_rows_norm(const void* x, int x_stride, const float* part, i
   const NormIn nin{(const uint16_t*)x, part, (const uint16_t*)res_in, (uint16_t*)res_out, (const uint16_t*)norm_w,
                    x_stride, splits, K, eps};
   const RowsRope rp{pos, cos_sin, slots, (uint16_t*)kc, (uint16_t*)vc, nq, nkv, BS};
-  return rows_any<true>(nullptr, 0, w, y, ldy, M, N, K, nf, 1, pos ? kRowsRope : kRowsSilu, rp, nin, s);
+  return rows_any<kRowsNorm>(nullptr, 0, w, y, ldy, M, N, K, nf, 1, pos ? kRowsRope : kRowsSilu, rp, nin, RowScale{}, s);
 }

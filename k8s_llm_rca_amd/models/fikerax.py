@@ -32,7 +32,7 @@ import torch
 from ..ops import norm as N
 from ..ops import row_step as R
 from ..ops import seq_ops as S
-from ..ops.linear import proj, proj_add, proj_f32out, proj_planes
+from ..ops.linear import proj, proj_add, proj_planes
 from ..parallel.groups import ParallelContext, single
 
 TAIL_ALIGN = 32     # the rotated key part of a latent cache row is filled up to a multiple of this
@@ -420,6 +420,7 @@ class FikeraxModel:
         cfg, eps, dt = self.cfg, self.cfg.norm_eps, self.dtype
         T, one = inp.input_ids.shape[0], self.one
         idx = S.wanted_rows(inp)
+        few = idx is None or T <= R.INTO_ROWS              # (few rows: the same products whichever of them are wanted)
         mix1 = one.view(1, 1)
         tables: Dict[int, torch.Tensor] = {}
         again = (inp.input_ids, self.embed, cfg.embed_scale)
@@ -432,7 +433,7 @@ class FikeraxModel:
             if r + 1 < len(self.runs):
                 j, add = self.runs[r + 1]
                 nxt = dict(nw=self.layers[j]["norm1"], again=again if add else None)
-            elif idx is None:                              # every row is wanted: the last write-back reads the head's input
+            elif few:                                      # the last write-back reads the head's input
                 nxt = dict(nw=self.final_norm)
             rms = None                                     # what the residual's pass makes up for behind the projection
             if spec.kind == "lightning":
@@ -444,28 +445,20 @@ class FikeraxModel:
             x = R.residual(h, x)
             w = L["wo"]
             if spec.ff:
-                y = proj_add(x[:, 0], y, w) if rms is None else proj_planes(y, w)
-                h = (N.hyper_read(x, None, L["norm2"], eps, dt) if y is None
-                     else R.step(x, y, one, mix1, L["norm2"], eps, dt, rms=rms))
+                h = R.add_product(x, y, w, one, mix1, L["norm2"], eps, dt, rms=rms)
                 y, w, rms = R.glu_proj(h, L["w13"]), L["w2"], None               # silu(gate) * up
                 x = R.residual(h, x)
-            # (a pass that reads the embedding once more adds the product too)
-            embeds = nxt is not None and nxt.get("again")
-            y = proj_planes(y, w) if embeds or rms is not None else proj_add(x[:, 0], y, w)
             if layers_out is not None:                     # the residual in front of the embedding added once more
                 after = x.clone()
-                if y is not None:
-                    N.hyper_step(after, y, one, mix1, rms=rms)
+                N.hyper_step(after, proj_planes(y, w), one, mix1, rms=rms)
                 layers_out.append(after[:, 0])
-            if y is None:
-                h = N.hyper_read(x, None, nxt["nw"], eps, dt) if nxt else None
-            elif nxt:
-                h = R.step(x, y, one, mix1, eps=eps, out_dtype=dt, rms=rms, **nxt)
+            if nxt:
+                h = R.add_product(x, y, w, one, mix1, eps=eps, out_dtype=dt, rms=rms, **nxt)
             else:
-                N.hyper_step(x, y, one, mix1, rms=rms)
-        if idx is not None:
-            h = N.hyper_read(x, idx, self.final_norm, eps, dt)
-            return proj_f32out(h, self.head)
+                y = proj_planes(y, w) if rms is not None else proj_add(x[:, 0], y, w)
+                if y is not None:
+                    N.hyper_step(x, y, one, mix1, rms=rms)
+        h = R.rows(h, idx) if few else N.hyper_read(x, idx, self.final_norm, eps, dt)
         return R.proj_f32out(h, self.head)
 
 

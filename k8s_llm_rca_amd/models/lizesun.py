@@ -36,7 +36,7 @@ import torch
 from ..ops import norm as N
 from ..ops import row_step as R
 from ..ops import seq_ops as S
-from ..ops.linear import proj_add, proj_f32out
+from ..ops.linear import proj_f32out
 from ..parallel.groups import ParallelContext, single
 
 
@@ -435,37 +435,36 @@ class LizesunModel:
         cfg, dt = self.cfg, self.dtype
         T, W, nl = inp.input_ids.shape[0], cfg.hidden, cfg.n_layers
         idx = S.wanted_rows(inp)
+        few = nl > 0 and (idx is None or T <= R.INTO_ROWS)   # (few rows: the same products whichever of them are wanted)
         x = torch.empty(T, W, dtype=torch.float32, device=self.device)
         first = self.layers[0]["norm1"] if nl else (1.0, None, None)
         h = N.embed_scale_dyt(inp.input_ids, self.embed, cfg.embed_scale, x, *first, out_dtype=dt)
         vmix: dict = {}
         tables: dict = {}
         for li, (spec, L) in enumerate(zip(cfg.layers, self.layers)):
-            # (the final norm reads the wanted rows only, or with the last layer where every row is wanted)
-            nxt = (self.layers[li + 1]["norm1"] if li + 1 < nl
-                   else (1.0, None, None) if idx is not None else self.final_norm)
+            # (the final norm reads the wanted rows only, or with the last layer where every row is wanted or there are few)
+            nxt = self.layers[li + 1]["norm1"] if li + 1 < nl else self.final_norm if few else (1.0, None, None)
             after = L["norm2"] if spec.ff else nxt
             if spec.kind == "parallel":
                 ol, orr = self._parallel(li, h, inp, kcs, vcs, vts, states, tables)
                 x = R.residual(h, x)
-                yl = proj_add(x, ol, L["wo_l"], spec.left_scale)
-                yr = proj_add(x, orr, L["wo_r"], spec.right_scale)
-                add = (yl, spec.left_scale, yr, spec.right_scale) if yl is not None else (yr, spec.right_scale, None, 1.0)
-                h = R.dyt_step(x, *add, *after, out_dtype=dt)
+                h = R.dyt_product(x, ol, L["wo_l"], spec.left_scale, orr, L["wo_r"], spec.right_scale, *after, out_dtype=dt)
             else:
                 o = (self._chunk_attention(li, h, inp, kcs, vcs, vts, vmix) if spec.kind == "attention"
                      else self._delta(li, h, inp, states))
                 x = R.residual(h, x)
-                h = R.dyt_step(x, proj_add(x, o, L["wo"]), 1.0, None, 1.0, *after, out_dtype=dt)
+                h = R.dyt_product(x, o, L["wo"], 1.0, None, None, 1.0, *after, out_dtype=dt)
             if spec.ff:
                 u = R.relu_sq_proj(h, L["w_up"])
                 x = R.residual(h, x)
-                h = R.dyt_step(x, proj_add(x, u, L["w_down"]), 1.0, None, 1.0, *nxt, out_dtype=dt)
+                h = R.dyt_product(x, u, L["w_down"], 1.0, None, None, 1.0, *nxt, out_dtype=dt)
             if layers_out is not None:
                 if isinstance(h, R.RowStep):
                     h = h.read()                                       # the residual as it is behind this layer
                 layers_out.append(x.clone())
-        if idx is not None or not nl:
+        if few:
+            h = R.rows(h, idx)
+        else:
             xr = x.index_select(0, idx).contiguous() if idx is not None else x
             h = N.add_dyt(xr, None, 1.0, None, 1.0, *self.final_norm, out_dtype=dt)
         return R.proj_f32out(h, self.lm_head)

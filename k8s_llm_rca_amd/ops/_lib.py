@@ -38,6 +38,9 @@ _SIGS = {
     "k8s_sample": [P, I, I, I, I, P, P, P, P, P, I, P, P, P, P, P, P, I, P, P, P, I],
     "k8s_gemm_skinny": [P, I, P, P, I, I, I, I, P],
     "k8s_gemm_rows": [P, I, P, P, I, I, I, I, I, I, I, P],
+    "k8s_gemm_rows_scaled": [P, I, P, P, I, I, I, I, I, I, I, P, I, F, F, P],
+    "k8s_gemm_step_rms": [P, I, P, P, P, I, F, F, P, P, F, P, P, P, I, I, I, P],
+    "k8s_gemm_step_dyt": [P, I, P, F, P, I, P, F, P, F, P, P, P, I, I, I, P],
     "k8s_gemm_stream_reduce": [P, I, P, I, I, I, P],
     "k8s_gemm_rows_rope": [P, I, P, P, I, I, I, I, I, P, P, P, P, P, I, I, I, P],
     "k8s_gemm_rows_norm": [P, I, P, I, P, P, P, F, P, P, I, I, I, I, I, P, P, P, P, P, I, I, I, P],

@@ -68,6 +68,15 @@ class RowStep:
         return out
 
 
+def rows(h, idx: Optional[torch.Tensor]):
+    """The activations of some rows (None: of all)."""
+    if idx is None:
+        return h
+    if isinstance(h, RowStep):
+        h = h.read()
+    return h.index_select(0, idx) if isinstance(h, torch.Tensor) else h.rows(idx)
+
+
 def residual(h, x: torch.Tensor) -> torch.Tensor:
     """The residual behind a product of ``h``: ``x`` itself, or where the pass put it."""
     return h.x.view(x.shape) if isinstance(h, RowStep) else x
@@ -139,22 +148,137 @@ def dyt_step(x: torch.Tensor, y: Optional[torch.Tensor], sy: float, y2: Optional
     return RowStep(x, L.ROWS_RELU2, launch, read)
 
 
+# ------------------------------------ a sublayer's last product with the residual's pass in its epilogue (gemm_step.hip)
+INTO_ROWS, INTO_LOADS, INTO_STRIP, PARTS = 16, (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16), 8, 256
+
+
+def into_ok(m: int, n: int, k: int, two: bool = False) -> bool:
+    """Whether a product of ``m`` rows takes the residual's pass into its epilogue (``two``: two products of K ``k`` do).
+
+    Every workgroup of 8 columns reads all of X, and with few columns there are few of them, where planes may cut K.  us of
+    planes and the norm's pass / of the fused product, and with the tanh pass:  2048 x 8192 at 1, 4, 8 rows 10.2 / 8.1, 11.0 /
+    8.9, 11.2 / 10.1 and 10.2 / 8.1, 10.4 / 8.8, 10.6 / 10.1, at 16 rows (8.4 and the pass) 13.5;  2048 x 2048 at 1, 8, 16
+    rows 6.5 / 4.4, 6.7 / 5.0, 6.9 / 5.8;  x 4096 at 16 8.9 / 8.2 and 8.2 / 8.2.  More columns: 3072 x 2048 at 12, 16 rows 8.5 /
+    7.6, 8.7 / 8.4 and 7.6 / 7.7, 7.9 / 8.2;  4096 x 4096 at 8, 12 rows 11.5 / 10.3, 11.8 / 12.4 and 10.5 / 10.1, 10.8 / 12.4;
+    6144 x 8192 at 2, 8 rows 26.5 / 21.9, 26.0 / 26.9.  Fewer:  1024 x 4096 at 8, 12 rows 7.0 / 6.2, 7.1 / 7.3;  1024 x 8192 at
+    2, 4 rows 8.1 / 7.5, 8.2 / 8.4;  512 x 4096 at 2, 8 rows 5.8 / 5.0, 5.8 / 6.1, x 8192 at 1 6.2 / 6.9, x 2048 at 16 5.7 / 5.4."""
+    waves = 4 if two else 8
+    if not (0 < m <= INTO_ROWS and n > 0 and n % INTO_STRIP == 0 and k % (64 * waves) == 0
+            and k // (64 * waves) in INTO_LOADS and (n, k) not in L.dispatch_table()):
+        return False
+    k *= 2 if two else 1
+    if n < 1536:
+        return k <= 2048 or k <= 4096 and m * k <= (32768 if n >= 1024 else 8192)
+    return m * k * -(-n // 2048) <= (65536 if n <= 2048 else 49152)
+
+
+class Scaled:
+    """Activations whose rows are still to be divided by the root mean square of the residual ``x``: what the products below
+    do to their sums.  ``part``: that residual's sums of squares in parts."""
+
+    def __init__(self, x: torch.Tensor, h: torch.Tensor, part: torch.Tensor, nw: torch.Tensor, eps: float):
+        self.x, self.h, self.part, self.nw, self.eps = x, h, part, nw, eps
+
+    def read(self) -> torch.Tensor:
+        """The activations by the separate pass over the residual."""
+        return N.hyper_read(self.x, None, self.nw, self.eps, self.h.dtype) if self.h.shape[0] else self.h
+
+    def rows(self, idx: torch.Tensor) -> "Scaled":
+        return Scaled(*(t.index_select(0, idx) for t in (self.x, self.h, self.part)), self.nw, self.eps)
+
+    def product(self, w: torch.Tensor, out_kind: int, plain, planes: bool = False, keep: bool = False):
+        (m, k), n = self.h.shape, w.shape[0] // (2 if out_kind == L.ROWS_SILU else 1)
+        if (out_kind == L.ROWS_RELU2 or keep or k != w.shape[1] or w.shape[0] % 2 and out_kind == L.ROWS_SILU
+                or not L.rows_ok(self.h, w) or (("silu", w.shape[0], k) in L.dispatch_table()) or (n, k) in L.dispatch_table()):
+            return plain(self.read(), w)
+        p = L.rows_plan(m, n, k, out_kind, planes)
+        if p is None:
+            return plain(self.read(), w)
+        out = torch.empty((p[1], m, n) if planes else (m, n), device=w.device,
+                          dtype=torch.float32 if out_kind == L.ROWS_F32 else w.dtype)
+        check(lib().k8s_gemm_rows_scaled(ptr(self.h), k, ptr(w), ptr(out), n, m, n, k, p[0], p[1], out_kind, ptr(self.part),
+                                         self.part.shape[1], float(k), float(self.eps), stream_ptr(w)), "gemm_rows_scaled")
+        return out
+
+
+def _into_operands(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, out_dtype) -> bool:
+    return (a.is_cuda and out_dtype == torch.bfloat16 and x.dtype == torch.float32 and x.is_contiguous()
+            and w.shape == (x.shape[-1], a.shape[1]) and w.device == x.device == a.device and L.rows_ok(a, w))
+
+
+def add_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, one: torch.Tensor, mix: torch.Tensor, nw: torch.Tensor,
+                eps: float, out_dtype, again: Optional[tuple] = None, rms: Optional[tuple] = None):
+    """The next sublayer's input behind ``x += a @ w.T`` (:func:`step` of that product): activations, :class:`RowStep` or
+    :class:`Scaled`."""
+    if a.shape[0] <= INTO_ROWS:                      # (before anything else: prompts pay for one comparison)
+        h = _rms_into(x, a, w, nw, eps, out_dtype, again, rms)
+        if h is not None:
+            return h
+    if again is None and rms is None:
+        y = L.proj_add(x[:, 0], a, w)
+        if y is None:
+            return N.hyper_read(x, None, nw, eps, out_dtype)
+    else:                                            # (a pass that reads the embedding once more adds the product too)
+        y = L.proj_planes(a, w)
+    return step(x, y, one, mix, nw, eps, out_dtype, again=again, rms=rms)
+
+
+def _rms_into(x, a, w, nw, eps, out_dtype, again, rms) -> Optional[Scaled]:
+    (m, k), W = a.shape, x.shape[-1]
+    ids, embed, escale = again if again is not None else (None, None, 0.0)
+    ss, width, reps = rms if rms is not None else (None, 1.0, 0.0)
+    if not (into_ok(m, W, k) and _into_operands(x, a, w, out_dtype) and x.shape[:2] == (m, 1) and W % 32 == 0
+            and W // INTO_STRIP <= PARTS and _fp32_row(nw, W)
+            and (ss is None or ss.dtype == torch.float32 and ss.is_contiguous() and ss.shape[0] == m
+                 and 0 < ss.numel() <= SUMS * m)
+            and (ids is None or ids.dtype == torch.int32 and ids.is_contiguous() and ids.numel() == m
+                 and embed.dtype == out_dtype and embed.is_contiguous() and embed.shape[1] == W)):
+        return None
+    h = torch.empty(m, W, dtype=out_dtype, device=x.device)
+    part = torch.empty(m, W // INTO_STRIP, dtype=torch.float32, device=x.device)
+    check(lib().k8s_gemm_step_rms(ptr(a), a.stride(0), ptr(w), ptr(x), ptr(ss), ss.numel() // m if ss is not None else 0,
+                                  float(width), float(reps), ptr(ids), ptr(embed), float(escale), ptr(nw), ptr(h), ptr(part),
+                                  m, W, k, stream_ptr(x)), "gemm_step_rms")
+    return Scaled(x, h, part, nw, eps)
+
+
+def dyt_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, sy: float, a2: Optional[torch.Tensor],
+                w2: Optional[torch.Tensor], sy2: float, alpha: float, nw: Optional[torch.Tensor], nb: Optional[torch.Tensor],
+                out_dtype):
+    """The next sublayer's input behind ``x += sy a @ w.T (+ sy2 a2 @ w2.T)`` (:func:`dyt_step` of those products)."""
+    (m, k), W = a.shape, x.shape[-1]
+    if (m <= INTO_ROWS and nw is not None and into_ok(m, W, k, a2 is not None) and _into_operands(x, a, w, out_dtype)
+            and x.shape == (m, W) and (a2 is None or a2.shape == a.shape and _into_operands(x, a2, w2, out_dtype))
+            and _fp32_row(nw, W) and _fp32_row(nb, W)):
+        h = torch.empty(m, W, dtype=out_dtype, device=x.device)
+        check(lib().k8s_gemm_step_dyt(ptr(a), a.stride(0), ptr(w), float(sy), ptr(a2), a2.stride(0) if a2 is not None else 0,
+                                      ptr(w2), float(sy2), ptr(x), float(alpha), ptr(nw), ptr(nb), ptr(h), m, W, k,
+                                      stream_ptr(x)), "gemm_step_dyt")
+        return h
+    y = L.proj_add(x, a, w, sy)
+    if a2 is None:
+        return dyt_step(x, y, sy, None, 1.0, alpha, nw, nb, out_dtype)
+    y2 = L.proj_add(x, a2, w2, sy2)
+    add = (y, sy, y2, sy2) if y is not None else (y2, sy2, None, 1.0)
+    return dyt_step(x, *add, alpha, nw, nb, out_dtype)
+
+
 # ------------------------------------------------------------------------- products of activations, or of what makes them
 def proj(h, w: torch.Tensor, keep: bool = False) -> torch.Tensor:
-    return h.product(w, L.ROWS_BF16, L.proj, keep=keep) if isinstance(h, RowStep) else L.proj(h, w)
+    return L.proj(h, w) if isinstance(h, torch.Tensor) else h.product(w, L.ROWS_BF16, L.proj, keep=keep)
 
 
 def proj_f32out(h, w: torch.Tensor) -> torch.Tensor:
-    return h.product(w, L.ROWS_F32, L.proj_f32out) if isinstance(h, RowStep) else L.proj_f32out(h, w)
+    return L.proj_f32out(h, w) if isinstance(h, torch.Tensor) else h.product(w, L.ROWS_F32, L.proj_f32out)
 
 
 def proj_planes(h, w: torch.Tensor) -> torch.Tensor:
-    return h.product(w, L.ROWS_F32, L.proj_planes, planes=True) if isinstance(h, RowStep) else L.proj_planes(h, w)
+    return L.proj_planes(h, w) if isinstance(h, torch.Tensor) else h.product(w, L.ROWS_F32, L.proj_planes, planes=True)
 
 
 def glu_proj(h, w: torch.Tensor) -> torch.Tensor:
-    return h.product(w, L.ROWS_SILU, L.glu_proj) if isinstance(h, RowStep) else L.glu_proj(h, w)
+    return L.glu_proj(h, w) if isinstance(h, torch.Tensor) else h.product(w, L.ROWS_SILU, L.glu_proj)
 
 
 def relu_sq_proj(h, w: torch.Tensor) -> torch.Tensor:
-    return h.product(w, L.ROWS_RELU2, L.relu_sq_proj) if isinstance(h, RowStep) else L.relu_sq_proj(h, w)
+    return L.relu_sq_proj(h, w) if isinstance(h, torch.Tensor) else h.product(w, L.ROWS_RELU2, L.relu_sq_proj)
