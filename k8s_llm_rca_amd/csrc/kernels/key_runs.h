@@ -23,4 +23,7 @@ __device__ __forceinline__ KeyRuns key_runs(int pos, int chunk, int window, int 
   return k;
 }
 
+// A value mixed with another layer's of the same token, the same bits in every kernel that does it.
+__device__ __forceinline__ float mix_value(float lam, float v, float other) { return fmaf(lam, other, (1.f - lam) * v); }
+
 }  // namespace k8s

@@ -207,7 +207,7 @@ __device__ __forceinline__ void write_values(const float* __restrict__ x, int qs
         if (k < nr) {
           const size_t o = (size_t)(r0 + k) * NV + c;
           if (v_keep) v_keep[o] = v[k];
-          if (v_other) v[k] = (1.f - lam) * v[k] + lam * vo[k];
+          if (v_other) v[k] = mix_value(lam, v[k], vo[k]);
         }
     }
     if (vt && run) {

@@ -235,24 +235,140 @@ __device__ __forceinline__ void tok_softmax(const float (&p)[8], int hq, float& 
   l += ps;
 }
 
+// The rows as their projection left them (fp32 planes: q | k | v), for the form that prepares them itself.
+struct TokPrep {
+  const float* x;         // [planes][T][qs], planes pstep apart
+  const float* bias;      // [(H + G) D + G V] or null
+  const float* q_w;       // [D] or null: the norm's weights
+  const float* k_w;
+  const float* cs;        // [T][rot]: cos | sin
+  const float* v_other;   // [T][G V] or null: v = (1 - lam) v + lam v_other
+  float* v_keep;          // [T][G V] or null: v as projected
+  const int* slots;
+  uint16_t* vc;           // [pages][BS][G V] or null
+  size_t pstep;
+  int qs, planes, rot, norm;
+  float eps, lam;
+};
+
+// LDS written before is there for the whole workgroup; leaves loads from memory in flight
+__device__ __forceinline__ void step_barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// What a thread prepares of a row: asked for first, used once the keys are on their way (more than four planes: added as they
+// come).  The arithmetic of attn_prep_half_kernel and write_values (masked_attn.hip).
+struct TokRow {
+  static constexpr int NP = 4;
+  f32x4 a[NP], b[NP], wa, wb, ba, bb, co, si;
+  __device__ __forceinline__ static f32x4 any4(const float* p) {      // of any alignment
+    f32x4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+  }
+  __device__ __forceinline__ static void ask(const TokPrep& p, const float* x, f32x4 (&v)[NP]) {
+    if (p.planes <= NP) {
+#pragma unroll
+      for (int k = 0; k < NP; ++k) v[k] = *reinterpret_cast<const f32x4*>(x + min(k, p.planes - 1) * p.pstep);
+    } else {
+      v[0] = sum_planes4(x, p.pstep, p.planes);
+    }
+  }
+  __device__ __forceinline__ static f32x4 sum(const TokPrep& p, const f32x4 (&v)[NP]) {
+    f32x4 t = v[0];
+#pragma unroll
+    for (int k = 1; k < NP; ++k)
+      if (k < p.planes && p.planes <= NP) t += v[k];
+    return t;
+  }
+  __device__ __forceinline__ void ask_head(const TokPrep& p, int row, int c0, int ia, int ib, bool turn, const float* w,
+                                           int half) {
+    const float* x = p.x + (size_t)row * p.qs + c0;
+    ask(p, x + ia, a);
+    ask(p, x + ib, b);
+    wa = wb = f32x4{1.f, 1.f, 1.f, 1.f};
+    ba = bb = co = si = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (w) wa = any4(w + ia), wb = any4(w + ib);
+    if (p.bias) ba = any4(p.bias + c0 + ia), bb = any4(p.bias + c0 + ib);
+    if (turn) {
+      const float* c = p.cs + (size_t)row * p.rot + ia;
+      co = *reinterpret_cast<const f32x4*>(c), si = *reinterpret_cast<const f32x4*>(c + half);
+    }
+  }
+  __device__ __forceinline__ void ask_value(const TokPrep& p, int row, int c0, size_t vo) {
+    ask(p, p.x + (size_t)row * p.qs + c0, a);
+    ba = wa = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (p.bias) ba = any4(p.bias + c0);
+    if (p.v_other) wa = *reinterpret_cast<const f32x4*>(p.v_other + vo);
+  }
+  template <int LPH>
+  __device__ __forceinline__ void head(const TokPrep& p, int D, bool turn, u16x4& ha, u16x4& hb) const {
+    f32x4 va = sum(p, a), vb = sum(p, b);
+    if (p.bias) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        va[k] += ba[k];
+        vb[k] += bb[k];
+      }
+    }
+    if (turn) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float ua = va[k], ub = vb[k];
+        va[k] = ua * co[k] - ub * si[k];
+        vb[k] = ub * co[k] + ua * si[k];
+      }
+    }
+    float rn = 1.f;
+    if (p.norm) {
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) ss = fmaf(va[k], va[k], fmaf(vb[k], vb[k], ss));
+#pragma unroll
+      for (int o = 1; o < LPH; o <<= 1) ss += __shfl_xor(ss, o, 64);
+      rn = 1.f / sqrtf(ss / (float)D + p.eps);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      ha[k] = f2bf(va[k] * (rn * wa[k]));
+      hb[k] = f2bf(vb[k] * (rn * wb[k]));
+    }
+  }
+  __device__ __forceinline__ u16x4 value(const TokPrep& p, size_t vo, bool store) const {
+    f32x4 v = sum(p, a);
+    if (p.bias) v += ba;
+    if (p.v_keep && store) *reinterpret_cast<f32x4*>(p.v_keep + vo) = v;
+    u16x4 h;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) h[k] = f2bf(p.v_other ? mix_value(p.lam, v[k], wa[k]) : v[k]);
+    return h;
+  }
+};
+
 struct MaskTokArgs {
   const uint16_t* q;      // [T][H * D] (H: heads x maps)
-  const uint16_t* kc;     // [pages][BS][G * maps * D]
-  const uint16_t* vt;     // [pages][G * V][BS]
+  uint16_t* kc;           // [pages][BS][G * maps * D]  (written by the form that prepares)
+  uint16_t* vt;           // [pages][G * V][BS]
   const int* bt;
   int maxb;
   const int* items;       // [rows][4]: segment, row, 1, position
   int G, BS, chunk, window, keep_first, part_blocks, most;   // a part: part_blocks, or more where most parts are too few
   float scale, softcap;
   TokOut t;
+  TokPrep p;
 };
 
 // grid (rows, key heads (x maps) x groups of 16 of their heads, parts); a part is a run of the row's list of 32-key blocks
 // (kept first tokens, then the window's or chunk's).
-template <int NDC, int NV, bool CAP, int NW, bool TURN>
+//
+// PREP (steps in which every sequence has one row): the pass between the projection and the attention (attn_prep_half_kernel,
+// masked_attn.hip: planes, bias, rotation, norm, the caches' rows) is made here, where it was a launch of 4 us with a handful
+// of workgroups.  Every workgroup prepares its own heads' queries; the one whose part ends with the row's position also its
+// key and value, which it writes to the pages and puts into the fragments of its last block itself.  The row is asked for in
+// front of the pages and keys, which are on their way while it is prepared.  The arithmetic, and every bit, is the pass's.
+template <int NDC, int NV, bool CAP, int NW, bool TURN, bool PREP>
 __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs a) {
   constexpr int D = NDC * 32, V = NV * 16;
   __shared__ TokLds<NW, V> lds;
+  __shared__ __attribute__((aligned(16))) uint16_t qs[PREP ? 16 * D : 8], ks[PREP ? D : 8], vs[PREP ? V : 8];
   const int lane = threadIdx.x & 63, r = lane & 15, hq = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sg = a.items[blockIdx.x * 4], row = a.items[blockIdx.x * 4 + 1], pos = a.items[blockIdx.x * 4 + 3];
@@ -270,10 +386,28 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
     tok_empty(a.t, head0, nh, blockIdx.z);
     return;
   }
+  // ---- the row as projected: D / 8 neighbouring threads a head of q or k, four entries of v a thread
+  constexpr int LPH = D / 8;
+  const int tid = threadIdx.x, kt = nh * LPH, vt0 = kt + LPH;        // the first threads of k and of v
+  const bool ends = PREP && b_lo + nb == nblk, heads = PREP && tid < (ends ? vt0 : kt);
+  const bool vals = ends && tid >= vt0 && tid < vt0 + V / 4;
+  const int j = tid % LPH, half = PREP ? a.p.rot >> 1 : 0, sl = ends ? a.p.slots[row] : -1;
+  const bool isk = tid >= kt, turn = PREP && 8 * j < a.p.rot;
+  const int pa = turn ? 4 * j : 8 * j, pb2 = turn ? pa + half : pa + 4;
+  const int c0 = isk ? (H + g) * D : (head0 + tid / LPH) * D, vc0 = (H + a.G) * D + gv * V + 4 * (tid - vt0);
+  TokRow tr;
+  if constexpr (PREP) {
+    if (heads)
+      tr.ask_head(a.p, row, c0, pa, pb2, turn, isk ? a.p.k_w : a.p.q_w, half);
+    else if (vals)
+      tr.ask_value(a.p, row, vc0, (size_t)row * NVt + gv * V + 4 * (tid - vt0));
+  }
   bf16x8 qf[NDC];
-  const uint16_t* qp = a.q + (size_t)row * H * D + (size_t)(head0 + min(r, nh - 1) * M) * D;
+  if constexpr (!PREP) {
+    const uint16_t* qp = a.q + (size_t)row * H * D + (size_t)(head0 + min(r, nh - 1) * M) * D;
 #pragma unroll
-  for (int cc = 0; cc < NDC; ++cc) qf[cc] = tld16(qp + 32 * cc + 8 * hq);
+    for (int cc = 0; cc < NDC; ++cc) qf[cc] = tld16(qp + 32 * cc + 8 * hq);
+  }
   float m = -INFINITY, l = 0.f;
   f32x4 o[NV];
 #pragma unroll
@@ -310,11 +444,58 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
   };
   if (my > 0) load(0, 0);
   if (my > 1) load(1, 1);
+  if constexpr (PREP) {
+    if (heads) {
+      u16x4 ha, hb;
+      tr.head<LPH>(a.p, D, turn, ha, hb);
+      uint16_t* to = isk ? ks : qs + (tid / LPH) * D;
+      *reinterpret_cast<u16x4*>(to + pa) = ha;
+      *reinterpret_cast<u16x4*>(to + pb2) = hb;
+      if (isk && sl >= 0 && hc == 0) {
+        uint16_t* kp = a.kc + (size_t)sl * NK + g * D;
+        *reinterpret_cast<u16x4*>(kp + pa) = ha;
+        *reinterpret_cast<u16x4*>(kp + pb2) = hb;
+      }
+    } else if (vals) {
+      const int c = gv * V + 4 * (tid - vt0);
+      const u16x4 v = tr.value(a.p, (size_t)row * NVt + c, hc == 0);
+      *reinterpret_cast<u16x4*>(vs + 4 * (tid - vt0)) = v;
+      if (sl >= 0 && hc == 0) {
+        uint16_t* vp = a.vt + ((size_t)(sl / a.BS) * NVt + c) * a.BS + sl % a.BS;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) vp[(size_t)k * a.BS] = v[k];
+        if (a.p.vc) *reinterpret_cast<u16x4*>(a.p.vc + (size_t)sl * NVt + c) = v;
+      }
+    }
+    step_barrier_lds();
+#pragma unroll
+    for (int cc = 0; cc < NDC; ++cc) qf[cc] = *reinterpret_cast<const bf16x8*>(qs + min(r, nh - 1) * D + 32 * cc + 8 * hq);
+  }
+  // the row's own key and value into the fragments of the block that holds its position
+  auto own = [&](int u) {
+    if (!PREP || sl < 0 || kb[u] + 32 <= pos) return;
+    const int at = pos - kb[u];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      if (8 * (lr >> 2) + 4 * t + (lr & 3) == at) {
+#pragma unroll
+        for (int cc = 0; cc < NDC; ++cc) kf[u][t][cc] = *reinterpret_cast<const bf16x8*>(ks + 32 * cc + 8 * lh);
+      }
+    if (lh == at >> 3) {
+#pragma unroll
+      for (int dt = 0; dt < NV; ++dt) {
+        const __bf16 v = __builtin_bit_cast(__bf16, vs[16 * dt + lr]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) vf[u][dt][i] = i == (at & 7) ? v : vf[u][dt][i];
+      }
+    }
+  };
   const int cq_lo = a.chunk > 0 ? (pos / a.chunk) * a.chunk : 0, wq_lo = a.window > 0 ? pos - a.window + 1 : 0;
   for (int k = 0; k < my; k += 2) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       if (k + u >= my) break;
+      own(u);
       float p[8];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -432,16 +613,16 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
   tok_join<NW, ND>(lds, a.t, row, head0, nh, blockIdx.y, m, l, o);
 }
 
-template <int NDC, int NV, int NW>
+template <int NDC, int NV, int NW, bool PREP>
 static int launch_mask_tok_nw(const MaskTokArgs& a, int rows, hipStream_t s) {
   const int hpg = a.t.H / (a.G * a.t.hs);
   const dim3 grid(rows, a.G * a.t.hs * ((hpg + 15) / 16), a.t.n_parts);
-  auto k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, false>
-                           : masked_attn_token_kernel<NDC, NV, false, NW, false>;
+  auto k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, false, PREP>
+                           : masked_attn_token_kernel<NDC, NV, false, NW, false, PREP>;
   if constexpr (NV == 2 * NDC && (NDC == 2 || NW == 8))      // keys as long as values, heads that share keys or are of 64
     if ((long)rows * grid.y * grid.z <= kTurnMasked)
-      k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, true>
-                          : masked_attn_token_kernel<NDC, NV, false, NW, true>;
+      k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, true, PREP>
+                          : masked_attn_token_kernel<NDC, NV, false, NW, true, PREP>;
   hipLaunchKernelGGL(k, grid, dim3(64 * NW), 0, s, a);
   if (a.t.n_parts > 1)
     hipLaunchKernelGGL(token_merge_kernel, dim3(rows * a.t.H), dim3(256), 0, s, a.t, a.items, NV * 16);
@@ -454,12 +635,27 @@ static int launch_mask_tok_nw(const MaskTokArgs& a, int rows, hipStream_t s) {
 // eight waves / this / tiles of 16 tokens:  16 heads over 16 of 128, 1 key 3.8 / 3.8 / 6.6 and 12.9 / 8.0 / 7.3, 200 keys
 // 6.6 / 7.5 / 20 and 28 / 24 / 32, 4000 keys 11.1 / 12.2 / 37 and 480 / 399 / 442;  12 over 6 of 64 at 4000 keys 64 rows
 // 122 / 78 / 94;  4 over 4 of 64 8.5 / 8.7 / 25 and 75 / 45 / 65.
+template <int NDC, int NV, bool PREP>
+static int launch_mask_tok_as(const MaskTokArgs& a, int rows, hipStream_t s) {
+  if constexpr (NDC == 2 && NV == 4)
+    return launch_mask_tok_nw<NDC, NV, 4, PREP>(a, rows, s);
+  else
+    return a.t.H > a.G * a.t.hs ? launch_mask_tok_nw<NDC, NV, 8, PREP>(a, rows, s)
+                                : launch_mask_tok_nw<NDC, NV, 2, PREP>(a, rows, s);
+}
 template <int NDC, int NV>
 static int launch_mask_tok(const MaskTokArgs& a, int rows, hipStream_t s) {
-  if constexpr (NDC == 2 && NV == 4)
-    return launch_mask_tok_nw<NDC, NV, 4>(a, rows, s);
-  else
-    return a.t.H > a.G * a.t.hs ? launch_mask_tok_nw<NDC, NV, 8>(a, rows, s) : launch_mask_tok_nw<NDC, NV, 2>(a, rows, s);
+  if constexpr (NDC != 3)
+    if (a.p.x) return launch_mask_tok_as<NDC, NV, true>(a, rows, s);
+  return launch_mask_tok_as<NDC, NV, false>(a, rows, s);
+}
+
+static int mask_tok_any(const MaskTokArgs& a, int D, int V, int rows, hipStream_t s) {
+  if (D == 96) return launch_mask_tok<3, 6>(a, rows, s);
+  if (D == 64 && V == 64) return launch_mask_tok<2, 4>(a, rows, s);
+  if (D == 64 && V == 128) return launch_mask_tok<2, 8>(a, rows, s);
+  if (D == 128 && V == 64) return launch_mask_tok<4, 4>(a, rows, s);
+  return launch_mask_tok<4, 8>(a, rows, s);
 }
 
 template <int NR, int NP>
@@ -503,17 +699,41 @@ K8S_API int k8s_masked_attn_token(const void* q, const void* kc, const void* vt,
       part_blocks < 1 || maps < 1 || most < 1 || n_parts > most || (n_parts > 1 && (!pml || !po)))
     return (int)hipErrorInvalidValue;
   MaskTokArgs a;
-  a.q = (const uint16_t*)q; a.kc = (const uint16_t*)kc; a.vt = (const uint16_t*)vt; a.bt = bt; a.maxb = maxb;
+  a.q = (const uint16_t*)q; a.kc = (uint16_t*)kc; a.vt = (uint16_t*)vt; a.bt = bt; a.maxb = maxb;
   a.items = items; a.G = G; a.BS = BS; a.chunk = chunk; a.window = window; a.keep_first = keep_first;
   a.part_blocks = part_blocks; a.most = most; a.scale = scale; a.softcap = softcap;
   a.t.sink = sink; a.t.gate = gate; a.t.gs = gs; a.t.out = out_f32 ? nullptr : (uint16_t*)out;
   a.t.out32 = out_f32 ? (float*)out : nullptr; a.t.ost = (long)H * maps * V; a.t.osh = V;
   a.t.po = po; a.t.pml = pml; a.t.H = H * maps; a.t.n_parts = n_parts; a.t.hs = maps;
-  if (D == 96) return launch_mask_tok<3, 6>(a, rows, s);
-  if (D == 64 && V == 64) return launch_mask_tok<2, 4>(a, rows, s);
-  if (D == 64 && V == 128) return launch_mask_tok<2, 8>(a, rows, s);
-  if (D == 128 && V == 64) return launch_mask_tok<4, 4>(a, rows, s);
-  return launch_mask_tok<4, 8>(a, rows, s);
+  a.p = TokPrep{};
+  return mask_tok_any(a, D, V, rows, s);
+}
+
+// The same on rows as their projection left them, every row the only one of its sequence (TokPrep): what k8s_attn_prep_half
+// and k8s_masked_attn_token give.  D 64 or 128, qs and pstep multiples of 4, rot a multiple of 8 with its table, x / kc / cs /
+// v_other / v_keep 16-byte aligned; vc may be null.
+K8S_API int k8s_masked_attn_token_prep(const float* x, int qs, int planes, long pstep, const float* bias, const float* q_w,
+                                       const float* k_w, float eps, int norm, const float* cs, int rot, float lam,
+                                       const float* v_other, float* v_keep, const int* slots, void* vc, void* kc, void* vt,
+                                       const int* bt, int maxb, const int* items, int rows, const float* sink,
+                                       const float* gate, int gs, void* out, int H, int G, int D, int V, int BS, int chunk,
+                                       int window, int keep_first, float scale, float softcap, hipStream_t s, int part_blocks,
+                                       int most, int n_parts, float* pml, float* po) {
+  if (rows <= 0) return 0;
+  auto off = [](const void* p) { return ((uintptr_t)p & 15) != 0; };
+  if (!k8s_masked_attn_mfma_ok(H, G, D, V) || D == 96 || BS % 32 || chunk < 0 || window < 0 || keep_first < 0 || n_parts < 1 ||
+      part_blocks < 1 || most < 1 || n_parts > most || (n_parts > 1 && (!pml || !po)) || !x || qs % 4 || planes < 1 ||
+      (planes > 1 && pstep % 4) || rot < 0 || rot > D || rot % 8 || (rot && !cs) || norm < 0 || norm > 1 || !slots || !kc ||
+      !vt || off(x) || off(cs) || off(kc) || off(v_other) || off(v_keep) || ((uintptr_t)vc & 7))
+    return (int)hipErrorInvalidValue;
+  MaskTokArgs a;
+  a.q = nullptr; a.kc = (uint16_t*)kc; a.vt = (uint16_t*)vt; a.bt = bt; a.maxb = maxb;
+  a.items = items; a.G = G; a.BS = BS; a.chunk = chunk; a.window = window; a.keep_first = keep_first;
+  a.part_blocks = part_blocks; a.most = most; a.scale = scale; a.softcap = softcap;
+  a.t.sink = sink; a.t.gate = gate; a.t.gs = gs; a.t.out = (uint16_t*)out; a.t.out32 = nullptr;
+  a.t.ost = (long)H * V; a.t.osh = V; a.t.po = po; a.t.pml = pml; a.t.H = H; a.t.n_parts = n_parts; a.t.hs = 1;
+  a.p = TokPrep{x, bias, q_w, k_w, cs, v_other, v_keep, slots, (uint16_t*)vc, (size_t)pstep, qs, planes, rot, norm, eps, lam};
+  return mask_tok_any(a, D, V, rows, s);
 }
 
 // items [rows][4]; n_parts > 1: po [rows][H][n_parts][R], pml [rows][H][n_parts][2]

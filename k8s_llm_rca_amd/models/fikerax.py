@@ -387,10 +387,9 @@ class FikeraxModel:
     def _attention(self, i: int, h, inp: S.SegStepInputs, tables, kc, vc, vt) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
         x = R.proj_planes(h, L["w_in"])
-        q = S.attn_prep(x, L["b_in"], c.heads, c.kv_heads, c.dim, c.vdim, inp.positions, inp.slots, kc, vc, self.dtype,
-                        norm="head", eps=self.cfg.norm_eps, rope=self.ropes[i], rope_cs=self._table(i, inp, tables), vt=vt)
-        o = S.masked_attention(q, c.heads, c.kv_heads, c.dim, c.vdim, kc, vc, inp.seg, c.scale, window=c.window, vt=vt)
-        return o
+        prep = dict(norm="head", eps=self.cfg.norm_eps, rope=self.ropes[i], rope_cs=self._table(i, inp, tables))
+        return S.prep_attention(x, L["b_in"], c.heads, c.kv_heads, c.dim, c.vdim, inp.positions, inp.slots, kc, vc, vt, inp.seg,
+                                self.dtype, c.scale, prep, dict(window=c.window))
 
     def _latent_attention(self, i: int, h, inp: S.SegStepInputs, tables, cache, cache_t) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix

@@ -388,12 +388,10 @@ class LizesunModel:
                 keep = vmix["v"] = torch.empty(x.shape[0], G * V, dtype=torch.float32, device=x.device)
             else:
                 other = vmix["v"]
-        q = S.attn_prep(x[:, :H * D + G * (D + V)], L["bias"], H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci],
-                        self.dtype, norm=True, q_w=L["q_w"], k_w=L["k_w"], eps=self.cfg.norm_eps, lam=L["lam"],
-                        v_other=other, v_keep=keep, vt=vts[ci])
-        o = S.masked_attention(q, H, G, D, V, kcs[ci], vcs[ci], inp.seg, a.scale, softcap=a.softcap, chunk=a.chunk,
-                               gate=x[:, H * D + G * (D + V):], vt=vts[ci])
-        return o
+        n = H * D + G * (D + V)
+        prep = dict(norm=True, q_w=L["q_w"], k_w=L["k_w"], eps=self.cfg.norm_eps, lam=L["lam"], v_other=other, v_keep=keep)
+        return S.prep_attention(x[:, :n], L["bias"], H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg,
+                                self.dtype, a.scale, prep, dict(softcap=a.softcap, chunk=a.chunk, gate=x[:, n:]))
 
     def _parallel(self, li: int, h, inp: S.SegStepInputs, kcs, vcs, vts, states, tables: dict):
         L, spec = self.layers[li], self.cfg.layers[li]
@@ -406,10 +404,9 @@ class LizesunModel:
         rope = self.ropes.get(key)
         if rope is not None and key not in tables:                     # cos | sin of the step's positions, made once
             tables[key] = S.rope_table(inp.positions, rope)
-        q = S.attn_prep(x[:, :nl], None, H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], self.dtype, norm=True,
-                        eps=self.cfg.norm_eps, rope=rope, rope_cs=tables.get(key), vt=vts[ci])
-        ol = S.masked_attention(q, H, G, D, V, kcs[ci], vcs[ci], inp.seg, a.scale, window=a.window,
-                                keep_first=a.keep_first, sink=L["sink"], vt=vts[ci])
+        prep = dict(norm=True, eps=self.cfg.norm_eps, rope=rope, rope_cs=tables.get(key))
+        ol = S.prep_attention(x[:, :nl], None, H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg,
+                              self.dtype, a.scale, prep, dict(window=a.window, keep_first=a.keep_first, sink=L["sink"]))
         xr = x[:, nl:]
         orr = S.memory_layer(xr, b.heads, b.dim, b.vdim, L["gate_bias"], b.gate_cap, states[f"mem{j}"], states[f"memn{j}"],
                              states[f"memm{j}"], inp.seg, L["mem_norm"], self.cfg.norm_eps, self.dtype)

@@ -1318,6 +1318,65 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
     return out
 
 
+# Workgroups up to which the attention of single tokens prepares rows of 64-entry heads itself: past that the registers that
+# hold the row take workgroups off the compute units.  us apart / together, 16 heads over 16 of 64:  7 rows at 700 keys (336
+# workgroups) 15.7 / 14.4, 16 at 450 (512) 17.2 / 16.2, 7 at 1500 (672) 20.9 / 23.8, 64 at 512 (2048) 40 / 47.  Heads of 128
+# gain at any number:  16 over 2 of 128 at 1 row and 100 keys 8.1 / 7.0, 7 at 700 14.0 / 12.2, 64 at 512 19.4 / 17.8;  8 over 8
+# 8.9 / 8.0, 16.4 / 14.1, 41 / 38, 64 at 1500 (3072) 91 / 89.
+PREP_GROUPS = 512
+
+
+def prep_attention(x: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D: int, V: int, positions: torch.Tensor,
+                   slots: torch.Tensor, kc: torch.Tensor, vc: Optional[torch.Tensor], vt: Optional[torch.Tensor], seg: SegMeta,
+                   out_dtype, scale: float, prep: dict, mask: dict) -> torch.Tensor:
+    """:func:`attn_prep` (keywords ``prep``) and :func:`masked_attention` (keywords ``mask``) of the same rows; in one launch
+    where every sequence has one row."""
+    o = _prep_tokens(x, bias, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, **prep, **mask)
+    if o is not None:
+        return o
+    q = attn_prep(x, bias, H, G, D, V, positions, slots, kc, vc, out_dtype, vt=vt, **prep)
+    return masked_attention(q, H, G, D, V, kc, vc, seg, scale, vt=vt, **mask)
+
+
+def _prep_tokens(x, bias, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, norm=False, q_w=None, k_w=None, eps=0.0,
+                 lam=0.0, v_other=None, v_keep=None, rope=None, rope_cs=None, softcap=0.0, chunk=0, window=0, keep_first=0,
+                 sink=None, gate=None) -> Optional[torch.Tensor]:
+    T = x.shape[-2]
+    if T != seg.n_seg:                               # (before anything else: prompts pay for one comparison)
+        return None
+    planes, pstep = (x.shape[0], x.stride(0)) if x.dim() == 3 else (1, 0)
+    rot, NV, cols = rope.dims if rope is not None else 0, G * V, (H + G) * D + G * V
+    if not (use_hip(x) and vt is not None and D in (64, 128) and norm in (False, None, True, "head")
+            and seg.singles() == T and masked_mfma_ok(H, G, D, V, out_dtype, x.device) and x.dtype == torch.float32
+            and x.shape[-1] == cols and x.stride(-1) == 1 and x.stride(-2) % 4 == 0 and pstep % 4 == 0
+            and (rope is None or not rope.pairs and rope_cs is not None and rot % 8 == 0 and rot <= D)):
+        return None
+    BS = kc.shape[1]
+    small = ((bias, cols), (q_w, D), (k_w, D), (v_other, T * NV), (v_keep, T * NV), (rope_cs, T * rot), (sink, H))
+    if not (all(t is None or t.dtype == torch.float32 and t.is_contiguous() and t.numel() == n for t, n in small)
+            and all(t is None or t.data_ptr() % 16 == 0 for t in (x, kc, vc, rope_cs, v_other, v_keep))
+            and all(t is None or t.is_contiguous() and t.dtype == out_dtype for t in (kc, vc, vt))
+            and kc.shape[2] == G * D and (vc is None or vc.shape[2] == NV) and vt.shape[1:] == (NV, BS) and BS % 32 == 0
+            and slots.dtype == torch.int32 and slots.is_contiguous() and seg.block_tables.is_contiguous()
+            and chunk >= 0 and window >= 0 and keep_first >= 0
+            and (gate is None or gate.dtype == torch.float32 and gate.stride(1) == 1 and gate.shape[1] >= H)):
+        return None
+    rows, parts, _, _, _, _ = seg._once(("mask plan", H, G, D, V, chunk, window, keep_first, 1),
+                                        lambda: _mask_plan(seg, H, G, D, V, int(chunk), int(window), int(keep_first), 1))
+    if D == 64 and T * G * -(-(H // G) // 16) * parts > PREP_GROUPS:
+        return None
+    out = torch.empty(T, H * V, dtype=out_dtype, device=x.device)
+    groups, po, pml = _token_groups(rows, H, parts, V)
+    for it in groups:
+        check(lib().k8s_masked_attn_token_prep(
+            ptr(x), x.stride(-2), planes, pstep, ptr(bias), ptr(q_w), ptr(k_w), float(eps), int(bool(norm)), ptr(rope_cs), rot,
+            float(lam), ptr(v_other), ptr(v_keep), ptr(slots), ptr(vc), ptr(kc), ptr(vt), ptr(seg.block_tables),
+            seg.block_tables.shape[1], ptr(it), it.shape[0], ptr(sink), ptr(gate), gate.stride(0) if gate is not None else 0,
+            ptr(out), H, G, D, V, BS, int(chunk), int(window), int(keep_first), float(scale), float(softcap), stream_ptr(x),
+            MASK_TOKEN_BLOCKS, TOKEN_PARTS, parts, ptr(pml), ptr(po)), "masked_attn_token_prep")
+    return out
+
+
 # Prompt tiles cut over their keys where few of them would leave the chip idle behind a long context.  us, whole / cut, 16
 # heads over 2 of 128: 200 rows at 1000 keys 39 / 21, at 2000 62 / 26, at 8000 205 / 40;  1200 rows 64 / 50, 87 / 61, 227 /
 # 136;  4 over 4 of 64 at 8000, 500 rows 242 / 24 (tiles of 16 tokens, cut over 32 parts, 74).  The more workgroups there are
