@@ -93,7 +93,7 @@ __device__ __forceinline__ void glds16(const uint16_t* src, unsigned char* lds_d
   __builtin_amdgcn_global_load_lds(src, (lds_void_t*)lds_dst, 16, 0, 0);
 }
 
-__device__ __forceinline__ float silu(float g) { return g / (1.f + __expf(-g)); }
+
 
 __device__ __forceinline__ void bar() {
   __builtin_amdgcn_sched_barrier(0);
@@ -552,7 +552,7 @@ __global__ void __launch_bounds__(512, 1) gemm_big_kernel(const uint16_t* __rest
 #pragma unroll
         for (int c = 0; c < NA; ++c) {
           const float gt = bf2f(f2bf(v[c])), up = bf2f(f2bf(v[NA + c]));
-          a[c] = silu(gt) * up;
+          a[c] = silu_hw(gt) * up;
         }
         if constexpr (NA == 4) {
           u16x4 ov;

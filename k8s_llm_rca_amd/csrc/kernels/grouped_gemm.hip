@@ -28,7 +28,6 @@ namespace k8s {
 
 constexpr int GG_BM = 64, GG_BN = 128, GG_BK = 64;
 
-__device__ __forceinline__ float silu_f(float g) { return g / (1.f + __expf(-g)); }
 
 template <bool FUSE_SILU>
 __global__ void __launch_bounds__(256, 2) grouped_gemm_kernel(const uint16_t* __restrict__ a, int lda,
@@ -86,7 +85,7 @@ __global__ void __launch_bounds__(256, 2) grouped_gemm_kernel(const uint16_t* __
       bf16x8 v;
       if constexpr (FUSE_SILU) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) v[t] = (__bf16)(silu_f((float)sa[2 * i][t]) * (float)sa[2 * i + 1][t]);
+        for (int t = 0; t < 8; ++t) v[t] = (__bf16)(silu_hw((float)sa[2 * i][t]) * (float)sa[2 * i + 1][t]);
       } else {
         v = sa[i];
       }
