@@ -456,6 +456,155 @@ __global__ void __launch_bounds__(512, 1) gemm_big_kernel(const uint16_t* __rest
   // n = tn*256 + 128 qw + 32 wc + 8 g + 4 j + v (g = lane >> 4).  SH 32: acc[Q][i][0][r],
   // m = m0 + 128 qx + 64 wr + 32 i + (lane & 31), n = tn*256 + 128 qw + 32 wc + 16 hh + r
   // (hh = lane >> 5).  SwiGLU: the two halves of a lane's values are gate and up.
+  if constexpr (MODE == 4) {
+    // Through LDS, half a tile (128 rows of 1 KB) at a time, so that a wave reads and writes whole rows of it; the residual is
+    // read with the non-temporal hint, and nothing is read while the half before is written.  What bounds it is the residual's
+    // way: of 165 us at 16384 x 2048 x 2048 (out of memory) 41 went with its read and 24 with its write.  us with the
+    // fragments' own 128-byte pieces / so:  16384 x 2048 x 2048 165 / 146, x 8192 414 / 399, 24730 x 2048 x 2048 252 / 240;
+    // without the hint 158, 404, 254;  the second half asked for in front of the first half's stores 168, 415, 252.
+    // 16-byte piece c of row r lies at c ^ (r & 15): no bank conflict in either direction.
+    static_assert(SH == 16);
+    constexpr int RW = 16;                                     // rows of a half that a wave takes
+    float* const o = reinterpret_cast<float*>(y) + tn * BN + 4 * lane;
+    f32x4 t[RW];
+    auto row = [&](int qx, int i) { return m0 + 128 * qx + 8 * i + wv; };
+    auto ask = [&](int qx) {
+#pragma unroll
+      for (int i = 0; i < RW; ++i)
+        t[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(o + (size_t)min(row(qx, i), M - 1) * ldy));
+    };
+    auto put = [&](auto QX) {
+      constexpr int qx = decltype(QX)::value;
+#pragma unroll
+      for (int i = 0; i < XT; ++i)
+#pragma unroll
+        for (int qw = 0; qw < 2; ++qw)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int r = 64 * wr + 16 * i + frow, c = (128 * qw + 32 * wc + 8 * fhi + 4 * j) >> 2;
+            *reinterpret_cast<f32x4*>(sm + r * 1024 + 16 * (c ^ frow)) = acc[qx ? 3 - qw : qw][i][j];
+          }
+    };
+    auto add = [&] {
+#pragma unroll
+      for (int i = 0; i < RW; ++i) {
+        const int r = 8 * i + wv;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(sm + r * 1024 + 16 * (lane ^ (r & 15)));
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[i][c] = fmaf(ra.scale, v[c], t[i][c]);
+      }
+    };
+    auto store = [&](int qx) {
+#pragma unroll
+      for (int i = 0; i < RW; ++i)
+        if (row(qx, i) < M) *reinterpret_cast<f32x4*>(o + (size_t)row(qx, i) * ldy) = t[i];
+    };
+    auto lds_bar = [&] {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      bar();
+    };
+    ask(0);
+    lds_bar();                                                 // (the last fragments are read)
+    put(ic<0>{});
+    lds_bar();
+    add();
+    store(0);
+    ask(1);
+    lds_bar();
+    put(ic<1>{});
+    lds_bar();
+    add();
+    store(1);
+    return;
+  }
+  if constexpr (MODE == 2) {
+    // head 2 tn + qw; a lane's NA dims d0 .. and their partners d0 + 64.  Positions and slots of all rows are asked for at once,
+    // a half's rotations in front of the other half's stores: stores count as loads do for a wait, so that a load behind a
+    // store waits for the memory twice, 16 times a tile (6144 x 4096 at 5590 and 8000 rows 276 -> 261, 333 -> 322 us).
+    constexpr int NA = 2 * WT * GG::NC;
+    typedef float fvec __attribute__((ext_vector_type(NA)));
+    typedef typename std::conditional<NA == 4, u16x4, u16x8>::type ovec;
+    const int d0 = 16 * wc + NA * fhi;
+    auto row = [&](int qx, int i) { return m0 + 128 * qx + 64 * wr + SH * i + frow; };
+    int ps[2][XT], sl[2][XT];
+#pragma unroll
+    for (int qx = 0; qx < 2; ++qx)
+#pragma unroll
+      for (int i = 0; i < XT; ++i) {
+        const int m = min(row(qx, i), M - 1);
+        ps[qx][i] = ra.pos[m];
+        sl[qx][i] = ra.slots ? ra.slots[m] : -1;
+      }
+    fvec co[XT], si[XT];
+    auto ask = [&](int qx) {
+#pragma unroll
+      for (int i = 0; i < XT; ++i) {
+        const float* cs = ra.cos_sin + (size_t)ps[qx][i] * 128 + d0;
+        __builtin_memcpy(&co[i], cs, sizeof(fvec));
+        __builtin_memcpy(&si[i], cs + 64, sizeof(fvec));
+      }
+    };
+    ovec lo[2][XT], hi[2][XT];                               // of both heads
+    auto turn = [&](auto QX) {
+#pragma unroll
+      for (int qw = 0; qw < 2; ++qw)
+#pragma unroll
+        for (int i = 0; i < XT; ++i) {
+          const auto& a = acc[decltype(QX)::value ? 3 - qw : qw][i];
+          const bool rot = 2 * tn + qw < ra.nq + ra.nkv;
+#pragma unroll
+          for (int c = 0; c < NA; ++c) {
+            float u, v;                                        // entries d0 + c and its partner
+            if constexpr (SH == 16)
+              u = a[0][c], v = a[1][c];
+            else
+              u = a[0][c], v = a[0][NA + c];
+            if (rot) {
+              float r0, r1;
+              rope_pair(bf2f(f2bf(u)), bf2f(f2bf(v)), co[i][c], si[i][c], r0, r1);
+              u = r0, v = r1;
+            }
+            lo[qw][i][c] = f2bf(u);
+            hi[qw][i][c] = f2bf(v);
+          }
+        }
+    };
+    auto store = [&](auto QX) {
+      constexpr int qx = decltype(QX)::value;
+#pragma unroll
+      for (int qw = 0; qw < 2; ++qw)
+#pragma unroll
+        for (int i = 0; i < XT; ++i) {
+          const int m = row(qx, i), hd = 2 * tn + qw, slot = sl[qx][i];
+          if (m >= M) continue;
+          uint16_t* o = y + (size_t)m * ldy + hd * 128 + d0;
+          *reinterpret_cast<ovec*>(o) = lo[qw][i];
+          *reinterpret_cast<ovec*>(o + 64) = hi[qw][i];
+          if (slot < 0 || hd < ra.nq) continue;
+          const int blk = slot / ra.BS, off = slot % ra.BS;
+          if (hd < ra.nq + ra.nkv) {  // K page row: dims contiguous
+            uint16_t* kp = ra.kc + (((size_t)blk * ra.nkv + (hd - ra.nq)) * ra.BS + off) * 128 + d0;
+            *reinterpret_cast<ovec*>(kp) = lo[qw][i];
+            *reinterpret_cast<ovec*>(kp + 64) = hi[qw][i];
+          } else {  // V page: [dim][token]
+            uint16_t* vp = ra.vc + ((size_t)blk * ra.nkv + (hd - ra.nq - ra.nkv)) * 128 * ra.BS + off;
+#pragma unroll
+            for (int c = 0; c < NA; ++c) {
+              vp[(size_t)(d0 + c) * ra.BS] = lo[qw][i][c];
+              vp[(size_t)(d0 + 64 + c) * ra.BS] = hi[qw][i][c];
+            }
+          }
+        }
+    };
+    ask(0);
+    turn(ic<0>{});
+    ask(1);
+    __builtin_amdgcn_sched_barrier(0);
+    store(ic<0>{});
+    turn(ic<1>{});
+    store(ic<1>{});
+    return;
+  }
 #pragma unroll
   for (int Q = 0; Q < 4; ++Q) {
     const int qx = (Q == 2 || Q == 3) ? 1 : 0, qw = (Q == 1 || Q == 2) ? 1 : 0;
@@ -480,61 +629,6 @@ __global__ void __launch_bounds__(512, 1) gemm_big_kernel(const uint16_t* __rest
         float* o = part + (size_t)slice * M * N + (size_t)m * N + tn * BN + 128 * qw + 32 * wc + NV * fhi;
 #pragma unroll
         for (int e = 0; e < NV; e += 4) *reinterpret_cast<f32x4*>(o + e) = f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
-      } else if (MODE == 2) {
-        // head 2 tn + qw; this lane's NA dims d0 .. and their partners d0 + 64
-        constexpr int NA = NV / 2;
-        const int hd = 2 * tn + qw, d0 = 16 * wc + NA * fhi;
-        uint16_t* o = y + (size_t)m * ldy + hd * 128 + d0;
-        const int slot = ra.slots ? ra.slots[m] : -1;
-        const int blk = slot >= 0 ? slot / ra.BS : 0, off = slot >= 0 ? slot % ra.BS : 0;
-        float lo[NA], hi[NA];
-        if (hd < ra.nq + ra.nkv) {
-          const float* cs = ra.cos_sin + (size_t)ra.pos[m] * 128;
-#pragma unroll
-          for (int c = 0; c < NA; ++c) {
-            const float co = cs[d0 + c], si = cs[64 + d0 + c];
-            const float a = bf2f(f2bf(v[c])), b = bf2f(f2bf(v[NA + c]));
-            rope_pair(a, b, co, si, lo[c], hi[c]);
-          }
-        } else {
-#pragma unroll
-          for (int c = 0; c < NA; ++c) {
-            lo[c] = v[c];
-            hi[c] = v[NA + c];
-          }
-        }
-        typedef typename std::conditional<NA == 4, u16x4, u16x8>::type ovec;
-        ovec olo, ohi;
-#pragma unroll
-        for (int c = 0; c < NA; ++c) {
-          olo[c] = f2bf(lo[c]);
-          ohi[c] = f2bf(hi[c]);
-        }
-        *reinterpret_cast<ovec*>(o) = olo;
-        *reinterpret_cast<ovec*>(o + 64) = ohi;
-        if (slot >= 0 && hd >= ra.nq) {
-          if (hd < ra.nq + ra.nkv) {  // K page row: dims contiguous
-            uint16_t* kp = ra.kc + (((size_t)blk * ra.nkv + (hd - ra.nq)) * ra.BS + off) * 128 + d0;
-            *reinterpret_cast<ovec*>(kp) = olo;
-            *reinterpret_cast<ovec*>(kp + 64) = ohi;
-          } else {  // V page: [dim][token]
-            uint16_t* vp = ra.vc + ((size_t)blk * ra.nkv + (hd - ra.nq - ra.nkv)) * 128 * ra.BS + off;
-#pragma unroll
-            for (int c = 0; c < NA; ++c) {
-              vp[(size_t)(d0 + c) * ra.BS] = olo[c];
-              vp[(size_t)(d0 + 64 + c) * ra.BS] = ohi[c];
-            }
-          }
-        }
-      } else if (MODE == 4) {
-        float* o = reinterpret_cast<float*>(y) + (size_t)m * ldy + tn * BN + 128 * qw + 32 * wc + NV * fhi;
-#pragma unroll
-        for (int e = 0; e < NV; e += 4) {
-          f32x4 t = *reinterpret_cast<const f32x4*>(o + e);
-#pragma unroll
-          for (int c = 0; c < 4; ++c) t[c] = fmaf(ra.scale, v[e + c], t[c]);
-          *reinterpret_cast<f32x4*>(o + e) = t;
-        }
       } else if (MODE == 0 || MODE == 3) {
         uint16_t* o = y + (size_t)m * ldy + tn * BN + 128 * qw + 32 * wc + NV * fhi;
 #pragma unroll

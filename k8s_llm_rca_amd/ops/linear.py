@@ -443,17 +443,21 @@ ADD_ROWS = 6144
 
 
 def big_add_pays(M: int, N: int, K: int) -> bool:
-    """Whether gemm_big adds a product to an fp32 residual quicker than the library: where its 256-row tiles all but fill their
-    waves, one or two of them or a long K.  us library / gemm_big at waves of tiles:  2048 x 8192 at 0.78 198 / 173, 1.00
-    207 / 196, 1.47 316 / 337, 2.00 412 / 405, 3.00 620 / 596, 4.00 826 / 788;  2048 x 2048 at 0.78 66 / 59, 1.00 70 / 65,
-    1.12 87 / 104, 2.00 130 / 127, 3.00 202 / 205, 4.00 267 / 283;  4096 x 4096 at 2.00 219 / 209, 2.25 254 / 292, 4.00
-    447 / 448;  2048 x 14336 at 1.00 345 / 332, 4096 x 8192 at 6.00 1207 / 1158;  1024 x 8192 at 0.50 116 / 127."""
+    """Whether gemm_big adds a product to an fp32 residual quicker than the library, by how far its 256-row tiles fill their
+    last wave of 256: whole waves, or a last one of two thirds, from the third on two fifths, with a K from 8192 on a fifth.
+    us library / gemm_big, the residual out of memory, at waves of tiles:  2048 x 2048 at 0.50 53 / 59, 0.88 77 / 71, 1.28 112 /
+    116, 1.47 119 / 120, 1.69 141 / 128, 2.00 154 / 144, 2.50 201 / 186, 3.00 220 / 204, 4.00 286 / 268;  2048 x 8192 at 0.69
+    165 / 175, 0.88 210 / 194, 1.28 313 / 299, 1.47 341 / 327, 2.00 418 / 397, 3.00 620 / 589, 3.50 752 / 712;  4096 x 4096 at
+    0.50 80 / 95, 0.88 119 / 110, 1.25 168 / 185, 1.44 190 / 199, 1.69 217 / 204, 2.50 427 / 302, 3.00 355 / 336, 4.00 462 / 462;
+    4096 x 14336 at 0.75 286 / 310, 0.88 330 / 322, 1.25 488 / 459, 2.00 689 / 670;  1024 x 4096 at 1.47 197 / 210, 1.69 225 /
+    215;  5120 x 2048 at 1.09 104 / 110, 1.64 141 / 127, 2.89 220 / 200."""
     if N % 256 or K % 128 or K < 2048:
         return False
     tiles = -(-M // 256) * (N // 256)
     if tiles <= 256:
         return tiles >= 196
-    return (tiles <= 512 or K >= 8192) and 100 * tiles >= 95 * 256 * -(-tiles // 256)
+    full, over = divmod(tiles, 256)
+    return not over or over >= (51 if K >= 8192 else 102 if full >= 2 else 166)
 
 
 def proj_add(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, scale: float = 1.0):
