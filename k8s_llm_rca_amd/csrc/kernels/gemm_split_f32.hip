@@ -1,0 +1,315 @@
+// Products of some tens to some thousands of fp32 rows, Y[M][N] = X[M][K] . W[N][K]^T, on the bf16 matrix instructions.
+//
+// The fp32 matrix instruction does a sixteenth of the bf16 one's work, and the library's fp32 products reach 120 to 140 TFLOP/s
+// at 600 rows.  An fp32 number is the exact sum of three bf16 numbers (8 significant bits each, rounded to nearest: a1 =
+// bf16(a), a2 = bf16(a - a1), a3 = a - a1 - a2), and of the nine products of two such sums six are kept: a1 b1, a1 b2, a2 b1,
+// a2 b2, a1 b3, a3 b1.  What is left out is below 2^-26 of the product, a quarter of fp32's own rounding; sums stay in fp32.
+// Relative error (2-norm, against 64 bits) of 622 rows of unit normals, the library / this:  K 2048 8.1e-7 / 7.0e-7 (in four
+// ranges 3.4e-7);  K 8192 1.6e-6 / 1.4e-6 (7.2e-7).
+//
+// X is split once, by a pass of its own, into three planes of bf16 (every column tile reads it).  A workgroup of four waves makes
+// 16 MT x 128 outputs, each wave 32 columns of all rows, K in steps of 32: X's planes go straight into LDS (16 rows x 64 bytes
+// an instruction, as the fragments are read: no bank conflict), two buffers of them; no wave shares its columns, so that W is
+// read in fragment order and split in registers, half a step's matrix instructions after it has come and a step's after it
+// was asked for.  Two workgroups share a compute unit.  The tiles of one panel of the larger operand
+// follow each other on one XCD.  Few tiles:
+// K in ranges, whose sums (planes) the consumer adds.
+//
+// What bounds it: the power (1.8 GHz at a bf16 rate of 1.1 PFLOP/s) and, where there are few workgroups, a step's chain (1.2 us
+// with four fragments, 2.0 with ten).  us, the library / the pass and this, out of memory:  16384 x 2048 at 333, 622, 1024 rows
+// 214 / 139, 373 / 236, 513 / 346;  8192 x 2048 at 622, 1024 187 / 133, 241 / 167;  2048 x 8192 in ranges 162 / 123, 243 / 183
+// and their sums.  With X split by every workgroup 330 instead of 236, with W in LDS as well 361; the splits placed between
+// the matrix instructions one by one 357.
+#include "common.h"
+
+namespace k8s {
+
+constexpr int kSfN = 128, kSfK = 32;
+constexpr float kSfWild = 3.39e38f;                               // rounds to an infinity in bf16, or a little less
+
+enum SplitOut { kSplitPlain = 0, kSplitGlu = 1 };
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+struct Split3 {
+  u32x2 p[3];            // four bf16 each
+};
+
+__device__ __forceinline__ uint32_t pair_bf(float a, float b) {                  // one instruction
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
+__device__ __forceinline__ float low_bf(uint32_t v) { return __uint_as_float(v << 16); }
+__device__ __forceinline__ float high_bf(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
+
+// Four numbers as sums of three.  wild: some lane has a number that bf16 rounds to an infinity, or one that is: its first part is
+// cut instead of rounded, and the others are zero where that is all of it (an infinity stays one, a NaN stays NaN).
+__device__ __forceinline__ void split3(const f32x4& a, Split3& s, bool wild) {
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const float u = a[2 * k], v = a[2 * k + 1];
+    uint32_t h = pair_bf(u, v);
+    if (wild) {
+      if (fabsf(u) >= kSfWild) h = (h & 0xffff0000u) | (__float_as_uint(u) >> 16);
+      if (fabsf(v) >= kSfWild) h = (h & 0xffffu) | (__float_as_uint(v) & 0xffff0000u);
+    }
+    s.p[0][k] = h;
+    float ru = u - low_bf(h), rv = v - high_bf(h);
+    if (wild) {
+      if (u == low_bf(h)) ru = 0.f;
+      if (v == high_bf(h)) rv = 0.f;
+    }
+    h = pair_bf(ru, rv);
+    s.p[1][k] = h;
+    s.p[2][k] = pair_bf(ru - low_bf(h), rv - high_bf(h));
+  }
+}
+
+// x [M][K] (rows ldx apart) -> p [3][M][K]
+__global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict__ x, int ldx, uint16_t* __restrict__ p, int M, int K) {
+  const int k4 = K >> 2;
+  const size_t n = (size_t)M * k4, plane = (size_t)M * K;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    const size_t m = i / k4, c = 4 * (i - m * k4);
+    Split3 s;
+    split3(*reinterpret_cast<const f32x4*>(x + m * ldx + c), s, true);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x2*>(p + q * plane + m * K + c) = s.p[q];
+  }
+}
+
+typedef __attribute__((address_space(3))) void sf_lds_t;
+__device__ __forceinline__ void sf_to_lds(const uint16_t* src, uint16_t* dst) {  // 16 bytes a lane, the wave's 1 KB in a row
+  __builtin_amdgcn_global_load_lds(src, (sf_lds_t*)dst, 16, 0, 0);
+}
+
+__device__ __attribute__((noinline)) float fp32_dot(const uint16_t* xpl, const float* w, int m, size_t wrow, int M, int K, int k0,
+                                                    int n) {
+  const uint16_t* a = xpl + (size_t)m * K + k0;
+  const float* b = w + wrow * K + k0;
+  const size_t plane = (size_t)M * K;
+  float t = 0.f;
+  for (int k = 0; k < n; ++k) t = fmaf(bf2f(a[k]) + bf2f(a[plane + k]) + bf2f(a[2 * plane + k]), b[k], t);
+  return t;
+}
+
+// grid: (row tiles x column tiles, K ranges)
+template <int MT, int OUT>
+__global__ void __launch_bounds__(256, 2)
+    gemm_split_f32_kernel(const uint16_t* __restrict__ xpl, const float* __restrict__ w, float* __restrict__ y, int M, int N,
+                          int K, int n_mt, int n_nt) {
+  constexpr int BM = 16 * MT, ND = 3 * MT, PER = (ND + 3) / 4;    // LDS-DMA instructions of a step, of a wave
+  __shared__ __attribute__((aligned(1024))) uint16_t xs[2][3][BM * kSfK];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the tiles that share the larger operand's panel on one XCD, one after the other
+  int tm, tn;
+  {
+    const bool by_w = 4 * (size_t)N * (OUT == kSplitGlu ? 2 : 1) >= 6 * (size_t)M;
+    const int outer = by_w ? n_nt : n_mt, inner = by_w ? n_mt : n_nt;
+    const int b = blockIdx.x, q = outer >> 3, whole = 8 * q * inner;
+    const int o = b < whole ? (b & 7) + 8 * ((b >> 3) / inner) : 8 * q + (b - whole) / inner;
+    const int i = b < whole ? (b >> 3) % inner : (b - whole) % inner;
+    tn = by_w ? o : i, tm = by_w ? i : o;
+  }
+  const int m0 = tm * BM, n0 = tn * (OUT == kSplitGlu ? kSfN / 2 : kSfN);
+  const int kr = K / gridDim.y, k0 = blockIdx.y * kr, steps = kr / kSfK;
+  const uint16_t* xp[PER];                                        // instruction wv + 4 i: plane / MT, fragment % MT
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int d = min(wv + 4 * i, ND - 1);                        // (past the last one: it again)
+    xp[i] = xpl + ((size_t)(d / MT) * M + min(m0 + 16 * (d % MT) + (lane >> 2), M - 1)) * K + k0 + 8 * (lane & 3);
+  }
+  const float* wp[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {                                   // SwiGLU: 16 gate rows and their up rows
+    const size_t row = OUT == kSplitGlu ? min(n0 + 16 * wv + r, N - 1) + (size_t)j * N : min(n0 + 32 * wv + 16 * j + r, N - 1);
+    wp[j] = w + row * K + k0 + 8 * g;
+  }
+  f32x4 wq[2][2];
+  bf16x8 wf[2][3];
+  auto load_x = [&](int s, int buf) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int d = min(wv + 4 * i, ND - 1);
+      sf_to_lds(xp[i] + s * kSfK, &xs[buf][0][d * 16 * kSfK]);
+    }
+  };
+  auto load_w = [&](int s) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wq[j][h] = *reinterpret_cast<const f32x4*>(wp[j] + s * kSfK + 4 * h);
+  };
+  auto wild = [&] {
+    float most = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) most = fmaxf(most, fabsf(wq[j >> 1][j & 1][k]));
+    return (bool)__any(most >= kSfWild);
+  };
+  auto take = [&](bf16x8 (&f)[2][3], bool wi) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      Split3 a, b;
+      split3(wq[j][0], a, wi);
+      split3(wq[j][1], b, wi);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        f[j][p] = __builtin_bit_cast(bf16x8, (u32x4{a.p[p][0], a.p[p][1], b.p[p][0], b.p[p][1]}));
+      }
+    }
+  };
+  auto take_any = [&](bf16x8 (&f)[2][3]) {
+    if (__builtin_expect(wild(), 0))
+      take(f, true);
+    else
+      take(f, false);
+  };
+  auto bar = [] {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x4 acc[MT][2];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  load_w(0);
+  load_x(0, 0);
+  take_any(wf);
+  load_w(min(1, steps - 1));
+  asm volatile("s_waitcnt vmcnt(4)" ::: "memory");                // X of step 0
+  bar();
+  // two rows of fragments: 24 matrix instructions
+  auto multiply = [&](int buf, int i) {
+    bf16x8 xf[2][3];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        xf[h][p] = *reinterpret_cast<const bf16x8*>(&xs[buf][p][(16 * (i + h) + r) * kSfK + 8 * g]);
+    constexpr int PX[6] = {2, 0, 1, 1, 0, 0}, PW[6] = {0, 2, 1, 0, 1, 0};        // small ones first
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i + h][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][PW[q]], xf[h][PX[q]], acc[i + h][j], 0, 0, 0);
+  };
+  for (int s = 0; s < steps; ++s) {                               // (the last step loads and splits what it has once more, unread)
+    const int buf = s & 1;
+    constexpr int H = MT / 4 * 2;
+    load_x(min(s + 1, steps - 1), buf ^ 1);
+#pragma unroll
+    for (int i = 0; i < H; i += 2) multiply(buf, i);
+    bf16x8 nf[2][3];
+    take_any(nf);
+    load_w(min(s + 2, steps - 1));
+#pragma unroll
+    for (int i = H; i < MT; i += 2) multiply(buf, i);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) wf[j][p] = nf[j][p];
+    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");   // the next step's X; this step's fragments are read
+    bar();
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // no load into LDS outlives the workgroup
+  // acc[i][j][v]: row m0 + 16 i + r, panel row 32 wv + 16 j + 4 g + v
+  //
+  // An infinity meets the other operand's parts of both signs, or none, and gives NaN where it should stay one: sums that are
+  // NaN are made again as fp32 makes them.
+  bool lost = false;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) lost |= acc[i][j][v] != acc[i][j][v];
+  if (__builtin_expect(__any(lost), 0)) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (acc[i][j][v] != acc[i][j][v]) {
+            const int c = 4 * g + v;
+            const size_t wr = OUT == kSplitGlu ? min(n0 + 16 * wv + c, N - 1) + (size_t)j * N : min(n0 + 32 * wv + 16 * j + c, N - 1);
+            acc[i][j][v] = fp32_dot(xpl, w, min(m0 + 16 * i + r, M - 1), wr, M, K, k0, kr);
+          }
+  }
+  float* const o = y + (size_t)blockIdx.y * M * N;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = m0 + 16 * i + r;
+    if (m >= M) continue;
+    if constexpr (OUT == kSplitGlu) {
+      const int n = n0 + 16 * wv + 4 * g;
+      if (n >= N) continue;
+      f32x4 t;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) t[v] = acc[i][0][v] / (1.f + expf(-acc[i][0][v])) * acc[i][1][v];
+      *reinterpret_cast<f32x4*>(o + (size_t)m * N + n) = t;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int n = n0 + 32 * wv + 16 * j + 4 * g;
+        if (n < N) *reinterpret_cast<f32x4*>(o + (size_t)m * N + n) = acc[i][j];
+      }
+    }
+  }
+}
+
+template <int OUT>
+static int split_f32(const uint16_t* xp, const float* w, float* y, int M, int N, int K, int mt, int ranges, hipStream_t s) {
+  if (M <= 0 || N <= 0 || N % 4 || K <= 0 || ranges < 1 || K % (kSfK * ranges) || !xp || !w || !y || ((uintptr_t)xp & 15) ||
+      ((uintptr_t)w & 15) || ((uintptr_t)y & 15) || (OUT == kSplitGlu && (ranges > 1 || N % 64)))
+    return (int)hipErrorInvalidValue;
+  const int bn = OUT == kSplitGlu ? kSfN / 2 : kSfN, n_nt = (N + bn - 1) / bn, n_mt = (M + 16 * mt - 1) / (16 * mt);
+#define K8S_SF(MT)                                                                                                        \
+  case MT:                                                                                                                \
+    hipLaunchKernelGGL((gemm_split_f32_kernel<MT, OUT>), dim3(n_mt * n_nt, ranges), dim3(256), 0, s, xp, w, y, M, N, K, n_mt, \
+                       n_nt);                                                                                             \
+    break
+  switch (mt) {
+    K8S_SF(4);
+    K8S_SF(6);
+    K8S_SF(8);
+    K8S_SF(10);
+    K8S_SF(12);
+    default: return (int)hipErrorInvalidValue;
+  }
+#undef K8S_SF
+  return (int)hipGetLastError();
+}
+
+}  // namespace k8s
+
+using namespace k8s;
+
+// x [M][K] fp32 (rows ldx apart, on 16 bytes) -> three bf16 planes p [3][M][K] whose sum it is.
+K8S_API int k8s_split_rows_f32(const float* x, int ldx, void* p, int M, int K, hipStream_t s) {
+  if (M <= 0 || K <= 0 || K % 4 || ldx % 4 || (M > 1 && ldx < K) || !x || !p || ((uintptr_t)x & 15) || ((uintptr_t)p & 7))
+    return (int)hipErrorInvalidValue;
+  const size_t n = ((size_t)M * K / 4 + 255) / 256;
+  hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)(n < 4096 ? n : 4096)), dim3(256), 0, s, x, ldx, (uint16_t*)p, M, K);
+  return (int)hipGetLastError();
+}
+
+// y [ranges][M][N] fp32: the products of xp's rows (three planes) and w [N][K] over K ranges.  mt: 16-row fragments of a tile, 4,
+// 6, 8, 10 or 12.  N a multiple of 4, K of 32 ranges; xp, w, y on 16 bytes.
+K8S_API int k8s_gemm_split_f32(const void* xp, const float* w, float* y, int M, int N, int K, int mt, int ranges, hipStream_t s) {
+  return split_f32<kSplitPlain>((const uint16_t*)xp, w, y, M, N, K, mt, ranges, s);
+}
+
+// y [M][N] = silu(x . w[0:N]^T) * (x . w[N:2N]^T), N a multiple of 64.
+K8S_API int k8s_gemm_split_glu_f32(const void* xp, const float* w, float* y, int M, int N, int K, int mt, hipStream_t s) {
+  return split_f32<kSplitGlu>((const uint16_t*)xp, w, y, M, N, K, mt, 1, s);
+}

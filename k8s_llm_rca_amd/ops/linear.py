@@ -196,6 +196,61 @@ def _few_f32_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.stride(0) < 2 ** 31)
 
 
+# fp32 products of many rows as bf16 ones (csrc/kernels/gemm_split_f32.hip)
+SPLIT_ROWS = 128, 4096
+SPLIT_TILES = (4, 6, 8, 10, 12)      # 16-row fragments of a tile
+
+
+@functools.lru_cache(maxsize=4096)
+def split_plan(M: int, N: int, K: int, planes: bool = False, glu: bool = False):
+    """(16-row fragments of a tile, K ranges) with which an fp32 product of many rows is quicker as products of bf16 parts than
+    on the library, or None.  ``N``: rows of the weight; ``planes``: K ranges may stay apart.
+
+    A step of a workgroup (K 32) takes some 0.5 us and 0.13 a fragment, less the fewer of them a compute unit has at once; the
+    rows' split is a pass of 4 us and their bytes, each range writes and reads the result once more; and the library takes its
+    operations at 120 TFLOP/s and a start.  us library / the split and this:  16384 x 2048 at 333, 622, 1024 rows 214 / 139,
+    373 / 236, 513 / 346, at 166 105 / 109;  8192 x 2048 at the same 108 / 105, 187 / 133, 241 / 167, 61 / 95;  2048 x 8192
+    (eight ranges, with the bytes of their sums) 108 / 88, 162 / 139, 243 / 188;  2048 x 2048 33 / 36, 46 / 52, 66 / 63;  2560 x
+    2048 at 1024 100 / 77."""
+    if not SPLIT_ROWS[0] <= M <= SPLIT_ROWS[1] or N < 512 or K < 512 or K % 32 or N % (128 if glu else 4):
+        return None
+    best = None
+    for mt in SPLIT_TILES:
+        for ranges in (1, 2, 4, 8) if planes else (1,):
+            if K % (32 * ranges) or K // ranges < 256:
+                continue
+            load = -(-M // (16 * mt)) * -(-N // 128) * ranges / 256
+            cost = K / 32 / ranges * (0.5 + 0.13 * mt) * max(1.15 + 0.2 * load, 0.55 + 0.7 * load, 0.95 * load)
+            if ranges > 1:
+                cost += ranges * M * N * 8 / 5e6
+            if best is None or cost < best[0]:
+                best = cost, mt, ranges
+    cost = best[0] + 4 + M * K * 10 / 5e6
+    return best[1:] if cost < 0.93 * (2 * M * N * K / 120e6 + 5) else None
+
+
+def _split_f32(x: torch.Tensor, w: torch.Tensor, planes: bool = False, glu: bool = False):
+    """The product as [ranges, M, N] (``glu``: [M, N / 2]), or None: another kernel is the quicker one or has to take it."""
+    M = x.shape[0]
+    if not SPLIT_ROWS[0] <= M <= SPLIT_ROWS[1] or w.dim() != 2 or x.shape[1] != w.shape[1]:
+        return None
+    N, K = w.shape
+    plan = split_plan(M, N, K, planes, glu) if x.is_cuda and x.dtype == torch.float32 == w.dtype and w.is_cuda else None
+    if plan is None or not unwatched(x, w) or not (
+            w.is_contiguous() and w.data_ptr() % 16 == 0 == x.data_ptr() % 16 and x.stride(1) == 1 and x.stride(0) % 4 == 0
+            and K <= x.stride(0) < 2 ** 31 and w.device == x.device):
+        return None
+    parts = torch.empty(3, M, K, dtype=torch.bfloat16, device=x.device)
+    check(lib().k8s_split_rows_f32(ptr(x), x.stride(0), ptr(parts), M, K, stream_ptr(x)), "split_rows_f32")
+    if glu:
+        out = torch.empty(M, N // 2, dtype=torch.float32, device=x.device)
+        check(lib().k8s_gemm_split_glu_f32(ptr(parts), ptr(w), ptr(out), M, N // 2, K, plan[0], stream_ptr(x)), "gemm_split_glu_f32")
+        return out
+    out = torch.empty(plan[1], M, N, dtype=torch.float32, device=x.device)
+    check(lib().k8s_gemm_split_f32(ptr(parts), ptr(w), ptr(out), M, N, K, *plan, stream_ptr(x)), "gemm_split_f32")
+    return out
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
     """``x @ w.T`` for ``x`` [M, K] and ``w`` [N, K]."""
     M, K = x.shape
@@ -205,6 +260,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torch.
             out = torch.empty((M, N), dtype=torch.float32, device=x.device)
             check(lib().k8s_few_rows_f32(ptr(x), x.stride(0), ptr(w), ptr(out), M, N, K, stream_ptr(x)), "few_rows_f32")
             return out
+        if out is None:
+            y = _split_f32(x, w)
+            if y is not None:
+                return y[0]
         return lib_gemm(x, w, out)
     layout = x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
     rows = M <= ROWS_MAX_M and rows_ok(x, w) and (out is None or out.stride(1) == 1)
@@ -427,7 +486,8 @@ def proj_planes(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             check(lib().k8s_gemm_stream_part(ptr(x), x.stride(0), ptr(w), None, N, M, N, K, cfg, S, ptr(out),
                                              stream_ptr(x)), "gemm_stream_part")
             return out
-    return proj_f32out(x, w)[None]
+    y = _split_f32(x, w, planes=True)
+    return y if y is not None else proj_f32out(x, w)[None]
 
 
 def _few_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -584,6 +644,10 @@ def glu_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         out = torch.empty((M, I), dtype=torch.float32, device=x.device)
         check(lib().k8s_few_rows_glu_f32(ptr(x), x.stride(0), ptr(w), ptr(out), M, I, K, stream_ptr(x)), "few_rows_glu_f32")
         return out
+    if w.shape[0] == 2 * I:
+        a = _split_f32(x, w, glu=True)
+        if a is not None:
+            return a
     return glu_clamp(linear(x, w), 1.0, math.inf, 0.0)
 
 

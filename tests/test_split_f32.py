@@ -1,0 +1,99 @@
+"""fp32 products of many rows as products of bf16 parts (csrc/kernels/gemm_split_f32.hip): against 64 bits, beside the library's
+error, with infinities, NaN and numbers at both ends of the range."""
+import pytest
+import torch
+
+from k8s_llm_rca_amd.ops import linear as L
+from k8s_llm_rca_amd.ops._lib import check, lib, ptr, stream_ptr
+
+gpu = pytest.mark.gpu
+
+
+def test_rule():
+    assert L.split_plan(622, 16384, 2048, glu=True) is not None and L.split_plan(622, 2048, 8192, True)[1] > 1
+    assert L.split_plan(166, 16384, 2048) is None and L.split_plan(333, 2048, 2048, True) is None
+    for m, n, k in ((64, 16384, 2048), (5000, 16384, 2048), (622, 16382, 2048), (622, 16384, 2050), (622, 16384, 256)):
+        assert L.split_plan(m, n, k) is None
+    for m in range(128, 4097, 57):
+        for n, k in ((2048, 8192), (2560, 2048), (1088, 4096), (8192, 512)):
+            p = L.split_plan(m, n, k, True)
+            assert p is None or p[0] in L.SPLIT_TILES and k % (32 * p[1]) == 0
+
+
+def _parts(x):
+    m, k = x.shape
+    p = torch.empty(3, m, k, dtype=torch.bfloat16, device=x.device)
+    check(lib().k8s_split_rows_f32(ptr(x), x.stride(0), ptr(p), m, k, stream_ptr(x)), "split")
+    return p
+
+
+def _product(x, w, mt, ranges):
+    (m, k), n = x.shape, w.shape[0]
+    y = torch.full((ranges, m, n), float("nan"), device=x.device)
+    check(lib().k8s_gemm_split_f32(ptr(_parts(x)), ptr(w), ptr(y), m, n, k, mt, ranges, stream_ptr(x)), "product")
+    return y
+
+
+@gpu
+@pytest.mark.parametrize("m", [1, 15, 64, 97, 160, 193])
+@pytest.mark.parametrize("n,k", [(4, 32), (132, 64), (1100, 288), (128, 2048)])
+@pytest.mark.parametrize("mt", L.SPLIT_TILES)
+def test_product(m, n, k, mt):
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn(m, k + 4, generator=g).cuda()[:, :k], (torch.randn(n, k, generator=g) * k ** -0.5).cuda()
+    x[0, 0], w[-1, -1] = 1e-30, 3e4
+    want = x.double() @ w.double().T
+    scale = x.double().abs() @ w.double().abs().T
+    for ranges in (1, 2, 4):
+        if k % (32 * ranges):
+            continue
+        y = _product(x, w, mt, ranges)
+        # each sum of k products, in fp32: a share of the sum of their sizes
+        assert bool(((y.double().sum(0) - want).abs() <= 2.0 ** -21 * scale).all())
+    assert torch.equal(_parts(x).float().sum(0), x)                    # exactly three parts (1e-30 as well)
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", [(622, 1024, 2048), (333, 512, 8192)])
+def test_no_further_off_than_the_library(m, n, k):
+    g = torch.Generator().manual_seed(k)
+    for heavy in (False, True):
+        x, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g) * k ** -0.5
+        if heavy:                                                      # a few large entries a row
+            x *= torch.exp(2.0 * torch.randn(m, k, generator=g))
+        x, w = x.cuda(), w.cuda()
+        want = x.double() @ w.double().T
+        err = [float((y.double() - want).norm() / want.norm()) for y in (_product(x, w, 8, 1)[0], torch.nn.functional.linear(x, w))]
+        assert err[0] <= err[1]
+
+
+@gpu
+def test_infinities_and_the_ends_of_the_range():
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(130, 96, generator=g).cuda(), torch.randn(140, 96, generator=g).cuda().abs()
+    x[3, 7], x[4, 9], x[5, 11], x[6, 0], x[7] = float("inf"), float("-inf"), float("nan"), 3.4e38, 0.0
+    w[9, 50], w[10, 0], w[11] = float("inf"), 3.402e38, 1e-3
+    y, want = _product(x, w, 4, 1)[0], torch.nn.functional.linear(x, w)
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.isinf(), want.isinf())
+    both = want.isinf()
+    assert torch.equal(y[both], want[both])
+    fin = want.isfinite()
+    assert bool(((y - want)[fin].abs() <= 2e-5 * (want[fin].abs() + 30)).all())
+
+
+@gpu
+def test_routes():
+    """Where the rule takes it: the plain product, planes, and the gated unit; and what torch has to see stays with torch."""
+    g = torch.Generator().manual_seed(7)
+    x, w = torch.randn(640, 2048, generator=g).cuda(), (torch.randn(8192, 2048, generator=g) * 0.02).cuda()
+    want = x.double() @ w.double().T
+    assert L.split_plan(640, 8192, 2048) is not None
+    assert float((L.linear(x, w).double() - want).norm() / want.norm()) < 1e-6
+    y = L.proj_planes(x, w)
+    assert float((y.double().sum(0) - want).norm() / want.norm()) < 1e-6
+    gate, up = want.split(4096, 1)
+    a = torch.nn.functional.silu(gate) * up
+    assert float((L.glu_proj(x, w).double() - a).norm() / a.norm()) < 2e-6
+    wg = w.clone().requires_grad_()
+    L.linear(x, wg).sum().backward()
+    assert wg.grad is not None
