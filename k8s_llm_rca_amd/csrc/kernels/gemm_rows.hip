@@ -21,11 +21,12 @@
 //   32768 x 2048, fp32 out    32.0 / 21.4  32.1 / 21.5  32.1 / 22.5  34.3 / 24.5
 //   128256 x 4096, fp32 out    184 / 160    194 / 165    199 / 171    210 / 194
 #include "common.h"
+#include "gates.h"
 #include "norm_prologue.h"
 
 namespace k8s {
 
-enum RowsOut { kRowsBf16 = 0, kRowsF32 = 1, kRowsSilu = 2, kRowsRelu2 = 3, kRowsRope = 4 };
+enum RowsOut { kRowsBf16 = 0, kRowsF32 = 1, kRowsSilu = 2, kRowsRelu2 = 3, kRowsRope = 4, kRowsConv = 5 };
 
 constexpr int kRowsWaves = 4;
 
@@ -38,6 +39,18 @@ struct RowsRope {
   uint16_t* vc;          // [blocks][nkv][128][BS]
   int nq, nkv, BS;
 };
+
+// The first `cols` columns rounded to bf16 and convolved with their sequence's last inputs (short_conv_tile_kernel, mixer_ops.hip:
+// every row the only one of its sequence), the rest as they are, in fp32
+struct RowsConv {
+  int cols, taps, ldr, act;
+  const float* w;        // [cols][taps], the last is the row's own
+  float* tail;           // [slots][taps - 1][cols]
+  const int* pos0;
+  const int* slot;
+  float* rest;           // [M][ldr]
+};
+constexpr int kConvTaps = 4;
 
 // How x comes: as it is; normed by every workgroup (NormIn); or the product's rows are divided by the root mean square of what
 // x was made from (RowScale), whose sums of squares a gemm_step (gemm_step.hip) left in parts.
@@ -65,10 +78,12 @@ constexpr int rows_lds(int MT, int NF, int CH) { return 16 * NF * (CH > 32 * MT 
 // (norm_prologue.h) while its first weights are on their way; the row's own loads are asked for in front of them (6144 x 4096
 // rotated 13.5 -> 11.6 us, 28672 x 4096 SwiGLU 39.4 -> 37.6, on four fragments instead of one 36.3).  Scaled: a wave sums the
 // parts of up to four rows, asked for in front of the weights, and every sum is multiplied before it is rounded or stored.
+// Convolved: a thread's first entry has its earlier inputs and taps asked for behind the first weights
+// (2304 columns and 144 others, K 2048, 1 and 16 rows: three launches of 10.6 and 12.4 us -> 5.3 and 6.2).
 template <int MT, int NF, int CH, int OUT, int IN>
 __global__ void __launch_bounds__(kRowsWaves * 64, 2)
     gemm_rows_kernel(const uint16_t* __restrict__ x, int ldx, const uint16_t* __restrict__ w, void* __restrict__ y, int ldy,
-                     int M, int N, int K, int kslice, RowsRope rp, NormIn nin, RowScale rsc) {
+                     int M, int N, int K, int kslice, RowsRope rp, NormIn nin, RowScale rsc, RowsConv cv) {
   constexpr bool NORM = IN == kRowsNorm, SCALED = IN == kRowsScaled;
   static_assert(!SCALED || MT == 1);
   constexpr bool kHalves = OUT == kRowsSilu || OUT == kRowsRope;
@@ -156,6 +171,26 @@ __global__ void __launch_bounds__(kRowsWaves * 64, 2)
       pv[q] = *reinterpret_cast<const f32x4*>(rsc.part + (size_t)min(wv + kRowsWaves * q, M - 1) * rsc.parts +
                                               min(4 * lane, rsc.parts - 4));
   }
+  // (rows and channels past the last: the last ones, not used)
+  struct ConvAt {
+    int p0;
+    float* tl;
+    const float* w;
+  };
+  auto conv_row = [&](int e) {
+    const int m = min(e / (16 * NF), M - 1), c = min(n0 + e % (16 * NF), cv.cols - 1);
+    return ConvAt{cv.pos0[m], cv.tail + (size_t)cv.slot[m] * (cv.taps - 1) * cv.cols + c, cv.w + (size_t)c * cv.taps};
+  };
+  float hist[kConvTaps], taps[kConvTaps];
+  auto conv_ask = [&](const ConvAt& at) {
+#pragma unroll
+    for (int j = 0; j < kConvTaps; ++j) {
+      taps[j] = at.w[min(j, cv.taps - 1)];
+      hist[j] = j < cv.taps - 1 && at.p0 - (cv.taps - 1 - j) >= 0 ? at.tl[(size_t)j * cv.cols] : 0.f;
+    }
+  };
+  ConvAt cat;
+  if constexpr (OUT == kRowsConv) cat = conv_row(threadIdx.x);
   __builtin_amdgcn_sched_barrier(0);
   load_w(0, 0);
   __builtin_amdgcn_sched_barrier(0);
@@ -163,6 +198,10 @@ __global__ void __launch_bounds__(kRowsWaves * 64, 2)
   __builtin_amdgcn_sched_barrier(0);
   if (NORM || nch > 1) load_w(1, nch > 1 ? 1 : 0);   // (no branch between the row and its use: the waits count what is in flight)
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (OUT == kRowsConv) {
+    conv_ask(cat);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   if constexpr (NORM) {
     __shared__ float nscr[16];
     norm_rows_to_lds<true>(k8s_norm_lds, M, nin, blockIdx.x == 0 && blockIdx.y == 0, nscr, nrow, nwv);
@@ -250,7 +289,22 @@ __global__ void __launch_bounds__(kRowsWaves * 64, 2)
     for (int e = threadIdx.x; e < 16 * NF * M; e += kRowsWaves * 64) {
       const int m = e / (16 * NF), n = e % (16 * NF);
       const float t = total(m, n);
-      if constexpr (OUT == kRowsF32)
+      if constexpr (OUT == kRowsConv) {
+        if (n0 >= cv.cols) {
+          cv.rest[(size_t)m * cv.ldr + n0 - cv.cols + n] = t;
+          continue;
+        }
+        if (e != (int)threadIdx.x) conv_ask(cat = conv_row(e));
+        const float own = bf2f(f2bf(t));
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < kConvTaps; ++j)
+          if (j < cv.taps) sum = fmaf(taps[j], j < cv.taps - 1 ? hist[j] : own, sum);
+        yb[(size_t)m * ldy + n0 + n] = f2bf(cv.act ? silu_f(sum) : sum);
+#pragma unroll
+        for (int j = 0; j < kConvTaps - 1; ++j)
+          if (j < cv.taps - 1) cat.tl[(size_t)j * cv.cols] = j < cv.taps - 2 ? hist[j + 1] : own;
+      } else if constexpr (OUT == kRowsF32)
         reinterpret_cast<float*>(y)[(size_t)blockIdx.y * M * N + (size_t)m * ldy + n0 + n] = t;
       else
         yb[(size_t)m * ldy + n0 + n] = f2bf(OUT == kRowsRelu2 ? relu_sq_f(t) : t);
@@ -260,13 +314,13 @@ __global__ void __launch_bounds__(kRowsWaves * 64, 2)
 
 template <int MT, int NF, int CH, int IN>
 static int rows_launch(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int ranges, int out,
-                       const RowsRope& rp, const NormIn& nin, const RowScale& rsc, hipStream_t s) {
+                       const RowsRope& rp, const NormIn& nin, const RowScale& rsc, const RowsConv& cv, hipStream_t s) {
   constexpr bool NORM = IN == kRowsNorm;
   const bool halves = out == kRowsSilu || out == kRowsRope;
   const int strip = (halves ? 8 : 16) * NF, cols = out == kRowsRope ? N / 2 : N;   // rope: columns counted as pairs
   if (M <= 0 || M > 16 * MT || (NORM && M > kNormMaxRows) || N <= 0 || N % (out == kRowsRope ? 128 : 1) || cols % strip ||
-      ranges < 1 || K <= 0 || K % (ranges * kRowsWaves * CH) || (ranges > 1 && out != kRowsF32) || ldy < N ||
-      (ranges > 1 && ldy != N) || !w || !y || ((uintptr_t)w & 15))
+      ranges < 1 || K <= 0 || K % (ranges * kRowsWaves * CH) || (ranges > 1 && out != kRowsF32) ||
+      ldy < (out == kRowsConv ? cv.cols : N) || (out == kRowsConv && (cv.cols % strip || cv.ldr < N - cv.cols)) || (ranges > 1 && ldy != N) || !w || !y || ((uintptr_t)w & 15))
     return (int)hipErrorInvalidValue;
   if (!NORM && (!x || ((uintptr_t)x & 15) || ldx % 8 || (M > 1 && ldx < K))) return (int)hipErrorInvalidValue;
   if (out == kRowsRope && rp.slots && (!rp.kc || !rp.vc)) return (int)hipErrorInvalidValue;
@@ -274,7 +328,7 @@ static int rows_launch(const void* x, int ldx, const void* w, void* y, int ldy, 
   const size_t lds = NORM ? (size_t)M * K * 2 : 0;
 #define K8S_ROWS(OUT)                                                                                                   \
   hipLaunchKernelGGL((gemm_rows_kernel<MT, NF, CH, OUT, IN>), g, b, lds, s, (const uint16_t*)x, ldx, (const uint16_t*)w, y, \
-                     ldy, M, N, K, K / ranges, rp, nin, rsc)
+                     ldy, M, N, K, K / ranges, rp, nin, rsc, cv)
   if constexpr (NORM) {
     switch (out) {
       case kRowsSilu: K8S_ROWS(kRowsSilu); break;
@@ -295,6 +349,11 @@ static int rows_launch(const void* x, int ldx, const void* w, void* y, int ldy, 
       case kRowsSilu: K8S_ROWS(kRowsSilu); break;
       case kRowsRelu2: K8S_ROWS(kRowsRelu2); break;
       case kRowsRope: K8S_ROWS(kRowsRope); break;
+      case kRowsConv:
+        if constexpr (MT == 1) {
+          K8S_ROWS(kRowsConv);
+          break;
+        }
       default: return (int)hipErrorInvalidValue;
     }
   }
@@ -304,8 +363,9 @@ static int rows_launch(const void* x, int ldx, const void* w, void* y, int ldy, 
 
 template <int IN>
 static int rows_any(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int nf, int ranges, int out,
-                    const RowsRope& rp, const NormIn& nin, const RowScale& rsc, hipStream_t s) {
-#define K8S_ROWS_AS(MT, NF, CH) return rows_launch<MT, NF, CH, IN>(x, ldx, w, y, ldy, M, N, K, ranges, out, rp, nin, rsc, s)
+                    const RowsRope& rp, const NormIn& nin, const RowScale& rsc, const RowsConv& cv, hipStream_t s) {
+#define K8S_ROWS_AS(MT, NF, CH) \
+  return rows_launch<MT, NF, CH, IN>(x, ldx, w, y, ldy, M, N, K, ranges, out, rp, nin, rsc, cv, s)
   if (M <= 16) {
     switch (nf) {
       case 1: K8S_ROWS_AS(1, 1, 128);
@@ -332,7 +392,7 @@ using namespace k8s;
 K8S_API int k8s_gemm_rows(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int nf, int ranges,
                           int out, hipStream_t s) {
   if (out < kRowsBf16 || out > kRowsRelu2) return (int)hipErrorInvalidValue;
-  return rows_any<kRowsPlain>(x, ldx, w, y, ldy, M, N, K, nf, ranges, out, RowsRope{}, NormIn{}, RowScale{}, s);
+  return rows_any<kRowsPlain>(x, ldx, w, y, ldy, M, N, K, nf, ranges, out, RowsRope{}, NormIn{}, RowScale{}, RowsConv{}, s);
 }
 
 // The same for up to 16 rows, row m divided by sqrt(sum(part[m]) / width + eps).  out: 0 bf16, 1 fp32, 2 SwiGLU.
@@ -341,7 +401,19 @@ K8S_API int k8s_gemm_rows_scaled(const void* x, int ldx, const void* w, void* y,
   if (!part || ((uintptr_t)part & 15) || parts < 4 || parts % 4 || parts > kRowsParts || M > 16 || !(width > 0.f))
     return (int)hipErrorInvalidValue;
   return rows_any<kRowsScaled>(x, ldx, w, y, ldy, M, N, K, nf, ranges, out, RowsRope{}, NormIn{},
-                               RowScale{part, parts, width, eps}, s);
+                               RowScale{part, parts, width, eps}, RowsConv{}, s);
+}
+
+// Up to 16 rows, each the only one of its sequence: y [M][cols] <- the first `cols` columns (a multiple of 16 nf) as
+// k8s_gemm_rows and k8s_short_conv (no bias, 1 to 4 taps) leave them, tail too; rest [M][N - cols] <- the others in fp32.
+K8S_API int k8s_gemm_rows_conv(const void* x, int ldx, const void* w, void* y, int cols, float* rest, int M, int N, int K, int nf,
+                               const float* conv_w, int taps, float* tail, const int* pos0, const int* slot, int act,
+                               hipStream_t s) {
+  if (M > 16 || cols <= 0 || cols > N || (cols < N && !rest) || !conv_w || taps < 1 || taps > kConvTaps || (taps > 1 && !tail) ||
+      !pos0 || !slot)
+    return (int)hipErrorInvalidValue;
+  return rows_any<kRowsPlain>(x, ldx, w, y, cols, M, N, K, nf, 1, kRowsConv, RowsRope{}, NormIn{}, RowScale{},
+                              RowsConv{cols, taps, N - cols, act, conv_w, tail, pos0, slot, rest}, s);
 }
 
 // qkv = x . w^T (w = [q heads; k heads; v heads] x 128 rows) with q and k rotated and k, v written to their pages: what
@@ -351,7 +423,7 @@ K8S_API int k8s_gemm_rows_rope(const void* x, int ldx, const void* w, void* qkv,
                                int BS, hipStream_t s) {
   if (N != (nq + 2 * nkv) * 128 || !pos || !cos_sin || BS <= 0) return (int)hipErrorInvalidValue;
   const RowsRope rp{pos, cos_sin, slots, (uint16_t*)kc, (uint16_t*)vc, nq, nkv, BS};
-  return rows_any<kRowsPlain>(x, ldx, w, qkv, ldq, M, N, K, nf, 1, kRowsRope, rp, NormIn{}, RowScale{}, s);
+  return rows_any<kRowsPlain>(x, ldx, w, qkv, ldq, M, N, K, nf, 1, kRowsRope, rp, NormIn{}, RowScale{}, RowsConv{}, s);
 }
 
 // The SwiGLU (pos null) or rotating form on X = rmsnorm(x [or the planes `part`] + res_in) * norm_w, made by every workgroup
@@ -369,5 +441,5 @@ K8S_API int k8s_gemm_rows_norm(const void* x, int x_stride, const float* part, i
   const NormIn nin{(const uint16_t*)x, part, (const uint16_t*)res_in, (uint16_t*)res_out, (const uint16_t*)norm_w,
                    x_stride, splits, K, eps};
   const RowsRope rp{pos, cos_sin, slots, (uint16_t*)kc, (uint16_t*)vc, nq, nkv, BS};
-  return rows_any<kRowsNorm>(nullptr, 0, w, y, ldy, M, N, K, nf, 1, pos ? kRowsRope : kRowsSilu, rp, nin, RowScale{}, s);
+  return rows_any<kRowsNorm>(nullptr, 0, w, y, ldy, M, N, K, nf, 1, pos ? kRowsRope : kRowsSilu, rp, nin, RowScale{}, RowsConv{}, s);
 }

@@ -9,6 +9,7 @@
 // seg_pos0 > 0.  All recurrences, their decays, step sizes and gates are fp32;
 // TA is the activation type (bf16 as uint16_t, or float).
 #include "common.h"
+#include "gates.h"
 
 namespace k8s {
 
@@ -25,7 +26,6 @@ __device__ __forceinline__ void stm<float>(float* p, size_t i, float v) { p[i] =
 template <>
 __device__ __forceinline__ void stm<uint16_t>(uint16_t* p, size_t i, float v) { p[i] = f2bf(v); }
 
-__device__ __forceinline__ float silu_f(float v) { return v / (1.f + expf(-v)); }
 
 // exp of the recurrence's decays (arguments <= 0): the full-precision routine where activations are
 // fp32; where they are bf16 the hardware exponential 2^x (about 1e-6 relative, tiny results flush to 0)

@@ -40,7 +40,12 @@ struct StepArgs {
   void* out;              // [T][H V]
   float* ssp;             // KIND 2: [T][H]
   int H, G, V;
+  const float* lr;        // LOW: rows of stride bs, ra entries for the decays' gates, rg for the output's
+  const uint16_t* la;     // LOW: [H D][ra]
+  const uint16_t* lg;     // LOW: [H V][rg]
+  int ra, rg;
 };
+constexpr int kLowMax = 128;              // LOW: ra and rg, at most
 
 template <typename T>
 __device__ __forceinline__ float ss_ld(const T* p);
@@ -81,9 +86,14 @@ __device__ __forceinline__ f32x4 sum_rows(f32x4 v, f32x4 (*red)[LV]) {
   return s;
 }
 
-template <int KIND, int LV, int DR, typename TA, typename TO, typename TG>
+// LOW (KIND 0): the two products of low rank in front (low_rank_pair, small_proj.hip) are made here, by every workgroup for its
+// own head, where they were a launch: a thread has a quarter of K of a column of each 64, asked for in front of the state
+// (16 heads of 64 x 128, ranks of 64, 1 and 5 sequences: 7.4 -> 6.4 us, 8.9 -> 7.5).  The sums are low_rank_pair's, to the bit.
+template <int KIND, int LV, int DR, typename TA, typename TO, typename TG, bool LOW>
 __global__ void __launch_bounds__(256) state_step_kernel(StepArgs a) {
-  constexpr int RG = 256 / LV, D = DR * RG;
+  constexpr int RG = 256 / LV, D = DR * RG, VC = 4 * LV, CB = (D + VC) / 64;
+  static_assert(!LOW || KIND == 0);
+  __shared__ float lx[LOW ? 2 * kLowMax : 1], lp[LOW ? 4 : 1][LOW ? D + VC : 1];
   __shared__ float sq[D], sk[D], sg[KIND == 0 ? D : 1], sc[3][4];
   __shared__ f32x4 red[2][4][LV];
   static_assert(D <= 256, "a thread per entry of q and k");
@@ -94,10 +104,24 @@ __global__ void __launch_bounds__(256) state_step_kernel(StepArgs a) {
   const bool fresh = a.pos0[it] == 0;
   const int kv = KIND == 0 ? a.G * D : H * D, kh = KIND == 0 ? hh / (H / a.G) : hh;
   float q = 0.f, k = 0.f, n = 0.f, g = 0.f;
+  float lxv = 0.f;
+  u16x8 lwv[LOW ? CB : 1][kLowMax / 32];
+  if constexpr (LOW) {
+    if (tid < a.ra + a.rg) lxv = a.lr[(size_t)it * a.bs + tid];
+#pragma unroll
+    for (int b = 0; b < CB; ++b) {
+      const bool dec = b < D / 64;
+      const int col = 64 * b + (tid & 63), K = dec ? a.ra : a.rg;
+      const uint16_t* lw = (dec ? a.la + (size_t)(hh * D + col) * K : a.lg + (size_t)(hh * V + col - D) * K) + wv * (K / 4);
+#pragma unroll
+      for (int p = 0; p < kLowMax / 32; ++p)
+        if (32 * p < K) lwv[b][p] = *reinterpret_cast<const u16x8*>(lw + 8 * p);
+    }
+  }
   if (tid < D) {
     q = ss_ld(row + kh * D + tid);
     k = ss_ld(row + kv + kh * D + tid);
-    if (KIND == 0) g = a.a[((size_t)it * H + hh) * D + tid] + a.bias[hh * D + tid];
+    if (KIND == 0) g = LOW ? a.bias[hh * D + tid] : a.a[((size_t)it * H + hh) * D + tid] + a.bias[hh * D + tid];
     if (KIND == 1 && !fresh) n = a.nstate[((size_t)slot * H + hh) * D + tid];
   }
   f32x4 v = ss_ld4(row + 2 * kv + hh * V + c);
@@ -107,8 +131,41 @@ __global__ void __launch_bounds__(256) state_step_kernel(StepArgs a) {
   for (int i = 0; i < DR; ++i) S[i] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : ss_ld4(st + (size_t)(rg + RG * i) * V);
   f32x4 gt = f32x4{0.f, 0.f, 0.f, 0.f}, w = f32x4{1.f, 1.f, 1.f, 1.f};
   if (tid < LV) {
-    gt = ss_ld4((const TG*)a.gate + (size_t)it * a.gs + hh * V + c);
+    if (!LOW) gt = ss_ld4((const TG*)a.gate + (size_t)it * a.gs + hh * V + c);
     if (a.w) w = ss_ld4(a.w + hh * a.wh + c);
+  }
+  if constexpr (LOW) {
+    if (tid < a.ra + a.rg) lx[tid] = bf2f(f2bf(lxv));
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < CB; ++b) {
+      const int KG = (b < D / 64 ? a.ra : a.rg) / 4;
+      const float* xs = lx + (b < D / 64 ? 0 : a.ra) + wv * KG;
+      float s = 0.f;
+#pragma unroll
+      for (int p = 0; p < kLowMax / 32; ++p)
+        if (8 * p < KG) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) s = fmaf(xs[8 * p + j], bf2f(lwv[b][p][j]), s);
+        }
+      lp[wv][64 * b + (tid & 63)] = s;
+    }
+    __syncthreads();
+    if (tid < D) {
+      float s = 0.f;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s += lp[u][tid];
+      g = s + g;
+    }
+    if (tid < LV) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float s = 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s += lp[u][D + c + j];
+        gt[j] = s;
+      }
+    }
   }
   float fa = 1.f, ia = 1.f, m = 0.f;
   if (KIND == 1) {
@@ -202,10 +259,10 @@ __global__ void __launch_bounds__(256) state_step_kernel(StepArgs a) {
   if (KIND == 2 && tid == 0) a.ssp[(size_t)it * H + hh] = ss;
 }
 
-template <int KIND, typename TA, typename TO, typename TG>
+template <int KIND, typename TA, typename TO, typename TG, bool LOW = false>
 static int launch_step(const StepArgs& a, int n, int D, hipStream_t s) {
   const dim3 grid(n, a.H);
-#define K8S_ST(LV, DR) hipLaunchKernelGGL((state_step_kernel<KIND, LV, DR, TA, TO, TG>), grid, dim3(256), 0, s, a)
+#define K8S_ST(LV, DR) hipLaunchKernelGGL((state_step_kernel<KIND, LV, DR, TA, TO, TG, LOW>), grid, dim3(256), 0, s, a)
   if (a.V == 128 && D == 128)
     K8S_ST(32, 16);
   else if (a.V == 128 && D == 64)
@@ -236,6 +293,22 @@ K8S_API int k8s_delta_step(const void* qkv, int dt, const float* a, const float*
   p.pos0 = pos0; p.slot = slot; p.gate = gate; p.gs = gs; p.w = w; p.wh = wh; p.eps = eps; p.unit_eps = unit_eps;
   p.out = out; p.H = H; p.G = G; p.V = V;
   return dt == 0 ? launch_step<0, uint16_t, uint16_t, float>(p, n, D, s) : launch_step<0, float, float, float>(p, n, D, s);
+}
+
+// The same in bf16 with a = bf16(lr[., 0 .. ra)) . la^T, the gate = bf16(lr[., ra .. ra + rg)) . lg^T and beta behind them in the
+// same rows (stride ls): k8s_low_rank_pair and k8s_delta_step, to the bit.  ra, rg: 32, 64, 96 or 128; la, lg 16-byte aligned.
+K8S_API int k8s_delta_step_low(const void* qkv, const float* lr, int ls, int ra, int rg, const void* la, const void* lg,
+                               const float* rate, const float* dt_bias, float* state, const int* pos0, const int* slot,
+                               const float* w, int wh, void* out, int n, int H, int G, int D, int V, float eps,
+                               float unit_eps, hipStream_t s) {
+  if (n <= 0) return 0;
+  auto off = [](int k, const void* p) { return k < 32 || k > kLowMax || k % 32 || !p || ((uintptr_t)p & 15); };
+  if (off(ra, la) || off(rg, lg) || !lr || ls < ra + rg + H || G < 1 || H % G) return (int)hipErrorInvalidValue;
+  StepArgs p{};
+  p.x = qkv; p.xs = 2 * G * D + H * V; p.rate = rate; p.bias = dt_bias; p.beta = lr + ra + rg; p.bs = ls; p.state = state;
+  p.pos0 = pos0; p.slot = slot; p.w = w; p.wh = wh; p.eps = eps; p.unit_eps = unit_eps; p.out = out; p.H = H; p.G = G; p.V = V;
+  p.lr = lr; p.ra = ra; p.rg = rg; p.la = (const uint16_t*)la; p.lg = (const uint16_t*)lg;
+  return launch_step<0, uint16_t, uint16_t, float, true>(p, n, D, s);
 }
 
 K8S_API int k8s_memory_step(const float* x, int xs, const float* gate_bias, float cap, float* state, float* nstate,

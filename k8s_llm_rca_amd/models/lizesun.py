@@ -354,10 +354,9 @@ class LizesunModel:
                 L["mem_norm"] = f32(b + "norm")
                 L["wo_r"] = put(b + "o")
             else:
-                L["w_qkv"] = put(p + "q", p + "k", p + "v")
+                # q | k | v, then the inputs of the decays and of the gate, beta (fp32 out)
+                L["w_in"] = put(p + "q", p + "k", p + "v", p + "a1", p + "g1", p + "b")
                 L["conv_w"] = f32(p + "q.conv", p + "k.conv", p + "v.conv")
-                L["ra"], L["rg"] = int(get(p + "a1").shape[0]), int(get(p + "g1").shape[0])
-                L["w_agb"] = put(p + "a1", p + "g1", p + "b")                   # one fp32-out GEMM
                 L["w_a2"], L["w_g2"] = put(p + "a2"), put(p + "g2")
                 L["rate"] = torch.exp(f32(p + "A_log")).contiguous()
                 L["dt_bias"] = f32(p + "dt_bias")
@@ -414,14 +413,10 @@ class LizesunModel:
 
     def _delta(self, li: int, h, inp: S.SegStepInputs, states) -> torch.Tensor:
         L, c = self.layers[li], self.cfg.layers[li].delta
-        j, ra, rg = self.delta_of[li], L["ra"], L["rg"]
-        qkv = R.proj(h, L["w_qkv"], keep=True)                       # [T, 2 G D + H V]
-        qkv = S.short_conv(qkv, L["conv_w"], None, states[f"dconv{j}"], inp.seg, act=True)
-        agb = R.proj_f32out(h, L["w_agb"])                             # [T, ra + rg + H] fp32
-        # [T, H D] before bias and softplus, [T, H V] before the sigmoid, both fp32
-        dec, gate = S.low_rank_pair(agb, 0, L["w_a2"], ra, L["w_g2"], self.dtype)
-        return S.delta_layer(qkv, c.heads, c.kv_heads, c.dim, c.vdim, dec, L["rate"], L["dt_bias"], agb[:, ra + rg:],
-                             states[f"delta{j}"], inp.seg, gate, L["delta_norm"], self.cfg.norm_eps, self.dtype)
+        j = self.delta_of[li]
+        qkv, agb = R.conv_proj(h, L["w_in"], L["conv_w"], states[f"dconv{j}"], inp.seg)      # [T, 2 G D + H V], [T, ra + rg + H]
+        return S.delta_low_rank(qkv, c.heads, c.kv_heads, c.dim, c.vdim, agb, L["w_a2"], L["w_g2"], L["rate"], L["dt_bias"],
+                                states[f"delta{j}"], inp.seg, L["delta_norm"], self.cfg.norm_eps, self.dtype)
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[torch.Tensor],
                 vts: List[Optional[torch.Tensor]], states: Dict[str, torch.Tensor],

@@ -39,6 +39,7 @@ _SIGS = {
     "k8s_gemm_skinny": [P, I, P, P, I, I, I, I, P],
     "k8s_gemm_rows": [P, I, P, P, I, I, I, I, I, I, I, P],
     "k8s_gemm_rows_scaled": [P, I, P, P, I, I, I, I, I, I, I, P, I, F, F, P],
+    "k8s_gemm_rows_conv": [P, I, P, P, I, P, I, I, I, I, P, I, P, P, P, I, P],
     "k8s_gemm_step_rms": [P, I, P, P, P, I, F, F, P, P, F, P, P, P, I, I, I, P],
     "k8s_gemm_step_dyt": [P, I, P, F, P, I, P, F, P, F, P, P, P, I, I, I, P],
     "k8s_gemm_stream_reduce": [P, I, P, I, I, I, P],
@@ -113,6 +114,7 @@ _SIGS = {
     "k8s_latent_attn_mfma": [P, P, P, P, I, P, I, P, I, P, I, I, I, F, P, L, L, P, I, L, L, I, P],
     "k8s_latent_attn_token": [P, L, L, P, I, P, P, P, I, P, I, P, I, P, P, L, L, P, P, I, I, I, I, I, I, I, F, P],
     "k8s_delta_step": [P, I, P, P, P, P, I, P, P, P, P, I, P, I, P, I, I, I, I, I, F, F, P],
+    "k8s_delta_step_low": [P, P, I, I, I, P, P, P, P, P, P, P, P, I, P, I, I, I, I, I, F, F, P],
     "k8s_memory_step": [P, I, P, F, P, P, P, P, P, P, I, P, I, P, I, I, I, I, I, F, F, P],
     "k8s_decay_step": [P, I, I, P, P, P, P, P, I, P, P, P, I, I, I, I, P],
     "k8s_head_proj": [P, L, L, P, P, L, L, I, I, I, I, P, P, I, I, I, P],

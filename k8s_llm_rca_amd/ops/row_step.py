@@ -282,3 +282,33 @@ def glu_proj(h, w: torch.Tensor) -> torch.Tensor:
 
 def relu_sq_proj(h, w: torch.Tensor) -> torch.Tensor:
     return L.relu_sq_proj(h, w) if isinstance(h, torch.Tensor) else h.product(w, L.ROWS_RELU2, L.relu_sq_proj)
+
+
+CONV_TAPS = 4
+
+
+def conv_proj(h, w: torch.Tensor, conv_w: torch.Tensor, tail: torch.Tensor, seg) -> tuple:
+    """``h @ w.T``: its first ``len(conv_w)`` columns behind :func:`..ops.seq_ops.short_conv` with SiLU, the others in fp32.
+
+    Up to 16 single tokens that is one product whose epilogue convolves (csrc/kernels/gemm_rows.hip).  us of three launches /
+    one, columns convolved + others x K, 4 taps, at 1, 5, 16 tokens: 2304 + 144 x 2048 10.6 / 5.3, 11.1 / 5.5, 12.4 / 6.2;  2048 +
+    64 x 1024 8.3 / 4.0, 9.2 / 4.3, 10.0 / 4.7;  6144 + 256 x 2048 12.8 / 7.3, 13.4 / 7.4, 14.8 / 8.8;  12288 + 512 x 4096 26.2 /
+    18.4, 26.8 / 20.1, 33.2 / 25.0."""
+    from . import seq_ops as S
+    C, taps = conv_w.shape
+    if isinstance(h, torch.Tensor) and h.shape[0] <= INTO_ROWS:      # (before anything else: prompts pay for one comparison)
+        (m, k), n = h.shape, w.shape[0]
+        if (m == seg.n_seg == seg.singles() and 0 < C < n and L.rows_ok(h, w) and w.device == h.device
+                and all((c, k) not in L.dispatch_table() for c in (C, n - C, n))
+                and 1 <= taps <= CONV_TAPS and conv_w.dtype == torch.float32 == tail.dtype and conv_w.is_contiguous()
+                and tail.is_contiguous() and tail.shape[1:] == (taps - 1, C)):
+            p = L.rows_plan(m, n, k)
+            if p is not None and C % (16 * p[0]) == 0:
+                out = torch.empty(m, C, dtype=h.dtype, device=h.device)
+                rest = torch.empty(m, n - C, dtype=torch.float32, device=h.device)
+                check(lib().k8s_gemm_rows_conv(ptr(h), h.stride(0), ptr(w), ptr(out), C, ptr(rest), m, n, k, p[0], ptr(conv_w),
+                                               taps, ptr(tail), ptr(seg.seg_pos0), ptr(seg.seg_slot), 1, stream_ptr(h)),
+                      "gemm_rows_conv")
+                return out, rest
+    x = proj(h, w[:C], keep=True)
+    return S.short_conv(x, conv_w, None, tail, seg, act=True), proj_f32out(h, w[C:])

@@ -1705,6 +1705,9 @@ def _step_ok(x: torch.Tensor, seg: SegMeta, D: int, V: int, state: torch.Tensor,
             and (w is None or (w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0)))
 
 
+DELTA_LOW_RANK, DELTA_LOW_HEAD, DELTA_LOW_ALL = 128, 24576, 6 << 20     # ranks; entries of a head's weights; of all that is read
+
+
 def delta_layer(qkv: torch.Tensor, H: int, G: int, D: int, V: int, a: torch.Tensor, rate: torch.Tensor,
                 dt_bias: torch.Tensor, beta: torch.Tensor, state: torch.Tensor, seg: SegMeta, gate: torch.Tensor,
                 w: Optional[torch.Tensor], eps: float, out_dtype) -> torch.Tensor:
@@ -1725,6 +1728,38 @@ def delta_layer(qkv: torch.Tensor, H: int, G: int, D: int, V: int, a: torch.Tens
         return out
     o = gated_delta(qkv, H, G, D, V, a, rate, dt_bias, beta, state, seg)
     return head_norm_gate(o, gate, w, H, V, eps, out_dtype)
+
+
+def delta_low_rank(qkv: torch.Tensor, H: int, G: int, D: int, V: int, lr: torch.Tensor, wa: torch.Tensor, wg: torch.Tensor,
+                   rate: torch.Tensor, dt_bias: torch.Tensor, state: torch.Tensor, seg: SegMeta, w: Optional[torch.Tensor],
+                   eps: float, out_dtype) -> torch.Tensor:
+    """:func:`delta_layer` with decays' and output gates as products of low rank: ``lr`` [T, ra + rg + H] fp32 holds their inputs
+    and beta's (:func:`low_rank_pair`, ``wa`` [H D, ra], ``wg`` [H V, rg]).
+
+    Of single tokens the state's kernel makes them itself, every workgroup (a head of one token) with its own head's weights.
+    us of two launches / one, H, D, V, both ranks:  16, 64, 128, 64, 64 at 1, 5, 32, 64 tokens 7.4 / 6.4, 8.9 / 7.5, 13.3 / 11.9,
+    18.9 / 23.3;  4, 64, 64, 32, 32 at 1, 64 7.0 / 5.4, 9.0 / 6.8;  64, 64, 128, 128, 128 at 1, 3, 5, 16 9.1 / 8.9, 10.5 / 9.8,
+    12.8 / 13.1, 21.7 / 27.6;  32, 128, 128, 64, 128 at 5, 16, 32 12.8 / 11.0, 20.4 / 19.8, 42.1 / 43.4: the line is what all of
+    them read.  And past 48 KB a head one token waits for them: 16, 128, 128, 128, 128 at 1, 3, 8 8.5 / 8.9, 10.1 / 10.4,
+    12.3 / 11.4."""
+    ra, rg, T = wa.shape[1], wg.shape[1], qkv.shape[0]
+    mine = wa.shape[0] // H * ra + wg.shape[0] // H * rg
+    if (0 < T * H * mine <= DELTA_LOW_ALL and mine <= DELTA_LOW_HEAD and qkv.dtype == torch.bfloat16 == out_dtype and _small_rows(qkv, wa) and _small_rows(qkv, wg)
+            and all(32 <= k <= DELTA_LOW_RANK and k % 32 == 0 and t.data_ptr() % 16 == 0 for k, t in ((ra, wa), (rg, wg)))
+            and _step_ok(qkv, seg, D, V, state, qkv, w) and qkv.is_contiguous() and lr.dtype == torch.float32
+            and lr.stride(1) == 1 and lr.shape == (T, ra + rg + H)):
+        assert qkv.shape[1] == 2 * G * D + H * V and H % G == 0 and state.is_contiguous() and state.shape[1:] == (H, D, V)
+        assert wa.shape[0] == H * D and wg.shape[0] == H * V and (w is None or w.numel() in (V, H * V))
+        assert rate.dtype == dt_bias.dtype == torch.float32 and rate.numel() == H and dt_bias.numel() == H * D
+        out = torch.empty(T, H * V, dtype=out_dtype, device=qkv.device)
+        check(lib().k8s_delta_step_low(ptr(qkv), ptr(lr), lr.stride(0), ra, rg, ptr(wa), ptr(wg), ptr(rate), ptr(dt_bias),
+                                       ptr(state), ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(w),
+                                       V if w is not None and w.numel() == H * V else 0, ptr(out), T, H, G, D, V, float(eps),
+                                       float(UNIT_EPS), stream_ptr(qkv)), "delta_step_low")
+        return out
+    # [T, H D] before bias and softplus, [T, H V] before the sigmoid, both fp32
+    dec, gate = low_rank_pair(lr, 0, wa, ra, wg, out_dtype)
+    return delta_layer(qkv, H, G, D, V, dec, rate, dt_bias, lr[:, ra + rg:], state, seg, gate, w, eps, out_dtype)
 
 
 def memory_layer(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tensor, cap: float, state: torch.Tensor,
