@@ -6,6 +6,7 @@
 // written once (TA: bf16 as uint16_t, or float).  Four consecutive columns per thread where the width
 // allows 16-byte accesses.
 #include "common.h"
+#include "rope_rows.h"
 
 namespace k8s {
 
@@ -82,12 +83,13 @@ __global__ void __launch_bounds__(256) add_dyt1_kernel(float* __restrict__ x, co
   }
 }
 
-// x = embed[id] * scale;  out = dyt(x) (w optional).  One workgroup per row.
+// x = embed[id] * scale;  out = dyt(x) (w optional).  One workgroup per row; those past the T rows: rope_rows.h.
 template <typename TE, typename TA>
 __global__ void __launch_bounds__(256) embed_scale_dyt_kernel(const int* __restrict__ ids, const TE* __restrict__ embed,
                                                               float scale, float* __restrict__ x, float alpha,
                                                               const float* __restrict__ w, const float* __restrict__ b,
-                                                              TA* __restrict__ out, int W) {
+                                                              TA* __restrict__ out, int W, int T, RopeTables rt) {
+  if ((int)blockIdx.x >= T) return rope_block(rt, T);
   const size_t o = (size_t)blockIdx.x * W, src = (size_t)ids[blockIdx.x] * W;
   for (int c = threadIdx.x; c < W; c += 256) {
     const float xv = ldd(embed, src + c) * scale;
@@ -106,7 +108,8 @@ template <typename TE, typename TA>
 __global__ void __launch_bounds__(512) embed_scale_dyt4_kernel(const int* __restrict__ ids, const TE* __restrict__ embed,
                                                                float scale, float* __restrict__ x, float alpha,
                                                                const float* __restrict__ w, const float* __restrict__ b,
-                                                               TA* __restrict__ out, int W) {
+                                                               TA* __restrict__ out, int W, int T, RopeTables rt) {
+  if ((int)blockIdx.x >= T) return rope_block(rt, T);
   const size_t o = (size_t)blockIdx.x * W, src = (size_t)ids[blockIdx.x] * W;
   for (int c = 4 * threadIdx.x; c < W; c += 4 * blockDim.x) {
     f32x4 v = ldd4(embed, src + c), wv = f32x4{0.f, 0.f, 0.f, 0.f}, bv = wv;
@@ -191,18 +194,22 @@ K8S_API int k8s_add_dyt(float* x, const float* y, float sy, const float* y2, flo
 }
 
 K8S_API int k8s_embed_scale_dyt(const int* ids, const void* embed, int edt, float scale, float* x, float alpha,
-                                const float* w, const float* b, void* out, int odt, int T, int W, hipStream_t s) {
+                                const float* w, const float* b, void* out, int odt, int T, int W, hipStream_t s,
+                                const int* pos, const double* freq0, float amp0, int half0,
+                                float* cs0, const double* freq1, float amp1, int half1, float* cs1) {
   if (T <= 0 || W <= 0) return 0;
   if ((w == nullptr) != (out == nullptr) || (w && !b)) return (int)hipErrorInvalidValue;
+  const RopeTables rt{pos, {freq0, freq1}, {cs0, cs1}, {amp0, amp1}, {half0, half1}};
+  if (!rope_tables_ok(rt)) return (int)hipErrorInvalidValue;
   const bool by4 = W % 4 == 0 && (((uintptr_t)embed | (uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)out) & 15) == 0;
-  const int t4 = (W / 4 + 63) / 64 * 64;
+  const int t4 = W > 2048 - 256 ? 512 : (W / 4 + 63) / 64 * 64;
 #define K8S_EMB(TE, TA)                                                                                                 \
   if (by4)                                                                                                              \
-    hipLaunchKernelGGL((embed_scale_dyt4_kernel<TE, TA>), dim3(T), dim3(t4 > 512 ? 512 : t4), 0, s, ids,                \
-                       (const TE*)embed, scale, x, alpha, w, b, (TA*)out, W);                                           \
+    hipLaunchKernelGGL((embed_scale_dyt4_kernel<TE, TA>), dim3(T + rope_blocks(rt, T, t4)), dim3(t4), 0, s, ids,        \
+                       (const TE*)embed, scale, x, alpha, w, b, (TA*)out, W, T, rt);                                    \
   else                                                                                                                  \
-    hipLaunchKernelGGL((embed_scale_dyt_kernel<TE, TA>), dim3(T), dim3(256), 0, s, ids, (const TE*)embed, scale, x,     \
-                       alpha, w, b, (TA*)out, W)
+    hipLaunchKernelGGL((embed_scale_dyt_kernel<TE, TA>), dim3(T + rope_blocks(rt, T, 256)), dim3(256), 0, s, ids,         \
+                       (const TE*)embed, scale, x, alpha, w, b, (TA*)out, W, T, rt)
   if (edt == 0 && odt == 0) {
     K8S_EMB(uint16_t, uint16_t);
   } else if (edt == 0) {

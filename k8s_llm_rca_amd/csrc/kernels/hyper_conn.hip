@@ -13,6 +13,7 @@
 // One workgroup per row; a thread owns VEC neighbouring columns of all streams, so the S x S mix is in
 // registers; the row of u stays in LDS between the sum of squares and the output.
 #include "common.h"
+#include "rope_rows.h"
 
 namespace k8s {
 
@@ -178,14 +179,15 @@ __global__ void __launch_bounds__(1024) hyper_step_kernel(float* __restrict__ x,
   if (h) norm_row<VEC>(u, ss, red, nw, w0, eps, h, o, W);
 }
 
-// x_s = embed[id] * scale for every stream s; h = the first sublayer's normed input.
+// x_s = embed[id] * scale for every stream s; h = the first sublayer's normed input.  Workgroups past the T rows: rope_rows.h.
 template <int VEC, typename TE, typename TA>
 __global__ void __launch_bounds__(1024) hyper_embed_kernel(const int* __restrict__ ids, const TE* __restrict__ embed,
                                                           float scale, float* __restrict__ x, int S,
                                                           const float* __restrict__ in, const float* __restrict__ nw,
-                                                          float eps, TA* __restrict__ h, int W) {
+                                                          float eps, TA* __restrict__ h, int W, int T, RopeTables rt) {
   extern __shared__ float u[];
   __shared__ float red[16];
+  if ((int)blockIdx.x >= T) return rope_block(rt, T);
   const size_t t = blockIdx.x, e0 = (size_t)ids[t] * W;
   float si = 0.f, w0[VEC];
   first_weights<VEC>(nw, W, true, w0);
@@ -295,12 +297,17 @@ K8S_API int k8s_hyper_step(float* x, const void* y, int ydt, const int* inv, con
 }
 
 K8S_API int k8s_hyper_embed(const int* ids, const void* embed, int edt, float scale, float* x, int S, const float* in,
-                            const float* nw, float eps, void* h, int hdt, int T, int W, hipStream_t s) {
+                            const float* nw, float eps, void* h, int hdt, int T, int W, hipStream_t s,
+                            const int* pos, const double* freq0, float amp0, int half0,
+                            float* cs0, const double* freq1, float amp1, int half1, float* cs1) {
   if (T <= 0) return 0;
   if (!hyper_row_ok(W) || S < 1 || !in || !nw || !h) return (int)hipErrorInvalidValue;
+  const RopeTables rt{pos, {freq0, freq1}, {cs0, cs1}, {amp0, amp1}, {half0, half1}};
+  if (!rope_tables_ok(rt)) return (int)hipErrorInvalidValue;
 #define K8S_HE(VEC, TE, TA)                                                                                       \
-  hipLaunchKernelGGL((hyper_embed_kernel<VEC, TE, TA>), dim3(T), dim3(hyper_threads(T, W, VEC)), W * sizeof(float), \
-                     s, ids, (const TE*)embed, scale, x, S, in, nw, eps, (TA*)h, W)
+  hipLaunchKernelGGL((hyper_embed_kernel<VEC, TE, TA>), dim3(T + rope_blocks(rt, T, hyper_threads(T, W, VEC))),   \
+                     dim3(hyper_threads(T, W, VEC)), W * sizeof(float), s, ids, (const TE*)embed, scale, x, S, in, nw, eps, \
+                     (TA*)h, W, T, rt)
 #define K8S_HEV(TE, TA)        \
   if (W % 4 == 0) {            \
     K8S_HE(4, TE, TA);         \

@@ -30,6 +30,7 @@
 // Scores, weights and accumulation are fp32; TA (bf16 as uint16_t, or float) is the type of q, the pages
 // and the output.
 #include "common.h"
+#include "rope_rows.h"
 #include "key_runs.h"
 
 namespace k8s {
@@ -156,18 +157,11 @@ __global__ void __launch_bounds__(256) attn_prep_kernel(const float* __restrict_
   }
 }
 
-// cs [T][2 half]: cos | sin of positions[t] * freq[j], times amp (the product in double).
 __global__ void __launch_bounds__(256) rope_table_kernel(const int* __restrict__ positions,
                                                          const double* __restrict__ freq, float amp,
                                                          float* __restrict__ cs, size_t n, int half) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const size_t t = i / half;
-  const int j = (int)(i - t * half);
-  double si, co;
-  sincos((double)positions[t] * freq[j], &si, &co);
-  cs[t * 2 * half + j] = (float)co * amp;
-  cs[t * 2 * half + half + j] = (float)si * amp;
+  if (i < n) rope_entry(positions, freq, amp, cs, half, i);
 }
 
 template <typename TA>

@@ -231,6 +231,7 @@ class FikeraxModel:
             if key is not None and key not in made:
                 made[key] = S.make_rope(key[1], key[2], self.device, **kw)
             self.ropes.append(made.get(key))
+        self.turns = list(made.values())
         if cfg.loop is not None:
             start, stop, times = cfg.loop
             if not 0 <= start <= stop <= len(cfg.layers) or times < 0:
@@ -368,15 +369,6 @@ class FikeraxModel:
         return sum(t.numel() * t.element_size() for t in ts)
 
     # -------------------------------------------------------------- forward
-    def _table(self, i: int, inp: S.SegStepInputs, tables) -> Optional[torch.Tensor]:
-        """cos | sin of the step's positions for layer ``i``'s rotation, made once per distinct rotation."""
-        rope = self.ropes[i]
-        if rope is None:
-            return None
-        if id(rope) not in tables:
-            tables[id(rope)] = S.rope_table(inp.positions, rope)
-        return tables[id(rope)]
-
     def _lightning(self, i: int, h, inp: S.SegStepInputs, state: torch.Tensor) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
         HV = c.heads * c.vdim
@@ -387,14 +379,14 @@ class FikeraxModel:
     def _attention(self, i: int, h, inp: S.SegStepInputs, tables, kc, vc, vt) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
         x = R.proj_planes(h, L["w_in"])
-        prep = dict(norm="head", eps=self.cfg.norm_eps, rope=self.ropes[i], rope_cs=self._table(i, inp, tables))
+        prep = dict(norm="head", eps=self.cfg.norm_eps, rope=self.ropes[i], rope_cs=tables.of(self.ropes[i]))
         return S.prep_attention(x, L["b_in"], c.heads, c.kv_heads, c.dim, c.vdim, inp.positions, inp.slots, kc, vc, vt, inp.seg,
                                 self.dtype, c.scale, prep, dict(window=c.window))
 
     def _latent_attention(self, i: int, h, inp: S.SegStepInputs, tables, cache, cache_t) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
         T, H, D, V, KR = inp.input_ids.shape[0], c.heads, c.dim, c.vdim, c.kv_rank
-        cs = self._table(i, inp, tables)
+        cs = tables.of(self.ropes[i])
         dn = R.proj_planes(h, L["w_in"])                                      # [., T, q_rank + KR + rot_dim] fp32
         cq = S.latent_norm(dn, L["dq_norm"], L["dkv_norm"], inp.slots, cache, c.q_rank, KR, self.cfg.norm_eps, self.dtype,
                            cache_t=cache_t, tail=c.rot_dim, tail_cs=cs)
@@ -421,10 +413,11 @@ class FikeraxModel:
         idx = S.wanted_rows(inp)
         few = idx is None or T <= R.INTO_ROWS              # (few rows: the same products whichever of them are wanted)
         mix1 = one.view(1, 1)
-        tables: Dict[int, torch.Tensor] = {}
+        tables = S.RopeTables(inp.positions, self.turns)   # cos | sin of the step's positions, one per distinct rotation
         again = (inp.input_ids, self.embed, cfg.embed_scale)
         x = torch.empty(T, 1, cfg.hidden, dtype=torch.float32, device=self.device)
-        h = N.hyper_embed(inp.input_ids, self.embed, cfg.embed_scale, x, one, self.layers[self.runs[0][0]]["norm1"], eps, dt)
+        h = N.hyper_embed(inp.input_ids, self.embed, cfg.embed_scale, x, one, self.layers[self.runs[0][0]]["norm1"], eps, dt,
+                          tables=tables)
         for r, (i, _) in enumerate(self.runs):
             spec, L, ci = cfg.layers[i], self.layers[i], self.cache_of[r]
             # the write-back of the run's last sublayer also reads the next run's input

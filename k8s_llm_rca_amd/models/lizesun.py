@@ -392,18 +392,15 @@ class LizesunModel:
         return S.prep_attention(x[:, :n], L["bias"], H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg,
                                 self.dtype, a.scale, prep, dict(softcap=a.softcap, chunk=a.chunk, gate=x[:, n:]))
 
-    def _parallel(self, li: int, h, inp: S.SegStepInputs, kcs, vcs, vts, states, tables: dict):
+    def _parallel(self, li: int, h, inp: S.SegStepInputs, kcs, vcs, vts, states, tables: S.RopeTables):
         L, spec = self.layers[li], self.cfg.layers[li]
         a, b = spec.left, spec.right
         ci, j = self.cache_of[li], self.mem_of[li]
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
         nl = H * D + G * (D + V)
         x = R.proj_f32out(h, L["w_in"])                                # left q | k | v, right q | k | v | g | i | f
-        key = (a.rot_dims, a.rot_base)
-        rope = self.ropes.get(key)
-        if rope is not None and key not in tables:                     # cos | sin of the step's positions, made once
-            tables[key] = S.rope_table(inp.positions, rope)
-        prep = dict(norm=True, eps=self.cfg.norm_eps, rope=rope, rope_cs=tables.get(key))
+        rope = self.ropes.get((a.rot_dims, a.rot_base))
+        prep = dict(norm=True, eps=self.cfg.norm_eps, rope=rope, rope_cs=tables.of(rope))
         ol = S.prep_attention(x[:, :nl], None, H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg,
                               self.dtype, a.scale, prep, dict(window=a.window, keep_first=a.keep_first, sink=L["sink"]))
         xr = x[:, nl:]
@@ -430,9 +427,9 @@ class LizesunModel:
         few = nl > 0 and (idx is None or T <= R.INTO_ROWS)   # (few rows: the same products whichever of them are wanted)
         x = torch.empty(T, W, dtype=torch.float32, device=self.device)
         first = self.layers[0]["norm1"] if nl else (1.0, None, None)
-        h = N.embed_scale_dyt(inp.input_ids, self.embed, cfg.embed_scale, x, *first, out_dtype=dt)
+        tables = S.RopeTables(inp.positions, self.ropes.values())      # cos | sin of the step's positions, made once
+        h = N.embed_scale_dyt(inp.input_ids, self.embed, cfg.embed_scale, x, *first, out_dtype=dt, tables=tables)
         vmix: dict = {}
-        tables: dict = {}
         for li, (spec, L) in enumerate(zip(cfg.layers, self.layers)):
             # (the final norm reads the wanted rows only, or with the last layer where every row is wanted or there are few)
             nxt = self.layers[li + 1]["norm1"] if li + 1 < nl else self.final_norm if few else (1.0, None, None)

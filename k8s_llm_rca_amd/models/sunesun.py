@@ -286,10 +286,8 @@ class SunesunModel:
         a, rope = self.cfg.layers[li].attn, self.ropes[li]
         H, G, D = a.heads, a.kv_heads, a.dim
         x = proj_f32out(h, L["w_in"])                                  # [T, H D + G D] fp32
-        if rope is not None and id(rope) not in tables:
-            tables[id(rope)] = S.rope_table(inp.positions, rope)
         q = S.attn_prep(x, None, H, G, D, D, inp.positions, inp.slots, kc, vc, self.dtype, rope=rope,
-                        rope_cs=tables.get(id(rope)), vt=vt, v_is_k=True)
+                        rope_cs=tables.of(rope), vt=vt, v_is_k=True)
         o = S.masked_attention(q, H, G, D, D, kc, vc, inp.seg, a.scale, softcap=a.softcap, window=a.window, vt=vt)
         return proj_f32out(o, L["wo"])
 
@@ -324,9 +322,11 @@ class SunesunModel:
         cfg, eps, dt = self.cfg, self.cfg.norm_eps, self.dtype
         T = inp.input_ids.shape[0]
         runs = [self.weights[s] for s in self.source]
-        tables: Dict[int, torch.Tensor] = {}       # cos | sin of the step's positions, one per distinct rotation
+        # cos | sin of the step's positions, one per distinct rotation
+        tables = S.RopeTables(inp.positions, {id(r): r for r in self.ropes if r is not None}.values())
         x = torch.empty(T, max(1, cfg.streams), cfg.hidden, dtype=torch.float32, device=self.device)
-        h = N.hyper_embed(inp.input_ids, self.embed, cfg.embed_scale, x, runs[0]["in1"], runs[0]["norm1"], eps, dt)
+        h = N.hyper_embed(inp.input_ids, self.embed, cfg.embed_scale, x, runs[0]["in1"], runs[0]["norm1"], eps, dt,
+                          tables=tables)
         for li, (spec, L) in enumerate(zip(cfg.layers, runs)):
             nxt = runs[li + 1] if li + 1 < len(runs) else None
             into = dict(inn=nxt["in1"], nw=nxt["norm1"], eps=eps, out_dtype=dt) if nxt is not None else {}

@@ -148,7 +148,7 @@ _SIGS = {
     "k8s_window_attn_mfma": [P, I, P, P, P, I, P, I, P, P, P, P, I, I, I, I, I, I, F, P, I, I, P, P],
     "k8s_window_attn_rows": [P, I, P, P, P, I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
     "k8s_add_dyt": [P, P, F, P, F, F, P, P, P, I, I, I, P, I, I],
-    "k8s_embed_scale_dyt": [P, P, I, F, P, F, P, P, P, I, I, I, P],
+    "k8s_embed_scale_dyt": [P, P, I, F, P, F, P, P, P, I, I, I, P, P, P, F, I, P, P, F, I, P],
     "k8s_relu_sq": [P, P, ctypes.c_long, I, P],
     "k8s_attn_prep": [P, I, P, I, I, I, I, P, P, P, P, P, I, P, I, I, P, P, F, I, F, F, P, P, I, P, I, F, I, P, F, I, P],
     "k8s_rope_table": [P, P, F, P, I, I, P],
@@ -163,7 +163,7 @@ _SIGS = {
     "k8s_head_norm_gate": [P, P, I, P, I, P, I, I, I, F, I, P, P, I, F, F, I],
     "k8s_ssd_scan": [P, I, P, I, I, P, I, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, I, P, P, I, P, P, P],
     "k8s_hyper_step": [P, P, I, P, P, I, P, P, P, P, F, P, I, I, I, I, P, P, P, F, I, P, I, F, F],
-    "k8s_hyper_embed": [P, P, I, F, P, I, P, P, F, P, I, I, I, P],
+    "k8s_hyper_embed": [P, P, I, F, P, I, P, P, F, P, I, I, I, P, P, P, F, I, P, P, F, I, P],
     "k8s_hyper_read": [P, P, I, I, P, P, F, P, I, I, P],
     "k8s_walks": [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P, P, P, P],
 }

@@ -274,9 +274,14 @@ def softcap_(logits: torch.Tensor, scale: float, cap: float) -> torch.Tensor:
 # ------------------------------------------------------------------ Dynamic Tanh norm around an fp32 residual
 # (csrc/kernels/dyt_ops.hip).  ``dyt(x) = tanh(alpha x) * w + b`` per element: no mean, no variance, so
 # nothing couples a row's entries and the residual add, the norm and the cast are one elementwise pass.
+def _tables(tables) -> tuple:
+    return (0, 0, 0.0, 0, 0, 0, 0.0, 0, 0) if tables is None else tables.args()
+
+
 def embed_scale_dyt(ids: torch.Tensor, embed: torch.Tensor, scale: float, x_out: torch.Tensor, alpha: float,
-                    w: Optional[torch.Tensor], b: Optional[torch.Tensor], out_dtype) -> Optional[torch.Tensor]:
-    """``x_out = embed[ids] * scale`` (fp32); with ``w, b`` also returns ``dyt(x_out)`` as activations."""
+                    w: Optional[torch.Tensor], b: Optional[torch.Tensor], out_dtype, tables=None) -> Optional[torch.Tensor]:
+    """``x_out = embed[ids] * scale`` (fp32); with ``w, b`` also returns ``dyt(x_out)`` as activations.  ``tables``
+    (:class:`..ops.seq_ops.RopeTables`): filled in the same launch."""
     T, W = ids.shape[0], embed.shape[1]
     h = torch.empty(T, W, dtype=out_dtype, device=embed.device) if w is not None else None
     if use_hip(embed):
@@ -284,8 +289,10 @@ def embed_scale_dyt(ids: torch.Tensor, embed: torch.Tensor, scale: float, x_out:
         assert embed.is_contiguous() and ids.dtype == torch.int32
         check(lib().k8s_embed_scale_dyt(ptr(ids), ptr(embed), _odt(embed.dtype), float(scale), ptr(x_out),
                                         float(alpha), ptr(w), ptr(b), ptr(h), _odt(out_dtype) if h is not None else 1,
-                                        T, W, stream_ptr(embed)), "embed_scale_dyt")
+                                        T, W, stream_ptr(embed), *_tables(tables)), "embed_scale_dyt")
         return h
+    if tables is not None:
+        tables.fill()
     x_out.copy_(embed[ids.long()].float() * scale)
     if h is not None:
         h.copy_((torch.tanh(alpha * x_out) * w + b).to(out_dtype))
@@ -337,9 +344,10 @@ def _rms_rows(u: torch.Tensor, w: torch.Tensor, eps: float, out_dtype) -> torch.
 
 
 def hyper_embed(ids: torch.Tensor, embed: torch.Tensor, scale: float, x: torch.Tensor, inn: torch.Tensor,
-                nw: torch.Tensor, eps: float, out_dtype) -> torch.Tensor:
+                nw: torch.Tensor, eps: float, out_dtype, tables=None) -> torch.Tensor:
     """Every stream of ``x`` becomes ``embed[ids] * scale``; returns the first sublayer's input
-    ``rms(sum_s inn[s] x_s) * nw`` as activations (same pass)."""
+    ``rms(sum_s inn[s] x_s) * nw`` as activations (same pass).  ``tables`` (:class:`..ops.seq_ops.RopeTables`): filled in the
+    same launch."""
     T, S, W = x.shape
     if use_hip(embed):
         assert x.dtype == torch.float32 and x.is_contiguous() and embed.is_contiguous() and embed.shape[1] == W
@@ -347,8 +355,11 @@ def hyper_embed(ids: torch.Tensor, embed: torch.Tensor, scale: float, x: torch.T
         assert inn.numel() == S and nw.numel() == W
         h = torch.empty(T, W, dtype=out_dtype, device=embed.device)
         check(lib().k8s_hyper_embed(ptr(ids), ptr(embed), _odt(embed.dtype), float(scale), ptr(x), S, ptr(inn), ptr(nw),
-                                    float(eps), ptr(h), _odt(out_dtype), T, W, stream_ptr(embed)), "hyper_embed")
+                                    float(eps), ptr(h), _odt(out_dtype), T, W, stream_ptr(embed), *_tables(tables)),
+              "hyper_embed")
         return h
+    if tables is not None:
+        tables.fill()
     x.copy_((embed[ids.long()].float() * scale)[:, None].expand(T, S, W))
     return _rms_rows(torch.einsum("s,tsw->tw", inn, x), nw, eps, out_dtype)
 

@@ -1094,6 +1094,35 @@ def rope_table(positions: torch.Tensor, rope: Rope) -> torch.Tensor:
     return torch.cat([ang.cos().float(), ang.sin().float()], 1) * rope.amp
 
 
+class RopeTables:
+    """:func:`rope_table` of a step's rotations: tensors that the launch which embeds the step's tokens fills
+    (:func:`.norm.hyper_embed`, :func:`.norm.embed_scale_dyt`: up to two of them), and further ones, filled at once."""
+    IN_EMBED = 2
+
+    def __init__(self, positions: torch.Tensor, ropes):
+        self.positions, self.ropes = positions, list(ropes)[:self.IN_EMBED]
+        self.cs = [torch.empty(positions.shape[0], r.dims, dtype=torch.float32, device=positions.device) for r in self.ropes]
+        self._of = {id(r): cs for r, cs in zip(self.ropes, self.cs)}
+        for r in list(ropes)[self.IN_EMBED:]:
+            self._of[id(r)] = rope_table(positions, r)
+
+    def of(self, rope: Optional[Rope]) -> Optional[torch.Tensor]:
+        return None if rope is None else self._of[id(rope)]
+
+    def fill(self) -> None:
+        for r, cs in zip(self.ropes, self.cs):
+            cs.copy_(rope_table(self.positions, r))
+
+    def args(self) -> tuple:
+        """What the launch takes."""
+        assert self.positions.dtype == torch.int32 and self.positions.is_contiguous()
+        out = [ptr(self.positions)]
+        for r, cs in zip(self.ropes, self.cs):
+            assert r.freq.dtype == torch.float64 and r.freq.device == self.positions.device
+            out += [ptr(r.freq), float(r.amp), r.dims // 2, ptr(cs)]
+        return tuple(out + [0, 0.0, 0, 0] * (self.IN_EMBED - len(self.ropes)))
+
+
 def attn_prep(qkv: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D: int, V: int,
               positions: torch.Tensor, slots: torch.Tensor, kc: Optional[torch.Tensor], vc: Optional[torch.Tensor],
               out_dtype, norm=False, q_w: Optional[torch.Tensor] = None, k_w: Optional[torch.Tensor] = None,
