@@ -32,7 +32,7 @@ import torch
 from ..ops import norm as N
 from ..ops import row_step as R
 from ..ops import seq_ops as S
-from ..ops.linear import proj, proj_add, proj_planes
+from ..ops.linear import proj_add, proj_planes
 from ..parallel.groups import ParallelContext, single
 
 TAIL_ALIGN = 32     # the rotated key part of a latent cache row is filled up to a multiple of this
@@ -388,9 +388,8 @@ class FikeraxModel:
         T, H, D, V, KR = inp.input_ids.shape[0], c.heads, c.dim, c.vdim, c.kv_rank
         cs = tables.of(self.ropes[i])
         dn = R.proj_planes(h, L["w_in"])                                      # [., T, q_rank + KR + rot_dim] fp32
-        cq = S.latent_norm(dn, L["dq_norm"], L["dkv_norm"], inp.slots, cache, c.q_rank, KR, self.cfg.norm_eps, self.dtype,
-                           cache_t=cache_t, tail=c.rot_dim, tail_cs=cs)
-        q = proj(cq, L["w_uq"])                                             # [T, H (D + rot_dim)]
+        q = S.latent_up(dn, L["dq_norm"], L["dkv_norm"], L["w_uq"], inp.slots, cache, c.q_rank, KR, self.cfg.norm_eps,
+                        self.dtype, cache_t=cache_t, tail=c.rot_dim, tail_cs=cs)      # [T, H (D + rot_dim)]
         qa, qr = S.latent_queries(q, L["uk"], cs, H, D, c.tail)               # [T, H, KR] head-major, [T, H, tail]
         kw = dict(window=c.window, sink=L["sink"], head_major=True)
         if cache_t is not None:

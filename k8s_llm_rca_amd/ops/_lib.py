@@ -109,6 +109,7 @@ _SIGS = {
     "k8s_mingru_chunked": [P, P, P, P, P, I, P, P, P, P, P, P, I, I, P],
     "k8s_postnorm": [P, P, I, P, I, P, I, I, F, F, P],
     "k8s_latent_norm": [P, I, P, P, P, P, P, P, I, I, I, I, F, I, P, I, I, P, I, L],
+    "k8s_latent_step": [P, I, I, L, P, P, P, P, P, P, P, I, I, I, I, I, F, I, I, P, P],
     "k8s_rotated_tail": [P, P, P, I, I, I, I, I, I, P],
     "k8s_latent_attn_mfma_ok": [I, I],
     "k8s_latent_attn_mfma": [P, P, P, P, I, P, I, P, I, P, I, I, I, F, P, L, L, P, I, L, L, I, P],

@@ -373,6 +373,46 @@ def _turn_pairs(x: torch.Tensor, cs: torch.Tensor) -> torch.Tensor:
     return torch.stack([a * co - b * si, b * co + a * si], -1).flatten(-2)
 
 
+LATENT_STEP_RANKS, LATENT_STEP_ROWS, LATENT_STEP_READ = (256, 512, 768, 1024, 1536, 2048), 16, 56 << 20
+
+
+def latent_up(dn: torch.Tensor, wq: torch.Tensor, wkv: torch.Tensor, w: torch.Tensor, slots: torch.Tensor,
+              cache: torch.Tensor, q_rank: int, kv_rank: int, eps: float, out_dtype, cache_t: Optional[torch.Tensor] = None,
+              tail: int = 0, tail_cs: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """:func:`latent_norm`, then its result ``@ w.T``.
+
+    Up to 16 rows in one launch (csrc/kernels/latent_step.hip), every strip of 16 columns of which reads all rows: the line
+    is what all strips read.  us of two launches / one at 1, 7, 16 rows, two planes:  768 + 256 + 64 numbers, 3072 columns
+    7.5 / 3.6, 7.9 / 4.1, 8.1 / 4.8;  1536 + 512 + 64, 3072 8.1 / 4.9, 8.5 / 5.7, 9.2 / 6.7;  1024 + 256 + 64, 8192 8.7 / 6.1,
+    8.6 / 7.5, 9.0 / 9.0;  2048 + 512 + 64, 6144 at 1, 4, 7 10.8 / 9.7, 11.3 / 10.5, 11.4 / 11.9;  1536 + 512 + 64, 24576 17.8 /
+    20.9, 18.7 / 25.7, 20.3 / 31.1."""
+    from .linear import dispatch_table, proj
+    T, N = dn.shape[-2], w.shape[0]
+    if 0 < T <= LATENT_STEP_ROWS and use_hip(dn):      # (before anything else: prompts pay for one comparison)
+        planes, pstep = (dn.shape[0], dn.stride(0)) if dn.dim() == 3 else (1, 0)
+        pad = cache.shape[-1] - kv_rank
+        small = ((wq, q_rank, out_dtype), (wkv, kv_rank, out_dtype), (tail_cs if tail else None, T * tail, torch.float32))
+        if (out_dtype == torch.bfloat16 == w.dtype and q_rank in LATENT_STEP_RANKS and planes in (1, 2, 4)
+                and N // 16 * q_rank * (32 + 4 * T * planes) <= LATENT_STEP_READ
+                and q_rank * planes <= 4096 and N > 0 and N % 16 == 0 and kv_rank + tail <= 2048 and (kv_rank + tail) % 4 == 0
+                and tail % 2 == 0 and pad >= tail and pad % 2 == 0 and dn.dtype == torch.float32 and dn.stride(-1) == 1
+                and dn.shape[-1] >= q_rank + kv_rank + tail and dn.stride(-2) % 4 == 0 and pstep % 4 == 0
+                and dn.stride(-2) >= q_rank + kv_rank + tail and dn.data_ptr() % 16 == 0 == w.data_ptr() % 16
+                and w.shape[1] == q_rank and w.is_contiguous() and w.device == dn.device and (N, q_rank) not in dispatch_table()
+                and all(t is None or t.dtype == d and t.is_contiguous() and t.numel() == n for t, n, d in small)
+                and wq.data_ptr() % 8 == 0 and slots.dtype == torch.int32 and slots.is_contiguous() and slots.numel() >= T
+                and (not tail or tail_cs is not None)
+                and all(t is None or t.is_contiguous() and t.dtype == out_dtype for t in (cache, cache_t))
+                and (cache_t is None or cache_t.shape[1:] == (kv_rank, cache.shape[1]))):
+            q = torch.empty(T, N, dtype=out_dtype, device=dn.device)
+            check(lib().k8s_latent_step(ptr(dn), dn.stride(-2), planes, pstep, ptr(wq), ptr(wkv), ptr(w), ptr(q), ptr(slots),
+                                        ptr(cache), ptr(cache_t), cache.shape[1], T, N, q_rank, kv_rank, float(eps), tail, pad,
+                                        ptr(tail_cs) if tail else 0, stream_ptr(dn)), "latent_step")
+            return q
+    cq = latent_norm(dn, wq, wkv, slots, cache, q_rank, kv_rank, eps, out_dtype, cache_t=cache_t, tail=tail, tail_cs=tail_cs)
+    return proj(cq, w)
+
+
 def rotated_tail(q: torch.Tensor, cs: torch.Tensor, H: int, N: int, pad: int) -> torch.Tensor:
     """The entries behind the first ``N`` of every head of ``q`` [T, H (N + R)], neighbours 2i, 2i + 1 turned by ``cs``
     [T, R] (a :func:`rope_table`), filled up with zeros to ``pad``: [T, H, pad]."""
