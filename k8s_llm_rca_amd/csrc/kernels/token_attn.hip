@@ -364,8 +364,14 @@ struct MaskTokArgs {
 // of workgroups.  Every workgroup prepares its own heads' queries; the one whose part ends with the row's position also its
 // key and value, which it writes to the pages and puts into the fragments of its last block itself.  The row is asked for in
 // front of the pages and keys, which are on their way while it is prepared.  The arithmetic, and every bit, is the pass's.
-template <int NDC, int NV, bool CAP, int NW, bool TURN, bool PREP>
-__global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs a) {
+//
+// ONE: no wave has more than one block (a part has at most as many blocks as there are waves, and no row more parts than the
+// launch: n_parts < most).  One block's registers instead of two's (104 for 250) let a second workgroup onto the compute unit,
+// which otherwise waits out each one's chain.  us before / this, with the preparation and the merge, 16 heads over 2 of 128:
+// 1 row at 100 keys 7.0 / 6.7, 64 at 512 15.8 / 15.7, 64 at 1500 32.5 / 27.5, 200 at 900 62.7 / 49.0;  32 over 8 of 128, 7 at
+// 1500 23.0 / 19.3, 64 at 512 45.3 / 36.7;  12 over 3 of 64 + 128, 64 at 512 20.6 / 17.4.
+template <int NDC, int NV, bool CAP, int NW, bool TURN, bool PREP, bool ONE>
+__global__ void __launch_bounds__(64 * NW, ONE ? 4 : 1) masked_attn_token_kernel(MaskTokArgs a) {
   constexpr int D = NDC * 32, V = NV * 16;
   __shared__ TokLds<NW, V> lds;
   __shared__ __attribute__((aligned(16))) uint16_t qs[PREP ? 16 * D : 8], ks[PREP ? D : 8], vs[PREP ? V : 8];
@@ -427,23 +433,35 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
   };
   fill(0);
   const int lr = TURN ? lane >> 2 : r, lh = TURN ? lane & 3 : hq, from = 4 * (4 * r + hq);
-  bf16x8 kf[2][2][NDC], vf[2][NV];
-  int kb[2];
-  auto load = [&](int u, int k) {
-    if (k - base == 64) fill(k);
+  constexpr int U = ONE ? 1 : 2;      // blocks of a wave in flight
+  bf16x8 kf[U][2][NDC], vf[U][NV];
+  int kb[U], page = 0, off = 0;
+  auto load_k = [&](int u, int k) {
+    if (!ONE && k - base == 64) fill(k);
     kb[u] = __shfl(kbv, k - base, 64);
-    const int page = __shfl(pgv, k - base, 64), off = __shfl(ofv, k - base, 64);
+    page = __shfl(pgv, k - base, 64), off = __shfl(ofv, k - base, 64);
     const uint16_t* kp = a.kc + ((size_t)page * a.BS + off) * NK + g * D + 8 * lh;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int cc = 0; cc < NDC; ++cc) kf[u][t][cc] = tld16(kp + (size_t)(8 * (lr >> 2) + 4 * t + (lr & 3)) * NK + 32 * cc);
+  };
+  auto load_v = [&](int u) {
     const uint16_t* vp = a.vt + ((size_t)page * NVt + (size_t)gv * V) * a.BS + off + 8 * lh;
 #pragma unroll
     for (int dt = 0; dt < NV; ++dt) vf[u][dt] = tld16(vp + (size_t)(16 * dt + lr) * a.BS);
   };
-  if (my > 0) load(0, 0);
-  if (my > 1) load(1, 1);
+  auto load = [&](int u, int k) {
+    load_k(u, k);
+    load_v(u);
+  };
+  if constexpr (ONE) {
+    if (my > 0) load_k(0, 0);
+    if (!PREP && my > 0) load_v(0);
+  } else {
+    if (my > 0) load(0, 0);
+    if (my > 1) load(1, 1);
+  }
   if constexpr (PREP) {
     if (heads) {
       u16x4 ha, hb;
@@ -467,6 +485,7 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
         if (a.p.vc) *reinterpret_cast<u16x4*>(a.p.vc + (size_t)sl * NVt + c) = v;
       }
     }
+    if (ONE && my > 0) load_v(0);
     step_barrier_lds();
 #pragma unroll
     for (int cc = 0; cc < NDC; ++cc) qf[cc] = *reinterpret_cast<const bf16x8*>(qs + min(r, nh - 1) * D + 32 * cc + 8 * hq);
@@ -491,9 +510,9 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
     }
   };
   const int cq_lo = a.chunk > 0 ? (pos / a.chunk) * a.chunk : 0, wq_lo = a.window > 0 ? pos - a.window + 1 : 0;
-  for (int k = 0; k < my; k += 2) {
+  for (int k = 0; k < my; k += ONE ? my : 2) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       if (k + u >= my) break;
       own(u);
       float p[8];
@@ -522,7 +541,7 @@ __global__ void __launch_bounds__(64 * NW) masked_attn_token_kernel(MaskTokArgs 
 #pragma unroll
       for (int dt = 0; dt < NV; ++dt)
         o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, tok_turn<TURN>(vf[u][dt], from), o[dt], 0, 0, 0);
-      if (k + u + 2 < my) load(u, k + u + 2);
+      if (!ONE && k + u + 2 < my) load(u, k + u + 2);
     }
   }
   l += __shfl_xor(l, 16, 64);
@@ -545,9 +564,12 @@ struct LatTokArgs {
 };
 
 // grid (rows, parts, groups of 16 heads); parts are ranges of the key index (a row's first one is that of its first
-// visible key).
-template <int NR, int NP, int NW, bool TURN>
-__global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a) {
+// visible key).  ONE as above, for R from 192 on: R 256 + 64, 16 heads, 1 row at 20 keys 5.9 / 5.5 us, 64 rows at 512 14.9 /
+// 15.2, at 1500 35.3 / 31.4, 200 at 900 67.9 / 57.0;  R 512 + 64 1 row at 100 12.3 / 11.3, 64 at 512 24.9 / 24.2;  below, where
+// the registers let several workgroups on anyway, R 128 + 32 7 rows at 700 9.2 / 9.6.  (All values asked for in front of the
+// scores: 7 rows at 700 11.2 / 11.4.)
+template <int NR, int NP, int NW, bool TURN, bool ONE>
+__global__ void __launch_bounds__(64 * NW, ONE ? 2 : 1) latent_attn_token_kernel(LatTokArgs a) {
   constexpr int R = NR * 32, ND = R / 16, NC = NR + NP, RW = R + 32 * NP, NH = ND / 2;
   __shared__ TokLds<NW, R> lds;
   const int lane = threadIdx.x & 63, r = lane & 15, hq = lane >> 4;
@@ -574,7 +596,7 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
   for (int dt = 0; dt < ND; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int* pages = a.bt + (size_t)sg * a.maxb;
   const int lr = TURN ? lane >> 2 : r, lh = TURN ? lane & 3 : hq, from = 4 * (4 * r + hq);
-  for (int b = wv; b < nb; b += NW) {
+  for (int b = wv; b < nb; b += ONE ? nb : NW) {
     const int kb = kb0 + 32 * b, page = pages[kb / a.BS], off = kb % a.BS;
     const uint16_t* cp = a.c + (size_t)page * a.BS * RW;
     const uint16_t* tp = a.ct + (size_t)page * R * a.BS + (size_t)lr * a.BS + off + 8 * lh;
@@ -613,16 +635,16 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_token_kernel(LatTokArgs a
   tok_join<NW, ND>(lds, a.t, row, head0, nh, blockIdx.y, m, l, o);
 }
 
-template <int NDC, int NV, int NW, bool PREP>
+template <int NDC, int NV, int NW, bool PREP, bool ONE>
 static int launch_mask_tok_nw(const MaskTokArgs& a, int rows, hipStream_t s) {
   const int hpg = a.t.H / (a.G * a.t.hs);
   const dim3 grid(rows, a.G * a.t.hs * ((hpg + 15) / 16), a.t.n_parts);
-  auto k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, false, PREP>
-                           : masked_attn_token_kernel<NDC, NV, false, NW, false, PREP>;
+  auto k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, false, PREP, ONE>
+                           : masked_attn_token_kernel<NDC, NV, false, NW, false, PREP, ONE>;
   if constexpr (NV == 2 * NDC && (NDC == 2 || NW == 8))      // keys as long as values, heads that share keys or are of 64
     if ((long)rows * grid.y * grid.z <= kTurnMasked)
-      k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, true, PREP>
-                          : masked_attn_token_kernel<NDC, NV, false, NW, true, PREP>;
+      k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, true, PREP, ONE>
+                          : masked_attn_token_kernel<NDC, NV, false, NW, true, PREP, ONE>;
   hipLaunchKernelGGL(k, grid, dim3(64 * NW), 0, s, a);
   if (a.t.n_parts > 1)
     hipLaunchKernelGGL(token_merge_kernel, dim3(rows * a.t.H), dim3(256), 0, s, a.t, a.items, NV * 16);
@@ -638,10 +660,12 @@ static int launch_mask_tok_nw(const MaskTokArgs& a, int rows, hipStream_t s) {
 template <int NDC, int NV, bool PREP>
 static int launch_mask_tok_as(const MaskTokArgs& a, int rows, hipStream_t s) {
   if constexpr (NDC == 2 && NV == 4)
-    return launch_mask_tok_nw<NDC, NV, 4, PREP>(a, rows, s);
+    return launch_mask_tok_nw<NDC, NV, 4, PREP, false>(a, rows, s);
+  else if (a.t.H == a.G * a.t.hs)
+    return launch_mask_tok_nw<NDC, NV, 2, PREP, false>(a, rows, s);
   else
-    return a.t.H > a.G * a.t.hs ? launch_mask_tok_nw<NDC, NV, 8, PREP>(a, rows, s)
-                                : launch_mask_tok_nw<NDC, NV, 2, PREP>(a, rows, s);
+    return a.t.n_parts < a.most && a.part_blocks <= 8 ? launch_mask_tok_nw<NDC, NV, 8, PREP, true>(a, rows, s)
+                                                      : launch_mask_tok_nw<NDC, NV, 8, PREP, false>(a, rows, s);
 }
 template <int NDC, int NV>
 static int launch_mask_tok(const MaskTokArgs& a, int rows, hipStream_t s) {
@@ -662,9 +686,14 @@ template <int NR, int NP>
 static void launch_lat_tok_np(const LatTokArgs& a, int rows, hipStream_t s) {
   constexpr int NW = 4;
   const dim3 grid(rows, a.t.n_parts, (a.t.H + 15) / 16);
-  auto k = latent_attn_token_kernel<NR, NP, NW, false>;
-  if constexpr (NR >= 6)
-    if ((long)rows * grid.y * grid.z <= (NR > 8 ? kTurnLong : kTurnLatent)) k = latent_attn_token_kernel<NR, NP, NW, true>;
+  auto k = latent_attn_token_kernel<NR, NP, NW, false, false>;
+  if constexpr (NR >= 6) {
+    const bool one = a.t.n_parts < a.most && a.part <= 32 * NW;
+    if ((long)rows * grid.y * grid.z <= (NR > 8 ? kTurnLong : kTurnLatent))
+      k = one ? latent_attn_token_kernel<NR, NP, NW, true, true> : latent_attn_token_kernel<NR, NP, NW, true, false>;
+    else if (one)
+      k = latent_attn_token_kernel<NR, NP, NW, false, true>;
+  }
   hipLaunchKernelGGL(k, grid, dim3(64 * NW), 0, s, a);
 }
 
