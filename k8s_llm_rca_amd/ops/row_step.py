@@ -149,6 +149,7 @@ def dyt_step(x: torch.Tensor, y: Optional[torch.Tensor], sy: float, y2: Optional
 
 
 # ------------------------------------ a sublayer's last product with the residual's pass in its epilogue (gemm_step.hip)
+INTO_F32_ROWS = 4
 INTO_ROWS, INTO_LOADS, INTO_STRIP, PARTS = 16, (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16), 8, 256
 
 
@@ -187,6 +188,8 @@ class Scaled:
         return Scaled(*(t.index_select(0, idx) for t in (self.x, self.h, self.part)), self.nw, self.eps)
 
     def product(self, w: torch.Tensor, out_kind: int, plain, planes: bool = False, keep: bool = False):
+        if self.h.dtype == torch.float32:
+            return self._product_f32(w, out_kind, plain, planes)
         (m, k), n = self.h.shape, w.shape[0] // (2 if out_kind == L.ROWS_SILU else 1)
         if (out_kind == L.ROWS_RELU2 or keep or k != w.shape[1] or w.shape[0] % 2 and out_kind == L.ROWS_SILU
                 or not L.rows_ok(self.h, w) or (("silu", w.shape[0], k) in L.dispatch_table()) or (n, k) in L.dispatch_table()):
@@ -200,10 +203,32 @@ class Scaled:
                                          self.part.shape[1], float(k), float(self.eps), stream_ptr(w)), "gemm_rows_scaled")
         return out
 
+    def _product_f32(self, w: torch.Tensor, out_kind: int, plain, planes: bool):
+        glu = out_kind == L.ROWS_SILU
+        if out_kind == L.ROWS_RELU2 or glu and w.shape[0] % 2 or not L._few_f32_ok(self.h, w):
+            return plain(self.read(), w)
+        (m, k), n = self.h.shape, w.shape[0] // (2 if glu else 1)
+        out = torch.empty((1, m, n) if planes else (m, n), dtype=torch.float32, device=w.device)
+        check(lib().k8s_few_rows_f32_scaled(ptr(self.h), k, ptr(w), ptr(out), m, n, k, int(glu), ptr(self.part), float(self.eps),
+                                            stream_ptr(w)), "few_rows_f32_scaled")
+        return out
+
 
 def _into_operands(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, out_dtype) -> bool:
     return (a.is_cuda and out_dtype == torch.bfloat16 and x.dtype == torch.float32 and x.is_contiguous()
             and w.shape == (x.shape[-1], a.shape[1]) and w.device == x.device == a.device and L.rows_ok(a, w))
+
+
+def _into_f32(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:
+    """The same of fp32 operands (csrc/kernels/few_rows_f32.hip).
+
+    Up to four rows, whose sums of squares the product behind reads with a wave each.  us of product, pass and product / of the
+    two at 1, 2, 4 and, with two rows a wave, 5, 8 rows:  2048 x 2048, gated 16384 x 2048 28.9 / 27.3, 30.8 / 29.6, 35.1 / 33.9, 37.4 /
+    42.9, 48.1 / 46.5;  2048 x 8192, 8192 x 2048 27.7 / 25.3, 28.9 / 25.5, 31.7 / 29.9, 34.4 / 36.0, 36.7 / 36.3;  512 x 2048, 1536 x
+    512 9.5 / 7.8, 9.9 / 8.1, 10.8 / 9.1, 11.9 / 10.0, 12.3 / 10.5;  4096 x 4096, 8192 x 4096 37.5 / 35.1, 40.0 / 38.3, 44.9 / 42.2,
+    47.7 / 49.4, 52.9 / 53.1."""
+    return (a.shape[0] <= INTO_F32_ROWS and L._few_f32_ok(a, w) and x.dtype == torch.float32 and x.is_contiguous() and w.shape[0] == x.shape[-1]
+            and w.device == x.device == a.device and w.shape[0] % 16 == 0 and w.shape[0] <= 4096)
 
 
 def add_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, one: torch.Tensor, mix: torch.Tensor, nw: torch.Tensor,
@@ -227,18 +252,21 @@ def _rms_into(x, a, w, nw, eps, out_dtype, again, rms) -> Optional[Scaled]:
     (m, k), W = a.shape, x.shape[-1]
     ids, embed, escale = again if again is not None else (None, None, 0.0)
     ss, width, reps = rms if rms is not None else (None, 1.0, 0.0)
-    if not (into_ok(m, W, k) and _into_operands(x, a, w, out_dtype) and x.shape[:2] == (m, 1) and W % 32 == 0
-            and W // INTO_STRIP <= PARTS and _fp32_row(nw, W)
+    f32 = out_dtype == torch.float32
+    fits = (_into_f32(x, a, w) if f32 else into_ok(m, W, k) and _into_operands(x, a, w, out_dtype) and W % 32 == 0
+            and W // INTO_STRIP <= PARTS)
+    if not (fits and x.shape[:2] == (m, 1) and _fp32_row(nw, W)
             and (ss is None or ss.dtype == torch.float32 and ss.is_contiguous() and ss.shape[0] == m
                  and 0 < ss.numel() <= SUMS * m)
             and (ids is None or ids.dtype == torch.int32 and ids.is_contiguous() and ids.numel() == m
                  and embed.dtype == out_dtype and embed.is_contiguous() and embed.shape[1] == W)):
         return None
     h = torch.empty(m, W, dtype=out_dtype, device=x.device)
-    part = torch.empty(m, W // INTO_STRIP, dtype=torch.float32, device=x.device)
-    check(lib().k8s_gemm_step_rms(ptr(a), a.stride(0), ptr(w), ptr(x), ptr(ss), ss.numel() // m if ss is not None else 0,
-                                  float(width), float(reps), ptr(ids), ptr(embed), float(escale), ptr(nw), ptr(h), ptr(part),
-                                  m, W, k, stream_ptr(x)), "gemm_step_rms")
+    part = torch.empty(m, W // (4 if f32 else INTO_STRIP), dtype=torch.float32, device=x.device)
+    launch = lib().k8s_few_rows_f32_add if f32 else lib().k8s_gemm_step_rms
+    check(launch(ptr(a), a.stride(0), ptr(w), ptr(x), ptr(ss), ss.numel() // m if ss is not None else 0,
+                 float(width), float(reps), ptr(ids), ptr(embed), float(escale), ptr(nw), ptr(h), ptr(part), m, W, k,
+                 stream_ptr(x)), "gemm_step_rms")
     return Scaled(x, h, part, nw, eps)
 
 
