@@ -38,7 +38,7 @@ struct StepArgs {
   int wh;
   float eps, unit_eps, den_eps;
   void* out;              // [T][H V]
-  float* ssp;             // KIND 2: [T][H]
+  float* ssp;             // KIND 2: [T][H][slices]
   int H, G, V;
   const float* lr;        // LOW: rows of stride bs, ra entries for the decays' gates, rg for the output's
   const uint16_t* la;     // LOW: [H D][ra]
@@ -98,7 +98,7 @@ __global__ void __launch_bounds__(256) state_step_kernel(StepArgs a) {
   __shared__ f32x4 red[2][4][LV];
   static_assert(D <= 256, "a thread per entry of q and k");
   const int it = blockIdx.x, hh = blockIdx.y, tid = threadIdx.x, lv = tid % LV, rg = tid / LV, wv = tid >> 6;
-  const int H = a.H, V = a.V, c = 4 * lv;
+  const int H = a.H, V = a.V, c = 4 * (KIND == 2 ? blockIdx.z * LV + lv : lv);
   const TA* row = (const TA*)a.x + (size_t)it * a.xs;
   const int slot = a.slot[it];
   const bool fresh = a.pos0[it] == 0;
@@ -256,21 +256,26 @@ __global__ void __launch_bounds__(256) state_step_kernel(StepArgs a) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc[j] = acc[j] * rn * w[j] * sigmoid_f(gt[j]);
   ss_st4((TO*)a.out + (size_t)it * H * V + hh * V + c, acc);
-  if (KIND == 2 && tid == 0) a.ssp[(size_t)it * H + hh] = ss;
+  if (KIND == 2 && tid == 0) a.ssp[((size_t)it * H + hh) * gridDim.z + blockIdx.z] = ss;
 }
 
 template <int KIND, typename TA, typename TO, typename TG, bool LOW = false>
-static int launch_step(const StepArgs& a, int n, int D, hipStream_t s) {
-  const dim3 grid(n, a.H);
+static int launch_step(const StepArgs& a, int n, int D, hipStream_t s, int slices = 1) {
+  const dim3 grid(n, a.H, slices);
+  const int V = a.V / slices;      // of a workgroup
 #define K8S_ST(LV, DR) hipLaunchKernelGGL((state_step_kernel<KIND, LV, DR, TA, TO, TG, LOW>), grid, dim3(256), 0, s, a)
-  if (a.V == 128 && D == 128)
+  if (V == 128 && D == 128)
     K8S_ST(32, 16);
-  else if (a.V == 128 && D == 64)
+  else if (V == 128 && D == 64)
     K8S_ST(32, 8);
-  else if (a.V == 64 && D == 128)
+  else if (V == 64 && D == 128)
     K8S_ST(16, 8);
-  else if (a.V == 64 && D == 64)
+  else if (V == 64 && D == 64)
     K8S_ST(16, 4);
+  else if (KIND == 2 && V == 32 && D == 128)
+    K8S_ST(8, 4);
+  else if (KIND == 2 && V == 32 && D == 64)
+    K8S_ST(8, 2);
   else
     return (int)hipErrorInvalidValue;
 #undef K8S_ST
@@ -322,14 +327,15 @@ K8S_API int k8s_memory_step(const float* x, int xs, const float* gate_bias, floa
   return odt == 0 ? launch_step<1, float, uint16_t, float>(p, n, D, s) : launch_step<1, float, float, float>(p, n, D, s);
 }
 
-// ssp [n][H]
+// ssp [n][H][slices]; slices: workgroups of a head, 1, 2 or 4 (32 columns or more each)
 K8S_API int k8s_decay_step(const void* x, int xs, int dt, const float* decay, float* state, const int* pos0, const int* slot,
                            const void* gate, int gs, const float* w, void* out, float* ssp, int n, int H, int D, int V,
-                           hipStream_t s) {
+                           hipStream_t s, int slices) {
   if (n <= 0) return 0;
+  if (slices < 1 || V % slices) return (int)hipErrorInvalidValue;
   StepArgs p{};
   p.x = x; p.xs = xs; p.rate = decay; p.state = state; p.pos0 = pos0; p.slot = slot; p.gate = gate; p.gs = gs; p.w = w;
   p.wh = V; p.out = out; p.ssp = ssp; p.H = H; p.G = H; p.V = V;
-  return dt == 0 ? launch_step<2, uint16_t, uint16_t, uint16_t>(p, n, D, s)
-                 : launch_step<2, float, float, float>(p, n, D, s);
+  return dt == 0 ? launch_step<2, uint16_t, uint16_t, uint16_t>(p, n, D, s, slices)
+                 : launch_step<2, float, float, float>(p, n, D, s, slices);
 }

@@ -119,7 +119,7 @@ _SIGS = {
     "k8s_delta_step": [P, I, P, P, P, P, I, P, P, P, P, I, P, I, P, I, I, I, I, I, F, F, P],
     "k8s_delta_step_low": [P, P, I, I, I, P, P, P, P, P, P, P, P, I, P, I, I, I, I, I, F, F, P],
     "k8s_memory_step": [P, I, P, F, P, P, P, P, P, P, I, P, I, P, I, I, I, I, I, F, F, P],
-    "k8s_decay_step": [P, I, I, P, P, P, P, P, I, P, P, P, I, I, I, I, P],
+    "k8s_decay_step": [P, I, I, P, P, P, P, P, I, P, P, P, I, I, I, I, P, I],
     "k8s_head_proj": [P, L, L, P, P, L, L, I, I, I, I, P, P, I, I, I, P],
     "k8s_low_rank_pair": [P, I, I, I, I, P, I, P, I, I, P, I, P, P],
     "k8s_masked_attn_prompt": [P, P, P, P, I, P, I, P, P, I, P, I, I, I, I, I, I, I, I, F, F, P, I, I, I, I, I, I, P, P],

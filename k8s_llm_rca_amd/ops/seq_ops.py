@@ -1852,10 +1852,19 @@ def memory_layer(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tenso
     return head_norm_gate(o, gate, w, H, V, eps, out_dtype, mul=mul)
 
 
+def decay_slices(T: int, H: int, V: int) -> int:
+    """Workgroups of a head in :func:`decay_layer`'s steps of ``T`` single tokens: four of 32 columns while half of the compute
+    units would have none.  A unit takes a state in and gives it back at some 40 KB a us.  us with 1 / 2 / 4 of them, 16 heads
+    of 128 x 128 at 1, 4, 7, 16, 32 tokens 4.4 / 4.0 / 3.8, 5.0 / 4.5 / 4.4, 5.9 / 5.5 / 5.6, 8.4 / 8.6 / 8.3, 13.5 / 15.3 / 15.1;  8
+    of them at 7, 16 4.9 / 4.5 / 4.3, 6.1 / 5.8 / 5.9;  16 of 64 x 128 at 1, 7 3.9 / 3.8 / 3.7, 4.4 / 4.2 / 4.3;  32 of 64 x 64 at 1,
+    7 3.8 / 3.7, 4.2 / 4.3."""
+    return 4 if V == 128 and T * H <= 128 and 4 * H <= 64 else 1      # (64 sums of squares a row: what the products behind take)
+
+
 def decay_layer(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor, state: torch.Tensor, seg: SegMeta,
                 gate: torch.Tensor, w: torch.Tensor, eps: float, out_dtype) -> tuple:
     """:func:`decay_attention` with silu, then one norm over all heads, its weight and the gates: (y, None), or for steps of
-    single tokens (y without the division by the row's root mean square, (sums of squares [T, H], H V, eps)), which
+    single tokens (y without the division by the row's root mean square, (sums of squares [T, .], H V, eps)), which
     :func:`.norm.hyper_step` makes up for behind the output projection."""
     if (_step_ok(x, seg, D, V, state, gate, w) and gate.dtype == x.dtype == out_dtype and w.numel() == H * V):
         T = x.shape[0]
@@ -1863,10 +1872,11 @@ def decay_layer(x: torch.Tensor, H: int, D: int, V: int, decay: torch.Tensor, st
         assert decay.dtype == torch.float32 and decay.numel() == H
         assert state.is_contiguous() and state.dtype == torch.float32 and state.shape[1:] == (H, D, V)
         out = torch.empty(T, H * V, dtype=out_dtype, device=x.device)
-        ss = torch.empty(T, H, dtype=torch.float32, device=x.device)
+        slices = decay_slices(T, H, V)
+        ss = torch.empty(T, H * slices, dtype=torch.float32, device=x.device)
         check(lib().k8s_decay_step(ptr(x), x.stride(0), _dt(x.dtype), ptr(decay), ptr(state), ptr(seg.seg_pos0),
                                    ptr(seg.seg_slot), ptr(gate), gate.stride(0), ptr(w), ptr(out), ptr(ss), T, H, D, V,
-                                   stream_ptr(x)), "decay_step")
+                                   stream_ptr(x), slices), "decay_step")
         return out, (ss, H * V, eps)
     o = decay_attention(x, H, D, V, decay, state, seg, silu=True)
     return head_norm_gate(o, gate, w, 1, H * V, eps, out_dtype), None
