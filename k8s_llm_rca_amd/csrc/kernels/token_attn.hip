@@ -16,6 +16,7 @@
 // keys 5.3 / 8.5 (8.4 / 13.5), 8 rows at 1500 10.7 / 12.5 (26 / 36), 64 rows at 400 12.3 / 14.3 (28 / 35).
 #include "common.h"
 #include "key_runs.h"
+#include "state_step.h"
 
 namespace k8s {
 
@@ -370,11 +371,39 @@ struct MaskTokArgs {
 // which otherwise waits out each one's chain.  us before / this, with the preparation and the merge, 16 heads over 2 of 128:
 // 1 row at 100 keys 7.0 / 6.7, 64 at 512 15.8 / 15.7, 64 at 1500 32.5 / 27.5, 200 at 900 62.7 / 49.0;  32 over 8 of 128, 7 at
 // 1500 23.0 / 19.3, 64 at 512 45.3 / 36.7;  12 over 3 of 64 + 128, 64 at 512 20.6 / 17.4.
-template <int NDC, int NV, bool CAP, int NW, bool TURN, bool PREP, bool ONE>
-__global__ void __launch_bounds__(64 * NW, ONE ? 4 : 1) masked_attn_token_kernel(MaskTokArgs a) {
+//
+// MEM: workgroups behind the attention's (grid z from n_parts on, two heads each) take the matrix memory of the same rows
+// (state_step.h), which a layer has beside it: neither waits for the other, and each alone leaves most of the chip idle.
+// us of both launches / of this, 16 heads over 2 of 128 beside 16 of 64 x 128: 1 row at 100 keys 11.1 / 7.1, 5 at 1100 15.9 / 11.8, 64
+// at 450 34.7 / 31.5.
+struct NoMemory {
+  struct Args {};
+  static constexpr bool on = false;
+  struct Lds {};
+};
+template <int LV, int DR>
+struct WithMemory {
+  using Args = StepArgs;
+  static constexpr bool on = true;
+  using Lds = StepLds<1, LV, DR, false>;
+  static __device__ __forceinline__ void run(const StepArgs& m, int z, Lds (&lds)[2]) {
+    const int h0 = 2 * (z * gridDim.y + blockIdx.y), half = threadIdx.x >> 8, h = h0 + half;
+    if (h0 >= m.H) return;                                 // (the whole workgroup)
+    state_step_head<1, LV, DR, float, uint16_t, float, false>(m, blockIdx.x, min(h, m.H - 1), 0, 1, threadIdx.x & 255, h < m.H,
+                                                              lds[half]);
+  }
+};
+
+template <int NDC, int NV, bool CAP, int NW, bool TURN, bool PREP, bool ONE, typename MEM = NoMemory>
+__global__ void __launch_bounds__(64 * NW, ONE ? 4 : 1) masked_attn_token_kernel(MaskTokArgs a, typename MEM::Args m2) {
   constexpr int D = NDC * 32, V = NV * 16;
   __shared__ TokLds<NW, V> lds;
   __shared__ __attribute__((aligned(16))) uint16_t qs[PREP ? 16 * D : 8], ks[PREP ? D : 8], vs[PREP ? V : 8];
+  if constexpr (MEM::on) {
+    static_assert(NW == 8 && 2 * sizeof(typename MEM::Lds) <= sizeof(lds), "two heads in the attention's LDS");
+    if ((int)blockIdx.z >= a.t.n_parts)
+      return MEM::run(m2, blockIdx.z - a.t.n_parts, reinterpret_cast<typename MEM::Lds(&)[2]>(lds));
+  }
   const int lane = threadIdx.x & 63, r = lane & 15, hq = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sg = a.items[blockIdx.x * 4], row = a.items[blockIdx.x * 4 + 1], pos = a.items[blockIdx.x * 4 + 3];
@@ -645,7 +674,7 @@ static int launch_mask_tok_nw(const MaskTokArgs& a, int rows, hipStream_t s) {
     if ((long)rows * grid.y * grid.z <= kTurnMasked)
       k = a.softcap > 0.f ? masked_attn_token_kernel<NDC, NV, true, NW, true, PREP, ONE>
                           : masked_attn_token_kernel<NDC, NV, false, NW, true, PREP, ONE>;
-  hipLaunchKernelGGL(k, grid, dim3(64 * NW), 0, s, a);
+  hipLaunchKernelGGL(k, grid, dim3(64 * NW), 0, s, a, NoMemory::Args{});
   if (a.t.n_parts > 1)
     hipLaunchKernelGGL(token_merge_kernel, dim3(rows * a.t.H), dim3(256), 0, s, a.t, a.items, NV * 16);
   return (int)hipGetLastError();
@@ -680,6 +709,28 @@ static int mask_tok_any(const MaskTokArgs& a, int D, int V, int rows, hipStream_
   if (D == 64 && V == 128) return launch_mask_tok<2, 8>(a, rows, s);
   if (D == 128 && V == 64) return launch_mask_tok<4, 4>(a, rows, s);
   return launch_mask_tok<4, 8>(a, rows, s);
+}
+
+template <int NDC, int NV>
+static int launch_mask_memory(const MaskTokArgs& a, const StepArgs& m, int MD, int rows, hipStream_t s) {
+  const int hpg = a.t.H / a.G, y = a.G * ((hpg + 15) / 16), z = ((m.H + 1) / 2 + y - 1) / y;
+  const dim3 grid(rows, y, a.t.n_parts + z);
+  const bool turn = NV == 2 * NDC && (long)rows * y * a.t.n_parts <= kTurnMasked;
+#define K8S_MM(LV, DR)                                                                                                  \
+  if (m.V == 4 * LV && MD == DR * (256 / LV)) {                                                                         \
+    using MEM = WithMemory<LV, DR>;                                                                                     \
+    hipLaunchKernelGGL((turn ? masked_attn_token_kernel<NDC, NV, false, 8, NV == 2 * NDC, true, true, MEM>              \
+                             : masked_attn_token_kernel<NDC, NV, false, 8, false, true, true, MEM>),                    \
+                       grid, dim3(512), 0, s, a, m);                                                                    \
+    if (a.t.n_parts > 1)                                                                                                \
+      hipLaunchKernelGGL(token_merge_kernel, dim3(rows * a.t.H), dim3(256), 0, s, a.t, a.items, NV * 16);               \
+    return (int)hipGetLastError();                                                                                      \
+  }
+  K8S_MM(32, 8)
+  K8S_MM(16, 8)
+  K8S_MM(16, 4)
+#undef K8S_MM
+  return (int)hipErrorInvalidValue;
 }
 
 template <int NR, int NP>
@@ -741,28 +792,54 @@ K8S_API int k8s_masked_attn_token(const void* q, const void* kc, const void* vt,
 // The same on rows as their projection left them, every row the only one of its sequence (TokPrep): what k8s_attn_prep_half
 // and k8s_masked_attn_token give.  D 64 or 128, qs and pstep multiples of 4, rot a multiple of 8 with its table, x / kc / cs /
 // v_other / v_keep 16-byte aligned; vc may be null.
-K8S_API int k8s_masked_attn_token_prep(const float* x, int qs, int planes, long pstep, const float* bias, const float* q_w,
-                                       const float* k_w, float eps, int norm, const float* cs, int rot, float lam,
-                                       const float* v_other, float* v_keep, const int* slots, void* vc, void* kc, void* vt,
-                                       const int* bt, int maxb, const int* items, int rows, const float* sink,
-                                       const float* gate, int gs, void* out, int H, int G, int D, int V, int BS, int chunk,
-                                       int window, int keep_first, float scale, float softcap, hipStream_t s, int part_blocks,
-                                       int most, int n_parts, float* pml, float* po) {
-  if (rows <= 0) return 0;
+#define K8S_PREP_PARAMS                                                                                                     \
+  const float *x, int qs, int planes, long pstep, const float *bias, const float *q_w, const float *k_w, float eps, int norm,  \
+      const float *cs, int rot, float lam, const float *v_other, float *v_keep, const int *slots, void *vc, void *kc, void *vt, \
+      const int *bt, int maxb, const int *items, int rows, const float *sink, const float *gate, int gs, void *out, int H,      \
+      int G, int D, int V, int BS, int chunk, int window, int keep_first, float scale, float softcap, hipStream_t s,            \
+      int part_blocks, int most, int n_parts, float *pml, float *po
+#define K8S_PREP_NAMES                                                                                                    \
+  x, qs, planes, pstep, bias, q_w, k_w, eps, norm, cs, rot, lam, v_other, v_keep, slots, vc, kc, vt, bt, maxb, items, rows, \
+      sink, gate, gs, out, H, G, D, V, BS, chunk, window, keep_first, scale, softcap, s, part_blocks, most, n_parts, pml, po
+static bool prep_args(MaskTokArgs& a, K8S_PREP_PARAMS) {
+  (void)s;
   auto off = [](const void* p) { return ((uintptr_t)p & 15) != 0; };
   if (!k8s_masked_attn_mfma_ok(H, G, D, V) || D == 96 || BS % 32 || chunk < 0 || window < 0 || keep_first < 0 || n_parts < 1 ||
       part_blocks < 1 || most < 1 || n_parts > most || (n_parts > 1 && (!pml || !po)) || !x || qs % 4 || planes < 1 ||
       (planes > 1 && pstep % 4) || rot < 0 || rot > D || rot % 8 || (rot && !cs) || norm < 0 || norm > 1 || !slots || !kc ||
       !vt || off(x) || off(cs) || off(kc) || off(v_other) || off(v_keep) || ((uintptr_t)vc & 7))
-    return (int)hipErrorInvalidValue;
-  MaskTokArgs a;
+    return false;
   a.q = nullptr; a.kc = (uint16_t*)kc; a.vt = (uint16_t*)vt; a.bt = bt; a.maxb = maxb;
   a.items = items; a.G = G; a.BS = BS; a.chunk = chunk; a.window = window; a.keep_first = keep_first;
   a.part_blocks = part_blocks; a.most = most; a.scale = scale; a.softcap = softcap;
   a.t.sink = sink; a.t.gate = gate; a.t.gs = gs; a.t.out = (uint16_t*)out; a.t.out32 = nullptr;
   a.t.ost = (long)H * V; a.t.osh = V; a.t.po = po; a.t.pml = pml; a.t.H = H; a.t.n_parts = n_parts; a.t.hs = 1;
   a.p = TokPrep{x, bias, q_w, k_w, cs, v_other, v_keep, slots, (uint16_t*)vc, (size_t)pstep, qs, planes, rot, norm, eps, lam};
-  return mask_tok_any(a, D, V, rows, s);
+  return true;
+}
+
+K8S_API int k8s_masked_attn_token_prep(K8S_PREP_PARAMS) {
+  if (rows <= 0) return 0;
+  MaskTokArgs a;
+  return prep_args(a, K8S_PREP_NAMES) ? mask_tok_any(a, D, V, rows, s) : (int)hipErrorInvalidValue;
+}
+
+// The same and k8s_memory_step of the same rows (its x: `mx`, bf16 out) in one launch.  Heads share keys (H > G), no softcap,
+// D and V not both 64, n_parts < most, part_blocks <= 8.
+K8S_API int k8s_masked_attn_memory(K8S_PREP_PARAMS, const float* mx, int mxs, const float* gate_bias, float cap, float* state,
+                                   float* nstate, float* mstate, const int* pos0, const int* slot, const float* mgate, int mgs,
+                                   const float* mw, int mwh, void* mout, int MH, int MD, int MV, float meps, float den_eps) {
+  if (rows <= 0) return 0;
+  MaskTokArgs a;
+  if (!prep_args(a, K8S_PREP_NAMES) || H <= G || softcap > 0.f || n_parts >= most || part_blocks > 8 || MH < 1 || !mx || !state ||
+      !nstate || !mstate || !pos0 || !slot || !mgate || !mout)
+    return (int)hipErrorInvalidValue;
+  const StepArgs m = memory_args(mx, mxs, gate_bias, cap, state, nstate, mstate, pos0, slot, mgate, mgs, mw, mwh, mout, MH, MV, meps,
+                                 den_eps);
+  if (D == 128 && V == 128) return launch_mask_memory<4, 8>(a, m, MD, rows, s);
+  if (D == 64 && V == 128) return launch_mask_memory<2, 8>(a, m, MD, rows, s);
+  if (D == 128 && V == 64) return launch_mask_memory<4, 4>(a, m, MD, rows, s);
+  return (int)hipErrorInvalidValue;
 }
 
 // items [rows][4]; n_parts > 1: po [rows][H][n_parts][R], pml [rows][H][n_parts][2]

@@ -401,12 +401,11 @@ class LizesunModel:
         x = R.proj_f32out(h, L["w_in"])                                # left q | k | v, right q | k | v | g | i | f
         rope = self.ropes.get((a.rot_dims, a.rot_base))
         prep = dict(norm=True, eps=self.cfg.norm_eps, rope=rope, rope_cs=tables.of(rope))
-        ol = S.prep_attention(x[:, :nl], None, H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg,
-                              self.dtype, a.scale, prep, dict(window=a.window, keep_first=a.keep_first, sink=L["sink"]))
-        xr = x[:, nl:]
-        orr = S.memory_layer(xr, b.heads, b.dim, b.vdim, L["gate_bias"], b.gate_cap, states[f"mem{j}"], states[f"memn{j}"],
-                             states[f"memm{j}"], inp.seg, L["mem_norm"], self.cfg.norm_eps, self.dtype)
-        return ol, orr
+        mask = dict(window=a.window, keep_first=a.keep_first, sink=L["sink"])
+        return S.attention_and_memory(x[:, :nl], H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg,
+                                      self.dtype, a.scale, prep, mask, x[:, nl:], b.heads, b.dim, b.vdim, L["gate_bias"],
+                                      b.gate_cap, states[f"mem{j}"], states[f"memn{j}"], states[f"memm{j}"], inp.seg,
+                                      L["mem_norm"], self.cfg.norm_eps, self.dtype)
 
     def _delta(self, li: int, h, inp: S.SegStepInputs, states) -> torch.Tensor:
         L, c = self.layers[li], self.cfg.layers[li].delta

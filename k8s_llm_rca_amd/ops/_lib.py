@@ -126,6 +126,8 @@ _SIGS = {
     "k8s_masked_attn_token": [P, P, P, P, I, P, I, P, P, I, P, I, I, I, I, I, I, I, I, F, F, P, I, I, I, P, P, I, I],
     "k8s_masked_attn_token_prep": [P, I, I, L, P, P, P, F, I, P, I, F, P, P, P, P, P, P, P, I, P, I, P, P, I, P, I, I, I, I, I,
                                    I, I, I, F, F, P, I, I, I, P, P],
+    "k8s_masked_attn_memory": [P, I, I, L, P, P, P, F, I, P, I, F, P, P, P, P, P, P, P, I, P, I, P, P, I, P, I, I, I, I, I, I, I, I, F,
+                               F, P, I, I, I, P, P, P, I, P, F, P, P, P, P, P, P, I, P, I, P, I, I, I, F, F],
     "k8s_latent_attn_rows": [P, P, P, I, P, P, P, P, I, P, I, I, I, I, I, F, I, P, L, L, P, I, L, L, I, P, I, P, P],
     "k8s_polynorm": [P, P, P, I, I, F, I, P],
     "k8s_glu_clamp": [P, P, I, I, F, F, F, I, P],

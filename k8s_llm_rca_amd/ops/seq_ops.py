@@ -1409,7 +1409,7 @@ def prep_attention(x: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int
 
 def _prep_tokens(x, bias, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, norm=False, q_w=None, k_w=None, eps=0.0,
                  lam=0.0, v_other=None, v_keep=None, rope=None, rope_cs=None, softcap=0.0, chunk=0, window=0, keep_first=0,
-                 sink=None, gate=None) -> Optional[torch.Tensor]:
+                 sink=None, gate=None, beside=None) -> Optional[torch.Tensor]:
     T = x.shape[-2]
     if T != seg.n_seg:                               # (before anything else: prompts pay for one comparison)
         return None
@@ -1434,16 +1434,43 @@ def _prep_tokens(x, bias, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, 
                                         lambda: _mask_plan(seg, H, G, D, V, int(chunk), int(window), int(keep_first), 1))
     if D == 64 and T * G * -(-(H // G) // 16) * parts > PREP_GROUPS:
         return None
+    if beside is not None and not (H > G and D + V > 128 and softcap == 0.0 and parts < TOKEN_PARTS and MASK_TOKEN_BLOCKS <= 8):
+        return None
     out = torch.empty(T, H * V, dtype=out_dtype, device=x.device)
     groups, po, pml = _token_groups(rows, H, parts, V)
+    if beside is not None and len(groups) > 1:
+        return None
     for it in groups:
-        check(lib().k8s_masked_attn_token_prep(
+        args = (
             ptr(x), x.stride(-2), planes, pstep, ptr(bias), ptr(q_w), ptr(k_w), float(eps), int(bool(norm)), ptr(rope_cs), rot,
             float(lam), ptr(v_other), ptr(v_keep), ptr(slots), ptr(vc), ptr(kc), ptr(vt), ptr(seg.block_tables),
             seg.block_tables.shape[1], ptr(it), it.shape[0], ptr(sink), ptr(gate), gate.stride(0) if gate is not None else 0,
             ptr(out), H, G, D, V, BS, int(chunk), int(window), int(keep_first), float(scale), float(softcap), stream_ptr(x),
-            MASK_TOKEN_BLOCKS, TOKEN_PARTS, parts, ptr(pml), ptr(po)), "masked_attn_token_prep")
+            MASK_TOKEN_BLOCKS, TOKEN_PARTS, parts, ptr(pml), ptr(po))
+        if beside is not None:
+            check(lib().k8s_masked_attn_memory(*args, *beside.args), "masked_attn_memory")
+        else:
+            check(lib().k8s_masked_attn_token_prep(*args), "masked_attn_token_prep")
     return out
+
+
+def attention_and_memory(x: torch.Tensor, H: int, G: int, D: int, V: int, positions: torch.Tensor, slots: torch.Tensor, kc, vc, vt,
+                         seg: SegMeta, out_dtype, scale: float, prep: dict, mask: dict, xm: torch.Tensor, *memory) -> tuple:
+    """:func:`prep_attention` (without a bias) of ``x`` and :func:`memory_layer` of ``xm`` (with the further arguments), columns of
+    the same rows.
+
+    Of single tokens in one launch (csrc/kernels/token_attn.hip, MEM), at every number of them: us of both launches / one, 16 heads
+    over 2 of 128 beside 16 of 64 x 128:  1 row at 100 keys 11.1 / 7.1, 5 at 1100 15.9 / 11.8, 64 at 450 34.7 / 31.5, 128 at 300 51.7 /
+    49.9;  12 over 3 of 64 + 128 beside 32 of 64 x 64 10.6 / 6.9, 15.1 / 11.2, 37.3 / 33.4, 57.1 / 57.0.  Heads of 128 x 128 stay
+    apart: their state does not fit beside the attention's registers."""
+    # (the rows before anything else: prompts pay for one comparison)
+    step = _memory_step(xm, *memory) if xm.shape[0] == seg.n_seg and out_dtype == torch.bfloat16 else None
+    if step is not None and (step.dim, step.vdim) != (128, 128):
+        o = _prep_tokens(x, None, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, **prep, **mask, beside=step)
+        if o is not None:
+            return o, step.out
+    return (prep_attention(x, None, H, G, D, V, positions, slots, kc, vc, vt, seg, out_dtype, scale, prep, mask),
+            memory_layer(xm, *memory))
 
 
 # Prompt tiles cut over their keys where few of them would leave the chip idle behind a long context.  us, whole / cut, 16
@@ -1831,23 +1858,41 @@ def delta_low_rank(qkv: torch.Tensor, H: int, G: int, D: int, V: int, lr: torch.
     return delta_layer(qkv, H, G, D, V, dec, rate, dt_bias, lr[:, ra + rg:], state, seg, gate, w, eps, out_dtype)
 
 
-def memory_layer(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tensor, cap: float, state: torch.Tensor,
-                 nstate: torch.Tensor, mstate: torch.Tensor, seg: SegMeta, w: Optional[torch.Tensor], eps: float,
-                 out_dtype) -> torch.Tensor:
-    """:func:`matrix_memory`, then :func:`head_norm_gate` over each head with the gates that stand behind the values."""
-    gate = x[:, 2 * H * D + H * V:2 * H * (D + V)]
-    if _step_ok(x, seg, D, V, state, gate, w):
-        T = x.shape[0]
+class _MemoryStep:
+    """What a launch of one token per sequence through the matrix memory takes, and its result."""
+
+    def __init__(self, x, H, D, V, gate_bias, cap, state, nstate, mstate, seg, w, eps, out_dtype, gate):
         assert x.dtype == torch.float32 and x.shape[1] == 2 * H * (D + V) + 2 * H
         assert gate_bias.dtype == torch.float32 and gate_bias.numel() == 2 * H and (w is None or w.numel() in (V, H * V))
         assert state.is_contiguous() and state.shape[1:] == (H, D, V) and nstate.is_contiguous()
         assert nstate.shape[1:] == (H, D) and mstate.is_contiguous() and mstate.shape[1:] == (H,)
-        out = torch.empty(T, H * V, dtype=out_dtype, device=x.device)
-        check(lib().k8s_memory_step(ptr(x), x.stride(0), ptr(gate_bias), float(cap), ptr(state), ptr(nstate), ptr(mstate),
-                                    ptr(seg.seg_pos0), ptr(seg.seg_slot), ptr(gate), gate.stride(0), ptr(w),
-                                    V if w is not None and w.numel() == H * V else 0, ptr(out), _dt(out_dtype), T, H, D, V,
-                                    float(eps), float(DEN_EPS), stream_ptr(x)), "memory_step")
-        return out
+        self.heads, self.dim, self.vdim = H, D, V
+        self.out = torch.empty(x.shape[0], H * V, dtype=out_dtype, device=x.device)
+        self.args = (ptr(x), x.stride(0), ptr(gate_bias), float(cap), ptr(state), ptr(nstate), ptr(mstate), ptr(seg.seg_pos0),
+                     ptr(seg.seg_slot), ptr(gate), gate.stride(0), ptr(w), V if w is not None and w.numel() == H * V else 0,
+                     ptr(self.out), H, D, V, float(eps), float(DEN_EPS))
+
+
+def _memory_gate(x: torch.Tensor, H: int, D: int, V: int) -> torch.Tensor:
+    return x[:, 2 * H * D + H * V:2 * H * (D + V)]
+
+
+def _memory_step(x, H, D, V, gate_bias, cap, state, nstate, mstate, seg, w, eps, out_dtype) -> Optional[_MemoryStep]:
+    gate = _memory_gate(x, H, D, V)
+    if not _step_ok(x, seg, D, V, state, gate, w):
+        return None
+    return _MemoryStep(x, H, D, V, gate_bias, cap, state, nstate, mstate, seg, w, eps, out_dtype, gate)
+
+
+def memory_layer(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tensor, cap: float, state: torch.Tensor,
+                 nstate: torch.Tensor, mstate: torch.Tensor, seg: SegMeta, w: Optional[torch.Tensor], eps: float,
+                 out_dtype) -> torch.Tensor:
+    """:func:`matrix_memory`, then :func:`head_norm_gate` over each head with the gates that stand behind the values."""
+    step = _memory_step(x, H, D, V, gate_bias, cap, state, nstate, mstate, seg, w, eps, out_dtype)
+    if step is not None:
+        check(lib().k8s_memory_step(*step.args[:14], _dt(out_dtype), x.shape[0], *step.args[14:], stream_ptr(x)), "memory_step")
+        return step.out
+    gate = _memory_gate(x, H, D, V)
     o, mul = matrix_memory(x, H, D, V, gate_bias, cap, state, nstate, mstate, seg, defer_scale=True)
     return head_norm_gate(o, gate, w, H, V, eps, out_dtype, mul=mul)
 

@@ -1,0 +1,54 @@
+"""Attention and matrix memory of single tokens in one launch (csrc/kernels/token_attn.hip, MEM) against the two launches: the same
+bits in both results, the caches and the states."""
+import pytest
+import torch
+
+from k8s_llm_rca_amd.ops import seq_ops as S
+
+pytestmark = pytest.mark.gpu
+BF, BS = torch.bfloat16, 64
+
+
+def meta(pos, maxb):
+    n = len(pos)
+
+    def i32(v):
+        return torch.tensor(v, dtype=torch.int32, device="cuda")
+    tables = [[i * maxb + (j * 5) % maxb for j in range(maxb)] for i in range(n)]
+    slots = i32([tables[i][p // BS] * BS + p % BS for i, p in enumerate(pos)])
+    state = list(range(n, 0, -1))
+    return S.SegMeta(n, i32(range(n)), i32(range(n + 1)), i32(pos), i32(state), i32(tables), list(range(n + 1)), list(pos),
+                     state, n_single=n), slots
+
+
+@pytest.mark.parametrize("H,G,D,V", [(16, 2, 128, 128), (33, 1, 64, 128), (6, 2, 128, 64)])
+@pytest.mark.parametrize("MH,MD,MV", [(16, 64, 128), (3, 64, 64), (5, 128, 64), (2, 128, 128)])
+@pytest.mark.parametrize("pos", [[0], [5, 300, 0, 700, 255], [30] * 20])
+@pytest.mark.parametrize("kind", ["plain", "window"])
+def test_same_bits(H, G, D, V, MH, MD, MV, pos, kind):
+    n, maxb, g = len(pos), 12, torch.Generator().manual_seed(H + MH)
+    cols, mcols = (H + G) * D + G * V, 2 * MH * (MD + MV) + 2 * MH
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).cuda()
+    pad = -(cols + mcols) % 4
+    x = rnd(n, cols + mcols + pad)
+    k0, v0 = rnd(n * maxb, BS, G * D).to(BF), rnd(n * maxb, G * V, BS).to(BF)
+    gb, w = rnd(2 * MH), rnd(MV)
+    st0 = [rnd(n + 1, MH, MD, MV) * 0.3, rnd(n + 1, MH, MD), rnd(n + 1, MH)]
+    mask = dict(window=200, keep_first=40, sink=rnd(H)) if kind == "window" else {}
+    got = []
+    for one in (True, False):
+        seg, slots = meta(pos, maxb)
+        kc, vt, st = k0.clone(), v0.clone(), [s.clone() for s in st0]
+        memory = (MH, MD, MV, gb, 15.0, *st, seg, w, 1e-5, BF)
+        args = (H, G, D, V, seg.seg_pos0, slots, kc, None, vt, seg, BF, D ** -0.5)
+        prep = dict(norm=True, eps=1e-5)
+        if one:
+            o, m = S.attention_and_memory(x[:, :cols], *args, prep, mask, x[:, cols:cols + mcols], *memory)
+        else:
+            o = S.prep_attention(x[:, :cols], None, *args, prep, mask)
+            m = S.memory_layer(x[:, cols:cols + mcols], *memory)
+        got.append((o, m, kc, vt, *st))
+    for a, b in zip(*got):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
