@@ -457,7 +457,9 @@ __global__ void __launch_bounds__(256) gemm_glds_kernel(const uint16_t* __restri
                                                         int kslice, int silu_i, int act, K8sPush push) {
   __shared__ __attribute__((aligned(16))) uint16_t sm[glds_lds_elems<MTW, NB, NF>()];
   // strip: 16 NF W rows (plain: output columns n0 ..; SwiGLU: 8 NF act columns n0 ..)
-  const int n0 = blockIdx.x * (silu_i ? 8 : 16) * NF, split = blockIdx.y, kbeg = split * kslice;
+  // (act 2, fp32 out: the last strip may begin within the one before it, whose columns both then write alike)
+  const int n0 = min((int)blockIdx.x * (silu_i ? 8 : 16) * NF, N - (silu_i ? 8 : 16) * NF), split = blockIdx.y,
+            kbeg = split * kslice;
   f32x4 acc[MTW][NF];
 #pragma unroll
   for (int mt = 0; mt < MTW; ++mt)
@@ -469,7 +471,7 @@ __global__ void __launch_bounds__(256) gemm_glds_kernel(const uint16_t* __restri
     glds_push_store<MTW, NF>(acc, M, sm, push, n0, blockIdx.x);
   else if (silu_i)
     glds_store<MTW, NF>(acc, M, y + n0, ldy, nullptr, 0, true);
-  else if (gridDim.y == 1)
+  else if (gridDim.y == 1 && act != 2)
     glds_store<MTW, NF>(acc, M, y + n0, ldy, nullptr, 0, false, act);
   else
     glds_store<MTW, NF>(acc, M, nullptr, 0, part + (size_t)split * M * N + n0, N);
@@ -614,9 +616,11 @@ static int stream_launch(const void* x, int ldx, const void* w, void* y, int ldy
   // push (splits == 1): the LDS-DMA kernel's own epilogue pushes; splits > 1: the reduce pass does
   const K8sPush* gpush = (push && splits == 1) ? push : nullptr;
   if (push && (silu || !reduce || (splits == 1 && cfg < 13))) return (int)hipErrorInvalidValue;
-  if (act && (act != 1 || silu || push || splits != 1 || cfg < 13)) return (int)hipErrorInvalidValue;
+  if (act && (act > 2 || silu || push || splits != 1 || cfg < 13)) return (int)hipErrorInvalidValue;
+  const bool f32 = act == 2;                 // the sums as they are, to part [M][N]
   const int bn = (cfg > 30 ? 32 : cfg > 20 ? 128 : kSBN) / (silu ? 2 : 1);  // output columns per strip
-  if (M <= 0 || M > 256 || N % bn || splits < 1 || K % (splits * kSC) || (splits > 1 && part == nullptr) ||
+  if (M <= 0 || M > 256 || N < bn || N % (f32 ? 16 : bn) || splits < 1 || K % (splits * kSC) ||
+      ((splits > 1 || f32) && part == nullptr) || (!y && !push && !f32 && (splits == 1 || reduce)) ||
       (cfg != 4 && cfg != 8 && (cfg < 13 || cfg > 16) && cfg != 23 && cfg != 24 && cfg != 34 && cfg != 36) || ldx % 8 ||
       (splits > 1 && (M * N) % 8) || ((splits == 1 || reduce) && ldy < N) || (silu && splits != 1))
     return (int)hipErrorInvalidValue;
@@ -630,7 +634,7 @@ static int stream_launch(const void* x, int ldx, const void* w, void* y, int ldy
       (cfg > 30 && (mtw > 2 || push)))
     return (int)hipErrorInvalidValue;
   if (cfg == 8 && mtw > 2) return (int)hipErrorInvalidValue;  // an 8-deep X ring would not fit the VGPRs
-  const dim3 grid(N / bn, splits);
+  const dim3 grid((N + bn - 1) / bn, splits);
   const uint16_t* xx = (const uint16_t*)x;
   const uint16_t* ww = (const uint16_t*)w;
   uint16_t* yy = (uint16_t*)y;
@@ -719,6 +723,11 @@ K8S_API int k8s_gemm_stream(const void* x, int ldx, const void* w, void* y, int 
 K8S_API int k8s_gemm_stream_act(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int cfg,
                                 int act, hipStream_t s) {
   return stream_launch(x, ldx, w, y, ldy, M, N, K, cfg, 1, nullptr, true, s, false, nullptr, act);
+}
+
+// y [M][N] fp32, one K range; N a multiple of 16, no smaller than a strip.
+K8S_API int k8s_gemm_stream_f32(const void* x, int ldx, const void* w, float* y, int M, int N, int K, int cfg, hipStream_t s) {
+  return stream_launch(x, ldx, w, nullptr, N, M, N, K, cfg, 1, y, false, s, false, nullptr, 2);
 }
 
 extern "C" int k8s_ar_push_desc(int id, int N, int T, int mode, K8sPush* out);

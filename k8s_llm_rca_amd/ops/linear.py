@@ -402,6 +402,26 @@ def _skinny_f32(M: int, N: int, K: int) -> bool:
             and M * N <= (SKINNY_F32_SHORT_MN if K <= SKINNY_F32_SHORT_K else SKINNY_F32_MAX_MN))
 
 
+STREAM_F32_MAX_M = 64
+
+
+def stream_f32_cfg(M: int, N: int, K: int) -> int:
+    """The stream kernel's form for a product of 17 to 64 rows with an fp32 result that neither the row-streaming nor the skinny
+    kernel takes, or 0: the library.  Strips of 32 columns within one wave of workgroups, then of 64 where they fill their waves.
+    us of the library / this at 33, 64 rows:  2304 x 2048 8.8 / 8.6, 9.2 / 8.6;  2576 x 2048 9.0 / 8.7, 9.3 / 8.8;  2304 x 1024 8.6 /
+    5.7, 8.9 / 5.8;  6144 x 2048 10.1 / 8.8, 10.0 / 8.9;  8192 x 2048 12.8 / 10.9, 13.2 / 11.4;  8736 x 2048 14.7 / 12.7, 14.9 / 13.3;
+    12288 x 1024 9.9 / 7.6, 9.7 / 7.9;  16384 x 2048 18.2 / 17.7, 18.4 / 17.8;  32768 x 2048 36 / 31, 36 / 32;  65536 x 1024 32 / 28, 36 /
+    32;  at 17 rows 5136 x 2048 12.0 / 8.7, 12304 x 2048 16.7 / 13.8.  Not: 1088 x 2048 8.6 / 8.6, 576 x 2048 5.7 / 8.4, 2048 x 4096 9.5 /
+    14.1, 20480 x 1536 (1.25 waves) 18.0 / 19.1, 24576 x 2048 (1.5) 26.2 / 26.4, 50256 x 2048 (3.07) 50.6 / 52.3;  2576 x 2048 at
+    97 rows 9.8 / 10.9.  And the library's front end takes 12 us more of the host a call."""
+    if not (16 < M <= STREAM_F32_MAX_M and N >= 2304 and N % 16 == 0 and 1024 <= K <= 2048 and K % 64 == 0):
+        return 0
+    if N <= 32 * NARROW_WGS:
+        return 34
+    strips = -(-N // 64)
+    return 14 if strips <= 256 or 20 * strips >= 19 * 256 * -(-strips // 256) else 0
+
+
 def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` with an fp32 result: bf16 operands with fp32 accumulation (the weight-streaming kernel for a few rows,
     hipBLASLt otherwise), or fp32 throughout."""
@@ -417,6 +437,11 @@ def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         out = torch.empty((M, N), dtype=torch.float32, device=x.device)
         check(lib().k8s_gemm_skinny_f32(ptr(x), x.stride(0), ptr(w), ptr(out), N, M, N, K, stream_ptr(x)),
               "gemm_skinny_f32")
+        return out
+    cfg = stream_f32_cfg(M, N, K) if 16 < M <= STREAM_F32_MAX_M else 0
+    if cfg and (N, K) not in _dispatch and K == w.shape[1] and _few_ok(x, w):
+        out = torch.empty((M, N), dtype=torch.float32, device=x.device)
+        check(lib().k8s_gemm_stream_f32(ptr(x), x.stride(0), ptr(w), ptr(out), M, N, K, cfg, stream_ptr(x)), "gemm_stream_f32")
         return out
     return linear_f32out(x, w)
 
