@@ -183,6 +183,10 @@ struct K8sLlamaStep {
   // still reading the current one), so the current residual alternates.
   void* res2;
   int norm_fuse;
+  // the norm behind the last layer, into `out` [T][H] (TP = 1; null: the caller's): a split-K down projection's partials are
+  // reduced inside it, as inside the norms between the layers
+  const void* final_norm;
+  void* out;
 };
 
 namespace {
@@ -247,7 +251,8 @@ bool push_kind(const K8sGemmSel& g) { return g.kind == 4 && (g.cfg >= 13 || g.sp
   } while (0)
 
 // Layers [0, L): on return `y` holds nothing useful and `prev` + `residual`
-// are the inputs of the final norm (exactly as after the Python loop).
+// are the inputs of the final norm (exactly as after the Python loop), or with
+// `final_norm` its result is in `out`.
 // Where the step's dispatch picked a split-K kernel for the o or down
 // projection, its partials are reduced inside the following residual-add +
 // RMSNorm (k8s_splitk_addnorm), and a split-K qkv projection's inside the
@@ -373,8 +378,9 @@ K8S_API int k8s_llama_layers(const K8sLlamaStep* sp, hipStream_t st) {
       K8S_TRY(gemm(s, s.sel[2], s.y, H, s.wgu[l], s.gu, 2 * s.I, T, 2 * s.I, H, st));
       K8S_TRY(k8s_silu_mul(s.gu, s.act, T, s.I, st));
     }
-    // the last layer's down output is returned (`prev`) for the final norm
-    pend = !tp && deferred(s.sel[3], l + 1 < s.L);
+    // the last layer's down output is returned (`prev`) for the final norm, unless that is made here
+    const bool more = l + 1 < s.L || (s.final_norm && !s.nf_flags);
+    pend = !tp && deferred(s.sel[3], more);
     if (push_d && l + 1 < s.L) {  // the next layer's input norm rides on this all-reduce
       K8S_TRY(k8s_gemm_stream_push(s.act, s.I, s.wdown[l], T, H, s.I, s.sel[3].cfg, s.sel[3].splits, s.mid_part,
                                    s.ar_id, s.ar_mode, st));
@@ -382,13 +388,19 @@ K8S_API int k8s_llama_layers(const K8sLlamaStep* sp, hipStream_t st) {
                                        k8s::k8s_push_strips(s.sel[3].cfg, s.sel[3].splits, H), st));
       continue;
     }
-    K8S_TRY(gemm(s, s.sel[3], s.act, s.I, s.wdown[l], s.prev, H, T, H, s.I, st, !tp && l + 1 < s.L));
+    K8S_TRY(gemm(s, s.sel[3], s.act, s.I, s.wdown[l], s.prev, H, T, H, s.I, st, !tp && more));
     if (fuse_an && l + 1 < s.L)  // the next layer's input norm rides on this all-reduce
       K8S_TRY(k8s_ar_addnorm_bf16(s.ar_id, s.prev, s.residual, s.in_norm[l + 1], s.y, T, H, s.eps, s.ar_mode, st));
     else if (tp)
       K8S_TRY(k8s_ar_allreduce_bf16(s.ar_id, s.prev, s.prev, n_out, s.ar_mode, st));
   }
   if (s.nf_flags && !pend) K8S_TRY(k8s_nonfinite_flag(s.prev, n_out, s.nf_flags + s.L, st));
+  if (!tp && s.final_norm && s.L > 0) {
+    if (pend)
+      K8S_TRY(k8s_splitk_addnorm(part_of(s, s.sel[3]), s.sel[3].splits, rc, s.final_norm, s.out, T, H, H, s.eps, st));
+    else
+      K8S_TRY(k8s_rmsnorm(s.prev, rc, s.final_norm, s.out, T, H, H, H, s.eps, st));
+  }
   return (int)hipGetLastError();
 }
 

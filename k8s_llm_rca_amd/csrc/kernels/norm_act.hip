@@ -198,6 +198,19 @@ __global__ void __launch_bounds__(256) rope_kv_kernel(uint16_t* __restrict__ qkv
   for (int j = 0; j < 8; ++j) vp[(size_t)(d0 + j) * BS] = v[j];
 }
 
+// out[t] = embed[ids[t]], rows of `pieces` 16 bytes.  An id outside the table leaves a row of NaN.  In place of a cast of the ids and
+// a lookup of a row by a handful of threads: 16 rows of 8 KB 4.5 + 13.1 us -> one launch.
+__global__ void __launch_bounds__(512) lookup_rows_kernel(const int* __restrict__ ids, const u16x8* __restrict__ embed, int rows,
+                                                         u16x8* __restrict__ out, int pieces) {
+  const int id = ids[blockIdx.x];
+  const bool in = id >= 0 && id < rows;
+  const u16x8* src = embed + (size_t)(in ? id : 0) * pieces;
+  u16x8 nan;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) nan[k] = 0xffff;
+  for (int c = threadIdx.x; c < pieces; c += blockDim.x) out[(size_t)blockIdx.x * pieces + c] = in ? src[c] : nan;
+}
+
 }  // namespace k8s
 
 using namespace k8s;
@@ -239,6 +252,16 @@ K8S_API int k8s_unpack_step(const void* flat, int Bb, int mb, int n_items, void*
   hipLaunchKernelGGL(unpack_step_kernel, dim3(grid), dim3(256), 0, s, (const int*)flat, Bb, mb, n_items, (int*)ids,
                      (int*)pos, (int*)slots, (int*)ctx, (int*)bt, (int*)n_items_buf, (int*)items,
                      (const int*)spec_src, (const int*)tok, n_spec);
+  return (int)hipGetLastError();
+}
+
+// rows of `bytes` (a multiple of 16); embed and out on 16 bytes
+K8S_API int k8s_lookup_rows(const int* ids, const void* embed, int rows, void* out, int T, int bytes, hipStream_t s) {
+  if (T <= 0) return 0;
+  if (!ids || !embed || !out || rows < 1 || bytes < 16 || bytes % 16 || (((uintptr_t)embed | (uintptr_t)out) & 15))
+    return (int)hipErrorInvalidValue;
+  const int pieces = bytes / 16, threads = pieces >= 512 ? 512 : (pieces + 63) / 64 * 64;
+  hipLaunchKernelGGL(lookup_rows_kernel, dim3(T), dim3(threads), 0, s, ids, (const u16x8*)embed, rows, (u16x8*)out, pieces);
   return (int)hipGetLastError();
 }
 

@@ -23,7 +23,6 @@ from dataclasses import dataclass
 from typing import Dict, List, Optional
 
 import torch
-import torch.nn.functional as F
 
 from ..ops import attention as A
 from ..ops import layer_exec as LX
@@ -162,14 +161,12 @@ class LlamaModel:
         cfg = self.cfg
         T = inp.input_ids.shape[0]
         H = cfg.hidden
-        residual = F.embedding(inp.input_ids.long(), self.embed)     # [T, H]
+        residual = N.lookup_rows(inp.input_ids, self.embed)           # [T, H]
         if self._exec is None and LX.LlamaExecutor.eligible(self):
             self._exec = LX.LlamaExecutor(self)
         if self._exec is not None and LX.LlamaExecutor.eligible(self) and self._exec.fits(T):
             # the dense layer stack in one native call (ops/layer_exec.py): same kernels, same order
-            prev, residual = self._exec.run(inp, residual, k_cache, v_cache)
-            y = torch.empty_like(residual)
-            N.rmsnorm(prev, self.final_norm, cfg.rms_eps, residual=residual, out=y)
+            y = self._exec.run_normed(inp, residual, k_cache, v_cache, self.final_norm)
             sel = y.index_select(0, inp.logits_idx) if inp.logits_idx.numel() != T else y
             logits = self._lm_head(sel)
             return self.pc.all_gather_last(logits) if gather_logits else logits

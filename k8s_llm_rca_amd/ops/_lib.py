@@ -41,6 +41,7 @@ _SIGS = {
     "k8s_gemm_rows_scaled": [P, I, P, P, I, I, I, I, I, I, I, P, I, F, F, P],
     "k8s_few_rows_f32_add": [P, I, P, P, P, I, F, F, P, P, F, P, P, P, I, I, I, P],
     "k8s_few_rows_f32_scaled": [P, I, P, P, I, I, I, I, P, F, P],
+    "k8s_lookup_rows": [P, P, I, P, I, I, P],
     "k8s_gemm_stream_f32": [P, I, P, P, I, I, I, I, P],
     "k8s_gemm_rows_conv": [P, I, P, P, I, P, I, I, I, I, P, I, P, P, P, I, P],
     "k8s_gemm_step_rms": [P, I, P, P, P, I, F, F, P, P, F, P, P, P, I, I, I, P],

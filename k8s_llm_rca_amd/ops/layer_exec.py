@@ -44,7 +44,7 @@ class LlamaStep(ctypes.Structure):
         ("sel", GemmSel * 4),
         ("blaslt_ws", P), ("blaslt_ws_bytes", ctypes.c_size_t), ("mid_part", P), ("grp_part", P), ("grp_offs", P),
         ("ar_id", I), ("ar_mode", I), ("ar_fuse", I), ("ar_push", I), ("nf_flags", P),
-        ("res2", P), ("norm_fuse", I),
+        ("res2", P), ("norm_fuse", I), ("final_norm", P), ("out", P),
     ]
 
 
@@ -178,6 +178,22 @@ class LlamaExecutor:
             return self._run_nano(inp, residual, serial=_nano_serial)
         prev = scratch(tuple(residual.shape), residual.dtype, residual.device)
         return self._issue(self.st, inp, residual, prev, 0, T, inp.n_decode, stream_ptr(residual))
+
+    def run_normed(self, inp, residual: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                   norm: torch.Tensor) -> torch.Tensor:
+        """All layers and the norm behind them."""
+        from . import norm as N
+        y = torch.empty_like(residual)
+        if self._car is not None or self.st.L == 0 or self._nano_ok(inp, residual.shape[0]):
+            prev, residual = self.run(inp, residual, k_cache, v_cache)
+            N.rmsnorm(prev, norm, self.m.cfg.rms_eps, residual=residual, out=y)
+            return y
+        self.st.final_norm, self.st.out = norm.data_ptr(), y.data_ptr()
+        try:
+            self.run(inp, residual, k_cache, v_cache)
+        finally:
+            self.st.final_norm = self.st.out = None
+        return y
 
     # ------------------------------------------------------------ one layer stack
     def _issue(self, st: LlamaStep, inp, residual: torch.Tensor, prev: torch.Tensor, row0: int, T: int, nd: int,

@@ -5,7 +5,7 @@ from typing import Optional
 
 import torch
 
-from ._lib import check, lib, ptr, stream_ptr, use_hip
+from ._lib import check, lib, ptr, stream_ptr, unwatched, use_hip
 
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optional[torch.Tensor] = None,
@@ -269,6 +269,19 @@ def softcap_(logits: torch.Tensor, scale: float, cap: float) -> torch.Tensor:
     if cap > 0:
         logits.copy_(cap * torch.tanh(logits / cap))
     return logits
+
+
+def lookup_rows(ids: torch.Tensor, embed: torch.Tensor) -> torch.Tensor:
+    """``embed[ids]``: rows of 16-byte pieces by one launch (csrc/kernels/norm_act.hip)."""
+    W = embed.shape[1]
+    if (embed.is_cuda and ids.dtype == torch.int32 and ids.dim() == 1 and ids.is_contiguous() and ids.device == embed.device
+            and unwatched(embed, ids) and embed.is_contiguous() and W > 0 and W * embed.element_size() % 16 == 0
+            and embed.data_ptr() % 16 == 0):
+        out = torch.empty(ids.shape[0], W, dtype=embed.dtype, device=embed.device)
+        check(lib().k8s_lookup_rows(ptr(ids), ptr(embed), embed.shape[0], ptr(out), ids.shape[0], W * embed.element_size(),
+                                   stream_ptr(embed)), "lookup_rows")
+        return out
+    return torch.nn.functional.embedding(ids.long(), embed)
 
 
 # ------------------------------------------------------------------ Dynamic Tanh norm around an fp32 residual
