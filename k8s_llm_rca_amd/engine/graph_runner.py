@@ -27,6 +27,7 @@ from ..knobs import KNOBS
 from ..ops import attention as A
 from ..ops import sampling as SMP
 from ..ops._lib import scratch
+from ..ops.row_step import RowStep
 from ..ops.seq_ops import SegMeta, SegStepInputs
 from ..utils import tracing
 from .structured import GrammarState
@@ -309,9 +310,10 @@ class GraphRunnerMixin:
         of one sequence, too many rows, or a shape that has not come often enough).  A graph fixes the number of rows
         and how many cache pages the attention's grids are laid out for (the width of the block tables: a power of two up to
         8 pages, then in steps of 8, past 128 of 32); everything else a step's kernels need -- tokens, positions, cache and state slots,
-        pages, work items -- is read from one static buffer that each step fills with one copy.  The logits are copied
-        out: what a step returns stays the caller's.  A capture that fails -- it takes memory beside the allocator's free
-        blocks -- has run nothing, so the step runs eagerly."""
+        pages, work items -- is read from one static buffer that each step fills with one copy.  The last product is a launch
+        behind the graph, into memory of the step's own: what a step returns stays the caller's, without a copy of it (2 to 6 us
+        of 350 to 500 with one to seven rows of 32000 columns).  A capture that fails -- it takes memory beside the allocator's
+        free blocks -- has run nothing, so the step runs eagerly."""
         B, BS = len(decode), self.kv.block_size
         if B > max(self.cfg.graph_batch_sizes) or len(set(id(s) for s, _ in decode)) != B or KNOBS.sync_debug:
             return None                        # (a capture has no room for the synchronisation behind every launch)
@@ -353,16 +355,18 @@ class GraphRunnerMixin:
         else:
             got[1].copy_(host, non_blocking=True)
         self._trace_mark()
-        graph, _, out, _ = got
+        graph, _, h, whole, _ = got
         graph.replay()
+        out = h.clone() if whole else self.model.logits(h)
         if sample_idx == list(range(B)):
-            return out.clone()
+            return out
         return out.index_select(0, torch.tensor(sample_idx, dtype=torch.long).pin_memory().to(self.device,
                                                                                               non_blocking=True))
 
     def _seg_capture(self, B: int, width: int, host: torch.Tensor) -> tuple:
-        """(graph, its static input holding ``host``, its logits [B, vocab], its step) of a step of ``B`` single tokens.  The
-        step is kept with the graph: every tensor in it is read by each replay, the row offsets too, which no copy fills."""
+        """(graph, its static input holding ``host``, what the model makes logits of -- or, where their product cannot be made
+        again and again, the logits [B, vocab] themselves and True --, its step) of a step of ``B`` single tokens.  The step is
+        kept with the graph: every tensor in it is read by each replay, the row offsets too, which no copy fills."""
         t0 = time.perf_counter()
         cur = torch.cuda.current_stream(self.device)
         flat = host.to(self.device, non_blocking=True)
@@ -388,7 +392,10 @@ class GraphRunnerMixin:
             with torch.cuda.stream(self._seg_stream):
                 graph.capture_begin(pool=self._seg_pool, capture_error_mode="thread_local")
                 try:
-                    out = self.model.forward(inp, *self.kv.tensors(), states)
+                    out = self.model.forward(inp, *self.kv.tensors(), states, head=False)
+                    whole = isinstance(out, RowStep)
+                    if whole:
+                        out = self.model.logits(out)
                 except BaseException:
                     self._seg.off = True           # until the capture has ended
                     with contextlib.suppress(RuntimeError):        # (the first error is the one to report)
@@ -404,4 +411,4 @@ class GraphRunnerMixin:
         cur.wait_stream(self._seg_stream)
         self.stats["captures"] += 1
         self.stats["capture_s"] += time.perf_counter() - t0
-        return graph, flat, out, inp
+        return graph, flat, out, whole, inp

@@ -403,10 +403,11 @@ class FikeraxModel:
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[Optional[torch.Tensor]],
                 vts: List[Optional[torch.Tensor]], states: Optional[Dict[str, torch.Tensor]] = None,
-                layers_out: Optional[list] = None) -> torch.Tensor:
+                layers_out: Optional[list] = None, head: bool = True):
         """Logits [len(logits_idx), vocab] fp32.  ``kcs`` / ``vcs`` / ``vts``: the paged keys (latent rows), values and
         transposed values (latents) of every run of an attention layer; ``states``: the per-slot tensors of
-        :meth:`state_spec`.  ``layers_out`` (debugging): receives the residual after every layer run."""
+        :meth:`state_spec`.  ``layers_out`` (debugging): receives the residual after every layer run.
+        Without ``head``: what :meth:`logits` makes them of."""
         cfg, eps, dt = self.cfg, self.cfg.norm_eps, self.dtype
         T, one = inp.input_ids.shape[0], self.one
         idx = S.wanted_rows(inp)
@@ -450,6 +451,9 @@ class FikeraxModel:
                 if y is not None:
                     N.hyper_step(x, y, one, mix1, rms=rms)
         h = R.rows(h, idx) if few else N.hyper_read(x, idx, self.final_norm, eps, dt)
+        return self.logits(h) if head else h
+
+    def logits(self, h) -> torch.Tensor:
         return R.proj_f32out(h, self.head)
 
 

@@ -416,10 +416,11 @@ class LizesunModel:
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[torch.Tensor],
                 vts: List[Optional[torch.Tensor]], states: Dict[str, torch.Tensor],
-                layers_out: Optional[list] = None) -> torch.Tensor:
+                layers_out: Optional[list] = None, head: bool = True):
         """Logits [len(logits_idx), vocab] fp32.  ``kcs`` / ``vcs``: the paged keys and values of every
         attention (``vts``: the values' transposed twins, or None); ``states``: the per-slot tensors of
-        :meth:`state_spec`.  ``layers_out`` (debugging): receives a copy of the residual after every layer."""
+        :meth:`state_spec`.  ``layers_out`` (debugging): receives a copy of the residual after every layer.
+        Without ``head``: what :meth:`logits` makes them of."""
         cfg, dt = self.cfg, self.dtype
         T, W, nl = inp.input_ids.shape[0], cfg.hidden, cfg.n_layers
         idx = S.wanted_rows(inp)
@@ -455,6 +456,9 @@ class LizesunModel:
         else:
             xr = x.index_select(0, idx).contiguous() if idx is not None else x
             h = N.add_dyt(xr, None, 1.0, None, 1.0, *self.final_norm, out_dtype=dt)
+        return self.logits(h) if head else h
+
+    def logits(self, h) -> torch.Tensor:
         return R.proj_f32out(h, self.lm_head)
 
 
