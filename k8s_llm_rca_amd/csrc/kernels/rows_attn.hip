@@ -10,7 +10,8 @@
 // spread over a workgroup per part: both do the same arithmetic, so a row's result does not depend on how the prompt was cut
 // or on what else is in the step.
 //
-// What bounds it: the scores -- lookups of the first-level cache, one for every key that four neighbouring lanes read -- and
+// What bounds it (prompts in fp32 with whole tiles go to rows_attn_mfma_kernel): the scores -- lookups of the first-level
+// cache, one for every key that four neighbouring lanes read -- and
 // latency at few rows, for which reason the heads and the parts are spread over workgroups.  622 rows of two prompts, 16
 // heads, 256 + 64 numbers and 2 key heads of 128, median of both: a lane a key, four keys in four lanes, 150 us; three
 // workgroups a compute unit by their registers and 16 values on their way 126; two lanes a key 106; four lanes a key, two
@@ -19,6 +20,7 @@
 // of two prompts: 1451 -> 122 us; latent (16 heads, 256 + 64 numbers): 706 -> 39 and 719 -> 196 us.
 #include "common.h"
 #include "key_runs.h"
+#include <type_traits>
 
 namespace k8s {
 
@@ -289,6 +291,205 @@ __global__ void __launch_bounds__(256, FEW ? 1 : 4) rows_attn_kernel(RowsArgs p)
   }
 }
 
+// The same sums on the matrix units, fp32 throughout, for workgroups that walk all parts of a row: 16 heads are the rows of a
+// tile, and its columns 16 keys, then 16 value columns.  A v_mfma_f32_16x16x4_f32 adds its four products one after the other,
+// each with the rounding of a multiply-add, so a score and a value are the chains of rows_attn_kernel, to the bit.
+// For that the four numbers of an instruction have to stand beside each other in the key: four lanes read 64 bytes of a key, so
+// that it is looked up once per 16 numbers, and lane swaps turn the 4 x 4 of them.  Queries and weights stand in LDS as the lanes
+// want them, four instructions' in 16 bytes.
+// What bounds it: the chain of a part (slots, keys, softmax, values) with four to five workgroups a compute unit to cover it;
+// matrix instructions are a third of the time (with 8 heads of a key half of each is empty).  us of rows_attn_kernel / here, 622
+// rows of two prompts: 16 heads, 256 + 64 numbers 116 / 59;  16 heads over 2 of 128 67 / 42, over 16 of 64 190 / 121.  The
+// next part's slots and the first 32 keys' values asked for in front of the scores: 65 -> 60 and 45 -> 42, 300 single rows at
+// 500 keys 119 -> 82.  Eight waves, a tile of keys each: 69 and 51 (fewer workgroups at once), and with half of them for the values 65 and 64.
+constexpr int kRmKeys = kRaKeys + 4;    // a head's weights in LDS: 16 heads' neighbours in 64 banks
+// Where entry or key i of 16 stands in LDS: the four of an instruction's lane behind each other.
+__device__ __forceinline__ int rm_at(int i) { return (i & ~15) | (i & 3) << 2 | (i >> 2 & 3); }
+
+__device__ __forceinline__ void rm_turn(float& a, float& b, bool far) {
+  const auto t = far ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
+                     : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(t[0]);
+  b = __uint_as_float(t[1]);
+}
+
+template <int NE>
+__global__ void __launch_bounds__(256, 4) rows_attn_mfma_kernel(RowsArgs p) {
+  using cols = float __attribute__((ext_vector_type(NE)));
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int D = p.D1 + p.D2, V = p.V, hpg = p.H / (p.G * p.M), nhb = (hpg + 15) / 16, D4 = D + 4;
+  constexpr int kAhead = 8;                         // times four keys: whose values are on their way together
+  const int nvb = V / (64 * NE);
+  float* sq = sm;                                   // [16][D4]
+  float* sp = sq + 16 * D4;                         // [16][kRmKeys]
+  float* sl = sp + 16 * kRmKeys;                    // [16][2]: m, l of the part
+  int* slots = reinterpret_cast<int*>(sl + 32);     // [2][128]: cache slots of this part and the next
+  const int r = p.row_base + blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c16 = lane & 15, kg = lane >> 4;
+  int gi = blockIdx.y;
+  const int vb = gi % nvb;
+  gi /= nvb;
+  const int hb = gi % nhb, gm = gi / nhb, g = gm / p.M;
+  const int nh = min(16, hpg - hb * 16);
+  auto head = [&](int i) { return (g * hpg + hb * 16 + i) * p.M + gm % p.M; };
+  const int sg = p.row_seg[r], pos = p.seg_pos0[sg] + r - p.seg_row0[sg];
+  const KeyRuns kr = key_runs(pos, p.chunk, p.window, p.keep_first);
+  const int* bt = p.bt + (size_t)sg * p.maxb;
+  auto slot = [&](int x) {                          // (past the last key: that one again)
+    const int j = kr.key(min(x, kr.total - 1));
+    return bt[j / p.BS] * p.BS + j % p.BS;
+  };
+  if (tid < kRaKeys) slots[tid] = slot(tid);
+  for (int i = tid; i < nh * D; i += 256) {
+    const int h = i / D, d = i - h * D;
+    sq[h * D4 + rm_at(d)] = d < p.D1 ? ((const float*)p.q)[(size_t)r * p.qst + (size_t)head(h) * p.qsh + d]
+                                     : p.q2[((size_t)r * p.H + head(h)) * p.D2 + d - p.D1];
+  }
+  const int col = (vb * 4 + wv) * 16 * NE + c16 * NE;
+  const float* kbase = (const float*)p.kc + (size_t)gm * D + 4 * kg;
+  const float* vbase = (const float*)p.vc + (size_t)g * V + col;
+  float m[4], l[4];                                 // of head 4 kg + i
+  f32x4 o[NE];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const bool on = 4 * kg + i < nh && p.sink;
+    m[i] = on ? p.sink[head(4 * kg + i)] : -INFINITY;
+    l[i] = on ? 1.f : 0.f;
+  }
+#pragma unroll
+  for (int e = 0; e < NE; ++e) o[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int x0 = 0, par = 0; x0 < kr.total; x0 += kRaKeys, par ^= 1) {
+    const int nk = min(kRaKeys, kr.total - x0);
+    const int* ss = slots + par * kRaKeys;
+    __syncthreads();                                // slots (and queries) are there, the part before is read no more
+    const int next = tid < kRaKeys && x0 + kRaKeys < kr.total ? slot(x0 + kRaKeys + tid) : 0;
+    cols v[kAhead];                               // the first values, asked for in front of the scores
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) v[u] = *reinterpret_cast<const cols*>(vbase + (size_t)ss[4 * u + kg] * p.vs);
+    {  // scores of keys 16 wv .. and 64 + 16 wv ..
+      f32x4 a[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      const int x = 16 * wv + c16;
+      const float* k0 = kbase + (size_t)ss[x] * p.ks;
+      const float* k1 = kbase + (size_t)ss[x + 64] * p.ks;
+      const float* qh = sq + c16 * D4 + 4 * kg;
+      auto tiles = [&](auto both) {
+        constexpr int NT = decltype(both)::value ? 2 : 1;
+#pragma unroll 4
+        for (int d = 0; d < D; d += 16) {
+          f32x4 t[NT];
+          t[0] = rld4(k0 + d);
+          if constexpr (NT == 2) t[1] = rld4(k1 + d);
+          const f32x4 qv = *reinterpret_cast<const f32x4*>(qh + d);
+#pragma unroll
+          for (int f = 0; f < NT; ++f) {
+            float t0 = t[f][0], t1 = t[f][1], t2 = t[f][2], t3 = t[f][3];
+            rm_turn(t0, t2, true);
+            rm_turn(t1, t3, true);
+            rm_turn(t0, t1, false);
+            rm_turn(t2, t3, false);
+            t[f] = f32x4{t0, t1, t2, t3};
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int f = 0; f < NT; ++f) a[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[e], t[f][e], a[f], 0, 0, 0);
+        }
+      };
+      if (64 + 16 * wv < nk)
+        tiles(std::true_type{});
+      else if (16 * wv < nk)
+        tiles(std::false_type{});
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float s = a[f][i] * p.scale;
+          if (p.softcap > 0.f) s = p.softcap * tanhf(s / p.softcap);
+          sp[(4 * kg + i) * kRmKeys + rm_at(x) + 64 * f] = x + 64 * f < nk ? s : -INFINITY;
+        }
+    }
+    if (tid < kRaKeys) slots[(par ^ 1) * kRaKeys + tid] = next;
+    __syncthreads();
+    for (int h = wv; h < nh; h += 4) {              // the part's softmax, a wave per head
+      float* w = sp + h * kRmKeys + rm_at(lane);
+      const float s0 = w[0], s1 = w[64];
+      const float mp = wave_max(fmaxf(s0, s1)), ms = mp == -INFINITY ? 0.f : mp;
+      const float e0 = expf(s0 - ms), e1 = expf(s1 - ms);
+      w[0] = e0;
+      w[64] = e1;
+      const float lp = wave_sum(e0 + e1);
+      if (lane == 0) {
+        sl[2 * h] = mp;
+        sl[2 * h + 1] = lp;
+      }
+    }
+    __syncthreads();
+    f32x4 op[NE];
+#pragma unroll
+    for (int e = 0; e < NE; ++e) op[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float* wp = sp + c16 * kRmKeys + 4 * kg;
+    f32x4 w;
+    for (int j0 = 0; j0 < nk; j0 += 4 * kAhead) {
+      if (j0) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) v[u] = *reinterpret_cast<const cols*>(vbase + (size_t)ss[j0 + 4 * u + kg] * p.vs);
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int j = j0 + 4 * u;
+        if (j >= nk) break;
+        if (u % 4 == 0) w = *reinterpret_cast<const f32x4*>(wp + j);
+#pragma unroll
+        for (int e = 0; e < NE; ++e)                // (weights past nk are zero, and zero times an infinity would be NaN)
+          op[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u % 4], j + kg < nk ? v[u][e] : 0.f, op[e], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int h = 4 * kg + i;
+      if (h < nh) {
+        float a, b;
+        ra_join(m[i], l[i], sl[2 * h], sl[2 * h + 1], a, b);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) o[e][i] = ra_join_out(o[e][i], a, op[e][i], b);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int h = 4 * kg + i;
+    if (h < nh) {
+      const int hh = head(h);
+      cols v;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        v[e] = o[e][i] / l[i];
+        if (p.gate) v[e] *= 1.f / (1.f + expf(-p.gate[(size_t)r * p.gs + hh]));
+      }
+      *reinterpret_cast<cols*>((float*)p.out + (size_t)r * p.ost + (size_t)hh * p.osh + col) = v;
+    }
+  }
+}
+
+// Wherever whole tiles of 16 entries and 64 value columns are read and written by 16 bytes, at any number of heads a key, most of
+// a tile empty or not: us of rows_attn_kernel / this at 622 rows, 64 entries, 1, 2, 4 heads a key 190 / 121, 102 / 71, 62 / 48;
+// latent, 1 head of 64 + 16 31 / 19, 3 of 256 + 64 61 / 50, 40 of 512 + 64 (329 rows) 251 / 159;  one row at 100 keys, 16
+// heads over 2 of 128 17.6 / 11.7, latent 27 / 21.
+static bool rows_mfma_ok(const RowsArgs& p) {
+  const int D = p.D1 + p.D2;
+  return !p.po && D % 16 == 0 && D <= 1024 && p.V % 64 == 0 && p.ks % 4 == 0 && p.vs % 4 == 0 &&
+         p.ost % 4 == 0 && p.osh % 4 == 0 && (((uintptr_t)p.kc | (uintptr_t)p.vc | (uintptr_t)p.out) & 15) == 0;
+}
+
+static int launch_rows_mfma(const RowsArgs& p, int T, hipStream_t s) {
+  const int hpg = p.H / (p.G * p.M), ne = p.V % 256 == 0 ? 4 : p.V % 128 == 0 ? 2 : 1;
+  const size_t lds = sizeof(float) * (16 * ((size_t)p.D1 + p.D2 + 4) + 16 * kRmKeys + 32 + 2 * kRaKeys);
+  auto k = ne == 4 ? rows_attn_mfma_kernel<4> : ne == 2 ? rows_attn_mfma_kernel<2> : rows_attn_mfma_kernel<1>;
+  if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
+    return (int)hipGetLastError();
+  hipLaunchKernelGGL(k, dim3(T, p.G * p.M * ((hpg + 15) / 16) * (p.V / (64 * ne))), dim3(256), lds, s, p);
+  return (int)hipGetLastError();
+}
+
 // joins the parts of a (row, head) in order
 template <typename TO>
 __global__ void __launch_bounds__(256) rows_attn_merge_kernel(RowsArgs p) {
@@ -311,6 +512,7 @@ __global__ void __launch_bounds__(256) rows_attn_merge_kernel(RowsArgs p) {
 
 template <typename TQ, typename TC, typename TO>
 static int launch_rows(const RowsArgs& p, int T, hipStream_t s) {
+  if (sizeof(TQ) == 4 && sizeof(TC) == 4 && sizeof(TO) == 4 && rows_mfma_ok(p)) return launch_rows_mfma(p, T, s);
   const int D = p.D1 + p.D2, hpg = p.H / (p.G * p.M), z = p.po ? p.n_parts : 1;
   auto groups = [&](int most) { return p.G * p.M * ((hpg + most - 1) / most) * ((p.V + 255) / 256); };
   const bool few = p.po && (long)T * groups(kRaFew) * z <= (sizeof(TC) == 4 ? 512 : 256);
