@@ -430,13 +430,22 @@ template <>
 __device__ __forceinline__ float act_silu<float>(float z) { return silu_f(z); }
 template <>
 __device__ __forceinline__ float act_silu<uint16_t>(float z) { return bf2f(f2bf(silu_hw(z))); }
+__device__ __forceinline__ f32x4 ldm4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ f32x4 ldm4(const uint16_t* p) {
+  const u16x4 v = *reinterpret_cast<const u16x4*>(p);
+  return f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
+}
 constexpr int kRetTb = 16;    // tokens per batch
 // MODE 0: blockIdx.x = segment, from the slot's state (or zero at position 0) to the slot's state.
 // Long segments are cut into chunks ([n][4]: segment, first row, rows, -) that run in parallel:
 // MODE 1: a chunk from a zero state, its end state goes to cs [chunks][H][D][V], no output;
 // (retention_carry_kernel then turns cs into every chunk's START state and advances the slot's state)
 // MODE 2: the chunk again from its start state, writing o.
-template <int DPT, int MODE, typename TA, bool SILU>
+// FULL: D = DPT NDG, every thread has DPT entries, which it reads from LDS by 16 bytes and without a question each; rows are read
+// by 16 bytes where they allow it.  Bound by LDS reads (a key's and a query's entry for every product) and by instructions.
+// us, both passes and the carry, 16 heads of 128 x 128, 622 fp32 rows of two prompts with SILU: 153 -> 140 (reads, no queries in
+// MODE 1) -> 98 (FULL); 8 of 64 x 64 80 -> 45; two of 7 rows 11.6 -> 6.3; bf16, 96 x 128 (not FULL) 134 -> 125.
+template <int DPT, int MODE, typename TA, bool SILU, bool FULL>
 __global__ void __launch_bounds__(256) retention_scan_kernel(const TA* __restrict__ qkvg, int qs,
                                                              const float* __restrict__ decay, float* __restrict__ state,
                                                              const int* __restrict__ seg_row0,
@@ -444,7 +453,7 @@ __global__ void __launch_bounds__(256) retention_scan_kernel(const TA* __restric
                                                              const int* __restrict__ seg_slot, float* __restrict__ oraw,
                                                              int H, int D, int V, int VBS,
                                                              const int* __restrict__ chunks, float* __restrict__ cs) {
-  extern __shared__ float sm[];
+  extern __shared__ __attribute__((aligned(16))) float sm[];
   const int it = blockIdx.x, hh = blockIdx.y, v0 = blockIdx.z * VBS, tid = threadIdx.x;
   const int NDG = 256 / VBS;
   float* sq = sm;                          // [TB][D]
@@ -468,26 +477,44 @@ __global__ void __launch_bounds__(256) retention_scan_kernel(const TA* __restric
     st = cs + ((size_t)it * H + hh) * D * V + v0;
   }
   const float dec = decay[hh];
+  const bool vec = ((D | V | VBS | qs) & 3) == 0 && ((uintptr_t)qkvg & (4 * sizeof(TA) - 1)) == 0;
   float S[DPT];
 #pragma unroll
   for (int i = 0; i < DPT; ++i) {
     const int d = dg * DPT + i;
-    S[i] = (own && d < D && !fresh) ? st[(size_t)d * V + v] : 0.f;
+    S[i] = (own && (FULL || d < D) && !fresh) ? st[(size_t)d * V + v] : 0.f;
   }
   for (int t0 = r0; t0 < r1; t0 += kRetTb) {
     const int nb = min(kRetTb, r1 - t0);
     __syncthreads();
-    for (int e = tid; e < nb * D; e += 256) {
-      const int tb = e / D, d = e - tb * D;
-      const size_t row = (size_t)(t0 + tb) * qs;
-      const float qv = ldm(qkvg, row + hh * D + d), kv = ldm(qkvg, row + (H + hh) * D + d);
-      sq[e] = SILU ? act_silu<TA>(qv) : qv;
-      sk[e] = SILU ? act_silu<TA>(kv) : kv;
-    }
-    for (int e = tid; e < nb * VBS; e += 256) {
-      const int tb = e / VBS, vv = e - tb * VBS;
-      const float xv = v0 + vv < V ? ldm(qkvg, (size_t)(t0 + tb) * qs + 2 * H * D + hh * V + v0 + vv) : 0.f;
-      sv[e] = SILU ? act_silu<TA>(xv) : xv;
+    auto act = [](float z) { return SILU ? act_silu<TA>(z) : z; };
+    auto act4 = [&](const TA* x) {
+      const f32x4 z = ldm4(x);
+      return f32x4{act(z[0]), act(z[1]), act(z[2]), act(z[3])};
+    };
+    if (vec) {                                           // (MODE 1 needs no queries)
+      for (int e = 4 * tid; e < nb * D; e += 1024) {
+        const int tb = e / D, d = e - tb * D;
+        const TA* row = qkvg + (size_t)(t0 + tb) * qs + hh * D + d;
+        if (MODE != 1) *reinterpret_cast<f32x4*>(sq + e) = act4(row);
+        *reinterpret_cast<f32x4*>(sk + e) = act4(row + H * D);
+      }
+      for (int e = 4 * tid; e < nb * VBS; e += 1024) {
+        const int tb = e / VBS, vv = e - tb * VBS;
+        *reinterpret_cast<f32x4*>(sv + e) = v0 + vv < V ? act4(qkvg + (size_t)(t0 + tb) * qs + 2 * H * D + hh * V + v0 + vv)
+                                                        : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    } else {
+      for (int e = tid; e < nb * D; e += 256) {
+        const int tb = e / D, d = e - tb * D;
+        const size_t row = (size_t)(t0 + tb) * qs;
+        if (MODE != 1) sq[e] = act(ldm(qkvg, row + hh * D + d));
+        sk[e] = act(ldm(qkvg, row + (H + hh) * D + d));
+      }
+      for (int e = tid; e < nb * VBS; e += 256) {
+        const int tb = e / VBS, vv = e - tb * VBS;
+        sv[e] = act(v0 + vv < V ? ldm(qkvg, (size_t)(t0 + tb) * qs + 2 * H * D + hh * V + v0 + vv) : 0.f);
+      }
     }
     __syncthreads();
     if (dg < NDG) {
@@ -499,7 +526,7 @@ __global__ void __launch_bounds__(256) retention_scan_kernel(const TA* __restric
 #pragma unroll
         for (int i = 0; i < DPT; ++i) {
           const int d = dg * DPT + i;
-          if (d < D) {
+          if (FULL || d < D) {
             S[i] = fmaf(dec, S[i], kq[d] * vv);
             if (MODE != 1) acc = fmaf(S[i], qq[d], acc);
           }
@@ -523,7 +550,7 @@ __global__ void __launch_bounds__(256) retention_scan_kernel(const TA* __restric
 #pragma unroll
     for (int i = 0; i < DPT; ++i) {
       const int d = dg * DPT + i;
-      if (own && d < D) st[(size_t)d * V + v] = S[i];
+      if (own && (FULL || d < D)) st[(size_t)d * V + v] = S[i];
     }
   }
 }
@@ -711,7 +738,7 @@ static int launch_decay_scan(const TA* x, int xs, const float* decay, float* sta
   const int vb = (V + VBS - 1) / VBS;
 #define K8S_RET_M(DP, MODE, items)                                                                              \
   {                                                                                                             \
-    auto k = retention_scan_kernel<DP, MODE, TA, SILU>;                                                         \
+    auto k = D == DP * NDG ? retention_scan_kernel<DP, MODE, TA, SILU, true> : retention_scan_kernel<DP, MODE, TA, SILU, false>; \
     if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)) \
       return (int)hipGetLastError();                                                                            \
     hipLaunchKernelGGL(k, dim3(items, H, vb), dim3(256), lds, s, x, xs, decay, state, seg_row0, seg_pos0,       \
