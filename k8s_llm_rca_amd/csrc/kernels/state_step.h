@@ -1,5 +1,6 @@
 // One token per sequence through a matrix state, with what stands around it: the reply steps of the gated delta rule and the
-// matrix memory (matrix_mem.hip) and of the decaying linear attention (mixer_ops.hip), same arithmetic, in one launch each.
+// matrix memory (matrix_mem.hip) and of the decaying linear attention (mixer_ops.hip), same arithmetic, in one launch each
+// (state_step.hip) or, of the matrix memory, in further workgroups of the attention beside it (token_attn.hip).
 //
 // KIND 0, delta rule:  q, k to unit length, decays and beta from their gates,  S <- g S;  u = beta (v - S^T k);
 //   S <- S + k u^T;  o = S^T q,  then the head's norm, its weight and the output gate.
@@ -9,7 +10,7 @@
 //   The norm spans all heads, which no workgroup sees: the sum of squares of every head goes to ssp, and
 //   whoever adds the output projection to the residual divides by the root mean square (the factor is one per row).
 //
-// A workgroup has a head of one sequence (V = 4 LV, D = DR RG); a thread four neighbouring columns of DR rows RG apart, so a
+// A workgroup has a head of one sequence (V = 4 LV, D = DR RG), or of KIND 2 a slice of its columns; a thread four neighbouring columns of DR rows RG apart, so a
 // wave's accesses to the state are whole lines.  Nothing waits for anything but the state's address: rows,
 // gates and state are asked for together.  What bounds it: the state's bytes, read and written once (64 KB a head), and
 // for few sequences that one compute unit takes 20 to 30 KB a us.

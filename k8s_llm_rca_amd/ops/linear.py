@@ -423,8 +423,8 @@ def stream_f32_cfg(M: int, N: int, K: int) -> int:
 
 
 def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x @ w.T`` with an fp32 result: bf16 operands with fp32 accumulation (the weight-streaming kernel for a few rows,
-    hipBLASLt otherwise), or fp32 throughout."""
+    """``x @ w.T`` with an fp32 result: bf16 operands with fp32 accumulation (the weight-streaming kernels for up to 64
+    rows, hipBLASLt otherwise), or fp32 throughout."""
     if not x.is_cuda or x.dtype != torch.bfloat16:
         return linear(x, w)
     M, K = x.shape

@@ -1,10 +1,12 @@
-"""A residual's pass that is not made yet, for the product that stands behind it (csrc/kernels/gemm_row_step.hip).
+"""A residual's pass without a launch of its own: in a reply chain each costs 3 to 4 us in which the chip waits.
 
-With one row the pass (:func:`..ops.norm.hyper_step` with one stream, :func:`..ops.norm.add_dyt`) is a launch of 3 to 4 us
-in which the chip waits; the kernel makes the row in every workgroup of the product instead, under the weights' way from
-memory.  A model asks for its next sublayer's input with :func:`step` / :func:`dyt_step`, which return either the activations
-(the residual updated in place) or a :class:`RowStep`; the products below take both, and :func:`residual` says where the
-residual is afterwards."""
+Up to 16 rows (fp32: four) a sublayer's last product takes the pass into its epilogue (:func:`add_product`,
+:func:`dyt_product`; csrc/kernels/gemm_step.hip, few_rows_f32.hip): what is behind it then gets the activations, or a
+:class:`Scaled`, whose rows the next product divides by their root mean square.  Where that does not pay and there is one row,
+the next product makes the pass in every workgroup instead, under the weights' way from memory (:func:`step`,
+:func:`dyt_step`, :class:`RowStep`; csrc/kernels/gemm_row_step.hip).  Otherwise it is the launch it was
+(:func:`..ops.norm.hyper_step`, :func:`..ops.norm.add_dyt`).  The products below take any of the three, and
+:func:`residual` says where the residual is afterwards."""
 from typing import Optional
 
 import torch
