@@ -533,12 +533,16 @@ ROWS_SCRATCH = 1 << 28      # floats of partial results past which it does so as
 
 
 def _rows_parts(seg: SegMeta, T: int, heads: int, per_key: int, V: int, dev, chunk: int = 0, window: int = 0,
-                keep_first: int = 0) -> tuple:
+                keep_first: int = 0, tiles: bool = False) -> tuple:
     """(parts, scratch for their outputs, for their maxima and sums) of a step of the vector-pipe attention whose rows do
     not fill the chip: a workgroup per part of a row's keys, the same sums either way.  (0, None, None): a workgroup per
     row and group of heads.  One workgroup -> parts, us, fp32, 16 heads over 2 of 128: 2 rows at 340 keys 55 -> 27, 16 at
     1024 visible ones 148 -> 28, 128 at 300 68 -> 52, 256 at 400 113 -> 118 (the line; past it the parts save a tenth at
-    most and write heads x parts results per row).  ``per_key``: heads that share a key."""
+    most and write heads x parts results per row).  ``per_key``: heads that share a key.
+
+    ``tiles``: the one workgroup uses matrix instructions (whole tiles in fp32), so that with two parts at most half of that
+    fills the chip: the same at 128 rows of 150, 200 of 200, 250 of 250 keys 21 / 26, 22 / 26, 25 / 31, latent 256 + 64 numbers 34 /
+    38, 33 / 42, 35 / 52;  three parts, 128 rows of 300 32 / 31, 53 / 47;  fewer rows, 64 of 300 31 / 26, 50 / 38."""
     groups = heads // per_key * -(-per_key // ROWS_HEADS) * -(-V // 256)
     if T * groups >= ROWS_FILL:
         return 0, None, None
@@ -548,7 +552,8 @@ def _rows_parts(seg: SegMeta, T: int, heads: int, per_key: int, V: int, dev, chu
     if window > 0:
         most = min(most, window + keep_first)
     parts = -(-most // ROWS_PART)
-    if parts <= 1 or T * heads * parts * (V + 2) > ROWS_SCRATCH:
+    if (parts <= 1 or T * heads * parts * (V + 2) > ROWS_SCRATCH
+            or tiles and parts <= 2 and T * groups >= ROWS_FILL // 2):
         return 0, None, None
     return (parts, scratch(T * heads * parts * V, torch.float32, dev), scratch(T * heads * parts * 2, torch.float32, dev))
 
@@ -637,7 +642,8 @@ def latent_attention(qa: torch.Tensor, cache: torch.Tensor, gate: Optional[torch
         assert qr is None or (qr.dtype == torch.float32 and qr.is_contiguous() and qr.shape == (T, H, W - R))
         assert sink is None or (sink.dtype == torch.float32 and sink.numel() == H)
         assert seg.block_tables.is_contiguous()
-        parts, po, pml = _rows_parts(seg, T, H, H, R, qa.device, window=int(window))
+        parts, po, pml = _rows_parts(seg, T, H, H, R, qa.device, window=int(window),
+                                     tiles=cache.dtype == torch.float32 and cache.shape[-1] % 16 == 0 == R % 64)
         check(lib().k8s_latent_attn_rows(ptr(qa), ptr(cache), ptr(seg.block_tables), seg.block_tables.shape[1],
                                          ptr(seg.row_seg), ptr(seg.seg_row0), ptr(seg.seg_pos0), ptr(gate),
                                          gate.stride(0) if gate is not None else 0, ptr(out), 0, T, H, R, BS,
@@ -1347,7 +1353,8 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
                                                    ptr(pml)), "masked_attn_prompt")
             return out
         assert vc is not None          # the vector-pipe kernel reads token-major values
-        parts, po, pml = _rows_parts(seg, T, HQ, H // G, V, q.device, int(chunk), int(window), int(keep_first))
+        parts, po, pml = _rows_parts(seg, T, HQ, H // G, V, q.device, int(chunk), int(window), int(keep_first),
+                                     tiles=q.dtype == torch.float32 and D % 16 == 0 == V % 64)
         check(lib().k8s_masked_attn_rows(ptr(q), ptr(kc), ptr(vc), ptr(seg.block_tables), seg.block_tables.shape[1],
                                          ptr(seg.row_seg), ptr(seg.seg_row0), ptr(seg.seg_pos0), ptr(sink), ptr(gate),
                                          gs, ptr(out), T, H, G, D, V, BS, int(chunk), int(window), int(keep_first),
