@@ -301,8 +301,10 @@ __global__ void __launch_bounds__(256, FEW ? 1 : 4) rows_attn_kernel(RowsArgs p)
 // matrix instructions are a third of the time (with 8 heads of a key half of each is empty).  us of rows_attn_kernel / here, 622
 // rows of two prompts: 16 heads, 256 + 64 numbers 116 / 59;  16 heads over 2 of 128 67 / 42, over 16 of 64 190 / 121.  The
 // next part's slots and the first 32 keys' values asked for in front of the scores: 65 -> 60 and 45 -> 42, 300 single rows at
-// 500 keys 119 -> 82.  Eight waves, a tile of keys each: 69 and 51 (fewer workgroups at once), and with half of them for the values 65 and 64.
+// 500 keys 119 -> 82.  Eight waves, a tile of keys each: 69 and 51 (fewer workgroups at once), and with half of them for
+// the values 65 and 64.
 constexpr int kRmKeys = kRaKeys + 4;    // a head's weights in LDS: 16 heads' neighbours in 64 banks
+
 // Where entry or key i of 16 stands in LDS: the four of an instruction's lane behind each other.
 __device__ __forceinline__ int rm_at(int i) { return (i & ~15) | (i & 3) << 2 | (i >> 2 & 3); }
 

@@ -229,8 +229,8 @@ def _into_f32(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:
     42.9, 48.1 / 46.5;  2048 x 8192, 8192 x 2048 27.7 / 25.3, 28.9 / 25.5, 31.7 / 29.9, 34.4 / 36.0, 36.7 / 36.3;  512 x 2048, 1536 x
     512 9.5 / 7.8, 9.9 / 8.1, 10.8 / 9.1, 11.9 / 10.0, 12.3 / 10.5;  4096 x 4096, 8192 x 4096 37.5 / 35.1, 40.0 / 38.3, 44.9 / 42.2,
     47.7 / 49.4, 52.9 / 53.1."""
-    return (a.shape[0] <= INTO_F32_ROWS and L._few_f32_ok(a, w) and x.dtype == torch.float32 and x.is_contiguous() and w.shape[0] == x.shape[-1]
-            and w.device == x.device == a.device and w.shape[0] % 16 == 0 and w.shape[0] <= 4096)
+    return (a.shape[0] <= INTO_F32_ROWS and L._few_f32_ok(a, w) and x.dtype == torch.float32 and x.is_contiguous()
+            and w.shape[0] == x.shape[-1] and w.device == x.device == a.device and w.shape[0] % 16 == 0 and w.shape[0] <= 4096)
 
 
 def add_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, one: torch.Tensor, mix: torch.Tensor, nw: torch.Tensor,

@@ -1847,7 +1847,8 @@ def delta_low_rank(qkv: torch.Tensor, H: int, G: int, D: int, V: int, lr: torch.
     12.3 / 11.4."""
     ra, rg, T = wa.shape[1], wg.shape[1], qkv.shape[0]
     mine = wa.shape[0] // H * ra + wg.shape[0] // H * rg
-    if (0 < T * H * mine <= DELTA_LOW_ALL and mine <= DELTA_LOW_HEAD and qkv.dtype == torch.bfloat16 == out_dtype and _small_rows(qkv, wa) and _small_rows(qkv, wg)
+    if (0 < T * H * mine <= DELTA_LOW_ALL and mine <= DELTA_LOW_HEAD and qkv.dtype == torch.bfloat16 == out_dtype
+            and _small_rows(qkv, wa) and _small_rows(qkv, wg)
             and all(32 <= k <= DELTA_LOW_RANK and k % 32 == 0 and t.data_ptr() % 16 == 0 for k, t in ((ra, wa), (rg, wg)))
             and _step_ok(qkv, seg, D, V, state, qkv, w) and qkv.is_contiguous() and lr.dtype == torch.float32
             and lr.stride(1) == 1 and lr.shape == (T, ra + rg + H)):
