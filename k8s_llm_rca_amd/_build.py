@@ -97,6 +97,13 @@ def hip_sources() -> List[str]:
     return sorted(glob.glob(os.path.join(CSRC, "kernels", "*.hip")))
 
 
+def hip_flags() -> List[str]:
+    return ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-munsafe-fp-atomics",
+            "-ffp-contract=fast", "-I", os.path.join(CSRC, "kernels"),
+            # no packed fp32 arithmetic (v_pk_add / mul / fma_f32): scalar forms only
+            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+
+
 def build_hip(force: bool = False, jobs: int = 8) -> str:
     """Compile every kernel TU to an object (in parallel) and link one .so."""
     srcs = hip_sources()
@@ -104,10 +111,7 @@ def build_hip(force: bool = False, jobs: int = 8) -> str:
     out = hip_lib_path()
     objdir = os.path.join(PKG, "csrc", "build")
     os.makedirs(objdir, exist_ok=True)
-    flags = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-munsafe-fp-atomics",
-             "-ffp-contract=fast", "-I", os.path.join(CSRC, "kernels"),
-             # no packed fp32 arithmetic (v_pk_add / mul / fma_f32): scalar forms only
-             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+    flags = hip_flags()
     procs = []
     objs = []
     for s in srcs:

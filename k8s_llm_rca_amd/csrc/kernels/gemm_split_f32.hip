@@ -94,11 +94,12 @@ __device__ __attribute__((noinline)) float fp32_dot(const uint16_t* xpl, const f
   return t;
 }
 
-// grid: (row tiles x column tiles, K ranges)
+// grid: (row tiles x column tiles, K ranges).  The end of a step counts the loads behind its own into LDS, so their order is
+// fixed: no pointer here is __restrict__, since loads through such a one may pass any clobber (tests/test_split_f32_waits.py
+// reads the assembly).
 template <int MT, int OUT>
 __global__ void __launch_bounds__(256, 2)
-    gemm_split_f32_kernel(const uint16_t* __restrict__ xpl, const float* __restrict__ w, float* __restrict__ y, int M, int N,
-                          int K, int n_mt, int n_nt) {
+    gemm_split_f32_kernel(const uint16_t* xpl, const float* w, float* y, int M, int N, int K, int n_mt, int n_nt) {
   constexpr int BM = 16 * MT, ND = 3 * MT, PER = (ND + 3) / 4;    // LDS-DMA instructions of a step, of a wave
   __shared__ __attribute__((aligned(1024))) uint16_t xs[2][3][BM * kSfK];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
@@ -179,12 +180,16 @@ __global__ void __launch_bounds__(256, 2)
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto fence = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
   load_w(0);
   load_x(0, 0);
   take_any(wf);
-  load_w(min(1, steps - 1));
-  asm volatile("s_waitcnt vmcnt(4)" ::: "memory");                // X of step 0
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // X of step 0
   bar();
+  load_w(min(1, steps - 1));
   // two rows of fragments: 24 matrix instructions
   auto multiply = [&](int buf, int i) {
     bf16x8 xf[2][3];
@@ -205,18 +210,23 @@ __global__ void __launch_bounds__(256, 2)
   for (int s = 0; s < steps; ++s) {                               // (the last step loads and splits what it has once more, unread)
     const int buf = s & 1;
     constexpr int H = MT / 4 * 2;
+    fence();
     load_x(min(s + 1, steps - 1), buf ^ 1);
+    fence();
 #pragma unroll
     for (int i = 0; i < H; i += 2) multiply(buf, i);
     bf16x8 nf[2][3];
     take_any(nf);
-    load_w(min(s + 2, steps - 1));
+    fence();
+    load_w(min(s + 2, steps - 1));                                // four loads: what the wait below leaves on its way
+    fence();
 #pragma unroll
     for (int i = H; i < MT; i += 2) multiply(buf, i);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int p = 0; p < 3; ++p) wf[j][p] = nf[j][p];
+    fence();
     asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");   // the next step's X; this step's fragments are read
     bar();
   }
