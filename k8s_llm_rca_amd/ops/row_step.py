@@ -187,6 +187,7 @@ class Scaled:
         return N.hyper_read(self.x, None, self.nw, self.eps, self.h.dtype) if self.h.shape[0] else self.h
 
     def rows(self, idx: torch.Tensor) -> "Scaled":
+        """Some rows, which may be more than there are (one wanted several times)."""
         return Scaled(*(t.index_select(0, idx) for t in (self.x, self.h, self.part)), self.nw, self.eps)
 
     def product(self, w: torch.Tensor, out_kind: int, plain, planes: bool = False, keep: bool = False):
@@ -196,7 +197,7 @@ class Scaled:
         if (out_kind == L.ROWS_RELU2 or keep or k != w.shape[1] or w.shape[0] % 2 and out_kind == L.ROWS_SILU
                 or not L.rows_ok(self.h, w) or (("silu", w.shape[0], k) in L.dispatch_table()) or (n, k) in L.dispatch_table()):
             return plain(self.read(), w)
-        p = L.rows_plan(m, n, k, out_kind, planes)
+        p = L.rows_plan(m, n, k, out_kind, planes) if m <= INTO_ROWS else None
         if p is None:
             return plain(self.read(), w)
         out = torch.empty((p[1], m, n) if planes else (m, n), device=w.device,
@@ -207,7 +208,8 @@ class Scaled:
 
     def _product_f32(self, w: torch.Tensor, out_kind: int, plain, planes: bool):
         glu = out_kind == L.ROWS_SILU
-        if out_kind == L.ROWS_RELU2 or glu and w.shape[0] % 2 or not L._few_f32_ok(self.h, w):
+        if (out_kind == L.ROWS_RELU2 or glu and w.shape[0] % 2 or self.h.shape[0] > INTO_F32_ROWS
+                or not L._few_f32_ok(self.h, w)):
             return plain(self.read(), w)
         (m, k), n = self.h.shape, w.shape[0] // (2 if glu else 1)
         out = torch.empty((1, m, n) if planes else (m, n), dtype=torch.float32, device=w.device)
