@@ -316,11 +316,20 @@ class LLMEngine(SchedulerMixin, StepExecMixin, GraphRunnerMixin, SamplerMixin):
                top_k: int = 0, top_p: float = 1.0) -> None:
         """Set sequence ``sid``'s desired token list (prompt) and generate a reply
         (``top_k`` <= 0 and ``top_p`` >= 1 disable those filters)."""
+        tokens = self._ids(tokens)
         with self._cv:
-            self._incoming.append((sid, list(tokens), grammar, max_new,
+            self._incoming.append((sid, tokens, grammar, max_new,
                                    self.cfg.temperature if temperature is None else temperature, seed, on_done,
                                    top_k, top_p))
             self._cv.notify()
+
+    def _ids(self, tokens) -> List[int]:
+        """``tokens`` as a list of ids that the embedding has.  The kernels that look rows up have no way to refuse one, and what
+        they made of it would stand in the sequence's pages."""
+        ids, rows = list(map(int, tokens)), self.model.embed.shape[0]
+        if ids and not 0 <= min(ids) <= max(ids) < rows:
+            raise IndexError(f"token id {min(ids) if min(ids) < 0 else max(ids)} is outside the embedding's {rows} rows")
+        return ids
 
     def cancel(self, sid: int) -> None:
         """Cancel sequence ``sid``'s active request (thread-safe): its run fails

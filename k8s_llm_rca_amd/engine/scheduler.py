@@ -330,6 +330,7 @@ class SchedulerMixin:
             raise RuntimeError("feed() while a sampled step is in flight")
         if self._releases:
             self._apply_releases()
+        entries = [(sid, self._ids(toks), want) for sid, toks, want in entries]
         with self._lock:
             seqs = [self.seqs[sid] for sid, _, _ in entries]
         protect = set(s.id for s in seqs)
@@ -340,7 +341,7 @@ class SchedulerMixin:
                 raise ValueError("an entry without tokens")
             if s.n_cached != len(s.tokens):
                 raise RuntimeError(f"sequence {s.id} has tokens that were never run")
-            s.tokens.extend(int(t) for t in toks)
+            s.tokens.extend(toks)
             q = len(toks)
             if len(s.tokens) > self.kv.num_blocks * BS or not self.kvm.ensure_blocks(s, s.n_cached + q, protect):
                 raise MemoryError("KV pool exhausted")
