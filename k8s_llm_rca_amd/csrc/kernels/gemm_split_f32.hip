@@ -9,11 +9,12 @@
 //
 // X is split once, by a pass of its own, into three planes of bf16 (every column tile reads it).  A workgroup of four waves makes
 // 16 MT x 128 outputs, each wave 32 columns of all rows, K in steps of 32: X's planes go straight into LDS (16 rows x 64 bytes
-// an instruction, as the fragments are read: no bank conflict), two buffers of them; no wave shares its columns, so that W is
-// read in fragment order and split in registers, half a step's matrix instructions after it has come and a step's after it
-// was asked for.  Two workgroups share a compute unit.  The tiles of one panel of the larger operand
-// follow each other on one XCD.  Few tiles:
-// K in ranges, whose sums (planes) the consumer adds.
+// an instruction, as the fragments are read: no bank conflict), two buffers of them, a step ahead; no wave shares its columns, so
+// that W is read in fragment order and split in registers: asked for between the halves of a step's matrix instructions,
+// waited for in front of the next step's loads into LDS (so that no wait is for those: us without / so at 622 rows, ten
+// fragments, 16384 x 2048 203 / 196, 8192 x 2048 136 / 116, 2048 x 8192 in four ranges 136 / 117), split between that step's
+// halves.  Two workgroups share a compute unit.  The tiles of one panel of the larger operand follow each other on one XCD.
+// Few tiles: K in ranges, whose sums (planes) the consumer adds.
 //
 // What bounds it: the power (1.8 GHz at a bf16 rate of 1.1 PFLOP/s) and, where there are few workgroups, a step's chain (1.2 us
 // with four fragments, 2.0 with ten).  us, the library / the pass and this, out of memory:  16384 x 2048 at 333, 622, 1024 rows
@@ -210,6 +211,9 @@ __global__ void __launch_bounds__(256, 2)
   for (int s = 0; s < steps; ++s) {                               // (the last step loads and splits what it has once more, unread)
     const int buf = s & 1;
     constexpr int H = MT / 4 * 2;
+    // W of the next step has come before the loads into LDS are asked for: with these on their way the compiler waits for all
+    // loads where it needs one
+    asm volatile("" : "+v"(wq[0][0]), "+v"(wq[0][1]), "+v"(wq[1][0]), "+v"(wq[1][1])::"memory");
     fence();
     load_x(min(s + 1, steps - 1), buf ^ 1);
     fence();

@@ -37,27 +37,44 @@ def _blocks(lines):
 def unwaited(lines):
     """Barriers (block, index) that may be reached with a load into LDS on its way.  Followed through the function: the least
     number of memory instructions issued behind the last such load; a wait for that many or fewer ends it."""
+    return _follow(lines)[0]
+
+
+def overlap(lines):
+    """The least number of matrix instructions issued between a load into LDS that stands behind a barrier and its wait."""
+    return min(_follow(lines)[1], default=None)
+
+
+def _follow(lines):
     blocks = _blocks(lines)
-    state, todo, bad = {0: NONE}, [0], set()
+    state, todo, bad, between = {0: (NONE, 0, 0)}, [0], set(), {}
     while todo:
         i = todo.pop()
-        behind = state[i]
+        behind, matrix, met = state[i]             # memory and matrix instructions since the last load into LDS; barriers
         for k, text in enumerate(blocks[i][0]):
             op = text.split()[0]
             wait = re.search(r"vmcnt\((\d+)\)", text)
             if "load_lds" in op or (op.startswith("buffer_load") and " lds" in text):
-                behind = 0
+                behind, matrix = 0, 0
             elif op.startswith(("global_", "buffer_", "flat_", "scratch_")) and behind != NONE:
                 behind += 1
+            elif op.startswith("v_mfma") and behind != NONE:
+                matrix += 1
             elif op == "s_waitcnt" and wait and int(wait.group(1)) <= behind:
+                if behind != NONE and met:
+                    between[i, k] = min(matrix, between.get((i, k), matrix))
                 behind = NONE
-            elif op in ("s_barrier", "s_endpgm") and behind != NONE:
-                bad.add((i, k))
+            elif op in ("s_barrier", "s_endpgm"):
+                if behind != NONE:
+                    bad.add((i, k))
+                met = 1
         for j in blocks[i][1]:
-            if behind < state.get(j, NONE + 1):
-                state[j] = behind
+            old = state.get(j, (NONE + 1, NONE, 1))
+            new = (min(behind, old[0]), min(matrix if behind != NONE else NONE, old[1]), min(met, old[2]))
+            if new != old:
+                state[j] = new
                 todo.append(j)
-    return bad
+    return bad, list(between.values())
 
 
 def test_reading():
@@ -71,6 +88,7 @@ def test_reading():
     loop = "{0}\n.LBB0_1:\ns_waitcnt vmcnt({1})\ns_barrier\n{2}\ns_cbranch_scc1 .LBB0_1\n" + end
     assert not f(loop.format(f"{dma}\n{load}", 1, f"{dma}\n{load}"))
     assert f(loop.format(f"{dma}\n{load}", 1, f"{load}\n{dma}"))          # by the way back only
+    assert overlap(loop.format(dma, 0, f"{dma}\nv_mfma_f32 v0\nv_mfma_f32 v0").split("\n")) == 2
     assert f(f"{dma}\ns_cbranch_scc0 .LBB0_1\n{load}\n.LBB0_1:\ns_waitcnt vmcnt(1)\ns_barrier\n{end}")
 
 
@@ -83,5 +101,7 @@ def test_waits_cover_the_loads(tmp_path):
     assert len(kernels) == 10                                              # five tiles, plain and gated
     bad = {name: found for name, body in kernels if (found := unwaited(body.split("\n")))}
     assert not bad
-    for _, body in kernels:
+    for name, body in kernels:
+        # a step's matrix instructions (two columns, six products a fragment) stand between its loads and their wait
+        assert overlap(body.split("\n")) == 12 * int(re.search(r"ILi(\d+)E", name).group(1))
         assert "global_load_lds" in body and body.count("s_barrier") >= 2
