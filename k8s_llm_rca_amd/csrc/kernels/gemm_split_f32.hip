@@ -13,7 +13,7 @@
 // that W is read in fragment order and split in registers: asked for between the halves of a step's matrix instructions,
 // waited for in front of the next step's loads into LDS (so that no wait is for those: us without / so at 622 rows, ten
 // fragments, 16384 x 2048 203 / 196, 8192 x 2048 136 / 116, 2048 x 8192 in four ranges 136 / 117), split between that step's
-// halves.  Two workgroups share a compute unit.  The tiles of one panel of the larger operand follow each other on one XCD.
+// halves.  Two to four workgroups share a compute unit.  The tiles of one panel of the larger operand follow each other on one XCD.
 // Few tiles: K in ranges, whose sums (planes) the consumer adds.
 //
 // What bounds it: the power (1.8 GHz at a bf16 rate of 1.1 PFLOP/s) and, where there are few workgroups, a step's chain (1.2 us
@@ -67,17 +67,26 @@ __device__ __forceinline__ void split3(const f32x4& a, Split3& s, bool wild) {
   }
 }
 
-// x [M][K] (rows ldx apart) -> p [3][M][K]
-__global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict__ x, int ldx, uint16_t* __restrict__ p, int M, int K) {
-  const int k4 = K >> 2;
-  const size_t n = (size_t)M * k4, plane = (size_t)M * K;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-    const size_t m = i / k4, c = 4 * (i - m * k4);
+// x [M][K] (rows ldx apart) -> p [3][M][K], f [M]: 1, or NaN where a number of the row is.  A workgroup a row.
+__global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict__ x, int ldx, uint16_t* __restrict__ p,
+                                                         float* __restrict__ f, int M, int K) {
+  const int m = blockIdx.x, tid = threadIdx.x;
+  const size_t plane = (size_t)M * K;
+  x += (size_t)m * ldx;
+  p += (size_t)m * K;
+  bool nan = false;
+#pragma unroll 2
+  for (int c = 4 * tid; c < K; c += 1024) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(x + c);
     Split3 s;
-    split3(*reinterpret_cast<const f32x4*>(x + m * ldx + c), s, true);
+    split3(v, s, true);
 #pragma unroll
-    for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x2*>(p + q * plane + m * K + c) = s.p[q];
+    for (int k = 0; k < 4; ++k) nan |= v[k] != v[k];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x2*>(p + q * plane + c) = s.p[q];
   }
+  nan = __syncthreads_or(nan);
+  if (tid == 0) f[m] = nan ? __builtin_nanf("") : 1.f;
 }
 
 typedef __attribute__((address_space(3))) void sf_lds_t;
@@ -85,24 +94,37 @@ __device__ __forceinline__ void sf_to_lds(const uint16_t* src, uint16_t* dst) { 
   __builtin_amdgcn_global_load_lds(src, (sf_lds_t*)dst, 16, 0, 0);
 }
 
-__device__ __attribute__((noinline)) float fp32_dot(const uint16_t* xpl, const float* w, int m, size_t wrow, int M, int K, int k0,
+// One sum in fp32, by the whole wave (m, wrow alike in all lanes)
+__device__ __forceinline__ float fp32_dot(const uint16_t* xpl, const float* w, int m, size_t wrow, int M, int K, int k0,
                                                     int n) {
   const uint16_t* a = xpl + (size_t)m * K + k0;
   const float* b = w + wrow * K + k0;
   const size_t plane = (size_t)M * K;
   float t = 0.f;
-  for (int k = 0; k < n; ++k) t = fmaf(bf2f(a[k]) + bf2f(a[plane + k]) + bf2f(a[2 * plane + k]), b[k], t);
-  return t;
+  for (int k = 4 * (threadIdx.x & 63); k < n; k += 256) {
+    const u16x4 p0 = *reinterpret_cast<const u16x4*>(a + k), p1 = *reinterpret_cast<const u16x4*>(a + plane + k),
+                p2 = *reinterpret_cast<const u16x4*>(a + 2 * plane + k);
+    const f32x4 v = *reinterpret_cast<const f32x4*>(b + k);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) t = fmaf(bf2f(p0[j]) + bf2f(p1[j]) + bf2f(p2[j]), v[j], t);
+  }
+  return wave_sum(t);
 }
 
 // grid: (row tiles x column tiles, K ranges).  The end of a step counts the loads behind its own into LDS, so their order is
 // fixed: no pointer here is __restrict__, since loads through such a one may pass any clobber (tests/test_split_f32_waits.py
 // reads the assembly).
 template <int MT, int OUT>
-__global__ void __launch_bounds__(256, 2)
-    gemm_split_f32_kernel(const uint16_t* xpl, const float* w, float* y, int M, int N, int K, int n_mt, int n_nt) {
+__global__ void __launch_bounds__(256, MT <= 4 ? 4 : MT <= 8 ? 3 : 2)      // (what LDS lets onto a compute unit)
+    gemm_split_f32_kernel(const uint16_t* xpl, const float* xfac, const float* w, float* y, int M, int N, int K, int n_mt, int n_nt) {
   constexpr int BM = 16 * MT, ND = 3 * MT, PER = (ND + 3) / 4;    // LDS-DMA instructions of a step, of a wave
-  __shared__ __attribute__((aligned(1024))) uint16_t xs[2][3][BM * kSfK];
+  // (one variable: beside another one the compiler waits for the loads into LDS in front of every read of it)
+  __shared__ struct {
+    __attribute__((aligned(1024))) uint16_t xs[2][3][BM * kSfK];
+    float fac[BM];                                                // of X's rows
+  } lds;
+  auto& xs = lds.xs;
+  auto& fac = lds.fac;
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   // the tiles that share the larger operand's panel on one XCD, one after the other
@@ -129,6 +151,7 @@ __global__ void __launch_bounds__(256, 2)
     const size_t row = OUT == kSplitGlu ? min(n0 + 16 * wv + r, N - 1) + (size_t)j * N : min(n0 + 32 * wv + 16 * j + r, N - 1);
     wp[j] = w + row * K + k0 + 8 * g;
   }
+  if (tid < BM) fac[tid] = xfac[min(m0 + tid, M - 1)];            // (up to 192 rows; there when the first step ends)
   f32x4 wq[2][2];
   bf16x8 wf[2][3];
   auto load_x = [&](int s, int buf) {
@@ -177,20 +200,10 @@ __global__ void __launch_bounds__(256, 2)
     __builtin_amdgcn_sched_barrier(0);
   };
   f32x4 acc[MT][2];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto fence = [] {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  load_w(0);
-  load_x(0, 0);
-  take_any(wf);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // X of step 0
-  bar();
-  load_w(min(1, steps - 1));
   // two rows of fragments: 24 matrix instructions
   auto multiply = [&](int buf, int i) {
     bf16x8 xf[2][3];
@@ -208,6 +221,16 @@ __global__ void __launch_bounds__(256, 2)
         for (int j = 0; j < 2; ++j)
           acc[i + h][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][PW[q]], xf[h][PX[q]], acc[i + h][j], 0, 0, 0);
   };
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  load_w(0);
+  load_x(0, 0);
+  take_any(wf);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // X of step 0
+  bar();
+  load_w(min(1, steps - 1));
   for (int s = 0; s < steps; ++s) {                               // (the last step loads and splits what it has once more, unread)
     const int buf = s & 1;
     constexpr int H = MT / 4 * 2;
@@ -234,36 +257,62 @@ __global__ void __launch_bounds__(256, 2)
     asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");   // the next step's X; this step's fragments are read
     bar();
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // no load into LDS outlives the workgroup
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // no load into LDS outlives the workgroup
+  bar();                                                          // (anybody's)
   // acc[i][j][v]: row m0 + 16 i + r, panel row 32 wv + 16 j + 4 g + v
   //
   // An infinity meets the other operand's parts of both signs, or none, and gives NaN where it should stay one: sums that are
-  // NaN are made again as fp32 makes them.
+  // NaN though no number of their rows is are made again in fp32.
   bool lost = false;
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int i = 0; i < MT; ++i) {
+    const float f = fac[16 * i + r];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) lost |= acc[i][j][v] != acc[i][j][v];
+      for (int v = 0; v < 4; ++v) lost |= acc[i][j][v] != acc[i][j][v] && f == f;
+  }
   if (__builtin_expect(__any(lost), 0)) {
+    bool nan[2] = {false, false};                                 // of this lane's rows of W
+#pragma unroll 1
+    for (int s = 0; s < steps; ++s) {
+      load_w(s);
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+        for (int k = 0; k < 4; ++k) nan[j >> 1] |= wq[j >> 1][j & 1][k] != wq[j >> 1][j & 1][k];
+    }
+    float* const st = reinterpret_cast<float*>(&xs[0][0][0]) + wv * BM * 16;     // the wave's sums of 16 columns (X is done with)
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-          if (acc[i][j][v] != acc[i][j][v]) {
-            const int c = 4 * g + v;
-            const size_t wr = OUT == kSplitGlu ? min(n0 + 16 * wv + c, N - 1) + (size_t)j * N : min(n0 + 32 * wv + 16 * j + c, N - 1);
-            acc[i][j][v] = fp32_dot(xpl, w, min(m0 + 16 * i + r, M - 1), wr, M, K, k0, kr);
-          }
+    for (int j = 0; j < 2; ++j) {
+      const uint64_t bits = __ballot(nan[j]), bad = bits | bits >> 16 | bits >> 32 | bits >> 48;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) *reinterpret_cast<f32x4*>(st + (16 * i + r) * 16 + 4 * g) = acc[i][j];
+      fence();
+#pragma unroll 1
+      for (int e = lane; e < BM * 16; e += 64) {
+        const float t = st[e], f = fac[e >> 4];
+        for (uint64_t b = __ballot(t != t && f == f && !(bad >> (e & 15) & 1)); b; b &= b - 1) {
+          const int q = __ffsll((unsigned long long)b) - 1, at = e - lane + q, c = at & 15;
+          const size_t wr = OUT == kSplitGlu ? min(n0 + 16 * wv + c, N - 1) + (size_t)j * N : min(n0 + 32 * wv + 16 * j + c, N - 1);
+          const float sum = fp32_dot(xpl, w, min(m0 + (at >> 4), M - 1), wr, M, K, k0, kr);
+          if (lane == q) st[e] = sum;
+        }
+      }
+      fence();
+#pragma unroll
+      for (int i = 0; i < MT; ++i) acc[i][j] = *reinterpret_cast<const f32x4*>(st + (16 * i + r) * 16 + 4 * g);
+      fence();
+    }
   }
   float* const o = y + (size_t)blockIdx.y * M * N;
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int m = m0 + 16 * i + r;
     if (m >= M) continue;
+    const float f = fac[16 * i + r];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] *= f;
     if constexpr (OUT == kSplitGlu) {
       const int n = n0 + 16 * wv + 4 * g;
       if (n >= N) continue;
@@ -282,15 +331,15 @@ __global__ void __launch_bounds__(256, 2)
 }
 
 template <int OUT>
-static int split_f32(const uint16_t* xp, const float* w, float* y, int M, int N, int K, int mt, int ranges, hipStream_t s) {
-  if (M <= 0 || N <= 0 || N % 4 || K <= 0 || ranges < 1 || K % (kSfK * ranges) || !xp || !w || !y || ((uintptr_t)xp & 15) ||
+static int split_f32(const uint16_t* xp, const float* f, const float* w, float* y, int M, int N, int K, int mt, int ranges, hipStream_t s) {
+  if (M <= 0 || N <= 0 || N % 4 || K <= 0 || ranges < 1 || K % (kSfK * ranges) || !xp || !f || !w || !y || ((uintptr_t)xp & 15) ||
       ((uintptr_t)w & 15) || ((uintptr_t)y & 15) || (OUT == kSplitGlu && (ranges > 1 || N % 64)))
     return (int)hipErrorInvalidValue;
   const int bn = OUT == kSplitGlu ? kSfN / 2 : kSfN, n_nt = (N + bn - 1) / bn, n_mt = (M + 16 * mt - 1) / (16 * mt);
 #define K8S_SF(MT)                                                                                                        \
   case MT:                                                                                                                \
-    hipLaunchKernelGGL((gemm_split_f32_kernel<MT, OUT>), dim3(n_mt * n_nt, ranges), dim3(256), 0, s, xp, w, y, M, N, K, n_mt, \
-                       n_nt);                                                                                             \
+    hipLaunchKernelGGL((gemm_split_f32_kernel<MT, OUT>), dim3(n_mt * n_nt, ranges), dim3(256), 0, s, xp, f, w, y, M, N, K,   \
+                       n_mt, n_nt);                                                                                             \
     break
   switch (mt) {
     K8S_SF(4);
@@ -308,22 +357,24 @@ static int split_f32(const uint16_t* xp, const float* w, float* y, int M, int N,
 
 using namespace k8s;
 
-// x [M][K] fp32 (rows ldx apart, on 16 bytes) -> three bf16 planes p [3][M][K] whose sum it is.
-K8S_API int k8s_split_rows_f32(const float* x, int ldx, void* p, int M, int K, hipStream_t s) {
-  if (M <= 0 || K <= 0 || K % 4 || ldx % 4 || (M > 1 && ldx < K) || !x || !p || ((uintptr_t)x & 15) || ((uintptr_t)p & 7))
+// x [M][K] fp32 (rows ldx apart, on 16 bytes) -> three bf16 planes p [3][M][K] and f [M]: a row is the planes' sum (f: NaN where a
+// number of it is, else 1).
+K8S_API int k8s_split_rows_f32(const float* x, int ldx, void* p, float* f, int M, int K, hipStream_t s) {
+  if (M <= 0 || K <= 0 || K % 4 || ldx % 4 || (M > 1 && ldx < K) || !x || !p || !f || ((uintptr_t)x & 15) || ((uintptr_t)p & 7))
     return (int)hipErrorInvalidValue;
-  const size_t n = ((size_t)M * K / 4 + 255) / 256;
-  hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)(n < 4096 ? n : 4096)), dim3(256), 0, s, x, ldx, (uint16_t*)p, M, K);
+  hipLaunchKernelGGL(split_rows_kernel, dim3(M), dim3(256), 0, s, x, ldx, (uint16_t*)p, f, M, K);
   return (int)hipGetLastError();
 }
 
-// y [ranges][M][N] fp32: the products of xp's rows (three planes) and w [N][K] over K ranges.  mt: 16-row fragments of a tile, 4,
-// 6, 8, 10 or 12.  N a multiple of 4, K of 32 ranges; xp, w, y on 16 bytes.
-K8S_API int k8s_gemm_split_f32(const void* xp, const float* w, float* y, int M, int N, int K, int mt, int ranges, hipStream_t s) {
-  return split_f32<kSplitPlain>((const uint16_t*)xp, w, y, M, N, K, mt, ranges, s);
+// y [ranges][M][N] fp32: the products of xp's rows (three planes, f as above) and w [N][K] over K ranges.  mt: 16-row
+// fragments of a tile, 4, 6, 8, 10 or 12.  N a multiple of 4, K of 32 ranges; xp, w, y on 16 bytes.
+K8S_API int k8s_gemm_split_f32(const void* xp, const float* f, const float* w, float* y, int M, int N, int K, int mt, int ranges,
+                               hipStream_t s) {
+  return split_f32<kSplitPlain>((const uint16_t*)xp, f, w, y, M, N, K, mt, ranges, s);
 }
 
 // y [M][N] = silu(x . w[0:N]^T) * (x . w[N:2N]^T), N a multiple of 64.
-K8S_API int k8s_gemm_split_glu_f32(const void* xp, const float* w, float* y, int M, int N, int K, int mt, hipStream_t s) {
-  return split_f32<kSplitGlu>((const uint16_t*)xp, w, y, M, N, K, mt, 1, s);
+K8S_API int k8s_gemm_split_glu_f32(const void* xp, const float* f, const float* w, float* y, int M, int N, int K, int mt,
+                                   hipStream_t s) {
+  return split_f32<kSplitGlu>((const uint16_t*)xp, f, w, y, M, N, K, mt, 1, s);
 }

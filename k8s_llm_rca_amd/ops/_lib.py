@@ -54,9 +54,9 @@ _SIGS = {
     "k8s_gemm_skinny_f32": [P, I, P, P, I, I, I, I, P],
     "k8s_few_rows_f32": [P, I, P, P, I, I, I, P],
     "k8s_few_rows_glu_f32": [P, I, P, P, I, I, I, P],
-    "k8s_split_rows_f32": [P, I, P, I, I, P],
-    "k8s_gemm_split_f32": [P, P, P, I, I, I, I, I, P],
-    "k8s_gemm_split_glu_f32": [P, P, P, I, I, I, I, P],
+    "k8s_split_rows_f32": [P, I, P, P, I, I, P],
+    "k8s_gemm_split_f32": [P, P, P, P, I, I, I, I, I, P],
+    "k8s_gemm_split_glu_f32": [P, P, P, P, I, I, I, I, P],
     "k8s_gemm_skinny_rope": [P, I, P, P, I, I, I, I, P, P, P, P, P, I, I, I, P],
     "k8s_gemm_mid": [P, I, P, P, I, I, I, I, I, I, P, P],
     "k8s_gemm_mid_part": [P, I, P, P, I, I, I, I, I, I, P, P],

@@ -240,14 +240,15 @@ def _split_f32(x: torch.Tensor, w: torch.Tensor, planes: bool = False, glu: bool
             w.is_contiguous() and w.data_ptr() % 16 == 0 == x.data_ptr() % 16 and x.stride(1) == 1 and x.stride(0) % 4 == 0
             and K <= x.stride(0) < 2 ** 31 and w.device == x.device):
         return None
-    parts = torch.empty(3, M, K, dtype=torch.bfloat16, device=x.device)
-    check(lib().k8s_split_rows_f32(ptr(x), x.stride(0), ptr(parts), M, K, stream_ptr(x)), "split_rows_f32")
+    parts = torch.empty(3 * M * K + 2 * M, dtype=torch.bfloat16, device=x.device)      # and an fp32 factor a row
+    p, f = ptr(parts), ptr(parts) + 6 * M * K
+    check(lib().k8s_split_rows_f32(ptr(x), x.stride(0), p, f, M, K, stream_ptr(x)), "split_rows_f32")
     if glu:
         out = torch.empty(M, N // 2, dtype=torch.float32, device=x.device)
-        check(lib().k8s_gemm_split_glu_f32(ptr(parts), ptr(w), ptr(out), M, N // 2, K, plan[0], stream_ptr(x)), "gemm_split_glu_f32")
+        check(lib().k8s_gemm_split_glu_f32(p, f, ptr(w), ptr(out), M, N // 2, K, plan[0], stream_ptr(x)), "gemm_split_glu_f32")
         return out
     out = torch.empty(plan[1], M, N, dtype=torch.float32, device=x.device)
-    check(lib().k8s_gemm_split_f32(ptr(parts), ptr(w), ptr(out), M, N, K, *plan, stream_ptr(x)), "gemm_split_f32")
+    check(lib().k8s_gemm_split_f32(p, f, ptr(w), ptr(out), M, N, K, *plan, stream_ptr(x)), "gemm_split_f32")
     return out
 
 

@@ -20,17 +20,22 @@ def test_rule():
             assert p is None or p[0] in L.SPLIT_TILES and k % (32 * p[1]) == 0
 
 
-def _parts(x):
+def _split(x):
     m, k = x.shape
-    p = torch.empty(3, m, k, dtype=torch.bfloat16, device=x.device)
-    check(lib().k8s_split_rows_f32(ptr(x), x.stride(0), ptr(p), m, k, stream_ptr(x)), "split")
-    return p
+    p, f = torch.empty(3, m, k, dtype=torch.bfloat16, device=x.device), torch.empty(m, device=x.device)
+    check(lib().k8s_split_rows_f32(ptr(x), x.stride(0), ptr(p), ptr(f), m, k, stream_ptr(x)), "split")
+    return p, f
+
+
+def _parts(x):
+    return _split(x)[0]
 
 
 def _product(x, w, mt, ranges):
     (m, k), n = x.shape, w.shape[0]
     y = torch.full((ranges, m, n), float("nan"), device=x.device)
-    check(lib().k8s_gemm_split_f32(ptr(_parts(x)), ptr(w), ptr(y), m, n, k, mt, ranges, stream_ptr(x)), "product")
+    p, f = _split(x)
+    check(lib().k8s_gemm_split_f32(ptr(p), ptr(f), ptr(w), ptr(y), m, n, k, mt, ranges, stream_ptr(x)), "product")
     return y
 
 
@@ -79,6 +84,37 @@ def test_infinities_and_the_ends_of_the_range():
     assert torch.equal(y[both], want[both])
     fin = want.isfinite()
     assert bool(((y - want)[fin].abs() <= 2e-5 * (want[fin].abs() + 30)).all())
+
+
+@gpu
+def test_numbers_that_are_not():
+    """NaN where a number of either row is, without a sum of its own for each, and nowhere else."""
+    g = torch.Generator().manual_seed(11)
+    x, w = torch.randn(640, 2048, generator=g).cuda(), torch.randn(4096, 2048, generator=g).cuda() * 0.02
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+
+    def us(x, w):
+        best = 1e9
+        for _ in range(4):
+            ev[0].record()
+            y = _product(x, w, 10, 1)
+            ev[1].record()
+            torch.cuda.synchronize()
+            best = min(best, ev[0].elapsed_time(ev[1]) * 1e3)
+        return best, y[0]
+    plain, y0 = us(x, w)
+    xn, wn = x.clone(), w.clone()
+    xn[::2, 5], wn[1::2, 2047] = float("nan"), float("nan")
+    for a, b in ((xn, w), (x, wn), (xn, wn)):
+        t, y = us(a, b)
+        bad = a.isnan().any(1)[:, None] | b.isnan().any(1)
+        assert torch.equal(y.isnan(), bad) and torch.equal(y[~bad], y0[~bad])
+        assert t < 8 * plain + 100
+    # one infinity a row: a sum of its own each
+    xi = x.clone()
+    xi[7, 3], xi[639, 2000] = float("inf"), float("-inf")
+    y = us(xi, w)[1]
+    assert torch.equal(y[[7, 639]], torch.stack([xi[7, 3] * w[:, 3], xi[639, 2000] * w[:, 2000]]))
 
 
 @gpu

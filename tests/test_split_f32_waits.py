@@ -41,16 +41,16 @@ def unwaited(lines):
 
 
 def overlap(lines):
-    """The least number of matrix instructions issued between a load into LDS that stands behind a barrier and its wait."""
-    return min(_follow(lines)[1], default=None)
+    """The waits that end such loads, with the least number of matrix instructions issued between the two."""
+    return _follow(lines)[1]
 
 
 def _follow(lines):
     blocks = _blocks(lines)
-    state, todo, bad, between = {0: (NONE, 0, 0)}, [0], set(), {}
+    state, todo, bad, between = {0: (NONE, 0)}, [0], set(), {}
     while todo:
         i = todo.pop()
-        behind, matrix, met = state[i]             # memory and matrix instructions since the last load into LDS; barriers
+        behind, matrix = state[i]                  # memory and matrix instructions since the last load into LDS
         for k, text in enumerate(blocks[i][0]):
             op = text.split()[0]
             wait = re.search(r"vmcnt\((\d+)\)", text)
@@ -61,16 +61,14 @@ def _follow(lines):
             elif op.startswith("v_mfma") and behind != NONE:
                 matrix += 1
             elif op == "s_waitcnt" and wait and int(wait.group(1)) <= behind:
-                if behind != NONE and met:
-                    between[i, k] = min(matrix, between.get((i, k), matrix))
-                behind = NONE
-            elif op in ("s_barrier", "s_endpgm"):
                 if behind != NONE:
-                    bad.add((i, k))
-                met = 1
+                    between[i, k] = text, min(matrix, between.get((i, k), (text, matrix))[1])
+                behind = NONE
+            elif op in ("s_barrier", "s_endpgm") and behind != NONE:
+                bad.add((i, k))
         for j in blocks[i][1]:
-            old = state.get(j, (NONE + 1, NONE, 1))
-            new = (min(behind, old[0]), min(matrix if behind != NONE else NONE, old[1]), min(met, old[2]))
+            old = state.get(j, (NONE + 1, NONE))
+            new = (min(behind, old[0]), min(matrix if behind != NONE else NONE, old[1]))
             if new != old:
                 state[j] = new
                 todo.append(j)
@@ -88,7 +86,9 @@ def test_reading():
     loop = "{0}\n.LBB0_1:\ns_waitcnt vmcnt({1})\ns_barrier\n{2}\ns_cbranch_scc1 .LBB0_1\n" + end
     assert not f(loop.format(f"{dma}\n{load}", 1, f"{dma}\n{load}"))
     assert f(loop.format(f"{dma}\n{load}", 1, f"{load}\n{dma}"))          # by the way back only
-    assert overlap(loop.format(dma, 0, f"{dma}\nv_mfma_f32 v0\nv_mfma_f32 v0").split("\n")) == 2
+    mfma = "v_mfma_f32 v0\n" * 2
+    assert overlap(loop.format(dma, 1, f"{mfma}{dma}").split("\n")) == [("s_waitcnt vmcnt(0)", 0)]
+    assert overlap(loop.format(dma, 0, f"{dma}\n{mfma}").split("\n")) == [("s_waitcnt vmcnt(0)", 0), ("s_waitcnt vmcnt(0)", 2)]
     assert f(f"{dma}\ns_cbranch_scc0 .LBB0_1\n{load}\n.LBB0_1:\ns_waitcnt vmcnt(1)\ns_barrier\n{end}")
 
 
@@ -103,5 +103,6 @@ def test_waits_cover_the_loads(tmp_path):
     assert not bad
     for name, body in kernels:
         # a step's matrix instructions (two columns, six products a fragment) stand between its loads and their wait
-        assert overlap(body.split("\n")) == 12 * int(re.search(r"ILi(\d+)E", name).group(1))
+        ended = [n for text, n in overlap(body.split("\n")) if "vmcnt(4)" in text]
+        assert ended and set(ended) == {12 * int(re.search(r"ILi(\d+)E", name).group(1))}
         assert "global_load_lds" in body and body.count("s_barrier") >= 2
