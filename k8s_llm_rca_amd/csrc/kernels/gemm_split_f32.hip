@@ -17,10 +17,10 @@
 // Few tiles: K in ranges, whose sums (planes) the consumer adds.
 //
 // What bounds it: the power (1.8 GHz at a bf16 rate of 1.1 PFLOP/s) and, where there are few workgroups, a step's chain (1.2 us
-// with four fragments, 2.0 with ten).  us, the library / the pass and this, out of memory:  16384 x 2048 at 333, 622, 1024 rows
-// 214 / 139, 373 / 236, 513 / 346;  8192 x 2048 at 622, 1024 187 / 133, 241 / 167;  2048 x 8192 in ranges 162 / 123, 243 / 183
-// and their sums.  With X split by every workgroup 330 instead of 236, with W in LDS as well 361; the splits placed between
-// the matrix instructions one by one 357.
+// with four fragments, 1.65 with ten).  us, the library / the pass and this, out of memory:  16384 x 2048 at 333, 622, 1024 rows
+// 210 / 150, 380 / 231, 515 / 341;  8192 x 2048 at 622, 1024 183 / 131, 257 / 182;  2048 x 8192 in eight ranges 176 / 124, 246 / 207
+// and their sums.  In a first form, whose loads did not overlap: with X split by every workgroup 330 instead of 236, with
+// W in LDS as well 361; the splits placed between the matrix instructions one by one 357.
 #include "common.h"
 
 namespace k8s {
@@ -67,26 +67,45 @@ __device__ __forceinline__ void split3(const f32x4& a, Split3& s, bool wild) {
   }
 }
 
-// x [M][K] (rows ldx apart) -> p [3][M][K], f [M]: 1, or NaN where a number of the row is.  A workgroup a row.
+// A row (of X) or a row's K range (of W) whose largest number is below kSfLow, or kSfTiny, is multiplied by kSfUp, and its sums by
+// the inverse: the third part of a number below 2^-110 would fall out of bf16's range.  The largest is below 2^-26 then, so that
+// no sum overflows that did not.
+constexpr float kSfLow = 0x1p-90f, kSfTiny = 0x1p-100f, kSfUp = 0x1p64f;
+
+// x [M][K] (rows ldx apart) -> p [3][M][K], f [M]: what the row's sums are to be multiplied by (NaN: a number of the row is NaN).
+// A workgroup a row.
 __global__ void __launch_bounds__(256) split_rows_kernel(const float* __restrict__ x, int ldx, uint16_t* __restrict__ p,
                                                          float* __restrict__ f, int M, int K) {
+  __shared__ float red[4];
   const int m = blockIdx.x, tid = threadIdx.x;
   const size_t plane = (size_t)M * K;
   x += (size_t)m * ldx;
   p += (size_t)m * K;
+  float most = 0.f;
   bool nan = false;
+  auto pass = [&](float up) {
 #pragma unroll 2
-  for (int c = 4 * tid; c < K; c += 1024) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(x + c);
-    Split3 s;
-    split3(v, s, true);
+    for (int c = 4 * tid; c < K; c += 1024) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(x + c) * up;
+      Split3 s;
+      split3(v, s, true);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) nan |= v[k] != v[k];
+      for (int k = 0; k < 4; ++k) {
+        most = fmaxf(most, fabsf(v[k]));
+        nan |= v[k] != v[k];
+      }
 #pragma unroll
-    for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x2*>(p + q * plane + c) = s.p[q];
-  }
+      for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x2*>(p + q * plane + c) = s.p[q];
+    }
+  };
+  pass(1.f);
+  most = wave_max(most);
+  if ((tid & 63) == 0) red[tid >> 6] = most;
   nan = __syncthreads_or(nan);
-  if (tid == 0) f[m] = nan ? __builtin_nanf("") : 1.f;
+  most = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const bool low = most > 0.f && most < kSfLow;
+  if (low) pass(kSfUp);
+  if (tid == 0) f[m] = nan ? __builtin_nanf("") : low ? 1.f / kSfUp : 1.f;
 }
 
 typedef __attribute__((address_space(3))) void sf_lds_t;
@@ -122,6 +141,8 @@ __global__ void __launch_bounds__(256, MT <= 4 ? 4 : MT <= 8 ? 3 : 2)      // (w
   __shared__ struct {
     __attribute__((aligned(1024))) uint16_t xs[2][3][BM * kSfK];
     float fac[BM];                                                // of X's rows
+    float up[kSfN];                                               // of the panel's rows of W, made for a second walk
+    int low[4];
   } lds;
   auto& xs = lds.xs;
   auto& fac = lds.fac;
@@ -154,6 +175,7 @@ __global__ void __launch_bounds__(256, MT <= 4 ? 4 : MT <= 8 ? 3 : 2)      // (w
   if (tid < BM) fac[tid] = xfac[min(m0 + tid, M - 1)];            // (up to 192 rows; there when the first step ends)
   f32x4 wq[2][2];
   bf16x8 wf[2][3];
+  float top[2] = {0.f, 0.f};                                      // the largest numbers of this lane's rows of W
   auto load_x = [&](int s, int buf) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -168,19 +190,20 @@ __global__ void __launch_bounds__(256, MT <= 4 ? 4 : MT <= 8 ? 3 : 2)      // (w
       for (int h = 0; h < 2; ++h) wq[j][h] = *reinterpret_cast<const f32x4*>(wp[j] + s * kSfK + 4 * h);
   };
   auto wild = [&] {
-    float most = 0.f;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) most = fmaxf(most, fabsf(wq[j >> 1][j & 1][k]));
-    return (bool)__any(most >= kSfWild);
+      for (int k = 0; k < 4; ++k) top[j] = fmaxf(top[j], fmaxf(fabsf(wq[j][0][k]), fabsf(wq[j][1][k])));
+    return (bool)__any(fmaxf(top[0], top[1]) >= kSfWild);
   };
+  bool again = false;
   auto take = [&](bf16x8 (&f)[2][3], bool wi) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       Split3 a, b;
-      split3(wq[j][0], a, wi);
-      split3(wq[j][1], b, wi);
+      const float up = wi && again ? lds.up[32 * wv + 16 * j + r] : 1.f;
+      split3(wi ? wq[j][0] * up : wq[j][0], a, wi);
+      split3(wi ? wq[j][1] * up : wq[j][1], b, wi);
 #pragma unroll
       for (int p = 0; p < 3; ++p) {
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -189,7 +212,7 @@ __global__ void __launch_bounds__(256, MT <= 4 ? 4 : MT <= 8 ? 3 : 2)      // (w
     }
   };
   auto take_any = [&](bf16x8 (&f)[2][3]) {
-    if (__builtin_expect(wild(), 0))
+    if (__builtin_expect(wild() || again, 0))
       take(f, true);
     else
       take(f, false);
@@ -221,44 +244,71 @@ __global__ void __launch_bounds__(256, MT <= 4 ? 4 : MT <= 8 ? 3 : 2)      // (w
         for (int j = 0; j < 2; ++j)
           acc[i + h][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][PW[q]], xf[h][PX[q]], acc[i + h][j], 0, 0, 0);
   };
+  for (;;) {
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  load_w(0);
-  load_x(0, 0);
-  take_any(wf);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // X of step 0
-  bar();
-  load_w(min(1, steps - 1));
-  for (int s = 0; s < steps; ++s) {                               // (the last step loads and splits what it has once more, unread)
-    const int buf = s & 1;
-    constexpr int H = MT / 4 * 2;
-    // W of the next step has come before the loads into LDS are asked for: with these on their way the compiler waits for all
-    // loads where it needs one
-    asm volatile("" : "+v"(wq[0][0]), "+v"(wq[0][1]), "+v"(wq[1][0]), "+v"(wq[1][1])::"memory");
-    fence();
-    load_x(min(s + 1, steps - 1), buf ^ 1);
-    fence();
+      for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    load_w(0);
+    load_x(0, 0);
+    take_any(wf);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // X of step 0
+    bar();
+    load_w(min(1, steps - 1));
+    for (int s = 0; s < steps; ++s) {                               // (the last step loads and splits what it has once more, unread)
+      const int buf = s & 1;
+      constexpr int H = MT / 4 * 2;
+      // W of the next step has come before the loads into LDS are asked for: with these on their way the compiler waits for all
+      // loads where it needs one
+      asm volatile("" : "+v"(wq[0][0]), "+v"(wq[0][1]), "+v"(wq[1][0]), "+v"(wq[1][1])::"memory");
+      fence();
+      load_x(min(s + 1, steps - 1), buf ^ 1);
+      fence();
 #pragma unroll
-    for (int i = 0; i < H; i += 2) multiply(buf, i);
-    bf16x8 nf[2][3];
-    take_any(nf);
-    fence();
-    load_w(min(s + 2, steps - 1));                                // four loads: what the wait below leaves on its way
-    fence();
+      for (int i = 0; i < H; i += 2) multiply(buf, i);
+      bf16x8 nf[2][3];
+      take_any(nf);
+      fence();
+      load_w(min(s + 2, steps - 1));                                // four loads: what the wait below leaves on its way
+      fence();
 #pragma unroll
-    for (int i = H; i < MT; i += 2) multiply(buf, i);
+      for (int i = H; i < MT; i += 2) multiply(buf, i);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) wf[j][p] = nf[j][p];
+      fence();
+      asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");   // the next step's X; this step's fragments are read
+      bar();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // no load into LDS outlives the walk
+    // W's rows of tiny numbers (lanes 0 to 15 of a wave have two each): once more, with factors
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float t = fmaxf(top[j], __shfl_xor(top[j], 16, 64));
+      t = fmaxf(t, __shfl_xor(t, 32, 64));
+      const bool tiny = t > 0.f && t < kSfTiny;
+      if (!again) lds.up[32 * wv + 16 * j + r] = tiny ? kSfUp : 1.f;
+      any |= tiny;
+    }
+    any = __any(any);
+    if (lane == 0) lds.low[wv] = any;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bar();
+    if (__builtin_expect(again || !(lds.low[0] | lds.low[1] | lds.low[2] | lds.low[3]), 1)) break;
+    again = true;
+  }
+  if (__builtin_expect(again, 0)) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int p = 0; p < 3; ++p) wf[j][p] = nf[j][p];
-    fence();
-    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");   // the next step's X; this step's fragments are read
-    bar();
+      for (int v = 0; v < 4; ++v) {
+        const float down = 1.f / lds.up[32 * wv + 16 * j + 4 * g + v];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[i][j][v] *= down;
+      }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // no load into LDS outlives the workgroup
-  bar();                                                          // (anybody's)
   // acc[i][j][v]: row m0 + 16 i + r, panel row 32 wv + 16 j + 4 g + v
   //
   // An infinity meets the other operand's parts of both signs, or none, and gives NaN where it should stay one: sums that are
@@ -357,8 +407,8 @@ static int split_f32(const uint16_t* xp, const float* f, const float* w, float* 
 
 using namespace k8s;
 
-// x [M][K] fp32 (rows ldx apart, on 16 bytes) -> three bf16 planes p [3][M][K] and f [M]: a row is the planes' sum (f: NaN where a
-// number of it is, else 1).
+// x [M][K] fp32 (rows ldx apart, on 16 bytes) -> three bf16 planes p [3][M][K] and f [M]: a row is f times the planes' sum (NaN
+// where a number of it is).
 K8S_API int k8s_split_rows_f32(const float* x, int ldx, void* p, float* f, int M, int K, hipStream_t s) {
   if (M <= 0 || K <= 0 || K % 4 || ldx % 4 || (M > 1 && ldx < K) || !x || !p || !f || ((uintptr_t)x & 15) || ((uintptr_t)p & 7))
     return (int)hipErrorInvalidValue;
@@ -366,7 +416,7 @@ K8S_API int k8s_split_rows_f32(const float* x, int ldx, void* p, float* f, int M
   return (int)hipGetLastError();
 }
 
-// y [ranges][M][N] fp32: the products of xp's rows (three planes, f as above) and w [N][K] over K ranges.  mt: 16-row
+// y [ranges][M][N] fp32: the products of xp's rows (three planes and their factors) and w [N][K] over K ranges.  mt: 16-row
 // fragments of a tile, 4, 6, 8, 10 or 12.  N a multiple of 4, K of 32 ranges; xp, w, y on 16 bytes.
 K8S_API int k8s_gemm_split_f32(const void* xp, const float* f, const float* w, float* y, int M, int N, int K, int mt, int ranges,
                                hipStream_t s) {

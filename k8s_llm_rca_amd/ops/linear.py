@@ -208,10 +208,10 @@ def split_plan(M: int, N: int, K: int, planes: bool = False, glu: bool = False):
 
     A step of a workgroup (K 32) takes some 0.5 us and 0.13 a fragment, less the fewer of them a compute unit has at once; the
     rows' split is a pass of 4 us and their bytes, each range writes and reads the result once more; and the library takes its
-    operations at 120 TFLOP/s and a start.  us library / the split and this:  16384 x 2048 at 333, 622, 1024 rows 214 / 139,
-    373 / 236, 513 / 346, at 166 105 / 109;  8192 x 2048 at the same 108 / 105, 187 / 133, 241 / 167, 61 / 95;  2048 x 8192
-    (eight ranges, with the bytes of their sums) 108 / 88, 162 / 139, 243 / 188;  2048 x 2048 33 / 36, 46 / 52, 66 / 63;  2560 x
-    2048 at 1024 100 / 77."""
+    operations at 120 TFLOP/s and a start.  us library / the split and this:  16384 x 2048 at 333, 622, 1024 rows 210 / 150,
+    380 / 231, 515 / 341, at 166 104 / 99;  8192 x 2048 at the same 103 / 93, 183 / 131, 257 / 182, 59 / 84;  2048 x 8192 (eight
+    ranges, without the bytes of their sums) 107 / 87, 176 / 124, 246 / 207;  2048 x 2048 31 / 31, 46 / 43, 65 / 60;  2560 x
+    2048 at 1024 93 / 74.  Over 54 sizes that it takes, with what stands behind, 0.74 of the time before, none past 1.02."""
     if not SPLIT_ROWS[0] <= M <= SPLIT_ROWS[1] or N < 512 or K < 512 or K % 32 or N % (128 if glu else 4):
         return None
     best = None

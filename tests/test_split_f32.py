@@ -87,6 +87,31 @@ def test_infinities_and_the_ends_of_the_range():
 
 
 @gpu
+@pytest.mark.parametrize("sx,sw", [(-80, 0), (-112, 0), (-126, 0), (-140, 0), (0, -104), (0, -120), (0, -140), (-60, -60), (120, -118),
+                                   (-118, 120), (100, -135), (-135, 100), (-40, 127), (127, -40)])
+def test_small_and_large_numbers(sx, sw):
+    """Rows of one size as exact as those of another, down to the least numbers there are; some rows only, too."""
+    g = torch.Generator().manual_seed(9)
+    x0, w0 = torch.rand(70, 512, generator=g) * 2 - 1, torch.rand(200, 512, generator=g) * 2 - 1
+    for some in (False, True):
+        x, w = (x0.double() * 2.0 ** sx).float(), (w0.double() * 2.0 ** sw).float()
+        if some:
+            x[::3], w[::5] = x0[::3], w0[::5]
+        x, w = x.cuda(), w.cuda()
+        want = x.double() @ w.double().T
+        size = x.double().abs() @ w.double().abs().T
+        for mt in L.SPLIT_TILES:
+            for ranges in (1, 2):
+                y = _product(x, w, mt, ranges).double().sum(0)
+                # a share of the terms' sizes, and what fp32 cannot say below its least number;  terms that add up past its
+                # largest number (2^128) may overflow on the way, as they do in a plain fp32 sum
+                ok = ((y - want).abs() <= 2.0 ** -21 * size + 2.0 ** -148) | (size >= 2.0 ** 128)
+                assert bool(ok.all()), (mt, ranges)
+    (p, f), up = _split(x), 2.0 ** 64
+    assert set(f.tolist()) <= {1.0, 1 / up} and torch.equal((p.double().sum(0) * f.double()[:, None]).float(), x)
+
+
+@gpu
 def test_numbers_that_are_not():
     """NaN where a number of either row is, without a sum of its own for each, and nowhere else."""
     g = torch.Generator().manual_seed(11)
