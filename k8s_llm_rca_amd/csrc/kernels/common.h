@@ -57,6 +57,16 @@ __device__ __forceinline__ float relu_sq_f(float v) {
 // one, so the prompt and the decode form of a layer hold the same activations.
 __device__ __forceinline__ float silu_hw(float z) { return z * __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
 
+// The gate of SwiGLU, the quotient rounded to nearest.
+__device__ __forceinline__ float silu_gate(float z) { return z / (1.f + __expf(-z)); }
+// The same for |z| < 87, where nothing on the way leaves fp32's range: the approximate quotient and one step of Newton's, 4 of
+// the division's 11 instructions.  The same value for every bf16 z (tests/test_silu_gate.py).
+constexpr float kSiluNear = 86.f;         // (a number below it is one below 87 when rounded to bf16)
+__device__ __forceinline__ float silu_gate_near(float z) {
+  const float d = 1.f + __expf(-z), r = __builtin_amdgcn_rcpf(d), q = z * r;
+  return fmaf(fmaf(-d, q, z), r, q);
+}
+
 // RoPE of one (x[i], x[i + 64]) pair in a fixed operation order -- no choice
 // left to the compiler's contraction -- so every kernel that rotates (rope_kv,
 // the skinny and the prefill qkv GEMM epilogues) rounds identically.

@@ -106,7 +106,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_mid_kernel(const uint16_t* __res
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
             const float gv = bf2f(v[j]);
-            v[j] = f2bf(silu_hw(gv) * bf2f(xu[set][i][j]));
+            v[j] = f2bf(silu_gate(gv) * bf2f(xu[set][i][j]));
           }
         }
         *reinterpret_cast<u16x8*>(&xs[buf][xdst[i]]) = v;

@@ -163,7 +163,7 @@ __global__ void __launch_bounds__(64 * kStepWaves, 2)
   const int i = lane / G;
   if constexpr (OUT == kStepSilu) {
     const float fa = bf2f(f2bf(t)), fb = bf2f(f2bf(__shfl_xor(t, 32, 64)));   // rounded as the separate pass reads them
-    if (lane < 32 && lane % G == 0) reinterpret_cast<uint16_t*>(y)[n0 + i] = f2bf(silu_hw(fa) * fb);
+    if (lane < 32 && lane % G == 0) reinterpret_cast<uint16_t*>(y)[n0 + i] = f2bf(silu_gate(fa) * fb);
   } else if (lane % G == 0) {
     if constexpr (OUT == kStepF32)
       reinterpret_cast<float*>(y)[(size_t)blockIdx.y * N + n0 + i] = t;

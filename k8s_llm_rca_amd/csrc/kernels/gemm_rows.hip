@@ -258,7 +258,7 @@ __global__ void __launch_bounds__(kRowsWaves * 64, 2)
       uint16_t a = f2bf(total(m, n)), b = f2bf(total(m, HR + n));
       const float fa = bf2f(a), fb = bf2f(b);
       if constexpr (OUT == kRowsSilu) {       // gate and up rounded as the separate pass reads them
-        yb[(size_t)m * ldy + n0 + n] = f2bf(silu_hw(fa) * fb);
+        yb[(size_t)m * ldy + n0 + n] = f2bf(silu_gate(fa) * fb);
       } else {
         const int hd = (n0 + n) >> 6, d = (n0 + n) & 63;
         if (hd < rp.nq + rp.nkv) {

@@ -183,7 +183,7 @@ __global__ void __launch_bounds__(256) gemm_stream_kernel(const uint16_t* __rest
 #pragma unroll
           for (int cf = 0; cf < 2; ++cf)
             y[(size_t)m * ldy + n0 + 16 * cf + r] =
-                f2bf(silu_hw(bf2f(f2bf(acc[mt][cf][v]))) * bf2f(f2bf(acc[mt][cf + 2][v])));
+                f2bf(silu_gate(bf2f(f2bf(acc[mt][cf][v]))) * bf2f(f2bf(acc[mt][cf + 2][v])));
         }
       }
   } else if (gridDim.y == 1) {
@@ -401,7 +401,7 @@ __device__ __forceinline__ void glds_store(const f32x4 (&acc)[MTW][NF], int M, u
 #pragma unroll
           for (int cf = 0; cf < NF / 2; ++cf)
             y[(size_t)m * ldy + 16 * cf + r] =
-                f2bf(silu_hw(bf2f(f2bf(acc[mt][cf][v]))) * bf2f(f2bf(acc[mt][cf + NF / 2][v])));
+                f2bf(silu_gate(bf2f(f2bf(acc[mt][cf][v]))) * bf2f(f2bf(acc[mt][cf + NF / 2][v])));
         }
       }
     return;

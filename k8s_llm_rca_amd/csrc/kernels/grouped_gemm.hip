@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(256, 2) grouped_gemm_kernel(const uint16_t* __
       bf16x8 v;
       if constexpr (FUSE_SILU) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) v[t] = (__bf16)(silu_hw((float)sa[2 * i][t]) * (float)sa[2 * i + 1][t]);
+        for (int t = 0; t < 8; ++t) v[t] = (__bf16)(silu_gate((float)sa[2 * i][t]) * (float)sa[2 * i + 1][t]);
       } else {
         v = sa[i];
       }

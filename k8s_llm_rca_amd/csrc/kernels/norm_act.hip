@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(256) silu_mul_kernel(const uint16_t* __restric
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float gv = bf2f(g[j]);
-      o[j] = f2bf(silu_hw(gv) * bf2f(u[j]));
+      o[j] = f2bf(silu_gate(gv) * bf2f(u[j]));
     }
     *reinterpret_cast<u16x8*>(out + t * I + i * 8) = o;
   }
