@@ -376,8 +376,8 @@ def _turn_pairs(x: torch.Tensor, cs: torch.Tensor) -> torch.Tensor:
 LATENT_STEP_RANKS, LATENT_STEP_ROWS, LATENT_STEP_READ = (256, 512, 768, 1024, 1536, 2048), 16, 56 << 20
 
 
-def latent_up(dn: torch.Tensor, wq: torch.Tensor, wkv: torch.Tensor, w: torch.Tensor, slots: torch.Tensor,
-              cache: torch.Tensor, q_rank: int, kv_rank: int, eps: float, out_dtype, cache_t: Optional[torch.Tensor] = None,
+def latent_up(dn: torch.Tensor, wq: torch.Tensor, wkv: Optional[torch.Tensor], w: torch.Tensor, slots: torch.Tensor,
+              cache: Optional[torch.Tensor], q_rank: int, kv_rank: int, eps: float, out_dtype, cache_t: Optional[torch.Tensor] = None,
               tail: int = 0, tail_cs: Optional[torch.Tensor] = None) -> torch.Tensor:
     """:func:`latent_norm`, then its result ``@ w.T``.
 
@@ -388,7 +388,8 @@ def latent_up(dn: torch.Tensor, wq: torch.Tensor, wkv: torch.Tensor, w: torch.Te
     20.9, 18.7 / 25.7, 20.3 / 31.1."""
     from .linear import dispatch_table, proj
     T, N = dn.shape[-2], w.shape[0]
-    if 0 < T <= LATENT_STEP_ROWS and use_hip(dn):      # (before anything else: prompts pay for one comparison)
+    # (the rows before anything else: prompts pay for one comparison)
+    if 0 < T <= LATENT_STEP_ROWS and use_hip(dn) and wkv is not None and cache is not None:
         planes, pstep = (dn.shape[0], dn.stride(0)) if dn.dim() == 3 else (1, 0)
         pad = cache.shape[-1] - kv_rank
         small = ((wq, q_rank, out_dtype), (wkv, kv_rank, out_dtype), (tail_cs if tail else None, T * tail, torch.float32))

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from k8s_llm_rca_amd.ops import seq_ops as S
+from k8s_llm_rca_amd.ops.linear import proj
 
 pytestmark = pytest.mark.gpu
 BF, BS = torch.bfloat16, 32
@@ -37,3 +38,12 @@ def test_latent_up(monkeypatch, T, QR, KR, R, pad, N, planes):
     want = cq @ w.double().T
     # the normed rows rounded to bf16 (2^-9 of each term), fp32 sums, the result rounded; twice that
     assert bool(((q.double() - want).abs() <= 2.0 ** -8 * (cq.abs() @ w.double().abs().T + want.abs())).all())
+
+
+@pytest.mark.parametrize("T", [1, 16, 17])
+def test_queries_alone(T):
+    g = torch.Generator().manual_seed(T)
+    dn, wq = torch.randn(T, 256 + 64, generator=g).cuda(), torch.randn(256, generator=g).to(BF).cuda()
+    w, slots = torch.randn(64, 256, generator=g).to(BF).cuda(), torch.arange(T, dtype=torch.int32, device="cuda")
+    q = S.latent_up(dn, wq, None, w, slots, None, 256, 64, 1e-5, BF)          # no latent to write: as latent_norm has it
+    assert torch.equal(q, proj(S.latent_norm(dn, wq, None, slots, None, 256, 64, 1e-5, BF), w))
