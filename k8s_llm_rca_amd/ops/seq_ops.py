@@ -1472,7 +1472,7 @@ def attention_and_memory(x: torch.Tensor, H: int, G: int, D: int, V: int, positi
     49.9;  12 over 3 of 64 + 128 beside 32 of 64 x 64 10.6 / 6.9, 15.1 / 11.2, 37.3 / 33.4, 57.1 / 57.0.  Heads of 128 x 128 stay
     apart: their state does not fit beside the attention's registers."""
     # (the rows before anything else: prompts pay for one comparison)
-    step = _memory_step(xm, *memory) if xm.shape[0] == seg.n_seg and out_dtype == torch.bfloat16 else None
+    step = _memory_step(xm, *memory) if xm.shape[0] == seg.n_seg and out_dtype == torch.bfloat16 == memory[-1] else None
     if step is not None and (step.dim, step.vdim) != (128, 128):
         o = _prep_tokens(x, None, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, **prep, **mask, beside=step)
         if o is not None:

@@ -52,3 +52,17 @@ def test_same_bits(H, G, D, V, MH, MD, MV, pos, kind):
         got.append((o, m, kc, vt, *st))
     for a, b in zip(*got):
         assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+def test_results_of_two_types():
+    g = torch.Generator().manual_seed(3)
+    seg, slots = meta([40], 4)
+    x = torch.randn(1, 20 * 128 + 2 * 4 * 128 + 8, generator=g).cuda()
+    xm = x[:, 20 * 128:]
+    kc, vt = torch.zeros(4, BS, 256, dtype=BF, device="cuda"), torch.zeros(4, 256, BS, dtype=BF, device="cuda")
+    st = [torch.zeros(2, *s, device="cuda") for s in ((4, 64, 64), (4, 64), (4,))]
+    memory = (4, 64, 64, torch.zeros(8, device="cuda"), 15.0)
+    tail = (seg, None, 1e-5, torch.float32)               # the memory's result stays in fp32
+    o, m = S.attention_and_memory(x[:, :20 * 128], 16, 2, 128, 128, seg.seg_pos0, slots, kc, None, vt, seg, BF, 0.1,
+                                  dict(norm=True, eps=1e-5), {}, xm, *memory, *(s.clone() for s in st), *tail)
+    assert m.dtype == torch.float32 and torch.equal(m, S.memory_layer(xm, *memory, *st, *tail))
