@@ -1408,7 +1408,11 @@ def prep_attention(x: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int
                    out_dtype, scale: float, prep: dict, mask: dict) -> torch.Tensor:
     """:func:`attn_prep` (keywords ``prep``) and :func:`masked_attention` (keywords ``mask``) of the same rows; in one launch
     where every sequence has one row."""
-    o = _prep_tokens(x, bias, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, **prep, **mask)
+    return _prep_attention(x, bias, H, G, D, V, positions, slots, kc, vc, vt, seg, out_dtype, scale, prep, mask)
+
+
+def _prep_attention(x, bias, H, G, D, V, positions, slots, kc, vc, vt, seg, out_dtype, scale, prep, mask, beside=None):
+    o = _prep_tokens(x, bias, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, **prep, **mask, beside=beside)
     if o is not None:
         return o
     q = attn_prep(x, bias, H, G, D, V, positions, slots, kc, vc, out_dtype, vt=vt, **prep)
@@ -1418,6 +1422,7 @@ def prep_attention(x: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int
 def _prep_tokens(x, bias, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, norm=False, q_w=None, k_w=None, eps=0.0,
                  lam=0.0, v_other=None, v_keep=None, rope=None, rope_cs=None, softcap=0.0, chunk=0, window=0, keep_first=0,
                  sink=None, gate=None, beside=None) -> Optional[torch.Tensor]:
+    """``beside`` (:class:`_MemoryStep`): made in the same launch, and marked so, where that takes it."""
     T = x.shape[-2]
     if T != seg.n_seg:                               # (before anything else: prompts pay for one comparison)
         return None
@@ -1442,12 +1447,10 @@ def _prep_tokens(x, bias, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, 
                                         lambda: _mask_plan(seg, H, G, D, V, int(chunk), int(window), int(keep_first), 1))
     if D == 64 and T * G * -(-(H // G) // 16) * parts > PREP_GROUPS:
         return None
-    if beside is not None and not (H > G and D + V > 128 and softcap == 0.0 and parts < TOKEN_PARTS and MASK_TOKEN_BLOCKS <= 8):
-        return None
     out = torch.empty(T, H * V, dtype=out_dtype, device=x.device)
     groups, po, pml = _token_groups(rows, H, parts, V)
-    if beside is not None and len(groups) > 1:
-        return None
+    joint = (beside is not None and H > G and D + V > 128 and softcap == 0.0 and parts < TOKEN_PARTS and MASK_TOKEN_BLOCKS <= 8
+             and len(groups) == 1 and out_dtype == torch.bfloat16 == beside.out.dtype and (beside.dim, beside.vdim) != (128, 128))
     for it in groups:
         args = (
             ptr(x), x.stride(-2), planes, pstep, ptr(bias), ptr(q_w), ptr(k_w), float(eps), int(bool(norm)), ptr(rope_cs), rot,
@@ -1455,8 +1458,9 @@ def _prep_tokens(x, bias, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, 
             seg.block_tables.shape[1], ptr(it), it.shape[0], ptr(sink), ptr(gate), gate.stride(0) if gate is not None else 0,
             ptr(out), H, G, D, V, BS, int(chunk), int(window), int(keep_first), float(scale), float(softcap), stream_ptr(x),
             MASK_TOKEN_BLOCKS, TOKEN_PARTS, parts, ptr(pml), ptr(po))
-        if beside is not None:
+        if joint:
             check(lib().k8s_masked_attn_memory(*args, *beside.args), "masked_attn_memory")
+            beside.done = True
         else:
             check(lib().k8s_masked_attn_token_prep(*args), "masked_attn_token_prep")
     return out
@@ -1472,13 +1476,9 @@ def attention_and_memory(x: torch.Tensor, H: int, G: int, D: int, V: int, positi
     49.9;  12 over 3 of 64 + 128 beside 32 of 64 x 64 10.6 / 6.9, 15.1 / 11.2, 37.3 / 33.4, 57.1 / 57.0.  Heads of 128 x 128 stay
     apart: their state does not fit beside the attention's registers."""
     # (the rows before anything else: prompts pay for one comparison)
-    step = _memory_step(xm, *memory) if xm.shape[0] == seg.n_seg and out_dtype == torch.bfloat16 == memory[-1] else None
-    if step is not None and (step.dim, step.vdim) != (128, 128):
-        o = _prep_tokens(x, None, H, G, D, V, slots, kc, vc, vt, seg, out_dtype, scale, **prep, **mask, beside=step)
-        if o is not None:
-            return o, step.out
-    return (prep_attention(x, None, H, G, D, V, positions, slots, kc, vc, vt, seg, out_dtype, scale, prep, mask),
-            memory_layer(xm, *memory))
+    step = _memory_step(xm, *memory) if xm.shape[0] == seg.n_seg else None
+    o = _prep_attention(x, None, H, G, D, V, positions, slots, kc, vc, vt, seg, out_dtype, scale, prep, mask, beside=step)
+    return o, memory_layer(xm, *memory) if step is None else step.launch()
 
 
 # Prompt tiles cut over their keys where few of them would leave the chip idle behind a long context.  us, whole / cut, 16
@@ -1876,10 +1876,19 @@ class _MemoryStep:
         assert state.is_contiguous() and state.shape[1:] == (H, D, V) and nstate.is_contiguous()
         assert nstate.shape[1:] == (H, D) and mstate.is_contiguous() and mstate.shape[1:] == (H,)
         self.heads, self.dim, self.vdim = H, D, V
+        self.done = False
         self.out = torch.empty(x.shape[0], H * V, dtype=out_dtype, device=x.device)
         self.args = (ptr(x), x.stride(0), ptr(gate_bias), float(cap), ptr(state), ptr(nstate), ptr(mstate), ptr(seg.seg_pos0),
                      ptr(seg.seg_slot), ptr(gate), gate.stride(0), ptr(w), V if w is not None and w.numel() == H * V else 0,
                      ptr(self.out), H, D, V, float(eps), float(DEN_EPS))
+
+    def launch(self) -> torch.Tensor:
+        """The result, by a launch of its own if no other has made it."""
+        if not self.done:
+            check(lib().k8s_memory_step(*self.args[:14], _dt(self.out.dtype), self.out.shape[0], *self.args[14:],
+                                        stream_ptr(self.out)), "memory_step")
+            self.done = True
+        return self.out
 
 
 def _memory_gate(x: torch.Tensor, H: int, D: int, V: int) -> torch.Tensor:
@@ -1899,8 +1908,7 @@ def memory_layer(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tenso
     """:func:`matrix_memory`, then :func:`head_norm_gate` over each head with the gates that stand behind the values."""
     step = _memory_step(x, H, D, V, gate_bias, cap, state, nstate, mstate, seg, w, eps, out_dtype)
     if step is not None:
-        check(lib().k8s_memory_step(*step.args[:14], _dt(out_dtype), x.shape[0], *step.args[14:], stream_ptr(x)), "memory_step")
-        return step.out
+        return step.launch()
     gate = _memory_gate(x, H, D, V)
     o, mul = matrix_memory(x, H, D, V, gate_bias, cap, state, nstate, mstate, seg, defer_scale=True)
     return head_norm_gate(o, gate, w, H, V, eps, out_dtype, mul=mul)

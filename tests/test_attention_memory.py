@@ -21,11 +21,11 @@ def meta(pos, maxb):
                      state, n_single=n), slots
 
 
-@pytest.mark.parametrize("H,G,D,V", [(16, 2, 128, 128), (33, 1, 64, 128), (6, 2, 128, 64)])
+@pytest.mark.parametrize("H,G,D,V", [(16, 2, 128, 128), (33, 1, 64, 128), (6, 2, 128, 64), (2, 2, 128, 128), (4, 2, 64, 64)])
 @pytest.mark.parametrize("MH,MD,MV", [(16, 64, 128), (3, 64, 64), (5, 128, 64), (2, 128, 128)])
 @pytest.mark.parametrize("pos", [[0], [5, 300, 0, 700, 255], [30] * 20])
 @pytest.mark.parametrize("kind", ["plain", "window"])
-def test_same_bits(H, G, D, V, MH, MD, MV, pos, kind):
+def test_same_bits(monkeypatch, H, G, D, V, MH, MD, MV, pos, kind):
     n, maxb, g = len(pos), 12, torch.Generator().manual_seed(H + MH)
     cols, mcols = (H + G) * D + G * V, 2 * MH * (MD + MV) + 2 * MH
 
@@ -37,7 +37,8 @@ def test_same_bits(H, G, D, V, MH, MD, MV, pos, kind):
     gb, w = rnd(2 * MH), rnd(MV)
     st0 = [rnd(n + 1, MH, MD, MV) * 0.3, rnd(n + 1, MH, MD), rnd(n + 1, MH)]
     mask = dict(window=200, keep_first=40, sink=rnd(H)) if kind == "window" else {}
-    got = []
+    got, made, make = [], [], S._MemoryStep.__init__
+    monkeypatch.setattr(S._MemoryStep, "__init__", lambda self, *a: made.append(1) or make(self, *a))
     for one in (True, False):
         seg, slots = meta(pos, maxb)
         kc, vt, st = k0.clone(), v0.clone(), [s.clone() for s in st0]
@@ -50,6 +51,7 @@ def test_same_bits(H, G, D, V, MH, MD, MV, pos, kind):
             o = S.prep_attention(x[:, :cols], None, *args, prep, mask)
             m = S.memory_layer(x[:, cols:cols + mcols], *memory)
         got.append((o, m, kc, vt, *st))
+        assert len(made) == 2 - one                       # one step is prepared, joined or not
     for a, b in zip(*got):
         assert torch.isfinite(a).all() and torch.equal(a, b)
 
