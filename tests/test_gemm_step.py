@@ -87,15 +87,20 @@ def test_norm_form_and_the_products_behind(m, n, k, rn, add):
     for cols in (2048, 1088):
         wn = (_rand(g, cols, n) * n ** -0.5).to(BF)
         exact = (h.h.double() @ wn.double().T) * r
-        for got in (R.proj_f32out(h, wn), R.proj_planes(h, wn).sum(0)):
-            if L.rows_plan(m, cols, n, L.ROWS_F32) is not None:
-                _close(got, exact, n)
-        if L.rows_plan(m, cols, n) is not None:
-            _rounded(R.proj(h, wn), exact)
-        if L.rows_plan(m, cols // 2, n, L.ROWS_SILU) is not None:
-            gate, up = exact.split(cols // 2, 1)
-            s = torch.nn.functional.silu(gate) * up
-            assert bool(((R.glu_proj(h, wn).double() - s).abs() <= 2.0 ** -6 * s.abs() + 2e-3).all())
+        got = R.proj_f32out(h, wn), R.proj_planes(h, wn), R.proj(h, wn), R.glu_proj(h, wn)
+        plans = [L.rows_plan(m, cols, n, L.ROWS_F32), L.rows_plan(m, cols, n, L.ROWS_F32, True), L.rows_plan(m, cols, n, L.ROWS_BF16),
+                 L.rows_plan(m, cols // 2, n, L.ROWS_SILU)]
+        assert [p is None for p in plans] == [n % 512 != 0] * 4
+        if n % 512:                                         # a K that the dividing product does not take: normed rows, and the plain one
+            for a, plain in zip(got, (L.proj_f32out, L.proj_planes, L.proj, L.glu_proj)):
+                assert torch.equal(a, plain(full, wn))
+            continue
+        _close(got[0], exact, n)
+        _close(got[1].sum(0), exact, n)
+        _rounded(got[2], exact)
+        gate, up = exact.split(cols // 2, 1)
+        s = torch.nn.functional.silu(gate) * up
+        assert bool(((got[3].double() - s).abs() <= 2.0 ** -6 * s.abs() + 2e-3).all())
 
 
 @gpu
