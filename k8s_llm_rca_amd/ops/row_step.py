@@ -152,6 +152,8 @@ def dyt_step(x: torch.Tensor, y: Optional[torch.Tensor], sy: float, y2: Optional
 
 # ------------------------------------ a sublayer's last product with the residual's pass in its epilogue (gemm_step.hip)
 INTO_F32_ROWS = 4
+# loads a wave: a pair of kernels each.  Up to 8 every count; past that even ones alone are built, so that K of 9, 11, 13 and 15
+# times 512 (4608, 5632, ..) and past 8192 keep planes and the pass, with one row a RowStep.
 INTO_ROWS, INTO_LOADS, INTO_STRIP, PARTS = 16, (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16), 8, 256
 
 
