@@ -6,8 +6,8 @@
   loaded with ctypes *after* ``import torch`` so it binds to the same
   ``libamdhip64.so.7`` runtime torch already loaded (same SONAME).
 
-Both land next to this file so a ``gpurun`` snapshot carries them to the GPU
-box.  Rebuilds are incremental on CONTENT, not mtime: each
+Both land next to this file so a copy of the tree carries them to a GPU
+host.  Rebuilds are incremental on CONTENT, not mtime: each
 output has a ``.sha`` sidecar holding the SHA-256 of its compiler command,
 sources and headers, and anything whose digest differs is rebuilt -- a snapshot
 whose objects are newer than edited sources still recompiles.  Every compile
@@ -166,8 +166,7 @@ if __name__ == "__main__":
 
 
 def build_graphcore_sanitized(out_dir: str) -> str:
-    """Standalone test driver of the graph core under ASan + UBSan (host only;
-    SURVEY.md §5.2).  Returns the executable path."""
+    """Standalone test driver of the graph core under ASan + UBSan (host only).  Returns the executable path."""
     src = os.path.join(CSRC, "graph", "graphcore_test.cpp")
     exe = os.path.join(out_dir, "graphcore_test_asan")
     _run(["g++", "-O1", "-g", "-std=c++17", "-fsanitize=address,undefined", "-fno-omit-frame-pointer",

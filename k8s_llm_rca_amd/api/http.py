@@ -242,7 +242,7 @@ def create_app(service: AssistantService, engine=None, graphs: Optional[Dict[str
 
 
 def prometheus_text(service: AssistantService, engine=None) -> str:
-    """Prometheus exposition of run states and engine counters (SURVEY §5.5)."""
+    """Prometheus exposition of run states and engine counters."""
     from prometheus_client import CollectorRegistry, generate_latest
     from prometheus_client.core import CounterMetricFamily, GaugeMetricFamily
 

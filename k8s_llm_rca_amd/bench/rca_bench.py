@@ -1,4 +1,4 @@
-"""RCA benchmark: analyses/s and p50 end-to-end latency (BASELINE.json headline).
+"""RCA benchmark: analyses/s and p50 end-to-end latency.
 
 Each rank runs ``--incidents`` (128) concurrent RCA pipelines (locate ->
 generate query -> analyze, the full reference pipeline,
@@ -41,7 +41,7 @@ METRIC = "RCA analyses/sec + p50 end-to-end latency, Llama-3-8B backend, 10k-nod
 # the prefill is re-prefill after a cut (~half in the steady state), so they
 # are pinned here, checked against the backend and reported in the JSON config.
 TRUNCATION_CONTRACT = {"trunc_low": 0.5, "keep_seed": 2, "policy": "sticky"}
-REF_MAX_ANALYSES_PER_S = 0.033  # BASELINE.md: 1/(20 s + 10 s) best case of the sequential driver
+REF_MAX_ANALYSES_PER_S = 0.033  # 1/(20 s + 10 s) best case of the sequential driver
 
 
 def _tail_foreign(eng) -> int:
@@ -581,7 +581,7 @@ def parser() -> argparse.ArgumentParser:
     p = argparse.ArgumentParser(description=__doc__)
     p.add_argument("--gpus", type=int, default=None,
                    help="GPUs = ranks; without torchrun's WORLD_SIZE, bench.py spawns this many rank processes")
-    p.add_argument("--preset", default=None, choices=sorted(PRESETS), help="a BASELINE.json config")
+    p.add_argument("--preset", default=None, choices=sorted(PRESETS), help="a named workload")
     p.add_argument("--steps", type=int, default=10, help="timed steps; one step = --quantum completed analyses per GPU")
     p.add_argument("--warmup", type=int, default=3, help="untimed steps streamed before the timer starts")
     p.add_argument("--quantum", type=int, default=16, help="completed analyses per GPU per step")
@@ -608,7 +608,7 @@ def parser() -> argparse.ArgumentParser:
     # profiles/r5/curve/, profiles/r5/ab_defer96/) while p50 grows with concurrency
     # (Little's law: 17.6 s at 96, 18.7 s at 100, 19.2-19.9 s at 104, 20.2 s at 112,
     # 26.9 s at 128), so the default is the point with p50 a clear second under the
-    # reference's 20 s latency floor (BASELINE.md) at the plateau's throughput.
+    # reference's 20 s latency floor at the plateau's throughput.
     p.add_argument("--incidents", type=int, default=100,
                    help="concurrent RCA analyses (pipelines) per GPU (default: the p50 < 20 s operating point)")
     p.add_argument("--graph-nodes", type=int, default=10_000)
@@ -636,7 +636,7 @@ def parser() -> argparse.ArgumentParser:
     return p
 
 
-# One preset per BASELINE.json config; explicit flags override.
+# One preset per named workload; explicit flags override.
 PRESETS: Dict[str, Dict[str, Any]] = {
     # "OPT-125m CPU backend, 10-node toy k8s dependency graph, single pod-crash RCA (plumbing, no GPU)"
     "opt125m-cpu-toy": dict(model="opt-125m", device="cpu", graph_nodes=10, incidents=1, quantum=1, steps=1,

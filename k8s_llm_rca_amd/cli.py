@@ -21,7 +21,7 @@
                  in-process engine
 
 Backends: ``engine`` (MI355X LLM engine, default), ``opt-cpu`` (OPT-125m
-plumbing backend on CPU, BASELINE config 1) and ``oracle`` (scripted replies
+plumbing backend on CPU) and ``oracle`` (scripted replies
 from the grammar hints; no model).
 """
 from __future__ import annotations
@@ -146,7 +146,7 @@ def cmd_run(args) -> int:
                "analyses_per_s": round(st.analyses_per_s, 3),
                "p50_latency_s": round(st.pct(0.5), 3), "p90_latency_s": round(st.pct(0.9), 3),
                "errors": len(st.errors), "output": args.output}
-    if args.output:  # per-stage spans (and engine counters) next to the result file (SURVEY.md §5.1/§5.5)
+    if args.output:  # per-stage spans (and engine counters) next to the result file
         from .utils import tracing
         spans = {"stages": tracing.snapshot(), "summary": summary}
         if eng is not None:
@@ -232,7 +232,7 @@ def cmd_token_probe(args) -> int:
     assistant, two messages with a run each, then get_token_usage over the
     window.  The reference sleeps 60 s per run and uses int() second bounds;
     here each run is awaited and the window is taken in float seconds, so the
-    usage of fast runs is not lost (SURVEY.md §2 A1.8 quirk)."""
+    usage of fast runs is not lost."""
     from .api.assistant import GenericAssistant
     svc, eng = _service(args)
     tutor = GenericAssistant(svc)

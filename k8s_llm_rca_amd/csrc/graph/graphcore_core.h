@@ -1,7 +1,7 @@
 // Pure C++ core of the host graph operators (no Python): shared by the pybind11
 // module (graphcore.cpp) and the sanitizer test driver (graphcore_test.cpp),
 // so the exact code the extension runs is what ASan/UBSan exercise
-// (SURVEY.md §5.2).  See graphcore.cpp for what each operator replaces.
+// (see graphcore.cpp for what each operator replaces).
 #pragma once
 #include <cstdint>
 #include <cstring>

@@ -1,4 +1,4 @@
-// Custom all-reduce over xGMI peer memory (B14 in SURVEY.md §2 Part B; §5.8).
+// Custom all-reduce over xGMI peer memory.
 //
 // For the latency-bound TP all-reduces of decode (16 KiB .. a few MiB, two per
 // layer) RCCL's ring pays per-step launch + protocol latency; on a full xGMI

@@ -1,4 +1,4 @@
-// Paged GQA attention for gfx950 (B6 prefill / B7 decode in SURVEY.md §2 Part B).
+// Paged GQA attention for gfx950, prefill and decode.
 //
 // KV cache layout (per layer), page = BS tokens (BS % 32 == 0):
 //   K : [num_blocks][n_kv][BS][128]   row-major keys
@@ -421,10 +421,10 @@ __device__ __forceinline__ void decode_epilogue(const RowState& st, const AttnAr
   }
 }
 
-// (Round 2-3 also had an in-kernel split-KV merge by the last-arriving wave of
+// (There was also an in-kernel split-KV merge by the last-arriving wave of
 // each (row group, kv head), K8SRCA_DECODE_MERGE=1: its per-item ticket cost
 // what the separate reduce launch saves -- profiles/r2_decode_merge/ -- and it
-// was retired in round 4; attn_reduce_kernel merges.)
+// was retired; attn_reduce_kernel merges.)
 template <bool NT>
 __global__ void __launch_bounds__(64, 2) attn_decode_items_kernel(AttnArgs a) {
   const int lane = threadIdx.x;

@@ -326,7 +326,7 @@ __device__ __forceinline__ void glds_strip(const uint16_t* __restrict__ x, int l
         // out of order) would let a wait pass before its fragment landed.  No
         // instruction from before the block may move into it (this barrier), and
         // none from after it (glds_mm's barrier behind each column's MFMAs);
-        // the reads' own addresses are VALU / SALU arithmetic (ADVICE r4).
+        // the reads' own addresses are VALU / SALU arithmetic.
         __builtin_amdgcn_sched_barrier(0);
         bf16x8 xf[MTW], wf[NF];
 #pragma unroll

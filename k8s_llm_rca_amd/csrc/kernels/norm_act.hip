@@ -118,8 +118,7 @@ __global__ void __launch_bounds__(256) silu_mul_kernel(const uint16_t* __restric
 // order (split 0, then += 1, 2, ...) and rounded to bf16 before the rotation,
 // and the reduced (then rotated) row is stored back into qkv, so qkv, the K
 // page and the V page are bit-identical to reduce kernel + this kernel -- one
-// launch and one [T][ld] bf16 round trip fewer per layer of a decode step
-// (SURVEY B3 "fuse into the QKV-GEMM epilogue").
+// launch and one [T][ld] bf16 round trip fewer per layer of a decode step.
 template <bool PART>
 __device__ __forceinline__ u16x8 qkv_piece(const uint16_t* row, const float* prow, int col, int splits, size_t MN) {
   if constexpr (!PART) {

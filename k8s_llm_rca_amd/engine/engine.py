@@ -263,7 +263,7 @@ class LLMEngine(SchedulerMixin, StepExecMixin, GraphRunnerMixin, SamplerMixin):
         # path's row-chunked GEMM / all-reduce overlap: its depth AND transport (the
         # xGMI kernels vs RCCL) per bucket, timed here.  On a "nccl" group the
         # prefill-size buckets the executor carries are timed too, for the report
-        # (VERDICT r5 #2: RCCL measured against the xGMI kernels on the fabric);
+        # (RCCL measured against the xGMI kernels on the fabric);
         # the executor keeps its fused xGMI epilogue for them.
         H = int(L0["wo"].shape[0])
         big = [T for T in (1024, 2048, 4096, 8192, 16384)

@@ -1,4 +1,4 @@
-"""Response grammars for constrained decoding (SURVEY.md §7.4 hard part #1).
+"""Response grammars for constrained decoding.
 
 The reference pipeline only proceeds when GPT-4 returns a fenced JSON block
 with a valid ``DestinationKind`` (``find_srckind_metapath_neo4j.py:193-196``)

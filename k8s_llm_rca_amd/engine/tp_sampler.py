@@ -1,4 +1,4 @@
-"""Vocab-parallel sampling across the TP ranks (SURVEY B10): one object per
+"""Vocab-parallel sampling across the TP ranks: one object per
 TP engine rank, with the mask-table state it keeps.
 
 Each rank holds the LM head's rows for its vocab shard, so each rank samples

@@ -114,7 +114,7 @@ class EngineConfig:
     tokenizer: Optional[str] = None  # tokenizer.json (default: the checkpoint's, else the built-in BPE)
     temperature: float = 0.7
     use_hints: bool = True
-    logits_fp32: bool = True   # lm_head writes fp32 logits for the sampler (SURVEY B9)
+    logits_fp32: bool = True   # lm_head writes fp32 logits for the sampler
     # KV host tier (engine/kv_offload.py): GB of page-locked host memory that idle
     # threads' pages are swapped to instead of being dropped (0 = off; TP = 1)
     kv_host_gb: float = field(default_factory=lambda: _knob("kv_host_gb", 0.0))

@@ -1,4 +1,4 @@
-"""AST of the supported Cypher subset (SURVEY.md §2 'Cypher constructs G8 must accept')."""
+"""AST of the supported Cypher subset."""
 from __future__ import annotations
 
 from dataclasses import dataclass, field

@@ -1,7 +1,7 @@
 """Lexer + recursive-descent parser for the Cypher subset.
 
 Accepts every construct in the reference's own queries and generation
-template (SURVEY.md §2 'Cypher constructs G8 must accept'): node/relationship
+template: node/relationship
 patterns incl. ``-[*1..3]-``, named paths, WHERE with boolean / comparison /
 ``CONTAINS`` / ``IN`` / ``IS NULL`` / list predicates / slicing / ``$params``,
 ``WITH``, ``RETURN [DISTINCT] ... AS``, ``ORDER BY``, ``SKIP``, ``LIMIT``,

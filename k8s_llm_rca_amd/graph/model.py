@@ -1,7 +1,7 @@
 """Result objects returned by the in-process graph engine.
 
 They honour the record contract the reference pipeline relies on when it talks
-to Neo4j (SURVEY.md §1.2):
+to Neo4j:
 
 * ``record['n2.kind2']`` / ``record[0]`` / iteration / ``len(record)``
   (``find_metapath/find_srckind_metapath_neo4j.py:88``, ``generate_query/generate_query.py:106,110``)

@@ -1,8 +1,7 @@
 """Kubernetes resource schema used by the metagraph and the stategraph generator.
 
 The reference keeps this schema inside a Neo4j "metagraph" that is not part
-of its repository; it is reconstructed here from what the reference code reads
-(SURVEY.md §1.6):
+of its repository; it is reconstructed here from what the reference code reads:
 
 * kind nodes carry ``kind`` and ``category`` (``NativeEntity`` /
   ``ExternalEntity``; ``find_metapath/find_srckind_metapath_neo4j.py:63-72``);

@@ -1,4 +1,4 @@
-"""Columnar property-graph store (G1 in SURVEY.md §2 Part B).
+"""Columnar property-graph store.
 
 Replaces the two Neo4j servers the reference talks to over Bolt
 (``common/neo4j_query_executor.py:6-24``).  Layout:

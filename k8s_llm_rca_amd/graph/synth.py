@@ -1,7 +1,7 @@
 """Synthetic Kubernetes stategraph generator with fault injection (G9).
 
 The reference diagnoses incidents against a Neo4j dump of a real cluster that
-is not in its repository (SURVEY.md §1.6, §4).  This module builds an
+is not in its repository.  This module builds an
 equivalent instance-level graph deterministically from a seed:
 
 * entity nodes labelled by kind (``id``, ``kind2``, ``isNative``, ``isAtomic``,

@@ -221,7 +221,7 @@ def push_native(L=None) -> None:
         fn(slot, int(getattr(KNOBS, name)))
 
 
-# knob -> the module constant it was copied into at import (ADVICE r5: changing
+# knob -> the module constant it was copied into at import (changing
 # such a knob in a running process has no effect, so it is refused)
 AT_IMPORT = {f.name: f.metadata["at_import"] for f in fields(Knobs) if f.metadata.get("at_import")}
 

@@ -1,6 +1,6 @@
-"""Model presets for every backend named in BASELINE.json.
+"""Model presets of every backend.
 
-Shapes are the public architectures (SURVEY.md §2 Part B):
+Shapes are the public architectures:
 Llama-3-8B / 70B (GQA, RoPE theta 5e5), Mixtral-8x7B (8 experts top-2, theta
 1e6, vocab 32000) and OPT-125m (LayerNorm, ReLU, learned positions; the CPU
 plumbing backend).  ``tiny-*`` presets keep the same structure at test size.

@@ -69,7 +69,7 @@ class LlamaModel:
         self.layers: List[Dict[str, torch.Tensor]] = []
         self.moe: Optional[MOE.MoELayerSet] = None
         self.init_mode = init_mode
-        self.logits_f32 = True  # SURVEY B9: the sampler reads fp32 logits (EngineConfig.logits_fp32)
+        self.logits_f32 = True  # the sampler reads fp32 logits (EngineConfig.logits_fp32)
         if init:
             self._random_init(seed)
 

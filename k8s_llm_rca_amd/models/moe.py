@@ -101,7 +101,7 @@ class MoELayerSet:
         Prefill-sized batches run the grouped form of the 8-phase prefill GEMM
         (``ops/moe.py grouped_big``): gate_up with its SwiGLU epilogue, then
         down, two launches over every expert with the offsets read on the
-        device -- no ``offsets.tolist()`` host sync per layer (VERDICT r3), no
+        device -- no ``offsets.tolist()`` host sync per layer, no
         silu_mul launch.  The per-expert hipBLASLt loop remains only for shapes
         that kernel does not take."""
         H = x_perm.shape[1]

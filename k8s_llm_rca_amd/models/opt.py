@@ -1,4 +1,4 @@
-"""OPT-125m decoder -- the CPU plumbing backend (B16).
+"""OPT-125m decoder -- the CPU plumbing backend.
 
 Pre-LayerNorm blocks, learned positions (offset 2), ReLU FFN, MHA with
 biases, lm_head tied to the token embedding.  Uses the same paged KV pool and

@@ -1,6 +1,6 @@
 """Checkpoint IO: Hugging-Face-format safetensors <-> the engine's sharded layout.
 
-SURVEY.md §5.4: benchmarks use seeded random weights, but a user switching
+Benchmarks use seeded random weights, but a user switching
 from the reference (GPT-4 behind an API) wants real open weights.  This loads
 a HF Llama-3 / Mixtral checkpoint directory (``config.json`` + ``*.safetensors``
 + ``tokenizer.json``) straight into this rank's tensor-parallel shards:

@@ -246,7 +246,7 @@ def scratch(shape, dtype, device) -> torch.Tensor:
 
 
 def check(rc: int, name: str) -> None:
-    """Raise on a launch error.  ``K8SRCA_SYNC_DEBUG=1`` (SURVEY.md §5.2 debug
+    """Raise on a launch error.  ``K8SRCA_SYNC_DEBUG=1`` (a debug
     mode) also synchronises after every kernel so an asynchronous fault is
     reported at the op that caused it, not at a later sync."""
     if rc != 0:

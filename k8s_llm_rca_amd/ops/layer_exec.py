@@ -72,13 +72,13 @@ NORM_FUSE_MAX_T = 4
 # 2, 4 rows 15 / 11.8, 15 / 14.2, 15 / 18.4, 28672 x 4096 SwiGLU 40 / 36.3, 40.5 / 38.4, 40 / 44)
 NORM_FUSE_ROWS_T = 2
 NORM_FUSE_MAX_H = 4096      # norm_prologue.h: 256 threads, two 16-byte pieces each
-# (Round 3 also carried a row-chunked o / down GEMM with each chunk's
+# (There was also a row-chunked o / down GEMM with each chunk's
 # all-reduce on a side stream, and the prefill attention on a side stream beside
 # the decode attention: both measured as losses -- profiles/r3/ab/tp_overlap_*,
-# profiles/r3/overlap/ -- and were retired from the executor in round 4.)
+# profiles/r3/overlap/ -- and were retired from the executor.)
 # Mixed steps as two nano-batch layer stacks on two streams (decode rows beside
-# prefill rows, ops/layer_exec.py LlamaExecutor._run_nano); off by default: see
-# README "Round 6" for the measurement
+# prefill rows, ops/layer_exec.py LlamaExecutor._run_nano); off by default:
+# the README has the measurement
 _nano = KNOBS.nano_batch
 NANO_MIN_DECODE = 32
 NANO_MIN_PREFILL = 512

@@ -367,7 +367,7 @@ def lib_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor = None) -> torc
 
 def linear_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` with fp32 output (bf16 operands, fp32 accumulate): the
-    lm_head, whose logits the sampler reads in fp32 (SURVEY B9)."""
+    lm_head, whose logits the sampler reads in fp32."""
     if x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.stride(1) == 1 \
             and w.is_contiguous():
         M, K = x.shape
@@ -728,7 +728,7 @@ def reserve_big_ws(dev: torch.device, enable: bool = None) -> None:
 
 # ------------------------------------------------ hipBLASLt solution tables
 # (Engine-init tuning of hipBLASLt solutions over an M ladder lost 4 % end to
-# end -- profiles/r1_blaslt_tune_8b.txt -- and was retired in round 4; the
+# end -- profiles/r1_blaslt_tune_8b.txt -- and was retired; the
 # bucketed table below, verified per bucket, stays.)
 
 

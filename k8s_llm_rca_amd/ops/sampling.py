@@ -12,7 +12,7 @@ import torch
 
 from ._lib import check, lib, ptr, stream_ptr, use_hip
 
-CAND_K = 64  # per-rank candidates of a vocab-parallel top-k / top-p row (SURVEY B10: k <= 64)
+CAND_K = 64  # per-rank candidates of a vocab-parallel top-k / top-p row (k <= 64)
 
 
 def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor], seeds: Optional[torch.Tensor],

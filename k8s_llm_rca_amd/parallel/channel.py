@@ -5,8 +5,8 @@ layer; two all-reduces per layer), but only rank 0 owns the scheduler.  The
 step metadata -- token ids, positions, KV slots, block tables, the attention
 work plan, sampling inputs -- therefore travels from rank 0 to the workers
 every step.  Sending it as device tensors over RCCL made each worker block on
-a ``.cpu()`` of the header to size the next receive (a full GPU sync per step,
-VERDICT r1 weak #5).  This channel moves the metadata between HOST memories
+a ``.cpu()`` of the header to size the next receive (a full GPU sync per
+step).  This channel moves the metadata between HOST memories
 (gloo over loopback on one node): a worker receives step k+1's inputs while
 its GPU is still executing step k, uploads them with a pinned async copy and
 issues the forward -- the GPUs synchronise only inside the forward, at the

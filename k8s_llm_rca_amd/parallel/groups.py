@@ -88,7 +88,7 @@ class ParallelContext:
         k = k row chunks, chunk i's all-reduce on the comm stream beside chunk
         i+1's GEMM) AND its transport -- the xGMI kernels (two-shot over the
         hipIpc buffers, buffer-sized chunks past it) or RCCL's multi-channel
-        rings (the north star's RCCL path is measured against
+        rings (the RCCL path is measured against
         the custom kernels per bucket, not assumed away) -- timed ON THIS
         FABRIC with the real row-parallel weights [(name, w [H, K_local])].
         ``transports``: subset of ("xgmi", "rccl"); default every one this

@@ -1,6 +1,6 @@
 """Per-rank projection of a TP / EP deployment on ONE GPU (``bench --tp-sim N``).
 
-The 8-GPU configs of BASELINE.json (Llama-3-70B TP=8, Mixtral EP=8) cannot be
+The 8-GPU deployments (Llama-3-70B TP=8, Mixtral EP=8) cannot be
 run on a one-GPU box, but what one rank of them computes can: this context
 builds **rank 0's shard at the real shapes** (70B: 8 q / 1 kv heads,
 intermediate 3,584, vocab shard 16,032 per rank) and runs the real engine on
@@ -35,7 +35,7 @@ from ..ops._lib import lib, stream_ptr
 from .groups import ParallelContext
 from .xgmi import ONE_SHOT_MAX, _bind, _check, linear_push_addnorm, push_ok
 
-XGMI_LINK_GBPS = 153.0   # one xGMI link, per direction (SURVEY §5.8: 7 links per GPU)
+XGMI_LINK_GBPS = 153.0   # one xGMI link, per direction (7 links per GPU)
 XGMI_HOP_US = 2.5        # one flag hand-off across the fabric (signal -> visible on the peer)
 HOP_SENSITIVITY_US = (2.5, 5.0, 10.0)  # the projection is also reported at these hop latencies
 RCCL_BUS_GBPS = 300.0    # assumed RCCL all-reduce bus bandwidth on an 8-GPU xGMI node (not measured here)

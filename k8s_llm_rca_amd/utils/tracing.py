@@ -1,4 +1,4 @@
-"""Lightweight span recorder + ROCTX ranges (SURVEY.md §5.1).
+"""Lightweight span recorder + ROCTX ranges.
 
 ``span(name)`` records wall time per stage into a process-wide aggregator
 (count / total / max) and, when ``K8SRCA_ROCTX=1`` and
