@@ -86,6 +86,7 @@ constexpr int HALF_B = 128 * BK * 2;  // bytes per half-tile (16 KB)
 constexpr int BUF_B = 4 * HALF_B;     // one K-tile (64 KB)
 constexpr int OX0 = 0, OX1 = HALF_B, OW0 = 2 * HALF_B, OW1 = 3 * HALF_B;
 constexpr int GM = 4;  // M tiles per tile group
+constexpr int kRowParts = 16;  // parts of a row's sum of squares, at most
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
@@ -181,6 +182,9 @@ struct RopeArgs {
   uint16_t* vc;          // [blocks][nkv][128][BS]
   int nq, nkv, BS;
   float scale;           // MODE 4
+  const float* part;     // SCALED: [M][parts], row m is divided by sqrt(sum(part[m]) / width + eps) (gemm_add.hip)
+  int parts;
+  float width, eps;
 };
 
 // MODE 0: plain (N output columns = W rows); MODE 1: SwiGLU (N = I output
@@ -192,7 +196,9 @@ struct RopeArgs {
 // VAR bit 0: ping-pong stagger of waves
 // 4-7; bit 1: s_setprio(1) around the MFMA clusters; bit 2: the 32x32x16 MFMA
 // (1 = the default).
-template <int MODE, int VAR>
+// SCALED: MODE 1 of rows that are divided first (RopeArgs::part): 16384 x 8192 x 2048 808 us for 806 of the plain form.  The factors lie
+// behind the staged tiles: in front of them, with the tiles from 1 KB on, the main loop took a fifth longer (1000 us).
+template <int MODE, int VAR, bool SCALED = false>
 __global__ void __launch_bounds__(512, 1) gemm_big_kernel(const uint16_t* __restrict__ x, int ldx,
                                                           const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
                                                           int ldy, int M, int N, int K, int n_mt, int n_nt, int splits,
@@ -200,11 +206,12 @@ __global__ void __launch_bounds__(512, 1) gemm_big_kernel(const uint16_t* __rest
                                                           float* __restrict__ tws, int* __restrict__ tick,
                                                           const int* __restrict__ goffs, int G, RopeArgs ra,
                                                           const int* __restrict__ rowmap, int rdiv) {
+  static_assert(!SCALED || MODE == 1);
   constexpr int SH = (VAR & 4) ? 32 : 16;
   using GG = Geo<SH>;
   using acc_t = typename GG::acc_t;
   constexpr int XT = GG::XT, WT = GG::WT, KS = GG::KS;
-  __shared__ __attribute__((aligned(1024))) unsigned char sm[2 * BUF_B];
+  __shared__ __attribute__((aligned(1024))) unsigned char sm[2 * BUF_B + (SCALED ? 4 * BM : 0)];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wv >> 2, wc = wv & 3;
@@ -301,6 +308,16 @@ __global__ void __launch_bounds__(512, 1) gemm_big_kernel(const uint16_t* __rest
       for (int j = 0; j < WT; ++j) acc[q][i][j] = acc_t{};
   bf16x8 xf[XT][KS], wf0[WT][KS], wf1[WT][KS];
 
+  // the rows' factors: asked for in front of the first tiles, two threads a row
+  float* const rfac = reinterpret_cast<float*>(sm + 2 * BUF_B);
+  float rp[SCALED ? kRowParts / 2 : 1];
+  if constexpr (SCALED) {
+    const float* q = ra.part + (size_t)min(m0 + (tid >> 1), M - 1) * ra.parts;
+#pragma unroll
+    for (int i = 0; i < kRowParts / 2; ++i) rp[i] = q[min(2 * i + (tid & 1), ra.parts - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
   // prologue: tile 0 whole, tile 1's X half 0 and W half 0 (the main loop's issue order)
   issue(xs[0], OX0, 0);
   issue(wsrc[0], OW0, 0);
@@ -308,6 +325,13 @@ __global__ void __launch_bounds__(512, 1) gemm_big_kernel(const uint16_t* __rest
   issue(xs[1], OX1, 0);
   issue(xs[0], BUF_B + OX0, 1);
   issue(wsrc[0], BUF_B + OW0, 1);
+  if constexpr (SCALED) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < kRowParts / 2; ++i) t += 2 * i + (tid & 1) < ra.parts ? rp[i] : 0.f;
+    t += __shfl_xor(t, 1, 64);
+    if (!(tid & 1)) rfac[tid >> 1] = 1.f / sqrtf(t / ra.width + ra.eps);
+  }
   asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // this wave's part of X0h(0), W0h(0)
   bar();
   if ((VAR & 1) && wr == 1) bar();  // waves 4-7 run one barrier behind
@@ -609,6 +633,16 @@ __global__ void __launch_bounds__(512, 1) gemm_big_kernel(const uint16_t* __rest
   // 1240, 4351 rows 261 / 257 / 253, 8000 x 14336 x 4096 1346 / 1340 / 1336.
   bool near = false;
   if constexpr (MODE == 1) {
+    if constexpr (SCALED) {
+#pragma unroll
+      for (int Q = 0; Q < 4; ++Q)
+#pragma unroll
+        for (int i = 0; i < XT; ++i) {
+          const float f = rfac[128 * (Q >> 1) + 64 * wr + SH * i + frow];
+#pragma unroll
+          for (int j = 0; j < WT; ++j) acc[Q][i][j] *= f;
+        }
+    }
     float most = 0.f;
 #pragma unroll
     for (int Q = 0; Q < 4; ++Q)
@@ -745,7 +779,7 @@ static void tail_plan(int T, int nt, int& r, int& S) {
 // host state of the issuing thread, like the executor's launch sequence)
 static thread_local RopeArgs g_rope{};
 
-template <int MODE, int VAR>
+template <int MODE, int VAR, bool SCALED = false>
 static int launch(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int splits,
                   float* part, hipStream_t s) {
   const int n_mt = (M + BM - 1) / BM, n_nt = MODE == 1 ? N / 128 : N / BN;
@@ -775,7 +809,7 @@ static int launch(const void* x, int ldx, const void* w, void* y, int ldy, int M
     }
   }
   const int grid = splits > 1 ? T * splits : T - tr + tr * ts;
-  hipLaunchKernelGGL((gemm_big_kernel<MODE, VAR>), dim3(grid), dim3(512), 0, s, (const uint16_t*)x, ldx,
+  hipLaunchKernelGGL((gemm_big_kernel<MODE, VAR, SCALED>), dim3(grid), dim3(512), 0, s, (const uint16_t*)x, ldx,
                      (const uint16_t*)w, (uint16_t*)y, ldy, M, N, K, n_mt, n_nt, splits, part, tr, ts, tws, tick,
                      (const int*)nullptr, 0, g_rope, (const int*)nullptr, 1);
   return (int)hipGetLastError();
@@ -813,6 +847,9 @@ static int big_launch(const void* x, int ldx, const void* w, void* y, int ldy, i
       case 5: rc = launch<0, 5>(x, ldx, w, y, ldy, M, N, K, splits, pp, s); break;
       default: rc = launch<0, 7>(x, ldx, w, y, ldy, M, N, K, splits, pp, s); break;
     }
+  } else if (mode == 1 && g_rope.part) {
+    if (var != 1) return (int)hipErrorInvalidValue;
+    rc = launch<1, 1, true>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s);
   } else if (mode == 1) {
     rc = (var & 4) ? launch<1, 5>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s)
                    : launch<1, 1>(x, ldx, w, y, ldy, M, N, K, 1, nullptr, s);
@@ -912,6 +949,18 @@ K8S_API int k8s_gemm_big_rope(const void* x, int ldx, const void* w, void* qkv, 
     return (int)hipErrorInvalidValue;
   g_rope = RopeArgs{pos, cos_sin, slots, (uint16_t*)kc, (uint16_t*)vc, nq, nkv, BS};
   const int rc = big_launch(x, ldx, w, qkv, ldq, M, N, K, 2, var, 1, nullptr, true, s);
+  g_rope = RopeArgs{};
+  return rc;
+}
+
+// k8s_gemm_big's mode 1, row m of both products divided by sqrt(sum(part[m][parts]) / width + eps) before they are rounded.
+K8S_API int k8s_gemm_big_silu_scaled(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, const float* part,
+                                     int parts, float width, float eps, hipStream_t s) {
+  using namespace k8s::big;
+  if (!part || parts < 1 || parts > kRowParts || !(width > 0.f)) return (int)hipErrorInvalidValue;
+  g_rope = RopeArgs{};
+  g_rope.part = part, g_rope.parts = parts, g_rope.width = width, g_rope.eps = eps;
+  const int rc = big_launch(x, ldx, w, y, ldy, M, N, K, 1, 1, 1, nullptr, true, s);
   g_rope = RopeArgs{};
   return rc;
 }

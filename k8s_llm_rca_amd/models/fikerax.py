@@ -32,7 +32,7 @@ import torch
 from ..ops import norm as N
 from ..ops import row_step as R
 from ..ops import seq_ops as S
-from ..ops.linear import proj_add, proj_planes
+from ..ops.linear import proj_planes
 from ..parallel.groups import ParallelContext, single
 
 TAIL_ALIGN = 32     # the rotated key part of a latent cache row is filled up to a multiple of this
@@ -437,7 +437,7 @@ class FikeraxModel:
             x = R.residual(h, x)
             w = L["wo"]
             if spec.ff:
-                h = R.add_product(x, y, w, one, mix1, L["norm2"], eps, dt, rms=rms)
+                h = R.add_product(x, y, w, one, mix1, L["norm2"], eps, dt, rms=rms, glu=L["w13"])
                 y, w, rms = R.glu_proj(h, L["w13"]), L["w2"], None               # silu(gate) * up
                 x = R.residual(h, x)
             if layers_out is not None:                     # the residual in front of the embedding added once more
@@ -447,9 +447,7 @@ class FikeraxModel:
             if nxt:
                 h = R.add_product(x, y, w, one, mix1, eps=eps, out_dtype=dt, rms=rms, **nxt)
             else:
-                y = proj_planes(y, w) if rms is not None else proj_add(x[:, 0], y, w)
-                if y is not None:
-                    N.hyper_step(x, y, one, mix1, rms=rms)
+                R.add_rest(x, y, w, one, mix1, rms)
         h = R.rows(h, idx) if few else N.hyper_read(x, idx, self.final_norm, eps, dt)
         return self.logits(h) if head else h
 

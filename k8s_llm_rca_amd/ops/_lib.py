@@ -67,6 +67,9 @@ _SIGS = {
     "k8s_gemm_big_grouped": [P, I, P, P, I, P, I, I, I, I, I, I, P, P, I],
     "k8s_gemm_big_rope": [P, I, P, P, I, I, I, I, P, P, P, P, P, I, I, I, I, P],
     "k8s_gemm_big_add": [P, I, P, P, I, I, I, I, F, P],
+    "k8s_gemm_big_silu_scaled": [P, I, P, P, I, I, I, I, P, I, F, F, P],
+    "k8s_gemm_add": [P, I, P, P, F, P, I, F, F, P, P, F, I, F, P, P, P, P, I, I, I, I, P],
+    "k8s_add_rows": [P, I, P, F, P, I, F, F, P, P, F, I, F, P, P, P, P, I, I, P],
     "k8s_gemm_big_ws_bytes": [],
     "k8s_gemm_big_set_ws": [P],
     "k8s_gemm_big_claim_ws": [P],

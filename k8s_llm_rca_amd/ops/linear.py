@@ -568,6 +568,102 @@ def proj_add(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, scale: float = 1
     return None
 
 
+# -------------------- a prompt's products added to the residual, with what reads it next (csrc/kernels/gemm_add.hip)
+THEN_NOTHING, THEN_DYT, THEN_SCALED = 0, 1, 2
+# us of a wave of 256 tiles by rows of a tile / 32: at no K, and more for each entry of K (2048 columns at K 1024, 2048, 8192: 25,
+# 38, 121 with 128 rows, 29, 45, 136 with 160, 32, 53, 160 with 192, 43, 70, 193 with 256)
+ADD_WAVES = {4: (11.5, 0.01318), 5: (14.5, 0.0147), 6: (15.5, 0.0174), 8: (21.0, 0.0206)}
+ADD_MAX_N = 5120
+
+
+def _add_wave(M: int, N: int, K: int, f: int) -> float:
+    full, over = divmod(-(-M // (32 * f)) * (N // 256), 256)
+    t = ADD_WAVES[f][0] + ADD_WAVES[f][1] * K
+    return full * t + ((0.75 + 0.25 * over / 256) * t if over else 0.0)
+
+
+@functools.lru_cache(maxsize=4096)
+def add_plan(M: int, N: int, K: int, then: int):
+    """Row ranges (from, to, rows of a tile / 32) in which :func:`gemm_add` makes a product of ``M`` rows, or None: the product and
+    the pass behind it are the quicker.  Tiles that leave the least of their last wave of 256 idle, or whole waves of them and other
+    tiles, or (0) a product and a pass of its own, for the rest.
+
+    Taken by what the same work takes in whole waves of 256-row tiles, over what it takes so.  Time of product and pass over this,
+    at 0.40 of the whole waves' rate 0.86 (with tanh) and 0.98 (scaled), 0.48 1.00 and 1.17, 0.55 0.98 - 1.08 and 1.00 - 1.14, 0.66
+    1.13 - 1.18 and 1.25, 0.80 1.05 - 1.27 and 1.11 - 1.37, 1.00 1.01 - 1.19 and 1.01 - 1.27, over 1024 to 5120 columns and a K of
+    1024 to 14336.  Without a norm there is the pass that reads it left (with its time, product and pass over both: at 0.55 0.95 -
+    1.00, 0.66 1.01 - 1.06, 0.80 0.99 - 1.17, 0.85 1.00 - 1.20), and from ADD_ROWS on the product that adds itself (0.82 0.90, 0.86
+    0.98 - 1.17, 1.00 0.96 - 1.08: it stays)."""
+    if N % 256 or N > ADD_MAX_N or K % 64 or not 1024 <= K <= 16384 or M < 512 or then == THEN_NOTHING and M >= ADD_ROWS:
+        return None
+    nt = N // 256
+    best = min((_add_wave(M, N, K, f), ((0, M, f),)) for f in ADD_WAVES)
+    for f in ADD_WAVES:
+        for waves in range(1, -(-M // (32 * f)) * nt // 256 + 1):
+            cut = 256 * waves // nt * 32 * f
+            rest = M - cut
+            if rest <= 0:
+                break
+            c, g = min((_add_wave(rest, N, K, g), g) for g in ADD_WAVES)
+            apart = 10.0 + rest * N * K / 3.5e8 + rest * N / 2e5
+            if rest < 512 and apart < c:
+                c, g = apart, 0
+            best = min(best, (_add_wave(cut, N, K, f) + c, ((0, cut, f), (cut, M, g))))
+    whole = M * N / 2.0 ** 24 * (ADD_WAVES[8][0] + ADD_WAVES[8][1] * K)
+    return best[1] if whole >= (0.6 if then == THEN_NOTHING else 0.5) * best[0] else None
+
+
+def gemm_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, scale: float, plan, then: int, alpha: float = 0.0, nw=None,
+             nb=None, rms=None, again=None):
+    """``x += scale * (a @ w.T)`` on the fp32 residual ``x`` [M, N] by :func:`add_plan`; ``then`` the activations behind it:
+    ``tanh(alpha x) nw + nb``, or ``x nw`` and the sums of squares of the rows in parts [M, N / 256].  ``rms = (ss, width, eps)``: the
+    product's rows are divided by ``sqrt(sum(ss[m]) / width + eps)``;  ``again = (ids, embed, escale)``: ``embed[ids] * escale`` is
+    added too."""
+    (M, K), N = a.shape, w.shape[0]
+    h = torch.empty(M, N, dtype=a.dtype, device=x.device) if then else None
+    part = torch.empty(M, N // 256, dtype=torch.float32, device=x.device) if then == THEN_SCALED else None
+    ss, width, reps = rms if rms is not None else (None, 1.0, 0.0)
+    ids, embed, escale = again if again is not None else (None, None, 0.0)
+    rn = ss.shape[1] if ss is not None else 0
+    s = stream_ptr(x)
+    for lo, hi, f in plan:
+        def at(t, row):
+            return 0 if t is None else ptr(t) + t.element_size() * lo * row
+        rest = (at(x, N), float(scale), at(ss, rn), rn, float(width), float(reps), at(ids, 1), ptr(embed), float(escale), then,
+                float(alpha), ptr(nw), ptr(nb), at(h, N), at(part, N // 256), hi - lo, N)
+        if f:
+            check(lib().k8s_gemm_add(at(a, a.stride(0)), a.stride(0), ptr(w), *rest, K, f, s), "gemm_add")
+        else:
+            y = proj_planes(a[lo:hi], w)
+            check(lib().k8s_add_rows(ptr(y), y.shape[0], *rest, s), "add_rows")
+    return h, part
+
+
+def add_ok(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Layout :func:`gemm_add` needs of the residual [M, N] (or [M, 1, N]) and the operands."""
+    return (_few_ok(a, w) and a.shape[1] == w.shape[1] and x.dtype == torch.float32 and x.is_contiguous()
+            and x.data_ptr() % 16 == 0 and x.numel() == a.shape[0] * w.shape[0] and x.device == a.device == w.device)
+
+
+def silu_scales(M: int, w: torch.Tensor) -> bool:
+    """Whether :func:`glu_proj` of ``M`` rows is gemm_big's fused form, which can divide the rows of both products."""
+    N, K = w.shape[0] // 2, w.shape[1]
+    return (M > DISPATCH_MAX_M and w.dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0 and w.shape[0] == 2 * N
+            and K % 256 == 0 and K // 256 <= 16 and swiglu_choice(M, 2 * N, K, False) is None and big_shape_ok(M, N, K, True)
+            and big_fused(M, N, K, True))
+
+
+def gemm_big_silu_scaled(x: torch.Tensor, w: torch.Tensor, part: torch.Tensor, eps: float) -> torch.Tensor:
+    """:func:`glu_proj` of the rows ``x`` divided by ``sqrt(sum(part[m]) / K + eps)``."""
+    (M, K), N = x.shape, w.shape[0] // 2
+    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    if x.device not in _big_ws and _big_tail:
+        reserve_big_ws(x.device)
+    check(lib().k8s_gemm_big_silu_scaled(ptr(x), x.stride(0), ptr(w), ptr(out), N, M, N, K, ptr(part), part.shape[1], float(K),
+                                         float(eps), stream_ptr(x)), "gemm_big_silu_scaled")
+    return out
+
+
 def proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` as activations, with the 32-column stream form where it is the fastest: 17 to 128 rows (below, the skinny
     kernel) and one wave of strips with the K it was measured at.  us at 17..32 / 64 / 128 rows, hipBLASLt / this:

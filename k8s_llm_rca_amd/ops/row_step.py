@@ -193,6 +193,10 @@ class Scaled:
         return Scaled(*(t.index_select(0, idx) for t in (self.x, self.h, self.part)), self.nw, self.eps)
 
     def product(self, w: torch.Tensor, out_kind: int, plain, planes: bool = False, keep: bool = False):
+        if self.h.shape[0] > INTO_ROWS:
+            if out_kind == L.ROWS_SILU and L.silu_scales(self.h.shape[0], w) and w.shape[1] == self.h.shape[1]:
+                return L.gemm_big_silu_scaled(self.h, w, self.part, self.eps)
+            return plain(self.read(), w)
         if self.h.dtype == torch.float32:
             return self._product_f32(w, out_kind, plain, planes)
         (m, k), n = self.h.shape, w.shape[0] // (2 if out_kind == L.ROWS_SILU else 1)
@@ -238,13 +242,19 @@ def _into_f32(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def add_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, one: torch.Tensor, mix: torch.Tensor, nw: torch.Tensor,
-                eps: float, out_dtype, again: Optional[tuple] = None, rms: Optional[tuple] = None):
+                eps: float, out_dtype, again: Optional[tuple] = None, rms: Optional[tuple] = None,
+                glu: Optional[torch.Tensor] = None):
     """The next sublayer's input behind ``x += a @ w.T`` (:func:`step` of that product): activations, :class:`RowStep` or
-    :class:`Scaled`."""
+    :class:`Scaled`.  ``glu``: the weight of the gated product that is the only one to read it."""
     if a.shape[0] <= INTO_ROWS:                      # (before anything else: prompts pay for one comparison)
         h = _rms_into(x, a, w, nw, eps, out_dtype, again, rms)
         if h is not None:
             return h
+    elif out_dtype == torch.bfloat16 == a.dtype:
+        then = L.THEN_SCALED if glu is not None and glu.shape[1] == w.shape[0] and L.silu_scales(a.shape[0], glu) else L.THEN_NOTHING
+        made = _add(x, a, w, 1.0, then, nw, None, 0.0, rms, again)
+        if made is not None:
+            return Scaled(x, *made, nw, eps) if then else N.hyper_read(x, None, nw, eps, out_dtype)
     if again is None and rms is None:
         y = L.proj_add(x[:, 0], a, w)
         if y is None:
@@ -252,6 +262,33 @@ def add_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, one: torch.Te
     else:                                            # (a pass that reads the embedding once more adds the product too)
         y = L.proj_planes(a, w)
     return step(x, y, one, mix, nw, eps, out_dtype, again=again, rms=rms)
+
+
+def _add(x, a, w, scale, then, nw, nb, alpha, rms=None, again=None):
+    """:func:`..ops.linear.gemm_add` where it pays and takes the operands (None: nothing has been done)."""
+    M, N = a.shape[0], w.shape[0]
+    plan = L.add_plan(M, N, a.shape[1], then)
+    if plan is None or not L.add_ok(x, a, w) or x.shape[-1] != N or x.dim() == 3 and x.shape[1] != 1:
+        return None
+    if then and not (_fp32_row(nw, N) and (nb is None or _fp32_row(nb, N))):
+        return None
+    if rms is not None and not (rms[0].dtype == torch.float32 and rms[0].is_contiguous() and rms[0].dim() == 2
+                                and rms[0].shape[0] == M and 0 < rms[0].shape[1] <= SUMS):
+        return None
+    if again is not None and not (again[0].dtype == torch.int32 and again[0].is_contiguous() and again[0].numel() == M
+                                  and again[1].dtype == torch.bfloat16 and again[1].is_contiguous() and again[1].shape[1] == N
+                                  and again[1].data_ptr() % 8 == 0):
+        return None
+    return L.gemm_add(x, a, w, scale, plan, then, alpha, nw, nb, rms, again)
+
+
+def add_rest(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, one: torch.Tensor, mix: torch.Tensor, rms: Optional[tuple] = None):
+    """``x += a @ w.T`` [T, 1, W], with nothing that reads it behind (``rms`` as in :func:`..ops.norm.hyper_step`)."""
+    if a.shape[0] > INTO_ROWS and a.dtype == torch.bfloat16 and _add(x, a, w, 1.0, L.THEN_NOTHING, None, None, 0.0, rms) is not None:
+        return
+    y = L.proj_planes(a, w) if rms is not None else L.proj_add(x[:, 0], a, w)
+    if y is not None:
+        N.hyper_step(x, y, one, mix, rms=rms)
 
 
 def _rms_into(x, a, w, nw, eps, out_dtype, again, rms) -> Optional[Scaled]:
@@ -289,12 +326,32 @@ def dyt_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, sy: float, a2
                                       ptr(w2), float(sy2), ptr(x), float(alpha), ptr(nw), ptr(nb), ptr(h), m, W, k,
                                       stream_ptr(x)), "gemm_step_dyt")
         return h
+    if m > INTO_ROWS and out_dtype == torch.bfloat16 == a.dtype and x.dim() == 2:
+        h = _dyt_add(x, a, w, sy, a2, w2, sy2, alpha, nw, nb)
+        if h is not None:
+            return h
     y = L.proj_add(x, a, w, sy)
     if a2 is None:
         return dyt_step(x, y, sy, None, 1.0, alpha, nw, nb, out_dtype)
     y2 = L.proj_add(x, a2, w2, sy2)
     add = (y, sy, y2, sy2) if y is not None else (y2, sy2, None, 1.0)
     return dyt_step(x, *add, alpha, nw, nb, out_dtype)
+
+
+def _dyt_add(x, a, w, sy, a2, w2, sy2, alpha, nw, nb) -> Optional[torch.Tensor]:
+    """A prompt's products by :func:`..ops.linear.gemm_add`: the second of two, or the only one, leaves the activations."""
+    if nw is None:
+        return None
+    if a2 is None:
+        made = _add(x, a, w, sy, L.THEN_DYT, nw, nb, alpha)
+        return made and made[0]
+    M, W = x.shape
+    if not (L.add_plan(M, W, a2.shape[1], L.THEN_DYT) and L.add_ok(x, a2, w2) and L.add_ok(x, a, w) and _fp32_row(nw, W)
+            and _fp32_row(nb, W) and (M >= L.ADD_ROWS or L.add_plan(M, W, a.shape[1], L.THEN_NOTHING))):
+        return None
+    if _add(x, a, w, sy, L.THEN_NOTHING, None, None, 0.0) is None:
+        L.proj_add(x, a, w, sy)                      # (adds itself from ADD_ROWS on)
+    return _add(x, a2, w2, sy2, L.THEN_DYT, nw, nb, alpha)[0]
 
 
 # ------------------------------------------------------------------------- products of activations, or of what makes them
