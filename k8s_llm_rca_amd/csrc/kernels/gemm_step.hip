@@ -7,24 +7,33 @@
 //
 // A reply step is a chain of launches, in which the residual's pass between two products (sums of the K ranges, addition,
 // norm) was one of 4.6 us that moves some 100 KB.  For the epilogue to own its columns a workgroup takes 8 rows of W over all
-// of K: 256 workgroups at 2048 columns, every wave with an eighth of K and its whole share of W (NB loads) asked for up
-// front.  A load covers 8 rows x 128 bytes, whole lines.  The matrix instruction takes such a register as it is: columns 0 - 7
-// hold the rows' first 64 bytes, 8 - 15 the second, and where A is laid out the same way (up to 8 rows), the two diagonal
-// blocks of its result are the two halves of K; the blocks beside them are of no use.  (9 to 16 rows: one instruction with
-// each half of K of A, of which the result keeps the matching columns.)
+// of K: 256 workgroups at 2048 columns, every wave with an eighth of K and its whole share of W and A asked for up front, in
+// turn.  A load covers 8 rows x 128 bytes, whole lines, neighbouring lanes neighbouring pieces of a row, and is turned into
+// fragments in the wave's own LDS (piece p of row r at p ^ r: no bank conflicts).  The matrix instruction takes what 8 rows of
+// 128 bytes hold as it is: columns 0 - 7 are the rows' first 64 bytes, 8 - 15 the second, and where A is laid out the same way
+// (up to 8 rows), the two diagonal blocks of its result are the two halves of K; the blocks beside them are of no use.  (9 to 16
+// rows: one instruction with each half of K of A, of which the result keeps the matching columns.)
 //
-// What bounds it is the weights' way from memory, and from some rows on that of A, which every workgroup reads whole (2048 x
-// 8192 at 1, 8, 16 rows 8.1, 10.1, 13.5 us; without A's loads 7.9).  A and W are asked for in turn: all of A first 8.9, 10.4,
-// 14.6, all of W first 8.8, 10.9, 14.9.  us in a replayed chain with cold weights, planes (gemm_rows.hip), the pass and the
-// product behind it / this and the product that divides:  2048 x 8192 in front of 8192 x 2048 at 2, 5, 8 rows 18.4 / 15.6,
-// 18.6 / 16.3, 18.9 / 17.6;  2048 x 2048 in front of SwiGLU 16384 x 2048 at 2, 7, 16 rows 19.1 / 16.9, 19.5 / 17.4, 20.9 /
-// 19.2;  at one row, against the pass in front of the product (gemm_row_step.hip), 15.5 / 15.5 and 16.5 / 16.7.
+// What bounds it is the weights' way from memory; of A every workgroup reads all rows.  Loaded in fragment order (neighbouring
+// lanes in different rows), W and A came at 36 KB a us and compute unit out of the second-level cache, where rows of 128 bytes
+// come at 84, and A's share took as long as W's: us at 1, 4, 7, 8, 12, 16 rows so / turned in LDS:  2048 x 8192 8.2 / 8.0, 9.2 / 8.3,
+// 9.9 / 8.4, 10.3 / 8.8, 12.1 / 9.9, 13.4 / 10.5;  2048 x 2048 4.1 / 4.0, 4.4 / 4.1, 4.6 / 4.2, 4.7 / 4.2, 5.1 / 4.6, 5.6 / 4.8;  4096 x
+// 4096 8.0 / 7.9, 9.1 / 7.9, 10.2 / 8.5, 10.4 / 8.9, 12.6 / 9.9, 13.6 / 10.6;  6144 x 8192 20.4 / 19.4, 23.2 / 19.9, 26.2 / 21.0, 27.6 /
+// 21.5, 33.2 / 27.1, 37.0 / 28.6.  (4 slots of LDS a wave, with 9 rows and more 2, so that two workgroups fit a compute unit: 4096 x
+// 4096 at 16 rows 12.9 with four.)
 #include "common.h"
 
 namespace k8s {
 
 constexpr int kSpWaves = 8, kSpCols = 8, kSpStep = 64;    // K entries of a load instruction
 constexpr int kSpMaxLoads = 16, kSpMaxRows = 16, kSpSums = 64;
+
+// LDS of one wave: what its lanes wrote is there for its other lanes
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 struct StepProduct {
   const uint16_t* a;     // [M][lda]
@@ -46,6 +55,8 @@ struct StepProduct {
 // grid: strips of 8 rows of W.  MF: 8-row halves of the matrix instruction that A fills.
 template <int NB, int MF>
 __global__ void __launch_bounds__(64 * kSpWaves, 2) gemm_step_kernel(StepProduct p, int M, int N, int K) {
+  constexpr int SLOTS = MF == 1 ? 4 : 2, RING = NB < SLOTS ? NB : SLOTS;
+  __shared__ __attribute__((aligned(16))) uint16_t turn[kSpWaves][RING][8 * (MF + 1) * kSpStep];    // A's rows, then W's
   __shared__ float red[kSpWaves][2][8 * MF][kSpCols];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int r = lane & 15, g = lane >> 4;
@@ -72,17 +83,24 @@ __global__ void __launch_bounds__(64 * kSpWaves, 2) gemm_step_kernel(StepProduct
   // ---- this wave's K range, of the first or the second product
   const bool two = p.w2 != nullptr, second = two && wv >= kSpWaves / 2;
   const int kbeg = (second ? wv - kSpWaves / 2 : wv) * NB * kSpStep;
-  const uint16_t* wp = (second ? p.w2 : p.w) + (size_t)(n0 + (r & 7)) * K + kbeg + 8 * ((r >> 3) * 4 + g);
+  const uint16_t* wp = (second ? p.w2 : p.w) + (size_t)(n0 + (lane >> 3)) * K + kbeg + 8 * (lane & 7);
   const uint16_t* a = second ? p.a2 : p.a;
   const int lda = second ? p.lda2 : p.lda;
-  const uint16_t* ap = MF == 1 ? a + (size_t)min(r & 7, M - 1) * lda + kbeg + 8 * ((r >> 3) * 4 + g)
-                               : a + (size_t)min(r, M - 1) * lda + kbeg + 8 * g;
-  bf16x8 wq[NB], aq[NB][MF];
+  // A: lane -> row lane / 8 (of each 8), piece lane % 8 of 128 bytes, which lies at piece ^ row in LDS
+  const int ar = lane >> 3, apc = lane & 7;
+  const uint16_t* ap[MF];
+#pragma unroll
+  for (int f = 0; f < MF; ++f) ap[f] = a + (size_t)min(8 * f + ar, M - 1) * lda + kbeg + 8 * apc;
+  u16x8 wq[NB];
+  u16x8 aq[NB][MF];
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
-    wq[i] = ldw_nt<bf16x8>(wp + i * kSpStep);
+    wq[i] = ldw_nt<u16x8>(wp + i * kSpStep);
 #pragma unroll
-    for (int f = 0; f < MF; ++f) aq[i][f] = *reinterpret_cast<const bf16x8*>(ap + i * kSpStep + 32 * f);
+    for (int f = 0; f < MF; ++f) {
+      if constexpr (MF == 1) aq[i][f] = u16x8{};
+      if (MF == 2 || ar < M) aq[i][f] = *reinterpret_cast<const u16x8*>(ap[f] + i * kSpStep);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
   float ev = 0.f;
@@ -91,10 +109,23 @@ __global__ void __launch_bounds__(64 * kSpWaves, 2) gemm_step_kernel(StepProduct
   f32x4 acc[MF];
 #pragma unroll
   for (int f = 0; f < MF; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // fragments: MF 1: row r % 8, a piece of the half r / 8;  MF 2: row r, a piece of each half
+  const int fr = MF == 1 ? r & 7 : r, fp = MF == 1 ? (r >> 3) * 4 + g : g;
 #pragma unroll
-  for (int i = 0; i < NB; ++i)
+  for (int i = 0; i < NB; ++i) {
+    uint16_t* at = turn[wv][i % RING];
 #pragma unroll
-    for (int f = 0; f < MF; ++f) acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aq[i][f], wq[i], acc[f], 0, 0, 0);
+    for (int f = 0; f < MF; ++f) *reinterpret_cast<u16x8*>(at + (8 * f + ar) * kSpStep + 8 * (apc ^ ar)) = aq[i][f];
+    uint16_t* wt = at + 8 * MF * kSpStep;
+    *reinterpret_cast<u16x8*>(wt + ar * kSpStep + 8 * (apc ^ ar)) = wq[i];
+    wave_lds_fence();
+    const bf16x8 wf = *reinterpret_cast<const bf16x8*>(wt + (r & 7) * kSpStep + 8 * (((r >> 3) * 4 + g) ^ (r & 7)));
+#pragma unroll
+    for (int f = 0; f < MF; ++f) {
+      const bf16x8 af = *reinterpret_cast<const bf16x8*>(at + fr * kSpStep + 8 * ((fp + 4 * f) ^ (fr & 7)));
+      acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, wf, acc[f], 0, 0, 0);
+    }
+  }
   // acc[f][v]: row 4 g + v, column r (8 - 15: the second 64 bytes of the rows)
   if constexpr (MF == 1) {
     if ((g >> 1) == (r >> 3)) {

@@ -573,7 +573,7 @@ THEN_NOTHING, THEN_DYT, THEN_SCALED = 0, 1, 2
 # us of a wave of 256 tiles by rows of a tile / 32: at no K, and more for each entry of K (2048 columns at K 1024, 2048, 8192: 25,
 # 38, 121 with 128 rows, 29, 45, 136 with 160, 32, 53, 160 with 192, 43, 70, 193 with 256)
 ADD_WAVES = {4: (11.5, 0.01318), 5: (14.5, 0.0147), 6: (15.5, 0.0174), 8: (21.0, 0.0206)}
-ADD_MAX_N = 5120
+ADD_MIN_ROWS, ADD_MAX_N = 512, 5120
 
 
 def _add_wave(M: int, N: int, K: int, f: int) -> float:
@@ -594,7 +594,7 @@ def add_plan(M: int, N: int, K: int, then: int):
     1024 to 14336.  Without a norm there is the pass that reads it left (with its time, product and pass over both: at 0.55 0.95 -
     1.00, 0.66 1.01 - 1.06, 0.80 0.99 - 1.17, 0.85 1.00 - 1.20), and from ADD_ROWS on the product that adds itself (0.82 0.90, 0.86
     0.98 - 1.17, 1.00 0.96 - 1.08: it stays)."""
-    if N % 256 or N > ADD_MAX_N or K % 64 or not 1024 <= K <= 16384 or M < 512 or then == THEN_NOTHING and M >= ADD_ROWS:
+    if N % 256 or N > ADD_MAX_N or K % 64 or not 1024 <= K <= 16384 or M < ADD_MIN_ROWS or then == THEN_NOTHING and M >= ADD_ROWS:
         return None
     nt = N // 256
     best = min((_add_wave(M, N, K, f), ((0, M, f),)) for f in ADD_WAVES)

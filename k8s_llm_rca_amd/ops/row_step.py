@@ -157,24 +157,43 @@ INTO_F32_ROWS = 4
 INTO_ROWS, INTO_LOADS, INTO_STRIP, PARTS = 16, (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16), 8, 256
 
 
-def into_ok(m: int, n: int, k: int, two: bool = False) -> bool:
-    """Whether a product of ``m`` rows takes the residual's pass into its epilogue (``two``: two products of K ``k`` do).
-
-    Every workgroup of 8 columns reads all of X, and with few columns there are few of them, where planes may cut K.  us of
-    planes and the norm's pass / of the fused product, and with the tanh pass:  2048 x 8192 at 1, 4, 8 rows 10.2 / 8.1, 11.0 /
-    8.9, 11.2 / 10.1 and 10.2 / 8.1, 10.4 / 8.8, 10.6 / 10.1, at 16 rows (8.4 and the pass) 13.5;  2048 x 2048 at 1, 8, 16
-    rows 6.5 / 4.4, 6.7 / 5.0, 6.9 / 5.8;  x 4096 at 16 8.9 / 8.2 and 8.2 / 8.2.  More columns: 3072 x 2048 at 12, 16 rows 8.5 /
-    7.6, 8.7 / 8.4 and 7.6 / 7.7, 7.9 / 8.2;  4096 x 4096 at 8, 12 rows 11.5 / 10.3, 11.8 / 12.4 and 10.5 / 10.1, 10.8 / 12.4;
-    6144 x 8192 at 2, 8 rows 26.5 / 21.9, 26.0 / 26.9.  Fewer:  1024 x 4096 at 8, 12 rows 7.0 / 6.2, 7.1 / 7.3;  1024 x 8192 at
-    2, 4 rows 8.1 / 7.5, 8.2 / 8.4;  512 x 4096 at 2, 8 rows 5.8 / 5.0, 5.8 / 6.1, x 8192 at 1 6.2 / 6.9, x 2048 at 16 5.7 / 5.4."""
+def _into_fits(m: int, n: int, k: int, two: bool) -> bool:
+    """What csrc/kernels/gemm_step.hip takes (``two``: two products of K ``k``), of weights without a measured kernel."""
     waves = 4 if two else 8
-    if not (0 < m <= INTO_ROWS and n > 0 and n % INTO_STRIP == 0 and k % (64 * waves) == 0
-            and k // (64 * waves) in INTO_LOADS and (n, k) not in L.dispatch_table()):
-        return False
-    k *= 2 if two else 1
+    return (0 < m <= INTO_ROWS and n > 0 and n % INTO_STRIP == 0 and k % (64 * waves) == 0 and k // (64 * waves) in INTO_LOADS
+            and (n, k) not in L.dispatch_table())
+
+
+def into_ok(m: int, n: int, k: int, two: bool = False) -> bool:
+    """Whether a product of ``m`` rows takes the residual's pass into its epilogue: sizes at which little of X is read
+    (:func:`into_long`: those past them)."""
+    return _into_fits(m, n, k, two) and _into_few(m, n, k * 2 if two else k)
+
+
+def _into_few(m: int, n: int, k: int) -> bool:
     if n < 1536:
         return k <= 2048 or k <= 4096 and m * k <= (32768 if n >= 1024 else 8192)
     return m * k * -(-n // 2048) <= (65536 if n <= 2048 else 49152)
+
+
+def into_long(m: int, n: int, k: int, two: bool = False) -> bool:
+    """The sizes past :func:`into_ok` that take it too: every K up to 4096, and of longer ones as much as its workgroups of 8
+    columns, each of which reads all of X, can read meanwhile.  us of planes and the norm's pass / of the fused product, and with
+    the tanh pass:  2048 x 2048 at 1, 8, 16 rows 6.5 / 4.0, 7.0 / 4.2, 7.2 / 4.8 and 5.9 / 4.0, 6.3 / 4.2, 6.6 / 4.6;  x 4096 at 16
+    8.6 / 6.5 and 8.0 / 6.7;  x 8192 at 1, 8, 9, 16 11.2 / 8.3, 11.2 / 8.3, 11.4 / 9.7, 11.6 / 10.6 and 10.6 / 8.3, 10.5 / 8.2, 10.5 /
+    9.5, 11.0 / 10.5.  With the tanh pass:  3072 x 8192 at 9, 12, 16 rows 16.0 / 15.8, 16.6 / 16.8, 17.1 / 17.8;  4096 x 4096 at 16 11.2 /
+    10.3, x 8192 at 9, 12 18.0 / 17.4, 17.7 / 18.0;  6144 x 4096 at 16 14.3 / 14.0, x 8192 at 4, 8, 9 24.8 / 19.2, 24.9 / 20.6, 24.9 / 24.8.
+    Fewer columns:  1024 x 4096 at 16 6.6 / 6.0, x 8192 at 4, 8, 9 7.5 / 6.5, 7.6 / 7.3, 7.6 / 8.2;  512 x 4096 at 16 5.8 / 5.6, x 8192 at
+    2, 4, 8 5.9 / 5.8, 5.9 / 6.1, 6.2 / 6.8."""
+    fits = _into_fits(m, n, k, two) and n <= 6144
+    k *= 2 if two else 1
+    if not fits or _into_few(m, n, k):
+        return False
+    if k <= 4096:
+        return True
+    if n < 1536:
+        return n >= 1024 and m * k <= 65536
+    return m * k * -(-n // 2048) < 196608
 
 
 class Scaled:
@@ -250,7 +269,7 @@ def add_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, one: torch.Te
         h = _rms_into(x, a, w, nw, eps, out_dtype, again, rms)
         if h is not None:
             return h
-    elif out_dtype == torch.bfloat16 == a.dtype:
+    elif a.shape[0] >= L.ADD_MIN_ROWS and out_dtype == torch.bfloat16 == a.dtype:
         then = L.THEN_SCALED if glu is not None and glu.shape[1] == w.shape[0] and L.silu_scales(a.shape[0], glu) else L.THEN_NOTHING
         made = _add(x, a, w, 1.0, then, nw, None, 0.0, rms, again)
         if made is not None:
@@ -284,7 +303,7 @@ def _add(x, a, w, scale, then, nw, nb, alpha, rms=None, again=None):
 
 def add_rest(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, one: torch.Tensor, mix: torch.Tensor, rms: Optional[tuple] = None):
     """``x += a @ w.T`` [T, 1, W], with nothing that reads it behind (``rms`` as in :func:`..ops.norm.hyper_step`)."""
-    if a.shape[0] > INTO_ROWS and a.dtype == torch.bfloat16 and _add(x, a, w, 1.0, L.THEN_NOTHING, None, None, 0.0, rms) is not None:
+    if a.shape[0] >= L.ADD_MIN_ROWS and a.dtype == torch.bfloat16 and _add(x, a, w, 1.0, L.THEN_NOTHING, None, None, 0.0, rms) is not None:
         return
     y = L.proj_planes(a, w) if rms is not None else L.proj_add(x[:, 0], a, w)
     if y is not None:
@@ -296,8 +315,8 @@ def _rms_into(x, a, w, nw, eps, out_dtype, again, rms) -> Optional[Scaled]:
     ids, embed, escale = again if again is not None else (None, None, 0.0)
     ss, width, reps = rms if rms is not None else (None, 1.0, 0.0)
     f32 = out_dtype == torch.float32
-    fits = (_into_f32(x, a, w) if f32 else into_ok(m, W, k) and _into_operands(x, a, w, out_dtype) and W % 32 == 0
-            and W // INTO_STRIP <= PARTS)
+    fits = (_into_f32(x, a, w) if f32 else (into_ok(m, W, k) or into_long(m, W, k)) and _into_operands(x, a, w, out_dtype)
+            and W % 32 == 0 and W // INTO_STRIP <= PARTS)
     if not (fits and x.shape[:2] == (m, 1) and _fp32_row(nw, W)
             and (ss is None or ss.dtype == torch.float32 and ss.is_contiguous() and ss.shape[0] == m
                  and 0 < ss.numel() <= SUMS * m)
@@ -318,15 +337,17 @@ def dyt_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, sy: float, a2
                 out_dtype):
     """The next sublayer's input behind ``x += sy a @ w.T (+ sy2 a2 @ w2.T)`` (:func:`dyt_step` of those products)."""
     (m, k), W = a.shape, x.shape[-1]
-    if (m <= INTO_ROWS and nw is not None and into_ok(m, W, k, a2 is not None) and _into_operands(x, a, w, out_dtype)
-            and x.shape == (m, W) and (a2 is None or a2.shape == a.shape and _into_operands(x, a2, w2, out_dtype))
+    two = a2 is not None
+    if (m <= INTO_ROWS and nw is not None and (into_ok(m, W, k, two) or into_long(m, W, k, two))
+            and _into_operands(x, a, w, out_dtype) and x.shape == (m, W)
+            and (a2 is None or a2.shape == a.shape and _into_operands(x, a2, w2, out_dtype))
             and _fp32_row(nw, W) and _fp32_row(nb, W)):
         h = torch.empty(m, W, dtype=out_dtype, device=x.device)
         check(lib().k8s_gemm_step_dyt(ptr(a), a.stride(0), ptr(w), float(sy), ptr(a2), a2.stride(0) if a2 is not None else 0,
                                       ptr(w2), float(sy2), ptr(x), float(alpha), ptr(nw), ptr(nb), ptr(h), m, W, k,
                                       stream_ptr(x)), "gemm_step_dyt")
         return h
-    if m > INTO_ROWS and out_dtype == torch.bfloat16 == a.dtype and x.dim() == 2:
+    if m >= L.ADD_MIN_ROWS and out_dtype == torch.bfloat16 == a.dtype and x.dim() == 2:
         h = _dyt_add(x, a, w, sy, a2, w2, sy2, alpha, nw, nb)
         if h is not None:
             return h
