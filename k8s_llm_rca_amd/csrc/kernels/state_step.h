@@ -13,8 +13,13 @@
 // A workgroup has a head of one sequence (V = 4 LV, D = DR RG), or of KIND 2 a slice of its columns; a thread four neighbouring columns of DR rows RG apart, so a
 // wave's accesses to the state are whole lines.  Nothing waits for anything but the state's address: rows,
 // gates and state are asked for together.  What bounds it: the state's bytes, read and written once (64 KB a head each way):
-// where every unit has one or two heads, memory (KIND 2, 16 heads of 128 x 128, 32 sequences 13.5 us, 5 TB/s); with fewer, the
-// rate of a unit, some 40 KB a us of both (7 sequences 5.9 us, of which a launch takes 2.6).
+// where every unit has several heads, memory;  with fewer, the rate of a unit, some 40 KB a us of both (7 sequences 4.7 us, of
+// which a launch takes 2.6).  A step reads the model's weights between two visits to a state, so that no cache holds it: it is
+// read and written without a place in the second-level cache (non-temporal), which would else have its written lines to give back
+// when the kernel ends.  us as ordinary / non-temporal accesses of states no cache holds:  KIND 2, 16 heads of 128 x 128, 1, 7, 16, 32,
+// 64 sequences 3.7 / 3.3, 6.1 / 4.7, 9.9 / 6.9, 17.9 / 12.8, 34 / 26 (5.2 TB/s; either alone 33 and 28);  KIND 1, 16 of 64 x 128,
+// 1, 5, 16, 32, 64 4.6 / 4.3, 5.1 / 4.7, 6.9 / 5.5, 10.6 / 7.7, 19.3 / 15.1;  KIND 0 5.1 / 4.7, 5.5 / 5.0, 7.1 / 5.8, 10.9 / 7.9, 18.3 /
+// 14.4;  8 of 64 x 64 at 64 7.2 / 5.6 and 7.5 / 6.0.
 #pragma once
 #include "common.h"
 #include "gates.h"
@@ -146,7 +151,7 @@ __device__ __forceinline__ void state_step_head(const StepArgs& a, int it, int h
   float* st = a.state + ((size_t)slot * H + hh) * D * V + c;
   f32x4 S[DR];
 #pragma unroll
-  for (int i = 0; i < DR; ++i) S[i] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : ss_ld4(st + (size_t)(rg + RG * i) * V);
+  for (int i = 0; i < DR; ++i) S[i] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : ldw_nt<f32x4>(st + (size_t)(rg + RG * i) * V);
   f32x4 gt = f32x4{0.f, 0.f, 0.f, 0.f}, w = f32x4{1.f, 1.f, 1.f, 1.f};
   if (tid < LV) {
     if (!LOW) gt = ss_ld4((const TG*)a.gate + (size_t)it * a.gs + hh * V + c);
@@ -252,7 +257,7 @@ __device__ __forceinline__ void state_step_head(const StepArgs& a, int it, int h
         S[i][j] = fmaf(fa, S[i][j], kd * (KIND == 1 ? ia * v[j] : v[j]));
       acc[j] = fmaf(S[i][j], qd, acc[j]);
     }
-    if (on) *reinterpret_cast<f32x4*>(st + (size_t)(rg + RG * i) * V) = S[i];
+    if (on) __builtin_nontemporal_store(S[i], reinterpret_cast<f32x4*>(st + (size_t)(rg + RG * i) * V));
   }
   acc = sum_rows<LV>(acc, red[1], tid);
   if (tid >= 64) return;
