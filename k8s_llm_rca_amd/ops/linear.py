@@ -138,6 +138,72 @@ def gemm_rows(x: torch.Tensor, w: torch.Tensor, nf: int, out_kind: int = ROWS_BF
                               stream_ptr(x)), "gemm_rows")
     return out
 
+# ------------------------------------------------- products of 17 to 64 rows (csrc/kernels/gemm_batch.hip)
+BATCH_ROWS = 16, 64     # more than, up to
+
+
+@functools.lru_cache(maxsize=4096)
+def batch_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = False):
+    """(16-row fragments of a workgroup, K ranges) with which that kernel takes a product of ``N`` result columns, or None; ``planes``: K
+    ranges may stay apart.
+
+    Two fragments while their strips are one wave of 256 workgroups, else four.  What it costs grows with the rows (every workgroup
+    reads them all), the other kernels' cost by steps at 32 rows.  Time over that of the stream kernel, of the row-streaming kernel
+    up to 32 rows, or of the library, by whichever had it, at 24, 32 | 40, 48, 56, 64 rows:
+    SwiGLU 8192 x 2048 0.96, 0.95 | 0.81, 0.81, 0.89, 0.92;  4096 x 2048 0.92, 0.88 | 0.82, 0.80, 0.91, 0.92;  6144 x 2048 (0.75 waves of
+    four fragments) 0.86, 0.93 | 0.91, 0.93, 0.99, 1.02;  16384 x 2048 0.98, 0.96 | 0.82, 0.84, 0.86, 0.92;  8192 x 4096 0.93, 0.96 |
+    0.77, 0.65, 0.82, 0.87;  3072 x 1024 0.78, 0.76 | 0.86, 0.91, 0.95, 0.98;  8192 x 1024 0.94, 0.93 | 1.07, 1.05, 1.15, 1.17;  1024 x
+    512 0.82, 0.87 | 1.06 - 1.14;  4096 x 8192 0.96, 0.97 | 0.92 - 0.97.  Squared relu 8192 x 2048 0.88, 0.86 | 0.81, 0.84, 0.90, 0.91, x
+    4096 0.84, 0.86 | 0.71 - 0.83;  16384 x 2048 0.89, 0.95 | 0.69 - 0.77;  4096 x 512 0.77, 0.82 | 1.03 - 1.09.  bf16 2560 x 2048 0.70,
+    0.75 | 0.79 - 0.92;  1024 x 2048 0.76, 0.80 | 0.91, 0.97, 1.04, 1.09;  4096 x 4096 0.82, 0.90 | 0.97, 1.02, 1.12, 1.06;  8192 x 1024
+    0.89, 0.87 | 0.87 - 0.97;  2048 x 1024 0.75, 0.78 | 0.95, 0.97, 1.04, 1.07.  fp32 2576 x 2048 0.92, 0.88 | 0.80 - 0.92;  8736 x
+    2048 0.83, 0.77 | 0.92, 0.95, 1.01, 1.03;  32768 x 2048 0.99, 0.99 | 0.95, 0.96, 1.03, 1.05;  50256 x 4096 0.94, 0.96 | 1.01 - 1.13.
+    Planes (without the pass behind, which has fewer of them to read) 2048 x 2048 0.99, 0.94 | 0.93, 0.97, 0.97, 1.00, x 8192 0.87, 0.92 |
+    0.99, 1.02, 1.08, 1.10;  4096 x 2048 0.90, 0.87 | 0.90 - 0.96;  1024 x 4096 0.73, 0.75 | 0.85 - 0.88;  2048 x 1024 0.98, 0.96 | 1.10 -
+    1.15."""
+    big = N * (2 if out == ROWS_SILU else 1)
+    if not BATCH_ROWS[0] < M <= BATCH_ROWS[1] or N % 16 or big < 512 or K % 256 or not 512 <= K <= 8192:
+        return None
+    few = M <= 32
+    if planes:
+        if N > 4096 or K < 1024 or not few and (K < 2048 or K > 2048 and M > 48 and N > 1024 or K > 2048 and N > 2048 or N < 1024):
+            return None
+        ranges = 8
+        while ranges > 1 and (-(-N // 32) * ranges > 256 or K % (256 * ranges)):
+            ranges //= 2
+        return (2, ranges) if ranges > 1 else None
+    if K > 4096 and out != ROWS_SILU:
+        return None
+    nf = 2 if big <= 8192 else 4
+    if out == ROWS_SILU and N % (8 * nf):
+        return None
+    if few:
+        return (nf, 1) if big <= 16384 or out >= ROWS_SILU or K > 2048 or M > 24 else None
+    if K < 2048:
+        return (nf, 1) if K >= 1024 and 6144 <= big <= 8192 else None
+    if out >= ROWS_SILU:
+        return (nf, 1) if M <= 48 or not 8192 < big < 15360 or out == ROWS_RELU2 else None
+    if K > 2048 or M > 48 and (big < 2048 or 8192 < big < 15360 or big > 16384):
+        return None
+    return nf, 1
+
+
+def _batch(x: torch.Tensor, w: torch.Tensor, out: int, planes: bool = False):
+    """That product (planes [ranges, M, N]), or None."""
+    M, K = x.shape
+    if not BATCH_ROWS[0] < M <= BATCH_ROWS[1] or K != w.shape[1] or not planes and (w.shape[0], K) in _dispatch:
+        return None
+    if not (_few_ok(x, w) and K <= x.stride(0) <= 1 << 24) or out == ROWS_SILU and w.shape[0] % 2:
+        return None
+    N = w.shape[0] // (2 if out == ROWS_SILU else 1)
+    plan = batch_plan(M, N, K, out, planes)
+    if plan is None:
+        return None
+    f32 = out == ROWS_F32
+    y = torch.empty((plan[1], M, N) if planes else (M, N), dtype=torch.float32 if f32 else x.dtype, device=x.device)
+    check(lib().k8s_gemm_batch(ptr(x), x.stride(0), ptr(w), ptr(y), N, M, N, K, plan[0], plan[1], out, stream_ptr(x)), "gemm_batch")
+    return y
+
 
 def select_gemm(M: int, N: int, K: int, x_ok_layout: bool = True, out_contig: bool = True,
                 rows: bool = True, out_wide: bool = True) -> Tuple[int, int, int]:
@@ -372,6 +438,9 @@ def linear_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             and w.is_contiguous():
         M, K = x.shape
         N = w.shape[0]
+        y = _batch(x, w, ROWS_F32)
+        if y is not None:
+            return y
         plan = _rows_choice(x, w, M, N, K, ROWS_F32)
         if plan is not None:
             return gemm_rows(x, w, plan[0], ROWS_F32)
@@ -430,6 +499,9 @@ def proj_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return linear(x, w)
     M, K = x.shape
     N = w.shape[0]
+    y = _batch(x, w, ROWS_F32)
+    if y is not None:
+        return y
     plan = _rows_choice(x, w, M, N, K, ROWS_F32)
     if plan is not None:
         return gemm_rows(x, w, plan[0], ROWS_F32)
@@ -462,7 +534,7 @@ def _narrow_cfg(M: int) -> int:
 
 def plane_plan(M: int, N: int, K: int):
     """(stream configuration, K ranges) of :func:`proj_planes`, (ROWS_CFG + fragments, K ranges) where the row-streaming kernel
-    takes it; one range: the product is not cut.  The other forms: 2048 columns are 32 or
+    takes it, (BATCH_CFG + fragments, K ranges) :func:`batch_plan`'s; one range: the product is not cut.  The other forms: 2048 columns are 32 or
     64 strips for 256 compute units, so K is cut until each has a workgroup: four ranges of 32-column strips where K is
     short, eight of 64-column strips from 4096 on.  us with cold weights at 1 / 16 / 64 / 128 rows: 2048 x 2048 hipBLASLt
     8.1 / 8.3 / 8.9 / 8.8, the skinny kernel 4.9 / 6.2 / 11.7 / --, 64-column planes 4.2 / 4.5 / 5.5 / 7.2, 32-column
@@ -475,6 +547,9 @@ def plane_plan(M: int, N: int, K: int):
     6.4, 7.7 / 6.8;  2048 x 1024 5.7 / 6.1, 6.8 / 6.4;  4096 x 1024 6.2 / 7.6, 7.3 / 7.9, x 3072 10.6 / 13.3, 12.0 / 12.5, x
     6144 16.0 / 15.3, 18.6 / 15.5, x 8192 18.8 / 22.7, 22.1 / 22.5;  5120 x 1024 7.2 / 8.5, 9.2 / 9.0, x 2048 10.5 / 10.9,
     13.3 / 11.7;  2048 x 256 at 24 rows 5.6 / 6.1."""
+    plan = batch_plan(M, N, K, ROWS_F32, True)
+    if plan is not None:
+        return BATCH_CFG + plan[0], plan[1]
     plan = rows_plan(M, N, K, ROWS_F32, True) if M <= ROWS_MAX_M else None
     if plan is not None:
         return ROWS_CFG + plan[0], plan[1]
@@ -482,6 +557,7 @@ def plane_plan(M: int, N: int, K: int):
 
 
 ROWS_CFG = 100      # past every stream configuration
+BATCH_CFG = 200     # past those
 
 
 @functools.lru_cache(maxsize=4096)      # (asked for every product of a step; 1.2 us of the host worked out, 0.2 looked up)
@@ -503,6 +579,11 @@ def proj_planes(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     N = w.shape[0]
     if _few_ok(x, w):
         cfg, S = plane_plan(M, N, K)
+        if cfg > BATCH_CFG:
+            y = _batch(x, w, ROWS_F32, True)
+            if y is not None:
+                return y
+            cfg, S = _plane_plan(M, N, K, _enabled)
         if cfg > ROWS_CFG and K == w.shape[1]:
             return gemm_rows(x, w, cfg - ROWS_CFG, ROWS_F32, S).view(S, M, N)
         if cfg > ROWS_CFG:
@@ -671,6 +752,9 @@ def proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     9.2 / 8.3, 10.6 / 8.3, 10.5 / 10.6.  At 273 strips the second wave costs it the lead (8736 x 2048, 64 rows:
     15.3 / 17.2);  a long K over few strips does where the library cuts it (1024 x 2048 at 24 / 128 rows 8.1 / 9.0, 8.4 /
     10.3, 2048 x 2048 11.1 / 9.2, 11.4 / 13.0)."""
+    y = _batch(x, w, ROWS_BF16)
+    if y is not None:
+        return y
     M, K = x.shape
     N = w.shape[0]
     if (16 < M <= NARROW_MAX_M and 32 <= N <= 32 * NARROW_WGS and K <= 2048 and (N, K) not in _dispatch and _few_ok(x, w)
@@ -719,6 +803,9 @@ def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     (:func:`big_fused`); the fused forms square the fp32 sum.  Not for few rows of up to 4096 columns: the strips are half the
     card, and the skinny kernel and its pass are quicker (2048 x 2048 at 1, 8, 16 rows 6.6 / 9.2, 7.4 / 9.2, 8.0 / 9.2, x 1024
     5.0 / 5.7, 5.7 / 5.9, 6.0 / 5.9, x 512 4.4 / 4.4, 4.9 / 4.7, 5.2 / 4.6)."""
+    y = _batch(x, w, ROWS_RELU2)
+    if y is not None:
+        return y
     M, K = x.shape
     N = w.shape[0]
     if _few_ok(x, w):
@@ -745,6 +832,9 @@ def glu_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     (6144 x 2048 14.2 / 12.9, 18.5 / 13.4, 19.4 / 14.5, 22.7 / 18.4), from 8192 on the register ring up to 32 rows (8192 x
     2048 17.1 / 16.3, 22.5 / 16.3, then 21.3 / 17.3, 24.6 / 21.7).  Prompts: :func:`big_fused`."""
     a = swiglu_gemm(x, w)
+    if a is not None:
+        return a
+    a = _batch(x, w, ROWS_SILU)
     if a is not None:
         return a
     M, K = x.shape
