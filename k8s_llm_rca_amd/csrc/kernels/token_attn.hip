@@ -177,6 +177,120 @@ __global__ void __launch_bounds__(256) token_merge_kernel(TokOut a, const int* _
   tok_store4(a, row, head, 4 * c, acc);
 }
 
+// The same and, in the same launch, the merged heads out of latent space (head_proj_kernel, small_proj.hip, K -> N by w [H][K][N]):
+// out[row][h][n] = sum_k bf16(merged[h][k]) w[h][k][n], every bit that of the two launches.  Of a handful of rows both are a launch
+// and one trip to memory; here the parts, their maxima and the weights are on their way together.  A workgroup has 64 columns of
+// one head and TR rows, which it merges itself: a thread four entries of a row, all parts of them at once.  K = TR's threads x 4.
+// us with the attention in front, both launches / this, 16 heads 256 -> 128, at 2, 5, 9, 16 parts:  1 row 13.5 / 10.8, 13.6 / 10.9,
+// 13.5 / 10.8, 14.0 / 11.5;  7 rows 16.1 / 12.1, 16.2 / 12.6, 16.3 / 12.9, 17.0 / 14.1;  16 rows 16.1 / 12.3, 16.4 / 13.3, 17.6 / 14.2,
+// 19.5 / 16.7;  64 rows 18.6 / 14.7, 26.0 / 22.9, 32.3 / 29.7, 40.8 / 38.8.
+template <int TR, int NP, int K>
+__global__ void __launch_bounds__(256) token_merge_proj_kernel(TokOut a, const int* __restrict__ items, int n_items,
+                                                               const uint16_t* __restrict__ w, int N) {
+  constexpr int W = K / 4, S = 256 / W, KG = K / 8;        // S: groups of parts, as in token_merge_kernel
+  static_assert(TR * W <= 256 && TR <= 4 && NP <= 64);
+  __shared__ float xs[K > 512 ? K * TR : 512 * TR], fac[TR][NP], fin[TR];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, n0 = blockIdx.x * 64, h = blockIdx.y, t0 = blockIdx.z * TR;
+  const int nt = min(TR, n_items - t0), np = a.n_parts, c = 2 * (tid & 31), kg = tid >> 5;
+  const int t = tid / W, c4 = tid % W;
+  const size_t p0 = ((size_t)(t0 + min(t, nt - 1)) * a.H + h) * np;
+  const f32x4* po = reinterpret_cast<const f32x4*>(a.po + p0 * K) + c4;
+  f32x4 v[NP];
+  if (t < nt) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) v[p] = po[(size_t)(p < np ? p : 0) * W];
+  }
+  float m = -INFINITY, l = 0.f;
+  if (wv < nt && lane < np) {
+    const float* ml = a.pml + (((size_t)(t0 + wv) * a.H + h) * np + lane) * 2;
+    m = ml[0], l = ml[1];
+  }
+  const uint16_t* wp = w + ((size_t)h * K + (size_t)kg * KG) * N + n0 + c;
+  uint32_t wq[KG];
+#pragma unroll
+  for (int u = 0; u < KG; ++u) wq[u] = *reinterpret_cast<const uint32_t*>(wp + (size_t)u * N);
+  if (wv < nt) {                                           // wave -> row: the parts' factors
+    const float M = wave_max(m), f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+    const float L = wave_sum(fmaf(l, f, 0.f));
+    if (lane < NP) fac[wv][lane] = m == -INFINITY ? -1.f : f;        // -1: no visible key, its output was not written
+    if (lane == 0) {
+      float wf;
+      const float g = tok_finish(a, items[(t0 + wv) * 4 + 1], h, M, L, wf);
+      fin[wv] = wf * g;
+    }
+  }
+  __syncthreads();
+  if (t < TR) {
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (t < nt) {
+#pragma unroll
+      for (int g = 0; g < S; ++g) {
+        f32x4 one = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = g; p < NP; p += S) {
+          const float f = fac[t][p];
+          if (p < np && f != -1.f) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) one[k] = fmaf(v[p][k], f, one[k]);
+          }
+        }
+        if (g == 0)
+          acc = one;
+        else
+          acc += one;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] = bf2f(f2bf(acc[k] * fin[t]));
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) xs[(4 * c4 + k) * TR + t] = acc[k];
+  }
+  __syncthreads();
+  float acc[TR][2] = {};
+#pragma unroll
+  for (int u = 0; u < KG; ++u) {
+    const float w0 = bf2f((uint16_t)wq[u]), w1 = bf2f((uint16_t)(wq[u] >> 16));
+    const float* x = xs + (kg * KG + u) * TR;
+#pragma unroll
+    for (int i = 0; i < TR; ++i) {
+      acc[i][0] = fmaf(x[i], w0, acc[i][0]);
+      acc[i][1] = fmaf(x[i], w1, acc[i][1]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < TR; ++i) {
+    xs[(kg * TR + i) * 64 + c] = acc[i][0];
+    xs[(kg * TR + i) * 64 + c + 1] = acc[i][1];
+  }
+  __syncthreads();
+  for (int e = tid; e < nt * 64; e += 256) {
+    float r = 0.f;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) r += xs[g * TR * 64 + e];
+    a.out[(size_t)items[(t0 + e / 64) * 4 + 1] * a.ost + (size_t)h * a.osh + n0 + e % 64] = f2bf(r);
+  }
+}
+
+template <int K>
+static int launch_merge_proj(const TokOut& a, const int* items, int rows, const uint16_t* w, int N, hipStream_t s) {
+#define K8S_MP(TR, NP)                                                                                                        \
+  {                                                                                                                           \
+    hipLaunchKernelGGL((token_merge_proj_kernel<TR, NP, K>), dim3(N / 64, a.H, (rows + TR - 1) / TR), dim3(256), 0, s, a, items, rows, \
+                       w, N);                                                                                                 \
+    return (int)hipGetLastError();                                                                                            \
+  }
+  if (rows == 1) {
+    if (a.n_parts <= 4) K8S_MP(1, 4)
+    if (a.n_parts <= 9) K8S_MP(1, 9)
+    K8S_MP(1, 16)
+  }
+  if (a.n_parts <= 4) K8S_MP(4, 4)
+  if (a.n_parts <= 9) K8S_MP(4, 9)
+  K8S_MP(4, 16)
+#undef K8S_MP
+}
+
 __device__ __forceinline__ bf16x8 tld16(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
 // TURN: keys and values are loaded with lane 4 r + h at piece h of row r, so that four lanes beside each other read 64 bytes of
@@ -756,7 +870,7 @@ static int launch_lat_tok(const LatTokArgs& a, int np, int rows, hipStream_t s) 
     case 2: launch_lat_tok_np<NR, 2>(a, rows, s); break;
     default: return (int)hipErrorInvalidValue;
   }
-  if (a.t.n_parts > 1)
+  if (a.t.n_parts > 1 && a.t.out)
     hipLaunchKernelGGL(token_merge_kernel, dim3(rows * a.t.H), dim3(256), 0, s, a.t, a.items, NR * 32);
   return (int)hipGetLastError();
 }
@@ -842,14 +956,15 @@ K8S_API int k8s_masked_attn_memory(K8S_PREP_PARAMS, const float* mx, int mxs, co
   return (int)hipErrorInvalidValue;
 }
 
-// items [rows][4]; n_parts > 1: po [rows][H][n_parts][R], pml [rows][H][n_parts][2]
+// items [rows][4]; n_parts > 1: po [rows][H][n_parts][R], pml [rows][H][n_parts][2], and without out they are left to
+// k8s_latent_merge_proj
 K8S_API int k8s_latent_attn_token(const void* qa, long qst, long qsh, const void* qr, int RP, const void* c, const void* ct,
                                   const int* bt, int maxb, const int* items, int rows, const float* gate, int ldg,
                                   const float* sink, void* out, long ost, long osh, float* po, float* pml, int n_parts,
                                   int part, int most, int H, int R, int BS, int window, float scale, hipStream_t s) {
   if (rows <= 0) return 0;
   if (!k8s_latent_attn_mfma_ok(R, RP) || BS % 32 || H <= 0 || n_parts < 1 || n_parts > most || part <= 0 || part % 32 ||
-      (RP && !qr) || window < 0 || qst % 8 || qsh % 8 || (n_parts > 1 && (!pml || !po)))
+      (RP && !qr) || window < 0 || qst % 8 || qsh % 8 || (n_parts > 1 && (!pml || !po)) || (n_parts == 1 && !out))
     return (int)hipErrorInvalidValue;
   LatTokArgs a;
   a.qa = (const uint16_t*)qa; a.qst = qst; a.qsh = qsh; a.qr = (const uint16_t*)qr; a.c = (const uint16_t*)c;
@@ -869,4 +984,20 @@ K8S_API int k8s_latent_attn_token(const void* qa, long qst, long qsh, const void
     case 16: return launch_lat_tok<16>(a, RP / 32, rows, s);
     default: return (int)hipErrorInvalidValue;
   }
+}
+
+// out[row][h] = merged[row][h] . w[h] of the parts that k8s_latent_attn_token left (2 to 16 of them): w [H][R][N], R 128 or 256, N a
+// multiple of 64; po on 16 bytes, w on 4.
+K8S_API int k8s_latent_merge_proj(const float* po, const float* pml, int n_parts, const int* items, int rows, const float* gate, int ldg,
+                                  const float* sink, const void* w, void* out, long ost, long osh, int H, int R, int N,
+                                  hipStream_t s) {
+  if (rows <= 0) return 0;
+  if (!po || !pml || !items || !w || !out || n_parts < 2 || n_parts > 16 || H < 1 || (R != 128 && R != 256) || N < 64 || N % 64 ||
+      ((uintptr_t)po & 15) || ((uintptr_t)w & 3))
+    return (int)hipErrorInvalidValue;
+  TokOut t{};
+  t.sink = sink; t.gate = gate; t.gs = ldg; t.out = (uint16_t*)out; t.ost = ost; t.osh = osh;
+  t.po = const_cast<float*>(po); t.pml = const_cast<float*>(pml); t.H = H; t.n_parts = n_parts; t.hs = 1;
+  return R == 128 ? launch_merge_proj<128>(t, items, rows, (const uint16_t*)w, N, s)
+                  : launch_merge_proj<256>(t, items, rows, (const uint16_t*)w, N, s);
 }

@@ -393,13 +393,12 @@ class FikeraxModel:
         qa, qr = S.latent_queries(q, L["uk"], cs, H, D, c.tail)               # [T, H, KR] head-major, [T, H, tail]
         kw = dict(window=c.window, sink=L["sink"], head_major=True)
         if cache_t is not None:
-            o = S.latent_attention_mfma(qa, cache, cache_t, None, inp.seg, inp.positions, c.scale, qr=qr, **kw)
+            ov = S.latent_attention_mfma(qa, cache, cache_t, None, inp.seg, inp.positions, c.scale, qr=qr, up=L["uv_t"], **kw)
         else:
             o = S.latent_attention(qa.float(), cache, None, inp.seg, c.scale, self.dtype,
                                    qr=qr.float() if qr is not None else None, **kw)
-        ov = torch.empty(T, H, V, dtype=self.dtype, device=o.device)
-        S.head_proj(o, L["uv_t"], ov)                                         # written token-major: W_o reads it as it is
-        return ov.view(T, H * V)
+            ov = S.head_proj(o, L["uv_t"], torch.empty(T, H, V, dtype=self.dtype, device=o.device))
+        return ov.view(T, H * V)                                              # token-major: W_o reads it as it is
 
     def forward(self, inp: S.SegStepInputs, kcs: List[torch.Tensor], vcs: List[Optional[torch.Tensor]],
                 vts: List[Optional[torch.Tensor]], states: Optional[Dict[str, torch.Tensor]] = None,

@@ -121,6 +121,7 @@ _SIGS = {
     "k8s_rotated_tail": [P, P, P, I, I, I, I, I, I, P],
     "k8s_latent_attn_mfma_ok": [I, I],
     "k8s_latent_attn_mfma": [P, P, P, P, I, P, I, P, I, P, I, I, I, F, P, L, L, P, I, L, L, I, P],
+    "k8s_latent_merge_proj": [P, P, I, P, I, P, I, P, P, P, L, L, I, I, I, P],
     "k8s_latent_attn_token": [P, L, L, P, I, P, P, P, I, P, I, P, I, P, P, L, L, P, P, I, I, I, I, I, I, I, F, P],
     "k8s_delta_step": [P, I, P, P, P, P, I, P, P, P, P, I, P, I, P, I, I, I, I, I, F, F, P],
     "k8s_delta_step_low": [P, P, I, I, I, P, P, P, P, P, P, P, P, I, P, I, I, I, I, I, F, F, P],

@@ -584,11 +584,20 @@ def _token_groups(rows: torch.Tensor, heads: int, parts: int, V: int) -> tuple:
     return ([rows] if per == rows.shape[0] else rows.split(per), *(scratch(per * heads * parts * n, torch.float32, rows.device) for n in (V, 2)))
 
 
+def _merge_up(qa: torch.Tensor, up: torch.Tensor, n_parts: int) -> bool:
+    """Whether the parts of single tokens are merged by the product behind them (csrc/kernels/token_attn.hip,
+    token_merge_proj_kernel): where that product is the vector pipes' and a thread can hold all of its entries' parts (2 to 4 us less
+    at 1 to 64 rows and 2 to 16 parts, with both timed there)."""
+    T, H, R = qa.shape
+    return 2 <= n_parts <= 16 and R in (128, 256) and up.shape[2] % 64 == 0 and _small_heads(qa, up, H, R)
+
+
 def latent_attention_mfma(qa: torch.Tensor, cache: torch.Tensor, cache_t: torch.Tensor, gate: Optional[torch.Tensor],
                           seg: SegMeta, positions: torch.Tensor, scale: float, qr: Optional[torch.Tensor] = None,
-                          window: int = 0, sink: Optional[torch.Tensor] = None, head_major: bool = False) -> torch.Tensor:
+                          window: int = 0, sink: Optional[torch.Tensor] = None, head_major: bool = False,
+                          up: Optional[torch.Tensor] = None) -> torch.Tensor:
     """:func:`latent_attention` on the matrix cores: bf16 absorbed queries ``qa`` [T, H, R], the latent
-    pages and their transposed twins.  Decode rows (the step's first ``seg.n_single``) are split over
+    pages and their transposed twins.  ``up`` [H, R, N]: the result is :func:`head_proj`'s of it, [T, H, N].  Decode rows (the step's first ``seg.n_single``) are split over
     partitions of keys and merged; prompt portions run one wave per group of tokens."""
     T, H, R = qa.shape
     BS, W = cache.shape[1], cache.shape[2]
@@ -599,29 +608,35 @@ def latent_attention_mfma(qa: torch.Tensor, cache: torch.Tensor, cache_t: torch.
     assert (qr is None) == (W == R) and (qr is None or (qr.dtype == qa.dtype and qr.is_contiguous()
                                                         and qr.shape == (T, H, W - R)))
     assert sink is None or (sink.dtype == torch.float32 and sink.numel() == H)
-    out = _latent_out(qa, torch.bfloat16, head_major)
     tpi = tiles * (16 // min(H, 16))
     dec, pre, kmax = seg.attn_items(tpi)
     L, st = lib(), stream_ptr(qa)
     bt, maxb = seg.block_tables, seg.block_tables.shape[1]
     gs = gate.stride(0) if gate is not None else 0
+    part, n_parts, groups, po, pml = LATENT_PART, 1, [], None, None
     if dec.shape[0]:
-        part = LATENT_PART
         n_parts = -(-kmax // part)
         if window > 0:      # a row's parts start at the one its first visible key lies in
             n_parts = min(n_parts, (min(int(window), kmax) + part - 2) // part + 1)
         n_parts = min(n_parts, TOKEN_PARTS)
         groups, po, pml = _token_groups(dec, H, n_parts, R)
-        for it in groups:
-            check(L.k8s_latent_attn_token(ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), W - R, ptr(cache), ptr(cache_t),
-                                          ptr(bt), maxb, ptr(it), it.shape[0], ptr(gate), gs, ptr(sink), ptr(out),
-                                          out.stride(0), out.stride(1), ptr(po), ptr(pml), n_parts, part, TOKEN_PARTS, H,
-                                          R, BS, int(window), float(scale), st), "latent_attn_token")
+    fused = up is not None and dec.shape[0] == T and len(groups) == 1 and _merge_up(qa, up, n_parts)
+    out = None if fused else _latent_out(qa, torch.bfloat16, head_major)
+    for it in groups:
+        check(L.k8s_latent_attn_token(ptr(qa), qa.stride(0), qa.stride(1), ptr(qr), W - R, ptr(cache), ptr(cache_t),
+                                      ptr(bt), maxb, ptr(it), it.shape[0], ptr(gate), gs, ptr(sink), ptr(out),
+                                      *((0, 0) if fused else out.stride()[:2]), ptr(po), ptr(pml), n_parts, part, TOKEN_PARTS, H,
+                                      R, BS, int(window), float(scale), st), "latent_attn_token")
+    if fused:
+        out = torch.empty(T, H, up.shape[2], dtype=torch.bfloat16, device=qa.device)
+        check(L.k8s_latent_merge_proj(ptr(po), ptr(pml), n_parts, ptr(dec), T, ptr(gate), gs, ptr(sink), ptr(up), ptr(out),
+                                      out.stride(0), out.stride(1), H, R, up.shape[2], st), "latent_merge_proj")
+        return out
     if pre.shape[0]:
         check(L.k8s_latent_attn_mfma(ptr(qa), ptr(cache), ptr(cache_t), ptr(bt), maxb, ptr(pre), pre.shape[0], ptr(gate),
                                      gs, ptr(out), H, R, BS, float(scale), st, qa.stride(0), qa.stride(1), ptr(qr), W - R,
                                      out.stride(0), out.stride(1), int(window), ptr(sink)), "latent_attn_mfma")
-    return out
+    return out if up is None else head_proj(out, up, torch.empty(T, H, up.shape[2], dtype=out.dtype, device=out.device))
 
 
 def latent_attention(qa: torch.Tensor, cache: torch.Tensor, gate: Optional[torch.Tensor], seg: SegMeta, scale: float,
