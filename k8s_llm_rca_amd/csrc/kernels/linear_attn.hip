@@ -21,6 +21,7 @@
 // to cs [items][H][D][V];  decay_carry_kernel turns cs into every range's START state and advances the slot;
 // MODE 2: the range from its start state, writing o [T][H V] (fp32).
 #include "common.h"
+#include "state_carry.h"
 
 namespace k8s {
 
@@ -331,26 +332,20 @@ __global__ void __launch_bounds__(64 * NW, TWO ? 4 : 2) decay_attn_mfma_kernel(L
   }
 }
 
-// Between the two passes, one thread per state entry of a (segment, head): walk the segment's ranges, replace every
-// range's end-from-zero state by its START state, leave the final state in the slot.
+// Between the two passes (state_carry.h)
+template <int VEC>
 __global__ void __launch_bounds__(256) decay_carry_kernel(const float* __restrict__ decay, float* __restrict__ state,
                                                           const int* __restrict__ seg_pos0,
                                                           const int* __restrict__ seg_slot,
                                                           const int* __restrict__ seg_item0,
                                                           const int* __restrict__ items, float* __restrict__ cs, int H,
                                                           int DV) {
-  const int sg = blockIdx.x, hh = blockIdx.y, e = blockIdx.z * 256 + threadIdx.x;
+  const int sg = blockIdx.x, hh = blockIdx.y, e = VEC * (blockIdx.z * 256 + threadIdx.x);
   if (e >= DV) return;
-  float* st = state + ((size_t)seg_slot[sg] * H + hh) * DV + e;
-  float S = seg_pos0[sg] == 0 ? 0.f : *st;
+  const int k0 = seg_item0[sg];
   const float dec = decay[hh];
-  for (int k = seg_item0[sg]; k < seg_item0[sg + 1]; ++k) {
-    float* ck = cs + ((size_t)k * H + hh) * DV + e;
-    const float loc = *ck;
-    *ck = S;
-    S = fmaf(ipow(dec, items[k * 4 + 2]), S, loc);
-  }
-  *st = S;
+  carry_states<VEC>(state + ((size_t)seg_slot[sg] * H + hh) * DV + e, seg_pos0[sg] == 0, cs + ((size_t)k0 * H + hh) * DV + e,
+                    (size_t)H * DV, seg_item0[sg + 1] - k0, [&](int k) { return ipow(dec, items[(k0 + k) * 4 + 2]); });
 }
 
 template <int D, int NW, int MODE, bool SILU>
@@ -370,7 +365,9 @@ static int launch_la_all(const LinArgs& a, int n_seg, int n_items, const int* se
   if (n_items <= 0) return launch_la<D, NW, 0, SILU>(a, n_seg, s);
   int rc = launch_la<D, NW, 1, SILU>(a, n_items, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(decay_carry_kernel, dim3(n_seg, a.H, (D * a.V + 255) / 256), dim3(256), 0, s, a.decay, a.state,
+  const bool four = carry_by_four(a.state, a.cs, D * a.V);
+  hipLaunchKernelGGL((four ? decay_carry_kernel<4> : decay_carry_kernel<1>),
+                     dim3(n_seg, a.H, (D * a.V + (four ? 1023 : 255)) / (four ? 1024 : 256)), dim3(256), 0, s, a.decay, a.state,
                      a.seg_pos0, a.seg_slot, seg_item0, a.items, a.cs, a.H, D * a.V);
   rc = (int)hipGetLastError();
   return rc ? rc : launch_la<D, NW, 2, SILU>(a, n_items, s);

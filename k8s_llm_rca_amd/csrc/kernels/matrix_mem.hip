@@ -15,7 +15,7 @@
 //
 // The matrix memory's normaliser n is the state of one more column whose value is 1 for every token; its
 // read-out is n.q.  The gates and the running maximum are a scalar recurrence per head: a kernel of their
-// own runs it as a parallel scan over 64 tokens per wave (m_t = F_t + max(m_0, max_{s<=t}(i_s - F_s)) with F
+// own runs it as a parallel scan over 64 tokens per wave, eight waves at a time (m_t = F_t + max(m_0, max_{s<=t}(i_s - F_s)) with F
 // the running sum of f) and leaves per token the two factors and m.  m only keeps the exponentials in
 // range -- the state is e^(-m) times the unstabilised one for ANY sequence m as long as both factors of a
 // token use the same values -- so the scan's different rounding of m does not show in the output.
@@ -52,33 +52,46 @@ constexpr int kMemTb = 16;     // tokens per batch
 constexpr int kMemVb = 64;     // state columns per workgroup
 
 // Rows of x (fp32, stride xs): q [H][D] | k [H][D] | v [H][V] | gate [H][V] | i [H] | f [H].
-// ab [T][H][3] receives (forget factor, input factor, m) of every token; one wave per (segment, head),
-// 64 tokens at a time, one per lane.
-__global__ void __launch_bounds__(256) memory_gates_kernel(const float* __restrict__ x, int xs,
-                                                           const float* __restrict__ gate_bias, float cap,
-                                                           float* __restrict__ mstate,
-                                                           const int* __restrict__ seg_row0,
-                                                           const int* __restrict__ seg_pos0,
-                                                           const int* __restrict__ seg_slot, float* __restrict__ ab,
-                                                           int n_seg, int H, int D, int V) {
-  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (unit >= n_seg * H) return;
-  const int sg = unit / H, hh = unit - sg * H;
+// ab [T][H][3] receives (forget factor, input factor, m) of every token; one workgroup per (segment, head), 64 tokens a wave, one
+// per lane, eight waves a round: a round's sums and maxima wait for nothing, then every wave follows m_0 through the waves in front
+// of it.  The next round's rows (two numbers of a line each) are on their way meanwhile.  Bound by instructions (two tanh, a logarithm,
+// three exponentials and the exchanges a token) and by the trips to memory.  us with one wave for all batches, one after the other /
+// four of them at once / so, 16 heads:  5 sequences of 560 to 1100 tokens 29 / 19 / 9.4, 8 of 2048 58 / 35 / 15.6, 64 of 256 to 512 21.5 /
+// 15.9 / 15.1.
+constexpr int kGateWaves = 8;
+__global__ void __launch_bounds__(64 * kGateWaves) memory_gates_kernel(const float* __restrict__ x, int xs,
+                                                                       const float* __restrict__ gate_bias, float cap,
+                                                                       float* __restrict__ mstate,
+                                                                       const int* __restrict__ seg_row0,
+                                                                       const int* __restrict__ seg_pos0,
+                                                                       const int* __restrict__ seg_slot, float* __restrict__ ab,
+                                                                       int H, int D, int V) {
+  constexpr int NW = kGateWaves;
+  __shared__ float ends[2][NW][2];                 // of a wave's last token: the sum and the maximum
+  const int sg = blockIdx.x / H, hh = blockIdx.x - sg * H, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int r0 = seg_row0[sg], r1 = seg_row0[sg + 1];
   const size_t so = (size_t)seg_slot[sg] * H + hh;
   float m0 = seg_pos0[sg] == 0 ? 0.f : mstate[so];
-  const int go = 2 * H * D + 2 * H * V;
+  const float* xi = x + 2 * H * D + 2 * H * V + hh;
   const float bi = gate_bias[hh], bf = gate_bias[H + hh];
-  for (int t0 = r0; t0 < r1; t0 += 64) {
-    const int r = t0 + lane;
+  float ri = 0.f, rf = 0.f;
+  auto ask = [&](int r) {
+    if (r < r1) {
+      const float* row = xi + (size_t)r * xs;
+      ri = row[0], rf = row[H];
+    }
+  };
+  ask(r0 + (int)threadIdx.x);
+  for (int t0 = r0, p = 0; t0 < r1; t0 += 64 * NW, p ^= 1) {
+    const int tb = t0 + 64 * wv, r = tb + lane;
     const bool on = r < r1;
     float gi = -INFINITY, gf = 0.f;
     if (on) {
-      const float* row = x + (size_t)r * xs;
-      gi = cap * tanhf((row[go + hh] + bi) / cap);
-      gf = logsigmoid_f(cap * tanhf((row[go + H + hh] + bf) / cap));
+      gi = cap * tanhf((ri + bi) / cap);
+      gf = logsigmoid_f(cap * tanhf((rf + bf) / cap));
     }
-    float F = gf;                                  // running sum of f over the batch
+    ask(r + 64 * NW);
+    float F = gf;                                  // running sum of f over the wave
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const float up = __shfl_up(F, o, 64);
@@ -90,18 +103,26 @@ __global__ void __launch_bounds__(256) memory_gates_kernel(const float* __restri
       const float up = __shfl_up(pa, o, 64);
       if (lane >= o) pa = fmaxf(pa, up);
     }
-    const float m = F + fmaxf(m0, pa);
+    if (lane == min(63, r1 - tb - 1)) ends[p][wv][0] = F, ends[p][wv][1] = pa;
+    __syncthreads();
+    float mine = m0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      if (w == wv) mine = m0;
+      if (t0 + 64 * w < r1) m0 = ends[p][w][0] + fmaxf(m0, ends[p][w][1]);
+    }
+    const float m = F + fmaxf(mine, pa);
     const float mup = __shfl_up(m, 1, 64);
-    const float mprev = lane == 0 ? m0 : mup;
+    const float mprev = lane == 0 ? mine : mup;
     if (on) {
       float* o = ab + ((size_t)r * H + hh) * 3;
       o[0] = expf(gf + mprev - m);
       o[1] = expf(gi - m);
       o[2] = m;
     }
-    m0 = __shfl(m, min(63, r1 - t0 - 1), 64);
   }
-  if (lane == 0) mstate[so] = m0;
+  __syncthreads();                                 // every wave has read mstate
+  if (threadIdx.x == 0) mstate[so] = m0;
 }
 
 // mul[r][h] = D^(-1/2) / (max(|nq|, e^(-m)) + den_eps): what the raw read-out S^T q (q unscaled) is multiplied by
@@ -643,8 +664,8 @@ K8S_API int k8s_matrix_memory(const float* x, int xs, const float* gate_bias, fl
                               float* cs, float* cx, float* cdec, float* tile_ws) {
   if (n_seg <= 0 || T <= 0) return 0;
   if (D < 1 || D > 256 || cap <= 0.f) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(memory_gates_kernel, dim3((n_seg * H + 3) / 4), dim3(256), 0, s, x, xs, gate_bias, cap, mstate,
-                     seg_row0, seg_pos0, seg_slot, ab, n_seg, H, D, V);
+  hipLaunchKernelGGL(memory_gates_kernel, dim3(n_seg * H), dim3(64 * kGateWaves), 0, s, x, xs, gate_bias, cap, mstate,
+                     seg_row0, seg_pos0, seg_slot, ab, H, D, V);
   MatArgs p{};
   p.x = x;
   p.xs = xs;

@@ -9,6 +9,7 @@
 // seg_pos0 > 0.  All recurrences, their decays, step sizes and gates are fp32;
 // TA is the activation type (bf16 as uint16_t, or float).
 #include "common.h"
+#include "state_carry.h"
 #include "gates.h"
 
 namespace k8s {
@@ -557,27 +558,28 @@ __global__ void __launch_bounds__(256) retention_scan_kernel(const TA* __restric
 
 // Between the two chunk passes, one thread per state entry of a (segment, head): walk the segment's
 // chunks, replace every chunk's end-from-zero state by its START state, leave the final state in the slot.
+template <int VEC>
 __global__ void __launch_bounds__(256) retention_carry_kernel(const float* __restrict__ decay, float* __restrict__ state,
                                                               const int* __restrict__ seg_pos0,
                                                               const int* __restrict__ seg_slot,
                                                               const int* __restrict__ seg_chunk0,
                                                               const int* __restrict__ chunks, float* __restrict__ cs,
                                                               int H, int DV) {
-  const int sg = blockIdx.x, hh = blockIdx.y, e = blockIdx.z * 256 + threadIdx.x;
+  const int sg = blockIdx.x, hh = blockIdx.y, e = VEC * (blockIdx.z * 256 + threadIdx.x);
   if (e >= DV) return;
-  float* st = state + ((size_t)seg_slot[sg] * H + hh) * DV + e;
-  float S = seg_pos0[sg] == 0 ? 0.f : *st;
+  const int k0 = seg_chunk0[sg];
   const float dec = decay[hh];
-  for (int k = seg_chunk0[sg]; k < seg_chunk0[sg + 1]; ++k) {
-    float* ck = cs + ((size_t)k * H + hh) * DV + e;
-    const int n = chunks[k * 4 + 2];
-    float p = 1.f;
-    for (int i = 0; i < n; ++i) p *= dec;
-    const float loc = *ck;
-    *ck = S;
-    S = fmaf(p, S, loc);
-  }
-  *st = S;
+  int last = 0;
+  float p = 1.f;                       // dec ^ last (the chunks but a portion's last are alike)
+  carry_states<VEC>(state + ((size_t)seg_slot[sg] * H + hh) * DV + e, seg_pos0[sg] == 0, cs + ((size_t)k0 * H + hh) * DV + e,
+                    (size_t)H * DV, seg_chunk0[sg + 1] - k0, [&](int k) {
+                      const int n = chunks[(k0 + k) * 4 + 2];
+                      if (n != last) {
+                        p = 1.f, last = n;
+                        for (int i = 0; i < n; ++i) p *= dec;
+                      }
+                      return p;
+                    });
 }
 
 // out[r][h] = o / sqrt(mean(o^2 over V) + eps) * silu(g): one wave per (row, head).
@@ -749,7 +751,9 @@ static int launch_decay_scan(const TA* x, int xs, const float* decay, float* sta
     K8S_RET_M(DP, 0, n_seg)                                                                                     \
   } else {                                                                                                      \
     K8S_RET_M(DP, 1, n_chunks)                                                                                  \
-    hipLaunchKernelGGL(retention_carry_kernel, dim3(n_seg, H, (D * V + 255) / 256), dim3(256), 0, s, decay, state, \
+    const bool four = carry_by_four(state, cs, D * V);                                                          \
+    hipLaunchKernelGGL((four ? retention_carry_kernel<4> : retention_carry_kernel<1>),                          \
+                       dim3(n_seg, H, (D * V + (four ? 1023 : 255)) / (four ? 1024 : 256)), dim3(256), 0, s, decay, state, \
                        seg_pos0, seg_slot, seg_chunk0, chunks, cs, H, D * V);                                   \
     K8S_RET_M(DP, 2, n_chunks)                                                                                  \
   }
