@@ -378,8 +378,11 @@ class FikeraxModel:
 
     def _attention(self, i: int, h, inp: S.SegStepInputs, tables, kc, vc, vt) -> torch.Tensor:
         L, c = self.layers[i], self.cfg.layers[i].mix
-        x = R.proj_planes(h, L["w_in"])
         prep = dict(norm="head", eps=self.cfg.norm_eps, rope=self.ropes[i], rope_cs=tables.of(self.ropes[i]))
+        made = S.proj_prep(h, L["w_in"], L["b_in"], c.heads, c.kv_heads, c.dim, c.vdim, inp.slots, kc, vc, vt, inp.seg, **prep)
+        if made is not None:
+            return S.masked_attention(made[0], c.heads, c.kv_heads, c.dim, c.vdim, kc, vc, inp.seg, c.scale, vt=vt, window=c.window)
+        x = R.proj_planes(h, L["w_in"])
         return S.prep_attention(x, L["b_in"], c.heads, c.kv_heads, c.dim, c.vdim, inp.positions, inp.slots, kc, vc, vt, inp.seg,
                                 self.dtype, c.scale, prep, dict(window=c.window))
 

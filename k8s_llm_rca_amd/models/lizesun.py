@@ -380,15 +380,19 @@ class LizesunModel:
         L, a = self.layers[li], self.cfg.layers[li].attn
         ci = self.cache_of[li]
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
-        x = R.proj_f32out(h, L["w_in"])                                # [T, H D + G D + G V + H] fp32
         keep = other = None
         if a.v_mix:
             if li == self.vmix_first:
-                keep = vmix["v"] = torch.empty(x.shape[0], G * V, dtype=torch.float32, device=x.device)
+                keep = vmix["v"] = torch.empty(inp.slots.shape[0], G * V, dtype=torch.float32, device=self.device)
             else:
                 other = vmix["v"]
         n = H * D + G * (D + V)
         prep = dict(norm=True, q_w=L["q_w"], k_w=L["k_w"], eps=self.cfg.norm_eps, lam=L["lam"], v_other=other, v_keep=keep)
+        made = S.proj_prep(h, L["w_in"], L["bias"], H, G, D, V, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg, **prep)
+        if made is not None:
+            return S.masked_attention(made[0], H, G, D, V, kcs[ci], vcs[ci], inp.seg, a.scale, vt=vts[ci], softcap=a.softcap,
+                                      chunk=a.chunk, gate=made[1])
+        x = R.proj_f32out(h, L["w_in"])                                # [T, H D + G D + G V + H] fp32
         return S.prep_attention(x[:, :n], L["bias"], H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg,
                                 self.dtype, a.scale, prep, dict(softcap=a.softcap, chunk=a.chunk, gate=x[:, n:]))
 
@@ -398,10 +402,15 @@ class LizesunModel:
         ci, j = self.cache_of[li], self.mem_of[li]
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
         nl = H * D + G * (D + V)
-        x = R.proj_f32out(h, L["w_in"])                                # left q | k | v, right q | k | v | g | i | f
         rope = self.ropes.get((a.rot_dims, a.rot_base))
         prep = dict(norm=True, eps=self.cfg.norm_eps, rope=rope, rope_cs=tables.of(rope))
         mask = dict(window=a.window, keep_first=a.keep_first, sink=L["sink"])
+        made = S.proj_prep(h, L["w_in"], None, H, G, D, V, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg, **prep)
+        if made is not None:
+            o = S.masked_attention(made[0], H, G, D, V, kcs[ci], vcs[ci], inp.seg, a.scale, vt=vts[ci], **mask)
+            return o, S.memory_layer(made[1], b.heads, b.dim, b.vdim, L["gate_bias"], b.gate_cap, states[f"mem{j}"], states[f"memn{j}"],
+                                     states[f"memm{j}"], inp.seg, L["mem_norm"], self.cfg.norm_eps, self.dtype)
+        x = R.proj_f32out(h, L["w_in"])                                # left q | k | v, right q | k | v | g | i | f
         return S.attention_and_memory(x[:, :nl], H, G, D, V, inp.positions, inp.slots, kcs[ci], vcs[ci], vts[ci], inp.seg,
                                       self.dtype, a.scale, prep, mask, x[:, nl:], b.heads, b.dim, b.vdim, L["gate_bias"],
                                       b.gate_cap, states[f"mem{j}"], states[f"memn{j}"], states[f"memm{j}"], inp.seg,

@@ -38,6 +38,7 @@ _SIGS = {
     "k8s_sample": [P, I, I, I, I, P, P, P, P, P, I, P, P, P, P, P, P, I, P, P, P, I],
     "k8s_gemm_skinny": [P, I, P, P, I, I, I, I, P],
     "k8s_gemm_rows": [P, I, P, P, I, I, I, I, I, I, I, P],
+    "k8s_gemm_prep": [P, I, P, I, I, I, I, P, P, I, I, P, P, F, F, P, P, P, P, P, P, P, I, I, I, I, I, P, I, P],
     "k8s_gemm_batch": [P, I, P, P, I, I, I, I, I, I, I, P],
     "k8s_gemm_rows_scaled": [P, I, P, P, I, I, I, I, I, I, I, P, I, F, F, P],
     "k8s_few_rows_f32_add": [P, I, P, P, P, I, F, F, P, P, F, P, P, P, I, I, I, P],

@@ -657,10 +657,14 @@ ADD_WAVES = {4: (11.5, 0.01318), 5: (14.5, 0.0147), 6: (15.5, 0.0174), 8: (21.0,
 ADD_MIN_ROWS, ADD_MAX_N = 512, 5120
 
 
-def _add_wave(M: int, N: int, K: int, f: int) -> float:
-    full, over = divmod(-(-M // (32 * f)) * (N // 256), 256)
-    t = ADD_WAVES[f][0] + ADD_WAVES[f][1] * K
+def _waves_time(waves: dict, M: int, N: int, K: int, f: int) -> float:
+    full, over = divmod(-(-M // (32 * f)) * -(-N // 256), 256)
+    t = waves[f][0] + waves[f][1] * K
     return full * t + ((0.75 + 0.25 * over / 256) * t if over else 0.0)
+
+
+def _add_wave(M: int, N: int, K: int, f: int) -> float:
+    return _waves_time(ADD_WAVES, M, N, K, f)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -692,6 +696,27 @@ def add_plan(M: int, N: int, K: int, then: int):
             best = min(best, (_add_wave(cut, N, K, f) + c, ((0, cut, f), (cut, M, g))))
     whole = M * N / 2.0 ** 24 * (ADD_WAVES[8][0] + ADD_WAVES[8][1] * K)
     return best[1] if whole >= (0.6 if then == THEN_NOTHING else 0.5) * best[0] else None
+
+
+# The same of gemm_prep.hip (K 2048: 39 us with 128 rows, 48 with 160, 54 with 192, 65 with 256)
+PREP_WAVES = {4: (12.5, 0.01318), 5: (16.5, 0.0147), 6: (18.0, 0.0174), 8: (22.0, 0.0206)}
+PREP_MIN_ROWS = 1280
+
+
+@functools.lru_cache(maxsize=4096)
+def prep_plan(M: int, N: int, K: int):
+    """Rows of a tile / 32 with which csrc/kernels/gemm_prep.hip makes an attention's input product of ``M`` rows and ``N`` columns, or
+    None: product and pass apart are the quicker.  The tiles that leave the least of their last wave of 256 idle.  us apart / so, 16
+    heads over 2 of 128 and K 2048, 2560 columns (rotated), 2576 (values mixed), 8736:  512 rows 23 / 39, 23 / 40, 36 / 49;  1024 31 / 36, 31 /
+    37, 53 / 48;  1280 42 / 37, 43 / 38, 70 / 55;  2048 48 / 38, 49 / 39, 98 / 84;  3517 60 / 46, 63 / 48, 139 / 123;  4096 65 / 52, 71 / 54, 190 / 147;
+    4850 74 / 62, 81 / 64, 207 / 164;  8192 112 / 95, 128 / 95, 332 / 275;  16384 237 / 176, 248 / 176, 614 / 515;  24730 345 / 239, 405 / 259, 940 /
+    765.  K 1024 and 4096 at 1280 rows 36 / 27, 35 / 28, 54 / 39 and 58 / 56, 55 / 56, 110 / 87, at 4096 51 / 38, 56 / 39, 133 / 96 and 98 / 83, 104 /
+    90, 378 / 274.  Whole waves with one size and the rest with another, in two launches, gain up to 3 % and lose up to 8."""
+    if M < PREP_MIN_ROWS or K % 64 or not 1024 <= K <= 8192:
+        return None
+    t, f = min((_waves_time(PREP_WAVES, M, N, K, f), f) for f in PREP_WAVES)
+    whole = M * N / 2.0 ** 24 * (PREP_WAVES[8][0] + PREP_WAVES[8][1] * K)
+    return f if whole >= 0.33 * t else None
 
 
 def gemm_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, scale: float, plan, then: int, alpha: float = 0.0, nw=None,

@@ -1418,6 +1418,44 @@ def masked_attention(q: torch.Tensor, H: int, G: int, D: int, V: int, kc: torch.
 PREP_GROUPS = 512
 
 
+def proj_prep(h: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D: int, V: int, slots: torch.Tensor,
+              kc: torch.Tensor, vc: Optional[torch.Tensor], vt: Optional[torch.Tensor], seg: SegMeta, norm=False,
+              q_w: Optional[torch.Tensor] = None, k_w: Optional[torch.Tensor] = None, eps: float = 0.0, lam: float = 0.0,
+              v_other: Optional[torch.Tensor] = None, v_keep: Optional[torch.Tensor] = None, rope: Optional[Rope] = None,
+              rope_cs: Optional[torch.Tensor] = None) -> Optional[tuple]:
+    """:func:`attn_prep` of the first ``(H + G) D + G V`` columns of ``h @ w.T`` and the other columns in fp32 (None where there are
+    none), of many rows in one launch (csrc/kernels/gemm_prep.hip), or None: sizes, types or places that it does not take, or where
+    :func:`.linear.prep_plan` leaves product and pass apart."""
+    from . import linear as LIN
+    T = slots.shape[0]
+    if T < LIN.PREP_MIN_ROWS or T == seg.n_seg or not isinstance(h, torch.Tensor):
+        return None
+    NQ, NK, NV = H * D, G * D, G * V
+    n, (N, K), rot = NQ + NK + NV, w.shape, rope.dims if rope is not None else 0
+    if not (vt is not None and use_hip(h) and D in (64, 128) and norm in (False, None, True, "head") and N >= n and N % 4 == 0
+            and NQ % 256 == NK % 256 == NV % 256 == 0 and NV > 0 and h.shape == (T, K) and LIN._few_ok(h, w)
+            and (rope is None or not rope.pairs and rope_cs is not None and 8 <= rot <= D and rot & (rot - 1) == 0)
+            and unwatched(h, w)):
+        return None
+    BS, dt = kc.shape[1], torch.bfloat16
+    small = ((bias, n), (q_w, D), (k_w, D), (v_other, T * NV), (v_keep, T * NV), (rope_cs, T * rot))
+    if not (all(t is None or t.dtype == torch.float32 and t.is_contiguous() and t.numel() == m and t.data_ptr() % 16 == 0
+                and t.device == h.device for t, m in small)
+            and all(t is None or t.is_contiguous() and t.dtype == dt and t.data_ptr() % 16 == 0 for t in (kc, vc, vt))
+            and kc.shape[2] == NK and (vc is None or vc.shape[1:] == (BS, NV)) and vt.shape[1:] == (NV, BS)
+            and slots.dtype == torch.int32 and slots.is_contiguous()):
+        return None
+    f = LIN.prep_plan(T, N, K)
+    if f is None:
+        return None
+    q = torch.empty(T, NQ, dtype=dt, device=h.device)
+    rest = torch.empty(T, N - n, dtype=torch.float32, device=h.device) if N > n else None
+    check(lib().k8s_gemm_prep(ptr(h), h.stride(0), ptr(w), T, N, K, f, ptr(bias), ptr(rope_cs), rot, int(bool(norm)), ptr(q_w), ptr(k_w),
+                              float(eps), float(lam), ptr(v_other), ptr(v_keep), ptr(slots), ptr(q), ptr(kc), ptr(vt), ptr(vc), BS, NQ, NK,
+                              NV, D, ptr(rest), N - n, stream_ptr(h)), "gemm_prep")
+    return q, rest
+
+
 def prep_attention(x: torch.Tensor, bias: Optional[torch.Tensor], H: int, G: int, D: int, V: int, positions: torch.Tensor,
                    slots: torch.Tensor, kc: torch.Tensor, vc: Optional[torch.Tensor], vt: Optional[torch.Tensor], seg: SegMeta,
                    out_dtype, scale: float, prep: dict, mask: dict) -> torch.Tensor:
