@@ -553,7 +553,7 @@ def plane_plan(M: int, N: int, K: int):
     plan = rows_plan(M, N, K, ROWS_F32, True) if M <= ROWS_MAX_M else None
     if plan is not None:
         return ROWS_CFG + plan[0], plan[1]
-    return _plane_plan(M, N, K, _enabled) if 0 < M <= NARROW_MAX_M else (14, 1)
+    return _plane_plan(M, N, K, _enabled) if 0 < M <= NARROW_MAX_M else _more_rows_plan(M, N, K)
 
 
 ROWS_CFG = 100      # past every stream configuration
@@ -568,6 +568,19 @@ def _plane_plan(M: int, N: int, K: int, skinny: bool):
             return 14, 1
     cfg, bn, s, most = (34, 32, 4, 320) if K < 4096 else (14, 64, 8, 256)
     while s > 1 and (-(-N // bn) * s > most or K < 128 * s or not stream_shape_ok(M, N, K, cfg, s)):
+        s //= 2
+    return cfg, s
+
+
+def _more_rows_plan(M: int, N: int, K: int):
+    """The same for 129 to 256 rows: a long K over few columns, which the library does not cut.  us of the library / of 64-column planes
+    at 129, 192, 256 rows:  2048 x 8192 26.6 / 14.8, 26.6 / 16.5, 28.8 / 19.7;  4096 x 4096 22.4 / 14.8, 33.0 / 16.2, 22.8 / 19.5;  4096 x 14336
+    65.6 / 38.0, 104 / 43, 69.6 / 50.4.  Not 2048 x 2048 9.3 / 7.3, 9.4 / 8.1, 9.9 / 10.5 and 1024 x 2048 8.4 / 6.6, 8.5 / 6.9, 8.9 / 8.9: the
+    pass behind has eight planes to read."""
+    if not NARROW_MAX_M < M <= DISPATCH_MAX_M or K < 4096 or N > 4096:
+        return 14, 1
+    cfg, s = 14 if M <= 192 else 13, 8
+    while s > 1 and (-(-N // 64) * s > 256 or K < 512 * s or not stream_shape_ok(M, N, K, cfg, s)):
         s //= 2
     return cfg, s
 
