@@ -13,11 +13,11 @@ OUTS = (L.ROWS_BF16, L.ROWS_F32, L.ROWS_SILU, L.ROWS_RELU2)
 def test_rule():
     assert L.batch_plan(64, 8192, 2048, L.ROWS_SILU) == (4, 1) and L.batch_plan(17, 4096, 2048, L.ROWS_SILU) == (2, 1)
     assert L.batch_plan(64, 8192, 2048, L.ROWS_RELU2) == (2, 1) and L.batch_plan(48, 8736, 2048, L.ROWS_F32) == (4, 1)
-    assert L.batch_plan(17, 2048, 8192, L.ROWS_F32, True) == (2, 4) and L.batch_plan(64, 2048, 2048, L.ROWS_F32, True) == (2, 4)
+    assert L.batch_plan(17, 2048, 8192, L.ROWS_F32, True) == (2, 4) and L.batch_plan(48, 2048, 2048, L.ROWS_F32, True) == (2, 4)
     assert L.batch_plan(64, 2560, 2048, L.ROWS_F32, True) == (2, 2)
     for m, n, k, out, planes in ((16, 8192, 2048, 0, False), (65, 8192, 2048, 0, False), (64, 8200, 2048, 0, False),
                                  (64, 8192, 2112, 0, False), (64, 8192, 1024, 2, False), (64, 8736, 2048, 1, False),
-                                 (64, 2048, 8192, 1, True), (64, 32768, 2048, 1, False), (40, 4096, 4096, 0, False)):
+                                 (64, 2048, 8192, 1, True), (64, 2048, 2048, 1, True), (64, 32768, 2048, 1, False), (40, 4096, 4096, 0, False)):
         assert L.batch_plan(m, n, k, out, planes) is None
     for m in (17, 32, 33, 64):                  # whatever the rule gives away fits the kernel
         for n in range(16, 20000, 368):
