@@ -383,7 +383,7 @@ class LizesunModel:
         keep = other = None
         if a.v_mix:
             if li == self.vmix_first:
-                keep = vmix["v"] = torch.empty(inp.slots.shape[0], G * V, dtype=torch.float32, device=self.device)
+                keep = vmix["v"] = torch.empty(inp.input_ids.shape[0], G * V, dtype=torch.float32, device=self.device)
             else:
                 other = vmix["v"]
         n = H * D + G * (D + V)
