@@ -1,4 +1,5 @@
-// Products of up to 32 rows, Y[M][N] = X[M][K] . W[N][K]^T, bf16 operands, fp32 accumulation (steps of single tokens).
+// Products of up to 32 rows, Y[M][N] = X[M][K] . W[N][K]^T, bf16 operands, fp32 accumulation (steps of single tokens); of 17 to 32 rows
+// those that gemm_batch.hip leaves.
 //
 // What bounds them is the weights' way from memory, so the kernel is laid out for that stream: every load instruction of W
 // covers 256 bytes (CH = 128) or 128 bytes (CH = 64) of a row, not the 64 of a matrix fragment read straight from memory;

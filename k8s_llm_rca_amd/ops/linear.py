@@ -477,8 +477,8 @@ STREAM_F32_MAX_M = 64
 
 
 def stream_f32_cfg(M: int, N: int, K: int) -> int:
-    """The stream kernel's form for a product of 17 to 64 rows with an fp32 result that neither the row-streaming nor the skinny
-    kernel takes, or 0: the library.  Strips of 32 columns within one wave of workgroups, then of 64 where they fill their waves.
+    """The stream kernel's form for a product of 17 to 64 rows with an fp32 result that neither :func:`batch_plan` nor the
+    row-streaming nor the skinny kernel takes, or 0: the library.  Strips of 32 columns within one wave of workgroups, then of 64 where they fill their waves.
     us of the library / this at 33, 64 rows:  2304 x 2048 8.8 / 8.6, 9.2 / 8.6;  2576 x 2048 9.0 / 8.7, 9.3 / 8.8;  2304 x 1024 8.6 /
     5.7, 8.9 / 5.8;  6144 x 2048 10.1 / 8.8, 10.0 / 8.9;  8192 x 2048 12.8 / 10.9, 13.2 / 11.4;  8736 x 2048 14.7 / 12.7, 14.9 / 13.3;
     12288 x 1024 9.9 / 7.6, 9.7 / 7.9;  16384 x 2048 18.2 / 17.7, 18.4 / 17.8;  32768 x 2048 36 / 31, 36 / 32;  65536 x 1024 32 / 28, 36 /
@@ -785,8 +785,8 @@ def gemm_big_silu_scaled(x: torch.Tensor, w: torch.Tensor, part: torch.Tensor, e
 
 
 def proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x @ w.T`` as activations, with the 32-column stream form where it is the fastest: 17 to 128 rows (below, the skinny
-    kernel) and one wave of strips with the K it was measured at.  us at 17..32 / 64 / 128 rows, hipBLASLt / this:
+    """``x @ w.T`` as activations, where neither :func:`batch_plan` nor another rule has it with the 32-column stream form where that is the
+    fastest: 17 to 128 rows (below, the skinny kernel) and one wave of strips with the K it was measured at.  us at 17..32 / 64 / 128 rows, hipBLASLt / this:
     8192 x 2048 12.3 / 10.2, 12.8 / 11.1, 15.6 / 13.7;  4736 x 2048 12.3 / 9.7, 12.9 / 10.7, 15.2 / 13.6;  2048 x 2048
     9.2 / 8.3, 10.6 / 8.3, 10.5 / 10.6.  At 273 strips the second wave costs it the lead (8736 x 2048, 64 rows:
     15.3 / 17.2);  a long K over few strips does where the library cuts it (1024 x 2048 at 24 / 128 rows 8.1 / 9.0, 8.4 /
@@ -837,7 +837,7 @@ def big_fused(M: int, N: int, K: int, silu: bool) -> bool:
 
 
 def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``max(x @ w.T, 0)^2`` as activations.  In one launch for up to 128 rows over one wave of 32-column strips (us apart /
+    """``max(x @ w.T, 0)^2`` as activations (17 to 64 rows: :func:`batch_plan`).  In one launch for up to 128 rows over one wave of 32-column strips (us apart /
     fused at 8192 x 2048: 1 row 10.5 / 9.8, 16 rows 12.9 / 10.1, 64 rows 15.5 / 11.0, 128 rows 17.9 / 13.9) and for prompts
     (:func:`big_fused`); the fused forms square the fp32 sum.  Not for few rows of up to 4096 columns: the strips are half the
     card, and the skinny kernel and its pass are quicker (2048 x 2048 at 1, 8, 16 rows 6.6 / 9.2, 7.4 / 9.2, 8.0 / 9.2, x 1024
@@ -864,7 +864,8 @@ def relu_sq_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def glu_proj(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``silu(x @ Wg.T) * (x @ Wu.T)`` as activations (w = [Wg; Wu]): what a dispatch table says, then one launch by shape.
+    """``silu(x @ Wg.T) * (x @ Wu.T)`` as activations (w = [Wg; Wu]): what a dispatch table says, then one launch by shape, of
+    17 to 64 rows as :func:`batch_plan` has it.
     Up to 128 rows (us apart / fused at 1, 16, 64, 128 rows): up to 256 strips of 16 outputs the 32-row strips, except where
     few weight bytes leave the skinny kernel ahead (4096 x 2048 11.4 / 9.9, 13.1 / 10.3, 15.8 / 11.1, 18.2 / 14.1;  2048 x
     2048 7.7 / 9.3, 9.3 / 9.6, 14.8 / 10.4, 17.8 / 13.5;  640 x 384 6.1 / 3.3 .. 9.4 / 4.6); wider weights the 64-row strips
