@@ -371,7 +371,9 @@ def _dyt_add(x, a, w, sy, a2, w2, sy2, alpha, nw, nb) -> Optional[torch.Tensor]:
             and _fp32_row(nb, W) and (M >= L.ADD_ROWS or L.add_plan(M, W, a.shape[1], L.THEN_NOTHING))):
         return None
     if _add(x, a, w, sy, L.THEN_NOTHING, None, None, 0.0) is None:
-        L.proj_add(x, a, w, sy)                      # (adds itself from ADD_ROWS on)
+        y = L.proj_add(x, a, w, sy)
+        if y is not None:                            # (from ADD_ROWS on it adds itself)
+            N.add_dyt(x, y, sy)
     return _add(x, a2, w2, sy2, L.THEN_DYT, nw, nb, alpha)[0]
 
 
