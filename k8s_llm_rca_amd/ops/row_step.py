@@ -212,8 +212,9 @@ class Scaled:
         return Scaled(*(t.index_select(0, idx) for t in (self.x, self.h, self.part)), self.nw, self.eps)
 
     def product(self, w: torch.Tensor, out_kind: int, plain, planes: bool = False, keep: bool = False):
-        if self.h.shape[0] > INTO_ROWS:
-            if out_kind == L.ROWS_SILU and L.silu_scales(self.h.shape[0], w) and w.shape[1] == self.h.shape[1]:
+        if self.h.shape[0] > INTO_ROWS:              # (chosen rows of fewer have their parts in other sizes)
+            if (out_kind == L.ROWS_SILU and w.shape[1] == self.h.shape[1] == 256 * self.part.shape[1]
+                    and L.silu_scales(self.h.shape[0], w)):
                 return L.gemm_big_silu_scaled(self.h, w, self.part, self.eps)
             return plain(self.read(), w)
         if self.h.dtype == torch.float32:
@@ -222,7 +223,7 @@ class Scaled:
         if (out_kind == L.ROWS_RELU2 or keep or k != w.shape[1] or w.shape[0] % 2 and out_kind == L.ROWS_SILU
                 or not L.rows_ok(self.h, w) or (("silu", w.shape[0], k) in L.dispatch_table()) or (n, k) in L.dispatch_table()):
             return plain(self.read(), w)
-        p = L.rows_plan(m, n, k, out_kind, planes) if m <= INTO_ROWS else None
+        p = L.rows_plan(m, n, k, out_kind, planes) if m <= INTO_ROWS and self.part.shape[1] % 4 == 0 else None
         if p is None:
             return plain(self.read(), w)
         out = torch.empty((p[1], m, n) if planes else (m, n), device=w.device,
