@@ -246,7 +246,8 @@ class Scaled:
 
 def _into_operands(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, out_dtype) -> bool:
     return (a.is_cuda and out_dtype == torch.bfloat16 and x.dtype == torch.float32 and x.is_contiguous()
-            and w.shape == (x.shape[-1], a.shape[1]) and w.device == x.device == a.device and L.rows_ok(a, w))
+            and w.shape == (x.shape[-1], a.shape[1]) and w.device == x.device == a.device and L.rows_ok(a, w)
+            and (a.shape[0] == 1 or a.stride(0) >= a.shape[1]))
 
 
 def _into_f32(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:

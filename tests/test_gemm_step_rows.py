@@ -59,3 +59,22 @@ def test_past_the_line(m, n, k, two):
     assert float((x.double() - want).abs().max()) < bound
     ref = torch.tanh(0.7 * want) * nw.double() + nb.double()
     assert bool(((h.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 4 * bound).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,stride", [(3, 64, 3072, 8), (16, 64, 4096, 0), (12, 64, 4096, 2048), (1, 64, 4096, 0)])
+def test_rows_that_overlap(m, n, k, stride):
+    """Rows of X that share memory go where they went: the kernel takes rows that lie apart, and any single one."""
+    assert R.into_long(m, n, k) or R.into_ok(m, n, k)
+    g = torch.Generator().manual_seed(m + stride)
+    a = torch.randn(m * stride + k, generator=g).to(BF).cuda().as_strided((m, k), (stride, 1))
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(BF).cuda()
+    x0, nw, nb = (torch.randn(*s, generator=g).cuda() for s in ((m, n), (n,), (n,)))
+    x = x0.clone()
+    h = R.dyt_product(x, a, w, 0.5, None, None, 1.0, 0.7, nw, nb, BF)
+    want = x0.double() + 0.5 * (a.double() @ w.double().T)
+    bound = 4e-6 * (k ** 0.5 + 1)
+    ref = torch.tanh(0.7 * want) * nw.double() + nb.double()
+    if isinstance(h, R.RowStep):
+        h = h.read()
+    assert bool(((h.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 4 * bound).all())
