@@ -158,21 +158,31 @@ def batch_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = Fals
     0.75 | 0.79 - 0.92;  1024 x 2048 0.76, 0.80 | 0.91, 0.97, 1.04, 1.09;  4096 x 4096 0.82, 0.90 | 0.97, 1.02, 1.12, 1.06;  8192 x 1024
     0.89, 0.87 | 0.87 - 0.97;  2048 x 1024 0.75, 0.78 | 0.95, 0.97, 1.04, 1.07.  fp32 2576 x 2048 0.92, 0.88 | 0.80 - 0.92;  8736 x
     2048 0.83, 0.77 | 0.92, 0.95, 1.01, 1.03;  32768 x 2048 0.99, 0.99 | 0.95, 0.96, 1.03, 1.05;  50256 x 4096 0.94, 0.96 | 1.01 - 1.13.
-    Planes (without the pass behind, which has fewer of them to read) 2048 x 2048 0.99, 0.94 | 0.93, 0.97, 0.97, 1.00 (in a model's
-    step of 64 rows 5.1 - 5.2 / 5.7 us: not past 48), x 8192 0.87, 0.92 | 0.99, 1.02, 1.08, 1.10;  4096 x 2048 0.90, 0.87 | 0.90 - 0.96;
-    1024 x 4096 0.73, 0.75 | 0.85 - 0.88;  2048 x 1024 0.98, 0.96 | 1.10 - 1.15."""
+    Planes with the pass behind, by K ranges, over 512 to 4096 columns, weights out of memory: eight 0.80 - 0.99 at every number of rows;
+    four 0.80 - 0.98 up to 32 rows (2048 x 8192 0.93), 0.91 - 1.01 up to 48, past that 0.93 - 1.05 (8192 entries of K 1.00 - 1.05);  two, which
+    is all that 2560, 3584, 4608 and 7680 allow, leave up to 2048 columns on few units: at 17, 24, 32 | 48 rows 1024 x 2560 0.96, 1.00,
+    1.02 | 1.12, x 3584 0.94, 0.97, 0.99 | 1.10, x 4608 1.02, 1.05, 1.08 | 1.18, x 7680 1.10, 1.20, 1.25 | 1.37 (but x 1536 0.94 - 0.97);  two
+    of more than 2048 columns, whose strips fill the units, 0.74 - 0.99 up to 32 rows, 0.84 - 0.99 past them with K up to 3584, from
+    4096 on 0.94 - 1.10."""
     big = N * (2 if out == ROWS_SILU else 1)
     if not BATCH_ROWS[0] < M <= BATCH_ROWS[1] or N % 16 or big < 512 or K % 256 or not 512 <= K <= 8192:
         return None
     few = M <= 32
     if planes:
-        if N > 4096 or K < 1024 or not few and (K < 2048 or N < 1024 or K > 2048 and N > 2048 or M > 48
-                                                   and (N <= 2048 if K == 2048 else N > 1024)):
+        if N > 4096 or K < (1024 if few else 2048):
             return None
         ranges = 8
         while ranges > 1 and (-(-N // 32) * ranges > 256 or K % (256 * ranges)):
             ranges //= 2
-        return (2, ranges) if ranges > 1 else None
+        if ranges == 1:
+            return None
+        if ranges == 4 and M > 48:                   # (more planes to read than gain)
+            return None
+        if ranges == 2 and N <= 2048 and (not few or K > 2048 and (M > 24 or K >= 4096)):      # K that more ranges do not divide
+            return None
+        if ranges == 2 and not few and K >= 4096:
+            return None
+        return 2, ranges
     if K > 4096 and out != ROWS_SILU:
         return None
     nf = 2 if big <= 8192 else 4

@@ -29,6 +29,22 @@ def test_rule():
                         assert n >= strip and k % (256 * plan[1]) == 0 and (out != L.ROWS_SILU or n % strip == 0)
 
 
+def test_planes_rule():
+    """Which planes it takes turns on how far K is cut and on the rows, and on both sides of a line for a range of widths."""
+    def took(n, k, m):
+        return L.batch_plan(m, n, k, L.ROWS_F32, True) is not None
+    for n in (512, 640, 768, 896, 1024):                    # eight ranges: at every number of rows
+        assert all(took(n, k, m) for k in (2048, 4096, 6144, 8192) for m in (17, 32, 33, 48, 49, 64))
+    for n in (1040, 1280, 1536, 2048):                      # four: up to 48 rows
+        assert all(took(n, k, m) == (m <= 48) for k in (2048, 3072, 4096, 5120, 8192) for m in (17, 32, 33, 48, 49, 64))
+    for n in (512, 1024, 1536, 2048):                       # two, of K that no more divide
+        for k, most in ((1536, 32), (2560, 24), (3584, 24), (4608, 0), (5632, 0), (7680, 0)):
+            assert all(took(n, k, m) == (m <= most) for m in (17, 24, 25, 32, 33, 48, 64))
+    for n in (2064, 2304, 3072, 4096):                      # two that fill the units
+        for k, most in ((1024, 32), (2048, 64), (2560, 64), (3584, 64), (4096, 32), (8192, 32)):
+            assert all(took(n, k, m) == (m <= most) for m in (17, 32, 33, 48, 64))
+
+
 def check_one(m, n, k, nf, ranges, out, pad=8):
     g = torch.Generator().manual_seed(m + n + k)
     rows = n * (2 if out == L.ROWS_SILU else 1)
