@@ -153,7 +153,11 @@ def batch_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = Fals
     SwiGLU 8192 x 2048 0.96, 0.95 | 0.81, 0.81, 0.89, 0.92;  4096 x 2048 0.92, 0.88 | 0.82, 0.80, 0.91, 0.92;  6144 x 2048 (0.75 waves of
     four fragments) 0.86, 0.93 | 0.91, 0.93, 0.99, 1.02;  16384 x 2048 0.98, 0.96 | 0.82, 0.84, 0.86, 0.92;  8192 x 4096 0.93, 0.96 |
     0.77, 0.65, 0.82, 0.87;  3072 x 1024 0.78, 0.76 | 0.86, 0.91, 0.95, 0.98;  8192 x 1024 0.94, 0.93 | 1.07, 1.05, 1.15, 1.17;  1024 x
-    512 0.82, 0.87 | 1.06 - 1.14;  4096 x 8192 0.96, 0.97 | 0.92 - 0.97.  Squared relu 8192 x 2048 0.88, 0.86 | 0.81, 0.84, 0.90, 0.91, x
+    512 0.82, 0.87 | 1.06 - 1.14;  4096 x 8192 0.96, 0.97 | 0.92 - 0.97.  A long
+    K over few strips is the library's, which cuts it (weights out of memory, at 17, 28 | 40, 48 | 56 rows): 512 x 5632 0.99, 1.07 | 1.26,
+    1.33 | 1.41, x 8192 1.10, 1.20 | 1.36, 1.39 | 1.47;  1024 x 5120 0.67, 0.72 | 0.99, 1.08 | 1.18, x 6144 0.98, 1.04 | 0.92, 0.97 | 1.07, x 8192
+    1.00, 1.08 | 1.27, 1.21 | 1.36;  1408 x 6144 0.70, 0.76 | 0.86, 0.91 | 0.98, x 8192 0.96, 0.99 | 0.91, 0.93 | 1.05;  2304 x 8192 0.71,
+    0.80 | 0.57, 0.58 | 0.86.  Squared relu 8192 x 2048 0.88, 0.86 | 0.81, 0.84, 0.90, 0.91, x
     4096 0.84, 0.86 | 0.71 - 0.83;  16384 x 2048 0.89, 0.95 | 0.69 - 0.77;  4096 x 512 0.77, 0.82 | 1.03 - 1.09.  bf16 2560 x 2048 0.70,
     0.75 | 0.79 - 0.92;  1024 x 2048 0.76, 0.80 | 0.91, 0.97, 1.04, 1.09;  4096 x 4096 0.82, 0.90 | 0.97, 1.02, 1.12, 1.06;  8192 x 1024
     0.89, 0.87 | 0.87 - 0.97;  2048 x 1024 0.75, 0.78 | 0.95, 0.97, 1.04, 1.07.  fp32 2576 x 2048 0.92, 0.88 | 0.80 - 0.92;  8736 x
@@ -188,6 +192,8 @@ def batch_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = Fals
     nf = 2 if big <= 8192 else 4
     if out == ROWS_SILU and N % (8 * nf):
         return None
+    if K >= 5120 and big <= (4096 if M > 48 else 2560 if not few else 2048 if K > 5120 else 0):
+        return None                                  # a long K over few strips, which the library cuts
     if few:
         return (nf, 1) if big <= 16384 or out >= ROWS_SILU or K > 2048 or M > 24 else None
     if K < 2048:

@@ -45,6 +45,15 @@ def test_planes_rule():
             assert all(took(n, k, m) == (m <= most) for m in (17, 32, 33, 48, 64))
 
 
+def test_long_k_over_few_strips():
+    def took(big, k, m):
+        return L.batch_plan(m, big // 2, k, L.ROWS_SILU) is not None
+    for k, least in ((4096, (0, 0, 0)), (4864, (0, 0, 0)), (5120, (0, 2560, 4096)), (5632, (2048, 2560, 4096)), (8192, (2048, 2560, 4096))):
+        for big in (512, 1024, 2048, 2112, 2560, 2624, 4096, 4160, 8192):
+            for m, line in ((17, least[0]), (32, least[0]), (33, least[1]), (48, least[1]), (49, least[2]), (64, least[2])):
+                assert took(big, k, m) == (big > line), (big, k, m)
+
+
 def check_one(m, n, k, nf, ranges, out, pad=8):
     g = torch.Generator().manual_seed(m + n + k)
     rows = n * (2 if out == L.ROWS_SILU else 1)
