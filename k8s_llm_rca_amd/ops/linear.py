@@ -157,7 +157,9 @@ def batch_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = Fals
     K over few strips is the library's, which cuts it (weights out of memory, at 17, 28 | 40, 48 | 56 rows): 512 x 5632 0.99, 1.07 | 1.26,
     1.33 | 1.41, x 8192 1.10, 1.20 | 1.36, 1.39 | 1.47;  1024 x 5120 0.67, 0.72 | 0.99, 1.08 | 1.18, x 6144 0.98, 1.04 | 0.92, 0.97 | 1.07, x 8192
     1.00, 1.08 | 1.27, 1.21 | 1.36;  1408 x 6144 0.70, 0.76 | 0.86, 0.91 | 0.98, x 8192 0.96, 0.99 | 0.91, 0.93 | 1.05;  2304 x 8192 0.71,
-    0.80 | 0.57, 0.58 | 0.86.  Squared relu 8192 x 2048 0.88, 0.86 | 0.81, 0.84, 0.90, 0.91, x
+    0.80 | 0.57, 0.58 | 0.86.  More than a wave of four
+    fragments (8256, 10240, 12288 | 14336 at 17, 20, 24 rows), x 768 1.04, 1.02, 0.98, 1.04, 1.02, 0.97, 1.10, 1.07, 1.02 | 0.97, 0.98, 0.96, x 2048
+    1.03, 1.01, 0.99, 1.01, 1.00, 0.99, 1.05, 1.05, 1.01 | 0.97, 0.97, 0.98: up to there the row-streaming kernel has two of them.  Squared relu 8192 x 2048 0.88, 0.86 | 0.81, 0.84, 0.90, 0.91, x
     4096 0.84, 0.86 | 0.71 - 0.83;  16384 x 2048 0.89, 0.95 | 0.69 - 0.77;  4096 x 512 0.77, 0.82 | 1.03 - 1.09.  bf16 2560 x 2048 0.70,
     0.75 | 0.79 - 0.92;  1024 x 2048 0.76, 0.80 | 0.91, 0.97, 1.04, 1.09;  4096 x 4096 0.82, 0.90 | 0.97, 1.02, 1.12, 1.06;  8192 x 1024
     0.89, 0.87 | 0.87 - 0.97;  2048 x 1024 0.75, 0.78 | 0.95, 0.97, 1.04, 1.07.  fp32 2576 x 2048 0.92, 0.88 | 0.80 - 0.92;  8736 x
@@ -195,7 +197,10 @@ def batch_plan(M: int, N: int, K: int, out: int = ROWS_BF16, planes: bool = Fals
     if K >= 5120 and big <= (4096 if M > 48 else 2560 if not few else 2048 if K > 5120 else 0):
         return None                                  # a long K over few strips, which the library cuts
     if few:
-        return (nf, 1) if big <= 16384 or out >= ROWS_SILU or K > 2048 or M > 24 else None
+        if M <= 24 and big > 16384 and (out < ROWS_SILU and K <= 2048
+                                        or out >= ROWS_SILU and big <= 24576 and rows_plan(M, N, K, out) == (2, 1)):
+            return None                              # up to one and a half waves of strips: the row-streaming kernel's two fragments
+        return nf, 1
     if K < 2048:
         return (nf, 1) if K >= 1024 and 6144 <= big <= 8192 else None
     if out >= ROWS_SILU:

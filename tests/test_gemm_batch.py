@@ -54,6 +54,17 @@ def test_long_k_over_few_strips():
                 assert took(big, k, m) == (big > line), (big, k, m)
 
 
+def test_more_than_a_wave_of_few_rows():
+    """Up to 24 rows the row-streaming kernel keeps what it takes with two fragments; where it has four, or nothing, this one goes on."""
+    for out in (L.ROWS_SILU, L.ROWS_RELU2):
+        for big in (16384, 16640, 18432, 20480, 24576, 28672, 32768):
+            for k in (512, 768, 1024, 1536, 2048, 3072, 4096):
+                for m in (17, 24, 25, 32):
+                    n = big // 2 if out == L.ROWS_SILU else big
+                    left = m <= 24 and 16384 < big <= 24576 and k not in (1536, 3072)
+                    assert (L.batch_plan(m, n, k, out) is None) == left, (out, big, k, m)
+
+
 def check_one(m, n, k, nf, ranges, out, pad=8):
     g = torch.Generator().manual_seed(m + n + k)
     rows = n * (2 if out == L.ROWS_SILU else 1)
