@@ -59,17 +59,16 @@ constexpr int kMemVb = 64;     // state columns per workgroup
 // four of them at once / so, 16 heads:  5 sequences of 560 to 1100 tokens 29 / 19 / 9.4, 8 of 2048 58 / 35 / 15.6, 64 of 256 to 512 21.5 /
 // 15.9 / 15.1.
 constexpr int kGateWaves = 8;
-__global__ void __launch_bounds__(64 * kGateWaves) memory_gates_kernel(const float* __restrict__ x, int xs,
-                                                                       const float* __restrict__ gate_bias, float cap,
-                                                                       float* __restrict__ mstate,
-                                                                       const int* __restrict__ seg_row0,
-                                                                       const int* __restrict__ seg_pos0,
-                                                                       const int* __restrict__ seg_slot, float* __restrict__ ab,
-                                                                       int H, int D, int V) {
-  constexpr int NW = kGateWaves;
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) memory_gates_kernel(const float* __restrict__ x, int xs,
+                                                               const float* __restrict__ gate_bias, float cap, float* __restrict__ mstate,
+                                                               const int* __restrict__ seg_row0, const int* __restrict__ seg_pos0,
+                                                               const int* __restrict__ seg_slot, float* __restrict__ ab, int H, int D, int V) {
   __shared__ float ends[2][NW][2];                 // of a wave's last token: the sum and the maximum
   const int sg = blockIdx.x / H, hh = blockIdx.x - sg * H, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int r0 = seg_row0[sg], r1 = seg_row0[sg + 1];
+  const bool alone = NW == 1 || r1 - r0 <= 64;     // one wave has all of it
+  if (alone && wv) return;
   const size_t so = (size_t)seg_slot[sg] * H + hh;
   float m0 = seg_pos0[sg] == 0 ? 0.f : mstate[so];
   const float* xi = x + 2 * H * D + 2 * H * V + hh;
@@ -103,13 +102,18 @@ __global__ void __launch_bounds__(64 * kGateWaves) memory_gates_kernel(const flo
       const float up = __shfl_up(pa, o, 64);
       if (lane >= o) pa = fmaxf(pa, up);
     }
-    if (lane == min(63, r1 - tb - 1)) ends[p][wv][0] = F, ends[p][wv][1] = pa;
-    __syncthreads();
+    const int last = min(63, r1 - tb - 1);
     float mine = m0;
+    if (alone) {
+      m0 = __shfl(F, last, 64) + fmaxf(m0, __shfl(pa, last, 64));
+    } else {
+      if (lane == last) ends[p][wv][0] = F, ends[p][wv][1] = pa;
+      __syncthreads();
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      if (w == wv) mine = m0;
-      if (t0 + 64 * w < r1) m0 = ends[p][w][0] + fmaxf(m0, ends[p][w][1]);
+      for (int w = 0; w < NW; ++w) {
+        if (w == wv) mine = m0;
+        if (t0 + 64 * w < r1) m0 = ends[p][w][0] + fmaxf(m0, ends[p][w][1]);
+      }
     }
     const float m = F + fmaxf(mine, pa);
     const float mup = __shfl_up(m, 1, 64);
@@ -121,7 +125,7 @@ __global__ void __launch_bounds__(64 * kGateWaves) memory_gates_kernel(const flo
       o[2] = m;
     }
   }
-  __syncthreads();                                 // every wave has read mstate
+  if (!alone) __syncthreads();                     // every wave has read mstate
   if (threadIdx.x == 0) mstate[so] = m0;
 }
 
@@ -664,8 +668,9 @@ K8S_API int k8s_matrix_memory(const float* x, int xs, const float* gate_bias, fl
                               float* cs, float* cx, float* cdec, float* tile_ws) {
   if (n_seg <= 0 || T <= 0) return 0;
   if (D < 1 || D > 256 || cap <= 0.f) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(memory_gates_kernel, dim3(n_seg * H), dim3(64 * kGateWaves), 0, s, x, xs, gate_bias, cap, mstate,
-                     seg_row0, seg_pos0, seg_slot, ab, H, D, V);
+  const bool short_all = T - n_seg < 64;             // no sequence has more rows than a wave
+  hipLaunchKernelGGL((short_all ? memory_gates_kernel<1> : memory_gates_kernel<kGateWaves>), dim3(n_seg * H),
+                     dim3(short_all ? 64 : 64 * kGateWaves), 0, s, x, xs, gate_bias, cap, mstate, seg_row0, seg_pos0, seg_slot, ab, H, D, V);
   MatArgs p{};
   p.x = x;
   p.xs = xs;

@@ -74,3 +74,9 @@ def test_gates(rows):
             assert float((ab[t].double() - want).abs().max()) < 1e-4 * (1 + float(new.abs().max())), (i, t)
             m = new
         assert float((ms[i].double() - m).abs().max()) < 1e-4 * (1 + float(m.abs().max()))
+
+
+@pytest.mark.parametrize("rows", [[10, 1, 30, 19], [70, 0, 0, 0, 0, 0, 0, 0], [64, 1, 129], [64] * 3 + [1] * 9])
+def test_gates_of_short_sequences(rows):
+    """Sequences that one wave has alone, among themselves and beside a longer one, and one wave for more rows than it has lanes."""
+    test_gates(rows)
