@@ -598,8 +598,14 @@ def _more_rows_plan(M: int, N: int, K: int):
     """The same for 129 to 256 rows: a long K over few columns, which the library does not cut.  us of the library / of 64-column planes
     at 129, 192, 256 rows:  2048 x 8192 26.6 / 14.8, 26.6 / 16.5, 28.8 / 19.7;  4096 x 4096 22.4 / 14.8, 33.0 / 16.2, 22.8 / 19.5;  4096 x 14336
     65.6 / 38.0, 104 / 43, 69.6 / 50.4.  Not 2048 x 2048 9.3 / 7.3, 9.4 / 8.1, 9.9 / 10.5 and 1024 x 2048 8.4 / 6.6, 8.5 / 6.9, 8.9 / 8.9: the
-    pass behind has eight planes to read."""
-    if not NARROW_MAX_M < M <= DISPATCH_MAX_M or K < 4096 or N > 4096:
+    pass behind has eight planes to read.  Nor few columns, which the library does cut, of a long K or past 192 rows (three stages of
+    the ring; one strip is the same either way), with that pass at 129, 192, 193, 256 rows:  64 x 4096 13.8 / 11.7, 13.7 / 12.3, 13.8 / 14.0,
+    13.8 / 14.1;  256 x 4096 14.0 / 11.8, 13.8 / 12.6, 13.9 / 14.4, 13.9 / 14.6, x 8192 14.4 / 15.6, 14.1 / 16.9, 14.2 / 19.6, 14.2 / 19.9;  512 x
+    8192 16.2 / 16.9, 17.4 / 17.7, 16.6 / 20.0, 17.1 / 20.8;  768 x 8192 16.6 / 16.9, 23.5 / 18.4, 23.4 / 20.7, 22.6 / 21.7;  1024 x 4096 15.8 /
+    13.9, 16.0 / 15.4, 15.9 / 17.1, 16.0 / 18.2;  1280 x 4096 16.1 / 14.6, 16.3 / 16.4, 17.9 / 17.9, 19.4 / 18.0."""
+    strips = -(-N // 64)
+    if (not NARROW_MAX_M < M <= DISPATCH_MAX_M or K < 4096 or N > 4096 or strips < 8 and K > 5120
+            or M > 192 and 1 < strips < (20 if K <= 5120 else 12)):
         return 14, 1
     cfg, s = 14 if M <= 192 else 13, 8
     while s > 1 and (-(-N // 64) * s > 256 or K < 512 * s or not stream_shape_ok(M, N, K, cfg, s)):

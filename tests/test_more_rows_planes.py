@@ -13,6 +13,15 @@ def test_rule():
         assert L.plane_plan(m, n, k)[1] == 1
 
 
+def test_few_columns():
+    """Few columns are cut where the library is the slower: K up to 5120 at up to 192 rows, and past that one strip, or enough of them."""
+    for k in (4096, 4608, 5120, 6144, 8192, 14336):
+        for n in (64, 128, 256, 448, 512, 704, 768, 1024, 1216, 1280, 2048, 4096):
+            for m in (129, 192, 193, 256):
+                cut = (k <= 5120 or n >= 512) if m <= 192 else (n == 64 or n >= 1280) if k <= 5120 else n >= 768
+                assert (L.plane_plan(m, n, k)[1] > 1) == cut, (m, n, k)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m", [129, 192, 193, 256])
 @pytest.mark.parametrize("n,k", [(2048, 8192), (64, 4096), (4096, 4096 + 512)])
