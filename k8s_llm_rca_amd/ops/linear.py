@@ -745,19 +745,29 @@ PREP_MIN_ROWS = 1280
 
 
 @functools.lru_cache(maxsize=4096)
-def prep_plan(M: int, N: int, K: int):
-    """Rows of a tile / 32 with which csrc/kernels/gemm_prep.hip makes an attention's input product of ``M`` rows and ``N`` columns, or
-    None: product and pass apart are the quicker.  The tiles that leave the least of their last wave of 256 idle.  us apart / so, 16
+def prep_plan(M: int, N: int, K: int, n: int = 0):
+    """Rows of a tile / 32 with which csrc/kernels/gemm_prep.hip makes an attention's input product of ``M`` rows and ``N`` columns, of
+    which the first ``n`` (0: all) are rotated, normed or paged, or None: product and pass apart are the quicker.  The tiles that leave the least of their last wave of 256 idle.  us apart / so, 16
     heads over 2 of 128 and K 2048, 2560 columns (rotated), 2576 (values mixed), 8736:  512 rows 23 / 39, 23 / 40, 36 / 49;  1024 31 / 36, 31 /
     37, 53 / 48;  1280 42 / 37, 43 / 38, 70 / 55;  2048 48 / 38, 49 / 39, 98 / 84;  3517 60 / 46, 63 / 48, 139 / 123;  4096 65 / 52, 71 / 54, 190 / 147;
     4850 74 / 62, 81 / 64, 207 / 164;  8192 112 / 95, 128 / 95, 332 / 275;  16384 237 / 176, 248 / 176, 614 / 515;  24730 345 / 239, 405 / 259, 940 /
     765.  K 1024 and 4096 at 1280 rows 36 / 27, 35 / 28, 54 / 39 and 58 / 56, 55 / 56, 110 / 87, at 4096 51 / 38, 56 / 39, 133 / 96 and 98 / 83, 104 /
-    90, 378 / 274.  Whole waves with one size and the rest with another, in two launches, gain up to 3 % and lose up to 8."""
+    90, 378 / 274.  Whole waves with one size and the rest with another, in two launches, gain up to 3 % and lose up to 8.
+
+    Taken by what the same work takes in whole waves of 256-row tiles, over what it takes so: the longer K, the better the library has a
+    wave that is not full, and the fewer columns the pass has, the less there is to save.  us apart / so at 1280, 1536, 1800, 2048, 2600 rows
+    (0.37, 0.43, 0.49, 0.55, 0.66 of the whole waves' rate):  2576 columns, K 3072 46 / 46, 48 / 47, 53 / 48, 57 / 49, 66 / 52;  4096 53 / 55, 55 / 56,
+    61 / 58, 68 / 59, 77 / 63;  6144 66 / 74, 69 / 74, 77 / 76, 84 / 79, 105 / 86;  8192 77 / 89, 82 / 89, 93 / 97, 104 / 97, 123 / 106;  2560 with K 8192
+    80 / 89, 83 / 89, 96 / 97, 101 / 100, 120 / 102.  2048 columns with 1536 for the pass (0.31, 0.36, 0.41, 0.46, 0.56): K 2048 34 / 36, 35 / 36, 37 / 37,
+    37 / 36, 42 / 38;  4096 44 / 52, 45 / 54, 49 / 55, 51 / 55, 60 / 56;  8192 66 / 87, 68 / 87, 77 / 90, 80 / 91, 101 / 95."""
     if M < PREP_MIN_ROWS or K % 64 or not 1024 <= K <= 8192:
         return None
     t, f = min((_waves_time(PREP_WAVES, M, N, K, f), f) for f in PREP_WAVES)
     whole = M * N / 2.0 ** 24 * (PREP_WAVES[8][0] + PREP_WAVES[8][1] * K)
-    return f if whole >= 0.33 * t else None
+    least = 0.33 + (0.06 * max(0, min(K, 4096) - 2048) + 0.02 * max(0, K - 4096)) / 1024
+    if K >= 2048 and n:
+        least += min(0.1, 0.4 * (1 - n / N))
+    return f if whole >= least * t else None
 
 
 def gemm_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, scale: float, plan, then: int, alpha: float = 0.0, nw=None,

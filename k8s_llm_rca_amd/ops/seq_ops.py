@@ -1445,7 +1445,7 @@ def proj_prep(h: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], H:
             and kc.shape[2] == NK and (vc is None or vc.shape[1:] == (BS, NV)) and vt.shape[1:] == (NV, BS)
             and slots.dtype == torch.int32 and slots.is_contiguous()):
         return None
-    f = LIN.prep_plan(T, N, K)
+    f = LIN.prep_plan(T, N, K, n)
     if f is None:
         return None
     q = torch.empty(T, NQ, dtype=dt, device=h.device)

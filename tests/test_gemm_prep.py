@@ -17,6 +17,16 @@ def test_plan():
         assert L.prep_plan(*bad) is None
 
 
+def test_plan_of_long_k():
+    """Product and pass stay apart where the library has a wave that is not full the quicker: sizes timed on both sides."""
+    def took(m, n, k, prepared):
+        return L.prep_plan(m, n, k, prepared) is not None
+    for n, k, prepared, line in ((2576, 2048, 2560, 1280), (2576, 3072, 2560, 1400), (2576, 4096, 2560, 1800), (2576, 6144, 2560, 2048),
+                                 (2560, 8192, 2560, 2048), (2048, 2048, 1536, 2048), (2048, 4096, 1536, 2600), (8736, 8192, 2560, 1280)):
+        for rows in (1280, 1400, 1536, 1800, 2048, 2600, 3517):
+            assert took(rows, n, k, prepared) == (rows >= line), (rows, n, k)
+
+
 def oracle(h, w, bias, H, G, D, NV, cs, rot, norm, qw, kw, eps, lam, vo):
     x = h.double() @ w.double().T
     n = (H + G) * D + NV
