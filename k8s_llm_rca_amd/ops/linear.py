@@ -704,15 +704,25 @@ def _waves_time(waves: dict, M: int, N: int, K: int, f: int) -> float:
     return full * t + ((0.75 + 0.25 * over / 256) * t if over else 0.0)
 
 
-def _add_wave(M: int, N: int, K: int, f: int) -> float:
-    return _waves_time(ADD_WAVES, M, N, K, f)
+# us of a second launch: its own, and a chip that the first one leaves to drain
+CUT_US = 5.0
+
+
+def _add_time(M: int, N: int, K: int, f: int) -> float:
+    """With 4096 columns the 32 tiles an XCD has at a time are half of four row tiles' columns, and in every XCD the same half where
+    their ranges begin with a group: half of the memory's channels.  us of one launch / of two that do not, with tanh: K 1024 at 16384 rows
+    272 / 235, 2048 at 8192 165 / 154, at 16384 351 / 319, 4096 505 / 479, 8192 829 / 808."""
+    t = _waves_time(ADD_WAVES, M, N, K, f)
+    return t * 1.05 if N == 4096 and -(-M // (32 * f)) % 32 == 0 else t
 
 
 @functools.lru_cache(maxsize=4096)
 def add_plan(M: int, N: int, K: int, then: int):
     """Row ranges (from, to, rows of a tile / 32) in which :func:`gemm_add` makes a product of ``M`` rows, or None: the product and
-    the pass behind it are the quicker.  Tiles that leave the least of their last wave of 256 idle, or whole waves of them and other
-    tiles, or (0) a product and a pass of its own, for the rest.
+    the pass behind it are the quicker.  Tiles that leave the least of their last wave of 256 idle, or whole waves of them and, where that
+    is worth a second launch, other tiles, or (0) a product and a pass of its own, for the rest.  us of two launches of the same tiles / of
+    one, with tanh:  12288 x 2048, K 1024 90 / 85, 10000 x 2048, K 2048 109 / 105, 8192 285 / 276, 16384 x 5120, K 2048 419 / 391;  of others:
+    12288 x 2048, K 2048 123 / 116, 24576 x 1024 123 / 116, but 20000 x 2048, K 8192 542 / 574, 8192 x 3072 335 / 358.
 
     Taken by what the same work takes in whole waves of 256-row tiles, over what it takes so.  Time of product and pass over this,
     at 0.40 of the whole waves' rate 0.86 (with tanh) and 0.98 (scaled), 0.48 1.00 and 1.17, 0.55 0.98 - 1.08 and 1.00 - 1.14, 0.66
@@ -723,20 +733,23 @@ def add_plan(M: int, N: int, K: int, then: int):
     if N % 256 or N > ADD_MAX_N or K % 64 or not 1024 <= K <= 16384 or M < ADD_MIN_ROWS or then == THEN_NOTHING and M >= ADD_ROWS:
         return None
     nt = N // 256
-    best = min((_add_wave(M, N, K, f), ((0, M, f),)) for f in ADD_WAVES)
+    best = min((_add_time(M, N, K, f), ((0, M, f),)) for f in ADD_WAVES)
+    took = best[0]                                   # (of that or a cut, the second launch left out)
     for f in ADD_WAVES:
         for waves in range(1, -(-M // (32 * f)) * nt // 256 + 1):
             cut = 256 * waves // nt * 32 * f
             rest = M - cut
             if rest <= 0:
                 break
-            c, g = min((_add_wave(rest, N, K, g), g) for g in ADD_WAVES)
+            c, g = min((_add_time(rest, N, K, g), g) for g in ADD_WAVES)
             apart = 10.0 + rest * N * K / 3.5e8 + rest * N / 2e5
             if rest < 512 and apart < c:
                 c, g = apart, 0
-            best = min(best, (_add_wave(cut, N, K, f) + c, ((0, cut, f), (cut, M, g))))
+            c += _add_time(cut, N, K, f)
+            took = min(took, c)
+            best = min(best, (c + CUT_US, ((0, cut, f), (cut, M, g))))
     whole = M * N / 2.0 ** 24 * (ADD_WAVES[8][0] + ADD_WAVES[8][1] * K)
-    return best[1] if whole >= (0.6 if then == THEN_NOTHING else 0.5) * best[0] else None
+    return best[1] if whole >= (0.6 if then == THEN_NOTHING else 0.5) * took else None
 
 
 # The same of gemm_prep.hip (K 2048: 39 us with 128 rows, 48 with 160, 54 with 192, 65 with 256)
