@@ -144,6 +144,13 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// LDS of one wave: what its lanes wrote is there for its other lanes
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The wave's sum in its last lane (only), on the vector pipe alone: no trip through LDS for an exchange.
 __device__ __forceinline__ float wave_sum_dpp(float v) {
   auto add = [&](auto ctrl, auto rows) {

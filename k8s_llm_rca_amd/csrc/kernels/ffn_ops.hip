@@ -124,11 +124,6 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i) {
     }
   }
 }
-// LDS written by one lane is read by another of the same wave: no reordering across this point
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
 
 // One token's choice by one wave: sc [Et] logits (LDS) -> weights and experts; ch [E], gs [NG]: scratch (LDS).
 struct RouteArgs {

@@ -29,13 +29,6 @@ enum Out { kBf16 = 0, kF32 = 1, kSilu = 2, kRelu2 = 3 };
 constexpr int NW = 4;                    // waves
 constexpr int CH = 64;                   // K entries of a chunk: rows of 128 bytes
 
-// LDS of one wave: what its lanes wrote is there for its other lanes
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // a wave's LDS: a chunk of W and of X, at the end its share of the sums (fp32)
 constexpr int wave_lds(int MT, int NF) {
   const int staged = 2 * CH * 16 * (MT + NF), sums = 4 * 16 * MT * 16 * NF;
@@ -43,7 +36,7 @@ constexpr int wave_lds(int MT, int NF) {
 }
 
 // grid (strips, K ranges); K range of kslice = NW waves x whole chunks.  MT, NF: 16-row fragments of X and of W.  SwiGLU: 8 NF gate rows,
-// then their up rows.  The last strip may begin within the one before it, whose columns both then write alike.
+// then their up rows.  The last strip may begin within the one before it, which writes the columns that both have.
 template <int MT, int NF, int OUT>
 __global__ void __launch_bounds__(64 * NW, MT + NF < 7 ? 2 : 1)
     gemm_batch_kernel(const uint16_t* __restrict__ x, int ldx, const uint16_t* __restrict__ w, void* __restrict__ y, int ldy, int M,

@@ -64,13 +64,6 @@ struct RowScale {
   float width, eps;
 };
 
-// LDS of one wave: what its lanes wrote is there for its other lanes
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // a wave's LDS: one chunk of W, at the end its share of the sums (fp32)
 constexpr int rows_lds(int MT, int NF, int CH) { return 16 * NF * (CH > 32 * MT ? CH : 32 * MT); }
 

@@ -28,13 +28,6 @@ namespace k8s {
 constexpr int kSpWaves = 8, kSpCols = 8, kSpStep = 64;    // K entries of a load instruction
 constexpr int kSpMaxLoads = 16, kSpMaxRows = 16, kSpSums = 64;
 
-// LDS of one wave: what its lanes wrote is there for its other lanes
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 struct StepProduct {
   const uint16_t* a;     // [M][lda]
   const uint16_t* w;     // [N][K]

@@ -13,8 +13,8 @@
 // A workgroup has a head of one sequence (V = 4 LV, D = DR RG), or of KIND 2 a slice of its columns; a thread four neighbouring columns of DR rows RG apart, so a
 // wave's accesses to the state are whole lines.  Nothing waits for anything but the state's address: rows,
 // gates and state are asked for together.  What bounds it: the state's bytes, read and written once (64 KB a head each way):
-// where every unit has several heads, memory;  with fewer, the rate of a unit, some 40 KB a us of both (7 sequences 4.7 us, of
-// which a launch takes 2.6).  A step reads the model's weights between two visits to a state, so that no cache holds it: it is
+// where every unit has a head, memory (KIND 2 with a workgroup a head of 128 x 128, 16 sequences of 16 heads: 7.2 us, of which a launch
+// takes 2.6);  with fewer, the rate of a unit, 48 to 68 KB a us of both (7 and 1 sequences 5.3 and 4.5 us).  A step reads the model's weights between two visits to a state, so that no cache holds it: it is
 // read and written without a place in the second-level cache (non-temporal), which would else have its written lines to give back
 // when the kernel ends.  us as ordinary / non-temporal accesses of states no cache holds:  KIND 2, 16 heads of 128 x 128, 1, 7, 16, 32,
 // 64 sequences 3.7 / 3.3, 6.1 / 4.7, 9.9 / 6.9, 17.9 / 12.8, 34 / 26 (5.2 TB/s; either alone 33 and 28);  KIND 1, 16 of 64 x 128,

@@ -1969,10 +1969,10 @@ def memory_layer(x: torch.Tensor, H: int, D: int, V: int, gate_bias: torch.Tenso
 
 def decay_slices(T: int, H: int, V: int) -> int:
     """Workgroups of a head in :func:`decay_layer`'s steps of ``T`` single tokens: four of 32 columns while half of the compute
-    units would have none.  A unit takes a state in and gives it back at some 40 KB a us (both counted).  us with 1 / 2 / 4 of
-    them, 16 heads of 128 x 128 at 1, 4, 7, 16, 32 tokens 4.6 / 3.8 / 3.3, 4.8 / 4.2 / 3.8, 5.2 / 4.6 / 4.7, 6.9 / 7.2 / 7.4, 12.8 /
-    14.9 / 14.9.  (Of states that a cache may hold:  8 heads at 7, 16 4.9 / 4.5 / 4.3, 6.1 / 5.8 / 5.9;  16 of 64 x 128 at 1, 7 3.9 /
-    3.8 / 3.7, 4.4 / 4.2 / 4.3;  32 of 64 x 64 at 1, 7 3.8 / 3.7, 4.2 / 4.3.)"""
+    units would have none.  A unit takes a state in and gives it back at some 48 to 68 KB a us (both counted, a launch's 2.6 us left
+    out).  us with 1 / 2 / 4 of them, states no cache holds:  16 heads of 128 x 128 at 1, 4, 7, 16, 32 tokens 4.5 / 3.8 / 3.3, 4.9 / 4.2 /
+    3.8, 5.3 / 4.7 / 4.7, 7.2 / 7.6 / 7.6, 13.4 / 15.0 / 15.2;  8 heads at 7, 16, 32 4.9 / 4.2 / 3.8, 5.4 / 4.8 / 5.1, 7.3 / 7.2 / 7.8;  16 of 64 x 128
+    at 1, 7, 16 3.6 / 3.3 / 3.1, 4.0 / 3.8 / 3.9, 5.0 / 5.0 / 5.5."""
     return 4 if V == 128 and T * H <= 128 and 4 * H <= 64 else 1      # (64 sums of squares a row: what the products behind take)
 
 

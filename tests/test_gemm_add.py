@@ -153,6 +153,29 @@ def test_gated(m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,quarters", [(4000, 2560, 64), (4096, 2816, 96)])
+def test_gated_in_a_split_tail(m, n, quarters):
+    """The same where the last wave's tiles go in four and in two, whose sums meet before they are divided: 64 and 96 of them."""
+    k = 4096
+    assert -(-m // 256) * (n // 128) % 256 == quarters
+    x, nw = rnd(m, k), 1 + 0.1 * rnd(k, seed=1)
+    w = (rnd(2 * n, k, seed=2) * k ** -0.5).to(BF)
+    h = (x * nw).to(BF)
+    part = (x * x).view(m, k // 256, 256).sum(2).contiguous()
+    L.reserve_big_ws(x.device)                           # (the workspace is the next stream's that asks for it: this one)
+    foreign = L.big_tail_foreign(x.device)
+    for _ in range(2):
+        got = L.gemm_big_silu_scaled(h, w, part, 1e-5)
+    assert L.big_tail_foreign(x.device) == foreign
+    g, u = ((h.double() @ w.double().T) / torch.sqrt((x.double() ** 2).mean(1, keepdim=True) + 1e-5)).split(n, 1)
+    # gate, up and the result are rounded to bf16 (2^-8 each), the sums in fp32 before that; the gate's slope is at most 1.1
+    half, s = 2.0 ** -8 * 1.01, 4e-6 * k ** 0.5
+    act = torch.nn.functional.silu(g)
+    tol = 1.1 * (half * g.abs() + s) * u.abs() + act.abs() * (half * u.abs() + s) + half * (act * u).abs() + s * s + 1e-6
+    assert float(((got.double() - act * u).abs() / tol).max()) < 1
+
+
+@pytest.mark.gpu
 def test_sublayers():
     """What the models call, at rows that take it: the pass and its product apart are the oracle."""
     m, W, F = 2600, 2048, 2048

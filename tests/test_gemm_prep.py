@@ -133,6 +133,55 @@ def test_entry_point(rows, D, over, pairs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,D,over,extras", [((700, 1, 599), 128, 0, False), ((1250, 50), 128, 16, True), ((1900, 900, 700), 128, 16, True),
+                                                ((3500,), 64, 0, True), ((2000, 1, 1499), 64, 512, False)])
+def test_entry_point_in_one_launch(rows, D, over, extras):
+    """Sizes that the rule gives to it, every sequence on pages of its own: what it gives against 64 bits, entry by entry, and against
+    product and pass of the same rows."""
+    H, G, V, K, BS, T = 2048 // D, 256 // D, D, 2048, 64, sum(rows)
+    NV, n = G * V, (H + 2 * G) * D
+    assert L.prep_plan(T, n + over, K, n) is not None
+    g = torch.Generator().manual_seed(T + D + over)
+    h, w = torch.randn(T, K, generator=g).to(BF).cuda(), (torch.randn(n + over, K, generator=g) * K ** -0.5).to(BF).cuda()
+    bias, qw, kw, vo = ((torch.randn(*s, generator=g).cuda() if extras else None) for s in ((n,), (D,), (D,), (T, NV)))
+    page0 = [sum(-(-r // BS) + 1 for r in rows[:i]) for i in range(len(rows) + 1)]
+    pages = page0[-1]
+    slots = torch.cat([torch.arange(r) + p * BS for r, p in zip(rows, page0)]).to(torch.int32).cuda()
+    pos = torch.cat([torch.arange(r) for r in rows]).to(torch.int32).cuda()
+    rope = None if extras and D == 128 else S.make_rope(D // 2, 1e4, "cuda")
+    cs = S.rope_table(pos, rope) if rope is not None else None
+
+    class Seg:
+        n_seg = len(rows)
+    out = []
+    for fused in (True, False):
+        kc, vt, vc = (torch.full(s, 7.0, device="cuda", dtype=BF) for s in ((pages, BS, G * D), (pages, NV, BS), (pages, BS, NV)))
+        keep = torch.empty(T, NV, device="cuda") if extras else None
+        prep = dict(norm=True, q_w=qw, k_w=kw, eps=1e-5, lam=0.3, v_other=vo, v_keep=keep, rope=rope, rope_cs=cs)
+        if fused:
+            made = S.proj_prep(h, w, bias, H, G, D, V, slots, kc, vc, vt, Seg, **prep)
+            assert made is not None and (made[1] is None) == (over == 0)
+            q, rest = made
+        else:
+            x = L.proj_f32out(h, w)
+            q, rest = S.attn_prep(x[:, :n], bias, H, G, D, V, pos, slots, kc, vc, BF, vt=vt, **prep), x[:, n:]
+        out.append((q, kc.view(-1, G * D)[slots.long()], vt.transpose(1, 2).reshape(-1, NV)[slots.long()], vc.view(-1, NV)[slots.long()],
+                    keep, rest if over else None))
+        written = torch.zeros(pages * BS, dtype=torch.bool, device="cuda")
+        written[slots.long()] = True
+        assert all(bool((t[~written] == 7).all()) for t in (kc.view(-1, G * D), vt.transpose(1, 2).reshape(-1, NV), vc.view(-1, NV)))
+    wq, wk, wv, wmix, wrest = oracle(h, w, bias, H, G, D, NV, cs, rope.dims if rope is not None else 0, True, qw, kw, 1e-5, 0.3, vo)
+    rel = 2.0 ** -8 * 1.01
+    for got in out:
+        for t, want, r in zip(got, (wq, wk, wmix, wmix, wv, wrest), (rel, rel, rel, rel, 1e-6, 1e-6)):
+            if t is not None:
+                close(t, want, r)
+    for a, b in zip(*out):
+        if a is not None:                                # two roundings of sums in different orders: a unit of bf16 apart
+            assert bool(((a.float() - b.float()).abs() <= 2.0 ** -7 * b.float().abs() + 2e-4).all())
+
+
+@pytest.mark.gpu
 def test_refused():
     z = torch.zeros(1 << 16, device="cuda", dtype=BF)
     f = torch.zeros(1 << 14, device="cuda")
