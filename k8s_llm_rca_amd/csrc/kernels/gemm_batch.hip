@@ -17,7 +17,8 @@
 //   2560 x 2048              9.3 / 6.6     9.4 / 7.0     9.9 / 8.1    10.1 / 9.3
 //   2576 x 2048, fp32 out    7.3 / 6.7     8.1 / 7.2     9.9 / 8.2    10.1 / 9.3
 //   16384 x 2048, fp32 out  13.6 / 13.1   14.2 / 13.4   17.8 / 14.7   18.0 / 16.3
-//   2048 x 8192, K ranges    9.2 / 8.0     9.1 / 8.4     9.5 / 9.7     9.7 / 10.7
+//   2048 x 8192, K ranges    9.2 / 8.0     9.1 / 8.4     9.5 / 9.7     9.7 / 10.7    (and the norm's pass, which has four planes to
+//                           13.2 / 12.1   13.3 / 11.8   13.6 / 13.2   14.1 / 14.4     read for eight)
 // The rule of what it takes: ops/linear.py, batch_plan.
 #include "common.h"
 #include "gates.h"
