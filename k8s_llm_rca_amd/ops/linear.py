@@ -814,7 +814,7 @@ def gemm_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, scale: float, pl
 
 def add_ok(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:
     """Layout :func:`gemm_add` needs of the residual [M, N] (or [M, 1, N]) and the operands."""
-    return (_few_ok(a, w) and a.shape[1] == w.shape[1] and x.dtype == torch.float32 and x.is_contiguous()
+    return (_few_ok(a, w) and a.shape[1] == w.shape[1] <= a.stride(0) and x.dtype == torch.float32 and x.is_contiguous()
             and x.data_ptr() % 16 == 0 and x.numel() == a.shape[0] * w.shape[0] and x.device == a.device == w.device)
 
 

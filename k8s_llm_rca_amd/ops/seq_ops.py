@@ -1433,7 +1433,7 @@ def proj_prep(h: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], H:
     NQ, NK, NV = H * D, G * D, G * V
     n, (N, K), rot = NQ + NK + NV, w.shape, rope.dims if rope is not None else 0
     if not (vt is not None and use_hip(h) and D in (64, 128) and norm in (False, None, True, "head") and N >= n and N % 4 == 0
-            and NQ % 256 == NK % 256 == NV % 256 == 0 and NV > 0 and h.shape == (T, K) and LIN._few_ok(h, w)
+            and NQ % 256 == NK % 256 == NV % 256 == 0 and NV > 0 and h.shape == (T, K) and LIN._few_ok(h, w) and h.stride(0) >= K
             and (rope is None or not rope.pairs and rope_cs is not None and 8 <= rot <= D and rot & (rot - 1) == 0)
             and unwatched(h, w)):
         return None
@@ -1442,6 +1442,7 @@ def proj_prep(h: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], H:
     if not (all(t is None or t.dtype == torch.float32 and t.is_contiguous() and t.numel() == m and t.data_ptr() % 16 == 0
                 and t.device == h.device for t, m in small)
             and all(t is None or t.is_contiguous() and t.dtype == dt and t.data_ptr() % 16 == 0 for t in (kc, vc, vt))
+            and all(t is None or t.shape == (T, m) for t, m in ((v_other, NV), (v_keep, NV), (rope_cs, rot)))
             and kc.shape[2] == NK and (vc is None or vc.shape[1:] == (BS, NV)) and vt.shape[1:] == (NV, BS)
             and slots.dtype == torch.int32 and slots.is_contiguous()):
         return None

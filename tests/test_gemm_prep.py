@@ -192,3 +192,22 @@ def test_refused():
                     (9, 12), (9, 16), (9, 128), (10, 2), (17, 0), (18, 0), (19, 0), (20, 0), (22, 0), (23, 128), (24, 128), (25, 0), (26, 96),
                     (26, 32)):
         assert lib().k8s_gemm_prep(*ok[:at], bad, *ok[at + 1:]) != 0, (at, bad)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stride,flat", [(0, False), (1024, False), (2048, True)])
+def test_left_to_product_and_pass(stride, flat):
+    """Rows that overlap, and another layer's values in another shape, are not taken: product and pass say what they say of them."""
+    T, K, H, G, D, NV, BS = 1300, 2048, 16, 2, 128, 256, 64
+    h = torch.zeros(T * stride + K, device="cuda", dtype=BF).as_strided((T, K), (stride, 1))
+    w, vo = torch.zeros(2560, K, device="cuda", dtype=BF), torch.zeros(T, NV, device="cuda")
+    kc, vt = (torch.zeros(T // BS + 1, *s, device="cuda", dtype=BF) for s in ((BS, G * D), (NV, BS)))
+    slots = torch.arange(T, dtype=torch.int32, device="cuda")
+
+    class Seg:
+        n_seg = 1
+    assert L.prep_plan(T, 2560, K, 2560) is not None
+    args = (w, None, H, G, D, 128, slots, kc, None, vt, Seg)
+    good = S.proj_prep(torch.zeros(T, K, device="cuda", dtype=BF), *args, norm=True, v_other=vo, lam=0.5)
+    assert good is not None
+    assert S.proj_prep(h, *args, norm=True, v_other=vo.view(-1) if flat else vo, lam=0.5) is None
