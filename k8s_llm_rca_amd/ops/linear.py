@@ -704,7 +704,10 @@ def _waves_time(waves: dict, M: int, N: int, K: int, f: int) -> float:
     return full * t + ((0.75 + 0.25 * over / 256) * t if over else 0.0)
 
 
-# us of a second launch: its own, and a chip that the first one leaves to drain
+# us of a second launch: its own, and a chip that the first one leaves to drain.  (But whole waves of 256-row tiles with tanh go in
+# two: inside an engine's prompts of 16000 and 16384 rows of 2048 columns, two launches / one 12.55 / 12.62 and 12.84 / 12.89 ms, 13.45 / 13.57 on
+# another card, though one of them after the other takes 176 / 172 us.  With the norm left, with smaller tiles and from three waves on one is
+# as quick or quicker: 19.10 / 19.06, 8.54 / 8.50, 19.04 / 19.04.)
 CUT_US = 5.0
 
 
@@ -744,12 +747,13 @@ def add_plan(M: int, N: int, K: int, then: int):
             if rest <= 0:
                 break
             c, g = min((_add_time(rest, N, K, g), g) for g in ADD_WAVES)
-            apart = 10.0 + rest * N * K / 3.5e8 + rest * N / 2e5
-            if rest < 512 and apart < c:
-                c, g = apart, 0
+            own = 10.0 + rest * N * K / 3.5e8 + rest * N / 2e5
+            if rest < 512 and own < c:
+                c, g = own, 0
             c += _add_time(cut, N, K, f)
             took = min(took, c)
-            best = min(best, (c + CUT_US, ((0, cut, f), (cut, M, g))))
+            charge = -1.0 if then == THEN_DYT and f == g == 8 and 256 % nt == 0 else CUT_US
+            best = min(best, (c + charge, ((0, cut, f), (cut, M, g))))
     whole = M * N / 2.0 ** 24 * (ADD_WAVES[8][0] + ADD_WAVES[8][1] * K)
     least = 0.5 + min(0.14, 0.02 * max(0, K - 4096) / 1024)
     return best[1] if whole >= (max(0.6, least) if then == THEN_NOTHING else least) * took else None
