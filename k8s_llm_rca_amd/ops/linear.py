@@ -732,7 +732,8 @@ def add_plan(M: int, N: int, K: int, then: int):
     1.13 - 1.18 and 1.25, 0.80 1.05 - 1.27 and 1.11 - 1.37, 1.00 1.01 - 1.19 and 1.01 - 1.27, over 1024 to 5120 columns and a K of
     1024 to 14336.  Without a norm there is the pass that reads it left (with its time, product and pass over both: at 0.55 0.95 -
     1.00, 0.66 1.01 - 1.06, 0.80 0.99 - 1.17, 0.85 1.00 - 1.20).  With a longer K the library has a wave that is not full the quicker; over
-    product and pass with tanh, K 6144 at 0.52 0.96, 0.54 1.01, 0.59 1.06;  8192 at 0.52 0.92, 0.54 1.02, 0.58 0.98, 0.59 1.05, 0.65 1.10;  11008 at
+    product and pass with tanh, K 6144 at 0.52 0.96, 0.54 1.01, 0.59 1.06;  8192 at 0.52 0.92, 0.54 1.02, 0.55 1.08 (2048 columns) and 1.12
+    (4096), 0.58 0.98, 0.59 1.05, 0.65 1.10;  11008 at
     0.52 - 0.57 0.90 - 0.99, 0.63 0.93, 0.65 1.11, 0.67 1.13 - 1.25;  14336 at 0.51 - 0.59 0.83 - 0.98, 0.63 0.94, 0.65 1.06, 0.67 1.12 and more.
     Without a norm, from ADD_ROWS on, there is the product that adds itself (0.82 0.90, 0.86 0.98 - 1.17, 1.00 0.96 - 1.08: it stays)."""
     if N % 256 or N > ADD_MAX_N or K % 64 or not 1024 <= K <= 16384 or M < ADD_MIN_ROWS or then == THEN_NOTHING and M >= ADD_ROWS:
@@ -755,7 +756,7 @@ def add_plan(M: int, N: int, K: int, then: int):
             charge = -1.0 if then == THEN_DYT and f == g == 8 and 256 % nt == 0 else CUT_US
             best = min(best, (c + charge, ((0, cut, f), (cut, M, g))))
     whole = M * N / 2.0 ** 24 * (ADD_WAVES[8][0] + ADD_WAVES[8][1] * K)
-    least = 0.5 + min(0.14, 0.02 * max(0, K - 4096) / 1024)
+    least = 0.5 + min(0.14, (0.0115 * max(0, min(K, 8192) - 4096) + 0.032 * max(0, K - 8192)) / 1024)
     return best[1] if whole >= (max(0.6, least) if then == THEN_NOTHING else least) * took else None
 
 

@@ -52,11 +52,12 @@ def test_plan_cuts():
 
 
 def test_plan_of_long_k():
-    """Product and pass apart while few of a wave's tiles have a long K: sizes timed on both sides."""
-    for n, k, yes, no in ((2048, 4096, 2400, 2048), (2048, 6144, 2800, 2400), (2048, 8192, 2800, 2400), (5120, 8192, 1300, 1100),
+    """Product and pass apart while few of a wave's tiles have a long K: sizes on both sides of the line (nearly all of them timed)."""
+    for n, k, yes, no in ((2048, 4096, 2400, 2048), (2048, 6144, 2800, 2400), (2048, 8192, 2600, 2400),
                           (3072, 11008, 2400, 2048), (4096, 11008, 1684, 1300), (2048, 14336, 3300, 2800), (5120, 14336, 1300, 1100)):
         assert L.add_plan(yes, n, k, L.THEN_DYT) and L.add_plan(yes, n, k, L.THEN_SCALED)
         assert L.add_plan(no, n, k, L.THEN_DYT) is None and L.add_plan(no, n, k, L.THEN_NOTHING) is None, (no, n, k)
+    assert L.add_plan(1300, 4096, 8192, L.THEN_DYT)
     assert L.add_plan(3517, 2048, 8192, L.THEN_NOTHING) and L.add_plan(3072, 3072, 14336, L.THEN_NOTHING)
     assert L.add_plan(2048, 3072, 14336, L.THEN_NOTHING) is None and L.add_plan(2048, 3072, 8192, L.THEN_NOTHING)
 
