@@ -13,9 +13,9 @@
 // What bounds it: with 256-row tiles the power limit (1.4 PFLOP/s); with 128 and 160 rows the fragments' way out of LDS, a
 // phase's 12 to 14 reads a wave in front of 16 to 20 matrix instructions (1.15 - 1.2 PFLOP/s, what the library's tiles of that size
 // do).  us of product and pass / of this with tanh, 2048 x 2048 and 2048 x 8192 at 2600, 4096, 4850, 6144, 10000, 16384 rows:
-//   45 / 43, 61 / 49, 71 / 56, 72 / 65, 116 / 106, 169 / 161;   102 / 94, 139 / 119, 160 / 140, 173 / 167, 350 / 289, 434 / 418;
-// with the norm left to the product behind 44 / 40, 58 / 45, 70 / 51, 72 / 59, 113 / 96, 168 / 145;   98 / 94, 134 / 117, 156 / 133, 172 / 163,
-// 349 / 276, 431 / 406.  tanh is 5 to 11 us of it a wave of tiles: vector instructions while the matrix units wait.
+//   45 / 42, 60 / 48, 70 / 55, 71 / 64, 112 / 105, 170 / 159;   107 / 99, 136 / 120, 160 / 138, 174 / 169, 344 / 284, 424 / 419;
+// with the norm left to the product behind 44 / 39, 57 / 44, 69 / 51, 71 / 58, 112 / 98, 169 / 146;   101 / 94, 134 / 117, 159 / 136, 168 / 163,
+// 341 / 274, 429 / 405.  tanh is 5 to 11 us of it a wave of tiles: vector instructions while the matrix units wait.
 // The residual asked for in front of the last tile's products, with that tile's code of its own, changed nothing (registers).
 #include "row_tiles.h"
 
